@@ -282,6 +282,116 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
   return HGPU_OK;
 }
 
+// Large fp32 products on the bf16 matrix cores (gemm_split.hip).  Takes products whose row, column, contracted and
+// batch indices are single dims with strides that a 32-bit byte offset reaches.
+int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out) {
+  if (p.m.nd != 1 || p.n.nd != 1 || p.k.nd != 1 || p.bt.nd != 1) return HGPU_OK;
+  const int64_t nt = n_terms > 0 ? n_terms : 1;
+  SplitParams q{};
+  int64_t sam = p.m.sa[0], sak = p.k.sa[0], sbn = p.n.sb[0], sbk = p.k.sb[0], scm = p.m.sc[0], scn = p.n.sc[0], M = p.M, N = p.N;
+  int64_t bsa = p.bt.sa[0], bsb = p.bt.sb[0];
+  bool swap = scm == 1 && scn != 1;          // the lanes of a result block run along its columns
+  if (swap) {
+    std::swap(sam, sbn);
+    std::swap(sak, sbk);
+    std::swap(scm, scn);
+    std::swap(M, N);
+    std::swap(bsa, bsb);
+  }
+  if (sam < 0 || sak < 0 || sbn < 0 || sbk < 0 || p.K > (1 << 24)) return HGPU_OK;
+  const int64_t a_bytes = ((M - 1) * sam + (p.K - 1) * sak + 1) * 4, b_bytes = ((N - 1) * sbn + (p.K - 1) * sbk + 1) * 4;
+  if (a_bytes > 0x7fffff00 || b_bytes > 0x7fffff00 || M > 0x3fffffff || N > 0x3fffffff) return HGPU_OK;
+  q.M = (int)M;
+  q.N = (int)N;
+  q.K = (int)p.K;
+  q.sam = (uint32_t)(sam * 4);
+  q.sak = (uint32_t)(sak * 4);
+  q.sbn = (uint32_t)(sbn * 4);
+  q.sbk = (uint32_t)(sbk * 4);
+  q.scm = scm;
+  q.scn = scn;
+  q.bsa = bsa;
+  q.bsb = bsb;
+  q.bsc = p.bt.sc[0];
+  q.a_bytes = (uint32_t)a_bytes;
+  q.b_bytes = (uint32_t)b_bytes;
+  q.n_terms = n_terms;
+  for (int t = 0; t < n_terms; ++t) {
+    q.a_term[t] = (const float*)(swap ? p.b_term[t] : p.a_term[t]);
+    q.b_term[t] = (const float*)(swap ? p.a_term[t] : p.b_term[t]);
+  }
+  const int64_t out_n = nelem(out);
+  int cfg = 0, split = 1;
+  {
+    // Microseconds, as measured: a step of 16 k of a 256 x 256 tile (one block on a CU) 3.4, of a 128 x 128 tile
+    // 1.4 alone on its CU and 0.92 for each of several; 8 for the launch with its first loads and last stores; for
+    // partial results a second launch and their bytes once out and once in.  (2048 x 8192 over 2048: 395-425 us
+    // in 256 x 256 tiles, 450-480 in 128 x 128; 2048 x 784 over 8192, where 256-wide tiles would be a quarter
+    // empty: 217 against 203; 300 x 5000 over 784: 37 with its partial sums in 128 x 128 tiles and K in four.)
+    double best = 1e300;
+    for (int c = 0; c < 2; ++c) {
+      const int64_t bm = c == 0 ? 256 : 128, tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * p.BT * nt;
+      for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
+        const int64_t per_cu = (tiles * sp + ctx->num_cu - 1) / ctx->num_cu, steps = ((p.K + sp - 1) / sp + 15) / 16;
+        const double step = c == 0 ? 3.4 * per_cu : (per_cu == 1 ? 1.4 : 0.92 * per_cu);
+        const double us = 8 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 4 / 3.2e6 : 0);
+        if (us < best) { best = us; cfg = c; split = (int)sp; }
+      }
+    }
+  }
+  const int64_t BM = cfg == 0 ? 256 : 128, BN = BM;
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  q.kchunk = (int)(((p.K + split - 1) / split + 15) / 16 * 16);
+  q.term_split = (int)((p.K + q.kchunk - 1) / q.kchunk);
+  split = (int)(q.term_split * nt);
+  if (split > 65535 || tiles * split > 0x3fffffff || (split > 1 && (double)out_n * split > 5e8)) return HGPU_OK;
+  hgpu_buffer* part = nullptr;
+  if (split > 1) {
+    int rc = buffer_alloc(ctx, (size_t)out_n * split * 4, &part);
+    if (rc) return rc;
+  }
+  q.c_split_stride = split > 1 ? out_n : 0;
+  {
+    const double flops = 2.0 * M * N * p.K * p.BT * nt;
+    const double bytes = (((double)M * p.K + (double)N * p.K) * nt + (double)M * N) * p.BT * 4;
+    const char* label = "gemm_f32";
+    if (ctx->profiling && ctx->profile_shapes) {
+      char buf[128];
+      char terms[24] = "";
+      if (nt > 1) snprintf(terms, sizeof terms, ",terms%lld", (long long)nt);
+      snprintf(buf, sizeof buf, "%s[M%lldxN%lldxK%lldxB%lld,s%d,%s%s,split3,t%lldx%lld%s]", label, (long long)M, (long long)N, (long long)p.K, (long long)p.BT, split,
+               sak == 1 ? "K" : "M", sbk == 1 ? "K" : "N", (long long)BM, (long long)BN, terms);
+      label = intern_label(ctx, buf);
+    }
+    void* cdst = split > 1 ? part->ptr : data_ptr(out);
+    LaunchArgs la{ctx->stream, cfg, 0, 0, sak == 1, sbk == 1, dim3((unsigned)tiles, (unsigned)split, (unsigned)p.BT), swap ? pb : pa, swap ? pa : pb, cdst, nullptr, nullptr};
+    {
+      LaunchGuard lg(ctx, label, bytes, flops);
+      la.ev_start = lg.start_event();
+      la.ev_stop = lg.stop_event();
+      launch_split_f32(q, la);
+    }
+    if (split > 1 && partials_out && split <= 3 && is_dense(out)) {
+      int64_t sh[HGPU_MAX_RANK + 1], st[HGPU_MAX_RANK + 1];
+      sh[0] = split;
+      for (int d = 0; d < out->rank; ++d) sh[d + 1] = out->shape[d];
+      dense_strides(out->rank + 1, sh, st);
+      *partials_out = new_view(ctx, part, HGPU_F32, out->rank + 1, sh, st, 0);
+    } else if (split > 1) {
+      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * 4, (double)out_n * split);
+      launch_sum_partials<float>(ctx, out_n, split, (const float*)part->ptr, (float*)data_ptr(out));
+    }
+  }
+  const hipError_t e = hipGetLastError();
+  if (part) buffer_release(part);
+  if (e != hipSuccess) {
+    if (partials_out && *partials_out) { hgpu_release(*partials_out); *partials_out = nullptr; }
+    return check_hip(ctx, e, "gemm");
+  }
+  *handled = true;
+  return HGPU_OK;
+}
+
 }  // namespace
 
 namespace hg {
@@ -406,6 +516,11 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     const hgpu_array* none = nullptr;
     const int slot = 0;
     int rc = try_smallk(ctx, n_terms > 0 ? n_terms : 1, ta, tb, n_keep, 1, &none, 0, 0, nullptr, std::vector<int>{a->dtype}, 1, &slot, &out, handled);
+    if (rc || *handled) return rc;
+  }
+  // (a side under 96 leaves more than a quarter of a 128-wide tile empty: the smaller tiles of the fp32 instruction)
+  if (a->dtype == HGPU_F32 && p.M >= 96 && p.N >= 96 && p.K >= 64) {
+    int rc = gemm_split(ctx, p, pa, pb, out, handled, n_terms, partials_out);
     if (rc || *handled) return rc;
   }
   // (under a long K the staged kernel's coalesced tile loads win even with most of a 32-wide tile empty: the recurrent network's

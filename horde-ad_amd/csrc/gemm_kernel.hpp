@@ -774,6 +774,22 @@ void launch(const GemmParams& p, const LaunchArgs& a) {
   }
 }
 
+// Products whose rows, columns, contracted and batch dims are single dims with non-negative strides
+// (gemm_split.hip).  Strides of the operands in bytes, of the result in elements.
+struct SplitParams {
+  int M, N, K;
+  uint32_t sam, sak, sbn, sbk;
+  int64_t scm, scn;
+  int64_t bsa, bsb, bsc;        // batch strides in elements
+  uint32_t a_bytes, b_bytes;    // extent of one batch element of an operand
+  int kchunk;
+  int64_t c_split_stride;
+  int n_terms, term_split;
+  const float* a_term[kMaxTerms];
+  const float* b_term[kMaxTerms];
+};
+void launch_split_f32(const SplitParams& p, const LaunchArgs& a);
+
 // defined in gemm_f32.hip / gemm_f64.hip
 void launch_f32(const GemmParams& p, const LaunchArgs& a);
 void launch_f64(const GemmParams& p, const LaunchArgs& a);

@@ -1,0 +1,356 @@
+// fp32 matrix products on the bf16 matrix cores, without giving up fp32.
+//
+// An fp32 number with a normal exponent is the exact sum of three bf16 numbers
+// (8 + 8 + 8 significant bits): x = h + m + l, each part the nearest bf16 of
+// what is left.  A product of two such sums has nine terms; the six largest are
+// h h', h m', m h', m m', h l', l h', and the three left out (m l', l m', l l')
+// together stay below 2^-25 of the product -- half of what rounding the product
+// to fp32 would cost.  Every term of the six is a product of two 8-bit numbers,
+// exact in fp32, and they are added into fp32 accumulators, as
+// v_mfma_f32_32x32x2_f32 adds its products.
+//
+// Exactness of the split needs |x| (when not zero) between 2^-100 and 2^127: below,
+// a part could be subnormal, above, rounding to bf16 could overflow, and an
+// infinity or NaN has no remainder.  Every staged element is checked; a block
+// that has met an element outside that range computes its tile again with
+// v_mfma_f32_32x32x2_f32, so such inputs give what they always gave.
+//
+// What bounds it: the power the matrix cores draw.  Six bf16 instructions of 32 x 32 x 16 do the work of eight
+// fp32 ones of 32 x 32 x 2 in under half the cycles; at 2048 x 8192 over 2048 the clock falls to 1.8 GHz and
+// orders of the loop's instructions that differ by a fifth in stalls measure the same.  So the tile is the largest
+// whose accumulators leave two wavefronts to a SIMD (256 x 256, eight wavefronts, each operand element is split
+// once for 256 columns): 645 us on the fp32 instruction, 417-425 here (165 TFLOP/s) on normally distributed
+// numbers, 577 and 375-395 on the activations of a wide relu network (128 x 128: 450-480).  Sixteen products are
+// summed from zero and then added to the accumulator with one rounded addition: fed to the matrix cores on
+// top of a large accumulator the small terms lose their low bits (error against fp64, 2048 terms, normal /
+// positive: 2.3e-7 / 1.7e-7; with the accumulator in the chain 7.0e-7 / 4.3e-7 at 375 us; fp32 instruction
+// 8.1e-7 / 3.5e-7).
+#include "gemm_kernel.hpp"
+
+using namespace hg;
+using namespace hg::gemm;
+
+namespace {
+
+using bf8 = __bf16 __attribute__((ext_vector_type(8)));
+using bf2 = __bf16 __attribute__((ext_vector_type(2)));
+using f2 = float __attribute__((ext_vector_type(2)));
+using f4u = float __attribute__((ext_vector_type(4), aligned(4)));
+using f16v = float __attribute__((ext_vector_type(16)));
+using u4 = uint32_t __attribute__((ext_vector_type(4)));
+
+constexpr int SK = 16;                      // k of one step: one MFMA deep
+
+// Eight consecutive k of one row on their way to LDS.
+struct Slot { float v[8]; };
+
+// Range of the elements met so far, as bit patterns shifted left by one (the sign gone).
+struct Seen { uint32_t hi, lo; };          // largest; smallest of the non-zero ones, minus one
+constexpr uint32_t kLargest = 0xfe000000u; // 2^127, doubled pattern
+constexpr uint32_t kSmallest = 0x1b000000u - 1;  // 2^-100
+
+__device__ __forceinline__ uint32_t pack(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf2));
+}
+
+// the three parts of two neighbours
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = pack(a, b);
+  const float a1 = a - __builtin_bit_cast(float, h << 16), b1 = b - __builtin_bit_cast(float, h & 0xffff0000u);
+  m = pack(a1, b1);
+  l = pack(a1 - __builtin_bit_cast(float, m << 16), b1 - __builtin_bit_cast(float, m & 0xffff0000u));
+}
+
+// Element (16 bytes) of row r, k half h within one part of a tile: rows of 32 bytes, the halves
+// swapped in every other group of four rows so that eight neighbouring rows of one half lie in different banks.
+__device__ __forceinline__ int lds_at(int r, int h) { return r * 2 + (h ^ ((r >> 3) & 1)); }
+
+// One operand's share of a tile: ROWS rows of SK elements, a lane owns NS pieces of eight k each.
+// Loads go through a buffer descriptor over the operand: a fixed 32-bit offset per lane plus a
+// scalar one for the step, and whatever lies past the end (rows, k) reads as zero.
+template <int ROWS, bool KC, int NT>
+struct Side {
+  static constexpr int NS = ROWS * 2 / NT;
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off[NS];                         // bytes
+  int at[NS];
+  uint32_t ks;                              // bytes between neighbouring k
+
+  __device__ __forceinline__ void init(int t, const float* base, uint32_t bytes, uint32_t rs, int r0, int rows, uint32_t stride) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00027000);
+    ks = stride;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      // lanes run along whichever of k and the rows is contiguous
+      const int r = KC ? t / 2 + i * (NT / 2) : (t + i * NT) % ROWS;
+      const int h = KC ? t & 1 : (t + i * NT) / ROWS;
+      off[i] = (uint32_t)(r0 + r < rows ? r0 + r : rows - 1) * rs + 8 * h * ks;   // (rows past the end: never stored)
+      at[i] = lds_at(r, h);
+    }
+  }
+  // A whole step that starts at k0.
+  __device__ __forceinline__ void load(int k0, Slot* s) const {
+    const uint32_t so = (uint32_t)k0 * ks;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      if constexpr (KC) {
+        const f4u a = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[i], so, 0));
+        const f4u b = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[i] + 16, so, 0));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { s[i].v[j] = a[j]; s[i].v[4 + j] = b[j]; }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[i].v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[i], so + j * ks, 0));
+      }
+    }
+  }
+  // The last step of a chunk when it is not a whole one: `left` elements of k.
+  __device__ __forceinline__ void load_tail(int t, int k0, int left, Slot* s) const {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int h = KC ? 8 * (t & 1) : 8 * ((t + i * NT) / ROWS);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        s[i].v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, h + j < left ? off[i] + (k0 + j) * ks : 0xfffffff0u, 0, 0));
+    }
+  }
+  // parts: [3][ROWS * 2] of 16 bytes
+  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, Seen& seen) const {
+    u4 h, m, l;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = s.v[2 * j], b = s.v[2 * j + 1];
+      uint32_t ph, pm, pl;
+      split2(a, b, ph, pm, pl);
+      h[j] = ph;
+      m[j] = pm;
+      l[j] = pl;
+      const uint32_t ua = __builtin_bit_cast(uint32_t, a) << 1, ub = __builtin_bit_cast(uint32_t, b) << 1;
+      seen.hi = max(seen.hi, max(ua, ub));
+      seen.lo = min(seen.lo, min(ua - 1, ub - 1));
+    }
+    parts[at[i]] = h;
+    parts[ROWS * 2 + at[i]] = m;
+    parts[ROWS * 4 + at[i]] = l;
+  }
+};
+
+// Wavefronts WM x WN, each TM x TN blocks of 32 x 32.
+template <int WM, int WN, int TM, int TN, bool AKC, bool BKC>
+__global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
+  constexpr int CH = 2;                     // blocks of a wavefront whose chains of products alternate
+  constexpr int NT = 64 * WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
+  constexpr int PA = 3 * BM * 2, PB = 3 * BN * 2;       // 16-byte elements of one buffer
+  __shared__ u4 lds[2][PA + PB];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+
+  // each XCD works on a contiguous range of (K chunk, tile) pairs, as in k_gemm
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  const int ntiles = tiles_m * tiles_n;
+  const int nblocks = ntiles * gridDim.y;
+  int lin = blockIdx.x + ntiles * blockIdx.y;
+  if (nblocks >= 64) {
+    const int x = lin & 7, per = nblocks >> 3, rem = nblocks & 7;
+    lin = x * per + (x < rem ? x : rem) + (lin >> 3);
+  }
+  const int s = lin / ntiles, bid = lin - s * ntiles;
+  // tiles in bands of eight rows of tiles: neighbours in the order share operands
+  const int band = bid / (8 * tiles_n), in_band = bid - band * 8 * tiles_n;
+  const int rows_in_band = tiles_m - band * 8 < 8 ? tiles_m - band * 8 : 8;
+  const int tile_n = in_band / rows_in_band, tile_m = band * 8 + (in_band - tile_n * rows_in_band);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+  int sk = s;
+  if (p.n_terms > 0) {
+    const int term = s / p.term_split;
+    sk = s - term * p.term_split;
+    A = p.a_term[term];
+    B = p.b_term[term];
+  }
+  A += (int64_t)blockIdx.z * p.bsa;
+  B += (int64_t)blockIdx.z * p.bsb;
+  const int kbeg = sk * p.kchunk;
+  const int kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
+
+  Side<BM, AKC, NT> sa;
+  Side<BN, BKC, NT> sb;
+  sa.init(t, A, p.a_bytes, p.sam, m0, p.M, p.sak);
+  sb.init(t, B, p.b_bytes, p.sbn, n0, p.N, p.sbk);
+  constexpr int NA = Side<BM, AKC, NT>::NS, NB = Side<BN, BKC, NT>::NS;
+
+  f16v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+  Seen seen{0, 0xffffffffu};
+
+  const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
+  Slot ra[NA], rb[NB];
+  auto fetch = [&](int i) {                 // (chosen outside the main loop: a load on one side of a branch would be waited for where the sides meet)
+    sa.load(kbeg + i * SK, ra);
+    sb.load(kbeg + i * SK, rb);
+  };
+  auto fetch_tail = [&](int i) {
+    sa.load_tail(t, kbeg + i * SK, kend - kbeg - i * SK, ra);
+    sb.load_tail(t, kbeg + i * SK, kend - kbeg - i * SK, rb);
+  };
+  if (whole > 0) fetch(0);
+  else fetch_tail(0);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) sa.store(ra[i], i, lds[0], seen);
+#pragma unroll
+  for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, seen);
+  __syncthreads();
+
+  const int fra = lds_at(wm * TM * 32 + (lane & 31), lane >> 5), frb = lds_at(wn * TN * 32 + (lane & 31), lane >> 5);
+  // One step: the loads of the next step go out, the products of this one are formed, and the
+  // next step's elements are split and stored to the other buffer behind the products.
+  // next: 0 = there is none, 1 = a whole step, 2 = the rest of K.
+  auto step = [&](int i0, auto next) {
+    constexpr bool more = decltype(next)::value != 0;
+    const int cur = i0 & 1;
+    if constexpr (decltype(next)::value == 1) fetch(i0 + 1);
+    if constexpr (decltype(next)::value == 2) fetch_tail(i0 + 1);
+    __builtin_amdgcn_sched_barrier(0);      // (left to itself the compiler moves the loads down to their use)
+    const u4* la = lds[cur] + fra;
+    const u4* lb = lds[cur] + PA + frb;
+    u4* ln = lds[cur ^ 1];
+    bf8 fa[TM][3];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fa[i][q] = __builtin_bit_cast(bf8, la[q * BM * 2 + i * 64]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      bf8 fb[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fb[q] = __builtin_bit_cast(bf8, lb[q * BN * 2 + j * 64]);
+      // The six terms of 16 k are summed from zero, the smallest first, and added to the accumulators with one
+      // rounded addition: small terms fed to the matrix cores on top of a large accumulator lose their low bits.
+#pragma unroll
+      for (int i0 = 0; i0 < TM; i0 += CH) {
+        f16v c[CH];
+        auto add = [&](int qa, int qb) {
+#pragma unroll
+          for (int i = 0; i < CH; ++i) c[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i0 + i][qa], fb[qb], c[i], 0, 0, 0);
+        };
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) c[i][r] = 0;
+        add(2, 0);
+        add(0, 2);
+        add(1, 1);
+        add(1, 0);
+        add(0, 1);
+        add(0, 0);
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] += c[i][r];
+      }
+      if constexpr (more) {       // the loads have had the first columns' products to arrive
+        constexpr int first = 2;
+        if (j >= first) {
+          const int u = j - first;
+          if (u < NA) sa.store(ra[u], u, ln, seen);
+          else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, seen);
+        }
+      }
+    }
+    if constexpr (more) {
+      constexpr int first = 2;
+#pragma unroll
+      for (int u = TN - first; u < NA + NB; ++u) {
+        if (u < NA) sa.store(ra[u], u, ln, seen);
+        else sb.store(rb[u - NA], u - NA, ln + PA, seen);
+      }
+    }
+    __syncthreads();
+  };
+  int i0 = 0;
+#pragma unroll 1
+  for (; i0 + 1 < whole; ++i0) step(i0, std::integral_constant<int, 1>{});
+  if (i0 + 1 < steps) {
+    step(i0, std::integral_constant<int, 2>{});
+    ++i0;
+  }
+  step(i0, std::integral_constant<int, 0>{});
+
+  float* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)s * p.c_split_stride;
+  auto put = [&](int i, int j, const f16v& c) {
+    const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
+    if (n >= p.N) return;
+    float* col = Cout + (int64_t)n * p.scn;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = m0 + (wm * TM + i) * 32 + MfmaF32W::row(lane, r);
+      if (m < p.M) col[(int64_t)m * p.scm] = c[r];
+    }
+  };
+  if (__syncthreads_or(seen.hi >= kLargest || seen.lo < kSmallest)) {
+    // an element that three bf16 cannot hold exactly: the tile again, on the fp32 instruction
+#pragma unroll 1
+    for (int ij = 0; ij < TM * TN; ++ij) {
+      const int i = ij / TN, j = ij - i * TN;
+      const int rowa = m0 + (wm * TM + i) * 32 + (lane & 31), rowb = n0 + (wn * TN + j) * 32 + (lane & 31);
+      const uint32_t ga = (uint32_t)(rowa < p.M ? rowa : p.M - 1) * p.sam, gb = (uint32_t)(rowb < p.N ? rowb : p.N - 1) * p.sbn;
+      f16v c;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c[r] = 0;
+#pragma unroll 1
+      for (int k0 = kbeg; k0 < kend; k0 += 8) {
+        float fa[4], fb[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int k = k0 + 2 * u + (lane >> 5);
+          fa[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sa.rsrc, k < kend ? ga + k * sa.ks : 0xfffffff0u, 0, 0));
+          fb[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb.rsrc, k < kend ? gb + k * sb.ks : 0xfffffff0u, 0, 0));
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u], fb[u], c, 0, 0, 0);
+      }
+      put(i, j, c);
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) put(i, j, acc[i][j]);
+}
+
+template <typename F>
+void launch_as(const LaunchArgs& a, int threads, F kernel, const SplitParams& p) {
+  const float* A = (const float*)a.A;
+  const float* B = (const float*)a.B;
+  float* C = (float*)a.C;
+  if (a.ev_start || a.ev_stop) hipExtLaunchKernelGGL(kernel, a.grid, dim3(threads), 0, a.stream, a.ev_start, a.ev_stop, 0, p, A, B, C);
+  else hipLaunchKernelGGL(kernel, a.grid, dim3(threads), 0, a.stream, p, A, B, C);
+}
+
+template <int WM, int WN, int TM, int TN>
+void launch_tile(const SplitParams& p, const LaunchArgs& a) {
+  constexpr int threads = 64 * WM * WN;
+  if (a.va && a.vb) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, true, true>, p);
+  else if (a.va) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, true, false>, p);
+  else if (a.vb) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, false, true>, p);
+  else launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, false, false>, p);
+}
+
+}  // namespace
+
+namespace hg {
+namespace gemm {
+
+void launch_split_f32(const SplitParams& p, const LaunchArgs& a) {
+  if (a.cfg == 0) launch_tile<4, 2, 2, 4>(p, a);
+  else launch_tile<2, 2, 2, 2>(p, a);
+}
+
+}  // namespace gemm
+}  // namespace hg

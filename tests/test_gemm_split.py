@@ -1,0 +1,68 @@
+"""Large fp32 products on the bf16 matrix cores (csrc/gemm_split.hip): every operand is the exact sum of
+three bf16 numbers, elements that are not send their tile to the fp32 instruction."""
+import numpy as np
+import pytest
+
+from conftest import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def product(ctx, x, y, lay):
+    """x [M, K] times y [N, K]^T; lay: "K" = stored with k contiguous, "R" = stored with the rows contiguous."""
+    a = ctx.upload(x) if lay[0] == "K" else ctx.upload(np.ascontiguousarray(x.T)).transpose([1, 0])
+    b = ctx.upload(y) if lay[1] == "K" else ctx.upload(np.ascontiguousarray(y.T)).transpose([1, 0])
+    return a.replicate([y.shape[0]]).transpose([1, 0, 2]).contract(b.replicate([x.shape[0]]), 2)
+
+
+def assert_close(out, x, y, k):
+    """Sixteen products per rounded addition plus the roundings inside the sixteen and of the partial sums:
+    at most (K / 16 + 16) half-ulps of the sum of magnitudes; the three terms left out stay under 2^-25 of it."""
+    x, y = x.astype(np.float64), y.astype(np.float64)
+    bound = (k / 16 + 17) * 2.0 ** -24 * (np.abs(x) @ np.abs(y).T) + 1e-45
+    assert np.all(np.abs(out.astype(np.float64) - x @ y.T) <= bound)
+
+
+@pytest.mark.parametrize("lay", ["KK", "KR", "RK", "RR"])
+@pytest.mark.parametrize("m,n,k", [(128, 128, 1040), (129, 257, 1041), (300, 500, 1077), (255, 96, 2063), (2050, 514, 520), (97, 2300, 1025)])
+def test_ragged_shapes(gpu, m, n, k, lay):
+    rng = np.random.default_rng(m + n + k)
+    x, y = rng.standard_normal((m, k)).astype(np.float32), rng.uniform(0, 1, (n, k)).astype(np.float32)
+    assert_close(product(gpu, x, y, lay).numpy(), x, y, k)
+
+
+@pytest.mark.parametrize("scale", [1e-35, 1e-30, 1e30, 1.5e38])
+def test_elements_that_three_bf16_cannot_hold(gpu, scale):
+    """Tiny and huge operands: the products themselves stay in fp32's normal range."""
+    m, n, k = 200, 300, 1030
+    rng = np.random.default_rng(5)
+    x = (rng.uniform(-1, 1, (m, k)) * scale).astype(np.float32)
+    y = (rng.uniform(-1, 1, (n, k)) / scale / (64 if scale > 1 else 1)).astype(np.float32)
+    out = product(gpu, x, y, "KR").numpy()
+    xd, yd = x.astype(np.float64), y.astype(np.float64)
+    # (the fp32 instruction rounds once per product)
+    assert np.all(np.abs(out - xd @ yd.T) <= (k + 17) * 2.0 ** -24 * (np.abs(xd) @ np.abs(yd).T))
+
+
+def test_infinities_and_nans_stay_where_they_belong(gpu):
+    m, n, k = 260, 140, 1100
+    rng = np.random.default_rng(6)
+    x, y = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(0.5, 1, (n, k)).astype(np.float32)
+    x[3, 7], x[200, 1099], y[130, 0] = np.inf, np.nan, -np.inf
+    out = product(gpu, x, y, "RK").numpy()
+    want = x.astype(np.float64) @ y.astype(np.float64).T
+    assert np.array_equal(np.isnan(out), np.isnan(want))
+    assert np.array_equal(np.isposinf(out), np.isposinf(want)) and np.array_equal(np.isneginf(out), np.isneginf(want))
+    fine = np.isfinite(want)
+    assert np.all(np.abs(out[fine] - want[fine]) <= (k + 17) * 2.0 ** -24 * want[fine])
+
+
+@pytest.mark.parametrize("terms", [2, 5])
+def test_sum_of_products(gpu, terms):
+    m, n, k = 130, 100, 2000
+    rng = np.random.default_rng(terms)
+    xs = [rng.standard_normal((m, k)).astype(np.float32) for _ in range(terms)]
+    ys = [rng.standard_normal((n, k)).astype(np.float32) for _ in range(terms)]
+    pairs = [(gpu.upload(x).replicate([n]).transpose([1, 0, 2]), gpu.upload(y).replicate([m])) for x, y in zip(xs, ys)]
+    out = gpu.contract_sum(pairs, 2).numpy()
+    assert_close(out, np.concatenate(xs, 1), np.concatenate(ys, 1), terms * k)
