@@ -384,6 +384,312 @@ hipError_t scatter_sorted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, i
   return e;
 }
 
+// ---- scatter-add by counting -------------------------------------------------
+// Up to 2^20 positions into a table whose cells are hit a few hundred times on average: instead of
+// sorting all positions by destination, count the hits of every cell, hand every cell a stretch of `val`,
+// drop the positions there in any order, and let the lanes that add up a cell put its few positions in
+// ascending order first.  Five short passes over 4-byte words (M positions, C cells) replace the ten launches
+// of a radix or merge sort of (key, position) pairs, and the pass that adds up writes every cell, empty ones
+// too, so that the result is not cleared beforehand.  100,000 rows of 512 bytes into 20,000 cells: 134 us with
+// the sort, 37 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
+// position gets varies from run to run, the sums do not.
+constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (beyond, a run that a whole block adds up could hold too large a share of the work)
+constexpr int64_t kCountedPerCell = 512;
+constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; longer runs: k_cell_big
+constexpr int kBigList = 8192;       // positions of one run that k_cell_big orders in LDS; longer runs: found in order by reading all of cell[]
+
+// cell[m] = position m's destination (or ~0: skipped), rank[m] = how many positions of that cell counted before it.
+// Lanes of a wavefront that go to one cell count with one addition (twice, for the commonest cells of a skewed table).
+__global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, uint32_t* __restrict__ counts, uint32_t* __restrict__ cell, uint32_t* __restrict__ rank) {
+  const int64_t step = (int64_t)gridDim.x * kBlock;
+  const int lane = threadIdx.x & 63;
+  for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63); base < M; base += step) {
+    const int64_t m = base + lane;
+    int64_t toff = 0, doff;
+    const bool ok = m < M && resolve(sp, m, &toff, &doff);
+    const uint32_t c = ok ? (uint32_t)toff : 0xffffffffu;
+    uint32_t r = 0;
+    bool todo = ok;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const unsigned long long open = __ballot(todo);
+      if (!open) break;
+      const int first = __ffsll((long long)open) - 1;
+      const uint32_t c0 = __shfl(c, first);
+      const unsigned long long same = __ballot(todo && c == c0);
+      uint32_t b = 0;
+      if (lane == first) b = atomicAdd(&counts[c0], (uint32_t)__popcll(same));
+      b = __shfl(b, first);
+      if (todo && c == c0) {
+        r = b + (uint32_t)__popcll(same & ((1ull << lane) - 1));
+        todo = false;
+      }
+    }
+    if (todo) r = atomicAdd(&counts[c], 1u);
+    if (m < M) {
+      cell[m] = c;
+      rank[m] = r;
+    }
+  }
+}
+
+// Where each cell's stretch of val starts: the cells of a block side by side, the blocks in any order (globals[0] is
+// the next free place).  Cells with long runs are listed (globals[1] of them).
+constexpr int kCellsPerBlock = 1024;
+__global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_t* __restrict__ counts, uint32_t* __restrict__ starts, uint32_t* __restrict__ globals, uint32_t* __restrict__ big) {
+  __shared__ uint32_t sums[kBlock];
+  __shared__ uint32_t base;
+  const int t = threadIdx.x;
+  const int64_t c0 = (int64_t)blockIdx.x * kCellsPerBlock + 4 * t;
+  uint32_t n[4], total = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    n[i] = c0 + i < C ? counts[c0 + i] : 0;
+    total += n[i];
+  }
+  sums[t] = total;
+  __syncthreads();
+  for (int d = 1; d < kBlock; d <<= 1) {
+    const uint32_t v = t >= d ? sums[t - d] : 0;
+    __syncthreads();
+    sums[t] += v;
+    __syncthreads();
+  }
+  if (t == kBlock - 1) base = atomicAdd(&globals[0], sums[t]);
+  __syncthreads();
+  uint32_t at = base + sums[t] - total;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (c0 + i < C) starts[c0 + i] = at;
+    at += n[i];
+    if (n[i] > kSmallRun) big[atomicAdd(&globals[1], 1u)] = (uint32_t)(c0 + i);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_cell_place(int64_t M, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ rank, uint32_t* __restrict__ val) {
+  const int64_t step = (int64_t)gridDim.x * kBlock;
+  for (int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x; m < M; m += step) {
+    const uint32_t c = cell[m];
+    if (c != 0xffffffffu) val[starts[c] + rank[m]] = (uint32_t)m;
+  }
+}
+
+template <typename T, int V> struct UnitOf { using type = T __attribute__((ext_vector_type(V), aligned(sizeof(T)))); };
+template <typename T> struct UnitOf<T, 1> { using type = T; };
+
+// A group of G lanes (8 to 64) per cell: its positions go to LDS, every lane finds the ranks of its share of them, and
+// then the lanes run along the cell's N elements (V at a time) and add the positions' slices in ascending order,
+// four loads in flight.
+template <typename T, int V>
+__global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts,
+                                                     const uint32_t* __restrict__ val, const T* __restrict__ src, T* __restrict__ out) {
+  using U = typename UnitOf<T, V>::type;
+  __shared__ uint32_t raw_all[kBlock / 8][kSmallRun], list_all[kBlock / 8][kSmallRun];
+  const int g = threadIdx.x / G, l = threadIdx.x % G;
+  uint32_t* raw = raw_all[g];
+  uint32_t* list = list_all[g];
+  const int64_t units = N / V, step = (int64_t)gridDim.x * (kBlock / G);
+  for (int64_t c = (int64_t)blockIdx.x * (kBlock / G) + g; c < C; c += step) {
+    const uint32_t n = counts[c];
+    if (n > kSmallRun) continue;
+    const uint32_t* mine = val + starts[c];
+    for (uint32_t e = l; e < n; e += G) raw[e] = mine[e];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t e = l; e < n; e += G) {
+      const uint32_t p = raw[e];
+      uint32_t r = 0;
+      for (uint32_t d = 0; d < n; ++d) r += raw[d] < p ? 1 : 0;
+      list[r] = p;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int64_t u = l; u < units; u += G) {
+      int64_t io[1] = {u * V};
+      if constexpr (V == 1) decompose<1>(inner, u, io);
+      const T* from = src + io[0];
+      U acc{};
+      uint32_t j = 0;
+      for (; j + 4 <= n; j += 4) {
+        const U a = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])), b = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 1]));
+        const U d = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 2])), e = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 3]));
+        acc = (U)(acc + a);
+        acc = (U)(acc + b);
+        acc = (U)(acc + d);
+        acc = (U)(acc + e);
+      }
+      for (; j < n; ++j) acc = (U)(acc + *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])));
+      *reinterpret_cast<U*>(out + c * N + u * V) = acc;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Cells hit more than kSmallRun times, a block for each: the positions in ascending order (sorted in LDS, or, for a
+// run that does not fit there, met in order by going through cell[]), cut into segments of kSeg, the lanes
+// sharing segments and elements between them, segment sums added in ascending order.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_cell_big(IxSpace sp, Dims inner, int64_t M, int64_t N, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts,
+                                                     const uint32_t* __restrict__ val, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ globals,
+                                                     const uint32_t* __restrict__ big, const T* __restrict__ src, T* __restrict__ out) {
+  __shared__ uint32_t list[kBigList];
+  __shared__ T red[kBlock];
+  __shared__ uint32_t wave_n[8][4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t n_big = globals[1];
+  for (uint32_t i = blockIdx.x; i < n_big; i += gridDim.x) {
+    const uint32_t c = big[i], n = counts[c];
+    const bool fits = n <= (uint32_t)kBigList;
+    if (fits) {
+      const uint32_t* mine = val + starts[c];
+      uint32_t P = 2 * kSmallRun;
+      while (P < n) P <<= 1;
+      for (uint32_t e = t; e < P; e += kBlock) list[e] = e < n ? mine[e] : 0xffffffffu;
+      for (uint32_t k = 2; k <= P; k <<= 1)
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+          __syncthreads();
+          for (uint32_t q = t; q < P / 2; q += kBlock) {
+            const uint32_t a = (q / j) * 2 * j + q % j, b = a + j;
+            const uint32_t x = list[a], y = list[b];
+            if ((x > y) == ((a & k) == 0)) {
+              list[a] = y;
+              list[b] = x;
+            }
+          }
+        }
+      __syncthreads();
+    }
+    for (int64_t n0 = 0; n0 < N; n0 += kBlock) {
+      const int nc = (int)(N - n0 < kBlock ? N - n0 : kBlock), R = kBlock / nc;
+      const int seg = t / nc, col = t - seg * nc;
+      int64_t io[1] = {0};
+      if (seg < R) decompose<1>(inner, n0 + col, io);
+      const T* from = src + io[0];
+      T tot = T(0);
+      bool have = false;
+      auto add_list = [&](uint32_t cnt) {      // list[0 .. cnt) starts a segment
+        const uint32_t segs = (cnt + kSeg - 1) / kSeg;
+        for (uint32_t g0 = 0; g0 < segs; g0 += R) {
+          T acc = T(0);
+          const uint32_t me = g0 + seg;
+          if (seg < R && me < segs) {
+            const uint32_t e1 = me * kSeg + kSeg < cnt ? me * kSeg + kSeg : cnt;
+            uint32_t j = me * kSeg;
+            for (; j + 4 <= e1; j += 4) {
+              const T a = from[data_offset(sp, (int64_t)list[j])], b = from[data_offset(sp, (int64_t)list[j + 1])];
+              const T d = from[data_offset(sp, (int64_t)list[j + 2])], e = from[data_offset(sp, (int64_t)list[j + 3])];
+              acc = (T)(acc + a);
+              acc = (T)(acc + b);
+              acc = (T)(acc + d);
+              acc = (T)(acc + e);
+            }
+            for (; j < e1; ++j) acc = (T)(acc + from[data_offset(sp, (int64_t)list[j])]);
+          }
+          red[t] = acc;
+          __syncthreads();
+          if (t < nc)
+            for (int r = 0; r < R && g0 + r < segs; ++r) {
+              const T v = red[r * nc + t];
+              tot = have ? (T)(tot + v) : v;
+              have = true;
+            }
+          __syncthreads();
+        }
+      };
+      if (fits) {
+        add_list(n);
+      } else {
+        uint32_t held = 0;
+        for (int64_t m0 = 0; m0 < M; m0 += 8 * kBlock) {
+          bool is[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int64_t m = m0 + j * kBlock + t;
+            is[j] = m < M && cell[m] == c;
+            const unsigned long long b = __ballot(is[j]);
+            if (lane == 0) wave_n[j][wave] = (uint32_t)__popcll(b);
+          }
+          __syncthreads();
+          uint32_t at = held;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const unsigned long long b = __ballot(is[j]);
+            uint32_t before = at;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const uint32_t k = wave_n[j][w];
+              if (w < wave) before += k;
+              at += k;
+            }
+            if (is[j]) list[before + (uint32_t)__popcll(b & ((1ull << lane) - 1))] = (uint32_t)(m0 + j * kBlock + t);
+          }
+          held = at;
+          __syncthreads();
+          if (held > (uint32_t)(kBigList - 8 * kBlock)) {      // no room for another round: add the whole segments
+            const uint32_t whole = held / kSeg * kSeg, rest = held - whole;
+            add_list(whole);
+            const uint32_t keep = t < (int)rest ? list[whole + t] : 0;
+            __syncthreads();
+            if (t < (int)rest) list[t] = keep;
+            held = rest;
+            __syncthreads();
+          }
+        }
+        add_list(held);
+      }
+      if (t < nc) out[(int64_t)c * N + n0 + t] = tot;
+    }
+    __syncthreads();
+  }
+}
+
+// k_cell_count -> k_cell_starts -> k_cell_place -> k_cell_sum, k_cell_big.  sp's table strides are in slices; every
+// element of o is written.
+hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, int64_t M, int64_t N, int64_t C, const hgpu_array* src, hgpu_array* o, int* rc_out) {
+  const int64_t n_big = M / (kSmallRun + 1) + 1;
+  hgpu_buffer* wb = nullptr;
+  const int64_t head = (C + 2 + 3) / 4 * 4;        // counters and the two globals, cleared together
+  *rc_out = buffer_alloc(ctx, (size_t)(head + C + 3 * M + n_big) * 4, &wb);
+  if (*rc_out) return hipSuccess;
+  uint32_t* counts = (uint32_t*)wb->ptr;
+  uint32_t* globals = counts + C;
+  uint32_t* starts = counts + head;
+  uint32_t* cell = starts + C;
+  uint32_t* rank = cell + M;
+  uint32_t* val = rank + M;
+  uint32_t* big = val + M;
+  const size_t es = dtype_size(src->dtype);
+  *rc_out = zero_fill(ctx, counts, (size_t)head * 4);
+  if (*rc_out) { buffer_release(wb); return hipSuccess; }
+  LaunchGuard lg(ctx, "scatter_counted", 2.0 * M * N * es + 8.0 * M * sp.n_ix, (double)M * N);
+  const unsigned gm = grid_for(M, kBlock, ctx->num_cu * 8);
+  hipLaunchKernelGGL(k_cell_count, dim3(gm), dim3(kBlock), 0, ctx->stream, sp, M, counts, cell, rank);
+  hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, globals, big);
+  hipLaunchKernelGGL(k_cell_place, dim3(gm), dim3(kBlock), 0, ctx->stream, M, (const uint32_t*)starts, (const uint32_t*)cell, (const uint32_t*)rank, val);
+  // 16-byte units when the slices are contiguous and every one starts on a boundary of its elements
+  const bool contiguous = inner.nd == 1 && (inner.st[0][0] == 1 || N == 1);
+  const int V = es >= 4 && (src->dtype == HGPU_F64 || src->dtype == HGPU_F32) && contiguous && N % (int64_t)(16 / es) == 0 ? (int)(16 / es) : 1;
+  int G = 8;
+  while (G < 64 && G < N / V) G <<= 1;
+  const unsigned gc = grid_for(C, kBlock / G, ctx->num_cu * 16);
+  if (V == 2)
+    hipLaunchKernelGGL((k_cell_sum<double, 2>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts, (const uint32_t*)val, (const double*)data_ptr(src), (double*)data_ptr(o));
+  else if (V == 4)
+    hipLaunchKernelGGL((k_cell_sum<float, 4>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts, (const uint32_t*)val, (const float*)data_ptr(src), (float*)data_ptr(o));
+  else
+    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_sum<T, 1>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts,
+                                                        (const uint32_t*)val, (const T*)data_ptr(src), (T*)data_ptr(o)));
+  if (M > kSmallRun) {
+    const unsigned gb = (unsigned)(n_big < ctx->num_cu * 2 ? n_big : ctx->num_cu * 2);
+    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_big<T>), dim3(gb), dim3(kBlock), 0, ctx->stream, sp, inner, M, N, (const uint32_t*)counts, (const uint32_t*)starts,
+                                                        (const uint32_t*)val, (const uint32_t*)cell, (const uint32_t*)globals, (const uint32_t*)big, (const T*)data_ptr(src), (T*)data_ptr(o)));
+  }
+  const hipError_t e = hipGetLastError();
+  buffer_release(wb);
+  return e;
+}
+
 int build_space(hgpu_ctx* ctx, const char* who, int n_ix, const hgpu_array* const* ix, int rank_m, const int64_t* shm,
                 const int64_t* data_st, IxSpace* sp) {
   if (n_ix < 0 || n_ix > kMaxIx) return fail(ctx, HGPU_ERR_UNSUPPORTED, "%s: %d index arrays (at most %d)", who, n_ix, kMaxIx);
@@ -530,8 +836,12 @@ int hgpu_scatter_add(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_
   for (int i = 0; i < n_ix; ++i) osh[i] = shp[i];
   for (int i = 0; i < rank_m; ++i) M *= src->shape[i];
   for (int i = 0; i < rank_n; ++i) { osh[n_ix + i] = src->shape[rank_m + i]; N *= src->shape[rank_m + i]; }
+  int64_t C = 1;
+  for (int i = 0; i < n_ix; ++i) C *= shp[i];
+  // (more cells than eight to a position: passes over the cells would outweigh those over the positions)
+  const bool counted = (flags & 1) == 0 && M > 0 && N > 0 && C > 0 && M <= kCountedPositions && M <= kCountedPerCell * C && C <= 8 * M + 4096;
   hgpu_array* o = nullptr;
-  int rc = new_zeros(ctx, src->dtype, n_ix + rank_n, osh, &o);
+  int rc = counted ? new_dense(ctx, src->dtype, n_ix + rank_n, osh, &o) : new_zeros(ctx, src->dtype, n_ix + rank_n, osh, &o);
   if (rc) return rc;
   if (M * N == 0 || nelem(o) == 0) { *out = o; return HGPU_OK; }
   IxSpace sp;
@@ -539,7 +849,7 @@ int hgpu_scatter_add(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_
   if (rc) { hgpu_release(o); return rc; }
   for (int k = 0; k < n_ix; ++k) {
     sp.extent[k] = shp[k];
-    sp.table_st[k] = o->strides[k];
+    sp.table_st[k] = counted ? o->strides[k] / N : o->strides[k];
   }
   const int64_t* is[1] = {src->strides + rank_m};
   Dims inner;
@@ -557,7 +867,9 @@ int hgpu_scatter_add(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_
   // sort the positions by destination (stable: colliding positions stay in ascending order), then sum every run in that order
   if (M >= (int64_t)1 << 32) { hgpu_release(o); return fail(ctx, HGPU_ERR_UNSUPPORTED, "scatter: %lld positions", (long long)M); }
   hipError_t e;
-  {
+  if (counted) {
+    e = scatter_counted(ctx, sp, inner, M, N, C, src, o, &rc);
+  } else {
     LaunchGuard lg(ctx, "scatter_sorted", 2.0 * M * N * dtype_size(src->dtype) + 8.0 * M * n_ix, (double)M * N);
     // destinations that fit 32 bits sort as 32-bit keys: half the bytes per sorting pass
     e = nelem(o) < (int64_t)0xffffffff ? scatter_sorted<uint32_t>(ctx, sp, inner, M, N, src, o, &rc) : scatter_sorted<uint64_t>(ctx, sp, inner, M, N, src, o, &rc);

@@ -1,0 +1,60 @@
+"""The scatter-add that counts the hits of every cell (csrc/index.hip): bit-equal to the checker while no cell is hit
+more than 256 times (positions of a cell are added in ascending order), within rounding of the sum of magnitudes beyond."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def check(both, src, idx, cells):
+    arr, ix = both.upload(src), [both.upload(idx)]
+    res = both.scatter_add(arr, ix, 1, [cells])
+    g, o = res.numpy()
+    inside = (idx >= 0) & (idx < cells)
+    hits = np.bincount(idx[inside], minlength=cells)
+    short = hits <= 256
+    assert np.array_equal(g[short], o[short])
+    if src.dtype.kind == "f" and not short.all():
+        mass = np.zeros((cells,) + src.shape[1:])
+        np.add.at(mass, idx[inside], np.abs(src[inside]).astype(np.float64))
+        eps = np.finfo(src.dtype).eps
+        bound = (256 + hits / 256.0 + 2)[(slice(None),) + (None,) * (src.ndim - 1)] * eps * mass
+        # (the checker adds a whole run front to back: its own error is hits * eps)
+        assert np.all(np.abs(g - o.astype(np.float64)) <= bound + hits.reshape((-1,) + (1,) * (src.ndim - 1)) * eps * mass)
+    else:
+        assert np.array_equal(g, o)
+    assert np.array_equal(g, both.scatter_add(arr, ix, 1, [cells]).numpy()[0])     # the same again
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int64, np.int16, np.int8])
+@pytest.mark.parametrize("width", [1, 2, 7, 16, 128, 300])
+def test_runs_at_the_edges_of_the_kernels(both, dt, width):
+    """Cells hit 0, 1, 63 .. 65, 255 .. 257 times: a group's LDS list, a segment, one more."""
+    rng = np.random.default_rng(width)
+    counts = np.array([0, 1, 2, 8, 63, 64, 65, 127, 128, 129, 255, 256, 257, 0, 512, 513, 3])
+    idx = rng.permutation(np.concatenate([np.repeat(np.arange(len(counts)), counts), [-1, len(counts), 1 << 40]])).astype(np.int64)
+    shape = (len(idx),) if width == 1 else (len(idx), width)
+    src = rng.integers(-100, 100, shape).astype(dt) if np.dtype(dt).kind == "i" else rng.standard_normal(shape).astype(dt)
+    check(both, src, idx, len(counts))
+
+
+@pytest.mark.parametrize("width", [1, 5])
+def test_runs_longer_than_the_lds_list(both, width):
+    rng = np.random.default_rng(9)
+    idx = rng.permutation(np.concatenate([np.full(8192, 3), np.full(8193, 7), np.full(21001, 90), rng.integers(0, 400, 5000)])).astype(np.int64)
+    src = rng.standard_normal((len(idx),) if width == 1 else (len(idx), width))
+    check(both, src, idx, 400)
+
+
+def test_many_cells_and_two_index_dims(both):
+    rng = np.random.default_rng(10)
+    i, j = rng.integers(-1, 151, 40000).astype(np.int64), rng.integers(0, 90, 40000).astype(np.int64)
+    src = both.upload(rng.standard_normal((40000, 12)).astype(np.float32))
+    g, o = both.scatter_add(src, [both.upload(i), both.upload(j)], 1, [150, 90]).numpy()
+    assert np.array_equal(g, o)
+    check(both, rng.standard_normal((3000, 32)), rng.integers(0, 25000, 3000).astype(np.int64), 25000)
+    # a strided view of the data: slices that are not contiguous
+    wide = both.upload(rng.standard_normal((24, 3000)))
+    idx = both.upload(rng.integers(0, 700, 3000).astype(np.int64))
+    g, o = both.scatter_add(wide.transpose([1, 0]), [idx], 1, [700]).numpy()
+    assert np.array_equal(g, o)
