@@ -4,6 +4,7 @@
 // (src/HordeAd/Core/DeltaEval.hs:391-595).  Each rule cites the delta
 // constructor it transposes.
 #include <algorithm>
+#include <cstring>
 
 #include "host.hpp"
 
@@ -30,6 +31,7 @@ static void accum(std::vector<T>& slots, int node, const T& cot) {
 }
 
 std::vector<T> Tape::backward(const D& out, const T& dt, const std::vector<D>& inputs) {
+  be->unit_products.clear();
   std::vector<T> slots(recs.size());
   std::vector<bool> keep(recs.size(), false);
   for (auto& i : inputs)
@@ -48,6 +50,11 @@ std::vector<T> Tape::backward(const D& out, const T& dt, const std::vector<D>& i
     if (i.node >= 0 && slots[(size_t)i.node].valid()) res.push_back(slots[(size_t)i.node]);
     else res.push_back(zeros(be, i.primal.dtype(), i.primal.shape()));   // tdefTarget
   }
+  // A leaf that came through products with one only is an array of the forward pass: the caller gets its own copy.
+  for (T& r : res)
+    for (const auto& u : be->unit_products)
+      if (r.holder() == u && u->h) { r = materialize(r); break; }
+  be->unit_products.clear();
   // The gradient leaves are what the caller asked for: nothing stays pending,
   // and leaves of one shape that are still elementwise programs share a pass.
   force_many(res);
@@ -62,7 +69,26 @@ D d_const(const T& t) {
 
 // Products made by transposition rules stay pending: most are summed at once
 // by the rule of a `replicate` further up, which then is a single contraction.
-static T mul(const T& a, const T& b) { return lazy_mul(a, b); }
+// A factor that is the constant one at every position (the seed of a reverse pass, `grad`'s dt) leaves the
+// other factor as it is: no pass over it (rows of 51 MB that a lookup's cotangent multiplied by one: 16 us).
+static bool is_one(const T& t) {
+  Backend* be = t.be();
+  if (!be->fuse) return false;
+  const double one = 1.0;
+  uint64_t bits;
+  std::memcpy(&bits, &one, 8);
+  auto it = be->const_cache.find(std::make_pair(t.dtype(), bits));
+  if (it == be->const_cache.end()) return false;
+  const ArrHolder* h = t.holder().get();
+  for (int hop = 0; h && hop < 4; ++hop, h = h->scalar_src.get())
+    if (h == it->second.get()) return true;
+  return false;
+}
+static T mul(const T& a, const T& b) {
+  if (is_one(b)) { a.be()->unit_products.push_back(a.holder()); return a; }
+  if (is_one(a)) { b.be()->unit_products.push_back(b.holder()); return b; }
+  return lazy_mul(a, b);
+}
 static T add(const T& a, const T& b) { return ewise2(HGPU_ADD, a, b); }
 static T neg(const T& a) { return ewise1(HGPU_NEG, a); }
 static T recip(const T& a) { return ewise1(HGPU_RECIP, a); }

@@ -146,6 +146,7 @@ struct Backend {
   uint64_t walk_gen = 0;    // walks over pending expressions number themselves: a node seen carries the walk's number
   std::vector<std::weak_ptr<ArrHolder>> pending_dimsums;   // sums over all dims but one of an expression, not yet taken (ArrHolder::ones_b)
   std::vector<std::weak_ptr<ArrHolder>> pending_sums;   // sums of all elements of an expression, not yet taken (ArrHolder::ssrc)
+  std::vector<std::shared_ptr<ArrHolder>> unit_products;   // factors that a transposition rule multiplied by the constant one in the reverse pass under way
   std::map<std::string, int64_t> counters;   // how often each rewrite onto a fused entry point was taken (diagnostic)
   void check(int rc) const;
 };
