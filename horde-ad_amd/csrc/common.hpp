@@ -179,6 +179,18 @@ struct RedJob {
   const char* label = nullptr;
   double bytes = 0, flops = 0;
 };
+// One dense copy between two arrays that do not overlap (hgpu_assign): `bytes` bytes in units of 2^unit bytes, to which both sides are aligned.
+struct CopyJob {
+  const void* src;
+  void* dst;
+  int64_t bytes;
+  int unit;
+};
+constexpr int kMaxCopyJobs = 48;
+// ewise.hip: launches up to kMaxCopyJobs independent copies as one kernel (the caller holds launch_mu)
+hipError_t launch_copy_group(hgpu_ctx* ctx, const CopyJob* const* jobs, int n);
+// smallk.hip: holds a copy back (retaining both buffers) to be launched with the copies that follow it
+void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst);
 // contract.hip: launches up to four such reductions of one element type as one kernel (the caller holds launch_mu)
 hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int n);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now

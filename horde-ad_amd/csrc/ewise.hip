@@ -170,6 +170,44 @@ __global__ void __launch_bounds__(kBlock) k_copy(Dims d, int64_t n, const T* __r
   }
 }
 
+// Several dense copies as one launch: a block moves one piece of kCopyPiece bytes of one of them, found by walking
+// the table of first blocks (uniform, from the kernel's arguments).  Bound by launches, not by bytes: a training
+// step hands back 3 arrays per parameter (24 copies of 16 bytes to 400 KB for the CNN), which as launches of their
+// own cost 1.9 us each and a gap in a recorded graph (CNN training step, batch 250, fp32: 224 us with 24 launches,
+// 182 us with one).
+constexpr int kCopyPiece = 8192;
+struct CopyTable {
+  CopyJob job[kMaxCopyJobs];
+  uint32_t first[kMaxCopyJobs + 1];     // first block of each copy
+};
+static_assert(sizeof(CopyTable) <= 4000, "kernel arguments");
+
+// bytes [at, end), `at` a multiple of the unit; what is left of the last unit byte by byte
+template <typename U>
+__device__ __forceinline__ void copy_piece(const CopyJob& j, int64_t at, int64_t end) {
+  const U* a = (const U*)((const char*)j.src + at);
+  U* o = (U*)((char*)j.dst + at);
+  const int n = (int)((end - at) / (int64_t)sizeof(U));
+  for (int i = threadIdx.x; i < n; i += kBlock) o[i] = a[i];
+  const int64_t rest = at + (int64_t)n * (int64_t)sizeof(U) + threadIdx.x;
+  if (rest < end) ((char*)j.dst)[rest] = ((const char*)j.src)[rest];
+}
+
+__global__ void __launch_bounds__(kBlock) k_copy_group(CopyTable t) {
+  int k = 0;
+  while (blockIdx.x >= t.first[k + 1]) ++k;
+  const CopyJob j = t.job[k];
+  const int64_t at = (int64_t)(blockIdx.x - t.first[k]) * kCopyPiece;
+  const int64_t end = at + kCopyPiece < j.bytes ? at + kCopyPiece : j.bytes;
+  switch (j.unit) {
+    case 4: copy_piece<uint4>(j, at, end); break;
+    case 3: copy_piece<uint64_t>(j, at, end); break;
+    case 2: copy_piece<uint32_t>(j, at, end); break;
+    case 1: copy_piece<uint16_t>(j, at, end); break;
+    default: copy_piece<uint8_t>(j, at, end); break;
+  }
+}
+
 // Zero padding in one pass over the result: the dims of the (dense) result in
 // memory order, for each the padding in front, the source's extent and stride.
 struct PadDims {
@@ -284,6 +322,20 @@ int zero_fill(hgpu_ctx* ctx, void* p, size_t bytes) {
   hipLaunchKernelGGL(k_zero16, dim3(grid_for(n16, kBlock, max_blocks(ctx))), dim3(kBlock), 0, ctx->stream, n16, (uint4*)p);
   HG_CHECK_LAUNCH(ctx, "zero_fill");
   return HGPU_OK;
+}
+
+hipError_t launch_copy_group(hgpu_ctx* ctx, const CopyJob* const* jobs, int n) {
+  CopyTable t{};
+  uint32_t blocks = 0;
+  for (int i = 0; i < kMaxCopyJobs; ++i) {
+    t.first[i] = blocks;
+    if (i >= n) continue;
+    t.job[i] = *jobs[i];
+    blocks += (uint32_t)((jobs[i]->bytes + kCopyPiece - 1) / kCopyPiece);
+  }
+  t.first[kMaxCopyJobs] = blocks;
+  hipLaunchKernelGGL(k_copy_group, dim3(blocks), dim3(kBlock), 0, ctx->stream, t);
+  return hipGetLastError();
 }
 
 int copy_view(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const void* src, const int64_t* sst,

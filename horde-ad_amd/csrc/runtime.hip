@@ -612,6 +612,15 @@ int hgpu_assign(hgpu_ctx* ctx, hgpu_array* dst, const hgpu_array* src) {
     std::lock_guard<std::mutex> lk(ctx->launch_mu);
     ctx->write_epoch++;
   }
+  // Dense copies wait for the ones that follow (a step hands back all its parameters and moments, one call
+  // each) and go out as one launch.  From 16 MB on a copy is worth a launch of its own.
+  const size_t bytes = (size_t)nelem(dst) * dtype_size(dst->dtype);
+  if (is_dense(src) && src->buf && dst->buf && bytes < (16u << 20)) {
+    CopyJob j{data_ptr(src), data_ptr(dst), (int64_t)bytes, 4};
+    while ((((uintptr_t)j.src | (uintptr_t)j.dst) & (((uintptr_t)1 << j.unit) - 1)) != 0) --j.unit;
+    hold_copy(ctx, j, src->buf, dst->buf);
+    return HGPU_OK;
+  }
   return copy_view(ctx, dst->dtype, dst->rank, dst->shape, data_ptr(src), src->strides, data_ptr(dst), dst->strides);
 }
 

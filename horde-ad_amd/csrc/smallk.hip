@@ -619,7 +619,9 @@ namespace hg {
 // reads and writes (retained, so that none is handed out again before the launch).
 struct Deferred {
   bool is_reduction = false;   // a reduction of contract.hip (`red`) instead of a small product
+  bool is_copy = false;        // a copy into an existing array (`copy`); see hold_copy
   RedJob red;
+  CopyJob copy{};
   const std::string* body = nullptr;   // the problem's device code (kept with the known kernels) and the number that stands for it
   int body_id = -1;
   std::string kname;
@@ -633,8 +635,12 @@ struct Deferred {
   int level = 0;
 };
 
+// Products and reductions write new arrays only; copies write existing ones.  The
+// queue holds either products and reductions, or copies that touch no memory of
+// one another: whatever does not fit flushes it first.
 struct DeferredQueue {
   std::vector<Deferred> items;
+  bool copies = false;               // what `items` holds
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
 };
@@ -780,7 +786,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     for (auto* b : d.writes) buffer_retain(b);
     std::lock_guard<std::mutex> lk(ctx->launch_mu);
     if (!ctx->dq) ctx->dq = new DeferredQueue;
-    if (ctx->dq->items.size() >= kMaxHeld) flush_deferred_locked(ctx);
+    if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->copies) flush_deferred_locked(ctx);
     ctx->dq->items.push_back(std::move(d));
     ctx->dq_pending = true;
     *handled = true;
@@ -808,6 +814,32 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
   std::vector<Deferred> items;
   items.swap(ctx->dq->items);
   (void)hipSetDevice(ctx->device);
+  auto release_items = [&] {
+    for (auto& d : items) {
+      for (auto* b : d.reads) buffer_release(b);
+      for (auto* b : d.writes) buffer_release(b);
+    }
+  };
+  if (ctx->dq->copies) {
+    ctx->dq->copies = false;
+    std::vector<const CopyJob*> jobs;
+    double bytes = 0;
+    for (auto& d : items) { jobs.push_back(&d.copy); bytes += d.bytes; }
+    hgpu_ctx::ProfRec r{"copy_group", nullptr, nullptr, bytes, 0};
+    const bool timed = ctx->profiling && !ctx->cap && hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess;
+    if (timed) (void)hipEventRecord(r.a, ctx->stream);
+    const hipError_t err = launch_copy_group(ctx, jobs.data(), (int)jobs.size());
+    if (timed) {
+      (void)hipEventRecord(r.b, ctx->stream);
+      ctx->prof.push_back(r);
+    }
+    if (err != hipSuccess) {
+      int rc = check_hip(ctx, err, "grouped copy launch");
+      if (!ctx->deferred_rc) ctx->deferred_rc = rc;
+    }
+    release_items();
+    return;
+  }
   std::map<const hgpu_buffer*, int> written_at;
   int top = 0;
   for (auto& d : items) {
@@ -939,10 +971,7 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
       ctx->dq->n_launches += fn ? 1 : (long)grp.size();
     }
   }
-  for (auto& d : items) {
-    for (auto* b : d.reads) buffer_release(b);
-    for (auto* b : d.writes) buffer_release(b);
-  }
+  release_items();
 }
 
 // A single-launch reduction joins the queue: held back until something else needs the stream, levelled with
@@ -963,10 +992,38 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
   for (auto* b : d.writes) buffer_retain(b);
   std::lock_guard<std::mutex> lk(ctx->launch_mu);
   if (!ctx->dq) ctx->dq = new DeferredQueue;
-  if (ctx->dq->items.size() >= kMaxHeld) flush_deferred_locked(ctx);
+  if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->copies) flush_deferred_locked(ctx);
   ctx->dq->items.push_back(std::move(d));
   ctx->dq_pending = true;
   return true;
+}
+
+// A copy into an existing array joins the queue.  It waits only for copies: anything else that is enqueued goes
+// after the held copies (every launch flushes the queue), and a copy whose source or destination a held copy
+// writes, or whose destination a held copy reads, flushes them first.
+void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst) {
+  Deferred d;
+  d.is_copy = true;
+  d.copy = job;
+  d.bytes = 2.0 * (double)job.bytes;
+  d.reads.push_back(src);
+  d.writes.push_back(dst);
+  buffer_retain(src);
+  buffer_retain(dst);
+  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  if (!ctx->dq) ctx->dq = new DeferredQueue;
+  DeferredQueue& q = *ctx->dq;
+  static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
+  bool fits = q.items.empty() || (q.copies && q.items.size() < (size_t)kMaxCopyJobs);
+  for (size_t i = 0; fits && i < q.items.size(); ++i) {
+    const hgpu_buffer *r = q.items[i].reads[0], *w = q.items[i].writes[0];
+    fits = w != src && w != dst && r != dst;
+  }
+  if (!fits) flush_deferred_locked(ctx);
+  q.items.push_back(std::move(d));
+  q.copies = true;
+  ctx->dq_pending = true;
+  if (!hold) flush_deferred_locked(ctx);
 }
 
 void flush_deferred(hgpu_ctx* ctx) {
