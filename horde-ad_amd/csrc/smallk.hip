@@ -131,6 +131,8 @@ struct Spec {
   // instead of one block walking all of K); each block writes its partial tile, and a second launch of one block
   // per tile adds the partial tiles up in the order of K and runs the program
   int splits = 1, chunks_per_split = 0;
+  // WK = 4: a 16 x 16 tile per block, each wavefront a quarter of every chunk's k (see choose_flat); 1: wavefronts share K
+  int WK = 1;
 };
 
 // LDS pitch of a tile: the fragment reads of 16 rows x 4 k must not collide.
@@ -221,7 +223,8 @@ std::string generate_body(const Spec& sp) {
   const int64_t nbp = (sp.P + sp.BP - 1) / sp.BP, nbq = (sp.Q + sp.BQ - 1) / sp.BQ;
   const int S = sp.splits;
   const int64_t nblk = nbp * nbq, per_xcd = (nblk * S + 7) / 8;
-  const bool vec_epi = !sp.f64 && sp.P % 4 == 0;
+  const bool flat = sp.WK > 1;
+  const bool vec_epi = !flat && !sp.f64 && sp.P % 4 == 0;
   s << "typedef " << (sp.f64 ? "double" : "float") << " T;\n";
   s << "typedef T V2 __attribute__((ext_vector_type(2), aligned(" << (sp.f64 ? 8 : 4) << ")));\n";
   s << "typedef T V4 __attribute__((ext_vector_type(4), aligned(" << (sp.f64 ? 8 : 4) << ")));\n";
@@ -277,7 +280,9 @@ std::string generate_body(const Spec& sp) {
     else s << "  " << ct << " w" << i << "[4];\n";
   }
   s << "  int unused;\n};\n";
-  s << "__device__ __forceinline__ EpiIn epi_load(const Args& ar, i64 pb, i64 qb, int r, int g) {\n  EpiIn z;\n  z.unused = 0;\n";
+  // (only: the accumulator register this wavefront finishes; -1: all four)
+  const char* skip = flat ? "    if (e != only) continue;\n" : "";
+  s << "__device__ __forceinline__ EpiIn epi_load(const Args& ar, i64 pb, i64 qb, int r, int g, int only) {\n  EpiIn z;\n  z.unused = 0;\n";
   if (vec_epi) {
     s << "  i64 p = pb + 4 * g, q = qb + r;\n  p = p > " << sp.P - 4 << "LL ? " << sp.P - 4 << "LL : p;\n  q = q > " << sp.Q - 1 << "LL ? " << sp.Q - 1 << "LL : q;\n";
     for (int i = 0; i < sp.n_in; ++i) {
@@ -292,13 +297,13 @@ std::string generate_body(const Spec& sp) {
     bool any_q = false;
     for (int i = 0; i < sp.n_in; ++i) any_q = any_q || (i != sp.c_slot);
     if (any_q) {
-      s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n";
+      s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n" << skip;
       if (sp.f64) s << "    i64 p = pb + r, q = qb + 4 * e + g;\n";
       else s << "    i64 p = pb + 4 * g + e, q = qb + r;\n";
       s << "    p = p > " << sp.P - 1 << "LL ? " << sp.P - 1 << "LL : p;\n    q = q > " << sp.Q - 1 << "LL ? " << sp.Q - 1 << "LL : q;\n";
       for (int i = 0; i < sp.n_in; ++i) {
         if (i == sp.c_slot) continue;
-        if (sp.in_sp[(size_t)i] == 0 && !sp.f64) s << "    if (e == 0) z.w" << i << " = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
+        if (sp.in_sp[(size_t)i] == 0 && !sp.f64) s << (flat ? "    z.w" : "    if (e == 0) z.w") << i << " = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
         else if (sp.in_sp[(size_t)i] == 0) s << "    z.w" << i << "x[e] = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
         else s << "    z.w" << i << "[e] = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL + p * " << sp.in_sp[(size_t)i] << "LL];\n";
       }
@@ -306,7 +311,7 @@ std::string generate_body(const Spec& sp) {
     }
   }
   s << "  return z;\n}\n";
-  s << "__device__ __forceinline__ void epilogue(const Args& ar, i64 pb, i64 qb, int r, int g, const Acc& c, const EpiIn& z) {\n";
+  s << "__device__ __forceinline__ void epilogue(const Args& ar, i64 pb, i64 qb, int r, int g, const Acc& c, const EpiIn& z, int only) {\n";
   if (vec_epi) {
     // four consecutive p of one q
     s << "  const i64 p = pb + 4 * g, q = qb + r;\n  if (p >= " << sp.P << "LL || q >= " << sp.Q << "LL) return;\n";
@@ -327,7 +332,7 @@ std::string generate_body(const Spec& sp) {
       s << "    *reinterpret_cast<Vec4<" << ct << ">::type*>(ar.o" << o << " + q * " << sp.P << "LL + p) = w;\n  }\n";
     }
   } else {
-    s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n";
+    s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n" << skip;
     if (sp.f64) s << "    const i64 p = pb + r, q = qb + 4 * e + g;\n";
     else s << "    const i64 p = pb + 4 * g + e, q = qb + r;\n";
     s << "    if (p >= " << sp.P << "LL || q >= " << sp.Q << "LL) continue;\n";
@@ -356,7 +361,8 @@ std::string generate_body(const Spec& sp) {
   }
   s << "  const i64 q0 = (blk % " << nbq << "LL) * " << sp.BQ << ", p0 = (blk / " << nbq << "LL) * " << sp.BP << ";\n";
   s << "  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;\n";
-  s << "  const int wp = w % " << sp.WP << ", wq = w / " << sp.WP << ";\n";
+  if (flat) s << "  const int wp = 0, wq = 0, only = w;\n";
+  else s << "  const int wp = w % " << sp.WP << ", wq = w / " << sp.WP << ", only = -1;\n";
   s << "  Acc acc[" << TP << "][" << TQ << "];\n";
   s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b) acc[a][b] = Acc{0, 0, 0, 0};\n";
   const size_t nc = sp.chunks.size();
@@ -371,7 +377,7 @@ std::string generate_body(const Spec& sp) {
   if (n_read > 0) s << "  EpiIn ei[" << TP << "][" << TQ << "];\n";
   auto epi_loads = [&]() {
     s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b)\n";
-    s << "      ei[a][b] = epi_load(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g);\n";
+    s << "      ei[a][b] = epi_load(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, only);\n";
   };
   auto run_chunks = [&](size_t c0, size_t c1) {
     load(c0);
@@ -384,7 +390,31 @@ std::string generate_body(const Spec& sp) {
       if (c + 1 < c1) s << "  __syncthreads();\n";
     }
   };
-  if (S == 1) {
+  if (flat) {
+    // every load of the block goes out at once, each chunk has its own place in LDS, one barrier
+    int xo = 0, yo = 0;
+    std::vector<int> xat, yat;
+    for (size_t c = 0; c < nc; ++c) {
+      load(c);
+      xat.push_back(xo);
+      yat.push_back(yo);
+      xo += tile_elems(sp.chunks[c].x, sp.chunks[c].kcp);
+      yo += tile_elems(sp.chunks[c].y, sp.chunks[c].kcp);
+    }
+    if (prefetch) epi_loads();
+    for (size_t c = 0; c < nc; ++c)
+      s << "  store_x" << c << "(rx" << c << ", xs + " << xat[c] << ", tid);\n  store_y" << c << "(ry" << c << ", ys + " << yat[c] << ", tid);\n";
+    s << "  __syncthreads();\n";
+    for (size_t c = 0; c < nc; ++c) {
+      const Chunk& ch = sp.chunks[c];
+      const int kq = ch.kcp / sp.WK;      // a wavefront's k of this chunk
+      s << "  compute<" << kq << ", " << ch.x.layout << ", " << ch.x.pitch << ", " << ch.y.layout << ", " << ch.y.pitch << ">(xs + " << xat[c] << " + w * "
+        << kq * (ch.x.layout == 0 ? ch.x.pitch : 1) << ", ys + " << yat[c] << " + w * " << kq * (ch.y.layout == 0 ? ch.y.pitch : 1) << ", acc, r, g, wp, wq);\n";
+    }
+    // the quarters meet in LDS (free once every wavefront has read its fragments); wavefront w finishes register w of every lane
+    s << "  __syncthreads();\n#pragma unroll\n  for (int e = 0; e < 4; ++e) lds[(w * 4 + e) * 64 + lane] = acc[0][0][e];\n  __syncthreads();\n";
+    s << "  {\n    const T* q4 = lds + w * 64 + lane;\n    const T t = (q4[0] + q4[256]) + (q4[512] + q4[768]);\n    acc[0][0] = Acc{t, t, t, t};\n  }\n";
+  } else if (S == 1) {
     run_chunks(0, nc);
   } else {
     for (int sp_i = 0; sp_i < S; ++sp_i) {
@@ -405,7 +435,7 @@ std::string generate_body(const Spec& sp) {
     s << "  if (blk >= " << nblk << "LL) return;\n";
     s << "  const i64 q0 = (blk % " << nbq << "LL) * " << sp.BQ << ", p0 = (blk / " << nbq << "LL) * " << sp.BP << ";\n";
     s << "  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;\n";
-    s << "  const int wp = w % " << sp.WP << ", wq = w / " << sp.WP << ";\n";
+    s << "  const int wp = w % " << sp.WP << ", wq = w / " << sp.WP << ", only = -1;\n";
     s << "  Acc acc[" << TP << "][" << TQ << "];\n";
     if (n_read > 0) s << "  EpiIn ei[" << TP << "][" << TQ << "];\n";
     s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b) acc[a][b] = Acc{0, 0, 0, 0};\n";
@@ -415,8 +445,8 @@ std::string generate_body(const Spec& sp) {
   }
   if (n_read > 0 && !prefetch) epi_loads();
   s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b)\n";
-  if (n_read > 0) s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], ei[a][b]);\n";
-  else s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], EpiIn{0});\n";
+  if (n_read > 0) s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], ei[a][b], only);\n";
+  else s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], EpiIn{0}, only);\n";
   s << "}\n";
   return s.str();
 }
@@ -484,6 +514,26 @@ void choose_tile(hgpu_ctx* ctx, Spec& sp, int64_t ktot) {
   }
 }
 
+// Few rows (a minibatch of 150 through a recurrence of width 128: 20 tiles of 32 x 32 on 256 CUs): what a launch
+// takes is the chain load, store to LDS, multiply, repeated per chunk, and the 64 dependent MFMAs of a wavefront that
+// walks all of K alone.  So each block takes a 16 x 16 tile, loads both operands whole at once, its four wavefronts
+// multiply a quarter of K each, and their sums meet in LDS.  Gradient of a two-layer recurrence of width 128, 28
+// steps, batch 150, fp64: 537 -> 402 us.  Taken while the tiles find a CU each and two blocks fit a CU; beyond, the
+// larger tiles read each operand element less often and win again (14 steps, us, larger tiles / these: fp64 batch 300
+// 350 / 305, 600 382 / 384, 900 370 / 401; fp32 150 268 / 234, 300 278 / 265, 600 283 / 291, 1000 259 / 279).
+bool choose_flat(hgpu_ctx* ctx, Spec& sp) {
+  static const bool off = getenv("HORDEAD_SMALLK_NOFLAT") != nullptr;    // for measurements
+  const int64_t tiles = ((sp.P + 15) / 16) * ((sp.Q + 15) / 16);
+  if (off || tiles > ctx->num_cu) return false;
+  int64_t kpad = 0;
+  for (const Term& t : sp.terms) kpad += (t.K + 15) / 16 * 16 + 8;
+  if (kpad * 32 * (sp.f64 ? 8 : 4) > 80 * 1024) return false;
+  sp.BP = sp.BQ = 16;
+  sp.WP = sp.WQ = 1;
+  sp.WK = 4;
+  return true;
+}
+
 // Cuts the contracted dims of the terms into chunks and lays their tiles out in LDS.
 bool plan_chunks(Spec& sp) {
   // K elements per chunk: 64 (the recurrent layer's grouped step products, fp32, K 28 + 128 and 128 + 128: the
@@ -495,6 +545,23 @@ bool plan_chunks(Spec& sp) {
   }
   sp.x_elems = sp.y_elems = 0;
   sp.chunks.clear();
+  if (sp.WK > 1) {           // one chunk per term, all of them in LDS together
+    for (int t = 0; t < (int)sp.terms.size(); ++t) {
+      const Term& tm = sp.terms[(size_t)t];
+      Chunk c;
+      c.term = t;
+      c.k0 = 0;
+      c.kc = (int)tm.K;
+      c.kcp = (c.kc + 4 * sp.WK - 1) / (4 * sp.WK) * (4 * sp.WK);
+      c.x = make_operand(sp.f64, sp.BP, sp.P, tm.sxp, tm.sxk, c.kc, c.kcp);
+      c.y = make_operand(sp.f64, sp.BQ, sp.Q, tm.syq, tm.syk, c.kc, c.kcp);
+      sp.x_elems += tile_elems(c.x, c.kcp);
+      sp.y_elems += tile_elems(c.y, c.kcp);
+      sp.chunks.push_back(c);
+    }
+    sp.x_elems = (std::max(sp.x_elems, 1024) + 3) / 4 * 4;      // (the exchange of the quarters: 4 x 256 elements)
+    return true;
+  }
   for (int t = 0; t < (int)sp.terms.size(); ++t) {
     const Term& tm = sp.terms[(size_t)t];
     int n = (int)((tm.K + kcmax - 1) / kcmax);
@@ -519,7 +586,7 @@ bool plan_chunks(Spec& sp) {
 }
 
 // Everything generate_body reads.
-static_assert(sizeof(Spec) == 224 && sizeof(Chunk) == 96 && sizeof(Term) == 56, "spec_key must cover every field of Spec, Chunk, Operand and Term");
+static_assert(sizeof(Spec) == 232 && sizeof(Chunk) == 96 && sizeof(Term) == 56, "spec_key must cover every field of Spec, Chunk, Operand and Term");
 Key spec_key(const Spec& sp) {
   Key k;
   k.put(sp.f64).put(sp.P).put(sp.Q).put(sp.BP).put(sp.BQ).put(sp.WP).put(sp.WQ).put(sp.terms.size());
@@ -530,7 +597,7 @@ Key spec_key(const Spec& sp) {
     for (const Operand* o : {&c.x, &c.y}) k.put(o->rows).put(o->layout).put(o->V).put(o->pitch).put(o->sr).put(o->sk).put(o->extent);
   }
   k.put(sp.n_in).put(sp.c_slot).put(sp.n_instr, sp.prog).put(sp.dt).put(sp.in_sp).put(sp.in_sq).put(sp.out_slots);
-  k.put(sp.x_elems).put(sp.y_elems).put(sp.splits).put(sp.chunks_per_split);
+  k.put(sp.x_elems).put(sp.y_elems).put(sp.splits).put(sp.chunks_per_split).put(sp.WK);
   return k;
 }
 
@@ -697,7 +764,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     if (!fits_int(sp.in_sp[(size_t)i] * sp.P) || !fits_int(sp.in_sq[(size_t)i] * sp.Q)) return HGPU_OK;
   }
   sp.out_slots.assign(out_slots, out_slots + n_out);
-  choose_tile(ctx, sp, ktot);
+  if (!choose_flat(ctx, sp)) choose_tile(ctx, sp, ktot);
   if (!plan_chunks(sp)) return HGPU_OK;
   const int64_t ntiles = ((sp.P + sp.BP - 1) / sp.BP) * ((sp.Q + sp.BQ - 1) / sp.BQ);
   {
