@@ -250,16 +250,18 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
     }
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
     // an operand contiguous along K is read four elements at a time
-    auto k_vector = [&](const void* base, const int64_t* ks, const int64_t* rs, const Group& rows, const int64_t* bs) {
+    auto k_vector = [&](const void* base, const void* const* terms, const int64_t* ks, const int64_t* rs, const Group& rows, const int64_t* bs) {
       const int64_t v = (int64_t)(16 / es);
       const int kd = p.k.nd - 1;
+      for (int t = 0; t < n_terms; ++t)
+        if (((uintptr_t)terms[t] & 15) != 0) return false;
       if (((uintptr_t)base & 15) != 0 || p.K < 16 || ks[kd] != 1 || p.k.shape[kd] % 4 != 0) return false;
       for (int i = 0; i < kd; ++i) if (ks[i] % v != 0) return false;
       for (int i = 0; i < rows.nd; ++i) if (rs[i] % v != 0) return false;
       for (int i = 0; i < p.bt.nd; ++i) if (bs[i] % v != 0) return false;
       return true;
     };
-    const bool va = k_vector(pa, p.k.sa, p.m.sa, p.m, p.bt.sa), vb = k_vector(pb, p.k.sb, p.n.sb, p.n, p.bt.sb);
+    const bool va = k_vector(pa, p.a_term, p.k.sa, p.m.sa, p.m, p.bt.sa), vb = k_vector(pb, p.b_term, p.k.sb, p.n.sb, p.n, p.bt.sb);
     LaunchArgs la{ctx->stream, -1, tm, tn, va, vb, grid, pa, pb, cdst, ka, kb};
     {
       LaunchGuard lg(ctx, label, bytes, flops);
@@ -491,7 +493,9 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
   // Worth the matrix cores only when there is reuse on both sides.
   if (p.K < 4 || p.M * p.N < 256) return HGPU_OK;
   if (p.BT > 65535) return HGPU_OK;
-  if ((double)p.M * p.N * p.K * p.BT < 2.0e6) return HGPU_OK;
+  // (all terms of a sum together: 28 products of 128 x 28 over 150, a minibatch's input weight gradient, ran as one
+  // reduction per output, 58 us; the recurrent network at that batch, fp64: 402 -> 373 us)
+  if ((double)p.M * p.N * p.K * p.BT * (n_terms > 0 ? n_terms : 1) < 2.0e6) return HGPU_OK;
   // a thousand outputs under a long K (the last layer's weight gradient: 100 x 10
   // over 5000): the split-K kernels have a handful of wavefronts to work with,
   // a wavefront per output in the reduction kernels has a thousand
