@@ -284,11 +284,13 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
   return HGPU_OK;
 }
 
-// Large fp32 products on the bf16 matrix cores (gemm_split.hip).  Takes products whose row, column, contracted and
-// batch indices are single dims with strides that a 32-bit byte offset reaches.
-int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out) {
+// Products whose row, column, contracted and batch indices are single dims with strides that a 32-bit byte offset
+// reaches: fp32 on the bf16 matrix cores (gemm_split.hip), fp64 in tiles without address arithmetic (gemm_wide_f64.hip).
+int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out) {
   if (p.m.nd != 1 || p.n.nd != 1 || p.k.nd != 1 || p.bt.nd != 1) return HGPU_OK;
   const int64_t nt = n_terms > 0 ? n_terms : 1;
+  const bool f64 = dtype == HGPU_F64;
+  const int64_t es = f64 ? 8 : 4;
   SplitParams q{};
   int64_t sam = p.m.sa[0], sak = p.k.sa[0], sbn = p.n.sb[0], sbk = p.k.sb[0], scm = p.m.sc[0], scn = p.n.sc[0], M = p.M, N = p.N;
   int64_t bsa = p.bt.sa[0], bsb = p.bt.sb[0];
@@ -301,15 +303,15 @@ int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* p
     std::swap(bsa, bsb);
   }
   if (sam < 0 || sak < 0 || sbn < 0 || sbk < 0 || p.K > (1 << 24)) return HGPU_OK;
-  const int64_t a_bytes = ((M - 1) * sam + (p.K - 1) * sak + 1) * 4, b_bytes = ((N - 1) * sbn + (p.K - 1) * sbk + 1) * 4;
+  const int64_t a_bytes = ((M - 1) * sam + (p.K - 1) * sak + 1) * es, b_bytes = ((N - 1) * sbn + (p.K - 1) * sbk + 1) * es;
   if (a_bytes > 0x7fffff00 || b_bytes > 0x7fffff00 || M > 0x3fffffff || N > 0x3fffffff) return HGPU_OK;
   q.M = (int)M;
   q.N = (int)N;
   q.K = (int)p.K;
-  q.sam = (uint32_t)(sam * 4);
-  q.sak = (uint32_t)(sak * 4);
-  q.sbn = (uint32_t)(sbn * 4);
-  q.sbk = (uint32_t)(sbk * 4);
+  q.sam = (uint32_t)(sam * es);
+  q.sak = (uint32_t)(sak * es);
+  q.sbn = (uint32_t)(sbn * es);
+  q.sbk = (uint32_t)(sbk * es);
   q.scm = scm;
   q.scn = scn;
   q.bsa = bsa;
@@ -319,12 +321,24 @@ int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* p
   q.b_bytes = (uint32_t)b_bytes;
   q.n_terms = n_terms;
   for (int t = 0; t < n_terms; ++t) {
-    q.a_term[t] = (const float*)(swap ? p.b_term[t] : p.a_term[t]);
-    q.b_term[t] = (const float*)(swap ? p.a_term[t] : p.b_term[t]);
+    q.a_term[t] = swap ? p.b_term[t] : p.a_term[t];
+    q.b_term[t] = swap ? p.a_term[t] : p.b_term[t];
   }
   const int64_t out_n = nelem(out);
   int cfg = 0, split = 1;
-  {
+  if (f64) {
+    // Microseconds, as measured: a step of 16 k of a 64 x 64 tile takes 0.62 alone on its CU, 0.56 with another one
+    // there, 0.5 with more; 5 for the launch; partial results as below.  (300 x 784 over 5000, main kernel / with the
+    // sums: 4 chunks = 260 blocks 82 / 89, 7 = 455 56 / 63, 10 = 650 54 / 63, 32 = 2080 52 / 65.)
+    double best = 1e300;
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64) * p.BT * nt;
+    for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
+      const int64_t per_cu = (tiles * sp + ctx->num_cu - 1) / ctx->num_cu, steps = ((p.K + sp - 1) / sp + 15) / 16;
+      const double step = per_cu == 1 ? 0.62 : per_cu == 2 ? 1.12 : 0.5 * per_cu;
+      const double us = 5 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 8 / 6e6 : 0);
+      if (us < best) { best = us; split = (int)sp; }
+    }
+  } else {
     // Microseconds, as measured: a step of 16 k of a 256 x 256 tile (one block on a CU) 3.4, of a 128 x 128 tile
     // 1.4 alone on its CU and 0.92 for each of several; 8 for the launch with its first loads and last stores; for
     // partial results a second launch and their bytes once out and once in.  (2048 x 8192 over 2048: 395-425 us
@@ -341,7 +355,7 @@ int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* p
       }
     }
   }
-  const int64_t BM = cfg == 0 ? 256 : 128, BN = BM;
+  const int64_t BM = f64 ? 64 : (cfg == 0 ? 256 : 128), BN = BM;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   q.kchunk = (int)(((p.K + split - 1) / split + 15) / 16 * 16);
   q.term_split = (int)((p.K + q.kchunk - 1) / q.kchunk);
@@ -349,20 +363,20 @@ int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* p
   if (split > 65535 || tiles * split > 0x3fffffff || (split > 1 && (double)out_n * split > 5e8)) return HGPU_OK;
   hgpu_buffer* part = nullptr;
   if (split > 1) {
-    int rc = buffer_alloc(ctx, (size_t)out_n * split * 4, &part);
+    int rc = buffer_alloc(ctx, (size_t)(out_n * split * es), &part);
     if (rc) return rc;
   }
   q.c_split_stride = split > 1 ? out_n : 0;
   {
     const double flops = 2.0 * M * N * p.K * p.BT * nt;
-    const double bytes = (((double)M * p.K + (double)N * p.K) * nt + (double)M * N) * p.BT * 4;
-    const char* label = "gemm_f32";
+    const double bytes = (((double)M * p.K + (double)N * p.K) * nt + (double)M * N) * p.BT * es;
+    const char* label = f64 ? "gemm_f64" : "gemm_f32";
     if (ctx->profiling && ctx->profile_shapes) {
       char buf[128];
       char terms[24] = "";
       if (nt > 1) snprintf(terms, sizeof terms, ",terms%lld", (long long)nt);
-      snprintf(buf, sizeof buf, "%s[M%lldxN%lldxK%lldxB%lld,s%d,%s%s,split3,t%lldx%lld%s]", label, (long long)M, (long long)N, (long long)p.K, (long long)p.BT, split,
-               sak == 1 ? "K" : "M", sbk == 1 ? "K" : "N", (long long)BM, (long long)BN, terms);
+      snprintf(buf, sizeof buf, "%s[M%lldxN%lldxK%lldxB%lld,s%d,%s%s,%s,t%lldx%lld%s]", label, (long long)M, (long long)N, (long long)p.K, (long long)p.BT, split,
+               sak == 1 ? "K" : "M", sbk == 1 ? "K" : "N", f64 ? "wide" : "split3", (long long)BM, (long long)BN, terms);
       label = intern_label(ctx, buf);
     }
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
@@ -371,17 +385,19 @@ int gemm_split(hgpu_ctx* ctx, const GemmParams& p, const void* pa, const void* p
       LaunchGuard lg(ctx, label, bytes, flops);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
-      launch_split_f32(q, la);
+      if (f64) launch_wide_f64(q, la);
+      else launch_split_f32(q, la);
     }
     if (split > 1 && partials_out && split <= 3 && is_dense(out)) {
       int64_t sh[HGPU_MAX_RANK + 1], st[HGPU_MAX_RANK + 1];
       sh[0] = split;
       for (int d = 0; d < out->rank; ++d) sh[d + 1] = out->shape[d];
       dense_strides(out->rank + 1, sh, st);
-      *partials_out = new_view(ctx, part, HGPU_F32, out->rank + 1, sh, st, 0);
+      *partials_out = new_view(ctx, part, dtype, out->rank + 1, sh, st, 0);
     } else if (split > 1) {
-      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * 4, (double)out_n * split);
-      launch_sum_partials<float>(ctx, out_n, split, (const float*)part->ptr, (float*)data_ptr(out));
+      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * es, (double)out_n * split);
+      if (f64) launch_sum_partials<double>(ctx, out_n, split, (const double*)part->ptr, (double*)data_ptr(out));
+      else launch_sum_partials<float>(ctx, out_n, split, (const float*)part->ptr, (float*)data_ptr(out));
     }
   }
   const hipError_t e = hipGetLastError();
@@ -514,6 +530,16 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     int rc = try_footprint(ctx, p, a->dtype, pa, pb, out, handled);
     if (rc || *handled) return rc;
   }
+  // (a side under 96 leaves more than a quarter of a 128-wide tile empty: the smaller tiles of the fp32 instruction; fp64: a side under 64)
+  const bool tiled = (a->dtype == HGPU_F32 ? p.M >= 96 && p.N >= 96 : p.M >= 64 && p.N >= 64) && p.K >= 64;
+  // fp64 with four 64 x 64 tiles for every CU: those run faster than the kernel over a short K, which is at its best with
+  // few tiles or a program over the result (1024 x 4096 over 128 / 256 / 500: 25.6 / 42.8 / 79 us against 28.9 / 48.8 / 91;
+  // 700 x 300 over 500: 18.0 against 10.2)
+  const bool early = tiled && a->dtype == HGPU_F64 && ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.BT >= 4 * (int64_t)ctx->num_cu;
+  if (early) {
+    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out);
+    if (rc || *handled) return rc;
+  }
   if ((p.K <= 512 || (p.K <= 1024 && p.M * p.N <= 160000)) && p.BT == 1) {   // the whole contracted dim in LDS: no K loop, no K table
     const hgpu_array* const* ta = n_terms > 0 ? as : &a;
     const hgpu_array* const* tb = n_terms > 0 ? bs : &b;
@@ -522,14 +548,13 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     int rc = try_smallk(ctx, n_terms > 0 ? n_terms : 1, ta, tb, n_keep, 1, &none, 0, 0, nullptr, std::vector<int>{a->dtype}, 1, &slot, &out, handled);
     if (rc || *handled) return rc;
   }
-  // (a side under 96 leaves more than a quarter of a 128-wide tile empty: the smaller tiles of the fp32 instruction)
-  if (a->dtype == HGPU_F32 && p.M >= 96 && p.N >= 96 && p.K >= 64) {
-    int rc = gemm_split(ctx, p, pa, pb, out, handled, n_terms, partials_out);
+  if (tiled && !early) {
+    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out);
     if (rc || *handled) return rc;
   }
   // (under a long K the staged kernel's coalesced tile loads win even with most of a 32-wide tile empty: the recurrent network's
   // input weight gradient, 128 x 28 over 28 x 5000, 52 -> 45 us)
-  if ((p.M <= 32 || p.N <= 32) && p.M <= 1024 && p.N <= 1024 && p.K < 4096) return gemm_direct(ctx, p, a->dtype, pa, pb, out, handled, n_terms);
+  if ((p.M <= 32 || p.N <= 32) && p.M <= 1024 && p.N <= 1024 && p.K * (n_terms > 0 ? n_terms : 1) < 4096) return gemm_direct(ctx, p, a->dtype, pa, pb, out, handled, n_terms);
 
   const int64_t nt = n_terms > 0 ? n_terms : 1;      // products summed by this launch
   const int64_t out_elems = p.M * p.N * p.BT;

@@ -775,7 +775,7 @@ void launch(const GemmParams& p, const LaunchArgs& a) {
 }
 
 // Products whose rows, columns, contracted and batch dims are single dims with non-negative strides
-// (gemm_split.hip).  Strides of the operands in bytes, of the result in elements.
+// (gemm_split.hip, gemm_wide_f64.hip).  Strides of the operands in bytes, of the result in elements.
 struct SplitParams {
   int M, N, K;
   uint32_t sam, sak, sbn, sbk;
@@ -785,9 +785,10 @@ struct SplitParams {
   int kchunk;
   int64_t c_split_stride;
   int n_terms, term_split;
-  const float* a_term[kMaxTerms];
-  const float* b_term[kMaxTerms];
+  const void* a_term[kMaxTerms];
+  const void* b_term[kMaxTerms];
 };
+void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a);
 
 // defined in gemm_f32.hip / gemm_f64.hip

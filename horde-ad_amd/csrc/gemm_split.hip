@@ -165,8 +165,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   if (p.n_terms > 0) {
     const int term = s / p.term_split;
     sk = s - term * p.term_split;
-    A = p.a_term[term];
-    B = p.b_term[term];
+    A = (const float*)p.a_term[term];
+    B = (const float*)p.b_term[term];
   }
   A += (int64_t)blockIdx.z * p.bsa;
   B += (int64_t)blockIdx.z * p.bsb;

@@ -1,0 +1,239 @@
+// fp64 matrix products whose operands are addressed by one stride per index (SplitParams).
+//
+// What bounds it: v_mfma_f64_16x16x4_f64 does not run beside other vector instructions.  A loop of nothing else
+// reaches 55-60 TFLOP/s with one wavefront per SIMD (84 cycles per instruction instead of 64), 65-67 with two to four,
+// and two integer instructions per MFMA take 67 down to 58.  So the K loop here has no vector instructions besides
+// MFMAs and memory operations -- loads go through a buffer descriptor with a fixed offset per lane and a scalar one
+// for the step, LDS addresses are fixed registers plus immediates -- and the tiles leave two to three blocks to a CU.
+//
+// A tile of an operand stands in LDS as [row][16 k], 16-byte pieces of two k; a lane's fragment of one read serves
+// two MFMAs (any assignment of k to the steps will do as long as A and B agree).  Piece c of row r sits at position
+// c ^ (r / 2 % 8), so that the 16 rows of a fragment read hit 64 different banks without padding.
+#include "gemm_kernel.hpp"
+
+using namespace hg;
+using namespace hg::gemm;
+
+namespace {
+
+using d2 = double __attribute__((ext_vector_type(2)));
+using u2 = uint32_t __attribute__((ext_vector_type(2)));
+using u4 = uint32_t __attribute__((ext_vector_type(4)));
+using Acc = MfmaF64::Acc;
+
+constexpr int SK = 16;                      // k of one step
+
+__device__ __forceinline__ int lds_at(int r, int c) { return r * 8 + (c ^ ((r >> 1) & 7)); }
+
+// One operand's share of a tile: ROWS rows of SK elements, a lane owns NS pieces of two k.
+template <int ROWS, bool KC>
+struct Side {
+  static constexpr int NS = ROWS * 8 / NT;
+  static_assert(NS * NT == ROWS * 8, "whole pieces");
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off[NS];                         // bytes
+  int at[NS];
+  uint32_t ks;                              // bytes between neighbouring k
+
+  __device__ __forceinline__ static int row(int t, int i) { return KC ? (t + i * NT) / 8 : (t + i * NT) % ROWS; }
+  __device__ __forceinline__ static int piece(int t, int i) { return KC ? (t + i * NT) % 8 : (t + i * NT) / ROWS; }
+
+  __device__ __forceinline__ void init(int t, const double* base, uint32_t bytes, uint32_t rs, int r0, int rows, uint32_t stride) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00027000);
+    ks = stride;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int r = row(t, i), c = piece(t, i);
+      off[i] = (uint32_t)(r0 + r < rows ? r0 + r : rows - 1) * rs + 2 * c * ks;      // (rows past the end: never stored)
+      at[i] = lds_at(r, c);
+    }
+  }
+  __device__ __forceinline__ static u4 both(u2 a, u2 b) { return u4{a[0], a[1], b[0], b[1]}; }
+  // A whole step that starts at k0.
+  __device__ __forceinline__ void load(int k0, u4* s) const {
+    const uint32_t so = (uint32_t)k0 * ks;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      if constexpr (KC) s[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[i], so, 0));
+      else
+        s[i] = both(__builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off[i], so, 0)),
+                    __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off[i], so + ks, 0)));
+    }
+  }
+  // The last step of a chunk when it is not a whole one: `left` elements of k, zeros behind them.
+  __device__ __forceinline__ void load_tail(int t, int k0, int left, u4* s) const {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int k = 2 * piece(t, i);
+      u2 v[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        v[j] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, k + j < left ? off[i] + (k0 + j) * ks : 0xfffffff0u, 0, 0));
+      s[i] = both(v[0], v[1]);
+    }
+  }
+  __device__ __forceinline__ void store(const u4* s, u4* tile) const {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) tile[at[i]] = s[i];
+  }
+};
+
+// AKC, BKC: the operand is contiguous along k (lanes stage 16 bytes of a row; otherwise a row each, 8 bytes of two k).
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C) {
+  constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 16 x 16 blocks of each
+  constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
+  __shared__ u4 lds[2][(BM + BN) * 8];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+
+  // each XCD works on a contiguous range of (K chunk, tile) pairs, as in k_gemm
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  const int ntiles = tiles_m * tiles_n;
+  const int nblocks = ntiles * gridDim.y;
+  int lin = blockIdx.x + ntiles * blockIdx.y;
+  if (nblocks >= 64) {
+    const int x = lin & 7, per = nblocks >> 3, rem = nblocks & 7;
+    lin = x * per + (x < rem ? x : rem) + (lin >> 3);
+  }
+  const int s = lin / ntiles, bid = lin - s * ntiles;
+  // tiles in bands of eight rows of tiles: neighbours in the order share operands
+  const int band = bid / (8 * tiles_n), in_band = bid - band * 8 * tiles_n;
+  const int rows_in_band = tiles_m - band * 8 < 8 ? tiles_m - band * 8 : 8;
+  const int tile_n = in_band / rows_in_band, tile_m = band * 8 + (in_band - tile_n * rows_in_band);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+  int sk = s;
+  if (p.n_terms > 0) {
+    const int term = s / p.term_split;
+    sk = s - term * p.term_split;
+    A = (const double*)p.a_term[term];
+    B = (const double*)p.b_term[term];
+  }
+  A += (int64_t)blockIdx.z * p.bsa;
+  B += (int64_t)blockIdx.z * p.bsb;
+  const int kbeg = sk * p.kchunk;
+  const int kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
+
+  Side<BM, AKC> sa;
+  Side<BN, BKC> sb;
+  sa.init(t, A, p.a_bytes, p.sam, m0, p.M, p.sak);
+  sb.init(t, B, p.b_bytes, p.sbn, n0, p.N, p.sbk);
+  constexpr int NA = Side<BM, AKC>::NS, NB = Side<BN, BKC>::NS;
+
+  Acc acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = MfmaF64::zero();
+
+  const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
+  u4 ra[NA], rb[NB];
+  auto fetch = [&](int i) {
+    sa.load(kbeg + i * SK, ra);
+    sb.load(kbeg + i * SK, rb);
+  };
+  auto fetch_tail = [&](int i) {
+    sa.load_tail(t, kbeg + i * SK, kend - kbeg - i * SK, ra);
+    sb.load_tail(t, kbeg + i * SK, kend - kbeg - i * SK, rb);
+  };
+  if (whole > 0) fetch(0);
+  else fetch_tail(0);
+  sa.store(ra, lds[0]);
+  sb.store(rb, lds[0] + BM * 8);
+  __syncthreads();
+
+  // where the lane's fragments of the two halves of a step start
+  const int r = lane & 15, q = lane >> 4;
+  int fa[2], fb[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    fa[h] = lds_at(wm * TM * 16 + r, 4 * h + q);
+    fb[h] = BM * 8 + lds_at(wn * TN * 16 + r, 4 * h + q);
+  }
+  // One step on buffer `cur`.  next: 0 = there is none behind it, 1 = a whole step, 2 = the rest of K.
+  auto step = [&](int i0, auto buffer, auto next) {
+    constexpr int cur = decltype(buffer)::value;
+    if constexpr (decltype(next)::value == 1) fetch(i0 + 1);
+    if constexpr (decltype(next)::value == 2) fetch_tail(i0 + 1);
+    __builtin_amdgcn_sched_barrier(0);      // (left to itself the compiler moves the loads down to their use)
+    d2 a[2][TM], b[2][TN];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[h][i] = __builtin_bit_cast(d2, lds[cur][fa[h] + i * 128]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[h][j] = __builtin_bit_cast(d2, lds[cur][fb[h] + j * 128]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = MfmaF64::run(a[h][i][u], b[h][j][u], acc[i][j]);
+    if constexpr (decltype(next)::value != 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      sa.store(ra, lds[cur ^ 1]);
+      sb.store(rb, lds[cur ^ 1] + BM * 8);
+    }
+    __syncthreads();
+  };
+  constexpr std::integral_constant<int, 0> b0{};
+  constexpr std::integral_constant<int, 1> b1{};
+  constexpr std::integral_constant<int, 2> rest{};
+  int i0 = 0;
+#pragma unroll 1
+  for (; i0 + 2 < whole; i0 += 2) {
+    step(i0, b0, b1);
+    step(i0 + 1, b1, b1);
+  }
+  // up to two whole steps and a last one that is not whole are left; i0 is even
+  if (i0 + 1 < whole) {
+    step(i0, b0, b1);
+    if (i0 + 2 < steps) {
+      step(i0 + 1, b1, rest);
+      step(i0 + 2, b0, b0);
+    } else {
+      step(i0 + 1, b1, b0);
+    }
+  } else if (i0 + 1 < steps) {
+    step(i0, b0, rest);
+    step(i0 + 1, b1, b0);
+  } else {
+    step(i0, b0, b0);
+  }
+
+  double* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)s * p.c_split_stride;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + (wn * TN + j) * 16 + MfmaF64::col(lane);
+    if (n >= p.N) continue;
+    double* col = Cout + (int64_t)n * p.scn;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + (wm * TM + i) * 16 + MfmaF64::row(lane, e);
+        if (m < p.M) col[(int64_t)m * p.scm] = acc[i][j][e];
+      }
+  }
+}
+
+}  // namespace
+
+namespace hg {
+namespace gemm {
+
+void launch_wide_f64(const SplitParams& p, const LaunchArgs& a) {
+  const double *A = (const double*)a.A, *B = (const double*)a.B;
+  double* C = (double*)a.C;
+  if (a.va && a.vb) launch_kernel(a, k_gemm_wide_f64<true, true>, p, A, B, C);
+  else if (a.va) launch_kernel(a, k_gemm_wide_f64<true, false>, p, A, B, C);
+  else if (a.vb) launch_kernel(a, k_gemm_wide_f64<false, true>, p, A, B, C);
+  else launch_kernel(a, k_gemm_wide_f64<false, false>, p, A, B, C);
+}
+
+}  // namespace gemm
+}  // namespace hg
