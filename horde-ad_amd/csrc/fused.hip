@@ -627,9 +627,52 @@ extern "C" int hgpu_fused_extremum(hgpu_ctx* ctx, int n_in, const hgpu_array* co
   return HGPU_OK;
 }
 
+// How a grid's blocks hand their partial sums to the one that finishes last.  A release fence before the ticket would
+// write the block's share of the outputs back out of its XCD's L2 and wait for it (16.8 M elements with three outputs:
+// 0.42 ms).  Only the sums have to be seen by another block, so they travel by atomics of device scope alone, which do
+// not stay in an L2: a sum is exchanged in, the returned old value says that it has arrived, and only then is the ticket
+// drawn.  Whoever draws the last one reads all of them with atomic loads, a batch in flight, always in the same order.
+// The counters are 17, the root one drawn from by the last block of each of 16: a thousand blocks on one address took
+// 10 ns apiece (1003 x 1021 fp32, three outputs: 22.3 us).  Gradient of the elementwise objective, us, a release fence
+// per block up to 131072 elements and a second launch beyond / this: 300 x 300 fp64 16.8 / 13.2, 1003 x 1021 fp32
+// 17.4 / 13.7, 2000 x 2000 fp32 27.4 / 25.5, 4096 x 4096 fp64 171.8 / 166.6.
+static const char* const kHandOver = R"HG(
+__device__ __forceinline__ void hand_over(unsigned long long* at, unsigned long long v) {
+  const unsigned long long old = __hip_atomic_exchange(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("" :: "v"(old) : "memory");    // a use of the returned value: nothing below starts before it is there
+}
+__device__ __forceinline__ bool last_of(unsigned* ticket, unsigned n) {
+  if (__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return false;
+  __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+  return true;
+}
+// 16 counters on cache lines of their own, and one that the last block of each draws from
+__device__ __forceinline__ bool last_block(unsigned* tickets) {
+  const unsigned n = gridDim.x, c = blockIdx.x & 15;
+  return last_of(tickets + 32 * (c + 1), (n - c + 15) / 16) && last_of(tickets, n < 16 ? n : 16);
+}
+template <typename A> __device__ __forceinline__ A sum_of_blocks(unsigned long long* part) {
+  asm volatile("" ::: "memory");
+  A acc = 0;
+  const int g = (int)gridDim.x;
+  for (int i0 = threadIdx.x; i0 < g; i0 += 8 * 256) {
+    unsigned long long u[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = i0 + q * 256;
+      u[q] = __hip_atomic_load(part + (i < g ? i : g - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (i0 + q * 256 < g) acc += *reinterpret_cast<A*>(&u[q]);
+  }
+  return acc;
+}
+)HG";
+
 // The sum of all elements of an elementwise program's result, evaluated on the
 // fly (the result is never written): per-block partial sums in double / int64,
-// added up in a fixed order by a second, one-block launch.  Inputs must be dense
+// added up in a fixed order by the block that finishes last.  Inputs must be dense
 // (16-byte aligned) or one broadcast element; anything else is left to the
 // caller (HGPU_ERR_UNSUPPORTED), who writes the result out and sums that.
 extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, int slot,
@@ -675,11 +718,9 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
     if (rc) { hgpu_release(o); return rc; }
   }
   auto drop_part = [&] { if (part) buffer_release(part); };
-  // Up to 131072 elements (at most a few hundred blocks) the block that finishes last adds the blocks' sums up; beyond, a second launch does
-  // (handing a sum over takes a fence per block, and the thousands of blocks of a large array would each pay it).
-  const bool ticketed = !single && n <= (1 << 17);
+  // The block that finishes last adds the blocks' sums up (hand_over).
   void* ticket = nullptr;
-  if (ticketed) {
+  if (!single) {
     rc = ticket_block(ctx, &ticket);
     if (rc) { drop_part(); hgpu_release(o); return rc; }
   }
@@ -692,6 +733,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   s << kPrelude;
   s << "template <typename T, int N> struct alignas(sizeof(T) * N) Vec { T v[N]; };\n";
   s << "typedef " << acc << " ACC;\n";
+  if (!single) s << kHandOver;
   s << "__device__ __forceinline__ ACC wave_sum(ACC v) {\n"
        "  for (int off = 32; off > 0; off >>= 1) {\n"
        "    unsigned long long u = *reinterpret_cast<unsigned long long*>(&v);\n"
@@ -702,8 +744,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   s << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") fused_sum(i64 n";
   for (int i = 0; i < n_in; ++i) s << ", const " << ctype(in[i]->dtype) << "* __restrict__ i" << i;
   if (single) s << ", " << ctype(odt) << "* __restrict__ out) {\n";
-  else if (ticketed) s << ", unsigned long long* part, unsigned int* ticket, " << ctype(odt) << "* __restrict__ out) {\n";
-  else s << ", ACC* __restrict__ part) {\n";
+  else s << ", unsigned long long* part, unsigned int* ticket, " << ctype(odt) << "* __restrict__ out) {\n";
   s << "  __shared__ ACC red[" << NT / 64 << "];\n";
   s << "  const i64 step = (i64)gridDim.x * " << NT << ";\n";
   for (int i = 0; i < n_in; ++i)
@@ -738,37 +779,19 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   s << "  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n";
   s << "  __syncthreads();\n";
   if (single) s << "  if (threadIdx.x == 0) {\n    ACC tot = 0;\n    for (int k = 0; k < " << NT / 64 << "; ++k) tot += red[k];\n    out[0] = (" << ctype(odt) << ")tot;\n  }\n";
-  else if (!ticketed) s << "  if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);\n";
   else {
-    // The block that finishes last adds the blocks' sums up, always in the same order, and writes the result:
-    // every block hands its sum over (store, fence, ticket), the last one to draw a ticket sees them all.
     s << "  __shared__ int last;\n";
     s << "  if (threadIdx.x == 0) {\n    ACC tot = (red[0] + red[1]) + (red[2] + red[3]);\n";
-    s << "    __hip_atomic_store(part + blockIdx.x, *reinterpret_cast<unsigned long long*>(&tot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n";
-    s << "    __threadfence();\n    last = atomicAdd(ticket, 1u) == gridDim.x - 1;\n  }\n";
-    s << "  __syncthreads();\n  if (!last) return;\n  __threadfence();\n";
-    s << "  acc = 0;\n";
-    s << "  for (int i = threadIdx.x; i < (int)gridDim.x; i += 256) {\n";
-    s << "    unsigned long long u = __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n    acc += *reinterpret_cast<ACC*>(&u);\n  }\n";
+    s << "    hand_over(part + blockIdx.x, *reinterpret_cast<unsigned long long*>(&tot));\n";
+    s << "    last = last_block(ticket);\n  }\n";
+    s << "  __syncthreads();\n  if (!last) return;\n";
+    s << "  acc = sum_of_blocks<ACC>(part);\n";
     s << "  acc = wave_sum(acc);\n";
     s << "  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n";
     s << "  __syncthreads();\n";
-    s << "  if (threadIdx.x == 0) {\n    out[0] = (" << ctype(odt) << ")((red[0] + red[1]) + (red[2] + red[3]));\n";
-    s << "    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch\n  }\n";
+    s << "  if (threadIdx.x == 0) {\n    out[0] = (" << ctype(odt) << ")((red[0] + red[1]) + (red[2] + red[3]));\n  }\n";
   }
   s << "}\n";
-  if (!single && !ticketed) {
-    // second launch: one block adds the partial sums up, in the same order
-    s << "extern \"C\" __global__ void __launch_bounds__(256) fused_sum_final(int g, const ACC* __restrict__ part, " << ctype(odt) << "* __restrict__ out) {\n";
-    s << "  __shared__ ACC red[4];\n";
-    s << "  ACC acc = 0;\n";
-    s << "  for (int i = threadIdx.x; i < g; i += 256) acc += part[i];\n";
-    s << "  acc = wave_sum(acc);\n";
-    s << "  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n";
-    s << "  __syncthreads();\n";
-    s << "  if (threadIdx.x == 0) out[0] = (" << ctype(odt) << ")((red[0] + red[1]) + (red[2] + red[3]));\n";
-    s << "}\n";
-  }
   std::string src = s.str();
 
   const char* label = "fused_sum";
@@ -799,17 +822,9 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   void* po = data_ptr(o);
   void* pp = single ? nullptr : part->ptr;
   if (!single) args.push_back(&pp);
-  if (ticketed) args.push_back(&ticket);
-  if (single || ticketed) args.push_back(&po);
-  hipFunction_t fin = nullptr;
-  hipError_t e = hipSuccess;
-  if (!single && !ticketed) e = hipModuleGetFunction(&fin, kernel.mod, "fused_sum_final");
-  if (e == hipSuccess) e = launch_module(lg, kernel.fn, grid, (unsigned)NT, args.data(), true, fin == nullptr);
-  if (e == hipSuccess && fin) {
-    int g = (int)grid;
-    void* fargs[] = {&g, &pp, &po};
-    e = launch_module(lg, fin, 1, 256, fargs, false, true);
-  }
+  if (!single) args.push_back(&ticket);
+  args.push_back(&po);
+  const hipError_t e = launch_module(lg, kernel.fn, grid, (unsigned)NT, args.data());
   drop_part();
   if (e != hipSuccess) { hgpu_release(o); return check_hip(ctx, e, "fused_sum launch"); }
   *out = o;
@@ -818,7 +833,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
 
 // hgpu_fused_map with sums: the map's outputs and the sums of some slots from
 // one pass over dense inputs.  Per-block partial sums (double / int64), added
-// up in a fixed order by the block that finishes last (by a second, one-block launch for large arrays).
+// up in a fixed order by the block that finishes last.
 extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, int n_out,
                                    const int* out_slots, hgpu_array** outs, int n_sum, const int* sum_slots, hgpu_array** sums) {
   if (!ctx || !in || !prog || (n_out > 0 && (!out_slots || !outs)) || (n_sum > 0 && (!sum_slots || !sums))) return HGPU_ERR_INVALID;
@@ -874,12 +889,9 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     if (rc) { release_all(); return rc; }
   }
   auto drop_part = [&] { if (part) buffer_release(part); };
-  // Up to 131072 elements (at most a few hundred blocks) the block that finishes last adds the blocks' sums up; beyond, a second launch
-  // does (handing the sums over takes a fence per block, which also waits for the block's share of the outputs
-  // to leave the cache: 16.8 M elements with three outputs take 0.42 ms that way, 0.18 ms with two launches).
-  const bool ticketed = !single && n <= (1 << 17);
+  // The block that finishes last adds the blocks' sums up (hand_over).
   void* ticket = nullptr;
-  if (ticketed) {
+  if (!single) {
     rc = ticket_block(ctx, &ticket);
     if (rc) { drop_part(); release_all(); return rc; }
   }
@@ -900,13 +912,13 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
        "    unsigned long long w = ((unsigned long long)hi << 32) | lo;\n"
        "    v += *reinterpret_cast<A*>(&w);\n"
        "  }\n  return v;\n}\n";
+  if (!single) s << kHandOver;
   auto acc_t = [&](int j) { return dtype_is_float(dt[(size_t)sum_slots[j]]) ? "double" : "i64"; };
   s << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") fused_map_sums(i64 n";
   for (int i = 0; i < n_in; ++i) s << ", const " << ctype(in[i]->dtype) << "* __restrict__ i" << i;
   for (int o = 0; o < n_out; ++o) s << ", " << ctype(res[(size_t)o]->dtype) << "* __restrict__ o" << o;
-  if (ticketed) s << ", unsigned long long* part, unsigned int* ticket";
-  else if (!single) s << ", unsigned long long* __restrict__ part";
-  if (single || ticketed) for (int j = 0; j < n_sum; ++j) s << ", " << ctype(dt[(size_t)sum_slots[j]]) << "* __restrict__ sum" << j;
+  if (!single) s << ", unsigned long long* part, unsigned int* ticket";
+  for (int j = 0; j < n_sum; ++j) s << ", " << ctype(dt[(size_t)sum_slots[j]]) << "* __restrict__ sum" << j;
   s << ") {\n";
   s << "  __shared__ unsigned long long red[" << NT / 64 << "];\n";
   s << "  const i64 step = (i64)gridDim.x * " << NT << ";\n";
@@ -954,42 +966,22 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     } else {
       s << "  if (threadIdx.x == 0) {\n    " << acc_t(j) << " t4[4];\n    for (int k = 0; k < 4; ++k) t4[k] = *reinterpret_cast<" << acc_t(j) << "*>(&red[k]);\n";
       s << "    " << acc_t(j) << " tot = (t4[0] + t4[1]) + (t4[2] + t4[3]);\n";
-      if (ticketed) s << "    __hip_atomic_store(part + ((i64)" << j << " * gridDim.x + blockIdx.x), *reinterpret_cast<unsigned long long*>(&tot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n  }\n";
-      else s << "    part[(i64)" << j << " * gridDim.x + blockIdx.x] = *reinterpret_cast<unsigned long long*>(&tot);\n  }\n";
+      s << "    hand_over(part + ((i64)" << j << " * gridDim.x + blockIdx.x), *reinterpret_cast<unsigned long long*>(&tot));\n  }\n";
     }
     s << "  __syncthreads();\n";
   }
-  if (ticketed) {
-    // The block that finishes last adds the blocks' sums up, always in the same order, and writes the results:
-    // every block hands its sums over (stores, fence, ticket), the last one to draw a ticket sees them all.
+  if (!single) {
     s << "  __shared__ int last;\n";
-    s << "  if (threadIdx.x == 0) {\n    __threadfence();\n    last = atomicAdd(ticket, 1u) == gridDim.x - 1;\n  }\n";
-    s << "  __syncthreads();\n  if (!last) return;\n  __threadfence();\n  const int g = (int)gridDim.x;\n";
+    s << "  if (threadIdx.x == 0) last = last_block(ticket);\n";
+    s << "  __syncthreads();\n  if (!last) return;\n";
     for (int j = 0; j < n_sum; ++j) {
-      s << "  {\n    " << acc_t(j) << " acc = 0;\n";
-      s << "    for (int i = threadIdx.x; i < g; i += 256) {\n";
-      s << "      unsigned long long u = __hip_atomic_load(part + ((i64)" << j << " * g + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n      acc += *reinterpret_cast<" << acc_t(j) << "*>(&u);\n    }\n";
+      s << "  {\n    " << acc_t(j) << " acc = sum_of_blocks<" << acc_t(j) << ">(part + (i64)" << j << " * gridDim.x);\n";
       s << "    acc = wave_sum(acc);\n    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = *reinterpret_cast<unsigned long long*>(&acc);\n    __syncthreads();\n";
       s << "    if (threadIdx.x == 0) {\n      " << acc_t(j) << " t4[4];\n      for (int k = 0; k < 4; ++k) t4[k] = *reinterpret_cast<" << acc_t(j) << "*>(&red[k]);\n";
       s << "      sum" << j << "[0] = (" << ctype(dt[(size_t)sum_slots[j]]) << ")((t4[0] + t4[1]) + (t4[2] + t4[3]));\n    }\n    __syncthreads();\n  }\n";
     }
-    s << "  if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch\n";
   }
   s << "}\n";
-  if (!single && !ticketed) {
-    // second launch: block j adds the partial sums of sum j, in the same order
-    s << "extern \"C\" __global__ void __launch_bounds__(256) fused_map_sums_final(int g, const unsigned long long* __restrict__ part";
-    for (int j = 0; j < n_sum; ++j) s << ", " << ctype(dt[(size_t)sum_slots[j]]) << "* __restrict__ out" << j;
-    s << ") {\n  __shared__ unsigned long long red[4];\n";
-    for (int j = 0; j < n_sum; ++j) {
-      s << "  if (blockIdx.x == " << j << ") {\n    " << acc_t(j) << " acc = 0;\n";
-      s << "    for (int i = threadIdx.x; i < g; i += 256) acc += *reinterpret_cast<const " << acc_t(j) << "*>(&part[(i64)" << j << " * g + i]);\n";
-      s << "    acc = wave_sum(acc);\n    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = *reinterpret_cast<unsigned long long*>(&acc);\n    __syncthreads();\n";
-      s << "    if (threadIdx.x == 0) {\n      " << acc_t(j) << " t4[4];\n      for (int k = 0; k < 4; ++k) t4[k] = *reinterpret_cast<" << acc_t(j) << "*>(&red[k]);\n";
-      s << "      out" << j << "[0] = (" << ctype(dt[(size_t)sum_slots[j]]) << ")((t4[0] + t4[1]) + (t4[2] + t4[3]));\n    }\n  }\n";
-    }
-    s << "}\n";
-  }
   std::string src = s.str();
 
   const char* label = "fused_map_sums";
@@ -1023,18 +1015,9 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
   for (int j = 0; j < n_sum; ++j) sptrs[(size_t)j] = data_ptr(sres[(size_t)j]);
   void* pp = part ? part->ptr : nullptr;
   if (!single) args.push_back(&pp);
-  if (ticketed) args.push_back(&ticket);
-  if (single || ticketed) for (int j = 0; j < n_sum; ++j) args.push_back(&sptrs[(size_t)j]);
-  hipFunction_t fin = nullptr;
-  hipError_t e = hipSuccess;
-  if (!single && !ticketed) e = hipModuleGetFunction(&fin, kernel.mod, "fused_map_sums_final");
-  if (e == hipSuccess) e = launch_module(lg, kernel.fn, grid, (unsigned)NT, args.data(), true, fin == nullptr);
-  if (e == hipSuccess && fin) {
-    int g = (int)grid;
-    std::vector<void*> fargs = {&g, &pp};
-    for (int j = 0; j < n_sum; ++j) fargs.push_back(&sptrs[(size_t)j]);
-    e = launch_module(lg, fin, (unsigned)n_sum, 256, fargs.data(), false, true);
-  }
+  if (!single) args.push_back(&ticket);
+  for (int j = 0; j < n_sum; ++j) args.push_back(&sptrs[(size_t)j]);
+  const hipError_t e = launch_module(lg, kernel.fn, grid, (unsigned)NT, args.data());
   drop_part();
   if (e != hipSuccess) { release_all(); return check_hip(ctx, e, "fused_map_sums launch"); }
   for (int o = 0; o < n_out; ++o) outs[o] = res[(size_t)o];
