@@ -189,6 +189,18 @@ struct CopyJob {
 constexpr int kMaxCopyJobs = 48;
 // ewise.hip: launches up to kMaxCopyJobs independent copies as one kernel (the caller holds launch_mu)
 hipError_t launch_copy_group(hgpu_ctx* ctx, const CopyJob* const* jobs, int n);
+// One elementwise pass over dense arrays (fused.hip): its kernel, the kernel that runs up to kMaxMapJobs of them, and the
+// arguments (element count, inputs, outputs) of 8 bytes each.
+constexpr int kMaxMapJobs = 16;
+struct MapJob {
+  hipFunction_t fn, group;
+  unsigned grid;
+  std::vector<uint64_t> args;
+  const char* label;
+  double bytes, flops;
+};
+// smallk.hip: holds an elementwise pass back (retaining the buffers) to be launched with those of the same kernel that follow it; the caller holds launch_mu
+void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);
 // smallk.hip: holds a copy back (retaining both buffers) to be launched with the copies that follow it
 void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst);
 // contract.hip: launches up to four such reductions of one element type as one kernel (the caller holds launch_mu)

@@ -31,6 +31,7 @@ using namespace hg::fusedgen;
 struct Compiled {
   hipModule_t mod;
   hipFunction_t fn;
+  hipFunction_t group = nullptr;     // fused_map over dense arrays: several passes as one launch
 };
 
 std::map<std::string, Compiled>& cache_of(hgpu_ctx* ctx) {
@@ -48,6 +49,10 @@ int compile(hgpu_ctx* ctx, const std::string& src, Compiled* out, const char* kn
   if (e != hipSuccess) return check_hip(ctx, e, "hipModuleLoadData");
   e = hipModuleGetFunction(&out->fn, out->mod, kname);
   if (e != hipSuccess) return check_hip(ctx, e, "hipModuleGetFunction");
+  if (src.find(" fused_map_group(") != std::string::npos) {
+    e = hipModuleGetFunction(&out->group, out->mod, "fused_map_group");
+    if (e != hipSuccess) return check_hip(ctx, e, "hipModuleGetFunction");
+  }
   return HGPU_OK;
 }
 
@@ -244,13 +249,15 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
   s << kPrelude;
   if (!all_simple) s << "struct FDims { int nd; i64 shape[" << HG_KDIMS << "]; i64 st[" << kMaxIn << "][" << HG_KDIMS << "]; };\n";
   s << "template <typename T, int N> struct alignas(sizeof(T) * N) Vec { T v[N]; };\n";
-  s << "extern \"C\" __global__ void __launch_bounds__(256) " << kernel_name << "(i64 n";
+  if (all_simple) s << "__device__ __forceinline__ void body(i64 n";
+  else s << "extern \"C\" __global__ void __launch_bounds__(256) " << kernel_name << "(i64 n";
   if (!all_simple && !bake) s << ", FDims d";
   for (int i = 0; i < n_in; ++i) s << ", const " << ctype(in[i]->dtype) << "* __restrict__ i" << i;
   for (int o = 0; o < n_out; ++o) s << ", " << ctype(res[(size_t)o]->dtype) << "* __restrict__ o" << o;
   if (sum_slot >= 0) s << ", " << ctype(dt[(size_t)sum_slot]) << "* __restrict__ part";
+  if (all_simple) s << ", unsigned bid, unsigned nblocks";
   s << ") {\n";
-  s << "  const i64 step = (i64)gridDim.x * 256;\n";
+  s << "  const i64 step = (i64)" << (all_simple ? "nblocks" : "gridDim.x") << " * 256;\n";
   for (int i = 0; i < n_in; ++i)
     if (layout[(size_t)i] == 's') s << "  const " << ctype(in[i]->dtype) << " s" << i << " = i" << i << "[0];\n";
   auto emit_program = [&](const char* ind, const std::string& lane_suffix) {
@@ -271,7 +278,7 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
   };
   if (all_simple) {
     s << "  const i64 nv = n / " << vec << ";\n";
-    s << "  for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < nv; i += step) {\n";
+    s << "  for (i64 i = (i64)bid * 256 + threadIdx.x; i < nv; i += step) {\n";
     for (int i = 0; i < n_in; ++i)
       if (layout[(size_t)i] == 'd') s << "    const Vec<" << ctype(in[i]->dtype) << ", " << vec << "> l" << i << " = reinterpret_cast<const Vec<" << ctype(in[i]->dtype) << ", " << vec << ">*>(i" << i << ")[i];\n";
     for (int o = 0; o < n_out; ++o) s << "    Vec<" << ctype(res[(size_t)o]->dtype) << ", " << vec << "> r" << o << ";\n";
@@ -290,7 +297,7 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     for (int o = 0; o < n_out; ++o) s << "    reinterpret_cast<Vec<" << ctype(res[(size_t)o]->dtype) << ", " << vec << ">*>(o" << o << ")[i] = r" << o << ";\n";
     s << "  }\n";
     // tail
-    s << "  const i64 t = nv * " << vec << " + (i64)blockIdx.x * 256 + threadIdx.x;\n";
+    s << "  const i64 t = nv * " << vec << " + (i64)bid * 256 + threadIdx.x;\n";
     s << "  if (t < n) {\n";
     for (int i = 0; i < n_in; ++i) {
       s << "    const " << ctype(in[i]->dtype) << " v" << i << "_t = ";
@@ -401,6 +408,29 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     s << "  }\n";
   }
   s << "}\n";
+  if (all_simple) {
+    // one pass per launch, or several: a block finds its pass in the table of first blocks
+    auto params = [&](const char* before, const char* after) {
+      for (int i = 0; i < n_in; ++i) s << before << "const " << ctype(in[i]->dtype) << "* __restrict__ i" << i << after;
+      for (int o = 0; o < n_out; ++o) s << before << ctype(res[(size_t)o]->dtype) << "* __restrict__ o" << o << after;
+    };
+    auto names = [&](const char* of) {
+      for (int i = 0; i < n_in; ++i) s << ", " << of << "i" << i;
+      for (int o = 0; o < n_out; ++o) s << ", " << of << "o" << o;
+    };
+    s << "extern \"C\" __global__ void __launch_bounds__(256) fused_map(i64 n";
+    params(", ", "");
+    s << ") { body(n";
+    names("");
+    s << ", blockIdx.x, gridDim.x); }\n";
+    s << "struct Job { i64 n; ";
+    params("", "; ");
+    s << "};\nstruct Group { Job job[" << kMaxMapJobs << "]; unsigned first[" << (kMaxMapJobs + 2) / 2 * 2 << "]; };\n";
+    s << "extern \"C\" __global__ void __launch_bounds__(256) fused_map_group(Group g) {\n  int k = 0;\n  while (blockIdx.x >= g.first[k + 1]) ++k;\n";
+    s << "  const Job j = g.job[k];\n  body(j.n";
+    names("j.");
+    s << ", blockIdx.x - g.first[k], g.first[k + 1] - g.first[k]);\n}\n";
+  }
   std::string src = s.str();
 
   const char* label = kernel_name;
@@ -416,10 +446,6 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     snprintf(buf, sizeof buf, "%s[%s,in%d(%s),instr%d(k%d.op%d..),out%d,vec%d,dt%d%s]", kernel_name, sh.c_str(), n_in, layout.c_str(), n_instr, prog[0].kind, prog[0].op, n_out, all_simple ? vec : gvec, a0->dtype, gst.c_str());
     label = intern_label(ctx, buf);
   }
-  std::unique_ptr<LaunchGuard> guard(new LaunchGuard(ctx, label, 0, 0));   // ends before the partial sums' own launch
-  LaunchGuard& lg = *guard;
-  Compiled kernel;
-  if (int rc = kernel_for(ctx, key, hit, src, kernel_name, &kernel)) { release_all(); return rc; }
   // algorithmic traffic: every distinct non-broadcast input once, every output once
   double bytes = 0;
   for (int i = 0; i < n_in; ++i) {
@@ -433,7 +459,32 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     if (!dup) bytes += (double)distinct * dtype_size(in[i]->dtype);
   }
   for (int o = 0; o < n_out; ++o) bytes += (double)n * dtype_size(res[(size_t)o]->dtype);
-  if (lg.timed) { ctx->prof.back().bytes = bytes; ctx->prof.back().flops = (double)n * n_instr; }
+  // Small passes over dense arrays wait for others of the same kernel while a recording is open: an optimizer's update is
+  // one pass per parameter (the CNN's eight, 104,000 parameters in all, as one launch: training step, batch 250, fp32,
+  // 182 -> 167 us).  From a million elements on a pass is worth a launch of its own.  Submitted one by one the host is
+  // what takes the time, and holding a pass costs it more than a launch's gap gives back (24 x 24 CNN: 642 -> 651 us).
+  static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
+  if (hold && ctx->cap && all_simple && n <= (1 << 20)) {
+    std::vector<hgpu_buffer*> reads, writes;
+    MapJob j{nullptr, nullptr, grid_for((n + vec - 1) / vec, 256, ctx->num_cu * 16), {(uint64_t)n}, label, bytes, (double)n * n_instr};
+    for (int i = 0; i < n_in; ++i) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(in[i])); if (in[i]->buf) reads.push_back(in[i]->buf); }
+    for (int o = 0; o < n_out; ++o) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(res[(size_t)o])); writes.push_back(res[(size_t)o]->buf); }
+    {
+      std::lock_guard<std::mutex> lk(ctx->launch_mu);
+      (void)hipSetDevice(ctx->device);
+      Compiled kernel;
+      if (int rc = kernel_for(ctx, key, hit, src, kernel_name, &kernel)) { release_all(); return rc; }
+      j.fn = kernel.fn;
+      j.group = kernel.group;
+      hold_map_locked(ctx, std::move(j), reads, writes);
+    }
+    for (int o = 0; o < n_out; ++o) outs[o] = res[(size_t)o];
+    return HGPU_OK;
+  }
+  std::unique_ptr<LaunchGuard> guard(new LaunchGuard(ctx, label, bytes, (double)n * n_instr));   // ends before the partial sums' own launch
+  LaunchGuard& lg = *guard;
+  Compiled kernel;
+  if (int rc = kernel_for(ctx, key, hit, src, kernel_name, &kernel)) { release_all(); return rc; }
 
   std::vector<void*> args;
   int64_t nn = n;

@@ -686,9 +686,9 @@ namespace hg {
 // reads and writes (retained, so that none is handed out again before the launch).
 struct Deferred {
   bool is_reduction = false;   // a reduction of contract.hip (`red`) instead of a small product
-  bool is_copy = false;        // a copy into an existing array (`copy`); see hold_copy
   RedJob red;
-  CopyJob copy{};
+  CopyJob copy{};              // a copy into an existing array (hold_copy)
+  MapJob map{};                // an elementwise pass (hold_map_locked)
   const std::string* body = nullptr;   // the problem's device code (kept with the known kernels) and the number that stands for it
   int body_id = -1;
   std::string kname;
@@ -702,12 +702,13 @@ struct Deferred {
   int level = 0;
 };
 
-// Products and reductions write new arrays only; copies write existing ones.  The
-// queue holds either products and reductions, or copies that touch no memory of
-// one another: whatever does not fit flushes it first.
+// Products, reductions and elementwise passes write new arrays only; copies write
+// existing ones.  The queue holds either products and reductions, or elementwise
+// passes that read no result of one another, or copies that touch no memory of one
+// another: whatever does not fit flushes it first.
 struct DeferredQueue {
   std::vector<Deferred> items;
-  bool copies = false;               // what `items` holds
+  enum Kind { kProducts, kMaps, kCopies } kind = kProducts;     // what `items` holds
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
 };
@@ -853,7 +854,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     for (auto* b : d.writes) buffer_retain(b);
     std::lock_guard<std::mutex> lk(ctx->launch_mu);
     if (!ctx->dq) ctx->dq = new DeferredQueue;
-    if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->copies) flush_deferred_locked(ctx);
+    if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
     ctx->dq->items.push_back(std::move(d));
     ctx->dq_pending = true;
     *handled = true;
@@ -867,6 +868,48 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   if (err != hipSuccess) return check_hip(ctx, err, "small-K product launch");
   *handled = true;
   return HGPU_OK;
+}
+
+// The held elementwise passes, those of one kernel together.
+static void launch_maps(hgpu_ctx* ctx, std::vector<Deferred>& items) {
+  for (size_t i0 = 0; i0 < items.size(); ++i0) {
+    MapJob& m = items[i0].map;
+    if (!m.fn) continue;               // went out with an earlier one
+    std::vector<MapJob*> jobs{&m};
+    for (size_t i = i0 + 1; m.group && i < items.size() && jobs.size() < (size_t)kMaxMapJobs; ++i)
+      if (items[i].map.fn == m.fn) jobs.push_back(&items[i].map);
+    hgpu_ctx::ProfRec r{jobs.size() > 1 ? "fused_map_group" : m.label, nullptr, nullptr, 0, 0};
+    for (auto* j : jobs) { r.bytes += j->bytes; r.flops += j->flops; }
+    const bool timed = ctx->profiling && !ctx->cap && hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess;
+    std::vector<uint64_t> block;       // struct Group of the kernel's text: the jobs' arguments, then the first block of each
+    std::vector<void*> args;
+    hipFunction_t fn = m.fn;
+    unsigned grid = m.grid;
+    if (jobs.size() > 1) {
+      const size_t words = m.args.size();
+      block.assign(words * kMaxMapJobs + (kMaxMapJobs + 2) / 2, 0);
+      unsigned* first = (unsigned*)(block.data() + words * kMaxMapJobs);
+      grid = 0;
+      for (int k = 0; k <= kMaxMapJobs; ++k) {
+        first[k] = grid;
+        if ((size_t)k >= jobs.size()) continue;
+        std::copy(jobs[(size_t)k]->args.begin(), jobs[(size_t)k]->args.end(), block.begin() + (long)(words * (size_t)k));
+        grid += jobs[(size_t)k]->grid;
+      }
+      fn = m.group;
+      args.push_back(block.data());
+    } else {
+      for (auto& w : m.args) args.push_back(&w);
+    }
+    const hipError_t err = timed ? hipExtModuleLaunchKernel(fn, grid * 256, 1, 1, 256, 1, 1, 0, ctx->stream, args.data(), nullptr, r.a, r.b, 0)
+                                 : hipModuleLaunchKernel(fn, grid, 1, 1, 256, 1, 1, 0, ctx->stream, args.data(), nullptr);
+    if (timed) ctx->prof.push_back(r);
+    if (err != hipSuccess) {
+      int rc = check_hip(ctx, err, "fused_map launch");
+      if (!ctx->deferred_rc) ctx->deferred_rc = rc;
+    }
+    for (auto* j : jobs) j->fn = nullptr;
+  }
 }
 
 // Launches what was held back.  Products are levelled by who reads whose
@@ -887,8 +930,14 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
       for (auto* b : d.writes) buffer_release(b);
     }
   };
-  if (ctx->dq->copies) {
-    ctx->dq->copies = false;
+  const DeferredQueue::Kind kind = ctx->dq->kind;
+  ctx->dq->kind = DeferredQueue::kProducts;
+  if (kind == DeferredQueue::kMaps) {
+    launch_maps(ctx, items);
+    release_items();
+    return;
+  }
+  if (kind == DeferredQueue::kCopies) {
     std::vector<const CopyJob*> jobs;
     double bytes = 0;
     for (auto& d : items) { jobs.push_back(&d.copy); bytes += d.bytes; }
@@ -1059,10 +1108,31 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
   for (auto* b : d.writes) buffer_retain(b);
   std::lock_guard<std::mutex> lk(ctx->launch_mu);
   if (!ctx->dq) ctx->dq = new DeferredQueue;
-  if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->copies) flush_deferred_locked(ctx);
+  if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
   ctx->dq->items.push_back(std::move(d));
   ctx->dq_pending = true;
   return true;
+}
+
+// An elementwise pass joins the queue: it waits for passes that read none of the held results (an optimizer's
+// updates, one per parameter), and goes out when anything else is enqueued.
+void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes) {
+  if (!ctx->dq) ctx->dq = new DeferredQueue;
+  DeferredQueue& q = *ctx->dq;
+  bool fits = q.items.empty() || (q.kind == DeferredQueue::kMaps && q.items.size() < kMaxHeld);
+  for (size_t i = 0; fits && i < q.items.size(); ++i)
+    for (auto* w : q.items[i].writes)
+      for (auto* r : reads) fits = fits && r != w;
+  if (!fits) flush_deferred_locked(ctx);
+  q.items.emplace_back();
+  Deferred& d = q.items.back();
+  d.map = std::move(job);
+  d.reads = reads;
+  d.writes = writes;
+  for (auto* b : d.reads) buffer_retain(b);
+  for (auto* b : d.writes) buffer_retain(b);
+  q.kind = DeferredQueue::kMaps;
+  ctx->dq_pending = true;
 }
 
 // A copy into an existing array joins the queue.  It waits only for copies: anything else that is enqueued goes
@@ -1070,7 +1140,6 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
 // writes, or whose destination a held copy reads, flushes them first.
 void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst) {
   Deferred d;
-  d.is_copy = true;
   d.copy = job;
   d.bytes = 2.0 * (double)job.bytes;
   d.reads.push_back(src);
@@ -1081,14 +1150,14 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
-  bool fits = q.items.empty() || (q.copies && q.items.size() < (size_t)kMaxCopyJobs);
+  bool fits = q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs);
   for (size_t i = 0; fits && i < q.items.size(); ++i) {
     const hgpu_buffer *r = q.items[i].reads[0], *w = q.items[i].writes[0];
     fits = w != src && w != dst && r != dst;
   }
   if (!fits) flush_deferred_locked(ctx);
   q.items.push_back(std::move(d));
-  q.copies = true;
+  q.kind = DeferredQueue::kCopies;
   ctx->dq_pending = true;
   if (!hold) flush_deferred_locked(ctx);
 }
