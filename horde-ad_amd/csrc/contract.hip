@@ -395,9 +395,9 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
   decompose<1>(keep, blockIdx.x, ko);
   const T* p = a + ko[0];
   const int t = threadIdx.x;
-  bool have = t < L;
-  T best = have ? p[(int64_t)t * sl] : T(0);
-  int64_t bi = t;
+  // a NaN is neither greater nor smaller than anything: it counts only in the first place, where it stays (below)
+  T best = t < L ? p[(int64_t)t * sl] : T(0);
+  int64_t bi = t < L && best == best ? t : INT64_MAX;
   // eight loads in flight; the comparisons keep the order of the positions
   int64_t j = (int64_t)t + 1024;
   for (; j + 7 * 1024 < L; j += 8 * 1024) {
@@ -406,17 +406,17 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
     for (int u = 0; u < 8; ++u) x[u] = p[(j + u * 1024) * sl];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      bool better = want_max ? (x[u] > best) : (x[u] < best);
+      bool better = bi == INT64_MAX ? x[u] == x[u] : (want_max ? (x[u] > best) : (x[u] < best));
       if (better) { best = x[u]; bi = j + u * 1024; }
     }
   }
   for (; j < L; j += 1024) {
     T x = p[j * sl];
-    bool better = want_max ? (x > best) : (x < best);
+    bool better = bi == INT64_MAX ? x == x : (want_max ? (x > best) : (x < best));
     if (better) { best = x; bi = j; }
   }
   sbest[t] = best;
-  sidx[t] = have ? bi : INT64_MAX;
+  sidx[t] = bi;
   __syncthreads();
   for (int off = 512; off > 0; off >>= 1) {
     if (t < off) {
@@ -431,8 +431,10 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
     __syncthreads();
   }
   if (t == 0) {
-    out[blockIdx.x] = sidx[0];
-    if (vals) vals[blockIdx.x] = sbest[0];
+    const T first = p[0];
+    const bool keep_first = !(first == first);
+    out[blockIdx.x] = keep_first ? 0 : sidx[0];
+    if (vals) vals[blockIdx.x] = keep_first ? first : sbest[0];
   }
 }
 
@@ -743,7 +745,8 @@ int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_
       collapse(1, psh, 2, ks2, &k2);
       collapse(1, psh + 1, 2, rs2, &r2);
       bool wave2 = n_out < 65536;
-      HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<A, T>(ctx, wave2, k2, r2, n_out, S, 1, pp, nullptr, out)); });
+      // few outputs under many partial sums: a block each (one output, 4096 partial sums: 8.0 us with a wavefront, 4.4 with a block)
+      HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<A, T>(ctx, wave2, k2, r2, n_out, S, n_out < 256 && S >= 256 ? 0 : 1, pp, nullptr, out)); });
     }
     if (part) buffer_release(part);
   }
@@ -1011,8 +1014,9 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
       HG_DISPATCH_DTYPE(a->dtype, T, hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, a->strides[a->rank - 1], want_max, G, piece, (const T*)data_ptr(a), (T*)pb, pi));
       HG_DISPATCH_DTYPE(a->dtype, T, hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, G, want_max, (const T*)pb, (const int64_t*)pi, (int64_t*)data_ptr(o), (T*)vp));
       buffer_release(scratch);
-    } else if (L >= 8192 && n_out <= 64) {
-      // few long rows: a whole block per row
+    } else if (L >= 512 && n_out <= 64) {
+      // few long rows: a whole block per row (one row of 2500 fp32, a minibatch's logits: a wavefront, load after load, takes
+      // 14.4 us, a block 5.8; one of 1500 fp64 9.9 and 5.0)
       HG_DISPATCH_DTYPE(a->dtype, T, hipLaunchKernelGGL(k_argminmax_block<T>, dim3((unsigned)n_out), dim3(1024), 0, ctx->stream, keep, L, a->strides[a->rank - 1], want_max, (const T*)data_ptr(a), (int64_t*)data_ptr(o), (T*)vp));
     } else if (L >= 256 && n_out < (int64_t)ctx->num_cu * 64) {
       unsigned g = grid_for(n_out * 64, kBlock, ctx->num_cu * 8);

@@ -1,0 +1,51 @@
+"""A few rows of some hundred to some thousand elements (csrc/contract.hip): extrema by a block per row, sums of many
+partial sums by a block per output."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int64, np.int8])
+@pytest.mark.parametrize("rows,n", [(1, 511), (1, 512), (1, 513), (3, 1024), (64, 1025), (65, 1025), (2, 8191), (1, 9217)])
+def test_first_extremum(gpu, dt, rows, n):
+    """Ties: the first position wins, within a lane's own positions and between lanes; rows contiguous and strided."""
+    rng = np.random.default_rng(n)
+    x = rng.integers(-100 if dt == np.int8 else -n, 100 if dt == np.int8 else n, (rows, n)).astype(dt)
+    x[0, n // 3] = x[0, -1] = x[0].max()
+    x[-1, 5] = x[-1, n // 2] = x[-1].min()
+    for a in (gpu.upload(x), gpu.upload(np.ascontiguousarray(x.T)).transpose([1, 0])):
+        for want_max in (True, False):
+            vals, idx = a.extremum_last(want_max)
+            want = (np.argmax if want_max else np.argmin)(x, axis=-1)
+            assert np.array_equal(idx.numpy(), want)
+            assert np.array_equal(vals.numpy(), np.take_along_axis(x, want[:, None], 1)[:, 0])
+
+
+def test_extrema_beside_nans(gpu):
+    """Element after element with > or <, as the checker goes: a NaN is passed over, and stays when it is the first."""
+    x = np.random.default_rng(4).uniform(-1, 1, (5, 1500))
+    x[0, 1:1400:2] = np.nan
+    x[1, 0] = np.nan
+    x[2, 1:] = np.nan
+    x[3, 1023], x[3, 70] = np.nan, np.inf
+    x[4, 1:1025] = np.nan
+    for want_max in (True, False):
+        vals, idx = gpu.upload(x).extremum_last(want_max)
+        want = (np.nanargmax if want_max else np.nanargmin)(x, axis=-1)
+        want[1] = 0
+        assert np.array_equal(idx.numpy(), want)
+        assert np.array_equal(vals.numpy(), np.take_along_axis(x, want[:, None], 1)[:, 0], equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int64])
+@pytest.mark.parametrize("outs,n", [(1, 3000001), (7, 600000), (300, 40000)])
+def test_sums_of_many_partial_sums(gpu, dt, outs, n):
+    rng = np.random.default_rng(outs)
+    x = (rng.integers(-9, 9, (outs, n)) if dt == np.int64 else rng.uniform(-1, 1, (outs, n))).astype(dt)
+    got = gpu.upload(x).contract(None, 1).numpy()
+    wide = x.astype(np.int64 if dt == np.int64 else np.float64)
+    if dt == np.int64:
+        assert np.array_equal(got, wide.sum(1))
+    else:      # summed in fp64 by either, rounded once to the result's type
+        assert np.all(np.abs(got - wide.sum(1)) <= n * 2.0 ** -52 * np.abs(wide).sum(1) / 100 + np.finfo(dt).eps * np.abs(wide.sum(1)))
