@@ -157,10 +157,56 @@ __device__ __forceinline__ A lane_strided_sum(const TI* __restrict__ pa, const T
   return (acc0 + acc1) + (acc2 + acc3);
 }
 
+// The same sum over [j0, j1) where a lies side by side (and b does, or stays on one element, as the ones of a plain sum
+// do): 16 bytes a load.  With four bytes a load, and b fetched for every element, rows of 5000 to 8192 fp32 went by at
+// 3.4 TB/s: 2048 rows of 8192 19.5 -> 17.4 us, 28 x 128 rows of 5000 19.9 -> 16.3 us.  Element-aligned: rows start anywhere.
+// For rows that fill one round of loads (4 KB): shorter ones are as fast either way.  Not in k_contract_group, whose
+// reductions are mostly short and which the additional registers slow down (CNN: 326.6 -> 328.1 us).
+template <typename TI> struct Vec16Of { using type = TI __attribute__((ext_vector_type(16 / sizeof(TI)), aligned(sizeof(TI)))); };
+template <typename TI, typename A, bool HASB>
+__device__ __forceinline__ A wide_sum(const TI* __restrict__ pa, const TI* __restrict__ pb, int64_t sb, int64_t j0, int64_t j1, int lane) {
+  using V = typename Vec16Of<TI>::type;
+  constexpr int N = 16 / sizeof(TI), U = 4;
+  const bool vb = HASB && sb != 0;
+  const A one_b = HASB && !vb ? (A)pb[0] : (A)1;
+  A acc[U] = {0, 0, 0, 0};
+  int64_t j = j0 + lane * N;
+  auto add = [&](A& c, const V& x, const V& y) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) c += HASB ? (A)x[e] * (vb ? (A)y[e] : one_b) : (A)x[e];
+  };
+  for (; j + (U - 1) * 64 * N + N <= j1; j += U * 64 * N) {
+    V x[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = *reinterpret_cast<const V*>(pa + j + u * 64 * N);
+    if (vb) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) y[u] = *reinterpret_cast<const V*>(pb + j + u * 64 * N);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) add(acc[u], x[u], y[u]);
+  }
+  for (; j + N <= j1; j += 64 * N) {
+    const V x = *reinterpret_cast<const V*>(pa + j);
+    V y = x;
+    if (vb) y = *reinterpret_cast<const V*>(pb + j);
+    add(acc[0], x, y);
+  }
+  for (; j < j1; ++j) acc[1] += HASB ? (A)pa[j] * (vb ? (A)pb[j] : one_b) : (A)pa[j];      // (less than a vector, one lane's)
+  return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+template <typename TI, typename A, bool HASB, bool WIDE>
+__device__ __forceinline__ A row_sum(const TI* __restrict__ pa, const TI* __restrict__ pb, int64_t sa, int64_t sb, int64_t j0, int64_t j1, int lane) {
+  if constexpr (WIDE && std::is_floating_point<TI>::value) {
+    if (sa == 1 && (!HASB || sb == 1 || sb == 0) && j1 - j0 >= 4096 / (int64_t)sizeof(TI)) return wide_sum<TI, A, HASB>(pa, pb, sb, j0, j1, lane);
+  }
+  return lane_strided_sum<TI, A, HASB>(pa, pb, sa, sb, j0 + lane, j1);
+}
+
 // One wavefront per work item.  `red` has its innermost dim split off:
 // Lin = extent, (sa_in, sb_in) = strides; `red` keeps the outer reduced dims
 // with Q = their product.  Chunks split Q when Q > 1, else Lin.
-template <typename TI, typename TO, bool HASB>
+template <typename TI, typename TO, bool HASB, bool WIDE>
 __device__ __forceinline__ void wave_body(const Dims& keep, const Dims& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                           int S, int64_t chunk, const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, const TermPtrs* tp, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
@@ -219,7 +265,7 @@ __device__ __forceinline__ void wave_body(const Dims& keep, const Dims& red, int
       decompose<2>(red, q, ro);
       const TI* pa = a + ko[0] + ro[0];
       const TI* pb = HASB ? b + ko[1] + ro[1] : nullptr;
-      acc += lane_strided_sum<TI, A, HASB>(pa, pb, sa_in, sb_in, j0 + lane, j1);
+      acc += row_sum<TI, A, HASB, WIDE>(pa, pb, sa_in, sb_in, j0, j1, lane);
     }
     acc = wave_sum<A>(acc);
     if (lane == 0) out[item] = (TO)acc;
@@ -228,7 +274,7 @@ __device__ __forceinline__ void wave_body(const Dims& keep, const Dims& red, int
 template <typename TI, typename TO, bool HASB>
 __global__ void __launch_bounds__(kBlock) k_contract_wave(Dims keep, Dims red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                                            int S, int64_t chunk, const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, TermPtrs tp) {
-  wave_body<TI, TO, HASB>(keep, red, n_out, Q, Lin, sa_in, sb_in, S, chunk, a0, b0, out, &tp, blockIdx.x, gridDim.x);
+  wave_body<TI, TO, HASB, true>(keep, red, n_out, Q, Lin, sa_in, sb_in, S, chunk, a0, b0, out, &tp, blockIdx.x, gridDim.x);
 }
 
 // One block of four wavefronts per output: for a few hundred outputs with a few
@@ -236,7 +282,7 @@ __global__ void __launch_bounds__(kBlock) k_contract_wave(Dims keep, Dims red, i
 // the device idle and splitting into chunks would cost a second launch.  The
 // wavefronts take every fourth outer reduced index (or a quarter of the inner
 // dim when there is no outer one) and combine through LDS in a fixed order.
-template <typename TI, typename TO, bool HASB>
+template <typename TI, typename TO, bool HASB, bool WIDE>
 __device__ __forceinline__ void block_body(const Dims& keep, const Dims& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                            const TI* __restrict__ a, const TI* __restrict__ b, TO* __restrict__ out, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
@@ -251,12 +297,12 @@ __device__ __forceinline__ void block_body(const Dims& keep, const Dims& red, in
       for (int64_t q = w; q < Q; q += NW) {
         int64_t ro[2];
         decompose<2>(red, q, ro);
-        acc += lane_strided_sum<TI, A, HASB>(a + ko[0] + ro[0], HASB ? b + ko[1] + ro[1] : nullptr, sa_in, sb_in, lane, Lin);
+        acc += row_sum<TI, A, HASB, WIDE>(a + ko[0] + ro[0], HASB ? b + ko[1] + ro[1] : nullptr, sa_in, sb_in, 0, Lin, lane);
       }
     } else {
       const int64_t quarter = (Lin + NW - 1) / NW;
       const int64_t j0 = w * quarter, j1 = j0 + quarter < Lin ? j0 + quarter : Lin;
-      acc = lane_strided_sum<TI, A, HASB>(a + ko[0], HASB ? b + ko[1] : nullptr, sa_in, sb_in, j0 + lane, j1);
+      acc = row_sum<TI, A, HASB, WIDE>(a + ko[0], HASB ? b + ko[1] : nullptr, sa_in, sb_in, j0, j1, lane);
     }
     acc = wave_sum<A>(acc);
     if (lane == 0) part[w] = acc;
@@ -273,7 +319,7 @@ __device__ __forceinline__ void block_body(const Dims& keep, const Dims& red, in
 template <typename TI, typename TO, bool HASB>
 __global__ void __launch_bounds__(kBlock) k_contract_block(Dims keep, Dims red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                                             const TI* __restrict__ a, const TI* __restrict__ b, TO* __restrict__ out) {
-  block_body<TI, TO, HASB>(keep, red, n_out, Q, Lin, sa_in, sb_in, a, b, out, blockIdx.x, gridDim.x);
+  block_body<TI, TO, HASB, true>(keep, red, n_out, Q, Lin, sa_in, sb_in, a, b, out, blockIdx.x, gridDim.x);
 }
 
 // Up to four single-launch reductions of one element type as one kernel: the first blocks are problem 0's, the
@@ -303,11 +349,11 @@ __global__ void __launch_bounds__(kBlock) k_contract_group(RedGroup g) {
   const T* b = (const T*)r.b;
   T* out = (T*)r.out;
   if (r.variant == 0) {
-    if (r.hasb) block_body<T, T, true>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, a, b, out, bid, r.grid);
-    else block_body<T, T, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, a, b, out, bid, r.grid);
+    if (r.hasb) block_body<T, T, true, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, a, b, out, bid, r.grid);
+    else block_body<T, T, false, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, a, b, out, bid, r.grid);
   } else if (r.variant == 1) {
-    if (r.hasb) wave_body<T, T, true>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
-    else wave_body<T, T, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
+    if (r.hasb) wave_body<T, T, true, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
+    else wave_body<T, T, false, false>(r.keep, r.red, r.n_out, r.Q, r.Lin, r.sa, r.sb, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
   } else {
     if (r.hasb) lane_body<T, T, true>(r.keep, r.red, r.n_out, r.R, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
     else lane_body<T, T, false>(r.keep, r.red, r.n_out, r.R, 1, r.chunk, a, b, out, nullptr, bid, r.grid);
