@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
-@pytest.mark.parametrize("rows,n", [(1, 1), (3, 63), (5, 255), (2, 257), (70, 1023), (9, 1025), (300, 4099), (2100, 1031), (130, 70001), (1, 1000003)])
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 63), (5, 255), (2, 257), (70, 1023), (9, 1025), (300, 4099), (2100, 1031), (1025, 1024), (4095, 1500), (130, 70001), (1, 1000003)])
 def test_rows_that_start_anywhere(gpu, dt, rows, n):
     """Whole tables, tables without their first or last columns (rows off 16-byte boundaries), reversed rows (the other path); plain
     sums, products with another table, with ones that are one element, and with one row for all."""
