@@ -38,7 +38,7 @@ SIGNATURES = {
     "init": (I, [I, PP]), "shutdown": (I, [P]), "sync": (I, [P]), "last_error": (C.c_char_p, [P]),
     "upload": (I, [P, I, I, LP, P, PP]), "download": (I, [P, P, P]), "read_scalar": (I, [P, P, P]),
     "retain": (I, [P]), "release": (I, [P]), "rank": (I, [P]), "dtype_of": (I, [P]), "size": (L, [P]),
-    "shape": (I, [P, LP]), "strides": (I, [P, LP]), "is_dense": (I, [P]),
+    "shape": (I, [P, LP]), "strides": (I, [P, LP]), "is_dense": (I, [P]), "shares_memory": (I, [P, P]),
     "transpose": (I, [P, P, I, IP, PP]), "reshape": (I, [P, P, I, LP, PP]),
     "slice": (I, [P, P, I, L, L, PP]), "reverse": (I, [P, P, I, PP]),
     "replicate": (I, [P, P, I, LP, PP]), "index_prefix": (I, [P, P, I, LP, PP]),

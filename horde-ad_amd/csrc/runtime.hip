@@ -692,6 +692,7 @@ int hgpu_strides(const hgpu_array* a, int64_t* s) {
   return HGPU_OK;
 }
 int hgpu_is_dense(const hgpu_array* a) { return a && is_dense(a) ? 1 : 0; }
+int hgpu_shares_memory(const hgpu_array* a, const hgpu_array* b) { return a && b && a->buf && a->buf == b->buf ? 1 : 0; }
 
 /* -------------------------------------------------------------------- views */
 

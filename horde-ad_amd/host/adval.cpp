@@ -4,7 +4,7 @@
 // (src/HordeAd/Core/DeltaEval.hs:391-595).  Each rule cites the delta
 // constructor it transposes.
 #include <algorithm>
-#include <cstring>
+#include <cstddef>
 
 #include "host.hpp"
 
@@ -30,14 +30,63 @@ static void accum(std::vector<T>& slots, int node, const T& cot) {
   s = s.valid() ? add_cotangents(s, cot) : cot;
 }
 
-std::vector<T> Tape::backward(const D& out, const T& dt, const std::vector<D>& inputs) {
-  be->unit_products.clear();
+// The factors that rules of the reverse pass under way multiplied by its seed of ones (mul below).  Such a product is the
+// factor itself, an array of the forward pass as a rule.
+static thread_local std::vector<std::shared_ptr<ArrHolder>>* unit_factors = nullptr;
+
+static bool knows_sharing(const Backend* be) {
+  return be->api->struct_size >= offsetof(hgpu_api, shares_memory) + sizeof(be->api->shares_memory) && be->api->shares_memory;
+}
+
+// A copy of r that its consumer makes, or that is made together with others.
+static T times_one(const T& r) { return lazy_mul(r, broadcast_scalar(seed_one(r.be(), r.dtype()), r.shape())); }
+
+// The gradient leaves, computed, each in memory of its own: a caller writes new values into parameters, into values it
+// kept of the forward pass, into the cotangent it handed in and into other gradients, and no gradient may change with them.
+// units: the factors taken for their product with one; dt: what the pass started from.
+static void own_leaves(Backend* be, std::vector<T>& res, const std::vector<std::shared_ptr<ArrHolder>>& units, const T& dt) {
+  // (a factor that is still pending would be computed into one array for the forward pass and for the caller)
+  for (T& r : res)
+    if (std::find(units.begin(), units.end(), r.holder()) != units.end()) r = times_one(r);
+  // Nothing stays pending: the leaves are what the caller asked for, and those of one shape that are still
+  // elementwise programs share a pass.
+  force_many(res);
+  if (!knows_sharing(be)) return;
+  // Views of a factor (the rules of transposes, reshapes, slices between the product and the input), of the caller's
+  // cotangent, of another leaf.  A view that repeats one element cannot be written into and may stay one.
+  const hgpu_api* api = be->api;
+  std::vector<T> copies;
+  for (size_t i = 0; i < res.size(); ++i) {
+    hgpu_array* h = res[i].h();
+    bool shared = false;
+    for (const auto& u : units) shared = shared || (u->h && api->shares_memory(h, u->h));
+    if (!shared && api->is_dense(h)) {
+      shared = dt.valid() && dt.holder()->h && api->shares_memory(h, dt.holder()->h);
+      for (size_t j = 0; j < i && !shared; ++j) shared = api->shares_memory(h, res[j].h());
+    }
+    if (!shared) continue;
+    res[i] = differentiable(res[i]) ? times_one(res[i]) : materialize(res[i]);
+    copies.push_back(res[i]);
+  }
+  force_many(copies);
+}
+
+std::vector<T> Tape::backward(const D& out, const T& dt_or_none, const std::vector<D>& inputs) {
+  std::vector<std::shared_ptr<ArrHolder>> units;
+  struct Scope {
+    std::vector<std::shared_ptr<ArrHolder>>* before;
+    explicit Scope(std::vector<std::shared_ptr<ArrHolder>>* u) : before(unit_factors) { unit_factors = u; }
+    ~Scope() { unit_factors = before; }
+  };
+  T dt = dt_or_none;
   std::vector<T> slots(recs.size());
   std::vector<bool> keep(recs.size(), false);
   for (auto& i : inputs)
     if (i.node >= 0) keep[(size_t)i.node] = true;
   if (out.node >= 0) {
+    if (!dt.valid()) dt = broadcast_scalar(seed_one(be, out.primal.dtype()), out.primal.shape());
     if (dt.shape() != out.primal.shape()) throw HostError(HGPU_ERR_INVALID, "backward: cotangent shape differs from the result's");
+    Scope scope(&units);
     slots[(size_t)out.node] = dt;
     for (int n = out.node; n >= 0; --n) {
       if (!slots[(size_t)n].valid()) continue;
@@ -47,17 +96,14 @@ std::vector<T> Tape::backward(const D& out, const T& dt, const std::vector<D>& i
   }
   std::vector<T> res;
   for (auto& i : inputs) {
-    if (i.node >= 0 && slots[(size_t)i.node].valid()) res.push_back(slots[(size_t)i.node]);
-    else res.push_back(zeros(be, i.primal.dtype(), i.primal.shape()));   // tdefTarget
+    if (i.node >= 0 && slots[(size_t)i.node].valid()) {
+      res.push_back(slots[(size_t)i.node]);
+      continue;
+    }
+    T z = zeros(be, i.primal.dtype(), i.primal.shape());   // tdefTarget
+    res.push_back(z.size() == 1 ? materialize(z) : z);     // (one element: not the library's constant itself)
   }
-  // A leaf that came through products with one only is an array of the forward pass: the caller gets its own copy.
-  for (T& r : res)
-    for (const auto& u : be->unit_products)
-      if (r.holder() == u && u->h) { r = materialize(r); break; }
-  be->unit_products.clear();
-  // The gradient leaves are what the caller asked for: nothing stays pending,
-  // and leaves of one shape that are still elementwise programs share a pass.
-  force_many(res);
+  own_leaves(be, res, units, dt);
   return res;
 }
 
@@ -69,24 +115,23 @@ D d_const(const T& t) {
 
 // Products made by transposition rules stay pending: most are summed at once
 // by the rule of a `replicate` further up, which then is a single contraction.
-// A factor that is the constant one at every position (the seed of a reverse pass, `grad`'s dt) leaves the
-// other factor as it is: no pass over it (rows of 51 MB that a lookup's cotangent multiplied by one: 16 us).
-static bool is_one(const T& t) {
-  Backend* be = t.be();
-  if (!be->fuse) return false;
-  const double one = 1.0;
-  uint64_t bits;
-  std::memcpy(&bits, &one, 8);
-  auto it = be->const_cache.find(std::make_pair(t.dtype(), bits));
-  if (it == be->const_cache.end()) return false;
+// A factor that is the one a reverse pass started from leaves the other factor as it is: no pass over it (rows of 51 MB that a
+// lookup's cotangent multiplied by one: 16 us).  Only that one: a constant that a caller can hold may be overwritten
+// between the launches of a recording, which then has to follow it.
+static bool is_seed(const T& t) {
+  const ArrHolder* one = t.be()->seed_one[t.dtype() == HGPU_F32].get();
   const ArrHolder* h = t.holder().get();
-  for (int hop = 0; h && hop < 4; ++hop, h = h->scalar_src.get())
-    if (h == it->second.get()) return true;
+  for (int hop = 0; one && h && hop < 4; ++hop, h = h->scalar_src.get())
+    if (h == one) return true;
   return false;
 }
 static T mul(const T& a, const T& b) {
-  if (is_one(b)) { a.be()->unit_products.push_back(a.holder()); return a; }
-  if (is_one(a)) { b.be()->unit_products.push_back(b.holder()); return b; }
+  if (unit_factors && a.be()->fuse && knows_sharing(a.be()))
+    for (int side = 0; side < 2; ++side)
+      if (is_seed(side ? a : b)) {
+        unit_factors->push_back((side ? b : a).holder());
+        return side ? b : a;
+      }
   return lazy_mul(a, b);
 }
 static T add(const T& a, const T& b) { return ewise2(HGPU_ADD, a, b); }

@@ -81,6 +81,7 @@ int hh_destroy(hh_ctx* c) {
   c->tape.recs.clear();
   c->be.iota_cache.clear();
   c->be.const_cache.clear();
+  for (auto& s : c->be.seed_one) s.reset();
   c->be.api->shutdown(c->be.ctx);
   // The context object stays: values released later still point at it.
   return HGPU_OK;
@@ -129,6 +130,7 @@ static bool has_graphs(const hgpu_api* api) {
 int hh_capture_begin(hh_ctx* c) {
   return guarded(c, [&] {
     if (!has_graphs(c->be.api)) throw HostError(HGPU_ERR_UNSUPPORTED, "this provider records no graphs");
+    for (int dt : {HGPU_F64, HGPU_F32}) (void)seed_one(&c->be, dt);      // (nothing is uploaded during a capture)
     c->be.check(c->be.api->capture_begin(c->be.ctx));
     c->be.capturing = true;
   });
@@ -227,7 +229,7 @@ int hh_backward(hh_ctx* c, hh_val* out, hh_val* dt, int n, hh_val* const* inputs
   return guarded(c, [&] {
     std::vector<D> ins;
     for (int i = 0; i < n; ++i) ins.push_back(inputs[i]->d);
-    std::vector<T> g = c->tape.backward(out->d, dt->d.primal, ins);
+    std::vector<T> g = c->tape.backward(out->d, dt ? dt->d.primal : T(), ins);
     for (int i = 0; i < n; ++i) grads[i] = box(d_const(g[(size_t)i]));
   });
 }

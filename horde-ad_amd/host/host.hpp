@@ -146,7 +146,8 @@ struct Backend {
   uint64_t walk_gen = 0;    // walks over pending expressions number themselves: a node seen carries the walk's number
   std::vector<std::weak_ptr<ArrHolder>> pending_dimsums;   // sums over all dims but one of an expression, not yet taken (ArrHolder::ones_b)
   std::vector<std::weak_ptr<ArrHolder>> pending_sums;   // sums of all elements of an expression, not yet taken (ArrHolder::ssrc)
-  std::vector<std::shared_ptr<ArrHolder>> unit_products;   // factors that a transposition rule multiplied by the constant one in the reverse pass under way
+  // The one that a reverse pass without a cotangent of the caller's starts from, per floating-point type: its own array, which no caller ever holds
+  std::shared_ptr<ArrHolder> seed_one[2];
   std::map<std::string, int64_t> counters;   // how often each rewrite onto a fused entry point was taken (diagnostic)
   void check(int rc) const;
 };
@@ -367,6 +368,7 @@ class T {
 T upload(Backend* be, int dtype, const Shape& shape, const void* host);
 T constant(Backend* be, int dtype, double value);                 // cached rank-0 array
 T constant_i(Backend* be, int dtype, int64_t value);
+T seed_one(Backend* be, int dtype);                                // Backend::seed_one
 T iota(Backend* be, int64_t n, int dtype);                         // cached
 T transpose(const T& a, const std::vector<int>& perm);
 T reshape(const T& a, const Shape& shape);
@@ -494,7 +496,7 @@ struct Tape {
   explicit Tape(Backend* b) : be(b) {}
   D input(const T& t);                                     // differentiable leaf
   int push(std::function<void(const T&, std::vector<T>&)> f);
-  // Cotangents of `inputs` given d(out) = dt.
+  // Cotangents of `inputs` given d(out) = dt (an empty T: one at every position).  Each has memory of its own.
   std::vector<T> backward(const D& out, const T& dt, const std::vector<D>& inputs);
 };
 

@@ -89,6 +89,12 @@ T constant(Backend* be, int dtype, double value) {
   return t;
 }
 
+T seed_one(Backend* be, int dtype) {
+  auto& s = be->seed_one[dtype == HGPU_F32];
+  if (!s) s = upload_scalar(be, dtype, 1.0, 0, false).holder();
+  return T(s);
+}
+
 T constant_i(Backend* be, int dtype, int64_t value) {
   if (dtype == HGPU_F64 || dtype == HGPU_F32) return constant(be, dtype, (double)value);
   auto key = std::make_pair(dtype + 100, (uint64_t)value);

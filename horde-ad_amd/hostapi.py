@@ -184,11 +184,9 @@ class Host:
 
     def grad(self, out, inputs, dt=None):
         """Cotangents of `inputs` for d(out) = dt (default: ones, as `grad` uses)."""
-        if dt is None:
-            dt = self.srepl(out.shape, 1.0, out.dtype)
         arr = (C.c_void_p * len(inputs))(*[v.h for v in inputs])
         outs = (C.c_void_p * len(inputs))()
-        self.check(self.dll.hh_backward(self.h, out.h, dt.h, len(inputs), arr, outs))
+        self.check(self.dll.hh_backward(self.h, out.h, dt.h if dt is not None else None, len(inputs), arr, outs))
         return [V(self, C.c_void_p(o)) for o in outs]
 
     # -- host loops of the tensor class (the reference's `Concrete` instance runs

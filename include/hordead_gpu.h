@@ -164,6 +164,9 @@ int hgpu_shape(const hgpu_array* a, int64_t* shape_out);
 int hgpu_strides(const hgpu_array* a, int64_t* strides_out);
 /* 1 when the view is dense row-major (what `stoVector` can return without a copy). */
 int hgpu_is_dense(const hgpu_array* a);
+/* 1 when the two arrays are views of one block of memory: what is written into
+ * one with hgpu_overwrite or hgpu_assign may show in the other. */
+int hgpu_shares_memory(const hgpu_array* a, const hgpu_array* b);
 
 /* ------------------------------------------------- views (no element traffic) */
 
@@ -549,6 +552,7 @@ typedef struct hgpu_api {
   int (*contract_sum_map)(hgpu_ctx*, int, const hgpu_array* const*, const hgpu_array* const*, int, int, const hgpu_array* const*, int, const hgpu_fused_instr*, int,
                          const int*, hgpu_array**);
   int (*fused_map_dimsum)(hgpu_ctx*, int, const hgpu_array* const*, int, const hgpu_fused_instr*, int, const int*, hgpu_array**, int, int, hgpu_array**);
+  int (*shares_memory)(const hgpu_array*, const hgpu_array*);
 } hgpu_api;
 
 /* The table of this library's own entry points. */

@@ -106,7 +106,10 @@ int hh_adam_step_size(hh_ctx* ctx, int dtype, double alpha, double beta1, double
 int hh_adam_apply(hh_ctx* ctx, hh_val* alphat, double beta1, double beta2, double epsilon, hh_val* m, hh_val* v, hh_val* params, hh_val* gradient,
                   hh_val** m_new, hh_val** v_new, hh_val** params_new);
 
-/* gradientFromDelta (DeltaEval.hs:64-78): cotangents of `inputs` for d(out)=dt. */
+/* gradientFromDelta (DeltaEval.hs:64-78): cotangents of `inputs` for d(out)=dt
+ * (NULL: one at every position, what `grad` starts from).  Every gradient has
+ * memory of its own: writing into the values of the forward pass, into dt or
+ * into another gradient leaves it as it is. */
 int hh_backward(hh_ctx* ctx, hh_val* out, hh_val* dt, int n, hh_val* const* inputs, hh_val** grads);
 
 /* Elementwise Num/Floating/IntegralH/RealFloatH methods (AstInterpret.hs:187-194). */

@@ -56,6 +56,11 @@ struct hgpu_array {
   int dtype;
   std::vector<int64_t> shape;
   std::vector<char> data;
+  // Arrays of horc_get_api_views only: the array this one is a view of (retained), where each element stands in
+  // it, and the views of this array.
+  hgpu_array* base = nullptr;
+  std::vector<int64_t> at;
+  std::vector<hgpu_array*> views;
 };
 
 namespace {
@@ -245,13 +250,22 @@ int horc_read_scalar(hgpu_ctx* c, const hgpu_array* a, void* host) {
   return HGPU_OK;
 }
 int horc_retain(hgpu_array* a) { a->refs++; return HGPU_OK; }
-int horc_release(hgpu_array* a) { if (a && --a->refs == 0) delete a; return HGPU_OK; }
+int horc_release(hgpu_array* a) {
+  while (a && --a->refs == 0) {
+    hgpu_array* base = a->base;
+    if (base) base->views.erase(std::find(base->views.begin(), base->views.end(), a));
+    delete a;
+    a = base;
+  }
+  return HGPU_OK;
+}
 int horc_rank(const hgpu_array* a) { return (int)a->shape.size(); }
 int horc_dtype_of(const hgpu_array* a) { return a->dtype; }
 int64_t horc_size(const hgpu_array* a) { return prod(a->shape); }
 int horc_shape(const hgpu_array* a, int64_t* s) { std::copy(a->shape.begin(), a->shape.end(), s); return HGPU_OK; }
 int horc_strides(const hgpu_array* a, int64_t* s) { auto st = dense_strides(a->shape); std::copy(st.begin(), st.end(), s); return HGPU_OK; }
 int horc_is_dense(const hgpu_array*) { return 1; }
+int horc_shares_memory(const hgpu_array* a, const hgpu_array* b) { return a && a == b && !a->data.empty(); }
 
 // Nested.stranspose: result dim i = source dim perm[i] (OpsConcrete.hs:647-649).
 int horc_transpose(hgpu_ctx* c, const hgpu_array* a, int np, const int* perm, hgpu_array** out) {
@@ -961,6 +975,7 @@ const hgpu_api* horc_get_api(void) {
       nullptr,   // no fused_map_sums
       nullptr,   // no contract_sum_map
       nullptr,   // no fused_map_dimsum
+      horc_shares_memory,
   };
   return &api;
 }
@@ -979,3 +994,94 @@ const hgpu_api* horc_get_api_fused(void) {
 }
 
 }  // extern "C"
+
+// ---- a table whose views share memory ----------------------------------------
+// Every array above owns its data, so nothing that goes wrong when two arrays share a block can be seen on those
+// tables.  On this one a view remembers what it is a view of, and assigning to an array shows in the arrays it shares memory
+// with, as on the device.
+
+// one past the other without a gap: what hgpu_assign takes as a destination
+static bool consecutive(const hgpu_array* a) {
+  for (size_t i = 1; i < a->at.size(); ++i)
+    if (a->at[i] != a->at[i - 1] + 1) return false;
+  return true;
+}
+static void read_base(hgpu_array* a) {
+  const size_t es = dsize(a->dtype);
+  for (size_t i = 0; i < a->at.size(); ++i) std::memcpy(a->data.data() + i * es, a->base->data.data() + (size_t)a->at[i] * es, es);
+  for (auto* v : a->views) read_base(v);
+}
+// `op` makes the view of any array of a's shape; told where the elements of a stand it says where the view's do.
+template <typename F>
+static int view_of(hgpu_ctx* c, const hgpu_array* a, hgpu_array** out, F op) {
+  hgpu_array *places = make(c, HGPU_I64, a->shape), *seen = nullptr;
+  for (int64_t i = 0, n = prod(a->shape); i < n; ++i) ptr<int64_t>(places)[i] = i;
+  int rc = op(places, &seen);
+  horc_release(places);
+  if (rc) return rc;
+  hgpu_array* o = make(c, a->dtype, seen->shape);
+  o->at.assign(ptr<int64_t>(seen), ptr<int64_t>(seen) + prod(seen->shape));
+  horc_release(seen);
+  o->base = const_cast<hgpu_array*>(a);
+  horc_retain(o->base);
+  o->base->views.push_back(o);
+  read_base(o);
+  *out = o;
+  return HGPU_OK;
+}
+static int view_transpose(hgpu_ctx* c, const hgpu_array* a, int n, const int* perm, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_transpose(c, x, n, perm, o); });
+}
+static int view_reshape(hgpu_ctx* c, const hgpu_array* a, int rank, const int64_t* shape, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_reshape(c, x, rank, shape, o); });
+}
+static int view_slice(hgpu_ctx* c, const hgpu_array* a, int dim, int64_t start, int64_t len, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_slice(c, x, dim, start, len, o); });
+}
+static int view_reverse(hgpu_ctx* c, const hgpu_array* a, int dim, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_reverse(c, x, dim, o); });
+}
+static int view_replicate(hgpu_ctx* c, const hgpu_array* a, int n, const int64_t* pre, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_replicate(c, x, n, pre, o); });
+}
+static int view_index_prefix(hgpu_ctx* c, const hgpu_array* a, int n, const int64_t* ix, hgpu_array** out) {
+  for (int i = 0; i < n && i < (int)a->shape.size(); ++i)
+    if (ix[i] < 0 || ix[i] >= a->shape[(size_t)i]) return horc_index_prefix(c, a, n, ix, out);   // zeros: no view
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_index_prefix(c, x, n, ix, o); });
+}
+static int view_as_strided(hgpu_ctx* c, const hgpu_array* a, int rank, const int64_t* shape, const int64_t* strides, int64_t offset, hgpu_array** out) {
+  return view_of(c, a, out, [&](const hgpu_array* x, hgpu_array** o) { return horc_as_strided(c, x, rank, shape, strides, offset, o); });
+}
+static const hgpu_array* root_of(const hgpu_array* a) {
+  while (a->base) a = a->base;
+  return a;
+}
+static int view_is_dense(const hgpu_array* a) { return consecutive(a); }
+static int view_shares_memory(const hgpu_array* a, const hgpu_array* b) { return a && b && root_of(a) == root_of(b) && !a->data.empty() && !b->data.empty(); }
+static int view_assign(hgpu_ctx* c, hgpu_array* dst, const hgpu_array* src) {
+  if (!consecutive(dst)) return fail(c, HGPU_ERR_INVALID, "assign: the destination is a strided view");
+  if (view_shares_memory(dst, src)) return fail(c, HGPU_ERR_INVALID, "assign: source and destination share memory");
+  int rc = horc_assign(c, dst, src);
+  if (rc) return rc;
+  for (; dst->base; dst = dst->base) {
+    const size_t es = dsize(dst->dtype);
+    for (size_t i = 0; i < dst->at.size(); ++i) std::memcpy(dst->base->data.data() + (size_t)dst->at[i] * es, dst->data.data() + i * es, es);
+  }
+  for (auto* v : dst->views) read_base(v);
+  return HGPU_OK;
+}
+
+extern "C" const hgpu_api* horc_get_api_views(void) {
+  static hgpu_api api = *horc_get_api_fused();
+  api.transpose = view_transpose;
+  api.reshape = view_reshape;
+  api.slice = view_slice;
+  api.reverse = view_reverse;
+  api.replicate = view_replicate;
+  api.index_prefix = view_index_prefix;
+  api.as_strided = view_as_strided;
+  api.is_dense = view_is_dense;
+  api.shares_memory = view_shares_memory;
+  api.assign = view_assign;
+  return &api;
+}
