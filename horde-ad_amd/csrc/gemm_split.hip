@@ -9,11 +9,15 @@
 // exact in fp32, and they are added into fp32 accumulators, as
 // v_mfma_f32_32x32x2_f32 adds its products.
 //
-// Exactness of the split needs |x| (when not zero) between 2^-100 and 2^127: below,
-// a part could be subnormal, above, rounding to bf16 could overflow, and an
-// infinity or NaN has no remainder.  Every staged element is checked; a block
-// that has met an element outside that range computes its tile again with
-// v_mfma_f32_32x32x2_f32, so such inputs give what they always gave.
+// Range.  Operands are multiplied by 2^23 on their way into the split (the first remainder is one fma, so it costs one
+// multiplication an element), the sums by 2^-46 on their way out: the smallest fp32 number, 2^-149, is then 2^-126, and no
+// part of any element is subnormal.  From above, the parts must not overflow, nor the sums of their products, which are
+// 2^-7 larger than the products themselves while only h h' has been added.  Every block knows the largest element of each
+// operand it has staged: where 2^23 of it or 2^46 K |a| |b| could pass 2^127 -- elements from 2^104, infinities, NaNs, products from
+// 2^81 / K -- the block computes its tile again with v_mfma_f32_32x32x2_f32, so such inputs give what they always gave.
+// (Limits at 2^-100 and 2^127 on the elements alone, without the scaling, sent every tile that met a softmax
+// probability under e^-69 the second way, 3.9 ms instead of 0.41 for 2048 x 8192 over 2048, and let products just
+// below 2^128 overflow.)
 //
 // What bounds it: the power the matrix cores draw.  Six bf16 instructions of 32 x 32 x 16 do the work of eight
 // fp32 ones of 32 x 32 x 2 in under half the cycles; at 2048 x 8192 over 2048 the clock falls to 1.8 GHz and
@@ -44,19 +48,17 @@ constexpr int SK = 16;                      // k of one step: one MFMA deep
 // Eight consecutive k of one row on their way to LDS.
 struct Slot { float v[8]; };
 
-// Range of the elements met so far, as bit patterns shifted left by one (the sign gone).
-struct Seen { uint32_t hi, lo; };          // largest; smallest of the non-zero ones, minus one
-constexpr uint32_t kLargest = 0xfe000000u; // 2^127, doubled pattern
-constexpr uint32_t kSmallest = 0x1b000000u - 1;  // 2^-100
+constexpr int kScaleLog = 23;               // operands are split after multiplication by 2^23
+constexpr float kScale = 8388608.0f, kUnscale = 1.0f / (8388608.0f * 8388608.0f);
 
 __device__ __forceinline__ uint32_t pack(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf2));
 }
 
-// the three parts of two neighbours
+// the three parts of two neighbours, scaled
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = pack(a, b);
-  const float a1 = a - __builtin_bit_cast(float, h << 16), b1 = b - __builtin_bit_cast(float, h & 0xffff0000u);
+  h = pack(a * kScale, b * kScale);
+  const float a1 = __builtin_fmaf(a, kScale, -__builtin_bit_cast(float, h << 16)), b1 = __builtin_fmaf(b, kScale, -__builtin_bit_cast(float, h & 0xffff0000u));
   m = pack(a1, b1);
   l = pack(a1 - __builtin_bit_cast(float, m << 16), b1 - __builtin_bit_cast(float, m & 0xffff0000u));
 }
@@ -115,7 +117,7 @@ struct Side {
     }
   }
   // parts: [3][ROWS * 2] of 16 bytes
-  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, Seen& seen) const {
+  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, uint32_t& largest) const {
     u4 h, m, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -126,8 +128,7 @@ struct Side {
       m[j] = pm;
       l[j] = pl;
       const uint32_t ua = __builtin_bit_cast(uint32_t, a) << 1, ub = __builtin_bit_cast(uint32_t, b) << 1;
-      seen.hi = max(seen.hi, max(ua, ub));
-      seen.lo = min(seen.lo, min(ua - 1, ub - 1));
+      largest = max(largest, max(ua, ub));
     }
     parts[at[i]] = h;
     parts[ROWS * 2 + at[i]] = m;
@@ -186,7 +187,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-  Seen seen{0, 0xffffffffu};
+  uint32_t top_a = 0, top_b = 0;            // the largest element of each operand met so far, as a bit pattern shifted left by one (the sign gone)
 
   const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
   Slot ra[NA], rb[NB];
@@ -201,9 +202,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   if (whole > 0) fetch(0);
   else fetch_tail(0);
 #pragma unroll
-  for (int i = 0; i < NA; ++i) sa.store(ra[i], i, lds[0], seen);
+  for (int i = 0; i < NA; ++i) sa.store(ra[i], i, lds[0], top_a);
 #pragma unroll
-  for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, seen);
+  for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, top_b);
   __syncthreads();
 
   const int fra = lds_at(wm * TM * 32 + (lane & 31), lane >> 5), frb = lds_at(wn * TN * 32 + (lane & 31), lane >> 5);
@@ -257,8 +258,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
         constexpr int first = 2;
         if (j >= first) {
           const int u = j - first;
-          if (u < NA) sa.store(ra[u], u, ln, seen);
-          else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, seen);
+          if (u < NA) sa.store(ra[u], u, ln, top_a);
+          else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, top_b);
         }
       }
     }
@@ -266,8 +267,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
       constexpr int first = 2;
 #pragma unroll
       for (int u = TN - first; u < NA + NB; ++u) {
-        if (u < NA) sa.store(ra[u], u, ln, seen);
-        else sb.store(rb[u - NA], u - NA, ln + PA, seen);
+        if (u < NA) sa.store(ra[u], u, ln, top_a);
+        else sb.store(rb[u - NA], u - NA, ln + PA, top_b);
       }
     }
     __syncthreads();
@@ -282,18 +283,37 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   step(i0, std::integral_constant<int, 0>{});
 
   float* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)s * p.c_split_stride;
-  auto put = [&](int i, int j, const f16v& c) {
+  auto put = [&](int i, int j, const f16v& c, float scale) {
     const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
     if (n >= p.N) return;
     float* col = Cout + (int64_t)n * p.scn;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int m = m0 + (wm * TM + i) * 32 + MfmaF32W::row(lane, r);
-      if (m < p.M) col[(int64_t)m * p.scm] = c[r];
+      if (m < p.M) col[(int64_t)m * p.scm] = c[r] * scale;
     }
   };
-  if (__syncthreads_or(seen.hi >= kLargest || seen.lo < kSmallest)) {
-    // an element that three bf16 cannot hold exactly: the tile again, on the fp32 instruction
+  // what the largest elements of the whole block allow: see the head of the file
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    top_a = max(top_a, (uint32_t)__shfl_xor(top_a, d));
+    top_b = max(top_b, (uint32_t)__shfl_xor(top_b, d));
+  }
+  uint32_t* tops = reinterpret_cast<uint32_t*>(lds[0]);      // (free: the last step ended with a barrier)
+  if (lane == 0) {
+    tops[2 * wave] = top_a;
+    tops[2 * wave + 1] = top_b;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WM * WN; ++w) {
+    top_a = max(top_a, tops[2 * w]);
+    top_b = max(top_b, tops[2 * w + 1]);
+  }
+  const int ea = (int)(top_a >> 24) - 126, eb = (int)(top_b >> 24) - 126;       // |a| < 2^ea, |b| < 2^eb
+  const int ek = 32 - __builtin_clz((uint32_t)(kend - kbeg));                      // K < 2^ek
+  if (ea + kScaleLog > 127 || eb + kScaleLog > 127 || ea + eb + 2 * kScaleLog + ek + 1 > 127) {
+    // elements or sums that could leave fp32's range: the tile again, on the fp32 instruction
 #pragma unroll 1
     for (int ij = 0; ij < TM * TN; ++ij) {
       const int i = ij / TN, j = ij - i * TN;
@@ -314,14 +334,14 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
 #pragma unroll
         for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u], fb[u], c, 0, 0, 0);
       }
-      put(i, j, c);
+      put(i, j, c, 1.0f);
     }
     return;
   }
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) put(i, j, acc[i][j]);
+    for (int j = 0; j < TN; ++j) put(i, j, acc[i][j], kUnscale);
 }
 
 template <typename F>

@@ -57,6 +57,56 @@ def test_infinities_and_nans_stay_where_they_belong(gpu):
     assert np.all(np.abs(out[fine] - want[fine]) <= (k + 17) * 2.0 ** -24 * want[fine])
 
 
+def test_products_close_to_the_largest_number(gpu):
+    """Products that fit fp32 although the product of their operands' leading parts, both rounded up, does not."""
+    m, n, k = 150, 200, 1030
+    x, y = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    x[:, 1:], y[:, 1:] = 2.0 ** -40, 2.0 ** -41
+    x[:, 0] = np.linspace(1.9961, 1.9999, m) * 2.0 ** 63
+    y[:, 0] = np.linspace(1.9961, 1.9999, n) * 2.0 ** 63
+    y[1::3, 0] *= -1
+    out, want = product(gpu, x, y, "KK").numpy(), x.astype(np.float64) @ y.astype(np.float64).T
+    assert np.all(np.abs(want) < 2.0 ** 128 * (1 - 2.0 ** -24)) and np.all(np.abs(want) > 2.0 ** 128 * (1 - 2.0 ** -8))
+    assert np.all(np.abs(out - want) <= 4 * 2.0 ** -24 * np.abs(want))
+
+
+def test_products_close_to_the_largest_number(gpu):
+    """Products that fit fp32 although the product of their operands' leading parts, both rounded up, does not."""
+    m, n, k = 150, 200, 1030
+    x, y = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    x[:, 1:], y[:, 1:] = 2.0 ** -40, 2.0 ** -41
+    x[:, 0] = np.linspace(1.9961, 1.9999, m) * 2.0 ** 63
+    y[:, 0] = np.linspace(1.9961, 1.9999, n) * 2.0 ** 63
+    y[1::3, 0] *= -1
+    out, want = product(gpu, x, y, "KK").numpy(), x.astype(np.float64) @ y.astype(np.float64).T
+    assert np.all(np.abs(want) < 2.0 ** 128 * (1 - 2.0 ** -24)) and np.all(np.abs(want) > 2.0 ** 128 * (1 - 2.0 ** -8))
+    assert np.all(np.abs(out - want) <= 4 * 2.0 ** -24 * np.abs(want))
+
+
+@pytest.mark.parametrize("small", [2.0 ** -99, 2.0 ** -101, 2.0 ** -110, 2.0 ** -126, 2.0 ** -140, 2.0 ** -149])
+def test_small_elements_keep_all_their_bits(gpu, small):
+    """Down to the smallest subnormal number an element takes part with all the bits it has."""
+    m, n, k = 140, 190, 1030
+    rng = np.random.default_rng(11)
+    x, y = (rng.uniform(1, 16, (m, k)) * small).astype(np.float32), rng.uniform(2.0 ** 20, 2.0 ** 21, (n, k)).astype(np.float32)
+    x[::2, 1:] = 0
+    out, xd, yd = product(gpu, x, y, "KR").numpy(), x.astype(np.float64), y.astype(np.float64)
+    bound = np.where(np.arange(m) % 2 == 0, 4, k / 16 + 17)[:, None] * 2.0 ** -24 * (xd @ yd.T) + 2.0 ** -149
+    assert np.all(np.abs(out - xd @ yd.T) <= bound)
+
+
+@pytest.mark.parametrize("top_x,top_y", [(2.0 ** 103, 1.0), (2.0 ** 104, 1.0), (2.0 ** 60, 2.0 ** 10), (2.0 ** 40, 2.0 ** 40), (2.0 ** 62, 2.0 ** 62), (1.0, 2.0 ** 126)])
+def test_large_elements_beside_ordinary_ones(gpu, top_x, top_y):
+    """Either side of the limits from which a tile goes to the fp32 instruction."""
+    m, n, k = 260, 150, 1040
+    rng = np.random.default_rng(12)
+    x, y = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    x[7, 3], x[200, 1039], y[140, 3] = top_x, -top_x * 0.7, top_y
+    out, xd, yd = product(gpu, x, y, "RK").numpy(), x.astype(np.float64), y.astype(np.float64)
+    # (the fp32 instruction rounds once per product)
+    assert np.all(np.abs(out - xd @ yd.T) <= (k + 17) * 2.0 ** -24 * (np.abs(xd) @ np.abs(yd).T))
+
+
 @pytest.mark.parametrize("terms", [2, 5])
 def test_sum_of_products(gpu, terms):
     m, n, k = 130, 100, 2000
