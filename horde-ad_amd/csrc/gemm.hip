@@ -325,7 +325,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     q.b_term[t] = swap ? p.a_term[t] : p.b_term[t];
   }
   const int64_t out_n = nelem(out);
-  int cfg = 0, split = 1;
+  int split = 1;
   if (f64) {
     // Microseconds, as measured: a step of 16 k of a 64 x 64 tile takes 0.62 alone on its CU, 0.56 with another one
     // there, 0.5 with more; 5 for the launch; partial results as below.  (300 x 784 over 5000, main kernel / with the
@@ -339,23 +339,19 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       if (us < best) { best = us; split = (int)sp; }
     }
   } else {
-    // Microseconds, as measured: a step of 16 k of a 256 x 256 tile (one block on a CU) 3.4, of a 128 x 128 tile
-    // 1.4 alone on its CU and 0.92 for each of several; 8 for the launch with its first loads and last stores; for
-    // partial results a second launch and their bytes once out and once in.  (2048 x 8192 over 2048: 395-425 us
-    // in 256 x 256 tiles, 450-480 in 128 x 128; 2048 x 784 over 8192, where 256-wide tiles would be a quarter
-    // empty: 217 against 203; 300 x 5000 over 784: 37 with its partial sums in 128 x 128 tiles and K in four.)
+    // Microseconds, as measured: a step of 16 k of a 128 x 128 tile 1.4 alone on its CU and 0.92 for each of several;
+    // 8 for the launch with its first loads and last stores; for partial results a second launch and their bytes once
+    // out and once in.  (Without the sums: 2048 x 8192 over 2048 464, 2048 x 784 over 8192 217, 300 x 5000 over 784 29.)
     double best = 1e300;
-    for (int c = 0; c < 2; ++c) {
-      const int64_t bm = c == 0 ? 256 : 128, tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * p.BT * nt;
-      for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
-        const int64_t per_cu = (tiles * sp + ctx->num_cu - 1) / ctx->num_cu, steps = ((p.K + sp - 1) / sp + 15) / 16;
-        const double step = c == 0 ? 3.4 * per_cu : (per_cu == 1 ? 1.4 : 0.92 * per_cu);
-        const double us = 8 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 4 / 3.2e6 : 0);
-        if (us < best) { best = us; cfg = c; split = (int)sp; }
-      }
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128) * p.BT * nt;
+    for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
+      const int64_t per_cu = (tiles * sp + ctx->num_cu - 1) / ctx->num_cu, steps = ((p.K + sp - 1) / sp + 15) / 16;
+      const double step = per_cu == 1 ? 1.4 : 0.92 * per_cu;
+      const double us = 8 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 4 / 3.2e6 : 0);
+      if (us < best) { best = us; split = (int)sp; }
     }
   }
-  const int64_t BM = f64 ? 64 : (cfg == 0 ? 256 : 128), BN = BM;
+  const int64_t BM = f64 ? 64 : 128, BN = BM;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   q.kchunk = (int)(((p.K + split - 1) / split + 15) / 16 * 16);
   q.term_split = (int)((p.K + q.kchunk - 1) / q.kchunk);
@@ -380,7 +376,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       label = intern_label(ctx, buf);
     }
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
-    LaunchArgs la{ctx->stream, cfg, 0, 0, sak == 1, sbk == 1, dim3((unsigned)tiles, (unsigned)split, (unsigned)p.BT), swap ? pb : pa, swap ? pa : pb, cdst, nullptr, nullptr};
+    LaunchArgs la{ctx->stream, 0, 0, 0, sak == 1, sbk == 1, dim3((unsigned)tiles, (unsigned)split, (unsigned)p.BT), swap ? pb : pa, swap ? pa : pb, cdst, nullptr, nullptr};
     {
       LaunchGuard lg(ctx, label, bytes, flops);
       la.ev_start = lg.start_event();

@@ -1,34 +1,41 @@
 // fp32 matrix products on the bf16 matrix cores, without giving up fp32.
 //
-// An fp32 number with a normal exponent is the exact sum of three bf16 numbers
-// (8 + 8 + 8 significant bits): x = h + m + l, each part the nearest bf16 of
-// what is left.  A product of two such sums has nine terms; the six largest are
-// h h', h m', m h', m m', h l', l h', and the three left out (m l', l m', l l')
-// together stay below 2^-25 of the product -- half of what rounding the product
-// to fp32 would cost.  Every term of the six is a product of two 8-bit numbers,
-// exact in fp32, and they are added into fp32 accumulators, as
-// v_mfma_f32_32x32x2_f32 adds its products.
+// An fp32 number is the exact sum of three bf16 numbers (8 + 8 + 8 significant
+// bits): x = h + m + l, each part the nearest bf16 of what is left, so that
+// |m| <= 2^-8 |x| and |l| <= 2^-17 |x|.  A product of two such sums has nine terms;
+// the six largest are h h', h m', m h', m m', h l', l h', and the three left out
+// (m l', l m', l l') together stay below 2^-24 of the product (plus 2^-34): as much as
+// rounding the product to fp32 may cost.  Every term of the six is a product of
+// two 8-bit numbers, exact in fp32.
+//
+// How the terms are added decides the rest.  The matrix cores drop low bits of what they add onto a larger number, so h h'
+// is summed from zero, sixteen at a time, and goes to its accumulator with one rounded addition, and the five small terms
+// have an accumulator of their own, on the matrix cores throughout (2^-7 of the other one: its lost bits do not
+// count); the two meet in one addition at the end.  Error against fp64 in units of 2^-24 of the sum of magnitudes, mean (max),
+// 2048 terms, beside v_mfma_f32_32x32x2_f32 and beside all six terms in one chain:
+//     normally distributed      0.039 (0.34)   0.098 (0.65)   0.064 (0.38)
+//     uniform in 0 .. 1         0.67  (3.8)    0.84  (4.7)    0.66  (3.5)
+//     e^-uniform(0, 100)        0.24  (2.2)    0.27  (2.1)    0.29  (2.1)
+//     one product, no others    0.366 (1.7)    0.361 (1.0)    0.457 (2.4)
+// With all eight terms the last row is 0.361 (1.0) too, and every product takes a fifth longer (464 -> 557 us below):
+// left at six.
 //
 // Range.  Operands are multiplied by 2^23 on their way into the split (the first remainder is one fma, so it costs one
 // multiplication an element), the sums by 2^-46 on their way out: the smallest fp32 number, 2^-149, is then 2^-126, and no
 // part of any element is subnormal.  From above, the parts must not overflow, nor the sums of their products, which are
 // 2^-7 larger than the products themselves while only h h' has been added.  Every block knows the largest element of each
-// operand it has staged: where 2^23 of it or 2^46 K |a| |b| could pass 2^127 -- elements from 2^104, infinities, NaNs, products from
+// operand it has staged: where 2^23 of it or 2^46 K |a| |b| could pass 2^127 -- elements from 2^104, infinities, products from
 // 2^81 / K -- the block computes its tile again with v_mfma_f32_32x32x2_f32, so such inputs give what they always gave.
 // (Limits at 2^-100 and 2^127 on the elements alone, without the scaling, sent every tile that met a softmax
 // probability under e^-69 the second way, 3.9 ms instead of 0.41 for 2048 x 8192 over 2048, and let products just
 // below 2^128 overflow.)
 //
-// What bounds it: the power the matrix cores draw.  Six bf16 instructions of 32 x 32 x 16 do the work of eight
-// fp32 ones of 32 x 32 x 2 in under half the cycles; at 2048 x 8192 over 2048 the clock falls to 1.8 GHz and
-// orders of the loop's instructions that differ by a fifth in stalls measure the same.  So the tile is the largest
-// whose accumulators leave two wavefronts to a SIMD (256 x 256, eight wavefronts, each operand element is split
-// once for 256 columns): 645 us on the fp32 instruction, 417-425 here (165 TFLOP/s) on normally distributed
-// numbers, 577 and 375-395 on the activations of a wide relu network (128 x 128: 450-480).  Sixteen products are
-// summed from zero and then added to the accumulator with one rounded addition: fed to the matrix cores on
-// top of a large accumulator the small terms lose their low bits (error against fp64, 2048 terms, normal /
-// positive: 2.3e-7 / 1.7e-7; with the accumulator in the chain 7.0e-7 / 4.3e-7 at 375 us; fp32 instruction
-// 8.1e-7 / 3.5e-7).
+// What bounds it: the vector instructions beside the products (an element's split, 7 of them, and the rounded
+// additions) and the power the matrix cores draw; orders of the loop's instructions that differ by a fifth in stalls
+// measure the same.  Six bf16 instructions of 32 x 32 x 16 do the work of eight fp32 ones of 32 x 32 x 2.  2048 x 8192
+// over 2048, normally distributed / behind a relu: fp32 instruction 649 / 615 us, here 464 / 428.  (256 x 256 tiles split an
+// element half as often, but two sets of accumulators do not fit: all six terms in one chain 407 / 378, the second
+// set added up by vector instructions 480 / 445.  256 x 128 tiles: 489 / 456.)
 #include "gemm_kernel.hpp"
 
 using namespace hg;
@@ -70,7 +77,7 @@ __device__ __forceinline__ int lds_at(int r, int h) { return r * 2 + (h ^ ((r >>
 // One operand's share of a tile: ROWS rows of SK elements, a lane owns NS pieces of eight k each.
 // Loads go through a buffer descriptor over the operand: a fixed 32-bit offset per lane plus a
 // scalar one for the step, and whatever lies past the end (rows, k) reads as zero.
-template <int ROWS, bool KC, int NT>
+template <int ROWS, bool KC>
 struct Side {
   static constexpr int NS = ROWS * 2 / NT;
   __amdgpu_buffer_rsrc_t rsrc;
@@ -117,7 +124,7 @@ struct Side {
     }
   }
   // parts: [3][ROWS * 2] of 16 bytes
-  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, uint32_t& largest) const {
+  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, float& largest) const {
     u4 h, m, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -127,8 +134,7 @@ struct Side {
       h[j] = ph;
       m[j] = pm;
       l[j] = pl;
-      const uint32_t ua = __builtin_bit_cast(uint32_t, a) << 1, ub = __builtin_bit_cast(uint32_t, b) << 1;
-      largest = max(largest, max(ua, ub));
+      asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(a), "v"(b));      // (passes NaNs over: their parts are NaNs)
     }
     parts[at[i]] = h;
     parts[ROWS * 2 + at[i]] = m;
@@ -136,11 +142,10 @@ struct Side {
   }
 };
 
-// Wavefronts WM x WN, each TM x TN blocks of 32 x 32.
-template <int WM, int WN, int TM, int TN, bool AKC, bool BKC>
-__global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
-  constexpr int CH = 2;                     // blocks of a wavefront whose chains of products alternate
-  constexpr int NT = 64 * WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
+  constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 32 x 32 blocks of each
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr int PA = 3 * BM * 2, PB = 3 * BN * 2;       // 16-byte elements of one buffer
   __shared__ u4 lds[2][PA + PB];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -174,20 +179,20 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   const int kbeg = sk * p.kchunk;
   const int kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
 
-  Side<BM, AKC, NT> sa;
-  Side<BN, BKC, NT> sb;
+  Side<BM, AKC> sa;
+  Side<BN, BKC> sb;
   sa.init(t, A, p.a_bytes, p.sam, m0, p.M, p.sak);
   sb.init(t, B, p.b_bytes, p.sbn, n0, p.N, p.sbk);
-  constexpr int NA = Side<BM, AKC, NT>::NS, NB = Side<BN, BKC, NT>::NS;
+  constexpr int NA = Side<BM, AKC>::NS, NB = Side<BN, BKC>::NS;
 
-  f16v acc[TM][TN];
+  f16v acc[TM][TN], low[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-  uint32_t top_a = 0, top_b = 0;            // the largest element of each operand met so far, as a bit pattern shifted left by one (the sign gone)
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0;
+  float top_a = 0, top_b = 0;               // the largest magnitude of each operand met so far
 
   const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
   Slot ra[NA], rb[NB];
@@ -230,32 +235,25 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
       bf8 fb[3];
 #pragma unroll
       for (int q = 0; q < 3; ++q) fb[q] = __builtin_bit_cast(bf8, lb[q * BN * 2 + j * 64]);
-      // The six terms of 16 k are summed from zero, the smallest first, and added to the accumulators with one
-      // rounded addition: small terms fed to the matrix cores on top of a large accumulator lose their low bits.
+      // h h' of 16 k is summed from zero and added with one rounded addition; the five smaller terms are summed on the
+      // matrix cores, the smallest first.
 #pragma unroll
-      for (int i0 = 0; i0 < TM; i0 += CH) {
-        f16v c[CH];
-        auto add = [&](int qa, int qb) {
+      for (int i = 0; i < TM; ++i) {
+        f16v zero;
 #pragma unroll
-          for (int i = 0; i < CH; ++i) c[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i0 + i][qa], fb[qb], c[i], 0, 0, 0);
-        };
+        for (int r = 0; r < 16; ++r) zero[r] = 0;
+        auto add = [&](int qa, int qb, const f16v& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[qb], c, 0, 0, 0); };
+        const f16v c = add(0, 0, zero);
+        low[i][j] = add(2, 0, low[i][j]);
+        low[i][j] = add(0, 2, low[i][j]);
+        low[i][j] = add(1, 1, low[i][j]);
+        low[i][j] = add(1, 0, low[i][j]);
+        low[i][j] = add(0, 1, low[i][j]);
 #pragma unroll
-        for (int i = 0; i < CH; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) c[i][r] = 0;
-        add(2, 0);
-        add(0, 2);
-        add(1, 1);
-        add(1, 0);
-        add(0, 1);
-        add(0, 0);
-#pragma unroll
-        for (int i = 0; i < CH; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] += c[i][r];
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += c[r];
       }
       if constexpr (more) {       // the loads have had the first columns' products to arrive
-        constexpr int first = 2;
+        constexpr int first = 1;
         if (j >= first) {
           const int u = j - first;
           if (u < NA) sa.store(ra[u], u, ln, top_a);
@@ -264,7 +262,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
       }
     }
     if constexpr (more) {
-      constexpr int first = 2;
+      constexpr int first = 1;
 #pragma unroll
       for (int u = TN - first; u < NA + NB; ++u) {
         if (u < NA) sa.store(ra[u], u, ln, top_a);
@@ -296,10 +294,10 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   // what the largest elements of the whole block allow: see the head of the file
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
-    top_a = max(top_a, (uint32_t)__shfl_xor(top_a, d));
-    top_b = max(top_b, (uint32_t)__shfl_xor(top_b, d));
+    top_a = fmaxf(top_a, __shfl_xor(top_a, d));
+    top_b = fmaxf(top_b, __shfl_xor(top_b, d));
   }
-  uint32_t* tops = reinterpret_cast<uint32_t*>(lds[0]);      // (free: the last step ended with a barrier)
+  float* tops = reinterpret_cast<float*>(lds[0]);      // (free: the last step ended with a barrier)
   if (lane == 0) {
     tops[2 * wave] = top_a;
     tops[2 * wave + 1] = top_b;
@@ -307,10 +305,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < WM * WN; ++w) {
-    top_a = max(top_a, tops[2 * w]);
-    top_b = max(top_b, tops[2 * w + 1]);
+    top_a = fmaxf(top_a, tops[2 * w]);
+    top_b = fmaxf(top_b, tops[2 * w + 1]);
   }
-  const int ea = (int)(top_a >> 24) - 126, eb = (int)(top_b >> 24) - 126;       // |a| < 2^ea, |b| < 2^eb
+  auto exponent = [](float x) { return (int)(__builtin_bit_cast(uint32_t, x) >> 23) - 126; };
+  const int ea = exponent(top_a), eb = exponent(top_b);                           // |a| < 2^ea, |b| < 2^eb
   const int ek = 32 - __builtin_clz((uint32_t)(kend - kbeg));                      // K < 2^ek
   if (ea + kScaleLog > 127 || eb + kScaleLog > 127 || ea + eb + 2 * kScaleLog + ek + 1 > 127) {
     // elements or sums that could leave fp32's range: the tile again, on the fp32 instruction
@@ -341,25 +340,16 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_split(SplitParams p, c
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) put(i, j, acc[i][j], kUnscale);
+    for (int j = 0; j < TN; ++j) put(i, j, acc[i][j] + low[i][j], kUnscale);
 }
 
 template <typename F>
-void launch_as(const LaunchArgs& a, int threads, F kernel, const SplitParams& p) {
+void launch_as(const LaunchArgs& a, F kernel, const SplitParams& p) {
   const float* A = (const float*)a.A;
   const float* B = (const float*)a.B;
   float* C = (float*)a.C;
-  if (a.ev_start || a.ev_stop) hipExtLaunchKernelGGL(kernel, a.grid, dim3(threads), 0, a.stream, a.ev_start, a.ev_stop, 0, p, A, B, C);
-  else hipLaunchKernelGGL(kernel, a.grid, dim3(threads), 0, a.stream, p, A, B, C);
-}
-
-template <int WM, int WN, int TM, int TN>
-void launch_tile(const SplitParams& p, const LaunchArgs& a) {
-  constexpr int threads = 64 * WM * WN;
-  if (a.va && a.vb) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, true, true>, p);
-  else if (a.va) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, true, false>, p);
-  else if (a.vb) launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, false, true>, p);
-  else launch_as(a, threads, k_gemm_split<WM, WN, TM, TN, false, false>, p);
+  if (a.ev_start || a.ev_stop) hipExtLaunchKernelGGL(kernel, a.grid, dim3(NT), 0, a.stream, a.ev_start, a.ev_stop, 0, p, A, B, C);
+  else hipLaunchKernelGGL(kernel, a.grid, dim3(NT), 0, a.stream, p, A, B, C);
 }
 
 }  // namespace
@@ -368,8 +358,10 @@ namespace hg {
 namespace gemm {
 
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a) {
-  if (a.cfg == 0) launch_tile<4, 2, 2, 4>(p, a);
-  else launch_tile<2, 2, 2, 2>(p, a);
+  if (a.va && a.vb) launch_as(a, k_gemm_split<true, true>, p);
+  else if (a.va) launch_as(a, k_gemm_split<true, false>, p);
+  else if (a.vb) launch_as(a, k_gemm_split<false, true>, p);
+  else launch_as(a, k_gemm_split<false, false>, p);
 }
 
 }  // namespace gemm

@@ -17,7 +17,7 @@ def product(ctx, x, y, lay):
 
 def assert_close(out, x, y, k):
     """Sixteen products per rounded addition plus the roundings inside the sixteen and of the partial sums:
-    at most (K / 16 + 16) half-ulps of the sum of magnitudes; the three terms left out stay under 2^-25 of it."""
+    at most (K / 16 + 16) half-ulps of the sum of magnitudes; the three terms left out stay under 2^-24 of it."""
     x, y = x.astype(np.float64), y.astype(np.float64)
     bound = (k / 16 + 17) * 2.0 ** -24 * (np.abs(x) @ np.abs(y).T) + 1e-45
     assert np.all(np.abs(out.astype(np.float64) - x @ y.T) <= bound)
@@ -29,6 +29,29 @@ def test_ragged_shapes(gpu, m, n, k, lay):
     rng = np.random.default_rng(m + n + k)
     x, y = rng.standard_normal((m, k)).astype(np.float32), rng.uniform(0, 1, (n, k)).astype(np.float32)
     assert_close(product(gpu, x, y, lay).numpy(), x, y, k)
+
+
+@pytest.mark.parametrize("rest", [0.0, 2.0 ** -40])
+@pytest.mark.parametrize("lay", ["KK", "RR"])
+@pytest.mark.parametrize("diagonal", [False, True])
+def test_rows_with_one_dominating_product(gpu, diagonal, lay, rest):
+    """One rounding to fp32 and the three terms left out: 2 units of 2^-24 of the product.  The five small terms, at
+    most 2^-7 of it, lose less than 2^-23 of themselves in each of five additions: 0.1 more with the tiny products."""
+    m, n, k = 300, 280, 1040
+    rng = np.random.default_rng(13)
+    x, y = (rng.standard_normal((r, k)) * rest for r in (m, n))
+    if diagonal:        # a matrix with a few large entries, one to a row, times an ordinary one
+        x[np.arange(m), np.arange(m) * 3] = rng.uniform(1, 2, m)
+        y = rng.standard_normal((n, k))
+    else:
+        x[:, 5], y[:, 5] = rng.uniform(1, 2, m), rng.uniform(1, 2, n)
+    x, y = x.astype(np.float32), y.astype(np.float32)
+    out, xd, yd = product(gpu, x, y, lay).numpy(), x.astype(np.float64), y.astype(np.float64)
+    mag = np.abs(xd) @ np.abs(yd).T
+    top = np.abs(xd).max(1)[:, None] * np.abs(yd)[:, np.arange(m) * 3].T if diagonal else mag
+    rows = top >= mag * (1 - 2.0 ** -20)     # (where the ordinary matrix holds something small the rest counts)
+    assert np.count_nonzero(rows) > 0.95 * rows.size
+    assert np.all(np.abs(out - xd @ yd.T)[rows] <= 2.1 * 2.0 ** -24 * mag[rows])
 
 
 @pytest.mark.parametrize("scale", [1e-35, 1e-30, 1e30, 1.5e38])
