@@ -142,6 +142,19 @@ struct Side {
   }
 };
 
+// Four consecutive k of one row from k on; zeros from kend on.
+template <bool KC>
+__device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, uint32_t ks, int k, bool whole, int kend, float* v) {
+  if (KC && whole) {
+    const f4u x = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(rsrc, row + k * ks, 0, 0));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = x[u];
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, k + u < kend ? row + (k + u) * ks : 0xfffffff0u, 0, 0));
+  }
+}
+
 template <bool AKC, bool BKC>
 __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
   constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 32 x 32 blocks of each
@@ -312,29 +325,52 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
   const int ea = exponent(top_a), eb = exponent(top_b);                           // |a| < 2^ea, |b| < 2^eb
   const int ek = 32 - __builtin_clz((uint32_t)(kend - kbeg));                      // K < 2^ek
   if (ea + kScaleLog > 127 || eb + kScaleLog > 127 || ea + eb + 2 * kScaleLog + ek + 1 > 127) {
-    // elements or sums that could leave fp32's range: the tile again, on the fp32 instruction
-#pragma unroll 1
-    for (int ij = 0; ij < TM * TN; ++ij) {
-      const int i = ij / TN, j = ij - i * TN;
-      const int rowa = m0 + (wm * TM + i) * 32 + (lane & 31), rowb = n0 + (wn * TN + j) * 32 + (lane & 31);
-      const uint32_t ga = (uint32_t)(rowa < p.M ? rowa : p.M - 1) * p.sam, gb = (uint32_t)(rowb < p.N ? rowb : p.N - 1) * p.sbn;
-      f16v c;
+    // elements or sums that could leave fp32's range: the tile again, on the fp32 instruction.  Fragments come straight from
+    // memory, eight k ahead (bound by their loads where those run along the rows); each serves a wavefront's whole
+    // row or column of blocks.  2048 x 8192 over 2048, one infinity / one in every tile: 930 / 1080 us (2380 for one
+    // with a block of 32 x 32 at a time and single elements loaded; 600-640 on the fp32 instruction from the start).
+    uint32_t ga[TM], gb[TN];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) c[r] = 0;
-#pragma unroll 1
-      for (int k0 = kbeg; k0 < kend; k0 += 8) {
-        float fa[4], fb[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = k0 + 2 * u + (lane >> 5);
-          fa[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sa.rsrc, k < kend ? ga + k * sa.ks : 0xfffffff0u, 0, 0));
-          fb[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb.rsrc, k < kend ? gb + k * sb.ks : 0xfffffff0u, 0, 0));
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u], fb[u], c, 0, 0, 0);
-      }
-      put(i, j, c, 1.0f);
+    for (int i = 0; i < TM; ++i) {
+      const int row = m0 + (wm * TM + i) * 32 + (lane & 31);
+      ga[i] = (uint32_t)(row < p.M ? row : p.M - 1) * p.sam;
     }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int row = n0 + (wn * TN + j) * 32 + (lane & 31);
+      gb[j] = (uint32_t)(row < p.N ? row : p.N - 1) * p.sbn;
+    }
+    struct Frag { float a[TM][4], b[TN][4]; };
+    auto fetch8 = [&](int k0, Frag& f) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) four<AKC>(sa.rsrc, ga[i], sa.ks, k0 + 4 * (lane >> 5), k0 + 8 <= kend, kend, f.a[i]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) four<BKC>(sb.rsrc, gb[j], sb.ks, k0 + 4 * (lane >> 5), k0 + 8 <= kend, kend, f.b[j]);
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    Frag now, next;
+    fetch8(kbeg, now);
+#pragma unroll 1
+    for (int k0 = kbeg; k0 < kend; k0 += 8) {
+      fetch8(k0 + 8, next);                 // (behind the end: zeros, without a fetch)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(now.a[i][u], now.b[j][u], acc[i][j], 0, 0, 0);
+      now = next;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) put(i, j, acc[i][j], 1.0f);
     return;
   }
 #pragma unroll
