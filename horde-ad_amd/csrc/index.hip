@@ -387,82 +387,113 @@ hipError_t scatter_sorted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, i
 // ---- scatter-add by counting -------------------------------------------------
 // Up to 2^20 positions into a table whose cells are hit a few hundred times on average: instead of
 // sorting all positions by destination, count the hits of every cell, hand every cell a stretch of `val`,
-// drop the positions there in any order, and let the lanes that add up a cell put its few positions in
-// ascending order first.  Five short passes over 4-byte words (M positions, C cells) replace the ten launches
+// drop the positions there in any order, and put each cell's few positions in ascending order where they are
+// added up.  Short passes over 4-byte words (M positions, C cells) replace the ten launches
 // of a radix or merge sort of (key, position) pairs, and the pass that adds up writes every cell, empty ones
 // too, so that the result is not cleared beforehand.  100,000 rows of 512 bytes into 20,000 cells: 134 us with
-// the sort, 37 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
+// the sort, 35 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
 // position gets varies from run to run, the sums do not.
-constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (beyond, a run that a whole block adds up could hold too large a share of the work)
+// A cell may be hit far more often than the average (a padding index): its run is put in order by a block of its own
+// and its segments of kSeg entries are added up wherever there is room, as after the sort.  Half of those 100,000 picks
+// on one row: 1470 us with the sort, 4750 with one block per long run, 108 so.
+constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (a bit for each fits the LDS of a CU: k_cell_order)
 constexpr int64_t kCountedPerCell = 512;
-constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; longer runs: k_cell_big
-constexpr int kBigList = 8192;       // positions of one run that k_cell_big orders in LDS; longer runs: found in order by reading all of cell[]
+constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; longer runs: k_cell_order
 
 // cell[m] = position m's destination (or ~0: skipped), rank[m] = how many positions of that cell counted before it.
-// Lanes of a wavefront that go to one cell count with one addition (twice, for the commonest cells of a skewed table).
-__global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, uint32_t* __restrict__ counts, uint32_t* __restrict__ cell, uint32_t* __restrict__ rank) {
-  const int64_t step = (int64_t)gridDim.x * kBlock;
-  const int lane = threadIdx.x & 63;
-  for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63); base < M; base += step) {
-    const int64_t m = base + lane;
-    int64_t toff = 0, doff;
-    const bool ok = m < M && resolve(sp, m, &toff, &doff);
-    const uint32_t c = ok ? (uint32_t)toff : 0xffffffffu;
-    uint32_t r = 0;
-    bool todo = ok;
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const unsigned long long open = __ballot(todo);
-      if (!open) break;
-      const int first = __ffsll((long long)open) - 1;
-      const uint32_t c0 = __shfl(c, first);
-      const unsigned long long same = __ballot(todo && c == c0);
-      uint32_t b = 0;
-      if (lane == first) b = atomicAdd(&counts[c0], (uint32_t)__popcll(same));
-      b = __shfl(b, first);
-      if (todo && c == c0) {
-        r = b + (uint32_t)__popcll(same & ((1ull << lane) - 1));
-        todo = false;
-      }
-    }
-    if (todo) r = atomicAdd(&counts[c], 1u);
-    if (m < M) {
-      cell[m] = c;
-      rank[m] = r;
-    }
+// A block counts its positions among themselves first, in a table of LDS (open addressing, twice as many slots
+// as positions), and then adds each cell's count to the table of all with one atomic: addresses that many positions share are
+// asked once a block (2^20 positions, all in 128 cells: 757 us with one atomic for a wavefront's equal cells, 95 us so).
+constexpr int kCountRounds = 16;     // positions of a lane, at most
+__global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, int rounds, uint32_t* __restrict__ counts, uint32_t* __restrict__ cell, uint32_t* __restrict__ rank) {
+  constexpr int kSlots = 2 * kCountRounds * kBlock, kPlaceBits = 13;
+  static_assert(kSlots <= 1 << kPlaceBits && kCountRounds * kBlock <= 1 << (32 - kPlaceBits), "a slot and a count in a word");
+  __shared__ uint32_t key[kSlots], cnt[kSlots], place[kCountRounds * kBlock];
+  const int t = threadIdx.x, slots = 2 * rounds * kBlock;        // (rounds is a power of two)
+  for (int i = t; i < slots; i += kBlock) {
+    key[i] = 0xffffffffu;
+    cnt[i] = 0;
   }
+  __syncthreads();
+  const int64_t m0 = (int64_t)blockIdx.x * rounds * kBlock;
+  const int here = M - m0 < (int64_t)rounds * kBlock ? (int)(M - m0) : rounds * kBlock;
+  for (int i = t; i < here; i += kBlock) {
+    int64_t toff = 0, doff;
+    const bool ok = resolve(sp, m0 + i, &toff, &doff);
+    const uint32_t c = ok ? (uint32_t)toff : 0xffffffffu;
+    cell[m0 + i] = c;
+    place[i] = 0xffffffffu;
+    if (!ok) continue;
+    uint32_t q = (c * 0x9e3779b1u) >> 8 & (uint32_t)(slots - 1);
+    for (;;) {                       // (at most half of the slots are taken: ends)
+      const uint32_t was = atomicCAS(&key[q], 0xffffffffu, c);
+      if (was == 0xffffffffu || was == c) break;
+      q = (q + 1) & (uint32_t)(slots - 1);
+    }
+    place[i] = atomicAdd(&cnt[q], 1u) << kPlaceBits | q;
+  }
+  __syncthreads();
+  for (int i = t; i < slots; i += kBlock)
+    if (key[i] != 0xffffffffu) cnt[i] = atomicAdd(&counts[key[i]], cnt[i]);
+  __syncthreads();
+  for (int i = t; i < here; i += kBlock)
+    if (place[i] != 0xffffffffu) rank[m0 + i] = cnt[place[i] & (kSlots - 1)] + (place[i] >> kPlaceBits);
 }
 
-// Where each cell's stretch of val starts: the cells of a block side by side, the blocks in any order (globals[0] is
-// the next free place).  Cells with long runs are listed (globals[1] of them).
+// Totals made on the way, cleared beforehand.
+struct CellTotals {
+  uint32_t placed;       // next free place of val
+  uint32_t runs;         // long runs listed
+  uint32_t segments;     // segments of kSeg entries of theirs
+  uint32_t parts;        // those that belong to runs of several segments
+};
+// A run of more than kSmallRun entries: its cell, its first segment, and the first row of the partial sums where it has several.
+struct LongRun { uint32_t cell, segment, part; };
+
+// Where each cell's stretch of val starts: the cells of a block side by side, the blocks in any order.  The totals are
+// drawn from once a block.
 constexpr int kCellsPerBlock = 1024;
-__global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_t* __restrict__ counts, uint32_t* __restrict__ starts, uint32_t* __restrict__ globals, uint32_t* __restrict__ big) {
-  __shared__ uint32_t sums[kBlock];
-  __shared__ uint32_t base;
+__global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_t* __restrict__ counts, uint32_t* __restrict__ starts, CellTotals* __restrict__ totals, LongRun* __restrict__ runs) {
+  __shared__ uint32_t sums[4][kBlock];
+  __shared__ uint32_t base[4];
   const int t = threadIdx.x;
   const int64_t c0 = (int64_t)blockIdx.x * kCellsPerBlock + 4 * t;
-  uint32_t n[4], total = 0;
+  uint32_t n[4], own[4] = {0, 0, 0, 0};        // entries, long runs, segments, partial sums
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     n[i] = c0 + i < C ? counts[c0 + i] : 0;
-    total += n[i];
+    const uint32_t segs = (n[i] + kSeg - 1) / kSeg;
+    own[0] += n[i];
+    if (n[i] > kSmallRun) { own[1] += 1; own[2] += segs; own[3] += segs > 1 ? segs : 0; }
   }
-  sums[t] = total;
+  const bool any = __syncthreads_or(own[1] != 0);
+  const int kinds = any ? 4 : 1;
+  for (int k = 0; k < kinds; ++k) sums[k][t] = own[k];
   __syncthreads();
   for (int d = 1; d < kBlock; d <<= 1) {
-    const uint32_t v = t >= d ? sums[t - d] : 0;
+    uint32_t v[4];
+    for (int k = 0; k < kinds; ++k) v[k] = t >= d ? sums[k][t - d] : 0;
     __syncthreads();
-    sums[t] += v;
+    for (int k = 0; k < kinds; ++k) sums[k][t] += v[k];
     __syncthreads();
   }
-  if (t == kBlock - 1) base = atomicAdd(&globals[0], sums[t]);
+  if (t < kinds) base[t] = atomicAdd(reinterpret_cast<uint32_t*>(totals) + t, sums[t][kBlock - 1]);
   __syncthreads();
-  uint32_t at = base + sums[t] - total;
+  uint32_t at = base[0] + sums[0][t] - own[0];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (c0 + i < C) starts[c0 + i] = at;
     at += n[i];
-    if (n[i] > kSmallRun) big[atomicAdd(&globals[1], 1u)] = (uint32_t)(c0 + i);
+  }
+  if (own[1] == 0) return;
+  uint32_t run = base[1] + sums[1][t] - own[1], segment = base[2] + sums[2][t] - own[2], part = base[3] + sums[3][t] - own[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (n[i] <= kSmallRun) continue;
+    const uint32_t segs = (n[i] + kSeg - 1) / kSeg;
+    runs[run++] = LongRun{(uint32_t)(c0 + i), segment, segs > 1 ? part : 0};
+    segment += segs;
+    if (segs > 1) part += segs;
   }
 }
 
@@ -474,25 +505,213 @@ __global__ void __launch_bounds__(kBlock) k_cell_place(int64_t M, const uint32_t
   }
 }
 
+// Puts the positions of the long runs in ascending order, in place, and notes the run of each segment.  A run of one
+// segment: a wavefront, every entry's rank by comparison with the others.  A longer one: a block, a bit of LDS per
+// position (BITS of them, M at most), set for the run's and read off in order -- the work grows with n + M / 32, which
+// beats sorting networks from a few hundred entries on and does not know a longest run.  A quarter of all positions and
+// more: the block goes through cell[] twice, counting and writing.  The words of 32 bits stand 33 to 32 so that lanes that
+// read 32 of them each hit different banks.
+constexpr int kOrderThreads = 1024;
+template <int BITS>
+__global__ void __launch_bounds__(kOrderThreads) k_cell_order(int64_t M, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts, const CellTotals* __restrict__ totals,
+                                                              const LongRun* __restrict__ runs, const uint32_t* __restrict__ cell, uint32_t* val, uint32_t* __restrict__ segment_run) {
+  constexpr int kWaves = kOrderThreads / 64, kWords = BITS / 32 + BITS / 1024;
+  static_assert(kWords >= kWaves * kSeg, "a run of one segment per wavefront");
+  __shared__ uint32_t lds[kWords];
+  __shared__ uint32_t sums[kWaves];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t n_runs = totals->runs;
+  uint32_t* mine = lds + wave * kSeg;
+  for (uint32_t i = blockIdx.x * kWaves + wave; i < n_runs; i += gridDim.x * kWaves) {
+    const LongRun run = runs[i];
+    const uint32_t n = counts[run.cell];
+    if (n > kSeg) continue;
+    uint32_t* at = val + starts[run.cell];
+    for (uint32_t e = lane; e < kSeg; e += 64) mine[e] = e < n ? at[e] : 0xffffffffu;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t p[kSeg / 64], r[kSeg / 64];
+#pragma unroll
+    for (int q = 0; q < kSeg / 64; ++q) { p[q] = mine[lane + 64 * q]; r[q] = 0; }
+    for (uint32_t d = 0; d < n; ++d) {
+      const uint32_t x = mine[d];
+#pragma unroll
+      for (int q = 0; q < kSeg / 64; ++q) r[q] += x < p[q] ? 1 : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < kSeg / 64; ++q)
+      if (lane + 64 * q < n) at[r[q]] = p[q];
+    if (lane == 0) segment_run[run.segment] = i;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  const int share = (int)((M + kOrderThreads - 1) / kOrderThreads) * 64;      // positions of a wavefront
+  const int words = (int)((M + 31) / 32), per = (words + kOrderThreads - 1) / kOrderThreads;
+  auto word_at = [](int w) { return w + (w >> 5); };
+  for (uint32_t i = blockIdx.x; i < n_runs; i += gridDim.x) {
+    const LongRun run = runs[i];
+    const uint32_t n = counts[run.cell];
+    if (n <= kSeg) continue;                                  // (the same for the whole block)
+    uint32_t* at = val + starts[run.cell];
+    for (uint32_t g = t; g < (n + kSeg - 1) / kSeg; g += kOrderThreads) segment_run[run.segment + g] = i;
+    if ((int64_t)n * 4 >= M) {
+      const int p0 = wave * share, p1 = (int64_t)p0 + share < M ? p0 + share : (int)M;
+      uint32_t o = 0;
+      for (int pass = 0; pass < 2; ++pass) {
+        for (int p = p0; p < p1; p += 8 * 64) {
+          uint32_t c[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) c[q] = p + 64 * q + lane < p1 ? cell[p + 64 * q + lane] : 0xffffffffu;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const unsigned long long hit = __ballot(c[q] == run.cell);
+            if (pass == 1 && c[q] == run.cell) at[o + (uint32_t)__popcll(hit & ((1ull << lane) - 1))] = (uint32_t)(p + 64 * q + lane);
+            o += (uint32_t)__popcll(hit);
+          }
+        }
+        if (pass == 1) break;
+        if (lane == 0) sums[wave] = o;
+        __syncthreads();
+        o = 0;
+        for (int w = 0; w < wave; ++w) o += sums[w];
+      }
+      __syncthreads();
+      continue;
+    }
+    for (int w = t; w < words; w += kOrderThreads) lds[word_at(w)] = 0;
+    __syncthreads();
+    for (uint32_t e = t; e < n; e += 4 * kOrderThreads) {
+      uint32_t p[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) p[q] = e + q * kOrderThreads < n ? at[e + q * kOrderThreads] : at[e];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) atomicOr(&lds[word_at((int)(p[q] >> 5))], 1u << (p[q] & 31));
+    }
+    __syncthreads();
+    uint32_t total = 0;
+    for (int w = t * per; w < (t + 1) * per && w < words; ++w) total += (uint32_t)__popc(lds[word_at(w)]);
+    uint32_t scan = total;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up(scan, d);
+      if (lane >= d) scan += v;
+    }
+    if (lane == 63) sums[wave] = scan;
+    __syncthreads();
+    uint32_t o = scan - total;
+    for (int w = 0; w < wave; ++w) o += sums[w];
+    for (int w = t * per; w < (t + 1) * per && w < words; ++w)
+      for (uint32_t bits = lds[word_at(w)]; bits; bits &= bits - 1) at[o++] = (uint32_t)(32 * w) + (uint32_t)(__ffs((int)bits) - 1);
+    __syncthreads();
+  }
+}
+
 template <typename T, int V> struct UnitOf { using type = T __attribute__((ext_vector_type(V), aligned(sizeof(T)))); };
 template <typename T> struct UnitOf<T, 1> { using type = T; };
 
-// A group of G lanes (8 to 64) per cell: its positions go to LDS, every lane finds the ranks of its share of them, and
-// then the lanes run along the cell's N elements (V at a time) and add the positions' slices in ascending order,
-// four loads in flight.
+// Adds the slices of `n` positions, in the order of `list`, to acc, F loads in flight.
+template <typename U, int F, typename T>
+__device__ __forceinline__ U add_positions(const IxSpace& sp, U acc, const uint32_t* list, uint32_t n, const T* __restrict__ from) {
+  uint32_t j = 0;
+  for (; j + F <= n; j += F) {
+    U x[F];
+#pragma unroll
+    for (int q = 0; q < F; ++q) x[q] = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + q]));
+#pragma unroll
+    for (int q = 0; q < F; ++q) acc = (U)(acc + x[q]);
+  }
+  for (; j < n; ++j) acc = (U)(acc + *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])));
+  return acc;
+}
+
+// Everything the last pass reads besides its operands.
+struct CellLists {
+  const uint32_t *counts, *starts, *val;
+  const CellTotals* totals;
+  const LongRun* runs;
+  const uint32_t* segment_run;
+  uint32_t* tickets;       // one per row of partial sums and piece of G units (those of a run's first row are used)
+  void* parts;             // [rows][N]
+};
+
+// A group of G lanes (8 to 64) per piece of work, a lane per unit of V elements.
+// First the segments of the long runs, a piece for every G units of each: a segment's slices are added front to back, eight
+// loads in flight (their positions come through LDS: 115 us for one segment of rows of 512 bytes when every round of
+// loads waited for its positions).  The sum of a run's only segment is the result; of several, whoever finishes the last adds the sums
+// in ascending order (the sums are written, a fence, a ticket; runs of several segments are rare enough for fences).
+// Then the cells, each in `stretches` pieces: the positions go to LDS, every lane finds the ranks of its share of them, and then the
+// lanes run along the piece and add the positions' slices in ascending order, four loads in flight.
 template <typename T, int V>
-__global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts,
-                                                     const uint32_t* __restrict__ val, const T* __restrict__ src, T* __restrict__ out) {
+__global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, int64_t stretches, CellLists in, const T* __restrict__ src, T* __restrict__ out) {
   using U = typename UnitOf<T, V>::type;
-  __shared__ uint32_t raw_all[kBlock / 8][kSmallRun], list_all[kBlock / 8][kSmallRun];
-  const int g = threadIdx.x / G, l = threadIdx.x % G;
-  uint32_t* raw = raw_all[g];
-  uint32_t* list = list_all[g];
-  const int64_t units = N / V, step = (int64_t)gridDim.x * (kBlock / G);
-  for (int64_t c = (int64_t)blockIdx.x * (kBlock / G) + g; c < C; c += step) {
-    const uint32_t n = counts[c];
+  constexpr int kList = 2 * kSmallRun;
+  __shared__ uint32_t lists[kBlock / 8][kList];
+  __shared__ bool last[kBlock / 8];
+  const int g = threadIdx.x / G, l = threadIdx.x % G, groups = kBlock / G;
+  uint32_t* list = lists[g];
+  const int64_t units = N / V, step = (int64_t)gridDim.x * groups;
+  auto element = [&](int64_t u) {
+    int64_t io[1] = {u * V};
+    if constexpr (V == 1) decompose<1>(inner, u, io);
+    return io[0];
+  };
+  {
+    const int64_t pieces = (units + G - 1) / G, items = (int64_t)in.totals->segments * pieces;
+    for (int64_t base = (int64_t)blockIdx.x * groups; base < items; base += step) {
+      const bool ok = base + g < items;
+      const int64_t seg = ok ? (base + g) / pieces : 0, piece = ok ? base + g - seg * pieces : 0, u = piece * G + l;
+      const LongRun run = in.runs[ok ? in.segment_run[seg] : 0];
+      const uint32_t n = in.counts[run.cell], segs = (n + kSeg - 1) / kSeg, at = (uint32_t)(seg - run.segment);
+      const bool live = ok && u < units, several = ok && segs > 1;
+      U* result = reinterpret_cast<U*>(out + (int64_t)run.cell * N + u * V);
+      U* part = reinterpret_cast<U*>((T*)in.parts + (int64_t)run.part * N + u * V);
+      const uint32_t* mine = in.val + in.starts[run.cell] + at * kSeg;
+      const uint32_t len = !ok ? 0 : n - at * kSeg < (uint32_t)kSeg ? n - at * kSeg : (uint32_t)kSeg;
+      const T* from = src + (live ? element(u) : 0);
+      U acc{};
+      for (uint32_t e0 = 0; e0 < len; e0 += kList) {
+        const uint32_t m = len - e0 < (uint32_t)kList ? len - e0 : (uint32_t)kList;
+        for (uint32_t e = l; e < m; e += G) list[e] = mine[e0 + e];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live) acc = add_positions<U, 8>(sp, acc, list, m, from);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (live) {
+        if (several) part[(int64_t)at * units] = acc;
+        else *result = acc;
+      }
+      if (!__syncthreads_or(several)) continue;
+      __threadfence();
+      __syncthreads();
+      if (l == 0) last[g] = several && atomicAdd(&in.tickets[(int64_t)run.part * pieces + piece], 1u) == segs - 1;
+      __syncthreads();
+      if (last[g] && live) {
+        __threadfence();
+        acc = part[0];
+        uint32_t j = 1;
+        for (; j + 8 <= segs; j += 8) {
+          U x[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) x[q] = part[(int64_t)(j + q) * units];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) acc = (U)(acc + x[q]);
+        }
+        for (; j < segs; ++j) acc = (U)(acc + part[(int64_t)j * units]);
+        *result = acc;
+      }
+      __syncthreads();
+    }
+  }
+  const int64_t len = (units + stretches - 1) / stretches;
+  for (int64_t i = (int64_t)blockIdx.x * groups + g; i < C * stretches; i += step) {
+    const int64_t c = stretches == 1 ? i : i / stretches, u0 = (i - c * stretches) * len, u1 = u0 + len < units ? u0 + len : units;
+    const uint32_t n = in.counts[c];
     if (n > kSmallRun) continue;
-    const uint32_t* mine = val + starts[c];
+    const uint32_t* mine = in.val + in.starts[c];
+    uint32_t *raw = list, *sorted = list + kSmallRun;
     for (uint32_t e = l; e < n; e += G) raw[e] = mine[e];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -500,191 +719,71 @@ __global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int
       const uint32_t p = raw[e];
       uint32_t r = 0;
       for (uint32_t d = 0; d < n; ++d) r += raw[d] < p ? 1 : 0;
-      list[r] = p;
+      sorted[r] = p;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    for (int64_t u = l; u < units; u += G) {
-      int64_t io[1] = {u * V};
-      if constexpr (V == 1) decompose<1>(inner, u, io);
-      const T* from = src + io[0];
-      U acc{};
-      uint32_t j = 0;
-      for (; j + 4 <= n; j += 4) {
-        const U a = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])), b = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 1]));
-        const U d = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 2])), e = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + 3]));
-        acc = (U)(acc + a);
-        acc = (U)(acc + b);
-        acc = (U)(acc + d);
-        acc = (U)(acc + e);
-      }
-      for (; j < n; ++j) acc = (U)(acc + *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])));
-      *reinterpret_cast<U*>(out + c * N + u * V) = acc;
-    }
+    for (int64_t u = u0 + l; u < u1; u += G)
+      *reinterpret_cast<U*>(out + c * N + u * V) = add_positions<U, 4>(sp, U{}, sorted, n, src + element(u));
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
 }
 
-// Cells hit more than kSmallRun times, a block for each: the positions in ascending order (sorted in LDS, or, for a
-// run that does not fit there, met in order by going through cell[]), cut into segments of kSeg, the lanes
-// sharing segments and elements between them, segment sums added in ascending order.
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_cell_big(IxSpace sp, Dims inner, int64_t M, int64_t N, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts,
-                                                     const uint32_t* __restrict__ val, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ globals,
-                                                     const uint32_t* __restrict__ big, const T* __restrict__ src, T* __restrict__ out) {
-  __shared__ uint32_t list[kBigList];
-  __shared__ T red[kBlock];
-  __shared__ uint32_t wave_n[8][4];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const uint32_t n_big = globals[1];
-  for (uint32_t i = blockIdx.x; i < n_big; i += gridDim.x) {
-    const uint32_t c = big[i], n = counts[c];
-    const bool fits = n <= (uint32_t)kBigList;
-    if (fits) {
-      const uint32_t* mine = val + starts[c];
-      uint32_t P = 2 * kSmallRun;
-      while (P < n) P <<= 1;
-      for (uint32_t e = t; e < P; e += kBlock) list[e] = e < n ? mine[e] : 0xffffffffu;
-      for (uint32_t k = 2; k <= P; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-          __syncthreads();
-          for (uint32_t q = t; q < P / 2; q += kBlock) {
-            const uint32_t a = (q / j) * 2 * j + q % j, b = a + j;
-            const uint32_t x = list[a], y = list[b];
-            if ((x > y) == ((a & k) == 0)) {
-              list[a] = y;
-              list[b] = x;
-            }
-          }
-        }
-      __syncthreads();
-    }
-    for (int64_t n0 = 0; n0 < N; n0 += kBlock) {
-      const int nc = (int)(N - n0 < kBlock ? N - n0 : kBlock), R = kBlock / nc;
-      const int seg = t / nc, col = t - seg * nc;
-      int64_t io[1] = {0};
-      if (seg < R) decompose<1>(inner, n0 + col, io);
-      const T* from = src + io[0];
-      T tot = T(0);
-      bool have = false;
-      auto add_list = [&](uint32_t cnt) {      // list[0 .. cnt) starts a segment
-        const uint32_t segs = (cnt + kSeg - 1) / kSeg;
-        for (uint32_t g0 = 0; g0 < segs; g0 += R) {
-          T acc = T(0);
-          const uint32_t me = g0 + seg;
-          if (seg < R && me < segs) {
-            const uint32_t e1 = me * kSeg + kSeg < cnt ? me * kSeg + kSeg : cnt;
-            uint32_t j = me * kSeg;
-            for (; j + 4 <= e1; j += 4) {
-              const T a = from[data_offset(sp, (int64_t)list[j])], b = from[data_offset(sp, (int64_t)list[j + 1])];
-              const T d = from[data_offset(sp, (int64_t)list[j + 2])], e = from[data_offset(sp, (int64_t)list[j + 3])];
-              acc = (T)(acc + a);
-              acc = (T)(acc + b);
-              acc = (T)(acc + d);
-              acc = (T)(acc + e);
-            }
-            for (; j < e1; ++j) acc = (T)(acc + from[data_offset(sp, (int64_t)list[j])]);
-          }
-          red[t] = acc;
-          __syncthreads();
-          if (t < nc)
-            for (int r = 0; r < R && g0 + r < segs; ++r) {
-              const T v = red[r * nc + t];
-              tot = have ? (T)(tot + v) : v;
-              have = true;
-            }
-          __syncthreads();
-        }
-      };
-      if (fits) {
-        add_list(n);
-      } else {
-        uint32_t held = 0;
-        for (int64_t m0 = 0; m0 < M; m0 += 8 * kBlock) {
-          bool is[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int64_t m = m0 + j * kBlock + t;
-            is[j] = m < M && cell[m] == c;
-            const unsigned long long b = __ballot(is[j]);
-            if (lane == 0) wave_n[j][wave] = (uint32_t)__popcll(b);
-          }
-          __syncthreads();
-          uint32_t at = held;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const unsigned long long b = __ballot(is[j]);
-            uint32_t before = at;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const uint32_t k = wave_n[j][w];
-              if (w < wave) before += k;
-              at += k;
-            }
-            if (is[j]) list[before + (uint32_t)__popcll(b & ((1ull << lane) - 1))] = (uint32_t)(m0 + j * kBlock + t);
-          }
-          held = at;
-          __syncthreads();
-          if (held > (uint32_t)(kBigList - 8 * kBlock)) {      // no room for another round: add the whole segments
-            const uint32_t whole = held / kSeg * kSeg, rest = held - whole;
-            add_list(whole);
-            const uint32_t keep = t < (int)rest ? list[whole + t] : 0;
-            __syncthreads();
-            if (t < (int)rest) list[t] = keep;
-            held = rest;
-            __syncthreads();
-          }
-        }
-        add_list(held);
-      }
-      if (t < nc) out[(int64_t)c * N + n0 + t] = tot;
-    }
-    __syncthreads();
-  }
-}
-
-// k_cell_count -> k_cell_starts -> k_cell_place -> k_cell_sum, k_cell_big.  sp's table strides are in slices; every
+// k_cell_count -> k_cell_starts -> k_cell_place -> k_cell_order -> k_cell_sum.  sp's table strides are in slices; every
 // element of o is written.
 hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, int64_t M, int64_t N, int64_t C, const hgpu_array* src, hgpu_array* o, int* rc_out) {
-  const int64_t n_big = M / (kSmallRun + 1) + 1;
+  const size_t es = dtype_size(src->dtype);
+  // 16-byte units when the slices are contiguous and every one starts on a boundary of its elements
+  const bool contiguous = inner.nd == 1 && (inner.st[0][0] == 1 || N == 1);
+  const int V = es >= 4 && (src->dtype == HGPU_F64 || src->dtype == HGPU_F32) && contiguous && N % (int64_t)(16 / es) == 0 ? (int)(16 / es) : 1;
+  const int64_t units = N / V;
+  int G = 8;
+  while (G < 64 && G < units) G <<= 1;
+  const int64_t stretches = 1;
+  const int64_t max_runs = M / (kSmallRun + 1) + 1, max_segments = M / kSeg + max_runs;
+  const int64_t max_parts = M > kSeg ? M / kSeg + M / (kSeg + 1) + 1 : 0;       // (a run of several segments has more than kSeg entries)
+  const int64_t pieces = (units + G - 1) / G, n_tickets = max_parts * pieces;
+  const int64_t head = (C + 4 + n_tickets + 3) / 4 * 4;        // counters, totals, tickets: cleared together
+  const int64_t words = (head + C + 3 * M + 3 * max_runs + max_segments + 3) / 4 * 4;
   hgpu_buffer* wb = nullptr;
-  const int64_t head = (C + 2 + 3) / 4 * 4;        // counters and the two globals, cleared together
-  *rc_out = buffer_alloc(ctx, (size_t)(head + C + 3 * M + n_big) * 4, &wb);
+  *rc_out = buffer_alloc(ctx, (size_t)words * 4 + (size_t)(max_parts * N) * es, &wb);
   if (*rc_out) return hipSuccess;
   uint32_t* counts = (uint32_t*)wb->ptr;
-  uint32_t* globals = counts + C;
+  CellTotals* totals = (CellTotals*)(counts + C);
   uint32_t* starts = counts + head;
   uint32_t* cell = starts + C;
   uint32_t* rank = cell + M;
   uint32_t* val = rank + M;
-  uint32_t* big = val + M;
-  const size_t es = dtype_size(src->dtype);
+  LongRun* runs = (LongRun*)(val + M);
+  uint32_t* segment_run = val + M + 3 * max_runs;
   *rc_out = zero_fill(ctx, counts, (size_t)head * 4);
   if (*rc_out) { buffer_release(wb); return hipSuccess; }
   LaunchGuard lg(ctx, "scatter_counted", 2.0 * M * N * es + 8.0 * M * sp.n_ix, (double)M * N);
   const unsigned gm = grid_for(M, kBlock, ctx->num_cu * 8);
-  hipLaunchKernelGGL(k_cell_count, dim3(gm), dim3(kBlock), 0, ctx->stream, sp, M, counts, cell, rank);
-  hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, globals, big);
+  int rounds = 1;                                              // positions of a lane: as many as leave every CU two blocks
+  while (rounds < kCountRounds && (int64_t)rounds * kBlock * ctx->num_cu * 2 < M) rounds <<= 1;
+  const unsigned gk = (unsigned)((M + (int64_t)rounds * kBlock - 1) / (rounds * kBlock));
+  hipLaunchKernelGGL(k_cell_count, dim3(gk), dim3(kBlock), 0, ctx->stream, sp, M, rounds, counts, cell, rank);
+  hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, totals, runs);
   hipLaunchKernelGGL(k_cell_place, dim3(gm), dim3(kBlock), 0, ctx->stream, M, (const uint32_t*)starts, (const uint32_t*)cell, (const uint32_t*)rank, val);
-  // 16-byte units when the slices are contiguous and every one starts on a boundary of its elements
-  const bool contiguous = inner.nd == 1 && (inner.st[0][0] == 1 || N == 1);
-  const int V = es >= 4 && (src->dtype == HGPU_F64 || src->dtype == HGPU_F32) && contiguous && N % (int64_t)(16 / es) == 0 ? (int)(16 / es) : 1;
-  int G = 8;
-  while (G < 64 && G < N / V) G <<= 1;
-  const unsigned gc = grid_for(C, kBlock / G, ctx->num_cu * 16);
-  if (V == 2)
-    hipLaunchKernelGGL((k_cell_sum<double, 2>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts, (const uint32_t*)val, (const double*)data_ptr(src), (double*)data_ptr(o));
-  else if (V == 4)
-    hipLaunchKernelGGL((k_cell_sum<float, 4>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts, (const uint32_t*)val, (const float*)data_ptr(src), (float*)data_ptr(o));
-  else
-    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_sum<T, 1>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, (const uint32_t*)counts, (const uint32_t*)starts,
-                                                        (const uint32_t*)val, (const T*)data_ptr(src), (T*)data_ptr(o)));
   if (M > kSmallRun) {
-    const unsigned gb = (unsigned)(n_big < ctx->num_cu * 2 ? n_big : ctx->num_cu * 2);
-    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_big<T>), dim3(gb), dim3(kBlock), 0, ctx->stream, sp, inner, M, N, (const uint32_t*)counts, (const uint32_t*)starts,
-                                                        (const uint32_t*)val, (const uint32_t*)cell, (const uint32_t*)globals, (const uint32_t*)big, (const T*)data_ptr(src), (T*)data_ptr(o)));
+    const unsigned go = (unsigned)std::min<int64_t>((max_runs + 15) / 16, ctx->num_cu);      // (most of the time nothing is long)
+    if (M <= (1 << 17))
+      hipLaunchKernelGGL((k_cell_order<1 << 17>), dim3(go), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs, (const uint32_t*)cell, val, segment_run);
+    else
+      hipLaunchKernelGGL((k_cell_order<kCountedPositions>), dim3(go), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs, (const uint32_t*)cell, val, segment_run);
   }
+  const CellLists in{counts, starts, val, totals, runs, segment_run, counts + C + 4, (char*)wb->ptr + words * 4};
+  // (blocks for the cells' pieces, or for the segments' where those are more)
+  const int64_t segment_items = M > kSmallRun ? (M / kSeg + 1) * pieces : 0;
+  const unsigned gc = grid_for(std::max(C * stretches, segment_items), kBlock / G, ctx->num_cu * 16);
+  if (V == 2)
+    hipLaunchKernelGGL((k_cell_sum<double, 2>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const double*)data_ptr(src), (double*)data_ptr(o));
+  else if (V == 4)
+    hipLaunchKernelGGL((k_cell_sum<float, 4>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const float*)data_ptr(src), (float*)data_ptr(o));
+  else
+    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_sum<T, 1>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const T*)data_ptr(src), (T*)data_ptr(o)));
   const hipError_t e = hipGetLastError();
   buffer_release(wb);
   return e;

@@ -58,3 +58,53 @@ def test_many_cells_and_two_index_dims(both):
     idx = both.upload(rng.integers(0, 700, 3000).astype(np.int64))
     g, o = both.scatter_add(wide.transpose([1, 0]), [idx], 1, [700]).numpy()
     assert np.array_equal(g, o)
+
+
+def in_segments(src, idx, cells):
+    """The sums in the documented order, with the type's own rounding: positions ascending, a run cut into segments of
+    256 entries that are added front to back, their sums added in ascending order."""
+    out = np.zeros((cells,) + src.shape[1:], src.dtype)
+    order = np.argsort(idx, kind="stable")
+    starts = np.searchsorted(idx[order], np.arange(cells + 1))
+    for c in range(cells):
+        rows = src[order[starts[c]:starts[c + 1]]]
+        sums = [np.add.accumulate(rows[i:i + 256], axis=0, dtype=src.dtype)[-1] for i in range(0, len(rows), 256)]
+        if sums:
+            out[c] = np.add.accumulate(np.stack(sums), axis=0, dtype=src.dtype)[-1]
+    return out
+
+
+def counted(gpu, src, idx, cells):
+    """The result and, the same again, the kernel family that made it."""
+    arr, ix = gpu.upload(src), [gpu.upload(idx)]
+    first = gpu.scatter_add(arr, ix, 1, [cells]).numpy()
+    gpu.profile(1)
+    again = gpu.scatter_add(arr, ix, 1, [cells]).numpy()
+    labels = list(gpu.profile_report())
+    gpu.profile(0)
+    assert "scatter_counted" in labels, labels
+    assert np.array_equal(first, again)
+    return first
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int8])
+@pytest.mark.parametrize("width", [1, 3, 40, 128, 301])
+@pytest.mark.parametrize("m,cells,hot", [(6000, 400, 1), (6000, 400, 3), (140000, 3000, 2)])
+def test_a_few_cells_take_half_of_the_hits(gpu, m, cells, hot, width, dt):
+    """A padding index: runs of thousands beside ordinary ones (and a table of bits of either size)."""
+    if m > 100000 and width > 40:
+        pytest.skip("the reference sums on the host")
+    rng = np.random.default_rng(width + hot)
+    idx = rng.integers(0, cells, m)
+    idx[: m // 2] = rng.integers(0, hot, m // 2) * 7
+    idx = rng.permutation(idx).astype(np.int64)
+    shape = (m,) if width == 1 else (m, width)
+    src = rng.integers(-100, 100, shape).astype(dt) if np.dtype(dt).kind == "i" else rng.standard_normal(shape).astype(dt)
+    assert np.array_equal(counted(gpu, src, idx, cells), in_segments(src, idx, cells))
+
+
+def test_all_positions_in_one_cell(gpu):
+    rng = np.random.default_rng(14)
+    m = 1 << 20
+    src, idx = rng.standard_normal(m).astype(np.float32), np.full(m, 2047, np.int64)
+    assert np.array_equal(counted(gpu, src, idx, 2048), in_segments(src, idx, 2048))
