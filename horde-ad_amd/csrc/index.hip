@@ -398,6 +398,7 @@ hipError_t scatter_sorted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, i
 // on one row: 1470 us with the sort, 4750 with one block per long run, 108 so.
 constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (a bit for each fits the LDS of a CU: k_cell_order)
 constexpr int64_t kCountedPerCell = 512;
+constexpr int64_t kCountedLeast = 1024;   // up to here the library sorts in one launch: 18.8 us submitted one after another against 21.4 by counting; from 1025 on 27 against 21.4
 constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; longer runs: k_cell_order
 
 // cell[m] = position m's destination (or ~0: skipped), rank[m] = how many positions of that cell counted before it.
@@ -640,7 +641,8 @@ struct CellLists {
 // loads in flight (their positions come through LDS: 115 us for one segment of rows of 512 bytes when every round of
 // loads waited for its positions).  The sum of a run's only segment is the result; of several, whoever finishes the last adds the sums
 // in ascending order (the sums are written, a fence, a ticket; runs of several segments are rare enough for fences).
-// Then the cells, each in `stretches` pieces: the positions go to LDS, every lane finds the ranks of its share of them, and then the
+// Then the cells, each in `stretches` pieces (more than one where few cells with wide slices would leave the
+// device idle): the positions go to LDS, every lane finds the ranks of its share of them, and then the
 // lanes run along the piece and add the positions' slices in ascending order, four loads in flight.
 template <typename T, int V>
 __global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, int64_t stretches, CellLists in, const T* __restrict__ src, T* __restrict__ out) {
@@ -740,7 +742,10 @@ hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, 
   const int64_t units = N / V;
   int G = 8;
   while (G < 64 && G < units) G <<= 1;
-  const int64_t stretches = 1;
+  // Pieces of a cell: as many as leave every lane four units, until the lanes fill the device.  (1500 slices of 120 KB into
+  // three cells: 434 us with the sort, 10.4 ms with a group of lanes per cell, 90 so.)
+  const int64_t room = ((int64_t)ctx->num_cu * 2048 + C * G - 1) / (C * G), longest = (units + 4 * G - 1) / (4 * G);
+  const int64_t stretches = std::max<int64_t>(1, std::min(room, longest));
   const int64_t max_runs = M / (kSmallRun + 1) + 1, max_segments = M / kSeg + max_runs;
   const int64_t max_parts = M > kSeg ? M / kSeg + M / (kSeg + 1) + 1 : 0;       // (a run of several segments has more than kSeg entries)
   const int64_t pieces = (units + G - 1) / G, n_tickets = max_parts * pieces;
@@ -938,7 +943,7 @@ int hgpu_scatter_add(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_
   int64_t C = 1;
   for (int i = 0; i < n_ix; ++i) C *= shp[i];
   // (more cells than eight to a position: passes over the cells would outweigh those over the positions)
-  const bool counted = (flags & 1) == 0 && M > 0 && N > 0 && C > 0 && M <= kCountedPositions && M <= kCountedPerCell * C && C <= 8 * M + 4096;
+  const bool counted = (flags & 1) == 0 && N > 0 && C > 0 && M > kCountedLeast && M <= kCountedPositions && M <= kCountedPerCell * C && C <= 8 * M + 4096;
   hgpu_array* o = nullptr;
   int rc = counted ? new_dense(ctx, src->dtype, n_ix + rank_n, osh, &o) : new_zeros(ctx, src->dtype, n_ix + rank_n, osh, &o);
   if (rc) return rc;

@@ -108,3 +108,15 @@ def test_all_positions_in_one_cell(gpu):
     m = 1 << 20
     src, idx = rng.standard_normal(m).astype(np.float32), np.full(m, 2047, np.int64)
     assert np.array_equal(counted(gpu, src, idx, 2048), in_segments(src, idx, 2048))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("cells,m,width", [(1, 1, 100003), (10, 32, 40000), (3, 300, 10001), (16, 16, 150528), (5, 64, 25004), (2, 65, 33), (4097, 2, 515), (7, 700, 2052), (3, 1500, 10001),
+                                          (4, 1100, 30000), (1, 512, 7000), (9, 1025, 2051), (200, 1024, 129)])
+def test_few_cells_with_wide_slices(gpu, cells, m, width, dt):
+    rng = np.random.default_rng(cells + m)
+    idx = rng.integers(-1, cells, m).astype(np.int64)
+    src = rng.standard_normal((m, width)).astype(dt)
+    inside = idx >= 0
+    arr, ix = gpu.upload(src), [gpu.upload(idx)]
+    assert np.array_equal(gpu.scatter_add(arr, ix, 1, [cells]).numpy(), in_segments(src[inside], idx[inside], cells))
