@@ -28,7 +28,12 @@ def assert_close(out, x, y, k):
 def test_ragged_shapes(gpu, m, n, k, lay):
     rng = np.random.default_rng(m + n + k)
     x, y = rng.standard_normal((m, k)).astype(np.float32), rng.uniform(0, 1, (n, k)).astype(np.float32)
-    assert_close(product(gpu, x, y, lay).numpy(), x, y, k)
+    gpu.profile(2)
+    out = product(gpu, x, y, lay).numpy()
+    labels = list(gpu.profile_report())
+    gpu.profile(0)
+    assert any(",split3,t128x128" in s for s in labels), labels
+    assert_close(out, x, y, k)
 
 
 @pytest.mark.parametrize("rest", [0.0, 2.0 ** -40])

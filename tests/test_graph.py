@@ -5,6 +5,8 @@ same kernels on the very same arrays.  Eager work runs between the replays, so
 a block of memory that leaked out of the recording's pool would show up as a
 changed result.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -59,14 +61,20 @@ def test_replays_match_eager(host, name, table):
         graph.free()
 
 
-def test_sorted_scatter_inside_a_recording(host):
-    """The general scatter-add (positions sorted by destination, runs added in order) recorded
-    into a graph: its sort is a library routine, so every replay is checked against the eager
-    result, with eager scatters of other sizes (which reuse the sort's workspace blocks) between
-    the replays, and again after the inputs changed."""
+@pytest.mark.parametrize("cells_n,hot,family", [(301, 0, "scatter_counted"), (301, 20000, "scatter_counted"), (90, 0, "scatter_sorted")])
+def test_sorted_scatter_inside_a_recording(host, cells_n, hot, family):
+    """The general scatter-add (positions counted and ordered cell by cell, one cell hit often or none;
+    or sorted by destination, by a library routine; runs added in order) recorded into a graph: every replay is
+    checked against the eager result, with eager scatters of other sizes (which reuse the workspace
+    blocks) between the replays, and again after the inputs changed."""
     rng = np.random.default_rng(21)
-    m, cells_n = 50000, 301
-    cells = host.concrete(rng.integers(-3, cells_n + 3, m).astype(np.int64))
+    m = 50000
+
+    def draw(low, high):
+        c = rng.integers(low, high, m).astype(np.int64)
+        c[rng.permutation(m)[:hot]] = 7
+        return c
+    cells = host.concrete(draw(-3, cells_n + 3))
     src = host.concrete(rng.standard_normal((m, 3)))
     other_cells = host.concrete(rng.integers(0, 9, 7777).astype(np.int64))
     other_src = host.concrete(rng.standard_normal(7777))
@@ -83,6 +91,13 @@ def test_sorted_scatter_inside_a_recording(host):
     want = program().numpy()
     np.testing.assert_allclose(want, numpy_scatter(cells.numpy(), src.numpy()), rtol=1e-10, atol=1e-12)
     assert host.counter("scatter_general") > 0
+    api = capi.Lib()
+    ctx = host.dll.hh_array_ctx(host.h)
+    assert api.profile_enable(ctx, 1) == 0
+    program().numpy()
+    report = C.create_string_buffer(1 << 16)
+    assert api.profile_report(ctx, report, len(report)) == 0 and api.profile_enable(ctx, 0) == 0
+    assert family in report.value.decode()
     graph, res = host.capture(program)
     try:
         for replay in range(3):
@@ -90,7 +105,7 @@ def test_sorted_scatter_inside_a_recording(host):
             host.sync()
             assert np.array_equal(res.numpy(), want), replay
             other_src.sscatter(1, [9], lambda i: [other_cells.sindex0([i])]).numpy()
-        new_cells = rng.integers(0, cells_n, m).astype(np.int64)
+        new_cells = draw(0, cells_n)
         new_src = rng.standard_normal((m, 3))
         cells.overwrite(new_cells)
         src.overwrite(new_src)
