@@ -12,9 +12,10 @@
 //
 // Scatter-add adds colliding positions in ascending row-major order of the
 // positions, the reference's own order (tscatterZSScalar walks `shsEnum shm`,
-// OpsConcrete.hs:1581-1619), and without atomics: the positions are sorted by
-// destination with a stable radix sort, and every destination's run is summed
-// front to back by one lane per element.  Results do not depend on the run and,
+// OpsConcrete.hs:1581-1619), and without atomics on data: the positions are
+// sorted by destination with a stable radix sort, or counted per destination and
+// put in order there, and every destination's run is summed front to back by
+// one lane per element.  Results do not depend on the run and,
 // for floating point, carry the rounding of that very order as long as no
 // destination is hit more than 256 times; a longer run is summed in segments
 // of 256 entries (each front to back) whose sums are added in ascending order,
@@ -393,13 +394,14 @@ hipError_t scatter_sorted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, i
 // too, so that the result is not cleared beforehand.  100,000 rows of 512 bytes into 20,000 cells: 134 us with
 // the sort, 35 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
 // position gets varies from run to run, the sums do not.
-// A cell may be hit far more often than the average (a padding index): its run is put in order by a block of its own
-// and its segments of kSeg entries are added up wherever there is room, as after the sort.  Half of those 100,000 picks
+// A cell may be hit far more often than the average (a padding index): a run of several segments of kSeg entries is put in
+// order by a block of its own, and its segments are added up wherever there is room, as after the sort.  Half of those 100,000 picks
 // on one row: 1470 us with the sort, 4750 with one block per long run, 108 so.
 constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (a bit for each fits the LDS of a CU: k_cell_order)
 constexpr int64_t kCountedPerCell = 512;
+constexpr int64_t kOrderedInPlace = (int64_t)1 << 17;     // up to here the runs of several segments are ordered in the launch that places the others (k_cell_place)
 constexpr int64_t kCountedLeast = 1024;   // up to here the library sorts in one launch: 18.8 us submitted one after another against 21.4 by counting; from 1025 on 27 against 21.4
-constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; longer runs: k_cell_order
+constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; up to kSeg a wavefront does
 
 // cell[m] = position m's destination (or ~0: skipped), rank[m] = how many positions of that cell counted before it.
 // A block counts its positions among themselves first, in a table of LDS (open addressing, twice as many slots
@@ -444,35 +446,35 @@ __global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, in
 // Totals made on the way, cleared beforehand.
 struct CellTotals {
   uint32_t placed;       // next free place of val
-  uint32_t runs;         // long runs listed
-  uint32_t segments;     // segments of kSeg entries of theirs
-  uint32_t parts;        // those that belong to runs of several segments
+  uint32_t runs;         // runs of more than kSmallRun entries listed
+  uint32_t parts;        // segments of kSeg entries of those that have several: rows of partial sums
+  uint32_t unused;
 };
-// A run of more than kSmallRun entries: its cell, its first segment, and the first row of the partial sums where it has several.
-struct LongRun { uint32_t cell, segment, part; };
+// A run of more than kSmallRun entries: its cell, and the row of its first partial sum where it has several segments.
+struct LongRun { uint32_t cell, part; };
 
-// Where each cell's stretch of val starts: the cells of a block side by side, the blocks in any order.  The totals are
-// drawn from once a block.
+// Where each cell's stretch of val starts (and, in the top bit, whether its run has several segments): the cells of a
+// block side by side, the blocks in any order.  The totals are drawn from once a block.
+constexpr uint32_t kSeveral = 0x80000000u;
 constexpr int kCellsPerBlock = 1024;
-__global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_t* __restrict__ counts, uint32_t* __restrict__ starts, CellTotals* __restrict__ totals, LongRun* __restrict__ runs) {
-  __shared__ uint32_t sums[4][kBlock];
-  __shared__ uint32_t base[4];
+__global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_t* __restrict__ counts, uint32_t* __restrict__ starts, CellTotals* __restrict__ totals, LongRun* __restrict__ runs, uint32_t* __restrict__ part_run) {
+  __shared__ uint32_t sums[3][kBlock];
+  __shared__ uint32_t base[3];
   const int t = threadIdx.x;
   const int64_t c0 = (int64_t)blockIdx.x * kCellsPerBlock + 4 * t;
-  uint32_t n[4], own[4] = {0, 0, 0, 0};        // entries, long runs, segments, partial sums
+  uint32_t n[4], own[3] = {0, 0, 0};        // as in CellTotals
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     n[i] = c0 + i < C ? counts[c0 + i] : 0;
-    const uint32_t segs = (n[i] + kSeg - 1) / kSeg;
     own[0] += n[i];
-    if (n[i] > kSmallRun) { own[1] += 1; own[2] += segs; own[3] += segs > 1 ? segs : 0; }
+    own[1] += n[i] > kSmallRun ? 1 : 0;
+    own[2] += n[i] > kSeg ? (n[i] + kSeg - 1) / kSeg : 0;
   }
-  const bool any = __syncthreads_or(own[1] != 0);
-  const int kinds = any ? 4 : 1;
+  const int kinds = __syncthreads_or(own[1] != 0) ? 3 : 1;
   for (int k = 0; k < kinds; ++k) sums[k][t] = own[k];
   __syncthreads();
   for (int d = 1; d < kBlock; d <<= 1) {
-    uint32_t v[4];
+    uint32_t v[3];
     for (int k = 0; k < kinds; ++k) v[k] = t >= d ? sums[k][t - d] : 0;
     __syncthreads();
     for (int k = 0; k < kinds; ++k) sums[k][t] += v[k];
@@ -483,101 +485,89 @@ __global__ void __launch_bounds__(kBlock) k_cell_starts(int64_t C, const uint32_
   uint32_t at = base[0] + sums[0][t] - own[0];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (c0 + i < C) starts[c0 + i] = at;
+    if (c0 + i < C) starts[c0 + i] = at | (n[i] > kSeg ? kSeveral : 0);
     at += n[i];
   }
   if (own[1] == 0) return;
-  uint32_t run = base[1] + sums[1][t] - own[1], segment = base[2] + sums[2][t] - own[2], part = base[3] + sums[3][t] - own[3];
+  uint32_t run = base[1] + sums[1][t] - own[1], part = base[2] + sums[2][t] - own[2];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (n[i] <= kSmallRun) continue;
-    const uint32_t segs = (n[i] + kSeg - 1) / kSeg;
-    runs[run++] = LongRun{(uint32_t)(c0 + i), segment, segs > 1 ? part : 0};
-    segment += segs;
-    if (segs > 1) part += segs;
+    const uint32_t segs = n[i] > kSeg ? (n[i] + kSeg - 1) / kSeg : 0;
+    for (uint32_t k = 0; k < segs; ++k) part_run[part + k] = run;
+    runs[run++] = LongRun{(uint32_t)(c0 + i), part};
+    part += segs;
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_cell_place(int64_t M, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ rank, uint32_t* __restrict__ val) {
-  const int64_t step = (int64_t)gridDim.x * kBlock;
-  for (int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x; m < M; m += step) {
-    const uint32_t c = cell[m];
-    if (c != 0xffffffffu) val[starts[c] + rank[m]] = (uint32_t)m;
-  }
-}
-
-// Puts the positions of the long runs in ascending order, in place, and notes the run of each segment.  A run of one
-// segment: a wavefront, every entry's rank by comparison with the others.  A longer one: a block, a bit of LDS per
-// position (BITS of them, M at most), set for the run's and read off in order -- the work grows with n + M / 32, which
-// beats sorting networks from a few hundred entries on and does not know a longest run.  A quarter of all positions and
-// more: the block goes through cell[] twice, counting and writing.  The words of 32 bits stand 33 to 32 so that lanes that
-// read 32 of them each hit different banks.
+// The positions of one run of several segments, in ascending order: the block goes through cell[] twice, counting and writing.
 constexpr int kOrderThreads = 1024;
-template <int BITS>
-__global__ void __launch_bounds__(kOrderThreads) k_cell_order(int64_t M, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts, const CellTotals* __restrict__ totals,
-                                                              const LongRun* __restrict__ runs, const uint32_t* __restrict__ cell, uint32_t* val, uint32_t* __restrict__ segment_run) {
-  constexpr int kWaves = kOrderThreads / 64, kWords = BITS / 32 + BITS / 1024;
-  static_assert(kWords >= kWaves * kSeg, "a run of one segment per wavefront");
-  __shared__ uint32_t lds[kWords];
-  __shared__ uint32_t sums[kWaves];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const uint32_t n_runs = totals->runs;
-  uint32_t* mine = lds + wave * kSeg;
-  for (uint32_t i = blockIdx.x * kWaves + wave; i < n_runs; i += gridDim.x * kWaves) {
-    const LongRun run = runs[i];
-    const uint32_t n = counts[run.cell];
-    if (n > kSeg) continue;
-    uint32_t* at = val + starts[run.cell];
-    for (uint32_t e = lane; e < kSeg; e += 64) mine[e] = e < n ? at[e] : 0xffffffffu;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    uint32_t p[kSeg / 64], r[kSeg / 64];
+__device__ __forceinline__ void order_by_scan(int64_t M, uint32_t c0, const uint32_t* __restrict__ cell, uint32_t* at, uint32_t* sums) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int share = (int)((M + kOrderThreads - 1) / kOrderThreads) * 64;      // positions of a wavefront
+  const int p0 = wave * share, p1 = (int64_t)p0 + share < M ? p0 + share : (int)M;
+  uint32_t o = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int p = p0; p < p1; p += 8 * 64) {
+      uint32_t c[8];
 #pragma unroll
-    for (int q = 0; q < kSeg / 64; ++q) { p[q] = mine[lane + 64 * q]; r[q] = 0; }
-    for (uint32_t d = 0; d < n; ++d) {
-      const uint32_t x = mine[d];
+      for (int q = 0; q < 8; ++q) c[q] = p + 64 * q + lane < p1 ? cell[p + 64 * q + lane] : 0xffffffffu;
 #pragma unroll
-      for (int q = 0; q < kSeg / 64; ++q) r[q] += x < p[q] ? 1 : 0;
+      for (int q = 0; q < 8; ++q) {
+        const unsigned long long hit = __ballot(c[q] == c0);
+        if (pass == 1 && c[q] == c0) at[o + (uint32_t)__popcll(hit & ((1ull << lane) - 1))] = (uint32_t)(p + 64 * q + lane);
+        o += (uint32_t)__popcll(hit);
+      }
     }
-#pragma unroll
-    for (int q = 0; q < kSeg / 64; ++q)
-      if (lane + 64 * q < n) at[r[q]] = p[q];
-    if (lane == 0) segment_run[run.segment] = i;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    if (pass == 1) break;
+    if (lane == 0) sums[wave] = o;
+    __syncthreads();
+    o = 0;
+    for (int w = 0; w < wave; ++w) o += sums[w];
   }
   __syncthreads();
-  const int share = (int)((M + kOrderThreads - 1) / kOrderThreads) * 64;      // positions of a wavefront
+}
+
+// Drops the positions into their cells' stretches.  With `order` the runs of several segments are left out and put in order
+// here, a block for each, from cell[] alone, which this launch only reads: a launch less than with k_cell_order
+// (2000 rows of 512 bytes submitted one after another: 21.3 -> 18.9 us), and up to 2^17 positions the passes over
+// cell[] are short (50,000 of 100,000 positions: 20 us).
+__global__ void __launch_bounds__(kOrderThreads) k_cell_place(int64_t M, bool order, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ rank,
+                                                              const CellTotals* __restrict__ totals, const LongRun* __restrict__ runs, uint32_t* val) {
+  __shared__ uint32_t sums[kOrderThreads / 64];
+  const int64_t step = (int64_t)gridDim.x * kOrderThreads;
+  for (int64_t m = (int64_t)blockIdx.x * kOrderThreads + threadIdx.x; m < M; m += step) {
+    const uint32_t c = cell[m];
+    if (c == 0xffffffffu) continue;
+    const uint32_t at = starts[c];
+    if (!(order && (at & kSeveral))) val[(at & ~kSeveral) + rank[m]] = (uint32_t)m;
+  }
+  if (!order) return;
+  const uint32_t n_runs = totals->parts ? totals->runs : 0;
+  for (uint32_t i = blockIdx.x; i < n_runs; i += gridDim.x) {
+    const uint32_t c = runs[i].cell, at = starts[c];
+    if (at & kSeveral) order_by_scan(M, c, cell, val + (at & ~kSeveral), sums);      // (the same for the whole block)
+  }
+}
+
+// The same for runs of more positions, after they have been placed: a block with a bit of LDS per position, set for the
+// run's and read off in order -- the work grows with n + M / 32, which beats sorting networks from a few hundred entries on
+// and does not know a longest run; from a quarter of all positions on by order_by_scan.  The words of 32 bits stand 33
+// to 32 so that lanes that read 32 of them each hit different banks.
+__global__ void __launch_bounds__(kOrderThreads) k_cell_order(int64_t M, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts, const CellTotals* __restrict__ totals,
+                                                              const LongRun* __restrict__ runs, const uint32_t* __restrict__ cell, uint32_t* val) {
+  __shared__ uint32_t lds[kCountedPositions / 32 + kCountedPositions / 1024];
+  __shared__ uint32_t sums[kOrderThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t n_runs = totals->parts ? totals->runs : 0;
   const int words = (int)((M + 31) / 32), per = (words + kOrderThreads - 1) / kOrderThreads;
   auto word_at = [](int w) { return w + (w >> 5); };
   for (uint32_t i = blockIdx.x; i < n_runs; i += gridDim.x) {
-    const LongRun run = runs[i];
-    const uint32_t n = counts[run.cell];
+    const uint32_t c = runs[i].cell, n = counts[c];
     if (n <= kSeg) continue;                                  // (the same for the whole block)
-    uint32_t* at = val + starts[run.cell];
-    for (uint32_t g = t; g < (n + kSeg - 1) / kSeg; g += kOrderThreads) segment_run[run.segment + g] = i;
+    uint32_t* at = val + (starts[c] & ~kSeveral);
     if ((int64_t)n * 4 >= M) {
-      const int p0 = wave * share, p1 = (int64_t)p0 + share < M ? p0 + share : (int)M;
-      uint32_t o = 0;
-      for (int pass = 0; pass < 2; ++pass) {
-        for (int p = p0; p < p1; p += 8 * 64) {
-          uint32_t c[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) c[q] = p + 64 * q + lane < p1 ? cell[p + 64 * q + lane] : 0xffffffffu;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const unsigned long long hit = __ballot(c[q] == run.cell);
-            if (pass == 1 && c[q] == run.cell) at[o + (uint32_t)__popcll(hit & ((1ull << lane) - 1))] = (uint32_t)(p + 64 * q + lane);
-            o += (uint32_t)__popcll(hit);
-          }
-        }
-        if (pass == 1) break;
-        if (lane == 0) sums[wave] = o;
-        __syncthreads();
-        o = 0;
-        for (int w = 0; w < wave; ++w) o += sums[w];
-      }
-      __syncthreads();
+      order_by_scan(M, c, cell, at, sums);
       continue;
     }
     for (int w = t; w < words; w += kOrderThreads) lds[word_at(w)] = 0;
@@ -631,66 +621,76 @@ struct CellLists {
   const uint32_t *counts, *starts, *val;
   const CellTotals* totals;
   const LongRun* runs;
-  const uint32_t* segment_run;
+  const uint32_t* part_run;
   uint32_t* tickets;       // one per row of partial sums and piece of G units (those of a run's first row are used)
   void* parts;             // [rows][N]
 };
 
-// A group of G lanes (8 to 64) per piece of work, a lane per unit of V elements.
-// First the segments of the long runs, a piece for every G units of each: a segment's slices are added front to back, eight
-// loads in flight (their positions come through LDS: 115 us for one segment of rows of 512 bytes when every round of
-// loads waited for its positions).  The sum of a run's only segment is the result; of several, whoever finishes the last adds the sums
-// in ascending order (the sums are written, a fence, a ticket; runs of several segments are rare enough for fences).
+// dst[0 .. n) = src[0 .. n), distinct numbers, in ascending order: every lane finds the ranks of its share.
+__device__ __forceinline__ void order_few(const uint32_t* src, uint32_t n, uint32_t* dst, int lane, int lanes) {
+  for (uint32_t e = lane; e < n; e += lanes) {
+    const uint32_t p = src[e];
+    uint32_t r = 0;
+    for (uint32_t d = 0; d < n; ++d) r += src[d] < p ? 1 : 0;
+    dst[r] = p;
+  }
+}
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// First the segments of the runs that have several, a group of G lanes (8 to 64) for every G units of V elements of each:
+// the positions come through LDS and the slices are added front to back, eight loads in flight (115 us for a segment of
+// rows of 512 bytes when every round of loads waited for its positions, 60 so).  Whoever finishes a run's last segment
+// adds the sums in ascending order (the sums are written, a fence, a ticket; such runs are rare enough for fences).
+// Then the runs of one segment, a wavefront for every 64 units: their positions are put in order in LDS.
 // Then the cells, each in `stretches` pieces (more than one where few cells with wide slices would leave the
-// device idle): the positions go to LDS, every lane finds the ranks of its share of them, and then the
-// lanes run along the piece and add the positions' slices in ascending order, four loads in flight.
+// device idle), a group of lanes for each: the positions are put in order in LDS, and the lanes run along the
+// piece and add the positions' slices in ascending order, four loads in flight.
 template <typename T, int V>
-__global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, int64_t stretches, CellLists in, const T* __restrict__ src, T* __restrict__ out) {
+__global__ void __launch_bounds__(kBlock, 6) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, int64_t stretches, CellLists in, const T* __restrict__ src, T* __restrict__ out) {
   using U = typename UnitOf<T, V>::type;
-  constexpr int kList = 2 * kSmallRun;
-  __shared__ uint32_t lists[kBlock / 8][kList];
-  __shared__ bool last[kBlock / 8];
-  const int g = threadIdx.x / G, l = threadIdx.x % G, groups = kBlock / G;
-  uint32_t* list = lists[g];
-  const int64_t units = N / V, step = (int64_t)gridDim.x * groups;
+  constexpr int kWaveWords = 64 / 8 * 2 * kSmallRun;         // two lists for each group of eight lanes, or two of a whole segment
+  static_assert(kWaveWords >= 2 * kSeg, "a segment's positions twice");
+  __shared__ uint32_t lists[kBlock / 64][kWaveWords];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t units = N / V;
   auto element = [&](int64_t u) {
     int64_t io[1] = {u * V};
     if constexpr (V == 1) decompose<1>(inner, u, io);
     return io[0];
   };
+  const int g = threadIdx.x / G, l = threadIdx.x % G, groups = kBlock / G, in_wave = 64 / G;
+  uint32_t* list = lists[wave] + lane / G * (2 * kSmallRun);
+  const uint32_t n_parts = in.totals->parts, n_runs = in.totals->runs;
   {
-    const int64_t pieces = (units + G - 1) / G, items = (int64_t)in.totals->segments * pieces;
-    for (int64_t base = (int64_t)blockIdx.x * groups; base < items; base += step) {
-      const bool ok = base + g < items;
-      const int64_t seg = ok ? (base + g) / pieces : 0, piece = ok ? base + g - seg * pieces : 0, u = piece * G + l;
-      const LongRun run = in.runs[ok ? in.segment_run[seg] : 0];
-      const uint32_t n = in.counts[run.cell], segs = (n + kSeg - 1) / kSeg, at = (uint32_t)(seg - run.segment);
-      const bool live = ok && u < units, several = ok && segs > 1;
-      U* result = reinterpret_cast<U*>(out + (int64_t)run.cell * N + u * V);
-      U* part = reinterpret_cast<U*>((T*)in.parts + (int64_t)run.part * N + u * V);
-      const uint32_t* mine = in.val + in.starts[run.cell] + at * kSeg;
+    const int64_t pieces = (units + G - 1) / G, items = (int64_t)n_parts * pieces;
+    for (int64_t i0 = ((int64_t)blockIdx.x * (kBlock / 64) + wave) * in_wave; i0 < items; i0 += (int64_t)gridDim.x * groups) {
+      const int64_t i = i0 + lane / G;
+      const bool ok = i < items;
+      const int64_t row = ok ? i / pieces : 0, piece = ok ? i - row * pieces : 0, u = piece * G + l;
+      const LongRun run = in.runs[in.part_run[row]];
+      const uint32_t n = in.counts[run.cell], segs = (n + kSeg - 1) / kSeg, at = (uint32_t)row - run.part;
       const uint32_t len = !ok ? 0 : n - at * kSeg < (uint32_t)kSeg ? n - at * kSeg : (uint32_t)kSeg;
+      const uint32_t* mine = in.val + (in.starts[run.cell] & ~kSeveral) + at * kSeg;
+      const bool live = ok && u < units;
       const T* from = src + (live ? element(u) : 0);
+      U* part = reinterpret_cast<U*>((T*)in.parts + (int64_t)run.part * N + u * V);
       U acc{};
-      for (uint32_t e0 = 0; e0 < len; e0 += kList) {
-        const uint32_t m = len - e0 < (uint32_t)kList ? len - e0 : (uint32_t)kList;
+      for (uint32_t e0 = 0; e0 < (uint32_t)kSeg; e0 += 2 * kSmallRun) {
+        const uint32_t m = len <= e0 ? 0 : len - e0 < 2 * kSmallRun ? len - e0 : 2 * kSmallRun;
         for (uint32_t e = l; e < m; e += G) list[e] = mine[e0 + e];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         if (live) acc = add_positions<U, 8>(sp, acc, list, m, from);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
       }
-      if (live) {
-        if (several) part[(int64_t)at * units] = acc;
-        else *result = acc;
-      }
-      if (!__syncthreads_or(several)) continue;
+      if (live) part[(int64_t)at * units] = acc;
       __threadfence();
-      __syncthreads();
-      if (l == 0) last[g] = several && atomicAdd(&in.tickets[(int64_t)run.part * pieces + piece], 1u) == segs - 1;
-      __syncthreads();
-      if (last[g] && live) {
+      uint32_t before = 0;
+      if (l == 0 && ok) before = atomicAdd(&in.tickets[(int64_t)run.part * pieces + piece], 1u);
+      before = (uint32_t)__shfl(before, lane / G * G);
+      if (live && before == segs - 1) {
         __threadfence();
         acc = part[0];
         uint32_t j = 1;
@@ -702,37 +702,44 @@ __global__ void __launch_bounds__(kBlock) k_cell_sum(IxSpace sp, Dims inner, int
           for (int q = 0; q < 8; ++q) acc = (U)(acc + x[q]);
         }
         for (; j < segs; ++j) acc = (U)(acc + part[(int64_t)j * units]);
-        *result = acc;
+        *reinterpret_cast<U*>(out + (int64_t)run.cell * N + u * V) = acc;
       }
-      __syncthreads();
     }
   }
-  const int64_t len = (units + stretches - 1) / stretches;
+  {
+    const int64_t pieces = (units + 63) / 64, items = (int64_t)n_runs * pieces;
+    uint32_t *raw = lists[wave], *sorted = raw + kSeg;
+    for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + wave; i < items; i += (int64_t)gridDim.x * (kBlock / 64)) {
+      const int64_t r = i / pieces, u = (i - r * pieces) * 64 + lane;
+      const uint32_t c = in.runs[r].cell, n = in.counts[c];
+      if (n > (uint32_t)kSeg) continue;
+      const uint32_t* mine = in.val + in.starts[c];
+      for (uint32_t e = lane; e < n; e += 64) raw[e] = mine[e];
+      wave_sync();
+      order_few(raw, n, sorted, lane, 64);
+      wave_sync();
+      if (u < units) *reinterpret_cast<U*>(out + (int64_t)c * N + u * V) = add_positions<U, 8>(sp, U{}, sorted, n, src + element(u));
+      wave_sync();
+    }
+  }
+  uint32_t *raw = list, *sorted = list + kSmallRun;
+  const int64_t step = (int64_t)gridDim.x * groups, len = (units + stretches - 1) / stretches;
   for (int64_t i = (int64_t)blockIdx.x * groups + g; i < C * stretches; i += step) {
     const int64_t c = stretches == 1 ? i : i / stretches, u0 = (i - c * stretches) * len, u1 = u0 + len < units ? u0 + len : units;
     const uint32_t n = in.counts[c];
     if (n > kSmallRun) continue;
     const uint32_t* mine = in.val + in.starts[c];
-    uint32_t *raw = list, *sorted = list + kSmallRun;
     for (uint32_t e = l; e < n; e += G) raw[e] = mine[e];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    for (uint32_t e = l; e < n; e += G) {
-      const uint32_t p = raw[e];
-      uint32_t r = 0;
-      for (uint32_t d = 0; d < n; ++d) r += raw[d] < p ? 1 : 0;
-      sorted[r] = p;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
+    order_few(raw, n, sorted, l, G);
+    wave_sync();
     for (int64_t u = u0 + l; u < u1; u += G)
       *reinterpret_cast<U*>(out + c * N + u * V) = add_positions<U, 4>(sp, U{}, sorted, n, src + element(u));
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
   }
 }
 
-// k_cell_count -> k_cell_starts -> k_cell_place -> k_cell_order -> k_cell_sum.  sp's table strides are in slices; every
+// k_cell_count -> k_cell_starts -> k_cell_place (-> k_cell_order) -> k_cell_sum.  sp's table strides are in slices; every
 // element of o is written.
 hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, int64_t M, int64_t N, int64_t C, const hgpu_array* src, hgpu_array* o, int* rc_out) {
   const size_t es = dtype_size(src->dtype);
@@ -746,11 +753,11 @@ hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, 
   // three cells: 434 us with the sort, 10.4 ms with a group of lanes per cell, 90 so.)
   const int64_t room = ((int64_t)ctx->num_cu * 2048 + C * G - 1) / (C * G), longest = (units + 4 * G - 1) / (4 * G);
   const int64_t stretches = std::max<int64_t>(1, std::min(room, longest));
-  const int64_t max_runs = M / (kSmallRun + 1) + 1, max_segments = M / kSeg + max_runs;
+  const int64_t max_runs = M / (kSmallRun + 1) + 1;
   const int64_t max_parts = M > kSeg ? M / kSeg + M / (kSeg + 1) + 1 : 0;       // (a run of several segments has more than kSeg entries)
   const int64_t pieces = (units + G - 1) / G, n_tickets = max_parts * pieces;
   const int64_t head = (C + 4 + n_tickets + 3) / 4 * 4;        // counters, totals, tickets: cleared together
-  const int64_t words = (head + C + 3 * M + 3 * max_runs + max_segments + 3) / 4 * 4;
+  const int64_t words = (head + C + 3 * M + 2 * max_runs + max_parts + 3) / 4 * 4;
   hgpu_buffer* wb = nullptr;
   *rc_out = buffer_alloc(ctx, (size_t)words * 4 + (size_t)(max_parts * N) * es, &wb);
   if (*rc_out) return hipSuccess;
@@ -761,28 +768,24 @@ hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, 
   uint32_t* rank = cell + M;
   uint32_t* val = rank + M;
   LongRun* runs = (LongRun*)(val + M);
-  uint32_t* segment_run = val + M + 3 * max_runs;
+  uint32_t* part_run = val + M + 2 * max_runs;
   *rc_out = zero_fill(ctx, counts, (size_t)head * 4);
   if (*rc_out) { buffer_release(wb); return hipSuccess; }
   LaunchGuard lg(ctx, "scatter_counted", 2.0 * M * N * es + 8.0 * M * sp.n_ix, (double)M * N);
-  const unsigned gm = grid_for(M, kBlock, ctx->num_cu * 8);
-  int rounds = 1;                                              // positions of a lane: as many as leave every CU two blocks
-  while (rounds < kCountRounds && (int64_t)rounds * kBlock * ctx->num_cu * 2 < M) rounds <<= 1;
+  int rounds = 1;                                              // positions of a lane: few while latency counts, then as many as leave every CU a block
+  while (rounds < kCountRounds && (int64_t)rounds * kBlock * ctx->num_cu * (M <= kOrderedInPlace ? 2 : 1) < M) rounds <<= 1;
   const unsigned gk = (unsigned)((M + (int64_t)rounds * kBlock - 1) / (rounds * kBlock));
   hipLaunchKernelGGL(k_cell_count, dim3(gk), dim3(kBlock), 0, ctx->stream, sp, M, rounds, counts, cell, rank);
-  hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, totals, runs);
-  hipLaunchKernelGGL(k_cell_place, dim3(gm), dim3(kBlock), 0, ctx->stream, M, (const uint32_t*)starts, (const uint32_t*)cell, (const uint32_t*)rank, val);
-  if (M > kSmallRun) {
-    const unsigned go = (unsigned)std::min<int64_t>((max_runs + 15) / 16, ctx->num_cu);      // (most of the time nothing is long)
-    if (M <= (1 << 17))
-      hipLaunchKernelGGL((k_cell_order<1 << 17>), dim3(go), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs, (const uint32_t*)cell, val, segment_run);
-    else
-      hipLaunchKernelGGL((k_cell_order<kCountedPositions>), dim3(go), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs, (const uint32_t*)cell, val, segment_run);
-  }
-  const CellLists in{counts, starts, val, totals, runs, segment_run, counts + C + 4, (char*)wb->ptr + words * 4};
-  // (blocks for the cells' pieces, or for the segments' where those are more)
-  const int64_t segment_items = M > kSmallRun ? (M / kSeg + 1) * pieces : 0;
-  const unsigned gc = grid_for(std::max(C * stretches, segment_items), kBlock / G, ctx->num_cu * 16);
+  hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, totals, runs, part_run);
+  const bool in_place = M <= kOrderedInPlace;
+  hipLaunchKernelGGL(k_cell_place, dim3(grid_for(M, kOrderThreads, ctx->num_cu * 2)), dim3(kOrderThreads), 0, ctx->stream, M, in_place, (const uint32_t*)starts, (const uint32_t*)cell,
+                     (const uint32_t*)rank, (const CellTotals*)totals, (const LongRun*)runs, val);
+  if (!in_place)
+    hipLaunchKernelGGL(k_cell_order, dim3((unsigned)ctx->num_cu), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs,
+                       (const uint32_t*)cell, val);
+  const CellLists in{counts, starts, val, totals, runs, part_run, counts + C + 4, (char*)wb->ptr + words * 4};
+  // (lanes for the cells' pieces, or for the segments' where those could be more)
+  const unsigned gc = grid_for(std::max(C * stretches * G, (M / kSeg + 1) * pieces * G), kBlock, ctx->num_cu * 16);
   if (V == 2)
     hipLaunchKernelGGL((k_cell_sum<double, 2>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const double*)data_ptr(src), (double*)data_ptr(o));
   else if (V == 4)

@@ -429,8 +429,8 @@ int hgpu_gather(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_array
  * bounds are skipped (OpsConcrete.hs:944-950).  Positions that land on one
  * place are added in ascending row-major order of the positions, starting
  * from zero -- the reference's order (`shsEnum`, OpsConcrete.hs:1594,1613) --
- * without atomics (a stable sort by destination, then every run summed front
- * to back): results are the same from run to run, for every element type of
+ * without atomics on data (the positions are put in order per destination, then
+ * every run is summed front to back): results are the same from run to run, for every element type of
  * the whitelist, and floating-point sums carry the rounding of that order.
  * `flags`: bit 0 = the caller guarantees distinct positions map to distinct
  * destinations (plain stores, no sort). */
