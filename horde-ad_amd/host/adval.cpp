@@ -43,8 +43,8 @@ static T times_one(const T& r) { return lazy_mul(r, broadcast_scalar(seed_one(r.
 
 // The gradient leaves, computed, each in memory of its own: a caller writes new values into parameters, into values it
 // kept of the forward pass, into the cotangent it handed in and into other gradients, and no gradient may change with them.
-// units: the factors taken for their product with one; dt: what the pass started from.
-static void own_leaves(Backend* be, std::vector<T>& res, const std::vector<std::shared_ptr<ArrHolder>>& units, const T& dt) {
+// units: the factors taken for their product with one; dt: what the pass started from, own_dt: an array of its own.
+static void own_leaves(Backend* be, std::vector<T>& res, const std::vector<std::shared_ptr<ArrHolder>>& units, const T& dt, bool own_dt) {
   // (a factor that is still pending would be computed into one array for the forward pass and for the caller)
   for (T& r : res)
     if (std::find(units.begin(), units.end(), r.holder()) != units.end()) r = times_one(r);
@@ -53,17 +53,18 @@ static void own_leaves(Backend* be, std::vector<T>& res, const std::vector<std::
   force_many(res);
   if (!knows_sharing(be)) return;
   // Views of a factor (the rules of transposes, reshapes, slices between the product and the input), of the caller's
-  // cotangent, of another leaf.  A view that repeats one element cannot be written into and may stay one.
+  // cotangent, of another leaf.  Of two leaves over one memory it is the dense one that can be written into, so that one is
+  // copied; strided views of what nobody can write into (sums spread over their input) stay views.
   const hgpu_api* api = be->api;
+  const std::vector<T> seen = res;
   std::vector<T> copies;
   for (size_t i = 0; i < res.size(); ++i) {
-    hgpu_array* h = res[i].h();
-    bool shared = false;
+    hgpu_array* h = seen[i].h();
+    const bool dense = api->is_dense(h);
+    bool shared = (dense || !own_dt) && dt.valid() && dt.holder()->h && api->shares_memory(h, dt.holder()->h);
     for (const auto& u : units) shared = shared || (u->h && api->shares_memory(h, u->h));
-    if (!shared && api->is_dense(h)) {
-      shared = dt.valid() && dt.holder()->h && api->shares_memory(h, dt.holder()->h);
-      for (size_t j = 0; j < i && !shared; ++j) shared = api->shares_memory(h, res[j].h());
-    }
+    for (size_t j = 0; dense && j < seen.size() && !shared; ++j)
+      shared = (j < i || (j > i && !api->is_dense(seen[j].h()))) && api->shares_memory(h, seen[j].h());
     if (!shared) continue;
     res[i] = differentiable(res[i]) ? times_one(res[i]) : materialize(res[i]);
     copies.push_back(res[i]);
@@ -103,7 +104,7 @@ std::vector<T> Tape::backward(const D& out, const T& dt_or_none, const std::vect
     T z = zeros(be, i.primal.dtype(), i.primal.shape());   // tdefTarget
     res.push_back(z.size() == 1 ? materialize(z) : z);     // (one element: not the library's constant itself)
   }
-  own_leaves(be, res, units, dt);
+  own_leaves(be, res, units, dt, !dt_or_none.valid());
   return res;
 }
 

@@ -132,6 +132,50 @@ def test_scalars_and_the_seed(host):
     host.tape_reset()
 
 
+@pytest.mark.parametrize("name", ["transpose", "reverse", "sum", "rows' sums"])
+def test_strided_views_of_the_callers_cotangent(host, name):
+    """Views that cannot be written into themselves change with the array behind them all the same."""
+    ops = {"transpose": (lambda x: x.stranspose([1, 0]), lambda d: d.T), "reverse": (lambda x: x.sreverse(), lambda d: d[::-1]),
+           "sum": (lambda x: x.ssum0(), lambda d: np.broadcast_to(d, (6, 4))),
+           "rows' sums": (lambda x: x.stranspose([1, 0]).ssum(), lambda d: np.broadcast_to(d[:, None], (6, 4)))}
+    op, back = ops[name]
+    x = host.param(A)
+    out = op(x)
+    d = np.random.default_rng(9).standard_normal(out.shape)
+    dt = host.concrete(d)
+    g, = host.grad(out, [x], dt=dt)
+    overwritten(dt, d * 0 + 7)
+    assert np.array_equal(g.numpy(), back(d))
+    host.tape_reset()
+
+
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("name", ["transpose", "reverse", "sum", "rows' sums"])
+def test_writes_into_a_gradient_that_another_one_is_a_view_of(host, name, swap):
+    y0 = {"transpose": B.T, "reverse": B, "sum": np.float64(2.0), "rows' sums": B[:, 0]}[name]
+    op = {"transpose": lambda x: x.stranspose([1, 0]), "reverse": lambda x: x.sreverse(), "sum": lambda x: x.ssum0(),
+          "rows' sums": lambda x: x.stranspose([1, 0]).ssum()}[name]
+    x, y = host.param(A), host.param(y0)
+    t = op(x) + y
+    inputs = [y, x] if swap else [x, y]
+
+    def gradients():
+        gs = host.grad((t * t).ssum0() if t.shape else t * t, inputs)
+        return gs[::-1] if swap else gs
+    gx, gy = gradients()
+    want = gx.numpy().copy()
+    wanty = gy.numpy().copy()
+    overwritten(gy, wanty * 0 + 7)
+    assert np.array_equal(gx.numpy(), want)
+    gx, gy = gradients()
+    try:
+        overwritten(gx, want * 0 + 7)
+    except capi.HgpuError:         # a view that is refused as a destination
+        assert np.array_equal(gx.numpy(), want)
+    assert np.array_equal(gy.numpy(), wanty)
+    host.tape_reset()
+
+
 def test_gradients_are_destinations(host):
     """What a gradient was taken through does not show in whether it can be written into."""
     for name, (view, shape, back) in VIEWS.items():
