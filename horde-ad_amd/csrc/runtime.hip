@@ -692,7 +692,20 @@ int hgpu_strides(const hgpu_array* a, int64_t* s) {
   return HGPU_OK;
 }
 int hgpu_is_dense(const hgpu_array* a) { return a && is_dense(a) ? 1 : 0; }
-int hgpu_shares_memory(const hgpu_array* a, const hgpu_array* b) { return a && b && a->buf && a->buf == b->buf ? 1 : 0; }
+int hgpu_shares_memory(const hgpu_array* a, const hgpu_array* b) {
+  if (!a || !b || !a->buf || a->buf != b->buf || nelem(a) == 0 || nelem(b) == 0) return 0;
+  // the stretches of bytes that the two lie in (slices of one array do not touch)
+  auto stretch = [](const hgpu_array* x, int64_t* lo, int64_t* hi) {
+    const int64_t es = (int64_t)dtype_size(x->dtype);
+    *lo = x->offset * es;
+    *hi = *lo + es;
+    for (int i = 0; i < x->rank; ++i) (x->strides[i] < 0 ? *lo : *hi) += (x->shape[i] - 1) * x->strides[i] * es;
+  };
+  int64_t al, ah, bl, bh;
+  stretch(a, &al, &ah);
+  stretch(b, &bl, &bh);
+  return al < bh && bl < ah ? 1 : 0;
+}
 
 /* -------------------------------------------------------------------- views */
 

@@ -164,8 +164,8 @@ int hgpu_shape(const hgpu_array* a, int64_t* shape_out);
 int hgpu_strides(const hgpu_array* a, int64_t* strides_out);
 /* 1 when the view is dense row-major (what `stoVector` can return without a copy). */
 int hgpu_is_dense(const hgpu_array* a);
-/* 1 when the two arrays are views of one block of memory: what is written into
- * one with hgpu_overwrite or hgpu_assign may show in the other. */
+/* 1 when what is written into one array with hgpu_overwrite or hgpu_assign may
+ * show in the other: views of one block of memory whose stretches of it meet. */
 int hgpu_shares_memory(const hgpu_array* a, const hgpu_array* b);
 
 /* ------------------------------------------------- views (no element traffic) */

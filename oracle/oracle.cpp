@@ -1057,10 +1057,25 @@ static const hgpu_array* root_of(const hgpu_array* a) {
   return a;
 }
 static int view_is_dense(const hgpu_array* a) { return consecutive(a); }
-static int view_shares_memory(const hgpu_array* a, const hgpu_array* b) { return a && b && root_of(a) == root_of(b) && !a->data.empty() && !b->data.empty(); }
+// the places of the first and the last element in memory
+static std::pair<int64_t, int64_t> stretch(const hgpu_array* a) {
+  if (!a->base) return {0, prod(a->shape) - 1};
+  int64_t lo = INT64_MAX, hi = -1;
+  for (int64_t p : a->at) {
+    for (const hgpu_array* b = a->base; b->base; b = b->base) p = b->at[(size_t)p];
+    lo = std::min(lo, p);
+    hi = std::max(hi, p);
+  }
+  return {lo, hi};
+}
+static int view_shares_memory(const hgpu_array* a, const hgpu_array* b) {
+  if (!a || !b || root_of(a) != root_of(b) || a->data.empty() || b->data.empty()) return 0;
+  const auto x = stretch(a), y = stretch(b);
+  return x.first <= y.second && y.first <= x.second;
+}
 static int view_assign(hgpu_ctx* c, hgpu_array* dst, const hgpu_array* src) {
   if (!consecutive(dst)) return fail(c, HGPU_ERR_INVALID, "assign: the destination is a strided view");
-  if (view_shares_memory(dst, src)) return fail(c, HGPU_ERR_INVALID, "assign: source and destination share memory");
+  if (root_of(dst) == root_of(src)) return fail(c, HGPU_ERR_INVALID, "assign: source and destination share memory");
   int rc = horc_assign(c, dst, src);
   if (rc) return rc;
   for (; dst->base; dst = dst->base) {

@@ -189,6 +189,30 @@ def test_gradients_are_destinations(host):
         host.tape_reset()
 
 
+def test_slices_of_one_cotangent(host):
+    """Neighbouring slices of one array share a block of memory and no element: nothing is copied for them."""
+    x, y, w = host.param(A), host.param(B), host.concrete(np.concatenate([C, Z]))
+    t = x.sappend(y) * w
+    gx, gy = host.grad((t * t).ssum0(), [x, y])
+    want = 2 * np.concatenate([A * C * C, B * Z * Z])
+    overwritten(gx, Z)
+    assert np.allclose(gy.numpy(), want[6:], rtol=1e-14) and np.array_equal(gx.numpy(), Z)
+    host.tape_reset()
+
+
+@pytest.mark.gpu
+def test_shares_memory(gpu):
+    a = gpu.upload(np.zeros((6, 4)))
+    shares = lambda x, y: gpu.lib.shares_memory(x.h, y.h)
+    top, low, mid = a.slice(0, 0, 3), a.slice(0, 3, 3), a.slice(0, 2, 3)
+    assert shares(a, top) and shares(a, a.transpose([1, 0])) and shares(mid, top) and shares(mid, low)
+    assert not shares(top, low) and not shares(top.transpose([1, 0]), low.reverse(0)) and not shares(low.reverse(1), top.reverse(0))
+    assert shares(top.reverse(0), mid.reverse(1)) and shares(a.slice(1, 0, 2), a.slice(1, 2, 2))      # (rows interleave)
+    assert not shares(a, gpu.upload(np.zeros((6, 4)))) and not shares(a, a.slice(0, 2, 0))
+    s = a.slice(0, 5, 1).slice(1, 3, 1).reshape([])
+    assert shares(s, low) and not shares(s, top) and shares(s.replicate([7]), low) and not shares(s.replicate([7]), top)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", VIEWS)
 def test_recorded_step_returns_gradients_of_the_old_parameters(name):
