@@ -392,14 +392,17 @@ hipError_t scatter_sorted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, i
 // added up.  Short passes over 4-byte words (M positions, C cells) replace the ten launches
 // of a radix or merge sort of (key, position) pairs, and the pass that adds up writes every cell, empty ones
 // too, so that the result is not cleared beforehand.  100,000 rows of 512 bytes into 20,000 cells: 134 us with
-// the sort, 35 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
+// the sort, 34 us so.  The counters are the only atomics, on integers: which of its places in the stretch a
 // position gets varies from run to run, the sums do not.
 // A cell may be hit far more often than the average (a padding index): a run of several segments of kSeg entries is put in
 // order by a block of its own, and its segments are added up wherever there is room, as after the sort.  Half of those 100,000 picks
-// on one row: 1470 us with the sort, 4750 with one block per long run, 108 so.
+// on one row: 1470 us with the sort, 4750 with one block per long run, 82 so.
 constexpr int64_t kCountedPositions = (int64_t)1 << 20;   // (a bit for each fits the LDS of a CU: k_cell_order)
 constexpr int64_t kCountedPerCell = 512;
 constexpr int64_t kOrderedInPlace = (int64_t)1 << 17;     // up to here the runs of several segments are ordered in the launch that places the others (k_cell_place)
+// ... and up to so many hits a cell on average: where most cells have a long run their passes over cell[] add up (131072
+// positions in 300 cells: 237 us, with k_cell_order 85; 100,000 rows of 16 floats into 250: 217 and 71)
+constexpr int64_t kOrderedInPlaceHits = 32;
 constexpr int64_t kCountedLeast = 1024;   // up to here the library sorts in one launch: 18.8 us submitted one after another against 21.4 by counting; from 1025 on 27 against 21.4
 constexpr int kSmallRun = 64;        // a cell's positions that its own group of lanes orders in LDS; up to kSeg a wavefront does
 
@@ -407,20 +410,22 @@ constexpr int kSmallRun = 64;        // a cell's positions that its own group of
 // A block counts its positions among themselves first, in a table of LDS (open addressing, twice as many slots
 // as positions), and then adds each cell's count to the table of all with one atomic: addresses that many positions share are
 // asked once a block (2^20 positions, all in 128 cells: 757 us with one atomic for a wavefront's equal cells, 95 us so).
-constexpr int kCountRounds = 16;     // positions of a lane, at most
-__global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, int rounds, uint32_t* __restrict__ counts, uint32_t* __restrict__ cell, uint32_t* __restrict__ rank) {
-  constexpr int kSlots = 2 * kCountRounds * kBlock, kPlaceBits = 13;
-  static_assert(kSlots <= 1 << kPlaceBits && kCountRounds * kBlock <= 1 << (32 - kPlaceBits), "a slot and a count in a word");
-  __shared__ uint32_t key[kSlots], cnt[kSlots], place[kCountRounds * kBlock];
-  const int t = threadIdx.x, slots = 2 * rounds * kBlock;        // (rounds is a power of two)
-  for (int i = t; i < slots; i += kBlock) {
+// SPAN: most positions of a block; the small one leaves LDS for more blocks on a CU.
+constexpr int kCountPositions = 4096, kCountThreads = 1024;
+template <int SPAN>
+__global__ void __launch_bounds__(SPAN / 4) k_cell_count(IxSpace sp, int64_t M, int span, uint32_t* __restrict__ counts, uint32_t* __restrict__ cell, uint32_t* __restrict__ rank) {
+  constexpr int kSlots = 2 * SPAN, kPlaceBits = 13;
+  static_assert(kSlots <= 1 << kPlaceBits && SPAN <= 1 << (32 - kPlaceBits), "a slot and a count in a word");
+  __shared__ uint32_t key[kSlots], cnt[kSlots], place[SPAN];
+  const int t = threadIdx.x, nt = blockDim.x, slots = 2 * span;        // (span: positions of a block, a power of two and a multiple of nt)
+  for (int i = t; i < slots; i += nt) {
     key[i] = 0xffffffffu;
     cnt[i] = 0;
   }
   __syncthreads();
-  const int64_t m0 = (int64_t)blockIdx.x * rounds * kBlock;
-  const int here = M - m0 < (int64_t)rounds * kBlock ? (int)(M - m0) : rounds * kBlock;
-  for (int i = t; i < here; i += kBlock) {
+  const int64_t m0 = (int64_t)blockIdx.x * span;
+  const int here = M - m0 < (int64_t)span ? (int)(M - m0) : span;
+  for (int i = t; i < here; i += nt) {
     int64_t toff = 0, doff;
     const bool ok = resolve(sp, m0 + i, &toff, &doff);
     const uint32_t c = ok ? (uint32_t)toff : 0xffffffffu;
@@ -436,10 +441,19 @@ __global__ void __launch_bounds__(kBlock) k_cell_count(IxSpace sp, int64_t M, in
     place[i] = atomicAdd(&cnt[q], 1u) << kPlaceBits | q;
   }
   __syncthreads();
-  for (int i = t; i < slots; i += kBlock)
-    if (key[i] != 0xffffffffu) cnt[i] = atomicAdd(&counts[key[i]], cnt[i]);
+  for (int i0 = t; i0 < slots; i0 += 8 * nt) {       // (eight atomics in flight)
+    uint32_t c[8], before[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c[u] = i0 + u * nt < slots ? key[i0 + u * nt] : 0xffffffffu;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (c[u] != 0xffffffffu) before[u] = atomicAdd(&counts[c[u]], cnt[i0 + u * nt]);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (c[u] != 0xffffffffu) cnt[i0 + u * nt] = before[u];
+  }
   __syncthreads();
-  for (int i = t; i < here; i += kBlock)
+  for (int i = t; i < here; i += nt)
     if (place[i] != 0xffffffffu) rank[m0 + i] = cnt[place[i] & (kSlots - 1)] + (place[i] >> kPlaceBits);
 }
 
@@ -535,6 +549,7 @@ __device__ __forceinline__ void order_by_scan(int64_t M, uint32_t c0, const uint
 __global__ void __launch_bounds__(kOrderThreads) k_cell_place(int64_t M, bool order, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ cell, const uint32_t* __restrict__ rank,
                                                               const CellTotals* __restrict__ totals, const LongRun* __restrict__ runs, uint32_t* val) {
   __shared__ uint32_t sums[kOrderThreads / 64];
+  const uint32_t n_runs = order && totals->parts ? totals->runs : 0;
   const int64_t step = (int64_t)gridDim.x * kOrderThreads;
   for (int64_t m = (int64_t)blockIdx.x * kOrderThreads + threadIdx.x; m < M; m += step) {
     const uint32_t c = cell[m];
@@ -542,21 +557,19 @@ __global__ void __launch_bounds__(kOrderThreads) k_cell_place(int64_t M, bool or
     const uint32_t at = starts[c];
     if (!(order && (at & kSeveral))) val[(at & ~kSeveral) + rank[m]] = (uint32_t)m;
   }
-  if (!order) return;
-  const uint32_t n_runs = totals->parts ? totals->runs : 0;
   for (uint32_t i = blockIdx.x; i < n_runs; i += gridDim.x) {
     const uint32_t c = runs[i].cell, at = starts[c];
     if (at & kSeveral) order_by_scan(M, c, cell, val + (at & ~kSeveral), sums);      // (the same for the whole block)
   }
 }
 
-// The same for runs of more positions, after they have been placed: a block with a bit of LDS per position, set for the
+// The same for more positions or hits, after they have been placed: runs of up to 1024 entries by their ranks, longer ones by a block with a bit of LDS per position, set for the
 // run's and read off in order -- the work grows with n + M / 32, which beats sorting networks from a few hundred entries on
 // and does not know a longest run; from a quarter of all positions on by order_by_scan.  The words of 32 bits stand 33
 // to 32 so that lanes that read 32 of them each hit different banks.
 __global__ void __launch_bounds__(kOrderThreads) k_cell_order(int64_t M, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ starts, const CellTotals* __restrict__ totals,
                                                               const LongRun* __restrict__ runs, const uint32_t* __restrict__ cell, uint32_t* val) {
-  __shared__ uint32_t lds[kCountedPositions / 32 + kCountedPositions / 1024];
+  __shared__ __attribute__((aligned(16))) uint32_t lds[kCountedPositions / 32 + kCountedPositions / 1024];
   __shared__ uint32_t sums[kOrderThreads / 64];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const uint32_t n_runs = totals->parts ? totals->runs : 0;
@@ -568,6 +581,19 @@ __global__ void __launch_bounds__(kOrderThreads) k_cell_order(int64_t M, const u
     uint32_t* at = val + (starts[c] & ~kSeveral);
     if ((int64_t)n * 4 >= M) {
       order_by_scan(M, c, cell, at, sums);
+      continue;
+    }
+    if (n <= kOrderThreads) {
+      const uint32_t p = (uint32_t)t < n ? at[t] : 0xffffffffu;
+      lds[t] = p;
+      __syncthreads();
+      uint32_t r = 0;
+      for (uint32_t d = 0; d < n; d += 8) {            // (up to the next eight: the places behind n hold what is never smaller)
+        const uint4 x = *reinterpret_cast<const uint4*>(lds + d), y = *reinterpret_cast<const uint4*>(lds + d + 4);
+        r += (x.x < p) + (x.y < p) + (x.z < p) + (x.w < p) + (y.x < p) + (y.y < p) + (y.z < p) + (y.w < p);
+      }
+      if ((uint32_t)t < n) at[r] = p;
+      __syncthreads();
       continue;
     }
     for (int w = t; w < words; w += kOrderThreads) lds[word_at(w)] = 0;
@@ -602,17 +628,20 @@ template <typename T, int V> struct UnitOf { using type = T __attribute__((ext_v
 template <typename T> struct UnitOf<T, 1> { using type = T; };
 
 // Adds the slices of `n` positions, in the order of `list`, to acc, F loads in flight.
-template <typename U, int F, typename T>
+// LINEAR: the positions have one merged dim, a position's slice starts at a multiple of its number (divisions in front of
+// every load otherwise: 100,000 rows of 16 floats into 400 cells 99 us, 73 without).
+template <typename U, int F, bool LINEAR, typename T>
 __device__ __forceinline__ U add_positions(const IxSpace& sp, U acc, const uint32_t* list, uint32_t n, const T* __restrict__ from) {
+  auto slice = [&](uint32_t m) { return from + (LINEAR ? (int64_t)m * sp.data_st[0] : data_offset(sp, (int64_t)m)); };
   uint32_t j = 0;
   for (; j + F <= n; j += F) {
     U x[F];
 #pragma unroll
-    for (int q = 0; q < F; ++q) x[q] = *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j + q]));
+    for (int q = 0; q < F; ++q) x[q] = *reinterpret_cast<const U*>(slice(list[j + q]));
 #pragma unroll
     for (int q = 0; q < F; ++q) acc = (U)(acc + x[q]);
   }
-  for (; j < n; ++j) acc = (U)(acc + *reinterpret_cast<const U*>(from + data_offset(sp, (int64_t)list[j])));
+  for (; j < n; ++j) acc = (U)(acc + *reinterpret_cast<const U*>(slice(list[j])));
   return acc;
 }
 
@@ -626,13 +655,24 @@ struct CellLists {
   void* parts;             // [rows][N]
 };
 
-// dst[0 .. n) = src[0 .. n), distinct numbers, in ascending order: every lane finds the ranks of its share.
+// dst[0 .. n) = src[0 .. n), distinct numbers, in ascending order: every lane finds the ranks of its share, E numbers at a time.
+template <int E>
 __device__ __forceinline__ void order_few(const uint32_t* src, uint32_t n, uint32_t* dst, int lane, int lanes) {
-  for (uint32_t e = lane; e < n; e += lanes) {
-    const uint32_t p = src[e];
-    uint32_t r = 0;
-    for (uint32_t d = 0; d < n; ++d) r += src[d] < p ? 1 : 0;
-    dst[r] = p;
+  for (uint32_t e = lane; e < n; e += E * lanes) {
+    uint32_t p[E], r[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      p[q] = e + q * lanes < n ? src[e + q * lanes] : 0;
+      r[q] = 0;
+    }
+    for (uint32_t d = 0; d < n; ++d) {
+      const uint32_t x = src[d];
+#pragma unroll
+      for (int q = 0; q < E; ++q) r[q] += x < p[q] ? 1 : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q)
+      if (e + q * lanes < n) dst[r[q]] = p[q];
   }
 }
 __device__ __forceinline__ void wave_sync() {
@@ -648,7 +688,7 @@ __device__ __forceinline__ void wave_sync() {
 // Then the cells, each in `stretches` pieces (more than one where few cells with wide slices would leave the
 // device idle), a group of lanes for each: the positions are put in order in LDS, and the lanes run along the
 // piece and add the positions' slices in ascending order, four loads in flight.
-template <typename T, int V>
+template <typename T, int V, bool LINEAR>
 __global__ void __launch_bounds__(kBlock, 6) k_cell_sum(IxSpace sp, Dims inner, int64_t C, int64_t N, int G, int64_t stretches, CellLists in, const T* __restrict__ src, T* __restrict__ out) {
   using U = typename UnitOf<T, V>::type;
   constexpr int kWaveWords = 64 / 8 * 2 * kSmallRun;         // two lists for each group of eight lanes, or two of a whole segment
@@ -664,9 +704,15 @@ __global__ void __launch_bounds__(kBlock, 6) k_cell_sum(IxSpace sp, Dims inner, 
   const int g = threadIdx.x / G, l = threadIdx.x % G, groups = kBlock / G, in_wave = 64 / G;
   uint32_t* list = lists[wave] + lane / G * (2 * kSmallRun);
   const uint32_t n_parts = in.totals->parts, n_runs = in.totals->runs;
+  // each kind of work starts at the block where the one before it ended: they go on side by side
+  int64_t block = blockIdx.x;
+  auto behind = [&](int64_t used) {
+    block -= used % gridDim.x;
+    if (block < 0) block += gridDim.x;
+  };
   {
     const int64_t pieces = (units + G - 1) / G, items = (int64_t)n_parts * pieces;
-    for (int64_t i0 = ((int64_t)blockIdx.x * (kBlock / 64) + wave) * in_wave; i0 < items; i0 += (int64_t)gridDim.x * groups) {
+    for (int64_t i0 = (block * (kBlock / 64) + wave) * in_wave; i0 < items; i0 += (int64_t)gridDim.x * groups) {
       const int64_t i = i0 + lane / G;
       const bool ok = i < items;
       const int64_t row = ok ? i / pieces : 0, piece = ok ? i - row * pieces : 0, u = piece * G + l;
@@ -682,7 +728,7 @@ __global__ void __launch_bounds__(kBlock, 6) k_cell_sum(IxSpace sp, Dims inner, 
         const uint32_t m = len <= e0 ? 0 : len - e0 < 2 * kSmallRun ? len - e0 : 2 * kSmallRun;
         for (uint32_t e = l; e < m; e += G) list[e] = mine[e0 + e];
         wave_sync();
-        if (live) acc = add_positions<U, 8>(sp, acc, list, m, from);
+        if (live) acc = add_positions<U, 8, LINEAR>(sp, acc, list, m, from);
         wave_sync();
       }
       if (live) part[(int64_t)at * units] = acc;
@@ -706,35 +752,37 @@ __global__ void __launch_bounds__(kBlock, 6) k_cell_sum(IxSpace sp, Dims inner, 
       }
     }
   }
-  {
+  if (n_runs > 0) {
+    if (n_parts > 0) behind(((int64_t)n_parts * ((units + G - 1) / G) + groups - 1) / groups);
     const int64_t pieces = (units + 63) / 64, items = (int64_t)n_runs * pieces;
     uint32_t *raw = lists[wave], *sorted = raw + kSeg;
-    for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + wave; i < items; i += (int64_t)gridDim.x * (kBlock / 64)) {
+    for (int64_t i = block * (kBlock / 64) + wave; i < items; i += (int64_t)gridDim.x * (kBlock / 64)) {
       const int64_t r = i / pieces, u = (i - r * pieces) * 64 + lane;
       const uint32_t c = in.runs[r].cell, n = in.counts[c];
       if (n > (uint32_t)kSeg) continue;
       const uint32_t* mine = in.val + in.starts[c];
       for (uint32_t e = lane; e < n; e += 64) raw[e] = mine[e];
       wave_sync();
-      order_few(raw, n, sorted, lane, 64);
+      order_few<4>(raw, n, sorted, lane, 64);
       wave_sync();
-      if (u < units) *reinterpret_cast<U*>(out + (int64_t)c * N + u * V) = add_positions<U, 8>(sp, U{}, sorted, n, src + element(u));
+      if (u < units) *reinterpret_cast<U*>(out + (int64_t)c * N + u * V) = add_positions<U, 8, LINEAR>(sp, U{}, sorted, n, src + element(u));
       wave_sync();
     }
+    behind((items + kBlock / 64 - 1) / (kBlock / 64));
   }
   uint32_t *raw = list, *sorted = list + kSmallRun;
   const int64_t step = (int64_t)gridDim.x * groups, len = (units + stretches - 1) / stretches;
-  for (int64_t i = (int64_t)blockIdx.x * groups + g; i < C * stretches; i += step) {
+  for (int64_t i = block * groups + g; i < C * stretches; i += step) {
     const int64_t c = stretches == 1 ? i : i / stretches, u0 = (i - c * stretches) * len, u1 = u0 + len < units ? u0 + len : units;
     const uint32_t n = in.counts[c];
     if (n > kSmallRun) continue;
     const uint32_t* mine = in.val + in.starts[c];
     for (uint32_t e = l; e < n; e += G) raw[e] = mine[e];
     wave_sync();
-    order_few(raw, n, sorted, l, G);
+    order_few<1>(raw, n, sorted, l, G);
     wave_sync();
     for (int64_t u = u0 + l; u < u1; u += G)
-      *reinterpret_cast<U*>(out + c * N + u * V) = add_positions<U, 4>(sp, U{}, sorted, n, src + element(u));
+      *reinterpret_cast<U*>(out + c * N + u * V) = add_positions<U, 4, LINEAR>(sp, U{}, sorted, n, src + element(u));
     wave_sync();
   }
 }
@@ -772,26 +820,35 @@ hipError_t scatter_counted(hgpu_ctx* ctx, const IxSpace& sp, const Dims& inner, 
   *rc_out = zero_fill(ctx, counts, (size_t)head * 4);
   if (*rc_out) { buffer_release(wb); return hipSuccess; }
   LaunchGuard lg(ctx, "scatter_counted", 2.0 * M * N * es + 8.0 * M * sp.n_ix, (double)M * N);
-  int rounds = 1;                                              // positions of a lane: few while latency counts, then as many as leave every CU a block
-  while (rounds < kCountRounds && (int64_t)rounds * kBlock * ctx->num_cu * (M <= kOrderedInPlace ? 2 : 1) < M) rounds <<= 1;
-  const unsigned gk = (unsigned)((M + (int64_t)rounds * kBlock - 1) / (rounds * kBlock));
-  hipLaunchKernelGGL(k_cell_count, dim3(gk), dim3(kBlock), 0, ctx->stream, sp, M, rounds, counts, cell, rank);
+  // Positions of a block: few while latency counts, then as many as leave every CU a block; and where cells are hit more
+  // than 64 times, no more than 64 blocks if that can be had, since one address takes their atomics one after
+  // another (100,000 positions in 400 cells: 390 blocks 44 us).
+  int span = kBlock;
+  while (span < kCountPositions && ((int64_t)span * ctx->num_cu * (M <= kOrderedInPlace ? 2 : 1) < M || (M > 64 * C && M > (int64_t)64 * span))) span <<= 1;
+  const int nt = std::clamp(span / 4, kBlock, kCountThreads);
+  const dim3 gk((unsigned)((M + span - 1) / span));
+  if (span <= 4 * kBlock) hipLaunchKernelGGL(k_cell_count<4 * kBlock>, gk, dim3((unsigned)nt), 0, ctx->stream, sp, M, span, counts, cell, rank);
+  else hipLaunchKernelGGL(k_cell_count<kCountPositions>, gk, dim3((unsigned)nt), 0, ctx->stream, sp, M, span, counts, cell, rank);
   hipLaunchKernelGGL(k_cell_starts, dim3((unsigned)((C + kCellsPerBlock - 1) / kCellsPerBlock)), dim3(kBlock), 0, ctx->stream, C, (const uint32_t*)counts, starts, totals, runs, part_run);
-  const bool in_place = M <= kOrderedInPlace;
+  const bool in_place = M <= kOrderedInPlace && M <= kOrderedInPlaceHits * C;
   hipLaunchKernelGGL(k_cell_place, dim3(grid_for(M, kOrderThreads, ctx->num_cu * 2)), dim3(kOrderThreads), 0, ctx->stream, M, in_place, (const uint32_t*)starts, (const uint32_t*)cell,
                      (const uint32_t*)rank, (const CellTotals*)totals, (const LongRun*)runs, val);
   if (!in_place)
     hipLaunchKernelGGL(k_cell_order, dim3((unsigned)ctx->num_cu), dim3(kOrderThreads), 0, ctx->stream, M, (const uint32_t*)counts, (const uint32_t*)starts, (const CellTotals*)totals, (const LongRun*)runs,
                        (const uint32_t*)cell, val);
   const CellLists in{counts, starts, val, totals, runs, part_run, counts + C + 4, (char*)wb->ptr + words * 4};
-  // (lanes for the cells' pieces, or for the segments' where those could be more)
-  const unsigned gc = grid_for(std::max(C * stretches * G, (M / kSeg + 1) * pieces * G), kBlock, ctx->num_cu * 16);
-  if (V == 2)
-    hipLaunchKernelGGL((k_cell_sum<double, 2>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const double*)data_ptr(src), (double*)data_ptr(o));
-  else if (V == 4)
-    hipLaunchKernelGGL((k_cell_sum<float, 4>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const float*)data_ptr(src), (float*)data_ptr(o));
-  else
-    HG_DISPATCH_DTYPE(src->dtype, T, hipLaunchKernelGGL((k_cell_sum<T, 1>), dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, (const T*)data_ptr(src), (T*)data_ptr(o)));
+  // lanes for the cells' pieces, and for the segments and the runs of one segment that a mean number of hits lets expect
+  const int64_t hits = M / C, long_lanes = hits <= kSmallRun / 2 ? 0 : (M / kSeg + 1) * pieces * G + std::min(C, max_runs) * ((units + 63) / 64) * 64;
+  const unsigned gc = grid_for(C * stretches * G + std::max(long_lanes, (M / kSeg + 1) * pieces * G), kBlock, ctx->num_cu * 16);
+  auto sum = [&](auto kernel, auto* from, auto* to) { hipLaunchKernelGGL(kernel, dim3(gc), dim3(kBlock), 0, ctx->stream, sp, inner, C, N, G, stretches, in, from, to); };
+  auto sum_as = [&](auto linear) {
+    constexpr bool L = decltype(linear)::value;
+    if (V == 2) sum(k_cell_sum<double, 2, L>, (const double*)data_ptr(src), (double*)data_ptr(o));
+    else if (V == 4) sum(k_cell_sum<float, 4, L>, (const float*)data_ptr(src), (float*)data_ptr(o));
+    else HG_DISPATCH_DTYPE(src->dtype, T, sum(k_cell_sum<T, 1, L>, (const T*)data_ptr(src), (T*)data_ptr(o)));
+  };
+  if (sp.nd == 1) sum_as(std::true_type{});
+  else sum_as(std::false_type{});
   const hipError_t e = hipGetLastError();
   buffer_release(wb);
   return e;

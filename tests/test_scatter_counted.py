@@ -122,3 +122,24 @@ def test_few_cells_with_wide_slices(gpu, cells, m, width, dt):
     inside = idx >= 0
     arr, ix = gpu.upload(src), [gpu.upload(idx)]
     assert np.array_equal(gpu.scatter_add(arr, ix, 1, [cells]).numpy(), in_segments(src[inside], idx[inside], cells))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("m,cells,width", [(100000, 400, 16), (131072, 300, 1), (131073, 300, 2), (131072, 4096, 3), (131072, 4095, 4), (9000, 20, 64), (70000, 140, 5), (1 << 20, 2100, 1),
+                                           (1 << 20, 16000, 1), (16385, 256, 8), (4097, 64, 1)])
+def test_many_cells_are_hit_often(gpu, m, cells, width, dt):
+    """Dozens to hundreds of hits for every cell: either way of ordering long runs, and blocks that count 256 to 4096 positions."""
+    rng = np.random.default_rng(m + cells)
+    idx = rng.integers(0, cells, m).astype(np.int64)
+    idx[rng.permutation(m)[: m // 50]] = 5            # (and one of thousands)
+    src = rng.standard_normal((m,) if width == 1 else (m, width)).astype(dt)
+    assert np.array_equal(counted(gpu, src, idx, cells), in_segments(src, idx, cells))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("cells,width", [(2000, 8), (60, 8), (60, 5)])
+def test_positions_in_two_dims_that_do_not_merge(gpu, cells, width, dt):
+    rng = np.random.default_rng(cells + width)
+    idx, src = rng.integers(0, cells, (130, 77)).astype(np.int64), rng.standard_normal((77, 130, width)).astype(dt)
+    out = gpu.scatter_add(gpu.upload(src).transpose([1, 0, 2]), [gpu.upload(idx)], 2, [cells]).numpy()
+    assert np.array_equal(out, in_segments(np.ascontiguousarray(src.transpose(1, 0, 2)).reshape(-1, width), idx.reshape(-1), cells))
