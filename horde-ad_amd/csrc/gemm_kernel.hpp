@@ -51,6 +51,15 @@ struct GemmParams {
   int64_t kmask, ksa, ksb; // K offsets: table[k & kmask] + k * ks; kmask 0 = no table (see KOff)
 };
 
+// XCD-aware numbering: blocks b, b+8, b+16, ... of the grid's x-then-y order share an XCD and its L2, and get a
+// contiguous range of the numbers.
+template <typename I>
+__device__ __forceinline__ I xcd_order(I block, I nblocks) {
+  if (nblocks < 64) return block;
+  const I x = block & 7, per = nblocks >> 3, rem = nblocks & 7;
+  return x * per + (x < rem ? x : rem) + (block >> 3);
+}
+
 __device__ __forceinline__ void group_off(const Group& g, int64_t lin, int64_t* oa, int64_t* ob, int64_t* oc) {
   int64_t a = 0, b = 0, c = 0;
   int64_t r = lin;
@@ -349,18 +358,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(waves_w
   const int lane = t & 63, wave = t >> 6;
   const int wm = wave / WGN, wn = wave % WGN;
 
-  // XCD-aware numbering of (K chunk, tile): blocks b, b+8, b+16, ... of the
-  // grid's x-then-y order share an XCD and its L2.  Each XCD gets a contiguous
-  // range of the chunk-major order, so the tiles that read the same rows of A
-  // or B over the same K chunk run on one XCD and share those rows in its L2.
+  // (K chunk, tile) pairs in chunk-major order: the tiles that read the same rows of A or B over
+  // the same K chunk run on one XCD and share those rows in its L2.
   const int64_t tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
   const int64_t ntiles = tiles_m * tiles_n;
   const int64_t nblocks = ntiles * gridDim.y;
-  int64_t lin = blockIdx.x + ntiles * (int64_t)blockIdx.y;
-  if (nblocks >= 64) {
-    const int64_t x = lin & 7, per = nblocks >> 3, rem = nblocks & 7;
-    lin = x * per + (x < rem ? x : rem) + (lin >> 3);
-  }
+  const int64_t lin = xcd_order<int64_t>(blockIdx.x + ntiles * (int64_t)blockIdx.y, nblocks);
   const int s = (int)(lin / ntiles);
   const int64_t bid = lin - s * ntiles;
   const int64_t tile_m = bid / tiles_n, tile_n = bid - tile_m * tiles_n;
@@ -788,6 +791,34 @@ struct SplitParams {
   const void* a_term[kMaxTerms];
   const void* b_term[kMaxTerms];
 };
+// The share of such a product that a block computes: rows from m0, columns from n0, k in [kbeg, kend), operands of its term
+// and batch element; s numbers the (term, K chunk) pairs.
+template <typename T>
+struct SplitShare {
+  const T *A, *B;
+  int m0, n0, kbeg, kend, s;
+};
+template <int BM, int BN, typename T>
+__device__ __forceinline__ SplitShare<T> split_share(const SplitParams& p, const T* A, const T* B) {
+  // each XCD works on a contiguous range of (K chunk, tile) pairs, as in k_gemm
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  const int ntiles = tiles_m * tiles_n;
+  const int lin = xcd_order<int>(blockIdx.x + ntiles * blockIdx.y, ntiles * gridDim.y);
+  const int s = lin / ntiles, bid = lin - s * ntiles;
+  // tiles in bands of eight rows of tiles: neighbours in the order share operands
+  const int band = bid / (8 * tiles_n), in_band = bid - band * 8 * tiles_n;
+  const int rows_in_band = tiles_m - band * 8 < 8 ? tiles_m - band * 8 : 8;
+  const int tile_n = in_band / rows_in_band, tile_m = band * 8 + (in_band - tile_n * rows_in_band);
+  int sk = s;
+  if (p.n_terms > 0) {
+    const int term = s / p.term_split;
+    sk = s - term * p.term_split;
+    A = (const T*)p.a_term[term];
+    B = (const T*)p.b_term[term];
+  }
+  const int kbeg = sk * p.kchunk, kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
+  return {A + (int64_t)blockIdx.z * p.bsa, B + (int64_t)blockIdx.z * p.bsb, tile_m * BM, tile_n * BN, kbeg, kend, s};
+}
 void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a);
 

@@ -164,38 +164,13 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
 
-  // each XCD works on a contiguous range of (K chunk, tile) pairs, as in k_gemm
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  const int ntiles = tiles_m * tiles_n;
-  const int nblocks = ntiles * gridDim.y;
-  int lin = blockIdx.x + ntiles * blockIdx.y;
-  if (nblocks >= 64) {
-    const int x = lin & 7, per = nblocks >> 3, rem = nblocks & 7;
-    lin = x * per + (x < rem ? x : rem) + (lin >> 3);
-  }
-  const int s = lin / ntiles, bid = lin - s * ntiles;
-  // tiles in bands of eight rows of tiles: neighbours in the order share operands
-  const int band = bid / (8 * tiles_n), in_band = bid - band * 8 * tiles_n;
-  const int rows_in_band = tiles_m - band * 8 < 8 ? tiles_m - band * 8 : 8;
-  const int tile_n = in_band / rows_in_band, tile_m = band * 8 + (in_band - tile_n * rows_in_band);
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-
-  int sk = s;
-  if (p.n_terms > 0) {
-    const int term = s / p.term_split;
-    sk = s - term * p.term_split;
-    A = (const float*)p.a_term[term];
-    B = (const float*)p.b_term[term];
-  }
-  A += (int64_t)blockIdx.z * p.bsa;
-  B += (int64_t)blockIdx.z * p.bsb;
-  const int kbeg = sk * p.kchunk;
-  const int kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
+  const auto share = split_share<BM, BN>(p, A, B);
+  const int m0 = share.m0, n0 = share.n0, kbeg = share.kbeg, kend = share.kend;
 
   Side<BM, AKC> sa;
   Side<BN, BKC> sb;
-  sa.init(t, A, p.a_bytes, p.sam, m0, p.M, p.sak);
-  sb.init(t, B, p.b_bytes, p.sbn, n0, p.N, p.sbk);
+  sa.init(t, share.A, p.a_bytes, p.sam, m0, p.M, p.sak);
+  sb.init(t, share.B, p.b_bytes, p.sbn, n0, p.N, p.sbk);
   constexpr int NA = Side<BM, AKC>::NS, NB = Side<BN, BKC>::NS;
 
   f16v acc[TM][TN], low[TM][TN];
@@ -293,7 +268,7 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
   }
   step(i0, std::integral_constant<int, 0>{});
 
-  float* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)s * p.c_split_stride;
+  float* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)share.s * p.c_split_stride;
   auto put = [&](int i, int j, const f16v& c, float scale) {
     const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
     if (n >= p.N) return;
