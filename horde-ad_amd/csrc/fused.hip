@@ -686,7 +686,7 @@ extern "C" int hgpu_fused_extremum(hgpu_ctx* ctx, int n_in, const hgpu_array* co
 // The counters are 17, the root one drawn from by the last block of each of 16: a thousand blocks on one address took
 // 10 ns apiece (1003 x 1021 fp32, three outputs: 22.3 us).  Gradient of the elementwise objective, us, a release fence
 // per block up to 131072 elements and a second launch beyond / this: 300 x 300 fp64 16.8 / 13.2, 1003 x 1021 fp32
-// 17.4 / 13.7, 2000 x 2000 fp32 27.4 / 25.5, 4096 x 4096 fp64 171.8 / 166.6.
+// 16.4 / 14.9 (runs of one build differ as much), 2000 x 2000 fp32 27.4 / 25.5, 4096 x 4096 fp64 171.8 / 166.6.
 static const char* const kHandOver = R"HG(
 __device__ __forceinline__ void hand_over(unsigned long long* at, unsigned long long v) {
   const unsigned long long old = __hip_atomic_exchange(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -341,7 +341,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
   } else {
     // Microseconds, as measured: a step of 16 k of a 128 x 128 tile 1.4 alone on its CU and 0.92 for each of several;
     // 8 for the launch with its first loads and last stores; for partial results a second launch and their bytes once
-    // out and once in.  (Without the sums: 2048 x 8192 over 2048 464, 2048 x 784 over 8192 217, 300 x 5000 over 784 29.)
+    // out and once in.  (One after another, without the sums: 2048 x 8192 over 2048 464, 2048 x 784 over 8192 217, 300 x 5000 over 784 29.)
     double best = 1e300;
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128) * p.BT * nt;
     for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
