@@ -195,10 +195,14 @@ __device__ __forceinline__ A wide_sum(const TI* __restrict__ pa, const TI* __res
   for (; j < j1; ++j) acc[1] += HASB ? (A)pa[j] * (vb ? (A)pb[j] : one_b) : (A)pa[j];      // (less than a vector, one lane's)
   return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
+// Rows that the WIDE kernels take.  Not fp64 beside a b that runs along too, where the additional registers cost more than the wide loads
+// give: us, wide / not, 10,000 rows of 1000 29.5 / 27.7, 5000 of 3000 37.0 / 36.1, 1100 of 14712 38.9 / 40.1; fp32 18.7 / 18.4, 23.1 / 23.2,
+// 24.6 / 25.5, 300 rows of 65000 28.4 / 30.8.
+bool wide_rows(size_t es, int64_t sa, const void* b, int64_t sb) { return sa == 1 && (!b || sb == 0 || (sb == 1 && es == 4)); }
 template <typename TI, typename A, bool HASB, bool WIDE>
 __device__ __forceinline__ A row_sum(const TI* __restrict__ pa, const TI* __restrict__ pb, int64_t sa, int64_t sb, int64_t j0, int64_t j1, int lane) {
   if constexpr (WIDE && std::is_floating_point<TI>::value) {
-    if (sa == 1 && (!HASB || sb == 1 || sb == 0) && j1 - j0 >= 4096 / (int64_t)sizeof(TI)) return wide_sum<TI, A, HASB>(pa, pb, sb, j0, j1, lane);
+    if (j1 - j0 >= 4096 / (int64_t)sizeof(TI)) return wide_sum<TI, A, HASB>(pa, pb, sb, j0, j1, lane);
   }
   return lane_strided_sum<TI, A, HASB>(pa, pb, sa, sb, j0 + lane, j1);
 }
@@ -271,10 +275,10 @@ __device__ __forceinline__ void wave_body(const Dims& keep, const Dims& red, int
     if (lane == 0) out[item] = (TO)acc;
   }
 }
-template <typename TI, typename TO, bool HASB>
+template <typename TI, typename TO, bool HASB, bool WIDE>
 __global__ void __launch_bounds__(kBlock) k_contract_wave(Dims keep, Dims red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                                            int S, int64_t chunk, const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, TermPtrs tp) {
-  wave_body<TI, TO, HASB, true>(keep, red, n_out, Q, Lin, sa_in, sb_in, S, chunk, a0, b0, out, &tp, blockIdx.x, gridDim.x);
+  wave_body<TI, TO, HASB, WIDE>(keep, red, n_out, Q, Lin, sa_in, sb_in, S, chunk, a0, b0, out, &tp, blockIdx.x, gridDim.x);
 }
 
 // One block of four wavefronts per output: for a few hundred outputs with a few
@@ -316,10 +320,10 @@ __device__ __forceinline__ void block_body(const Dims& keep, const Dims& red, in
     __syncthreads();
   }
 }
-template <typename TI, typename TO, bool HASB>
+template <typename TI, typename TO, bool HASB, bool WIDE>
 __global__ void __launch_bounds__(kBlock) k_contract_block(Dims keep, Dims red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                                             const TI* __restrict__ a, const TI* __restrict__ b, TO* __restrict__ out) {
-  block_body<TI, TO, HASB, true>(keep, red, n_out, Q, Lin, sa_in, sb_in, a, b, out, blockIdx.x, gridDim.x);
+  block_body<TI, TO, HASB, WIDE>(keep, red, n_out, Q, Lin, sa_in, sb_in, a, b, out, blockIdx.x, gridDim.x);
 }
 
 // Up to four single-launch reductions of one element type as one kernel: the first blocks are problem 0's, the
@@ -641,8 +645,12 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     int64_t Q = R / Lin;
     if (red.nd > 1) { red.nd -= 1; } else { red.shape[0] = 1; red.st[0][0] = red.st[1][0] = 0; }
     unsigned g = (unsigned)(n_out < (int64_t)maxb ? n_out : maxb);
-    if (b) hipLaunchKernelGGL((k_contract_block<TI, TO, true>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, (const TI*)a, (const TI*)b, (TO*)out);
-    else hipLaunchKernelGGL((k_contract_block<TI, TO, false>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, (const TI*)a, (const TI*)nullptr, (TO*)out);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, (const TI*)a, (const TI*)b, (TO*)out); };
+    const bool wide = wide_rows(sizeof(TI), sa, b, sb);
+    if (b && wide) go(k_contract_block<TI, TO, true, true>);
+    else if (b) go(k_contract_block<TI, TO, true, false>);
+    else if (wide) go(k_contract_block<TI, TO, false, true>);
+    else go(k_contract_block<TI, TO, false, false>);
   } else if (use_wave) {
     Dims red = red_full;
     int last = red.nd - 1;
@@ -653,8 +661,12 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     int64_t chunk = (span + S_per - 1) / S_per;
     int64_t items = n_out * S;
     unsigned g = grid_for(items * 64, kBlock, maxb);
-    if (b) hipLaunchKernelGGL((k_contract_wave<TI, TO, true>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, S, chunk, (const TI*)a, (const TI*)b, (TO*)out, tp);
-    else hipLaunchKernelGGL((k_contract_wave<TI, TO, false>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, S, chunk, (const TI*)a, (const TI*)nullptr, (TO*)out, tp);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, S, chunk, (const TI*)a, (const TI*)b, (TO*)out, tp); };
+    const bool wide = wide_rows(sizeof(TI), sa, b, sb);
+    if (b && wide) go(k_contract_wave<TI, TO, true, true>);
+    else if (b) go(k_contract_wave<TI, TO, true, false>);
+    else if (wide) go(k_contract_wave<TI, TO, false, true>);
+    else go(k_contract_wave<TI, TO, false, false>);
   } else {
     int64_t chunk = (R + S_per - 1) / S_per;
     unsigned g = grid_for(n_out * S, kBlock, maxb);
