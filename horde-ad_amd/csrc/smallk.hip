@@ -514,6 +514,14 @@ void choose_tile(hgpu_ctx* ctx, Spec& sp, int64_t ktot) {
   }
 }
 
+// Elements at the end of K that the flat kernel below takes as a chunk of their own: an fp32 operand whose k lies side by
+// side is read 16 bytes at a time only as far as whole vectors go, and element by element with lanes across its rows otherwise
+// (409 x 113 over 333: 6.9 us with K in one chunk, 4.9 so; 5.0 in 32 x 32 tiles, whose chunks are cut like this.  fp64,
+// with vectors of two, is as fast uncut: 385 x 149 over 169 5.0, 32 x 32 tiles 5.1).
+int flat_rest(const Spec& sp, const Term& t) {
+  return !sp.f64 && (t.sxk == 1 || t.syk == 1) && t.K >= 32 ? (int)(t.K % 4) : 0;
+}
+
 // Few rows (a minibatch of 150 through a recurrence of width 128: 20 tiles of 32 x 32 on 256 CUs): what a launch
 // takes is the chain load, store to LDS, multiply, repeated per chunk, and the 64 dependent MFMAs of a wavefront that
 // walks all of K alone.  So each block takes a 16 x 16 tile, loads both operands whole at once, its four wavefronts
@@ -526,7 +534,7 @@ bool choose_flat(hgpu_ctx* ctx, Spec& sp) {
   const int64_t tiles = ((sp.P + 15) / 16) * ((sp.Q + 15) / 16);
   if (off || tiles > ctx->num_cu) return false;
   int64_t kpad = 0;
-  for (const Term& t : sp.terms) kpad += (t.K + 15) / 16 * 16 + 8;
+  for (const Term& t : sp.terms) kpad += (t.K + 15) / 16 * 16 + 8;      // (without flat_rest's chunks: 2 KB each)
   if (kpad * 32 * (sp.f64 ? 8 : 4) > 80 * 1024) return false;
   sp.BP = sp.BQ = 16;
   sp.WP = sp.WQ = 1;
@@ -545,19 +553,23 @@ bool plan_chunks(Spec& sp) {
   }
   sp.x_elems = sp.y_elems = 0;
   sp.chunks.clear();
-  if (sp.WK > 1) {           // one chunk per term, all of them in LDS together
+  if (sp.WK > 1) {           // one chunk per term (and one for what flat_rest cuts off), all of them in LDS together
     for (int t = 0; t < (int)sp.terms.size(); ++t) {
       const Term& tm = sp.terms[(size_t)t];
-      Chunk c;
-      c.term = t;
-      c.k0 = 0;
-      c.kc = (int)tm.K;
-      c.kcp = (c.kc + 4 * sp.WK - 1) / (4 * sp.WK) * (4 * sp.WK);
-      c.x = make_operand(sp.f64, sp.BP, sp.P, tm.sxp, tm.sxk, c.kc, c.kcp);
-      c.y = make_operand(sp.f64, sp.BQ, sp.Q, tm.syq, tm.syk, c.kc, c.kcp);
-      sp.x_elems += tile_elems(c.x, c.kcp);
-      sp.y_elems += tile_elems(c.y, c.kcp);
-      sp.chunks.push_back(c);
+      const int rest = flat_rest(sp, tm);
+      for (int k0 = 0; k0 < tm.K;) {
+        Chunk c;
+        c.term = t;
+        c.k0 = k0;
+        c.kc = k0 == 0 ? (int)tm.K - rest : rest;
+        c.kcp = (c.kc + 4 * sp.WK - 1) / (4 * sp.WK) * (4 * sp.WK);
+        c.x = make_operand(sp.f64, sp.BP, sp.P, tm.sxp, tm.sxk, c.kc, c.kcp);
+        c.y = make_operand(sp.f64, sp.BQ, sp.Q, tm.syq, tm.syk, c.kc, c.kcp);
+        sp.x_elems += tile_elems(c.x, c.kcp);
+        sp.y_elems += tile_elems(c.y, c.kcp);
+        sp.chunks.push_back(c);
+        k0 += c.kc;
+      }
     }
     sp.x_elems = (std::max(sp.x_elems, 1024) + 3) / 4 * 4;      // (the exchange of the quarters: 4 x 256 elements)
     return true;

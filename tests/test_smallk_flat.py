@@ -60,3 +60,16 @@ def test_program_over_full_row_and_column_inputs(gpu, oracle, dt):
     assert np.max(np.abs(res[0][0] - res[1][0])) <= tol * scale
     assert np.max(np.abs(res[0][2] - res[1][2])) <= tol * np.max(np.abs(res[1][2]))
     assert np.mean(res[0][1] != res[1][1]) <= 1e-3       # (ties of the comparison)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("m,n,ks,layouts", [(100, 130, [301], ["mk"]), (40, 75, [623], ["mk"]), (131, 75, [302], ["km"]), (60, 200, [303], ["mk"]), (100, 200, [33, 101], ["mk", "mk"]), (100, 200, [31, 99], ["mk", "mk"]),
+                                            (17, 1000, [131, 66], ["mk", "km"]), (64, 130, [67, 5, 130], ["mk", "mk", "km"])])
+def test_k_of_no_whole_number_of_vectors(gpu, dt, m, n, ks, layouts):
+    """Operands with k side by side: whole vectors in one chunk, one to three elements in another; and products of two such."""
+    test_layers(gpu, dt, m, n, ks, layouts, dt == np.float32 or ks[0] < 312)
+    rng = np.random.default_rng(m)
+    x, y = rng.uniform(-1, 1, (m, ks[0])).astype(dt), rng.uniform(-1, 1, (n, ks[0])).astype(dt)
+    got = gpu.upload(x).replicate([n]).transpose([1, 0, 2]).contract(gpu.upload(y).replicate([m]), 2).numpy()
+    # (a rounding per product and per addition)
+    assert np.max(np.abs(got - x.astype(np.float64) @ y.astype(np.float64).T)) <= np.finfo(dt).eps * ks[0] * (ks[0] + 8) / 2
