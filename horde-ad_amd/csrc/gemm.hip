@@ -350,6 +350,12 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       const double us = 8 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 4 / 3.2e6 : 0);
       if (us < best) { best = us; split = (int)sp; }
     }
+    // Small products are left to the tiles of the fp32 instruction, which submitted one after another come to 6 us and a
+    // microsecond for six million multiplications of whole 64 x 64 tiles.  165 products of 8 to 1000 million, batches and long K: where this
+    // says no they took 1.46 to 0.96 times as long here (3 x 125 x 194 over 141 13.6 against 9.5 us, 122 x 113 over 1251
+    // 12.7 / 10.0), where it says yes 0.57 to 1.18 (52 x 101 x 264 over 107 13.8 / 24.3, 441 x 208 over 3108 20.8 / 26.5).
+    const double work = (double)((M + 63) / 64 * 64) * (double)((N + 63) / 64 * 64) * (double)p.K * (double)(p.BT * nt);
+    if (best >= 6 + work / 6e6) return HGPU_OK;
   }
   const int64_t BM = f64 ? 64 : 128, BN = BM;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
