@@ -49,3 +49,18 @@ def test_sums_of_many_partial_sums(gpu, dt, outs, n):
         assert np.array_equal(got, wide.sum(1))
     else:      # summed in fp64 by either, rounded once to the result's type
         assert np.all(np.abs(got - wide.sum(1)) <= n * 2.0 ** -52 * np.abs(wide).sum(1) / 100 + np.finfo(dt).eps * np.abs(wide.sum(1)))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int64, np.int8])
+def test_rows_of_the_types_own_extremum(gpu, dt):
+    """Nothing exceeds it: the first place, and the first one that does where there is one."""
+    lo, hi = (-np.inf, np.inf) if np.dtype(dt).kind == "f" else (np.iinfo(dt).min, np.iinfo(dt).max)
+    for want_max, end in ((True, lo), (False, hi)):
+        x = np.full((4, 1500), end, dt)
+        x[1, 1499] = x[2, 1030] = x[2, 1200] = 3
+        if np.dtype(dt).kind == "f":
+            x[3, 1:] = np.nan
+            x[0, 5::2] = np.nan
+        vals, idx = gpu.upload(x).extremum_last(want_max)
+        assert idx.numpy().tolist() == [0, 1499, 1030, 0]
+        assert np.array_equal(vals.numpy(), np.array([end, 3, 3, end], dt))
