@@ -9,8 +9,15 @@ pytestmark = pytest.mark.gpu
 
 
 def product(ctx, x, y, lay):
-    """x [M, K] times y [N, K]^T; lay: "K" = stored with k contiguous, "R" = stored with the rows contiguous.  Small products
-    are not formed from bf16 parts: as many of the same in a batch as make 5e8 multiplications, all of which have to agree."""
+    """x [M, K] times y [N, K]^T; lay: "K" = stored with k contiguous, "R" = stored with the rows contiguous."""
+    a = ctx.upload(x) if lay[0] == "K" else ctx.upload(np.ascontiguousarray(x.T)).transpose([1, 0])
+    b = ctx.upload(y) if lay[1] == "K" else ctx.upload(np.ascontiguousarray(y.T)).transpose([1, 0])
+    return a.replicate([y.shape[0]]).transpose([1, 0, 2]).contract(b.replicate([x.shape[0]]), 2)
+
+
+def repeated(ctx, x, y, lay):
+    """The values of `product`.  Small products are not formed from bf16 parts: as many of the same in a batch as make
+    5e8 multiplications, all of which have to agree."""
     c = -(-500_000_000 // (x.size * y.shape[0]))
     stack = lambda v, how: (ctx.upload(np.stack([v] * c)) if how == "K" else ctx.upload(np.stack([np.ascontiguousarray(v.T)] * c)).transpose([0, 2, 1]))
     a, b = stack(x, lay[0]), stack(y, lay[1])
@@ -33,7 +40,7 @@ def test_ragged_shapes(gpu, m, n, k, lay):
     rng = np.random.default_rng(m + n + k)
     x, y = rng.standard_normal((m, k)).astype(np.float32), rng.uniform(0, 1, (n, k)).astype(np.float32)
     gpu.profile(2)
-    out = product(gpu, x, y, lay)
+    out = repeated(gpu, x, y, lay)
     labels = list(gpu.profile_report())
     gpu.profile(0)
     assert any(",split3,t128x128" in s for s in labels), labels
@@ -55,7 +62,7 @@ def test_rows_with_one_dominating_product(gpu, diagonal, lay, rest):
     else:
         x[:, 5], y[:, 5] = rng.uniform(1, 2, m), rng.uniform(1, 2, n)
     x, y = x.astype(np.float32), y.astype(np.float32)
-    out, xd, yd = product(gpu, x, y, lay), x.astype(np.float64), y.astype(np.float64)
+    out, xd, yd = repeated(gpu, x, y, lay), x.astype(np.float64), y.astype(np.float64)
     mag = np.abs(xd) @ np.abs(yd).T
     top = np.abs(xd).max(1)[:, None] * np.abs(yd)[:, np.arange(m) * 3].T if diagonal else mag
     rows = top >= mag * (1 - 2.0 ** -20)     # (where the ordinary matrix holds something small the rest counts)
@@ -70,7 +77,7 @@ def test_elements_that_three_bf16_cannot_hold(gpu, scale):
     rng = np.random.default_rng(5)
     x = (rng.uniform(-1, 1, (m, k)) * scale).astype(np.float32)
     y = (rng.uniform(-1, 1, (n, k)) / scale / (64 if scale > 1 else 1)).astype(np.float32)
-    out = product(gpu, x, y, "KR")
+    out = repeated(gpu, x, y, "KR")
     xd, yd = x.astype(np.float64), y.astype(np.float64)
     # (the fp32 instruction rounds once per product)
     assert np.all(np.abs(out - xd @ yd.T) <= (k + 17) * 2.0 ** -24 * (np.abs(xd) @ np.abs(yd).T))
@@ -81,7 +88,7 @@ def test_infinities_and_nans_stay_where_they_belong(gpu):
     rng = np.random.default_rng(6)
     x, y = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(0.5, 1, (n, k)).astype(np.float32)
     x[3, 7], x[200, 1099], y[130, 0] = np.inf, np.nan, -np.inf
-    out = product(gpu, x, y, "RK")
+    out = repeated(gpu, x, y, "RK")
     want = x.astype(np.float64) @ y.astype(np.float64).T
     assert np.array_equal(np.isnan(out), np.isnan(want))
     assert np.array_equal(np.isposinf(out), np.isposinf(want)) and np.array_equal(np.isneginf(out), np.isneginf(want))
@@ -97,7 +104,7 @@ def test_products_close_to_the_largest_number(gpu):
     x[:, 0] = np.linspace(1.9961, 1.9999, m) * 2.0 ** 63
     y[:, 0] = np.linspace(1.9961, 1.9999, n) * 2.0 ** 63
     y[1::3, 0] *= -1
-    out, want = product(gpu, x, y, "KK"), x.astype(np.float64) @ y.astype(np.float64).T
+    out, want = repeated(gpu, x, y, "KK"), x.astype(np.float64) @ y.astype(np.float64).T
     assert np.all(np.abs(want) < 2.0 ** 128 * (1 - 2.0 ** -24)) and np.all(np.abs(want) > 2.0 ** 128 * (1 - 2.0 ** -8))
     assert np.all(np.abs(out - want) <= 4 * 2.0 ** -24 * np.abs(want))
 
@@ -109,7 +116,7 @@ def test_small_elements_keep_all_their_bits(gpu, small):
     rng = np.random.default_rng(11)
     x, y = (rng.uniform(1, 16, (m, k)) * small).astype(np.float32), rng.uniform(2.0 ** 20, 2.0 ** 21, (n, k)).astype(np.float32)
     x[::2, 1:] = 0
-    out, xd, yd = product(gpu, x, y, "KR"), x.astype(np.float64), y.astype(np.float64)
+    out, xd, yd = repeated(gpu, x, y, "KR"), x.astype(np.float64), y.astype(np.float64)
     bound = np.where(np.arange(m) % 2 == 0, 4, k / 16 + 17)[:, None] * 2.0 ** -24 * (xd @ yd.T) + 2.0 ** -149
     assert np.all(np.abs(out - xd @ yd.T) <= bound)
 
@@ -121,7 +128,7 @@ def test_large_elements_beside_ordinary_ones(gpu, top_x, top_y):
     rng = np.random.default_rng(12)
     x, y = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (n, k)).astype(np.float32)
     x[7, 3], x[200, 1039], y[140, 3] = top_x, -top_x * 0.7, top_y
-    out, xd, yd = product(gpu, x, y, "RK"), x.astype(np.float64), y.astype(np.float64)
+    out, xd, yd = repeated(gpu, x, y, "RK"), x.astype(np.float64), y.astype(np.float64)
     # (the fp32 instruction rounds once per product)
     assert np.all(np.abs(out - xd @ yd.T) <= (k + 17) * 2.0 ** -24 * (np.abs(xd) @ np.abs(yd).T))
 
