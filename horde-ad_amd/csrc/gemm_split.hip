@@ -34,7 +34,7 @@
 // additions) and the power the matrix cores draw; orders of the loop's instructions that differ by a fifth in stalls
 // measure the same.  Six bf16 instructions of 32 x 32 x 16 do the work of eight fp32 ones of 32 x 32 x 2.  2048 x 8192
 // over 2048, normally distributed / behind a relu: fp32 instruction 649 / 615 us, here 464 / 428 one after another
-// (380 to 410 in the wide dense network's gradient, among shorter kernels).  (256 x 256 tiles split an
+// (380 to 410 in the wide dense network's gradient, among shorter kernels, on two cards).  (256 x 256 tiles split an
 // element half as often, but two sets of accumulators do not fit: all six terms in one chain 407 / 378, the second
 // set added up by vector instructions 480 / 445.  256 x 128 tiles: 489 / 456.)
 #include "gemm_kernel.hpp"
