@@ -39,7 +39,9 @@
 // back (DeferredQueue) until something else needs the stream, and held-back
 // problems that do not read one another's results run as one kernel: each
 // problem's code in a namespace of its own, the first blocks of the grid for
-// problem 0, the next for problem 1, ...
+// problem 0, the next for problem 1, ...  Eight levels and more of problems
+// that read one another's results column by column are one kernel altogether
+// (smallk_chain.hpp).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -75,25 +77,6 @@ std::map<std::string, Compiled>& cache_of(hgpu_ctx* ctx) {
   auto it = ctx->jit_cache.find("__smallk__");
   if (it == ctx->jit_cache.end()) it = ctx->jit_cache.emplace("__smallk__", new std::map<std::string, Compiled>()).first;
   return *static_cast<std::map<std::string, Compiled>*>(it->second);
-}
-
-// A problem's kernel, found again by what its text depends on (the text itself
-// is only written the first time), and the kernels over sets of problems, found
-// by their members.
-struct Known {
-  std::string body;    // the problem's device code
-  int id = 0;          // stands for the body where sets of problems are keyed
-  std::string kname;
-  hipFunction_t fn = nullptr, finish_fn = nullptr;
-};
-struct KnownKernels {
-  std::unordered_map<std::string, Known> problems;
-  std::unordered_map<std::string, hipFunction_t> groups;   // by the members' ids, grids and LDS bytes in the order of the kernel's text
-};
-KnownKernels& known_of(hgpu_ctx* ctx) {
-  auto it = ctx->jit_cache.find("__smallk_known__");
-  if (it == ctx->jit_cache.end()) it = ctx->jit_cache.emplace("__smallk_known__", new KnownKernels()).first;
-  return *static_cast<KnownKernels*>(it->second);
 }
 
 struct Term {
@@ -134,6 +117,32 @@ struct Spec {
   // WK = 4: a 16 x 16 tile per block, each wavefront a quarter of every chunk's k (see choose_flat); 1: wavefronts share K
   int WK = 1;
 };
+
+// A problem's kernel, found again by what its text depends on (the text itself
+// is only written the first time), and the kernels over sets of problems, found
+// by their members.
+struct Known {
+  std::string body;    // the problem's device code
+  int id = 0;          // stands for the body where sets of problems are keyed
+  std::string kname;
+  hipFunction_t fn = nullptr, finish_fn = nullptr;
+  std::vector<hgpu_fused_instr> prog;
+  Spec spec;           // (the pointers of its terms are those of the first call)
+};
+struct KnownChain {
+  std::string src;
+  hipFunction_t fn = nullptr;
+};
+struct KnownKernels {
+  std::unordered_map<std::string, Known> problems;
+  std::unordered_map<std::string, hipFunction_t> groups;   // by the members' ids, grids and LDS bytes in the order of the kernel's text
+  std::unordered_map<std::string, KnownChain> chains;      // by chain_key
+};
+KnownKernels& known_of(hgpu_ctx* ctx) {
+  auto it = ctx->jit_cache.find("__smallk_known__");
+  if (it == ctx->jit_cache.end()) it = ctx->jit_cache.emplace("__smallk_known__", new KnownKernels()).first;
+  return *static_cast<KnownKernels*>(it->second);
+}
 
 // LDS pitch of a tile: the fragment reads of 16 rows x 4 k must not collide.
 int pitch_for(int layout, int rows, int kcp, bool f64) {
@@ -701,6 +710,7 @@ struct Deferred {
   RedJob red;
   CopyJob copy{};              // a copy into an existing array (hold_copy)
   MapJob map{};                // an elementwise pass (hold_map_locked)
+  const Known* kn = nullptr;   // a small product: what is kept of its kind
   const std::string* body = nullptr;   // the problem's device code (kept with the known kernels) and the number that stands for it
   int body_id = -1;
   std::string kname;
@@ -725,6 +735,10 @@ struct DeferredQueue {
   long n_launches = 0, n_grouped = 0;
 };
 }  // namespace hg
+
+namespace {
+#include "smallk_chain.hpp"
+}  // namespace
 
 namespace hg {
 
@@ -816,11 +830,15 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
       kn.body = generate_body(sp);
       kn.id = (int)known.size();
       kn.kname = kname;
+      kn.prog.assign(prog, prog + n_instr);
+      kn.spec = sp;
+      kn.spec.prog = kn.prog.data();
       kn.fn = compiled_kernel(ctx, {&kn.body}, {d.grid}, {d.lds_bytes}, kn.kname, sp.splits > 1 ? &kn.finish_fn : nullptr);
       it = known.emplace(key.bytes, std::move(kn)).first;
     } else if (check_keys() && (it->second.body != generate_body(sp) || it->second.kname != kname)) {
       return fail(ctx, HGPU_ERR_DEVICE, "small-K product: two different kernels under one key (%s)", kname);
     }
+    d.kn = &it->second;
     d.body = &it->second.body;
     d.body_id = it->second.id;
     d.fn = it->second.fn;
@@ -968,21 +986,10 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
     release_items();
     return;
   }
-  std::map<const hgpu_buffer*, int> written_at;
-  int top = 0;
-  for (auto& d : items) {
-    d.level = 0;
-    for (auto* b : d.reads) {
-      auto it = written_at.find(b);
-      if (it != written_at.end()) d.level = std::max(d.level, it->second + 1);
-    }
-    for (auto* b : d.writes) written_at[b] = d.level;
-    top = std::max(top, d.level);
-  }
-  auto timed_launch = [&](hipFunction_t fn, unsigned grid, const std::vector<const void*>& ar, const char* label, double bytes, double flops) {
+  auto timed_launch = [&](hipFunction_t fn, unsigned grid, const std::vector<const void*>& ar, const char* label, double bytes, double flops, unsigned block = 256) {
     // (timed: the launch carries its record's two events, which then hold the kernel's own begin and end)
     hipEvent_t ea = nullptr, eb = nullptr;
-    if (ctx->profiling && !ctx->cap && (uint64_t)grid * 256 <= 0xffffffffull) {
+    if (ctx->profiling && !ctx->cap && (uint64_t)grid * block <= 0xffffffffull) {
       hgpu_ctx::ProfRec r{label, nullptr, nullptr, bytes, flops};
       if (hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess) {
         ctx->prof.push_back(r);
@@ -991,13 +998,65 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
       }
     }
     void* args[] = {(void*)ar.data()};
-    hipError_t err = ea ? hipExtModuleLaunchKernel(fn, grid * 256, 1, 1, 256, 1, 1, 0, ctx->stream, args, nullptr, ea, eb, 0)
-                        : hipModuleLaunchKernel(fn, grid, 1, 1, 256, 1, 1, 0, ctx->stream, args, nullptr);
+    hipError_t err = ea ? hipExtModuleLaunchKernel(fn, grid * block, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr, ea, eb, 0)
+                        : hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr);
     if (err != hipSuccess) {
       int rc = check_hip(ctx, err, "small-K product launch");
       if (!ctx->deferred_rc) ctx->deferred_rc = rc;
     }
   };
+  // what a chain's kernel takes goes first: it reads no result of the others
+  std::vector<char> gone(items.size(), 0);
+  {
+    std::vector<ChainCand> cand;
+    const int n_levels = find_chain(items, cand);
+    std::vector<std::vector<int>> levels((size_t)n_levels);
+    if (n_levels)
+      for (size_t i = 0; i < items.size(); ++i)
+        if (cand[i].in) levels[(size_t)cand[i].level].push_back((int)i);
+    for (auto& l : levels) std::stable_sort(l.begin(), l.end(), [&](int a, int b) { return items[(size_t)a].body_id < items[(size_t)b].body_id; });
+    for (int l0 = 0, l1 = 0; l0 < n_levels; l0 = l1) {
+      ChainPlan plan;
+      hipFunction_t fn = nullptr;
+      // (fewer weights in registers where the compiler found too few for the rest)
+      for (int slack = 0; !fn && slack <= 32; slack += 32) {
+        plan = ChainPlan();
+        if (!plan_chain(cand, levels, ctx->num_cu, slack, l0, &l1, &plan)) break;
+        fn = chain_kernel(ctx, plan);
+      }
+      if (!fn) break;
+      std::vector<const void*> ar = plan.ptrs;
+      ar.resize(kChainMaxPtrs, nullptr);
+      int counts[kChainMaxSections] = {0};
+      for (size_t k = 0; k < plan.sections.size(); ++k) counts[k] = plan.sections[k].n_levels;
+      ar.resize((size_t)kChainMaxPtrs + kChainMaxSections / 2);
+      memcpy(ar.data() + kChainMaxPtrs, counts, sizeof counts);
+      const char* label = items[(size_t)levels[(size_t)l0][0]].label;
+      if (ctx->profiling && ctx->profile_shapes) {
+        char buf[160];
+        snprintf(buf, sizeof buf, "gemm_%s[chain:P%lld,levels%d,products%d,t%d]", plan.f64 ? "f64" : "f32", (long long)plan.P, plan.n_levels, plan.n_items, 4 * plan.NC);
+        label = intern_label(ctx, buf);
+      }
+      timed_launch(fn, (unsigned)((chain_blocks(plan) + 7) / 8 * 8), ar, label, plan.bytes, plan.flops, 512);
+      ctx->dq->n_launches += 1;
+      for (int l = l0; l < l1; ++l)
+        for (int i : levels[(size_t)l]) gone[(size_t)i] = 1;
+    }
+  }
+  std::map<const hgpu_buffer*, int> written_at;
+  int top = 0;
+  for (size_t i = 0; i < items.size(); ++i) {
+    Deferred& d = items[i];
+    d.level = -1;
+    if (gone[i]) continue;
+    d.level = 0;
+    for (auto* b : d.reads) {
+      auto it = written_at.find(b);
+      if (it != written_at.end()) d.level = std::max(d.level, it->second + 1);
+    }
+    for (auto* b : d.writes) written_at[b] = d.level;
+    top = std::max(top, d.level);
+  }
   for (int lv = 0; lv <= top; ++lv) {
     // the level's reductions: those of one element type go out together, four at a time
     {
