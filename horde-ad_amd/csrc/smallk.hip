@@ -769,9 +769,14 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     sp.terms.push_back(tm);
   }
   if (ktot < 4 || ktot > (sp.P * sp.Q <= kSmallOut ? kMaxKSmallOut : kMaxKTotal)) return HGPU_OK;
-  // below about a million multiply-adds the wave-per-output kernels are as fast; from there on this kernel wins, the more so with a program to
-  // run over the result (the CNN's readout layer and its cotangent, 10 x 1000 x 128 each: the gradient 0.453 -> 0.430 ms with them in)
-  if (sp.P < 16 || sp.Q < 4 || (double)sp.P * sp.Q * ktot < 1.0e6) return HGPU_OK;
+  // A product alone: below about a million multiply-adds the wave-per-output kernels are as fast.  With a program to run
+  // over the result, or several products to add, those take a launch or two more, and the steps of a small recurrence
+  // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than a tile has.
+  // Gradients in recorded graphs, us, with a million as the line for these too / without: dense 784-64-64-10 batch 32 fp32
+  // 83 / 56, batch 130 fp64 81 / 55; two recurrent layers of 12 steps, fp32, batch 64 width 32 571 / 104 and width 80
+  // 876 / 117, fp64 batch 300 width 50 393 / 139.
+  const bool whatever_size = n_terms > 1 || (n_instr > 0 && sp.Q >= 16);
+  if (sp.P < 16 || sp.Q < 4 || (!whatever_size && (double)sp.P * sp.Q * ktot < 1.0e6)) return HGPU_OK;
   for (int o = 0; o < n_out; ++o) {
     if (out_slots[o] < n_in && out_slots[o] != c_slot) return HGPU_OK;   // a copy of an input: not this kernel's business
     if (!outs[o]->buf) return HGPU_OK;
@@ -1019,7 +1024,7 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
       ChainPlan plan;
       hipFunction_t fn = nullptr;
       // (fewer weights in registers where the compiler found too few for the rest)
-      for (int slack = 0; !fn && slack <= 32; slack += 32) {
+      for (int slack = 0; !fn && slack <= 24; slack += 24) {
         plan = ChainPlan();
         if (!plan_chain(cand, levels, ctx->num_cu, slack, l0, &l1, &plan)) break;
         fn = chain_kernel(ctx, plan);
