@@ -66,6 +66,8 @@ namespace hg {
 struct DeferredQueue;                         // launches held back to be grouped (smallk.hip)
 void flush_deferred_locked(hgpu_ctx* ctx);    // the caller holds launch_mu
 void flush_deferred(hgpu_ctx* ctx);
+// Before a launch that reads the blocks of `reads` and writes new arrays only: launches what it needs of the held-back work (the caller holds launch_mu).
+void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads);
 void drop_deferred(hgpu_ctx* ctx);            // flush, then free the queue
 void forget_remembered_sums(hgpu_ctx* ctx);   // results kept for a later call, and the arrays held for them (footprint.hip)
 }  // namespace hg
@@ -163,12 +165,19 @@ struct Dims {
   int64_t st[4][HG_KDIMS];
 };
 
+// The same with two operands, as a grouped reduction's arguments hold it.
+struct Dims2 {
+  int nd;
+  int64_t shape[HG_KDIMS];
+  int64_t st[2][HG_KDIMS];
+};
+
 // One single-launch reduction of hgpu_contract (contract.hip) with every argument of its kernel: such a launch
 // can be held back like a small product, and reductions that do not read one another's results then go out as
 // one kernel (the bias and readout gradients at the end of a reverse pass).
 struct RedJob {
   int dtype = 0;              // element type of operands and result
-  int variant = 0;            // 0: a block per output, 1: a wavefront per output, 2: a lane per output
+  int variant = 0;            // 0: a block per output, 1: a wavefront per output, 2: a lane per output, kSumRows and up: sums of partial results
   int hasb = 0;
   Dims keep, red;
   int64_t n_out = 0, R = 0, Q = 0, Lin = 0, sa = 0, sb = 0, chunk = 0;
@@ -178,7 +187,13 @@ struct RedJob {
   void* out = nullptr;
   const char* label = nullptr;
   double bytes = 0, flops = 0;
+  // Sums of partial results: out[i] = sum over R partials s of a[s * sa + i] (kSumRows: of the doubles a[i * R + s]); outputs from n1 on go to out2.
+  int64_t n1 = 0;
+  void* out2 = nullptr;
+  bool is_sum() const { return variant >= kSumRows; }
+  enum { kSumRows = 3, kSumLane, kSum32, kSum8 };
 };
+constexpr int kMaxGroupReductions = 4, kMaxGroupSums = 12;
 // One dense copy between two arrays that do not overlap (hgpu_assign): `bytes` bytes in units of 2^unit bytes, to which both sides are aligned.
 struct CopyJob {
   const void* src;
@@ -203,10 +218,13 @@ struct MapJob {
 void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);
 // smallk.hip: holds a copy back (retaining both buffers) to be launched with the copies that follow it
 void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst);
-// contract.hip: launches up to four such reductions of one element type as one kernel (the caller holds launch_mu)
+// contract.hip: launches up to kMaxGroupReductions such reductions and kMaxGroupSums sums of partial results, all of one element type, as one kernel (the caller holds launch_mu)
 hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int n);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now
-bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write);
+bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write, hgpu_buffer* write2 = nullptr);
+// contract.hip: the `parts` partial results of n elements in `part` are added up in `out` (dense), or the first n1 in out1 and the other n - n1 in out2.
+// Held back where it can share a launch.
+int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1 = -1, const hgpu_array* out2 = nullptr);
 
 // Builds the merged iteration space of `nops` operands that share `shape`.
 // Size-1 dims vanish; adjacent dims merge when every operand's strides allow.
@@ -243,13 +261,18 @@ int copy_view(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const vo
 // Serialises enqueueing and, when profiling is on, brackets the launches made
 // while it lives with an event pair labelled `name`; `bytes` / `flops` are the
 // ALGORITHMIC traffic and work of those launches.
+//
+// `reads`: the launches write new arrays only, and these addresses lie in every block they read.  Held-back work whose
+// results they do not read then stays held back (arrays are written once, and held work keeps its blocks, so
+// reads-after-writes are the only order there is); without it everything held back goes first.
 struct LaunchGuard {
   hgpu_ctx* ctx;
   bool timed = false;
-  explicit LaunchGuard(hgpu_ctx* c, const char* name = nullptr, double bytes = 0, double flops = 0) : ctx(c) {
+  explicit LaunchGuard(hgpu_ctx* c, const char* name = nullptr, double bytes = 0, double flops = 0, const std::vector<const void*>* reads = nullptr) : ctx(c) {
     c->launch_mu.lock();
     (void)hipSetDevice(c->device);
-    if (c->dq_pending) flush_deferred_locked(c);   // what was held back goes first: stream order is program order
+    if (c->dq_pending && reads) make_way_locked(c, *reads);
+    else if (c->dq_pending) flush_deferred_locked(c);   // stream order is program order
     static const bool trace = getenv("HORDEAD_GPU_TRACE_LAUNCHES") != nullptr;   // one line per launch, in program order
     if (trace && name) fprintf(stderr, "hordead_gpu: launch %s\n", name);
     if (c->profiling && name && !c->cap) {
@@ -277,6 +300,13 @@ struct LaunchGuard {
     return ctx->prof.back().b;
   }
 };
+
+// What launches over these arrays read (see LaunchGuard).
+inline std::vector<const void*> reads_of(int n, const hgpu_array* const* in) {
+  std::vector<const void*> r;
+  for (int i = 0; i < n; ++i) r.push_back(data_ptr(in[i]));
+  return r;
+}
 
 // Launch of a run-time compiled kernel under a guard: `first` / `last` say whether this is the first / last
 // launch the guard's record is to cover.
@@ -325,8 +355,8 @@ inline int take_deferred_rc(hgpu_ctx* c) {
 // Device-side decomposition of a linear index over a merged iteration space.
 #ifdef __HIPCC__
 namespace hg {
-template <int NOPS>
-__device__ __forceinline__ void decompose(const Dims& d, int64_t lin, int64_t* off) {
+template <int NOPS, typename D>
+__device__ __forceinline__ void decompose(const D& d, int64_t lin, int64_t* off) {
 #pragma unroll
   for (int k = 0; k < NOPS; ++k) off[k] = 0;
   if (lin < (int64_t)0x7fffffff) {

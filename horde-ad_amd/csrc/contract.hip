@@ -65,8 +65,8 @@ __device__ __forceinline__ A wave_sum(A v) {
 // [s*chunk, min(R, (s+1)*chunk)).  out is dense [n_out, S].
 // (`bid` of `nb` blocks: the kernels below pass their own block index; the grouped kernel at the end of this
 // file passes a block's place among the blocks of its problem.  tp == nullptr: one product.)
-template <typename TI, typename TO, bool HASB>
-__device__ __forceinline__ void lane_body(const Dims& keep, const Dims& red, int64_t n_out, int64_t R, int S, int64_t chunk,
+template <typename TI, typename TO, bool HASB, typename D>
+__device__ __forceinline__ void lane_body(const D& keep, const D& red, int64_t n_out, int64_t R, int S, int64_t chunk,
                                           const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, const TermPtrs* tp, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
   int64_t items = n_out * S;
@@ -210,8 +210,8 @@ __device__ __forceinline__ A row_sum(const TI* __restrict__ pa, const TI* __rest
 // One wavefront per work item.  `red` has its innermost dim split off:
 // Lin = extent, (sa_in, sb_in) = strides; `red` keeps the outer reduced dims
 // with Q = their product.  Chunks split Q when Q > 1, else Lin.
-template <typename TI, typename TO, bool HASB, bool WIDE>
-__device__ __forceinline__ void wave_body(const Dims& keep, const Dims& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
+template <typename TI, typename TO, bool HASB, bool WIDE, typename D>
+__device__ __forceinline__ void wave_body(const D& keep, const D& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                           int S, int64_t chunk, const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, const TermPtrs* tp, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
   const int lane = threadIdx.x & 63;
@@ -286,8 +286,8 @@ __global__ void __launch_bounds__(kBlock) k_contract_wave(Dims keep, Dims red, i
 // the device idle and splitting into chunks would cost a second launch.  The
 // wavefronts take every fourth outer reduced index (or a quarter of the inner
 // dim when there is no outer one) and combine through LDS in a fixed order.
-template <typename TI, typename TO, bool HASB, bool WIDE>
-__device__ __forceinline__ void block_body(const Dims& keep, const Dims& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
+template <typename TI, typename TO, bool HASB, bool WIDE, typename D>
+__device__ __forceinline__ void block_body(const D& keep, const D& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                            const TI* __restrict__ a, const TI* __restrict__ b, TO* __restrict__ out, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
   __shared__ A part[kBlock / 64];
@@ -326,10 +326,116 @@ __global__ void __launch_bounds__(kBlock) k_contract_block(Dims keep, Dims red, 
   block_body<TI, TO, HASB, WIDE>(keep, red, n_out, Q, Lin, sa_in, sb_in, a, b, out, blockIdx.x, gridDim.x);
 }
 
-// Up to four single-launch reductions of one element type as one kernel: the first blocks are problem 0's, the
-// next ones problem 1's, ...; every block runs the code of the kernel its problem would have been launched with.
+// Sums the partial results of a split reduction: out[i] = sum_s part[s * stride + i].  A block owns
+// OPB consecutive outputs; its 256 / OPB groups of lanes each take every
+// (256 / OPB)-th partial (coalesced rows of OPB elements), several loads in
+// flight at a time, and combine through LDS in a fixed order.  Few outputs get
+// the narrow blocks: more of them, and fewer partials for a lane to walk through.
+struct SumArgs {
+  const void* part;
+  void* out;
+  void* out2;         // outputs from n1 on
+  int64_t n, n1, stride;
+  int S, kind;
+  unsigned grid, pad_;
+};
+
+template <typename T, int OPB>
+__device__ __forceinline__ void partials_body(const SumArgs& a, unsigned bid, unsigned nb) {
+  constexpr int G = 256 / OPB;
+  __shared__ T red[G][OPB + 1];
+  const T* __restrict__ part = (const T*)a.part;
+  const int ol = threadIdx.x % OPB, g = threadIdx.x / OPB;
+  for (int64_t base = (int64_t)bid * OPB; base < a.n; base += (int64_t)nb * OPB) {
+    int64_t i = base + ol;
+    T acc = T(0);
+    if (i < a.n) {
+#pragma unroll 8
+      for (int s = g; s < a.S; s += G) acc += part[(int64_t)s * a.stride + i];
+    }
+    red[g][ol] = acc;
+    __syncthreads();
+    if (g == 0 && i < a.n) {
+      T t = red[0][ol];
+#pragma unroll
+      for (int k = 1; k < G; ++k) t += red[k][ol];
+      if (i < a.n1) ((T*)a.out)[i] = t;
+      else ((T*)a.out2)[i - a.n1] = t;
+    }
+    __syncthreads();
+  }
+}
+
+// The same sum with an output per lane: for a handful of partials (S <= 8), where the blocks above would leave most of
+// their lane groups without one, and for many outputs, where they would go around several times and wait for their loads
+// each time (300 x 784 outputs of 15 fp64 partials with five other problems of a group: 23.7 us in such blocks, 18.2 so; 2048 x 784 of 9
+// fp32 ones, 4.5 to launch among them, 22 and 16).  Up to eight are added one after another (0 + p0 + p1 + ...),
+// more of them in four interleaved chains, eight loads in flight.
+template <typename T>
+__device__ __forceinline__ void partials_lane_body(const SumArgs& g, unsigned bid, unsigned nb) {
+  const int64_t step = (int64_t)nb * 256;
+  for (int64_t i = (int64_t)bid * 256 + threadIdx.x; i < g.n; i += step) {
+    const T* p = (const T*)g.part + i;
+    T c[4] = {T(0), T(0), T(0), T(0)};
+    int s = 0;
+    if (g.S > 8) {
+      for (; s + 7 < g.S; s += 8) {
+        T x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = p[(int64_t)(s + u) * g.stride];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u & 3] += x[u];
+      }
+    }
+    T x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = s + u < g.S ? p[(int64_t)(s + u) * g.stride] : T(0);
+    T acc = g.S > 8 ? (c[0] + c[1]) + (c[2] + c[3]) : T(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (s + u < g.S) acc += x[u];
+    if (i < g.n1) ((T*)g.out)[i] = acc;
+    else ((T*)g.out2)[i - g.n1] = acc;
+  }
+}
+
+// Partial sums in doubles that lie side by side, S for an output: a wavefront per output.
+template <typename T>
+__device__ __forceinline__ void partials_row_body(const SumArgs& g, unsigned bid, unsigned nb) {
+  const int lane = threadIdx.x & 63;
+  const int64_t nwaves = ((int64_t)nb * kBlock) >> 6;
+  for (int64_t o = ((int64_t)bid * kBlock + threadIdx.x) >> 6; o < g.n; o += nwaves) {
+    const double* p = (const double*)g.part + o * g.S;
+    double acc = lane_strided_sum<double, double, false>(p, nullptr, 1, 0, lane, g.S);
+    acc = wave_sum<double>(acc);
+    if (lane == 0) ((T*)g.out)[o] = (T)acc;
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void sum_body(const SumArgs& s, unsigned bid) {
+  if (s.kind == RedJob::kSumRows) partials_row_body<T>(s, bid, s.grid);
+  else if (s.kind == RedJob::kSumLane) partials_lane_body<T>(s, bid, s.grid);
+  else if (s.kind == RedJob::kSum32) partials_body<T, 32>(s, bid, s.grid);
+  else partials_body<T, 8>(s, bid, s.grid);
+}
+
+template <typename T, int KIND>
+__global__ void __launch_bounds__(kBlock) k_sum_partials(SumArgs s) {
+  if (KIND == RedJob::kSumRows) partials_row_body<T>(s, blockIdx.x, gridDim.x);
+  else if (KIND == RedJob::kSumLane) partials_lane_body<T>(s, blockIdx.x, gridDim.x);
+  else if (KIND == RedJob::kSum32) partials_body<T, 32>(s, blockIdx.x, gridDim.x);
+  else partials_body<T, 8>(s, blockIdx.x, gridDim.x);
+}
+
+// Up to four single-launch reductions and twelve sums of partial results of one element type as one kernel: the first
+// blocks are problem 0's, the next ones problem 1's, ...; every block runs the code of the kernel its problem would have
+// been launched with.  A launch costs 4.5 to 5 us in a recorded graph however little it does, and nobody waits for the
+// sums of a reverse pass.  Gradients, us, each sum as a launch of its own / so: two recurrent layers of width 128 over 28 steps,
+// fp32 batch 5000 636 / 608, fp64 batch 150 319 / 303; CNN 28 x 28 fp64 batch 1000 327 / 320, its training step at batch 250
+// fp32 152 / 144; dense 784-300-100-10 fp64 batch 5000 214 / 209; wide dense network fp32 1730 / 1720.
 struct RedArgs {
-  Dims keep, red;
+  Dims2 keep, red;
   int64_t n_out, R, Q, Lin, sa, sb, chunk;
   int variant, hasb;
   unsigned grid, pad_;
@@ -338,8 +444,9 @@ struct RedArgs {
   void* out;
 };
 struct RedGroup {
-  int n, pad_;
-  RedArgs j[4];
+  int n, n_sums;
+  RedArgs j[kMaxGroupReductions];
+  SumArgs s[kMaxGroupSums];
 };
 static_assert(sizeof(RedGroup) <= 4000, "the grouped reduction's arguments must fit the kernel argument block");
 
@@ -347,7 +454,13 @@ template <typename T>
 __global__ void __launch_bounds__(kBlock) k_contract_group(RedGroup g) {
   unsigned bid = blockIdx.x;
   int k = 0;
-  while (k < g.n - 1 && bid >= g.j[k].grid) { bid -= g.j[k].grid; ++k; }
+  while (k < g.n && bid >= g.j[k].grid) { bid -= g.j[k].grid; ++k; }
+  if (k == g.n) {
+    k = 0;
+    while (k < g.n_sums - 1 && bid >= g.s[k].grid) { bid -= g.s[k].grid; ++k; }
+    sum_body<T>(g.s[k], bid);
+    return;
+  }
   const RedArgs& r = g.j[k];
   const T* a = (const T*)r.a;
   const T* b = (const T*)r.b;
@@ -569,8 +682,9 @@ struct HoldBufs { hgpu_buffer* a; hgpu_buffer* b; hgpu_buffer* out; };
 
 template <typename TI, typename TO>
 int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red_full, int64_t n_out, int64_t R, int S, const void* a, const void* b, void* out,
-                 const TermPtrs* terms = nullptr, const HoldBufs* hold = nullptr, int dtype = -1) {
+                 const TermPtrs* terms = nullptr, const HoldBufs* hold = nullptr, int dtype = -1, bool fresh = true) {
   // with terms, S counts the chunks of all of them; each term is cut into s_per
+  // (fresh: out is a new array, see LaunchGuard)
   TermPtrs tp;
   tp.n = 0;
   tp.s_per = S;
@@ -637,7 +751,12 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     hgpu_buffer* reads[2] = {hold->a, hold->b};
     if (hold_reduction(ctx, j, reads, hold->b ? 2 : 1, hold->out)) return HGPU_OK;
   }
-  LaunchGuard lg(ctx, label, bytes, flops);
+  std::vector<const void*> reads{a, b};
+  if (tp.n) {
+    reads.insert(reads.end(), tp.a, tp.a + tp.n);
+    reads.insert(reads.end(), tp.b, tp.b + tp.n);
+  }
+  LaunchGuard lg(ctx, label, bytes, flops, fresh ? &reads : nullptr);
   if (use_wave && S == 0) {       // one block per output, no partials
     Dims red = red_full;
     int last = red.nd - 1;
@@ -680,16 +799,101 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
 }  // namespace
 
 namespace hg {
+static SumArgs sum_args(const RedJob& j) {
+  SumArgs s;
+  memset(&s, 0, sizeof s);
+  s.part = j.a;
+  s.out = j.out;
+  s.out2 = j.out2;
+  s.n = j.n_out;
+  s.n1 = j.n1;
+  s.stride = j.sa;
+  s.S = (int)j.R;
+  s.kind = j.variant;
+  s.grid = j.grid;
+  return s;
+}
+
+template <typename T>
+static void launch_sum(hgpu_ctx* ctx, const RedJob& j) {
+  const SumArgs s = sum_args(j);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(j.grid), dim3(kBlock), 0, ctx->stream, s); };
+  if (j.variant == RedJob::kSumRows) go(k_sum_partials<T, RedJob::kSumRows>);
+  else if (j.variant == RedJob::kSumLane) go(k_sum_partials<T, RedJob::kSumLane>);
+  else if (j.variant == RedJob::kSum32) go(k_sum_partials<T, RedJob::kSum32>);
+  else go(k_sum_partials<T, RedJob::kSum8>);
+}
+
+// Partial results of more than this are added up at once: such a sum is long enough for a launch of its own, and its
+// memory is better given back.
+constexpr double kMaxHeldPartials = 64.0 * (1 << 20);
+
+static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_array* out1, const hgpu_array* out2) {
+  j.a = part->ptr;
+  j.out = data_ptr(out1);
+  j.out2 = out2 ? data_ptr(out2) : nullptr;
+  j.label = "gemm_sum_partials";
+  j.flops = (double)j.n_out * j.R;
+  if (out1->buf && (!out2 || out2->buf) && (double)part->bytes <= kMaxHeldPartials &&
+      hold_reduction(ctx, j, &part, 1, out1->buf, out2 ? out2->buf : nullptr)) return HGPU_OK;
+  const std::vector<const void*> reads{j.a};
+  LaunchGuard ls(ctx, j.label, j.bytes, j.flops, &reads);
+  if (j.dtype == HGPU_F64) launch_sum<double>(ctx, j);
+  else launch_sum<float>(ctx, j);
+  HG_CHECK_LAUNCH(ctx, "gemm_sum_partials");
+  return HGPU_OK;
+}
+
+int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1, const hgpu_array* out2) {
+  const size_t es = dtype_size(dtype);
+  RedJob j;
+  j.dtype = dtype;
+  j.n_out = n;
+  j.n1 = n1 < 0 ? n : n1;
+  j.R = parts;
+  j.sa = n;
+  j.bytes = (double)n * (parts + 1) * es;
+  // fp32: rows of 32 are whole 128-byte lines (16384 outputs x 270 partials: 12.9 us with rows of 8, 7.1 us with rows of 32)
+  j.variant = parts <= 8 || (parts <= 64 && n >= 65536) ? RedJob::kSumLane : (es == 4 || n > 32768 || parts < 32) ? RedJob::kSum32 : RedJob::kSum8;
+  j.grid = grid_for(n, j.variant == RedJob::kSumLane ? 256 : j.variant == RedJob::kSum32 ? 32 : 8, ctx->num_cu * 8);
+  return queue_sum(ctx, j, part, out1, out2);
+}
+
+// A row of S sums in doubles for every output.
+static int sum_partial_rows(hgpu_ctx* ctx, int dtype, int64_t n, int64_t S, hgpu_buffer* part, const hgpu_array* out) {
+  RedJob j;
+  j.dtype = dtype;
+  j.variant = RedJob::kSumRows;
+  j.n_out = j.n1 = n;
+  j.R = S;
+  j.bytes = (double)n * (S * 8.0 + dtype_size(dtype));
+  j.grid = grid_for(n * 64, kBlock, ctx->num_cu * 8);
+  return queue_sum(ctx, j, part, out, nullptr);
+}
+
 hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int n) {
+  if (n == 1 && jobs[0]->is_sum()) {
+    if (jobs[0]->dtype == HGPU_F64) launch_sum<double>(ctx, *jobs[0]);
+    else launch_sum<float>(ctx, *jobs[0]);
+    return hipGetLastError();
+  }
   RedGroup g;
   memset(&g, 0, sizeof g);
-  g.n = n;
   unsigned grid = 0;
+  auto two = [](const Dims& d) {
+    Dims2 e;
+    memset(&e, 0, sizeof e);
+    e.nd = d.nd;
+    for (int i = 0; i < d.nd; ++i) { e.shape[i] = d.shape[i]; e.st[0][i] = d.st[0][i]; e.st[1][i] = d.st[1][i]; }
+    return e;
+  };
   for (int i = 0; i < n; ++i) {
     const RedJob& j = *jobs[i];
-    RedArgs& r = g.j[i];
-    r.keep = j.keep;
-    r.red = j.red;
+    grid += j.grid;
+    if (j.is_sum()) { g.s[g.n_sums++] = sum_args(j); continue; }
+    RedArgs& r = g.j[g.n++];
+    r.keep = two(j.keep);
+    r.red = two(j.red);
     r.n_out = j.n_out;
     r.R = j.R;
     r.Q = j.Q;
@@ -703,7 +907,6 @@ hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int 
     r.a = j.a;
     r.b = j.b;
     r.out = j.out;
-    grid += j.grid;
   }
   if (jobs[0]->dtype == HGPU_F64) hipLaunchKernelGGL((k_contract_group<double>), dim3(grid), dim3(kBlock), 0, ctx->stream, g);
   else hipLaunchKernelGGL((k_contract_group<float>), dim3(grid), dim3(kBlock), 0, ctx->stream, g);
@@ -729,7 +932,7 @@ int64_t min_abs_nonzero(const Dims& d, int dim) {
 // live in `scratch` when the caller brings one (then nothing is allocated here,
 // and a request whose partial sums exceed scratch_bytes is refused), else in a
 // block from the context's allocator.
-int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, void* out, void* scratch, size_t scratch_bytes, hgpu_buffer* out_buf = nullptr) {
+int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, void* out, void* scratch, size_t scratch_bytes, const hgpu_array* out_arr = nullptr) {
   int64_t n_out = 1, R = 1;
   for (int i = 0; i < n_keep; ++i) n_out *= a->shape[i];
   for (int i = n_keep; i < a->rank; ++i) R *= a->shape[i];
@@ -771,17 +974,18 @@ int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_
   const void* pb = b ? data_ptr(b) : nullptr;
   int rc = HGPU_OK;
   // (a caller that brings its own scratch wants its result written by the time the call returns to the stream: not held)
-  HoldBufs hb{a->buf, b ? b->buf : nullptr, out_buf};
-  const HoldBufs* hold = (out_buf && !scratch && a->buf && (!b || b->buf) && (a->dtype == HGPU_F64 || a->dtype == HGPU_F32)) ? &hb : nullptr;
+  HoldBufs hb{a->buf, b ? b->buf : nullptr, out_arr ? out_arr->buf : nullptr};
+  const bool fresh = scratch == nullptr;
+  const HoldBufs* hold = (hb.out && !scratch && a->buf && (!b || b->buf) && (a->dtype == HGPU_F64 || a->dtype == HGPU_F32)) ? &hb : nullptr;
   if (use_wave && ((n_out >= 64 && (n_out <= 1024 || S > 1) && R >= 1024 && R <= 65536) || (n_out < 64 && S > 1 && R >= 1024 && R <= 16384))) {
     // a few hundred outputs of a few thousand elements (or a handful of outputs, or so many that a wavefront each
     // leaves the device half empty, that would otherwise take a launch for partial sums and a second one to add them):
     // a block per output, one launch.  2048 rows of 8192 fp32: 17.2 us in two chunks a row and 4.7 to add them, 19.0 so.
     // Gradients, us, chunks / a block per output: wide dense network 1602 / 1557, recurrent network at batch 5000 (1280
     // outputs of 5000) 881 / 863.
-    HG_DISPATCH_DTYPE(a->dtype, T, rc = (launch_stage<T, T>(ctx, true, keep, red, n_out, R, 0, pa, pb, out, nullptr, hold, a->dtype)));
+    HG_DISPATCH_DTYPE(a->dtype, T, rc = (launch_stage<T, T>(ctx, true, keep, red, n_out, R, 0, pa, pb, out, nullptr, hold, a->dtype, fresh)));
   } else if (S == 1) {
-    HG_DISPATCH_DTYPE(a->dtype, T, rc = (launch_stage<T, T>(ctx, use_wave, keep, red, n_out, R, 1, pa, pb, out, nullptr, hold, a->dtype)));
+    HG_DISPATCH_DTYPE(a->dtype, T, rc = (launch_stage<T, T>(ctx, use_wave, keep, red, n_out, R, 1, pa, pb, out, nullptr, hold, a->dtype, fresh)));
   } else {
     // stage 1: partials [n_out, S] in the accumulator type; stage 2 sums them.
     const size_t need = (size_t)n_out * (size_t)S * 8;
@@ -797,8 +1001,11 @@ int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_
       pp = part->ptr;
     }
     int64_t psh[2] = {n_out, S}, pst[2] = {S, 1};
-    HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<T, A>(ctx, use_wave, keep, red, n_out, R, (int)S, pa, pb, pp)); });
-    if (!rc) {
+    HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<T, A>(ctx, use_wave, keep, red, n_out, R, (int)S, pa, pb, pp, nullptr, nullptr, -1, fresh)); });
+    const bool few_long = n_out < 256 && S >= 256;
+    if (!rc && hold && n_out < 65536 && !few_long) {
+      rc = sum_partial_rows(ctx, a->dtype, n_out, S, part, out_arr);
+    } else if (!rc) {
       Dims k2, r2;
       int64_t z1[1] = {0};
       const int64_t* ks2[2] = {pst, z1};
@@ -807,7 +1014,7 @@ int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_
       collapse(1, psh + 1, 2, rs2, &r2);
       bool wave2 = n_out < 65536;
       // few outputs under many partial sums: a block each (one output, 4096 partial sums: 8.0 us with a wavefront, 4.4 with a block)
-      HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<A, T>(ctx, wave2, k2, r2, n_out, S, n_out < 256 && S >= 256 ? 0 : 1, pp, nullptr, out)); });
+      HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<A, T>(ctx, wave2, k2, r2, n_out, S, few_long ? 0 : 1, pp, nullptr, out, nullptr, nullptr, -1, fresh)); });
     }
     if (part) buffer_release(part);
   }
@@ -887,7 +1094,9 @@ int contract_terms(hgpu_ctx* ctx, int n, const hgpu_array* const* as, const hgpu
   int rc = new_dense(ctx, accdt, 2, psh, &part);
   if (rc) return rc;
   HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<T, A>(ctx, use_wave, keep, red, n_out, R, (int)S_all, tp.a[0], tp.b[0], data_ptr(part), &tp)); });
-  if (!rc) {
+  if (!rc && n_out < 65536 && dtype_is_float(a->dtype)) {
+    rc = sum_partial_rows(ctx, a->dtype, n_out, S_all, part->buf, o);
+  } else if (!rc) {
     Dims k2, r2;
     int64_t z1[1] = {0};
     const int64_t* ks2[2] = {part->strides, z1};
@@ -1012,7 +1221,7 @@ int hgpu_contract(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n
   if (rc) { hgpu_release(o); return rc; }
   if (handled) { *out = o; return HGPU_OK; }
 
-  rc = reduce_views(ctx, a, b, n_keep, data_ptr(o), nullptr, 0, o->buf);
+  rc = reduce_views(ctx, a, b, n_keep, data_ptr(o), nullptr, 0, o);
   if (rc) { hgpu_release(o); return rc; }
   *out = o;
   return HGPU_OK;
@@ -1060,7 +1269,8 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
     const int64_t* ks[1] = {a->strides};
     Dims keep;
     if (!collapse(a->rank - 1, a->shape, 1, ks, &keep)) { hgpu_release(o); if (v) hgpu_release(v); return fail(ctx, HGPU_ERR_UNSUPPORTED, "argminmax: too many dims"); }
-    LaunchGuard lg(ctx, "argminmax", (double)n_out * (L * dtype_size(a->dtype) + 8 + (v ? dtype_size(a->dtype) : 0)), (double)n_out * L);
+    const std::vector<const void*> reads = reads_of(1, &a);
+    LaunchGuard lg(ctx, "argminmax", (double)n_out * (L * dtype_size(a->dtype) + 8 + (v ? dtype_size(a->dtype) : 0)), (double)n_out * L, &reads);
     void* vp = v ? data_ptr(v) : nullptr;
     if (L >= 16384 && n_out <= 16) {
       // very few, very long rows: pieces of a row to many blocks, then one pick per row

@@ -1176,10 +1176,6 @@ void remember_sum(hgpu_ctx* ctx, const VirtualOp& v, const std::vector<int>& kep
 
 namespace hg {
 
-// gemm.hip: out[i] = sum over the `parts` partial outputs of part[s * n + i], in a fixed order.
-int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, const void* part, void* out);
-int sum_partials_split(hgpu_ctx* ctx, int dtype, int64_t n1, int64_t n2, int parts, const void* part, void* out1, void* out2);
-
 int try_footprint_virtual(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* pa, const void* pb, hgpu_array* out, bool* handled,
                           const void* va_, const void* vb_);
 
@@ -1331,13 +1327,15 @@ int try_footprint_virtual(hgpu_ctx* ctx, const GemmParams& p, int dtype, const v
       label = intern_label(ctx, buf);
     }
     {
-      LaunchGuard lg(ctx, label, bytes, flops);
+      std::vector<const void*> reads{pa, pb};
+      reads.insert(reads.end(), vxa.begin(), vxa.end());
+      reads.insert(reads.end(), vya.begin(), vya.end());
+      LaunchGuard lg(ctx, label, bytes, flops, &reads);
       hipError_t e = launch_module(lg, kernel.fn, (unsigned)grid, 256u * (unsigned)pl.ks, args.data());
       if (e != hipSuccess) { if (part) buffer_release(part); if (colsum) hgpu_release(colsum); return check_hip(ctx, e, "footprint gemm launch"); }
     }
     if (pl.mode == 0) {
-      int rc = colsum ? sum_partials_split(ctx, dtype, out_n, n_colsum, (int)grid, (const void*)part->ptr, data_ptr(out), data_ptr(colsum))
-                      : sum_partials(ctx, dtype, out_n, (int)grid, (const void*)part->ptr, data_ptr(out));
+      int rc = colsum ? sum_partials(ctx, dtype, out_n + n_colsum, (int)grid, part, out, out_n, colsum) : sum_partials(ctx, dtype, out_n, (int)grid, part, out);
       buffer_release(part);
       if (rc) { if (colsum) hgpu_release(colsum); return rc; }
       if (colsum) remember_sum(ctx, *vy, colsum_dims, colsum);
@@ -1805,7 +1803,9 @@ int try_contract_map(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, in
                has_ext ? (L == 4 ? ",ext4" : (L == 2 ? ",ext2" : ",ext1")) : "");
       label = intern_label(ctx, buf);
     }
-    LaunchGuard lg(ctx, label, bytes, flops);
+    std::vector<const void*> reads{pa, pb};
+    reads.insert(reads.end(), ea.begin(), ea.end());
+    LaunchGuard lg(ctx, label, bytes, flops, &reads);
     hipError_t err = launch_module(lg, kernel.fn, (unsigned)grid, 256u * (unsigned)pl.ks, args);
     if (err != hipSuccess) { release_all(); return check_hip(ctx, err, "contract_map launch"); }
   }
@@ -2193,12 +2193,12 @@ int try_mapped_sum(hgpu_ctx* ctx, const VirtualOp& v, const hgpu_operand* o, int
       snprintf(buf, sizeof buf, "mapped_sum[out%lld,R%lld,S%lld,in%d,instr%d,vec%d%s]", (long long)n_out, (long long)R, (long long)S, v.n_in, v.n_instr, W, v.padded ? ",padded" : "");
       label = intern_label(ctx, buf);
     }
-    LaunchGuard lg(ctx, label, bytes, (double)n_out * R * (v.n_instr + 1));
+    LaunchGuard lg(ctx, label, bytes, (double)n_out * R * (v.n_instr + 1), &vxa);
     hipError_t e = launch_module(lg, it->second.fn, (unsigned)(n_out * S), 256, args);
     if (e != hipSuccess) { if (part) buffer_release(part); return check_hip(ctx, e, "mapped_sum launch"); }
   }
   if (part) {
-    int rc = hg::sum_partials(ctx, v.dtype, n_out, (int)S, part->ptr, data_ptr(out));
+    int rc = hg::sum_partials(ctx, v.dtype, n_out, (int)S, part, out);
     buffer_release(part);
     if (rc) return rc;
   }
@@ -2645,11 +2645,13 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
       snprintf(buf, sizeof buf, "onehot_contract[rows%d,cols%d,chunks%lld,positions%lld,onehot%lld,in%d,instr%d,es%d]", MR, NC, (long long)nch, (long long)G, (long long)EH, v.n_in, v.n_instr, es);
       label = intern_label(ctx, buf);
     }
-    LaunchGuard lg(ctx, label, bytes, 2.0 * MR * NC * (double)G * (double)nch);
+    std::vector<const void*> reads = ia;
+    reads.push_back(data_ptr(x));
+    LaunchGuard lg(ctx, label, bytes, 2.0 * MR * NC * (double)G * (double)nch, &reads);
     hipError_t e = launch_module(lg, kn.c.fn, (unsigned)grid, 256, args);
     if (e != hipSuccess) { buffer_release(part); hgpu_release(colsum); return check_hip(ctx, e, "onehot_contract launch"); }
   }
-  rc = hg::sum_partials_split(ctx, v.dtype, out_n, NC, (int)grid, part->ptr, data_ptr(out), data_ptr(colsum));
+  rc = hg::sum_partials(ctx, v.dtype, out_n + NC, (int)grid, part, out, out_n, colsum);
   buffer_release(part);
   if (rc) { hgpu_release(colsum); return rc; }
   remember_sum(ctx, v, colk, colsum);

@@ -100,7 +100,6 @@ struct FDims {
 }  // namespace
 
 namespace hg {
-int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, const void* part, void* out);
 }
 
 // hgpu_fused_map, and with sum_slot >= 0 hgpu_fused_map_dimsum: the same pass
@@ -481,7 +480,8 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     for (int o = 0; o < n_out; ++o) outs[o] = res[(size_t)o];
     return HGPU_OK;
   }
-  std::unique_ptr<LaunchGuard> guard(new LaunchGuard(ctx, label, bytes, (double)n * n_instr));   // ends before the partial sums' own launch
+  const std::vector<const void*> reads = reads_of(n_in, in);
+  std::unique_ptr<LaunchGuard> guard(new LaunchGuard(ctx, label, bytes, (double)n * n_instr, &reads));   // ends before the partial sums' own launch
   LaunchGuard& lg = *guard;
   Compiled kernel;
   if (int rc = kernel_for(ctx, key, hit, src, kernel_name, &kernel)) { release_all(); return rc; }
@@ -511,7 +511,7 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
   if (e != hipSuccess) { if (part) buffer_release(part); if (sums) hgpu_release(sums); release_all(); return check_hip(ctx, e, "fused_map launch"); }
   guard.reset();
   if (part) {
-    int rc = hg::sum_partials(ctx, dt[(size_t)sum_slot], dsC, (int)ds_chunks, part->ptr, data_ptr(sums));
+    int rc = hg::sum_partials(ctx, dt[(size_t)sum_slot], dsC, (int)ds_chunks, part, sums);
     buffer_release(part);
     if (rc) { hgpu_release(sums); release_all(); return rc; }
   }
@@ -657,7 +657,8 @@ extern "C" int hgpu_fused_extremum(hgpu_ctx* ctx, int n_in, const hgpu_array* co
       if (in[i]->strides[d] != 0) distinct *= in[i]->shape[d];
     bytes += (double)distinct * dtype_size(in[i]->dtype);
   }
-  LaunchGuard lg(ctx, label, bytes, (double)n_out * L * (n_instr + 1));
+  const std::vector<const void*> reads = reads_of(n_in, in);
+  LaunchGuard lg(ctx, label, bytes, (double)n_out * L * (n_instr + 1), &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_extremum", &kernel);
   if (rc) { hgpu_release(v); hgpu_release(ix); return rc; }
@@ -861,7 +862,8 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
       if (data_ptr(in[j]) == data_ptr(in[i]) && layout[(size_t)j] != 's') dup = true;
     if (!dup) bytes += (double)n * dtype_size(in[i]->dtype);
   }
-  LaunchGuard lg(ctx, label, bytes, (double)n * (n_instr + 1));
+  const std::vector<const void*> reads = reads_of(n_in, in);
+  LaunchGuard lg(ctx, label, bytes, (double)n * (n_instr + 1), &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_sum", &kernel);
   if (rc) { drop_part(); hgpu_release(o); return rc; }
@@ -1052,7 +1054,8 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     if (!dup) bytes += (double)n * dtype_size(in[i]->dtype);
   }
   for (int o = 0; o < n_out; ++o) bytes += (double)n * dtype_size(res[(size_t)o]->dtype);
-  LaunchGuard lg(ctx, label, bytes, (double)n * n_instr);
+  const std::vector<const void*> reads = reads_of(n_in, in);
+  LaunchGuard lg(ctx, label, bytes, (double)n * n_instr, &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_map_sums", &kernel);
   if (rc) { drop_part(); release_all(); return rc; }

@@ -53,79 +53,6 @@ __global__ void k_koff(Group k, int64_t K, int64_t Kp, int64_t* __restrict__ ka,
   }
 }
 
-// Sums the split-K partials: out[i] = sum_s part[s * stride + i].  A block owns
-// OPB consecutive outputs; its 256 / OPB groups of lanes each take every
-// (256 / OPB)-th partial (coalesced rows of OPB elements), several loads in
-// flight at a time, and combine through LDS in a fixed order.  Few outputs get
-// the narrow blocks: more of them, and fewer partials for a lane to walk through.
-template <typename T, int OPB>
-__global__ void __launch_bounds__(256) k_sum_partials(int64_t n, int S, int64_t stride, const T* __restrict__ part, T* __restrict__ out, int64_t n1, T* __restrict__ out2) {
-  constexpr int G = 256 / OPB;
-  __shared__ T red[G][OPB + 1];
-  const int ol = threadIdx.x % OPB, g = threadIdx.x / OPB;
-  for (int64_t base = (int64_t)blockIdx.x * OPB; base < n; base += (int64_t)gridDim.x * OPB) {
-    int64_t i = base + ol;
-    T acc = T(0);
-    if (i < n) {
-#pragma unroll 8
-      for (int s = g; s < S; s += G) acc += part[(int64_t)s * stride + i];
-    }
-    red[g][ol] = acc;
-    __syncthreads();
-    if (g == 0 && i < n) {
-      T t = red[0][ol];
-#pragma unroll
-      for (int k = 1; k < G; ++k) t += red[k][ol];
-      if (i < n1) out[i] = t;
-      else out2[i - n1] = t;
-    }
-    __syncthreads();
-  }
-}
-
-// The same sum for a handful of partials (S <= 8), where the blocks above would
-// leave most of their lane groups without a partial: one output per lane, the
-// partials added in the same order (0 + p0 + p1 + ...), four loads in flight.
-template <typename T>
-__global__ void __launch_bounds__(256) k_sum_partials_few(int64_t n, int S, int64_t stride, const T* __restrict__ part, T* __restrict__ out, int64_t n1, T* __restrict__ out2) {
-  const int64_t step = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
-    const T* p = part + i;
-    T acc = T(0);
-    int s = 0;
-    for (; s + 3 < S; s += 4) {
-      const T a = p[(int64_t)s * stride], b = p[(int64_t)(s + 1) * stride], c = p[(int64_t)(s + 2) * stride], d = p[(int64_t)(s + 3) * stride];
-      acc += a;
-      acc += b;
-      acc += c;
-      acc += d;
-    }
-    if (s + 1 < S) {
-      const T a = p[(int64_t)s * stride], b = p[(int64_t)(s + 1) * stride];
-      acc += a;
-      acc += b;
-      s += 2;
-    }
-    if (s < S) acc += p[(int64_t)s * stride];
-    if (i < n1) out[i] = acc;
-    else out2[i - n1] = acc;
-  }
-}
-
-// Outputs [0, n1) go to `out`, the rest to `out2` (two results whose partial sums one kernel wrote side by side).
-template <typename T>
-void launch_sum_partials(hgpu_ctx* ctx, int64_t n, int S, const T* part, T* out, int64_t n1 = -1, T* out2 = nullptr) {
-  if (n1 < 0) n1 = n;
-  if (S <= 8)
-    hipLaunchKernelGGL((k_sum_partials_few<T>), dim3(grid_for(n, 256, ctx->num_cu * 8)), dim3(256), 0, ctx->stream, n, S, n, part, out, n1, out2);
-  else if (sizeof(T) == 4)   // rows of 32 floats are whole 128-byte lines (16384 outputs x 270 partials: 12.9 us with rows of 8, 7.1 us with rows of 32)
-    hipLaunchKernelGGL((k_sum_partials<T, 32>), dim3(grid_for(n, 32, ctx->num_cu * 8)), dim3(256), 0, ctx->stream, n, S, n, part, out, n1, out2);
-  else if (n <= 32768 && S >= 32)
-    hipLaunchKernelGGL((k_sum_partials<T, 8>), dim3(grid_for(n, 8, ctx->num_cu * 8)), dim3(256), 0, ctx->stream, n, S, n, part, out, n1, out2);
-  else
-    hipLaunchKernelGGL((k_sum_partials<T, 32>), dim3(grid_for(n, 32, ctx->num_cu * 8)), dim3(256), 0, ctx->stream, n, S, n, part, out, n1, out2);
-}
-
 // Appends dim (extent e, strides a, b, c) to a group, merging with the previous dim when all strides allow.
 bool push_dim(Group& g, int64_t e, int64_t a, int64_t b, int64_t c) {
   if (e == 1) return true;
@@ -164,6 +91,14 @@ int64_t total(const Group& g) {
   int64_t n = 1;
   for (int i = 0; i < g.nd; ++i) n *= g.shape[i];
   return n;
+}
+
+// What a product's launch reads: see LaunchGuard.
+std::vector<const void*> product_reads(const void* pa, const void* pb, int n_terms, const void* const* as, const void* const* bs) {
+  std::vector<const void*> r{pa, pb};
+  r.insert(r.end(), as, as + n_terms);
+  r.insert(r.end(), bs, bs + n_terms);
+  return r;
 }
 
 // True when 16-byte loads along the direction the staging lanes run are safe
@@ -238,7 +173,8 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
     }
     // the helper launches are timed under their own names, the label times the MFMA kernel alone
     if (p.k.nd > 1) {
-      LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0);
+      const std::vector<const void*> none;
+      LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0, &none);
       hipLaunchKernelGGL(k_koff, dim3((unsigned)((Kp + 255) / 256)), dim3(256), 0, ctx->stream, p.k, p.K, Kp, ka, kb);
       p.kmask = -1;
       p.ksa = p.ksb = 0;
@@ -264,21 +200,19 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
     const bool va = k_vector(pa, p.a_term, p.k.sa, p.m.sa, p.m, p.bt.sa), vb = k_vector(pb, p.b_term, p.k.sb, p.n.sb, p.n, p.bt.sb);
     LaunchArgs la{ctx->stream, -1, tm, tn, va, vb, grid, pa, pb, cdst, ka, kb};
     {
-      LaunchGuard lg(ctx, label, bytes, flops);
+      const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
+      LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
       if (dtype == HGPU_F64) launch_f64(p, la);
       else launch_f32(p, la);
     }
-    if (split > 1) {
-      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * es, (double)out_n * split);
-      if (dtype == HGPU_F64) launch_sum_partials<double>(ctx, out_n, (int)split, (const double*)part->ptr, (double*)data_ptr(out));
-      else launch_sum_partials<float>(ctx, out_n, (int)split, (const float*)part->ptr, (float*)data_ptr(out));
-    }
+    if (split > 1) rc = sum_partials(ctx, dtype, out_n, (int)split, part, out);
   }
   hipError_t e = hipGetLastError();
   buffer_release(koff);
   if (part) buffer_release(part);
+  if (rc) return rc;
   if (e != hipSuccess) return check_hip(ctx, e, "gemm");
   *handled = true;
   return HGPU_OK;
@@ -364,8 +298,9 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
   split = (int)(q.term_split * nt);
   if (split > 65535 || tiles * split > 0x3fffffff || (split > 1 && (double)out_n * split > 5e8)) return HGPU_OK;
   hgpu_buffer* part = nullptr;
+  int rc = HGPU_OK;
   if (split > 1) {
-    int rc = buffer_alloc(ctx, (size_t)(out_n * split * es), &part);
+    rc = buffer_alloc(ctx, (size_t)(out_n * split * es), &part);
     if (rc) return rc;
   }
   q.c_split_stride = split > 1 ? out_n : 0;
@@ -384,7 +319,8 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
     LaunchArgs la{ctx->stream, 0, 0, 0, sak == 1, sbk == 1, dim3((unsigned)tiles, (unsigned)split, (unsigned)p.BT), swap ? pb : pa, swap ? pa : pb, cdst, nullptr, nullptr};
     {
-      LaunchGuard lg(ctx, label, bytes, flops);
+      const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
+      LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
       if (f64) launch_wide_f64(q, la);
@@ -397,13 +333,12 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       dense_strides(out->rank + 1, sh, st);
       *partials_out = new_view(ctx, part, dtype, out->rank + 1, sh, st, 0);
     } else if (split > 1) {
-      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * es, (double)out_n * split);
-      if (f64) launch_sum_partials<double>(ctx, out_n, split, (const double*)part->ptr, (double*)data_ptr(out));
-      else launch_sum_partials<float>(ctx, out_n, split, (const float*)part->ptr, (float*)data_ptr(out));
+      rc = sum_partials(ctx, dtype, out_n, (int)split, part, out);
     }
   }
   const hipError_t e = hipGetLastError();
   if (part) buffer_release(part);
+  if (rc) return rc;
   if (e != hipSuccess) {
     if (partials_out && *partials_out) { hgpu_release(*partials_out); *partials_out = nullptr; }
     return check_hip(ctx, e, "gemm");
@@ -472,26 +407,6 @@ bool classify_contraction(int rank, const int64_t* shape, const int64_t* st_a, c
   p->K = total(p->k);
   p->BT = total(p->bt);
   return true;
-}
-
-int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, const void* part, void* out) {
-  size_t es = dtype_size(dtype);
-  LaunchGuard ls(ctx, "gemm_sum_partials", (double)n * (parts + 1) * es, (double)n * parts);
-  if (dtype == HGPU_F64) launch_sum_partials<double>(ctx, n, parts, (const double*)part, (double*)out);
-  else launch_sum_partials<float>(ctx, n, parts, (const float*)part, (float*)out);
-  HG_CHECK_LAUNCH(ctx, "gemm_sum_partials");
-  return HGPU_OK;
-}
-
-// `parts` partial results of n1 + n2 elements each: the first n1 summed into out1, the other n2 into out2.
-int sum_partials_split(hgpu_ctx* ctx, int dtype, int64_t n1, int64_t n2, int parts, const void* part, void* out1, void* out2) {
-  const size_t es = dtype_size(dtype);
-  const int64_t n = n1 + n2;
-  LaunchGuard ls(ctx, "gemm_sum_partials", (double)n * (parts + 1) * es, (double)n * parts);
-  if (dtype == HGPU_F64) launch_sum_partials<double>(ctx, n, parts, (const double*)part, (double*)out1, n1, (double*)out2);
-  else launch_sum_partials<float>(ctx, n, parts, (const float*)part, (float*)out1, n1, (float*)out2);
-  HG_CHECK_LAUNCH(ctx, "gemm_sum_partials");
-  return HGPU_OK;
 }
 
 int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, hgpu_array* out, bool* handled,
@@ -715,7 +630,8 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     }
     // the helper launches are timed under their own names, the label times the MFMA kernel alone
     if (p.k.nd > 1) {
-      LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0);
+      const std::vector<const void*> none;
+      LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0, &none);
       hipLaunchKernelGGL(k_koff, dim3((unsigned)((Kp + 255) / 256)), dim3(256), 0, ctx->stream, p.k, p.K, Kp, ka, kb);
       p.kmask = -1;
       p.ksa = p.ksb = 0;
@@ -728,7 +644,8 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
     LaunchArgs la{ctx->stream, cfg, 0, 0, va, vb, grid, data_ptr(a), data_ptr(b), cdst, ka, kb};
     {
-      LaunchGuard lg(ctx, label, bytes, flops);
+      const std::vector<const void*> reads = product_reads(data_ptr(a), data_ptr(b), n_terms, p.a_term, p.b_term);
+      LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
       if (a->dtype == HGPU_F64) launch_f64(p, la);
@@ -741,14 +658,13 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
       dense_strides(out->rank + 1, sh, st);
       *partials_out = new_view(ctx, part, a->dtype, out->rank + 1, sh, st, 0);
     } else if (split > 1) {
-      LaunchGuard ls(ctx, "gemm_sum_partials", (double)out_n * (split + 1) * es, (double)out_n * split);
-      if (a->dtype == HGPU_F64) launch_sum_partials<double>(ctx, out_n, (int)split, (const double*)part->ptr, (double*)data_ptr(out));
-      else launch_sum_partials<float>(ctx, out_n, (int)split, (const float*)part->ptr, (float*)data_ptr(out));
+      rc = sum_partials(ctx, a->dtype, out_n, (int)split, part, out);
     }
   }
   hipError_t e = hipGetLastError();
   buffer_release(koff);
   if (part) buffer_release(part);
+  if (rc) return rc;
   if (e != hipSuccess) {
     if (partials_out && *partials_out) { hgpu_release(*partials_out); *partials_out = nullptr; }
     return check_hip(ctx, e, "gemm");

@@ -725,12 +725,14 @@ struct Deferred {
 };
 
 // Products, reductions and elementwise passes write new arrays only; copies write
-// existing ones.  The queue holds either products and reductions, or elementwise
-// passes that read no result of one another, or copies that touch no memory of one
-// another: whatever does not fit flushes it first.
+// existing ones.  The queue holds either products and reductions, and beside them
+// elementwise passes that read no result of one another, or copies that touch no memory
+// of one another: whatever does not fit flushes it first.  No held pass reads the
+// result of a held product or reduction, and none of those the result of a held pass.
 struct DeferredQueue {
   std::vector<Deferred> items;
-  enum Kind { kProducts, kMaps, kCopies } kind = kProducts;     // what `items` holds
+  enum Kind { kProducts, kCopies } kind = kProducts;     // what `items` holds
+  std::vector<Deferred> maps;
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
 };
@@ -741,6 +743,8 @@ namespace {
 }  // namespace
 
 namespace hg {
+
+static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d);
 
 // outs[i] (dense, of the kept shape, allocated by the caller) = slot
 // out_slots[i] of the program over sum_t contract(as[t], bs[t]).  *handled says
@@ -885,17 +889,12 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     for (int i = 0; i < n_in; ++i)
       if (i != c_slot) d.reads.push_back(in[i]->buf);
     for (int o = 0; o < n_out; ++o) d.writes.push_back(outs[o]->buf);
-    for (auto* b : d.reads) buffer_retain(b);
-    for (auto* b : d.writes) buffer_retain(b);
     std::lock_guard<std::mutex> lk(ctx->launch_mu);
-    if (!ctx->dq) ctx->dq = new DeferredQueue;
-    if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
-    ctx->dq->items.push_back(std::move(d));
-    ctx->dq_pending = true;
+    hold_item_locked(ctx, std::move(d));
     *handled = true;
     return HGPU_OK;
   }
-  LaunchGuard lg(ctx, d.label, d.bytes, d.flops);
+  LaunchGuard lg(ctx, d.label, d.bytes, d.flops, &d.args);
   void* args[] = {(void*)d.args.data()};
   hipError_t err = launch_module(lg, d.fn, d.grid, 256, args, true, finish_fn == nullptr);
   if (err == hipSuccess && finish_fn) err = launch_module(lg, finish_fn, (unsigned)((ntiles + 7) / 8 * 8), 256, args, false, true);
@@ -947,31 +946,23 @@ static void launch_maps(hgpu_ctx* ctx, std::vector<Deferred>& items) {
   }
 }
 
+static void release_held(std::vector<Deferred>& items) {
+  for (auto& d : items) {
+    for (auto* b : d.reads) buffer_release(b);
+    for (auto* b : d.writes) buffer_release(b);
+  }
+}
+
 // Launches what was held back.  Products are levelled by who reads whose
 // results (arrays are never written twice, so reads-after-writes are the only
 // order there is); the members of one level are independent and go out
 // together, the levels one after another.  For an unrolled recurrence of two
 // layers, issued layer by layer, level k holds step k + 1 of the first layer
 // and step k of the second: the diagonal of the time x layer grid.
-void flush_deferred_locked(hgpu_ctx* ctx) {
-  ctx->dq_pending = false;
-  if (!ctx->dq || ctx->dq->items.empty()) return;
-  std::vector<Deferred> items;
-  items.swap(ctx->dq->items);
+static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, DeferredQueue::Kind kind) {
+  if (items.empty()) return;
   (void)hipSetDevice(ctx->device);
-  auto release_items = [&] {
-    for (auto& d : items) {
-      for (auto* b : d.reads) buffer_release(b);
-      for (auto* b : d.writes) buffer_release(b);
-    }
-  };
-  const DeferredQueue::Kind kind = ctx->dq->kind;
-  ctx->dq->kind = DeferredQueue::kProducts;
-  if (kind == DeferredQueue::kMaps) {
-    launch_maps(ctx, items);
-    release_items();
-    return;
-  }
+  auto release_items = [&] { release_held(items); };
   if (kind == DeferredQueue::kCopies) {
     std::vector<const CopyJob*> jobs;
     double bytes = 0;
@@ -1063,7 +1054,7 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
     top = std::max(top, d.level);
   }
   for (int lv = 0; lv <= top; ++lv) {
-    // the level's reductions: those of one element type go out together, four at a time
+    // the level's reductions and sums of partial results: those of one element type go out together
     {
       std::vector<Deferred*> reds;
       for (auto& d : items)
@@ -1071,8 +1062,10 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
       std::stable_sort(reds.begin(), reds.end(), [](const Deferred* a, const Deferred* b) { return a->red.dtype < b->red.dtype; });
       for (size_t g0 = 0; g0 < reds.size();) {
         size_t g1 = g0 + 1;
-        while (g1 < reds.size() && g1 - g0 < 4 && reds[g1]->red.dtype == reds[g0]->red.dtype) ++g1;
-        const RedJob* jobs[4];
+        int n_sums = reds[g0]->red.is_sum() ? 1 : 0, n_reds = 1 - n_sums;
+        for (; g1 < reds.size() && reds[g1]->red.dtype == reds[g0]->red.dtype; ++g1)
+          if (reds[g1]->red.is_sum() ? ++n_sums > kMaxGroupSums : ++n_reds > kMaxGroupReductions) break;
+        const RedJob* jobs[kMaxGroupReductions + kMaxGroupSums];
         double bytes = 0, flops = 0;
         for (size_t i = g0; i < g1; ++i) { jobs[i - g0] = &reds[i]->red; bytes += reds[i]->bytes; flops += reds[i]->flops; }
         const char* label = reds[g0]->label;
@@ -1166,9 +1159,88 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
   release_items();
 }
 
+static void flush_maps_locked(hgpu_ctx* ctx) {
+  std::vector<Deferred> maps;
+  maps.swap(ctx->dq->maps);
+  ctx->dq_pending = !ctx->dq->items.empty();
+  if (maps.empty()) return;
+  (void)hipSetDevice(ctx->device);
+  launch_maps(ctx, maps);
+  release_held(maps);
+}
+
+static void flush_items_locked(hgpu_ctx* ctx) {
+  std::vector<Deferred> items;
+  items.swap(ctx->dq->items);
+  ctx->dq_pending = !ctx->dq->maps.empty();
+  const DeferredQueue::Kind kind = ctx->dq->kind;
+  ctx->dq->kind = DeferredQueue::kProducts;
+  launch_held_locked(ctx, items, kind);
+}
+
+void flush_deferred_locked(hgpu_ctx* ctx) {
+  ctx->dq_pending = false;
+  if (!ctx->dq) return;
+  flush_items_locked(ctx);
+  flush_maps_locked(ctx);
+}
+
+// The blocks of `reads` that a held item writes.
+static std::set<const hgpu_buffer*> written_by(const std::vector<Deferred>& items, const std::vector<const void*>& reads) {
+  std::set<const hgpu_buffer*> s;
+  for (auto& d : items)
+    for (auto* w : d.writes)
+      for (const void* r : reads)
+        if (r >= w->ptr && r < (const char*)w->ptr + w->bytes) s.insert(w);
+  return s;
+}
+
+// A product or reduction joins the queue (which retains its buffers).
+static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
+  for (auto* b : d.reads) buffer_retain(b);
+  for (auto* b : d.writes) buffer_retain(b);
+  if (!ctx->dq) ctx->dq = new DeferredQueue;
+  DeferredQueue& q = *ctx->dq;
+  if (q.items.size() >= kMaxHeld || q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
+  if (!q.maps.empty()) {
+    std::vector<const void*> reads;
+    for (auto* b : d.reads) reads.push_back(b->ptr);
+    if (!written_by(q.maps, reads).empty()) flush_maps_locked(ctx);
+  }
+  q.items.push_back(std::move(d));
+  ctx->dq_pending = true;
+}
+
+// Only reductions and sums of partial results wait beyond the launch that asks: they are the ends of a reverse pass's
+// branches, and the later they go out the more of them share a launch.  Held products go with the first that is needed,
+// as before: their groups and chains are found among all of them.
+void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads) {
+  DeferredQueue& q = *ctx->dq;
+  if (q.kind != DeferredQueue::kProducts) {
+    flush_deferred_locked(ctx);
+    return;
+  }
+  if (!q.maps.empty() && !written_by(q.maps, reads).empty()) flush_maps_locked(ctx);
+  std::set<const hgpu_buffer*> needed = written_by(q.items, reads);
+  if (needed.empty()) return;
+  // an item reads results of earlier ones only: from the last to the first, what goes out adds what it reads
+  std::vector<char> go(q.items.size(), 0);
+  for (size_t i = q.items.size(); i-- > 0;) {
+    Deferred& d = q.items[i];
+    go[i] = !d.is_reduction;
+    for (auto* w : d.writes) go[i] = go[i] || needed.count(w);
+    if (go[i]) needed.insert(d.reads.begin(), d.reads.end());
+  }
+  std::vector<Deferred> out, stay;
+  for (size_t i = 0; i < q.items.size(); ++i) (go[i] ? out : stay).push_back(std::move(q.items[i]));
+  q.items.swap(stay);
+  ctx->dq_pending = !q.items.empty() || !q.maps.empty();
+  launch_held_locked(ctx, out, DeferredQueue::kProducts);
+}
+
 // A single-launch reduction joins the queue: held back until something else needs the stream, levelled with
 // the held products by who reads whose results, and launched together with the other reductions of its level.
-bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write) {
+bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write, hgpu_buffer* write2) {
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
   if (!hold || !write) return false;
   Deferred d;
@@ -1180,34 +1252,29 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
   for (int i = 0; i < n_reads; ++i)
     if (reads[i]) d.reads.push_back(reads[i]);
   d.writes.push_back(write);
-  for (auto* b : d.reads) buffer_retain(b);
-  for (auto* b : d.writes) buffer_retain(b);
+  if (write2) d.writes.push_back(write2);
   std::lock_guard<std::mutex> lk(ctx->launch_mu);
-  if (!ctx->dq) ctx->dq = new DeferredQueue;
-  if (ctx->dq->items.size() >= kMaxHeld || ctx->dq->kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
-  ctx->dq->items.push_back(std::move(d));
-  ctx->dq_pending = true;
+  hold_item_locked(ctx, std::move(d));
   return true;
 }
 
 // An elementwise pass joins the queue: it waits for passes that read none of the held results (an optimizer's
-// updates, one per parameter), and goes out when anything else is enqueued.
+// updates, one per parameter), and goes out when something that reads its result, or may do so, is enqueued.
 void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes) {
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
-  bool fits = q.items.empty() || (q.kind == DeferredQueue::kMaps && q.items.size() < kMaxHeld);
-  for (size_t i = 0; fits && i < q.items.size(); ++i)
-    for (auto* w : q.items[i].writes)
-      for (auto* r : reads) fits = fits && r != w;
-  if (!fits) flush_deferred_locked(ctx);
-  q.items.emplace_back();
-  Deferred& d = q.items.back();
+  std::vector<const void*> from;
+  for (auto* b : reads) from.push_back(b->ptr);
+  // (one reduction asked for sends them all: the next passes, an optimizer's, will ask for the others)
+  if (q.kind != DeferredQueue::kProducts || !written_by(q.items, from).empty()) flush_items_locked(ctx);
+  if (q.maps.size() >= kMaxHeld || !written_by(q.maps, from).empty()) flush_maps_locked(ctx);
+  q.maps.emplace_back();
+  Deferred& d = q.maps.back();
   d.map = std::move(job);
   d.reads = reads;
   d.writes = writes;
   for (auto* b : d.reads) buffer_retain(b);
   for (auto* b : d.writes) buffer_retain(b);
-  q.kind = DeferredQueue::kMaps;
   ctx->dq_pending = true;
 }
 
@@ -1226,7 +1293,7 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
-  bool fits = q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs);
+  bool fits = q.maps.empty() && (q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs));
   for (size_t i = 0; fits && i < q.items.size(); ++i) {
     const hgpu_buffer *r = q.items[i].reads[0], *w = q.items[i].writes[0];
     fits = w != src && w != dst && r != dst;

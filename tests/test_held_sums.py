@@ -1,0 +1,109 @@
+"""Sums of partial results wait for one another (csrc/smallk.hip, make_way_locked; csrc/contract.hip, k_contract_group)."""
+import numpy as np
+import pytest
+
+from conftest import capi
+from test_gemm_split import product
+
+pytestmark = pytest.mark.gpu
+
+EPS = {np.float64: 2.0 ** -53, np.float32: 2.0 ** -24}
+
+
+class Value:
+    """A device array, what it should be and how far it may be from that."""
+
+    def __init__(self, arr, want, bound):
+        self.arr, self.want, self.bound = arr, want, bound
+
+    def check(self):
+        assert np.all(np.abs(self.arr.numpy() - self.want) <= self.bound)
+
+
+def times(gpu, x, y, dt):
+    """x y^T, split along its long inner dim: every product and addition rounds once at most, here and in the split into bf16 parts."""
+    k = x.shape[1]
+    a, b = x.astype(np.float64), y.astype(np.float64)
+    return Value(product(gpu, x, y, "KK"), a @ b.T, 4 * (k + 8) * EPS[dt] * (np.abs(a) @ np.abs(b).T))
+
+
+def row_sums(gpu, x, dt):
+    a = x.astype(np.float64)
+    return Value(gpu.upload(x).contract(None, 1), a.sum(1), 4 * x.shape[1] * EPS[dt] * np.abs(a).sum(1))
+
+
+def add(v, w, dt):
+    s = v.want + w.want
+    return Value(v.arr.ewise2("add", w.arr), s, v.bound + w.bound + 2 * EPS[dt] * (np.abs(s) + v.bound + w.bound))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("count", [1, 2, 5, 14, 27])
+def test_sums_of_many_shapes_together(gpu, dt, count):
+    """More of them than one launch takes (twelve), with a few and with many partial results, whole and partly filled
+    blocks of outputs; every third one is asked for while the others wait."""
+    rng = np.random.default_rng(count)
+    shapes = [(64, 64, 9000), (100, 37, 20000), (300, 130, 5000), (784, 300, 2000), (17, 16, 30000), (128, 128, 16411)]
+    vals, asked = [], []
+    for i in range(count):
+        m, n, k = shapes[i % len(shapes)]
+        vals.append(times(gpu, rng.uniform(-1, 1, (m, k)).astype(dt), rng.uniform(0, 1, (n, k)).astype(dt), dt))
+        if i % 3 == 1:
+            asked.append(add(vals[-1], vals[-1], dt))
+            vals.append(row_sums(gpu, rng.uniform(-1, 1, (100, 70000)).astype(dt), dt))
+    for v in asked + vals:
+        v.check()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("seed", range(4))
+def test_random_orders(gpu, dt, seed):
+    """Products, sums of rows, additions of earlier results and writes into memory that held launches read, in any order."""
+    rng = np.random.default_rng(seed)
+    m, n, k = 96, 80, 6001
+    xs = [rng.uniform(-1, 1, (m, k)).astype(dt) for _ in range(3)]
+    ups = [gpu.upload(x) for x in xs]
+    y = rng.uniform(-1, 1, (n, k)).astype(dt)
+    b = gpu.upload(y)
+    vals = [times(gpu, xs[0], y, dt)]
+    for _ in range(40):
+        what, i = rng.integers(0, 5), int(rng.integers(0, 3))
+        if what < 2:
+            a = xs[i].astype(np.float64)
+            c = y.astype(np.float64)
+            arr = ups[i].replicate([n]).transpose([1, 0, 2]).contract(b.replicate([m]), 2)
+            vals.append(Value(arr, a @ c.T, 4 * (k + 8) * EPS[dt] * (np.abs(a) @ np.abs(c).T)))
+        elif what == 2:
+            two = [v for v in vals if v.want.ndim == 2]
+            vals.append(add(two[int(rng.integers(0, len(two)))], two[-1], dt))
+        elif what == 3:
+            a = xs[i].astype(np.float64)
+            vals.append(Value(ups[i].contract(None, 1), a.sum(1), 4 * k * EPS[dt] * np.abs(a).sum(1)))
+        else:
+            xs[i] = rng.uniform(-1, 1, (m, k)).astype(dt)
+            ups[i].assign(gpu.upload(xs[i]))
+    for v in vals:
+        v.check()
+
+
+def test_a_sum_into_the_callers_array_comes_after_held_reads(gpu):
+    rng = np.random.default_rng(3)
+    x, out = rng.uniform(-1, 1, (100, 5000)), rng.uniform(-1, 1, 100)
+    a, o = gpu.upload(x), gpu.upload(out)
+    before = o.replicate([3000]).contract(None, 0)          # held, reads o
+    a.contract_noalloc(None, 1, o)
+    np.testing.assert_allclose(before.numpy(), out.sum() * 3000, rtol=1e-10, atol=1e-9)
+    np.testing.assert_allclose(o.numpy(), x.sum(1), rtol=1e-10, atol=1e-10)
+
+
+def test_few_launches(gpu):
+    """Three split products and two sums of rows: one launch adds up all their partial results."""
+    rng = np.random.default_rng(4)
+    pairs = [(gpu.upload(rng.uniform(-1, 1, (200, 8000))), gpu.upload(rng.uniform(-1, 1, (100, 8000)))) for _ in range(3)]
+    wide = gpu.upload(rng.uniform(-1, 1, (128, 140000)))
+    gpu.check(gpu.lib.profile_enable(gpu.h, 2))
+    out = [a.replicate([100]).transpose([1, 0, 2]).contract(b.replicate([200]), 2) for a, b in pairs] + [wide.contract(None, 1) for _ in range(2)]
+    out[0].numpy()
+    labels = list(gpu.profile_report())
+    gpu.check(gpu.lib.profile_enable(gpu.h, 0))
+    assert sum(s.startswith("contract_group") or s.startswith("gemm_sum_partials") for s in labels) == 1, labels
