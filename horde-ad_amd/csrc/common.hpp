@@ -191,7 +191,7 @@ struct RedJob {
   int64_t n1 = 0;
   void* out2 = nullptr;
   bool is_sum() const { return variant >= kSumRows; }
-  enum { kSumRows = 3, kSumLane, kSum32, kSum8 };
+  enum { kSumRows = 3, kSumLane, kSum32, kSum8, kSumPair };      // kSumPair: a[i] + b[i]
 };
 constexpr int kMaxGroupReductions = 4, kMaxGroupSums = 12;
 // One dense copy between two arrays that do not overlap (hgpu_assign): `bytes` bytes in units of 2^unit bytes, to which both sides are aligned.
@@ -220,6 +220,8 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
 void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst);
 // contract.hip: launches up to kMaxGroupReductions such reductions and kMaxGroupSums sums of partial results, all of one element type, as one kernel (the caller holds launch_mu)
 hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int n);
+// contract.hip: *acc += x, taking over x (the first term becomes the accumulator); the addition is held back where it can share a launch
+int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now
 bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write, hgpu_buffer* write2 = nullptr);
 // contract.hip: the `parts` partial results of n elements in `part` are added up in `out` (dense), or the first n1 in out1 and the other n - n1 in out2.

@@ -333,6 +333,7 @@ __global__ void __launch_bounds__(kBlock) k_contract_block(Dims keep, Dims red, 
 // the narrow blocks: more of them, and fewer partials for a lane to walk through.
 struct SumArgs {
   const void* part;
+  const void* other;  // kSumPair: the second of two
   void* out;
   void* out2;         // outputs from n1 on
   int64_t n, n1, stride;
@@ -412,9 +413,32 @@ __device__ __forceinline__ void partials_row_body(const SumArgs& g, unsigned bid
   }
 }
 
+// Two results that are added up, the first dense: vectors of 16 bytes where both start at multiples of that.  A second one
+// that is a view (a row's sum, repeated along the row) has rows of n1 elements, `stride` apart, their elements S apart.
+template <typename T>
+__device__ __forceinline__ void pair_body(const SumArgs& g, unsigned bid, unsigned nb) {
+  constexpr int V = 16 / sizeof(T);
+  typedef T Vec __attribute__((ext_vector_type(V)));
+  const T *a = (const T*)g.part, *b = (const T*)g.other;
+  T* o = (T*)g.out;
+  const int64_t at = (int64_t)bid * 256 + threadIdx.x, step = (int64_t)nb * 256;
+  if (g.n1 != g.n) {
+    for (int64_t i = at; i < g.n; i += step) {
+      const int64_t r = i / g.n1;
+      o[i] = a[i] + b[r * g.stride + (i - r * g.n1) * g.S];
+    }
+    return;
+  }
+  const bool wide = (((uintptr_t)a | (uintptr_t)b | (uintptr_t)o) & 15) == 0;
+  const int64_t nv = wide ? g.n / V : 0;
+  for (int64_t i = at; i < nv; i += step) ((Vec*)o)[i] = ((const Vec*)a)[i] + ((const Vec*)b)[i];
+  for (int64_t i = nv * V + at; i < g.n; i += step) o[i] = a[i] + b[i];
+}
+
 template <typename T>
 __device__ __forceinline__ void sum_body(const SumArgs& s, unsigned bid) {
-  if (s.kind == RedJob::kSumRows) partials_row_body<T>(s, bid, s.grid);
+  if (s.kind == RedJob::kSumPair) pair_body<T>(s, bid, s.grid);
+  else if (s.kind == RedJob::kSumRows) partials_row_body<T>(s, bid, s.grid);
   else if (s.kind == RedJob::kSumLane) partials_lane_body<T>(s, bid, s.grid);
   else if (s.kind == RedJob::kSum32) partials_body<T, 32>(s, bid, s.grid);
   else partials_body<T, 8>(s, bid, s.grid);
@@ -422,7 +446,8 @@ __device__ __forceinline__ void sum_body(const SumArgs& s, unsigned bid) {
 
 template <typename T, int KIND>
 __global__ void __launch_bounds__(kBlock) k_sum_partials(SumArgs s) {
-  if (KIND == RedJob::kSumRows) partials_row_body<T>(s, blockIdx.x, gridDim.x);
+  if (KIND == RedJob::kSumPair) pair_body<T>(s, blockIdx.x, gridDim.x);
+  else if (KIND == RedJob::kSumRows) partials_row_body<T>(s, blockIdx.x, gridDim.x);
   else if (KIND == RedJob::kSumLane) partials_lane_body<T>(s, blockIdx.x, gridDim.x);
   else if (KIND == RedJob::kSum32) partials_body<T, 32>(s, blockIdx.x, gridDim.x);
   else partials_body<T, 8>(s, blockIdx.x, gridDim.x);
@@ -803,6 +828,7 @@ static SumArgs sum_args(const RedJob& j) {
   SumArgs s;
   memset(&s, 0, sizeof s);
   s.part = j.a;
+  s.other = j.b;
   s.out = j.out;
   s.out2 = j.out2;
   s.n = j.n_out;
@@ -818,7 +844,8 @@ template <typename T>
 static void launch_sum(hgpu_ctx* ctx, const RedJob& j) {
   const SumArgs s = sum_args(j);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(j.grid), dim3(kBlock), 0, ctx->stream, s); };
-  if (j.variant == RedJob::kSumRows) go(k_sum_partials<T, RedJob::kSumRows>);
+  if (j.variant == RedJob::kSumPair) go(k_sum_partials<T, RedJob::kSumPair>);
+  else if (j.variant == RedJob::kSumRows) go(k_sum_partials<T, RedJob::kSumRows>);
   else if (j.variant == RedJob::kSumLane) go(k_sum_partials<T, RedJob::kSumLane>);
   else if (j.variant == RedJob::kSum32) go(k_sum_partials<T, RedJob::kSum32>);
   else go(k_sum_partials<T, RedJob::kSum8>);
@@ -834,7 +861,8 @@ static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_arr
   j.out2 = out2 ? data_ptr(out2) : nullptr;
   j.label = "gemm_sum_partials";
   j.flops = (double)j.n_out * j.R;
-  if (out1->buf && (!out2 || out2->buf) && (double)part->bytes <= kMaxHeldPartials &&
+  // (Submitted one by one, an objective's value goes out at once: the device would come to it only when the host asks.)
+  if (out1->buf && (!out2 || out2->buf) && (double)part->bytes <= kMaxHeldPartials && (ctx->cap || j.n_out >= 16) &&
       hold_reduction(ctx, j, &part, 1, out1->buf, out2 ? out2->buf : nullptr)) return HGPU_OK;
   const std::vector<const void*> reads{j.a};
   LaunchGuard ls(ctx, j.label, j.bytes, j.flops, &reads);
@@ -853,8 +881,10 @@ int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* pa
   j.R = parts;
   j.sa = n;
   j.bytes = (double)n * (parts + 1) * es;
+  // Rows of 8 for few outputs only: the recurrent network's three sums of 16384 fp64 outputs, 54 partials each, with rows of 8 /
+  // of 32 18.1 / 12.0 us in their group.
   // fp32: rows of 32 are whole 128-byte lines (16384 outputs x 270 partials: 12.9 us with rows of 8, 7.1 us with rows of 32)
-  j.variant = parts <= 8 || (parts <= 64 && n >= 65536) ? RedJob::kSumLane : (es == 4 || n > 32768 || parts < 32) ? RedJob::kSum32 : RedJob::kSum8;
+  j.variant = parts <= 8 || (parts <= 64 && n >= 65536) ? RedJob::kSumLane : (es == 4 || n > 8192 || parts < 32) ? RedJob::kSum32 : RedJob::kSum8;
   j.grid = grid_for(n, j.variant == RedJob::kSumLane ? 256 : j.variant == RedJob::kSum32 ? 32 : 8, ctx->num_cu * 8);
   return queue_sum(ctx, j, part, out1, out2);
 }
@@ -1044,16 +1074,55 @@ int scratch_of(hgpu_ctx* ctx, void** out) {
   return HGPU_OK;
 }
 
+}  // namespace
+
+namespace hg {
 // *acc += x, taking over x (the first term becomes the accumulator).
 int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x) {
   if (!*acc) { *acc = x; return HGPU_OK; }
   hgpu_array* sum = nullptr;
-  int rc = hgpu_ewise2(ctx, HGPU_ADD, *acc, x, &sum);
+  int rc = HGPU_OK;
+  const int64_t n = nelem(x);
+  // Both are results that may be held back: so is their sum, which joins the others' launch (the first step of a
+  // recurrence, its state a constant, apart from the other steps: the sum of the two sent every held sum before it).
+  const hgpu_array *first = *acc, *second = x;
+  if (!is_dense(first)) std::swap(first, second);
+  Dims d;
+  const int64_t* st[1] = {second->strides};
+  const bool rows = n > 0 && collapse(x->rank, x->shape, 1, st, &d) && d.nd <= 2 && d.st[0][d.nd - 1] >= INT32_MIN && d.st[0][d.nd - 1] <= INT32_MAX;
+  if (dtype_is_float(x->dtype) && n > 0 && n <= (1 << 20) && is_dense(first) && rows) {
+    rc = new_dense(ctx, x->dtype, x->rank, x->shape, &sum);
+    RedJob j;
+    j.dtype = x->dtype;
+    j.variant = RedJob::kSumPair;
+    j.n_out = j.n1 = n;
+    j.R = 2;
+    if (!is_dense(second)) {
+      j.n1 = d.nd == 2 ? d.shape[1] : 1;
+      j.sa = d.st[0][0];
+      j.R = d.nd == 2 ? d.st[0][1] : 0;
+    }
+    j.grid = grid_for(n, 256 * 16 / (int)dtype_size(x->dtype), ctx->num_cu * 8);
+    j.bytes = 3.0 * n * dtype_size(x->dtype);
+    j.flops = (double)n;
+    j.label = "gemm_sum_pair";
+    if (!rc) {
+      j.a = data_ptr(first);
+      j.b = data_ptr(second);
+      j.out = data_ptr(sum);
+      hgpu_buffer* reads[2] = {(*acc)->buf, x->buf};
+      if (!hold_reduction(ctx, j, reads, 2, sum->buf)) { hgpu_release(sum); sum = nullptr; }
+    }
+  }
+  if (!rc && !sum) rc = hgpu_ewise2(ctx, HGPU_ADD, *acc, x, &sum);
   hgpu_release(*acc);
   hgpu_release(x);
   *acc = rc ? nullptr : sum;
   return rc;
 }
+}  // namespace hg
+
+namespace {
 
 // out = sum_t contract(as[t], bs[t]) for terms of one layout that are not a
 // matrix product: the terms' chunks are reduced by one launch into partials

@@ -113,7 +113,11 @@ struct Spec {
   // K shared out between `splits` blocks per tile (few tiles, long K: the blocks of one tile run side by side
   // instead of one block walking all of K); each block writes its partial tile, and a second launch of one block
   // per tile adds the partial tiles up in the order of K and runs the program
+  // (a bare product writes whole partial results instead, which wait for other sums to be added up with: sum_partials;
+  // 784 x 128 over 1000 fp64, the launch that finished it was 4.7 us)
   int splits = 1, chunks_per_split = 0;
+  bool bare() const { return n_instr == 0 && n_in == 1 && out_slots.size() == 1; }
+  bool finishes() const { return splits > 1 && !bare(); }
   // WK = 4: a 16 x 16 tile per block, each wavefront a quarter of every chunk's k (see choose_flat); 1: wavefronts share K
   int WK = 1;
 };
@@ -246,7 +250,7 @@ std::string generate_body(const Spec& sp) {
   for (int i = 0; i < sp.n_in; ++i)
     if (i != sp.c_slot) s << "  const " << ctype(sp.dt[(size_t)i]) << "* i" << i << ";\n";
   for (size_t o = 0; o < sp.out_slots.size(); ++o) s << "  " << ctype(sp.dt[(size_t)sp.out_slots[o]]) << "* o" << o << ";\n";
-  if (sp.splits > 1) s << "  T* part;\n";
+  if (sp.finishes()) s << "  T* part;\n";
   s << "};\n";
   for (size_t c = 0; c < sp.chunks.size(); ++c) {
     emit_stage_fn(s, ("x" + std::to_string(c)).c_str(), sp.chunks[c].x, sp.chunks[c], "", "");
@@ -432,6 +436,8 @@ std::string generate_body(const Spec& sp) {
       run_chunks(c0, c1);
       s << "  }\n";
     }
+  }
+  if (sp.finishes()) {
     // hand the partial tile over: the registers of a lane side by side for the block's 256 lanes
     const int nreg = TP * TQ * 4;
     s << "  {\n    T* mine = ar.part + ((blk * " << S << " + sidx) * " << nreg << "LL) * 256 + tid;\n";
@@ -453,8 +459,11 @@ std::string generate_body(const Spec& sp) {
     s << "          acc[a][b][e] += theirs[((a * " << TQ << " + b) * 4 + e) * 256];\n  }\n";
   }
   if (n_read > 0 && !prefetch) epi_loads();
+  const bool parts = S > 1 && !sp.finishes();      // o0 holds a whole partial result for every share of K
+  if (parts) s << "  Args mine = ar;\n  mine.o0 += (i64)sidx * " << sp.P * sp.Q << "LL;\n";
   s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b)\n";
-  if (n_read > 0) s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], ei[a][b], only);\n";
+  if (parts) s << "      epilogue(mine, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], EpiIn{0}, only);\n";
+  else if (n_read > 0) s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], ei[a][b], only);\n";
   else s << "      epilogue(ar, p0 + (wp * " << TP << " + a) * 16, q0 + (wq * " << TQ << " + b) * 16, r, g, acc[a][b], EpiIn{0}, only);\n";
   s << "}\n";
   return s.str();
@@ -775,11 +784,12 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   if (ktot < 4 || ktot > (sp.P * sp.Q <= kSmallOut ? kMaxKSmallOut : kMaxKTotal)) return HGPU_OK;
   // A product alone: below about a million multiply-adds the wave-per-output kernels are as fast.  With a program to run
   // over the result, or several products to add, those take a launch or two more, and the steps of a small recurrence
-  // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than a tile has.
+  // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than half a tile has.
   // Gradients in recorded graphs, us, with a million as the line for these too / without: dense 784-64-64-10 batch 32 fp32
   // 83 / 56, batch 130 fp64 81 / 55; two recurrent layers of 12 steps, fp32, batch 64 width 32 571 / 104 and width 80
   // 876 / 117, fp64 batch 300 width 50 393 / 139.
-  const bool whatever_size = n_terms > 1 || (n_instr > 0 && sp.Q >= 16);
+  // (A readout of ten rows as a product and a pass 9 us, here 4.8.)
+  const bool whatever_size = n_terms > 1 || (n_instr > 0 && sp.Q >= 8);
   if (sp.P < 16 || sp.Q < 4 || (!whatever_size && (double)sp.P * sp.Q * ktot < 1.0e6)) return HGPU_OK;
   for (int o = 0; o < n_out; ++o) {
     if (out_slots[o] < n_in && out_slots[o] != c_slot) return HGPU_OK;   // a copy of an input: not this kernel's business
@@ -842,7 +852,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
       kn.prog.assign(prog, prog + n_instr);
       kn.spec = sp;
       kn.spec.prog = kn.prog.data();
-      kn.fn = compiled_kernel(ctx, {&kn.body}, {d.grid}, {d.lds_bytes}, kn.kname, sp.splits > 1 ? &kn.finish_fn : nullptr);
+      kn.fn = compiled_kernel(ctx, {&kn.body}, {d.grid}, {d.lds_bytes}, kn.kname, sp.finishes() ? &kn.finish_fn : nullptr);
       it = known.emplace(key.bytes, std::move(kn)).first;
     } else if (check_keys() && (it->second.body != generate_body(sp) || it->second.kname != kname)) {
       return fail(ctx, HGPU_ERR_DEVICE, "small-K product: two different kernels under one key (%s)", kname);
@@ -858,14 +868,14 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   for (auto& tm : sp.terms) { d.args.push_back(tm.x); d.args.push_back(tm.y); }
   for (int i = 0; i < n_in; ++i)
     if (i != c_slot) d.args.push_back(data_ptr(in[i]));
-  for (int o = 0; o < n_out; ++o) d.args.push_back(data_ptr(outs[o]));
   const double es = sp.f64 ? 8 : 4;
   hgpu_buffer* part = nullptr;
   if (sp.splits > 1) {
-    int rc = buffer_alloc(ctx, (size_t)nblk * (size_t)sp.BP * (size_t)sp.BQ * (size_t)es, &part);
+    int rc = buffer_alloc(ctx, sp.finishes() ? (size_t)nblk * (size_t)sp.BP * (size_t)sp.BQ * (size_t)es : (size_t)sp.splits * (size_t)sp.P * (size_t)sp.Q * (size_t)es, &part);
     if (rc) return rc;
-    d.args.push_back(part->ptr);
   }
+  for (int o = 0; o < n_out; ++o) d.args.push_back(part && !sp.finishes() ? part->ptr : data_ptr(outs[o]));
+  if (sp.finishes()) d.args.push_back(part->ptr);
   d.flops = 2.0 * (double)sp.P * sp.Q * ktot;
   d.bytes = ((double)sp.P + sp.Q) * ktot * es;
   for (int i = 0; i < n_in; ++i)
@@ -894,12 +904,17 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     *handled = true;
     return HGPU_OK;
   }
-  LaunchGuard lg(ctx, d.label, d.bytes, d.flops, &d.args);
-  void* args[] = {(void*)d.args.data()};
-  hipError_t err = launch_module(lg, d.fn, d.grid, 256, args, true, finish_fn == nullptr);
-  if (err == hipSuccess && finish_fn) err = launch_module(lg, finish_fn, (unsigned)((ntiles + 7) / 8 * 8), 256, args, false, true);
+  hipError_t err = hipSuccess;
+  {
+    LaunchGuard lg(ctx, d.label, d.bytes, d.flops, &d.args);
+    void* args[] = {(void*)d.args.data()};
+    err = launch_module(lg, d.fn, d.grid, 256, args, true, finish_fn == nullptr);
+    if (err == hipSuccess && finish_fn) err = launch_module(lg, finish_fn, (unsigned)((ntiles + 7) / 8 * 8), 256, args, false, true);
+  }
+  int rc = err == hipSuccess ? HGPU_OK : check_hip(ctx, err, "small-K product launch");
+  if (!rc && part && !sp.finishes()) rc = sum_partials(ctx, sp.f64 ? HGPU_F64 : HGPU_F32, sp.P * sp.Q, sp.splits, part, outs[0]);
   if (part) buffer_release(part);
-  if (err != hipSuccess) return check_hip(ctx, err, "small-K product launch");
+  if (rc) return rc;
   *handled = true;
   return HGPU_OK;
 }
@@ -1427,15 +1442,7 @@ extern "C" int hgpu_contract_sum_map(hgpu_ctx* ctx, int n_terms, const hgpu_arra
         if (!taken[(size_t)t] && same_shape(as[t], as[t0])) { ga.push_back(as[t]); gb.push_back(bs[t]); taken[(size_t)t] = 1; }
       hgpu_array* part = nullptr;
       int rc = hgpu_contract_sum(ctx, (int)ga.size(), ga.data(), gb.data(), n_keep, &part);
-      if (!rc && c) {
-        hgpu_array* sum = nullptr;
-        rc = hgpu_ewise2(ctx, HGPU_ADD, c, part, &sum);
-        hgpu_release(part);
-        hgpu_release(c);
-        c = sum;
-      } else if (!rc) {
-        c = part;
-      }
+      if (!rc) rc = add_into(ctx, &c, part);
       if (rc) { if (c) hgpu_release(c); return rc; }
     }
   }

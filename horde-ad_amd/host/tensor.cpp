@@ -1496,7 +1496,7 @@ T contract(const T& a, const T* b, int n_keep) {
     // ... and when the provider can sum in the pass that writes other expressions
     // of this shape, the sum waits for such a pass (the gradient's)
     if (be->fuse && api->struct_size >= offsetof(hgpu_api, fused_map_sums) + sizeof(api->fused_map_sums) && api->fused_map_sums && pending_size(a.holder()) <= 40 &&
-        a.size() >= 4096) {
+        a.size() >= 64) {
       auto p = new_holder(be, nullptr);
       p->ssrc = a.holder();
       auto& ps = be->pending_sums;
@@ -1519,7 +1519,7 @@ T contract(const T& a, const T* b, int n_keep) {
   }
   // sdot0 with an expression for an operand (`sdot0 (log soft) expected`, an objective's value): the sum
   // of the product expression, which waits for a pass over arrays of this shape like any other such sum
-  if (b && n_keep == 0 && (a.pending_expr() || b->pending_expr()) && a.dtype() == b->dtype() && a.shape() == b->shape() && a.size() >= 4096 &&
+  if (b && n_keep == 0 && (a.pending_expr() || b->pending_expr()) && a.dtype() == b->dtype() && a.shape() == b->shape() && a.size() >= 64 &&
       (a.dtype() == HGPU_F64 || a.dtype() == HGPU_F32) && fuses(a.be()) && pending_size(a.holder()) + pending_size(b->holder()) < 40) {
     const hgpu_api* api = a.be()->api;
     if (api->struct_size >= offsetof(hgpu_api, fused_map_sums) + sizeof(api->fused_map_sums) && api->fused_map_sums) {

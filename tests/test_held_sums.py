@@ -107,3 +107,34 @@ def test_few_launches(gpu):
     labels = list(gpu.profile_report())
     gpu.check(gpu.lib.profile_enable(gpu.h, 0))
     assert sum(s.startswith("contract_group") or s.startswith("gemm_sum_partials") for s in labels) == 1, labels
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [37, 128])
+@pytest.mark.parametrize("order", [(0, 1), (1, 0), (1, 2, 0), (0, 2), (1, 2)])
+def test_sums_of_products_of_several_layouts(gpu, dt, n, order):
+    """A product over k, a row's sum times one element that every column repeats, a column's repeated down the rows."""
+    rng = np.random.default_rng(n)
+    m, k = 130, 3001
+    x, y = rng.uniform(-1, 1, (m, k)).astype(dt), rng.uniform(-1, 1, (n, k)).astype(dt)
+    c = np.asarray(0.75, dt)
+    a = gpu.upload(x).replicate([n]).transpose([1, 0, 2])
+    b = gpu.upload(y).replicate([m])
+    one = gpu.upload(c).replicate([m, n, k])
+    a64, b64 = x.astype(np.float64), y.astype(np.float64)
+    pairs = [(a, b), (a, one), (one, b)]
+    want = [a64 @ b64.T, np.broadcast_to(0.75 * a64.sum(1)[:, None], (m, n)), np.broadcast_to(0.75 * b64.sum(1)[None, :], (m, n))]
+    size = [np.abs(a64) @ np.abs(b64).T, 0.75 * np.abs(a64).sum(1)[:, None] + np.zeros((m, n)), 0.75 * np.abs(b64).sum(1)[None, :] + np.zeros((m, n))]
+    got = gpu.contract_sum([pairs[i] for i in order], 2).numpy()
+    bound = 4 * (k + 8) * EPS[dt] * sum(size[i] for i in order)
+    assert np.all(np.abs(got - sum(want[i] for i in order)) <= bound)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("p,q,k", [(784, 128, 1000), (783, 127, 601), (500, 33, 1024), (96, 100, 1023)])
+def test_bare_products_with_k_shared_out(gpu, dt, p, q, k):
+    """Few tiles under a long K: whole partial results, tiles with one row or column among them."""
+    rng = np.random.default_rng(k)
+    vals = [times(gpu, rng.uniform(-1, 1, (q, k)).astype(dt), rng.uniform(-1, 1, (p, k)).astype(dt), dt) for _ in range(2)]
+    for v in vals:
+        v.check()
