@@ -1029,8 +1029,9 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     for (int l0 = 0, l1 = 0; l0 < n_levels; l0 = l1) {
       ChainPlan plan;
       hipFunction_t fn = nullptr;
-      // (fewer weights in registers where the compiler found too few for the rest)
-      for (int slack = 0; !fn && slack <= 24; slack += 24) {
+      // Fewer weights in registers where the compiler found too few for the rest, in small steps: LDS may have no room for many
+      // more (two layers of width 128 transposed, fp64: 68 bytes of scratch, 52 with eight registers less, no plan with 24 less).
+      for (int slack = 0; !fn && slack <= 24; slack += 8) {
         plan = ChainPlan();
         if (!plan_chain(cand, levels, ctx->num_cu, slack, l0, &l1, &plan)) break;
         fn = chain_kernel(ctx, plan);

@@ -24,7 +24,7 @@
 // What bounds it: in fp32 with 20 columns a block the matrix cores, 4.3 of the 5.6 us a level (two layers 128 wide; a level
 // by itself 10.6), the rest LDS latency after the barrier and the program; with 4 columns the chain LDS read, multiply,
 // program, LDS write, barrier: 1.3-1.6 us in fp32, in fp64 2.5 without and 3.3 with a tanh (a level by itself 4.7).
-// Gradients of two layers 128 wide over 28 steps, before / so: fp32 batch 5000 844 / 629 us, fp64 batch 150 344 / 298.
+// Gradients of two layers 128 wide over 28 steps, before / so: fp32 batch 5000 844 / 629 us, fp64 batch 150 278 / 252 for the second of its two chains.
 // Taken back: nontemporal stores of the results (no gain beside the movers' priority), all wavefronts on all layers (fp32
 // the same, fp64 forward 111 us for 100; still the form where one layer's weights do not fit its wavefronts).
 
