@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <string>
@@ -220,6 +221,13 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
 void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst);
 // contract.hip: launches up to kMaxGroupReductions such reductions and kMaxGroupSums sums of partial results, all of one element type, as one kernel (the caller holds launch_mu)
 hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int n);
+// One product that a recording may hold back (gemm.hip): its kernel, its arguments, and how such products are launched together.
+struct WideJob;
+// gemm.hip: launches up to kMaxWideJobs products of one kernel (the caller holds launch_mu)
+hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n);
+constexpr int kMaxWideJobs = 4;
+// smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it
+void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
 // contract.hip: *acc += x, taking over x (the first term becomes the accumulator); the addition is held back where it can share a launch
 int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now

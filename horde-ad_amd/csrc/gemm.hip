@@ -30,6 +30,15 @@
 
 #include "gemm_kernel.hpp"
 
+namespace hg {
+// A product of gemm_single_dims that is held back.
+struct WideJob {
+  bool f64, akc, bkc;
+  gemm::SplitJob j;
+};
+static_assert(kMaxWideJobs == gemm::kMaxSplitGroup, "");
+}  // namespace hg
+
 using namespace hg;
 using namespace hg::gemm;
 
@@ -220,7 +229,8 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
 
 // Products whose row, column, contracted and batch indices are single dims with strides that a 32-bit byte offset
 // reaches: fp32 on the bf16 matrix cores (gemm_split.hip), fp64 in tiles without address arithmetic (gemm_wide_f64.hip).
-int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out) {
+int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out,
+                     const std::vector<hgpu_buffer*>& operands) {
   if (p.m.nd != 1 || p.n.nd != 1 || p.k.nd != 1 || p.bt.nd != 1) return HGPU_OK;
   const int64_t nt = n_terms > 0 ? n_terms : 1;
   const bool f64 = dtype == HGPU_F64;
@@ -318,7 +328,17 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     }
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
     LaunchArgs la{ctx->stream, 0, 0, 0, sak == 1, sbk == 1, dim3((unsigned)tiles, (unsigned)split, (unsigned)p.BT), swap ? pb : pa, swap ? pa : pb, cdst, nullptr, nullptr};
-    {
+    // While a recording is open a product of a few rounds of blocks waits for others of its kernel, where nobody is about to
+    // read its result: a reverse pass's weight gradients.  (Submitted one by one, the device would idle meanwhile.)
+    static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
+    if (hold && ctx->cap && !partials_out && !operands.empty() && tiles * split * p.BT <= 4 * ctx->num_cu) {
+      auto job = std::make_shared<WideJob>();
+      job->f64 = f64;
+      job->akc = sak == 1;
+      job->bkc = sbk == 1;
+      job->j = SplitJob{q, la.A, la.B, cdst, (int)tiles, split, (int)p.BT};
+      hold_wide(ctx, std::move(job), (f64 ? 4 : 0) + (sak == 1 ? 2 : 0) + (sbk == 1 ? 1 : 0), label, bytes, flops, operands, split > 1 ? part : out->buf);
+    } else {
       const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
@@ -409,6 +429,24 @@ bool classify_contraction(int rank, const int64_t* shape, const int64_t* st_a, c
   return true;
 }
 
+hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
+  SplitGroup g;
+  memset(&g, 0, sizeof g);
+  const SplitJob* js[kMaxSplitGroup];
+  for (int k = 0; k < n; ++k) js[k] = &jobs[k]->j;
+  if (n == 1) {
+    const SplitJob& j = *js[0];
+    LaunchArgs la{ctx->stream, 0, 0, 0, jobs[0]->akc, jobs[0]->bkc, dim3((unsigned)j.tiles, (unsigned)j.splits, (unsigned)j.batches), j.A, j.B, j.C, nullptr, nullptr};
+    if (jobs[0]->f64) launch_wide_f64(j.p, la);
+    else launch_split_f32(j.p, la);
+    return hipGetLastError();
+  }
+  const unsigned grid = split_group(js, n, &g);
+  if (jobs[0]->f64) launch_wide_f64_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
+  else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
+  return hipGetLastError();
+}
+
 int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, hgpu_array* out, bool* handled,
              int n_terms, const hgpu_array* const* as, const hgpu_array* const* bs, hgpu_array** partials_out) {
   // n_terms > 0: out = sum_t contract(as[t], bs[t]); all terms have the shapes,
@@ -436,6 +474,8 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
 
   const void* pa = data_ptr(a);
   const void* pb = data_ptr(b);
+  std::vector<hgpu_buffer*> operands{a->buf, b->buf};
+  for (int t = 0; t < n_terms; ++t) { operands.push_back(as[t]->buf); operands.push_back(bs[t]->buf); }
   // A small output under a long K (weight gradients, the last layer of a
   // classifier) is better served by independent wavefronts than by staged tiles.
   static_assert(kMaxTerms == 32, "hgpu_contract_sum groups 32 terms to a launch");
@@ -454,7 +494,7 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
   // 700 x 300 over 500: 18.0 against 10.2)
   const bool early = tiled && a->dtype == HGPU_F64 && ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.BT >= 4 * (int64_t)ctx->num_cu;
   if (early) {
-    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out);
+    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out, operands);
     if (rc || *handled) return rc;
   }
   if ((p.K <= 512 || (p.K <= 1024 && p.M * p.N <= 160000)) && p.BT == 1) {   // the whole contracted dim in LDS: no K loop, no K table
@@ -466,7 +506,7 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     if (rc || *handled) return rc;
   }
   if (tiled && !early) {
-    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out);
+    int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out, operands);
     if (rc || *handled) return rc;
   }
   // (under a long K the staged kernel's coalesced tile loads win even with most of a 32-wide tile empty: the recurrent network's

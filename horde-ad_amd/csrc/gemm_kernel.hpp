@@ -798,12 +798,13 @@ struct SplitShare {
   const T *A, *B;
   int m0, n0, kbeg, kend, s;
 };
+// (block `nr` of the `nsplits` x tiles of batch element `batch`)
 template <int BM, int BN, typename T>
-__device__ __forceinline__ SplitShare<T> split_share(const SplitParams& p, const T* A, const T* B) {
+__device__ __forceinline__ SplitShare<T> split_share(const SplitParams& p, const T* A, const T* B, int nr, int nsplits, int batch) {
   // each XCD works on a contiguous range of (K chunk, tile) pairs, as in k_gemm
   const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
   const int ntiles = tiles_m * tiles_n;
-  const int lin = xcd_order<int>(blockIdx.x + ntiles * blockIdx.y, ntiles * gridDim.y);
+  const int lin = xcd_order<int>(nr, ntiles * nsplits);
   const int s = lin / ntiles, bid = lin - s * ntiles;
   // tiles in bands of eight rows of tiles: neighbours in the order share operands
   const int band = bid / (8 * tiles_n), in_band = bid - band * 8 * tiles_n;
@@ -817,10 +818,63 @@ __device__ __forceinline__ SplitShare<T> split_share(const SplitParams& p, const
     B = (const T*)p.b_term[term];
   }
   const int kbeg = sk * p.kchunk, kend = kbeg + p.kchunk < p.K ? kbeg + p.kchunk : p.K;
-  return {A + (int64_t)blockIdx.z * p.bsa, B + (int64_t)blockIdx.z * p.bsb, tile_m * BM, tile_n * BN, kbeg, kend, s};
+  return {A + (int64_t)batch * p.bsa, B + (int64_t)batch * p.bsb, tile_m * BM, tile_n * BN, kbeg, kend, s};
+}
+
+// Several such products as one kernel (weight gradients that a recording holds back).  A product of a few hundred blocks pays
+// for filling and emptying the device; and products with a common operand (W and V of `W x + V s`) meet it in the caches when
+// their shares of K run at one time, so their blocks take turns, eight at a time (one per XCD), where all have about as many.
+// us, one after another / so: three of 128 x 128 over 27 x 5000 fp32 141 / 133, over 27 x 150 fp64 23.4 / 15.7; 300 x 784 and
+// 100 x 300 over 5000 fp64 64.5 / 66.0, and the sums of both in one launch then; 2048 x 784 and 2048 x 2048 over 8192 fp32
+// 600 / 575.  (K is cut as for each alone: a replay gives the bits that the same work submitted one by one gives.)
+constexpr int kMaxSplitGroup = 4;
+struct SplitJob {
+  SplitParams p;
+  const void *A, *B;
+  void* C;
+  int tiles, splits, batches;
+  int blocks() const { return tiles * splits * batches; }
+};
+struct SplitGroup {
+  int n, turns;                 // turns: blocks of a job when they take turns, a multiple of 8; 0: one job after the other
+  int first[kMaxSplitGroup];
+  SplitJob job[kMaxSplitGroup];
+};
+static_assert(sizeof(SplitGroup) <= 4000, "the group's arguments must fit the kernel argument block");
+// Which job a block of the group works for, and its number there; -1: none.
+__device__ __forceinline__ int split_job(const SplitGroup& g, int block, int* nr) {
+  int k;
+  if (g.turns) {
+    const int turn = block >> 3;
+    k = turn % g.n;
+    *nr = (turn / g.n) * 8 + (block & 7);
+  } else {
+    k = g.n - 1;
+    while (k > 0 && block < g.first[k]) --k;
+    *nr = block - g.first[k];
+  }
+  return *nr < g.job[k].tiles * g.job[k].splits * g.job[k].batches ? k : -1;
+}
+// The group's arguments and its number of blocks.
+inline unsigned split_group(const SplitJob* const* jobs, int n, SplitGroup* g) {
+  g->n = n;
+  int most = 0, least = 0x7fffffff, total = 0;
+  for (int k = 0; k < kMaxSplitGroup; ++k) {
+    g->first[k] = total;
+    if (k >= n) continue;
+    g->job[k] = *jobs[k];
+    const int b = (jobs[k]->blocks() + 7) / 8 * 8;
+    most = b > most ? b : most;
+    least = b < least ? b : least;
+    total += b;
+  }
+  g->turns = most <= least + least / 8 ? most : 0;
+  return (unsigned)(g->turns ? most * n : total);
 }
 void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a);
+void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
 
 // defined in gemm_f32.hip / gemm_f64.hip
 void launch_f32(const GemmParams& p, const LaunchArgs& a);

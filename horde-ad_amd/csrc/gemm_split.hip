@@ -157,7 +157,7 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
 }
 
 template <bool AKC, bool BKC>
-__global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
+__device__ __forceinline__ void gemm_split_body(const SplitParams& p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 32 x 32 blocks of each
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr int PA = 3 * BM * 2, PB = 3 * BN * 2;       // 16-byte elements of one buffer
@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
 
-  const auto share = split_share<BM, BN>(p, A, B);
+  const auto share = split_share<BM, BN>(p, A, B, nr, nsplits, batch);
   const int m0 = share.m0, n0 = share.n0, kbeg = share.kbeg, kend = share.kend;
 
   Side<BM, AKC> sa;
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
   }
   step(i0, std::integral_constant<int, 0>{});
 
-  float* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)share.s * p.c_split_stride;
+  float* Cout = C + (int64_t)batch * p.bsc + (int64_t)share.s * p.c_split_stride;
   auto put = [&](int i, int j, const f16v& c, float scale) {
     const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
     if (n >= p.N) return;
@@ -355,6 +355,21 @@ __global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float
     for (int j = 0; j < TN; ++j) put(i, j, acc[i][j] + low[i][j], kUnscale);
 }
 
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
+  gemm_split_body<AKC, BKC>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
+}
+
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 2) k_gemm_split_group(SplitGroup g) {
+  int nr;
+  const int k = split_job(g, blockIdx.x, &nr);
+  if (k < 0) return;
+  const SplitJob& j = g.job[k];
+  const int per_batch = j.tiles * j.splits, batch = nr / per_batch;
+  gemm_split_body<AKC, BKC>(j.p, (const float*)j.A, (const float*)j.B, (float*)j.C, nr - batch * per_batch, j.splits, batch);
+}
+
 template <typename F>
 void launch_as(const LaunchArgs& a, F kernel, const SplitParams& p) {
   const float* A = (const float*)a.A;
@@ -374,6 +389,14 @@ void launch_split_f32(const SplitParams& p, const LaunchArgs& a) {
   else if (a.va) launch_as(a, k_gemm_split<true, false>, p);
   else if (a.vb) launch_as(a, k_gemm_split<false, true>, p);
   else launch_as(a, k_gemm_split<false, false>, p);
+}
+
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, g); };
+  if (akc && bkc) go(k_gemm_split_group<true, true>);
+  else if (akc) go(k_gemm_split_group<true, false>);
+  else if (bkc) go(k_gemm_split_group<false, true>);
+  else go(k_gemm_split_group<false, false>);
 }
 
 }  // namespace gemm

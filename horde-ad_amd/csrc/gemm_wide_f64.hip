@@ -80,14 +80,14 @@ struct Side {
 
 // AKC, BKC: the operand is contiguous along k (lanes stage 16 bytes of a row; otherwise a row each, 8 bytes of two k).
 template <bool AKC, bool BKC>
-__global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C) {
+__device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 16 x 16 blocks of each
   constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
   __shared__ u4 lds[2][(BM + BN) * 8];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
 
-  const auto share = split_share<BM, BN>(p, A, B);
+  const auto share = split_share<BM, BN>(p, A, B, nr, nsplits, batch);
   const int m0 = share.m0, n0 = share.n0, kbeg = share.kbeg, kend = share.kend;
 
   Side<BM, AKC> sa;
@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const do
     step(i0, b0, b0);
   }
 
-  double* Cout = C + (int64_t)blockIdx.z * p.bsc + (int64_t)share.s * p.c_split_stride;
+  double* Cout = C + (int64_t)batch * p.bsc + (int64_t)share.s * p.c_split_stride;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + (wn * TN + j) * 16 + MfmaF64::col(lane);
@@ -196,6 +196,21 @@ __global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const do
   }
 }
 
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C) {
+  gemm_wide_f64_body<AKC, BKC>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
+}
+
+template <bool AKC, bool BKC>
+__global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64_group(SplitGroup g) {
+  int nr;
+  const int k = split_job(g, blockIdx.x, &nr);
+  if (k < 0) return;
+  const SplitJob& j = g.job[k];
+  const int per_batch = j.tiles * j.splits, batch = nr / per_batch;
+  gemm_wide_f64_body<AKC, BKC>(j.p, (const double*)j.A, (const double*)j.B, (double*)j.C, nr - batch * per_batch, j.splits, batch);
+}
+
 }  // namespace
 
 namespace hg {
@@ -208,6 +223,14 @@ void launch_wide_f64(const SplitParams& p, const LaunchArgs& a) {
   else if (a.va) launch_kernel(a, k_gemm_wide_f64<true, false>, p, A, B, C);
   else if (a.vb) launch_kernel(a, k_gemm_wide_f64<false, true>, p, A, B, C);
   else launch_kernel(a, k_gemm_wide_f64<false, false>, p, A, B, C);
+}
+
+void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, g); };
+  if (akc && bkc) go(k_gemm_wide_f64_group<true, true>);
+  else if (akc) go(k_gemm_wide_f64_group<true, false>);
+  else if (bkc) go(k_gemm_wide_f64_group<false, true>);
+  else go(k_gemm_wide_f64_group<false, false>);
 }
 
 }  // namespace gemm

@@ -719,6 +719,9 @@ struct Deferred {
   RedJob red;
   CopyJob copy{};              // a copy into an existing array (hold_copy)
   MapJob map{};                // an elementwise pass (hold_map_locked)
+  std::shared_ptr<WideJob> wide;       // a large product (hold_wide), of kernel wide_kernel
+  int wide_kernel = 0;
+  bool may_wait() const { return is_reduction || wide; }      // nobody waits for it but who reads its result
   const Known* kn = nullptr;   // a small product: what is kept of its kind
   const std::string* body = nullptr;   // the problem's device code (kept with the known kernels) and the number that stands for it
   int body_id = -1;
@@ -1069,7 +1072,46 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     for (auto* b : d.writes) written_at[b] = d.level;
     top = std::max(top, d.level);
   }
+  // A reduction that no held product reads goes out as late as it can, where the sums that need other levels go too.
+  {
+    std::map<const hgpu_buffer*, int> read_at;
+    for (size_t i = items.size(); i-- > 0;) {
+      Deferred& d = items[i];
+      if (gone[i]) continue;
+      if (d.is_reduction) {
+        int last = top;
+        for (auto* b : d.writes) {
+          auto it = read_at.find(b);
+          if (it != read_at.end()) last = std::min(last, it->second - 1);
+        }
+        d.level = std::max(d.level, last);
+      }
+      for (auto* b : d.reads) {
+        auto it = read_at.emplace(b, d.level).first;
+        it->second = std::min(it->second, d.level);
+      }
+    }
+  }
   for (int lv = 0; lv <= top; ++lv) {
+    // the level's large products: those of one kernel go out together
+    {
+      std::vector<Deferred*> wide;
+      for (auto& d : items)
+        if (d.level == lv && d.wide) wide.push_back(&d);
+      std::stable_sort(wide.begin(), wide.end(), [](const Deferred* a, const Deferred* b) { return a->wide_kernel < b->wide_kernel; });
+      for (size_t g0 = 0, g1 = 0; g0 < wide.size(); g0 = g1) {
+        const WideJob* jobs[kMaxWideJobs];
+        int n = 0;
+        for (; g1 < wide.size() && n < kMaxWideJobs && wide[g1]->wide_kernel == wide[g0]->wide_kernel; ++g1) jobs[n++] = wide[g1]->wide.get();
+        const hipError_t err = launch_wide_group(ctx, jobs, n);
+        if (err != hipSuccess) {
+          int rc = check_hip(ctx, err, "grouped product launch");
+          if (!ctx->deferred_rc) ctx->deferred_rc = rc;
+        }
+        ctx->dq->n_launches += 1;
+        if (n > 1) ctx->dq->n_grouped += n;
+      }
+    }
     // the level's reductions and sums of partial results: those of one element type go out together
     {
       std::vector<Deferred*> reds;
@@ -1115,7 +1157,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     }
     std::vector<Deferred*> here;
     for (auto& d : items)
-      if (d.level == lv && !d.is_reduction) here.push_back(&d);
+      if (d.level == lv && !d.may_wait()) here.push_back(&d);
     for (size_t g0 = 0; g0 < here.size(); g0 += kMaxGroup) {
       std::vector<Deferred*> grp(here.begin() + (long)g0, here.begin() + (long)std::min(here.size(), g0 + kMaxGroup));
       hipFunction_t fn = nullptr;
@@ -1227,7 +1269,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
   ctx->dq_pending = true;
 }
 
-// Only reductions and sums of partial results wait beyond the launch that asks: they are the ends of a reverse pass's
+// Only large products, reductions and sums of partial results wait beyond the launch that asks: they are the ends of a reverse pass's
 // branches, and the later they go out the more of them share a launch.  Held products go with the first that is needed,
 // as before: their groups and chains are found among all of them.
 void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads) {
@@ -1243,7 +1285,7 @@ void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads) {
   std::vector<char> go(q.items.size(), 0);
   for (size_t i = q.items.size(); i-- > 0;) {
     Deferred& d = q.items[i];
-    go[i] = !d.is_reduction;
+    go[i] = !d.may_wait();
     for (auto* w : d.writes) go[i] = go[i] || needed.count(w);
     if (go[i]) needed.insert(d.reads.begin(), d.reads.end());
   }
@@ -1272,6 +1314,19 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
   std::lock_guard<std::mutex> lk(ctx->launch_mu);
   hold_item_locked(ctx, std::move(d));
   return true;
+}
+
+void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write) {
+  Deferred d;
+  d.wide = std::move(job);
+  d.wide_kernel = kernel;
+  d.label = label;
+  d.bytes = bytes;
+  d.flops = flops;
+  d.reads = reads;
+  d.writes.push_back(write);
+  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  hold_item_locked(ctx, std::move(d));
 }
 
 // An elementwise pass joins the queue: it waits for passes that read none of the held results (an optimizer's

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from conftest import capi
+from conftest import pkg
 from test_gemm_split import product
 
 pytestmark = pytest.mark.gpu
@@ -138,3 +138,56 @@ def test_bare_products_with_k_shared_out(gpu, dt, p, q, k):
     vals = [times(gpu, rng.uniform(-1, 1, (q, k)).astype(dt), rng.uniform(-1, 1, (p, k)).astype(dt), dt) for _ in range(2)]
     for v in vals:
         v.check()
+
+
+@pytest.fixture(scope="module")
+def host():
+    return pkg.hostapi.Host()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("shapes", [
+    [(128, 128, 30000)] * 3,                                        # as many blocks each: they take turns
+    [(128, 128, 30000), (129, 128, 30000)],                         # a tile row more
+    [(300, 784, 5000), (100, 300, 5000), (120, 100, 9001)],         # one after the other
+    [(130, 100, 20000)] * 5 + [(96, 96, 20011)],                    # more than one launch takes
+    [(1000, 300, 1100)],
+])
+@pytest.mark.parametrize("lay", ["KK", "RK", "KR", "RR"])
+def test_products_of_a_recording_go_out_together(host, dt, shapes, lay):
+    """Weight gradients, the first operand shared where sizes agree: every replay is what the products submitted one by one
+    give, bit for bit, and within rounding of numpy."""
+    rng = np.random.default_rng(len(shapes))
+    shared, pairs = {}, []
+    for m, n, k in shapes:
+        if (m, k) not in shared:
+            shared[m, k] = rng.uniform(-1, 1, (m, k)).astype(dt)
+        pairs.append((shared[m, k], rng.uniform(0, 1, (n, k)).astype(dt)))
+    up = {}
+
+    def put(x, how):
+        key = (id(x), how)
+        if key not in up:
+            up[key] = host.concrete(x) if how == "K" else host.concrete(np.ascontiguousarray(x.T)).stranspose([1, 0])
+        return up[key]
+
+    ops = [(put(x, lay[0]), put(y, lay[1]).stranspose([1, 0])) for x, y in pairs]
+
+    def program():
+        out = [a.smatmul2(b) for a, b in ops]
+        return out + [a.stranspose([1, 0]).ssum() for a, _ in ops[:2]]
+
+    eager = [v.numpy() for v in program()]
+    graph, res = host.capture(program)
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            for got, want in zip(res, eager):
+                assert np.array_equal(got.numpy(), want)
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
+    for (x, y), got in zip(pairs, eager):
+        a, b = x.astype(np.float64), y.astype(np.float64)
+        assert np.all(np.abs(got - a @ b.T) <= 4 * (x.shape[1] + 8) * EPS[dt] * (np.abs(a) @ np.abs(b).T))
