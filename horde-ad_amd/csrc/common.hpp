@@ -192,7 +192,7 @@ struct RedJob {
   int64_t n1 = 0;
   void* out2 = nullptr;
   bool is_sum() const { return variant >= kSumRows; }
-  enum { kSumRows = 3, kSumLane, kSum32, kSum8, kSumPair };      // kSumPair: a[i] + b[i]
+  enum { kSumRows = 3, kSumLane, kSum32, kSum8, kSumPair, kSumTiny };      // kSumPair: a[i] + b[i]; kSumTiny: R instructions, coded in sa
 };
 constexpr int kMaxGroupReductions = 4, kMaxGroupSums = 12;
 // One dense copy between two arrays that do not overlap (hgpu_assign): `bytes` bytes in units of 2^unit bytes, to which both sides are aligned.
@@ -228,6 +228,8 @@ hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n);
 constexpr int kMaxWideJobs = 4;
 // smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it
 void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
+// contract.hip: a program over a few elements (its last instruction's result is `out`), to be launched with held sums; false: left to the caller
+bool hold_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out);
 // contract.hip: *acc += x, taking over x (the first term becomes the accumulator); the addition is held back where it can share a launch
 int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now

@@ -435,9 +435,35 @@ __device__ __forceinline__ void pair_body(const SumArgs& g, unsigned bid, unsign
   for (int64_t i = nv * V + at; i < g.n; i += step) o[i] = a[i] + b[i];
 }
 
+// See hold_tiny_map.
+template <typename T>
+__device__ __forceinline__ void tiny_body(const SumArgs& g) {
+#pragma clang fp contract(off)
+  if (threadIdx.x >= g.n) return;
+  const uint64_t code = (uint64_t)g.stride;
+  T v[6];
+  v[0] = ((const T*)g.part)[code >> 48 & 1 ? threadIdx.x : 0];
+  v[1] = ((const T*)g.other)[code >> 49 & 1 ? threadIdx.x : 0];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[2 + k] = k > 0 ? v[1 + k] : v[0];
+    if (k >= g.S) continue;
+    const unsigned q = (unsigned)(code >> (12 * k)) & 0xfff, op = q & 15;
+    T x = v[0], y = v[0];
+#pragma unroll
+    for (int u = 1; u < 2 + k; ++u) {
+      if ((q >> 4 & 15) == (unsigned)u) x = v[u];
+      if ((q >> 8 & 15) == (unsigned)u) y = v[u];
+    }
+    v[2 + k] = op == 0 ? -x : op == 1 ? x + y : op == 2 ? x - y : x * y;
+  }
+  ((T*)g.out)[threadIdx.x] = v[5];
+}
+
 template <typename T>
 __device__ __forceinline__ void sum_body(const SumArgs& s, unsigned bid) {
-  if (s.kind == RedJob::kSumPair) pair_body<T>(s, bid, s.grid);
+  if (s.kind == RedJob::kSumTiny) tiny_body<T>(s);
+  else if (s.kind == RedJob::kSumPair) pair_body<T>(s, bid, s.grid);
   else if (s.kind == RedJob::kSumRows) partials_row_body<T>(s, bid, s.grid);
   else if (s.kind == RedJob::kSumLane) partials_lane_body<T>(s, bid, s.grid);
   else if (s.kind == RedJob::kSum32) partials_body<T, 32>(s, bid, s.grid);
@@ -446,7 +472,8 @@ __device__ __forceinline__ void sum_body(const SumArgs& s, unsigned bid) {
 
 template <typename T, int KIND>
 __global__ void __launch_bounds__(kBlock) k_sum_partials(SumArgs s) {
-  if (KIND == RedJob::kSumPair) pair_body<T>(s, blockIdx.x, gridDim.x);
+  if (KIND == RedJob::kSumTiny) tiny_body<T>(s);
+  else if (KIND == RedJob::kSumPair) pair_body<T>(s, blockIdx.x, gridDim.x);
   else if (KIND == RedJob::kSumRows) partials_row_body<T>(s, blockIdx.x, gridDim.x);
   else if (KIND == RedJob::kSumLane) partials_lane_body<T>(s, blockIdx.x, gridDim.x);
   else if (KIND == RedJob::kSum32) partials_body<T, 32>(s, blockIdx.x, gridDim.x);
@@ -628,10 +655,40 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
 
 // A few very long rows whose data one CU cannot fetch fast enough (a block
 // draws some tens of GB/s): G blocks per row scan consecutive pieces, then one
-// wavefront per row picks among the G candidates, the earlier piece winning ties.
+// wavefront per row picks among the G candidates, the earlier piece winning ties: of the block that finishes last (`tickets`
+// not null: a counter per row, 128 bytes apart, zero between launches), or of a second launch.  The candidates travel as the
+// partial sums of the fused sums do: exchanged in by atomics of device scope, the returned value says that they have arrived,
+// then the ticket is drawn.  One row of 50,000 fp64: 9.9 us in two launches, 7.3 in one, with 48 pieces for 24 6.6.
+// The extremum of a row among its G candidates, by one wavefront.
+template <typename T, typename V, typename I>
+__device__ __forceinline__ void pick_body(int G, int want_max, const V& value_of, const I& index_of, int64_t* __restrict__ out, T* __restrict__ vals) {
+  const int lane = threadIdx.x & 63;
+  T best = T(0);
+  int64_t bi = INT64_MAX;
+  for (int g = lane; g < G; g += 64) {
+    T x = value_of(g);
+    int64_t xi = index_of(g);
+    if (xi == INT64_MAX) continue;
+    bool better = bi == INT64_MAX || (want_max ? (x > best) : (x < best));    // pieces of a lane come in ascending order
+    if (better) { best = x; bi = xi; }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    T ob = __shfl_down(best, off);
+    int64_t oi = __shfl_down(bi, off);
+    if (oi != INT64_MAX) {
+      bool better = bi == INT64_MAX || (want_max ? (ob > best) : (ob < best)) || (ob == best && oi < bi);
+      if (better) { best = ob; bi = oi; }
+    }
+  }
+  if (lane == 0) {
+    *out = bi;
+    if (vals) *vals = best;
+  }
+}
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t L, int64_t sl, int want_max, int G, int64_t piece, const T* __restrict__ a,
-                                                              T* __restrict__ pbest, int64_t* __restrict__ pidx) {
+                                                              T* __restrict__ pbest, int64_t* __restrict__ pidx,
+                                                              unsigned long long* handed, unsigned* tickets, int64_t* __restrict__ out, T* __restrict__ vals) {
   __shared__ T sbest[kBlock];
   __shared__ int64_t sidx[kBlock];
   const int row = blockIdx.x / G, g = blockIdx.x % G;
@@ -673,33 +730,53 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t 
     }
     __syncthreads();
   }
-  if (t == 0) { pbest[blockIdx.x] = sbest[0]; pidx[blockIdx.x] = sidx[0]; }
+  if (!tickets) {
+    if (t == 0) { pbest[blockIdx.x] = sbest[0]; pidx[blockIdx.x] = sidx[0]; }
+    return;
+  }
+  __shared__ bool last;
+  if (t == 0) {
+    unsigned long long bits = 0;
+    __builtin_memcpy(&bits, &sbest[0], sizeof(T));
+    const unsigned long long v = __hip_atomic_exchange(handed + 2 * blockIdx.x, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long i = __hip_atomic_exchange(handed + 2 * blockIdx.x + 1, (unsigned long long)sidx[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" :: "v"(v), "v"(i) : "memory");      // uses of the returned values: nothing below starts before they are there
+    unsigned* ticket = tickets + 32 * row;
+    last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)G - 1;
+    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+  }
+  __syncthreads();
+  if (!last || t >= 64) return;
+  asm volatile("" ::: "memory");
+  auto load = [&](int at) { return __hip_atomic_load(handed + 2 * (int64_t)row * G + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  pick_body<T>(G, want_max, [&](int c) { const unsigned long long u = load(2 * c); T x; __builtin_memcpy(&x, &u, sizeof(T)); return x; },
+               [&](int c) { return (int64_t)load(2 * c + 1); }, out + row, vals ? vals + row : nullptr);
 }
 template <typename T>
 __global__ void __launch_bounds__(64) k_argminmax_pick(int G, int want_max, const T* __restrict__ pbest, const int64_t* __restrict__ pidx, int64_t* __restrict__ out,
                                                         T* __restrict__ vals) {
-  const int row = blockIdx.x, lane = threadIdx.x;
-  T best = T(0);
-  int64_t bi = INT64_MAX;
-  for (int g = lane; g < G; g += 64) {
-    T x = pbest[row * G + g];
-    int64_t xi = pidx[row * G + g];
-    if (xi == INT64_MAX) continue;
-    bool better = bi == INT64_MAX || (want_max ? (x > best) : (x < best));    // pieces of a lane come in ascending order
-    if (better) { best = x; bi = xi; }
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    T ob = __shfl_down(best, off);
-    int64_t oi = __shfl_down(bi, off);
-    if (oi != INT64_MAX) {
-      bool better = bi == INT64_MAX || (want_max ? (ob > best) : (ob < best)) || (ob == best && oi < bi);
-      if (better) { best = ob; bi = oi; }
-    }
-  }
-  if (lane == 0) {
-    out[row] = bi;
-    if (vals) vals[row] = best;
-  }
+  const int row = blockIdx.x;
+  pick_body<T>(G, want_max, [&](int g) { return pbest[row * G + g]; }, [&](int g) { return pidx[row * G + g]; }, out + row, vals ? vals + row : nullptr);
+}
+
+// A few very long rows, in pieces: see k_argminmax_pieces (the caller's guard is held).
+// (One row of 10,000 fp64: ten pieces 6.6 us, one block of 1024 lanes 6.4.)
+constexpr int64_t kPiecesFrom = 16384, kPiece = 1024;
+template <typename T>
+int extremum_pieces(hgpu_ctx* ctx, const Dims& keep, int64_t n_out, int64_t L, int64_t sl, int want_max, const void* a, unsigned* tickets, void* out, void* vp) {
+  const int G = (int)std::min<int64_t>(128, L / kPiece);
+  const int64_t piece = (L + G - 1) / G;
+  hgpu_buffer* scratch = nullptr;
+  const int rc = buffer_alloc(ctx, (size_t)n_out * G * 16, &scratch);
+  if (rc) return rc;
+  T* pv = (T*)scratch->ptr;
+  unsigned long long* handed = tickets ? (unsigned long long*)scratch->ptr : nullptr;
+  int64_t* pi = (int64_t*)scratch->ptr + (size_t)n_out * G;
+  hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, sl, want_max, G, piece, (const T*)a, pv, pi,
+  handed, tickets, (int64_t*)out, (T*)vp);
+  if (!tickets) hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, G, want_max, (const T*)pv, (const int64_t*)pi, (int64_t*)out, (T*)vp);
+  buffer_release(scratch);
+  return HGPU_OK;
 }
 
 // The buffers of a reduction whose launch may be held back (see RedJob): what it reads and what it writes.
@@ -844,7 +921,8 @@ template <typename T>
 static void launch_sum(hgpu_ctx* ctx, const RedJob& j) {
   const SumArgs s = sum_args(j);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(j.grid), dim3(kBlock), 0, ctx->stream, s); };
-  if (j.variant == RedJob::kSumPair) go(k_sum_partials<T, RedJob::kSumPair>);
+  if (j.variant == RedJob::kSumTiny) go(k_sum_partials<T, RedJob::kSumTiny>);
+  else if (j.variant == RedJob::kSumPair) go(k_sum_partials<T, RedJob::kSumPair>);
   else if (j.variant == RedJob::kSumRows) go(k_sum_partials<T, RedJob::kSumRows>);
   else if (j.variant == RedJob::kSumLane) go(k_sum_partials<T, RedJob::kSumLane>);
   else if (j.variant == RedJob::kSum32) go(k_sum_partials<T, RedJob::kSum32>);
@@ -1031,8 +1109,8 @@ int reduce_views(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_
       pp = part->ptr;
     }
     int64_t psh[2] = {n_out, S}, pst[2] = {S, 1};
-    HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type; rc = (launch_stage<T, A>(ctx, use_wave, keep, red, n_out, R, (int)S, pa, pb, pp, nullptr, nullptr, -1, fresh)); });
     const bool few_long = n_out < 256 && S >= 256;
+    HG_DISPATCH_DTYPE(a->dtype, T, { using A = typename acc_of<T>::type;  rc = (launch_stage<T, A>(ctx, use_wave, keep, red, n_out, R, (int)S, pa, pb, pp, nullptr, nullptr, -1, fresh)); });
     if (!rc && hold && n_out < 65536 && !few_long) {
       rc = sum_partial_rows(ctx, a->dtype, n_out, S, part, out_arr);
     } else if (!rc) {
@@ -1077,6 +1155,50 @@ int scratch_of(hgpu_ctx* ctx, void** out) {
 }  // namespace
 
 namespace hg {
+// A program over a few elements that an objective ends with (`negate sum * c`) joins the launch of a gradient's last sums: a
+// pass of its own is 4 us in a graph.  One or two operands, up to four negations, additions, subtractions and
+// multiplications: 12 bits each, in the order of the program, and above them which operands move.
+bool hold_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out) {
+  const int64_t n = nelem(out);
+  if (n_in < 1 || n_in > 2 || n_instr < 1 || n_instr > 4 || !dtype_is_float(out->dtype) || n < 1 || n > 64 || !out->buf) return false;
+  uint64_t code = 0;
+  for (int k = 0; k < n_instr; ++k) {
+    const hgpu_fused_instr& q = prog[k];
+    uint64_t op;
+    if (q.kind == HGPU_FUSED_OP1 && q.op == HGPU_NEG) op = 0;
+    else if (q.kind == HGPU_FUSED_OP2 && q.op == HGPU_ADD) op = 1;
+    else if (q.kind == HGPU_FUSED_OP2 && q.op == HGPU_SUB) op = 2;
+    else if (q.kind == HGPU_FUSED_OP2 && q.op == HGPU_MUL) op = 3;
+    else return false;
+    // (slots of this kernel: the operands are 0 and 1, results follow)
+    auto slot = [&](int s) { return (uint64_t)(s < n_in ? s : s - n_in + 2); };
+    code |= (op | slot(q.a) << 4 | (op ? slot(q.b) : 0) << 8) << (12 * k);
+  }
+  hgpu_buffer* reads[2] = {nullptr, nullptr};
+  for (int i = 0; i < n_in; ++i) {
+    if (in[i]->dtype != out->dtype || !in[i]->buf) return false;
+    bool still = true;
+    for (int d = 0; d < in[i]->rank; ++d) still = still && (in[i]->shape[d] == 1 || in[i]->strides[d] == 0);
+    if (!still && !is_dense(in[i])) return false;
+    if (!still) code |= 1ull << (48 + i);
+    reads[i] = in[i]->buf;
+  }
+  RedJob j;
+  j.dtype = out->dtype;
+  j.variant = RedJob::kSumTiny;
+  j.n_out = j.n1 = n;
+  j.R = n_instr;
+  j.sa = (int64_t)code;
+  j.grid = 1;
+  j.bytes = (double)n * (n_in + 1) * dtype_size(out->dtype);
+  j.flops = (double)n * n_instr;
+  j.label = "tiny_map";
+  j.a = data_ptr(in[0]);
+  j.b = n_in > 1 ? data_ptr(in[1]) : j.a;
+  j.out = data_ptr(out);
+  return hold_reduction(ctx, j, reads, n_in, out->buf);
+}
+
 // *acc += x, taking over x (the first term becomes the accumulator).
 int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x) {
   if (!*acc) { *acc = x; return HGPU_OK; }
@@ -1338,22 +1460,18 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
     const int64_t* ks[1] = {a->strides};
     Dims keep;
     if (!collapse(a->rank - 1, a->shape, 1, ks, &keep)) { hgpu_release(o); if (v) hgpu_release(v); return fail(ctx, HGPU_ERR_UNSUPPORTED, "argminmax: too many dims"); }
+    const bool pieces = L >= kPiecesFrom && n_out <= 16;
+    void* tickets = nullptr;
+    if (pieces && (ctx->ticket_block || !ctx->cap)) rc = ticket_block(ctx, &tickets);
+    if (rc) { hgpu_release(o); if (v) hgpu_release(v); return rc; }
     const std::vector<const void*> reads = reads_of(1, &a);
     LaunchGuard lg(ctx, "argminmax", (double)n_out * (L * dtype_size(a->dtype) + 8 + (v ? dtype_size(a->dtype) : 0)), (double)n_out * L, &reads);
     void* vp = v ? data_ptr(v) : nullptr;
-    if (L >= 16384 && n_out <= 16) {
+    if (pieces) {
       // very few, very long rows: pieces of a row to many blocks, then one pick per row
-      const int G = (int)std::min<int64_t>(128, L / 2048);
-      const int64_t piece = (L + G - 1) / G;
-      hgpu_buffer* scratch = nullptr;
-      const size_t vb = ((size_t)n_out * G * dtype_size(a->dtype) + 15) / 16 * 16;
-      rc = buffer_alloc(ctx, vb + (size_t)n_out * G * 8, &scratch);
+      // (a recording that meets the first such row of the process gets two launches: the counters cannot be cleared in it)
+      HG_DISPATCH_DTYPE(a->dtype, T, rc = extremum_pieces<T>(ctx, keep, n_out, L, a->strides[a->rank - 1], want_max, data_ptr(a), (unsigned*)tickets, data_ptr(o), vp));
       if (rc) { hgpu_release(o); if (v) hgpu_release(v); return rc; }
-      void* pb = scratch->ptr;
-      int64_t* pi = (int64_t*)((char*)scratch->ptr + vb);
-      HG_DISPATCH_DTYPE(a->dtype, T, hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, a->strides[a->rank - 1], want_max, G, piece, (const T*)data_ptr(a), (T*)pb, pi));
-      HG_DISPATCH_DTYPE(a->dtype, T, hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, G, want_max, (const T*)pb, (const int64_t*)pi, (int64_t*)data_ptr(o), (T*)vp));
-      buffer_release(scratch);
     } else if (L >= 512 && n_out <= 64) {
       // few long rows: a whole block per row (one row of 2500 fp32, a minibatch's logits: a wavefront, load after load, takes
       // 14.4 us, a block 5.8; one of 1500 fp64 9.9 and 5.0)

@@ -191,3 +191,80 @@ def test_products_of_a_recording_go_out_together(host, dt, shapes, lay):
     for (x, y), got in zip(pairs, eager):
         a, b = x.astype(np.float64), y.astype(np.float64)
         assert np.all(np.abs(got - a @ b.T) <= 4 * (x.shape[1] + 8) * EPS[dt] * (np.abs(a) @ np.abs(b).T))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int8, np.int64])
+@pytest.mark.parametrize("rows,n", [(1, 16384), (3, 16385), (1, 50000), (16, 40961), (2, 300001)])
+def test_extrema_of_long_rows(gpu, dt, rows, n):
+    """Pieces of a row to many blocks, the last of which picks: again and again, ties to the first."""
+    rng = np.random.default_rng(n)
+    x = rng.integers(-100, 100, (rows, n)).astype(dt)
+    x[:, n // 2] = x[:, n - 1] = 101
+    a = gpu.upload(x)
+    for _ in range(4):
+        assert np.array_equal(a.argminmax_last(True).numpy(), x.argmax(1))
+        assert np.array_equal(a.argminmax_last(False).numpy(), x.argmin(1))
+    if dt in (np.float64, np.float32):
+        x[0, 7] = np.inf
+        x[-1, n - 3] = -np.inf
+        a = gpu.upload(x)
+        assert np.array_equal(a.argminmax_last(True).numpy(), x.argmax(1))
+        assert np.array_equal(a.argminmax_last(False).numpy(), x.argmin(1))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("rows,n", [(128, 4200), (17, 30000), (300, 2000), (1, 9000)])
+def test_row_sums_in_chunks_wait(host, dt, rows, n):
+    """Both stages of a sum in chunks, the negation of a result, and a result read on the way, recorded and not."""
+    rng = np.random.default_rng(rows)
+    x, y = (rng.uniform(-1, 1, (28, rows, n // 28)).astype(dt) for _ in range(2))
+    a, b = host.concrete(x), host.concrete(y)
+
+    def program():
+        s, t = (v.stranspose([1, 0, 2]).sreshape((rows, 28 * (n // 28))).stranspose([1, 0]).ssum() for v in (a, b))
+        return [s, -t, s + t, -(a.ssum0())]
+
+    want = [x.astype(np.float64).sum((0, 2)), -y.astype(np.float64).sum((0, 2)), (x.astype(np.float64) + y).sum((0, 2)), -x.astype(np.float64).sum()]
+    size = [np.abs(x).sum((0, 2)), np.abs(y).sum((0, 2)), (np.abs(x) + np.abs(y)).sum((0, 2)), np.abs(x).sum()]
+    eager = [v.numpy() for v in program()]
+    graph, res = host.capture(program)
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            for got, e in zip(res, eager):
+                assert np.array_equal(got.numpy(), e)
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
+    for e, w, m in zip(eager, want, size):      # sums run in doubles: their roundings, and those to the result's type and of the addition
+        assert np.all(np.abs(e - w) <= 4 * (EPS[dt] + n * EPS[np.float64]) * m)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_programs_over_a_few_elements(host, dt):
+    """What an objective ends with: one and two operands, still and moving, sums of theirs read at once and later."""
+    rng = np.random.default_rng(5)
+    x, c = rng.uniform(-1, 1, (64, 4001)).astype(dt), np.asarray(0.37, dt)
+    a, k = host.concrete(x), host.concrete(c)
+
+    def program():
+        s = a.stranspose([1, 0]).ssum()
+        t = a.ssum0()
+        return [-(t * k), (t - k) * t, -s, s * k.sreplicate0N((64,)) - s, (-(t * k)) + k]
+
+    x, k64, e = x.astype(np.float64), float(c), EPS[dt]
+    s, t, ms, mt = x.sum(1), x.sum(), np.abs(x).sum(1), np.abs(x).sum()
+    want = [(-(t * k64), mt), ((t - k64) * t, 2 * (mt + 1) * mt), (-s, ms), (s * k64 - s, 2 * ms), (-(t * k64) + k64, mt + 1)]
+    eager = [v.numpy() for v in program()]
+    for got, (w, m) in zip(eager, want):         # 64-bit sums, one rounding to the type, one per operation
+        assert np.all(np.abs(got - w) <= 8 * (e + 70000 * EPS[np.float64]) * m)
+    graph, res = host.capture(program)
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            assert all(np.array_equal(r.numpy(), v) for r, v in zip(res, eager))
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
