@@ -787,12 +787,13 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   if (ktot < 4 || ktot > (sp.P * sp.Q <= kSmallOut ? kMaxKSmallOut : kMaxKTotal)) return HGPU_OK;
   // A product alone: below about a million multiply-adds the wave-per-output kernels are as fast.  With a program to run
   // over the result, or several products to add, those take a launch or two more, and the steps of a small recurrence
-  // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than half a tile has.
+  // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than
+  // half a tile has, and of fewer than a tile's where K, too, is less than 32 (both paddings: three quarters of the tile's work).
   // Gradients in recorded graphs, us, with a million as the line for these too / without: dense 784-64-64-10 batch 32 fp32
   // 83 / 56, batch 130 fp64 81 / 55; two recurrent layers of 12 steps, fp32, batch 64 width 32 571 / 104 and width 80
   // 876 / 117, fp64 batch 300 width 50 393 / 139.
-  // (A readout of ten rows as a product and a pass 9 us, here 4.8.)
-  const bool whatever_size = n_terms > 1 || (n_instr > 0 && sp.Q >= 8);
+  // (A readout of ten rows, K = 128, as a product and a pass 9 us, here 4.8.)
+  const bool whatever_size = n_terms > 1 || (n_instr > 0 && (sp.Q >= 16 || (sp.Q >= 8 && ktot >= 32)));
   if (sp.P < 16 || sp.Q < 4 || (!whatever_size && (double)sp.P * sp.Q * ktot < 1.0e6)) return HGPU_OK;
   for (int o = 0; o < n_out; ++o) {
     if (out_slots[o] < n_in && out_slots[o] != c_slot) return HGPU_OK;   // a copy of an input: not this kernel's business
