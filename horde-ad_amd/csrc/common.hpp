@@ -235,8 +235,8 @@ int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now
 bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write, hgpu_buffer* write2 = nullptr);
 // contract.hip: the `parts` partial results of n elements in `part` are added up in `out` (dense), or the first n1 in out1 and the other n - n1 in out2.
-// Held back where it can share a launch.
-int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1 = -1, const hgpu_array* out2 = nullptr);
+// Held back where it can share a launch; launched alone it counts under `label`, where that is given, as a part of the product that left the partials.
+int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1 = -1, const hgpu_array* out2 = nullptr, const char* label = nullptr);
 
 // Builds the merged iteration space of `nops` operands that share `shape`.
 // Size-1 dims vanish; adjacent dims merge when every operand's strides allow.

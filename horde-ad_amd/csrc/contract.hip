@@ -933,12 +933,12 @@ static void launch_sum(hgpu_ctx* ctx, const RedJob& j) {
 // memory is better given back.
 constexpr double kMaxHeldPartials = 64.0 * (1 << 20);
 
-static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_array* out1, const hgpu_array* out2) {
+static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_array* out1, const hgpu_array* out2, const char* label = nullptr) {
   j.a = part->ptr;
   j.out = data_ptr(out1);
   j.out2 = out2 ? data_ptr(out2) : nullptr;
-  j.label = "gemm_sum_partials";
-  j.flops = (double)j.n_out * j.R;
+  j.label = label ? label : "gemm_sum_partials";
+  j.flops = label ? 0 : (double)j.n_out * j.R;
   // (Submitted one by one, an objective's value goes out at once: the device would come to it only when the host asks.)
   if (out1->buf && (!out2 || out2->buf) && (double)part->bytes <= kMaxHeldPartials && (ctx->cap || j.n_out >= 16) &&
       hold_reduction(ctx, j, &part, 1, out1->buf, out2 ? out2->buf : nullptr)) return HGPU_OK;
@@ -950,7 +950,7 @@ static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_arr
   return HGPU_OK;
 }
 
-int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1, const hgpu_array* out2) {
+int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* part, const hgpu_array* out1, int64_t n1, const hgpu_array* out2, const char* label) {
   const size_t es = dtype_size(dtype);
   RedJob j;
   j.dtype = dtype;
@@ -964,7 +964,7 @@ int sum_partials(hgpu_ctx* ctx, int dtype, int64_t n, int parts, hgpu_buffer* pa
   // fp32: rows of 32 are whole 128-byte lines (16384 outputs x 270 partials: 12.9 us with rows of 8, 7.1 us with rows of 32)
   j.variant = parts <= 8 || (parts <= 64 && n >= 65536) ? RedJob::kSumLane : (es == 4 || n > 8192 || parts < 32) ? RedJob::kSum32 : RedJob::kSum8;
   j.grid = grid_for(n, j.variant == RedJob::kSumLane ? 256 : j.variant == RedJob::kSum32 ? 32 : 8, ctx->num_cu * 8);
-  return queue_sum(ctx, j, part, out1, out2);
+  return queue_sum(ctx, j, part, out1, out2, label);
 }
 
 // A row of S sums in doubles for every output.

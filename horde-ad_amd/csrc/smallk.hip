@@ -916,7 +916,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     if (err == hipSuccess && finish_fn) err = launch_module(lg, finish_fn, (unsigned)((ntiles + 7) / 8 * 8), 256, args, false, true);
   }
   int rc = err == hipSuccess ? HGPU_OK : check_hip(ctx, err, "small-K product launch");
-  if (!rc && part && !sp.finishes()) rc = sum_partials(ctx, sp.f64 ? HGPU_F64 : HGPU_F32, sp.P * sp.Q, sp.splits, part, outs[0]);
+  if (!rc && part && !sp.finishes()) rc = sum_partials(ctx, sp.f64 ? HGPU_F64 : HGPU_F32, sp.P * sp.Q, sp.splits, part, outs[0], -1, nullptr, d.label);
   if (part) buffer_release(part);
   if (rc) return rc;
   *handled = true;
