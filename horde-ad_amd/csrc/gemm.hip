@@ -33,7 +33,7 @@
 namespace hg {
 // A product of gemm_single_dims that is held back.
 struct WideJob {
-  bool f64, akc, bkc;
+  bool f64, akc, bkc, thin;
   gemm::SplitJob j;
 };
 static_assert(kMaxWideJobs == gemm::kMaxSplitGroup, "");
@@ -238,7 +238,8 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
   SplitParams q{};
   int64_t sam = p.m.sa[0], sak = p.k.sa[0], sbn = p.n.sb[0], sbk = p.k.sb[0], scm = p.m.sc[0], scn = p.n.sc[0], M = p.M, N = p.N;
   int64_t bsa = p.bt.sa[0], bsb = p.bt.sb[0];
-  bool swap = scm == 1 && scn != 1;          // the lanes of a result block run along its columns
+  const bool thin = !f64 && std::min(M, N) <= 32;
+  bool swap = thin ? M < N : scm == 1 && scn != 1;          // the lanes of a result block run along its columns; a thin side is its columns
   if (swap) {
     std::swap(sam, sbn);
     std::swap(sak, sbk);
@@ -282,6 +283,13 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       const double us = 5 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 8 / 6e6 : 0);
       if (us < best) { best = us; split = (int)sp; }
     }
+  } else if (thin) {
+    // Two blocks on a CU, four where two would have 512 k and more to walk each (their loads are what counts; more blocks
+    // leave more partial results).  us with the sums, two / four: 128 x 28 over 28 x 5000 (278 k) 25.7 / 26.8, 784 x 32 over
+    // 8192 (128) 16.6 / 17.6, 784 x 28 over 8 x 5000 (556) 41.2 / 37.0, 784 x 10 over 8 x 10000 (1112) 75.4 / 55.5.
+    const int64_t tiles = ((M + 127) / 128) * p.BT * nt;
+    auto chunks = [&](int64_t per_cu) { return std::max<int64_t>(1, std::min<int64_t>(per_cu * ctx->num_cu / tiles, p.K / 64)); };
+    split = (int)(p.K >= 512 * chunks(2) ? chunks(4) : chunks(2));
   } else {
     // Microseconds, as measured: a step of 16 k of a 128 x 128 tile 1.4 alone on its CU and 0.92 for each of several;
     // 8 for the launch with its first loads and last stores; for partial results a second launch and their bytes once
@@ -301,7 +309,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     const double work = (double)((M + 63) / 64 * 64) * (double)((N + 63) / 64 * 64) * (double)p.K * (double)(p.BT * nt);
     if (best >= 6 + work / 6e6) return HGPU_OK;
   }
-  const int64_t BM = f64 ? 64 : 128, BN = BM;
+  const int64_t BM = f64 ? 64 : 128, BN = thin ? 32 : BM;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   q.kchunk = (int)(((p.K + split - 1) / split + 15) / 16 * 16);
   q.term_split = (int)((p.K + q.kchunk - 1) / q.kchunk);
@@ -336,15 +344,16 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       job->f64 = f64;
       job->akc = sak == 1;
       job->bkc = sbk == 1;
+      job->thin = thin;
       job->j = SplitJob{q, la.A, la.B, cdst, (int)tiles, split, (int)p.BT};
-      hold_wide(ctx, std::move(job), (f64 ? 4 : 0) + (sak == 1 ? 2 : 0) + (sbk == 1 ? 1 : 0), label, bytes, flops, operands, split > 1 ? part : out->buf);
+      hold_wide(ctx, std::move(job), (thin ? 8 : f64 ? 4 : 0) + (sak == 1 ? 2 : 0) + (sbk == 1 ? 1 : 0), label, bytes, flops, operands, split > 1 ? part : out->buf);
     } else {
       const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
       if (f64) launch_wide_f64(q, la);
-      else launch_split_f32(q, la);
+      else launch_split_f32(q, la, thin);
     }
     if (split > 1 && partials_out && split <= 3 && is_dense(out)) {
       int64_t sh[HGPU_MAX_RANK + 1], st[HGPU_MAX_RANK + 1];
@@ -438,12 +447,12 @@ hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
     const SplitJob& j = *js[0];
     LaunchArgs la{ctx->stream, 0, 0, 0, jobs[0]->akc, jobs[0]->bkc, dim3((unsigned)j.tiles, (unsigned)j.splits, (unsigned)j.batches), j.A, j.B, j.C, nullptr, nullptr};
     if (jobs[0]->f64) launch_wide_f64(j.p, la);
-    else launch_split_f32(j.p, la);
+    else launch_split_f32(j.p, la, jobs[0]->thin);
     return hipGetLastError();
   }
   const unsigned grid = split_group(js, n, &g);
   if (jobs[0]->f64) launch_wide_f64_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
-  else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
+  else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, jobs[0]->thin, ctx->stream);
   return hipGetLastError();
 }
 
@@ -505,13 +514,19 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     int rc = try_smallk(ctx, n_terms > 0 ? n_terms : 1, ta, tb, n_keep, 1, &none, 0, 0, nullptr, std::vector<int>{a->dtype}, 1, &slot, &out, handled);
     if (rc || *handled) return rc;
   }
-  if (tiled && !early) {
+  // Weight gradients of narrow layers, fp32: 8 to 32 rows or columns under a long K, bound by the loads of the long side, which
+  // a tile of 128 x 32 reads once.  us with the sums, tiles of the fp32 instruction / so: 128 x 28 over 28 x 5000 34.9 / 25.7,
+  // 50 x 28 over 20 x 1000 9.4 / 8.4, 2048 x 10 over 8192 26.1 / 21.4, 784 x 32 over 8192 24.5 / 16.6; error against fp64 0.4 to 0.6 of
+  // what it was.  Fewer columns leave the tile empty (784 x 4 over 8 x 10000 61 / 83); with rows further apart than 65536
+  // elements the wider tiles read longer pieces (1000 x 20 over 50000 57.6 / 54.0, over 100,000 101 / 104).
+  const int64_t k_all = p.K * (n_terms > 0 ? n_terms : 1);
+  const bool thin = a->dtype == HGPU_F32 && std::min(p.M, p.N) >= 8 && std::min(p.M, p.N) <= 32 && std::max(p.M, p.N) > 32 && p.K >= 64 && p.K <= 65536 && k_all >= 4096;
+  if ((tiled && !early) || thin) {
     int rc = gemm_single_dims(ctx, p, a->dtype, pa, pb, out, handled, n_terms, partials_out, operands);
     if (rc || *handled) return rc;
   }
-  // (under a long K the staged kernel's coalesced tile loads win even with most of a 32-wide tile empty: the recurrent network's
-  // input weight gradient, 128 x 28 over 28 x 5000, 52 -> 45 us)
-  if ((p.M <= 32 || p.N <= 32) && p.M <= 1024 && p.N <= 1024 && p.K * (n_terms > 0 ? n_terms : 1) < 4096) return gemm_direct(ctx, p, a->dtype, pa, pb, out, handled, n_terms);
+  // (under a long K the staged kernels' coalesced tile loads win even with most of a 32-wide tile empty: 128 x 28 over 28 x 5000, 52 -> 45 us)
+  if ((p.M <= 32 || p.N <= 32) && p.M <= 1024 && p.N <= 1024 && k_all < 4096) return gemm_direct(ctx, p, a->dtype, pa, pb, out, handled, n_terms);
 
   const int64_t nt = n_terms > 0 ? n_terms : 1;      // products summed by this launch
   const int64_t out_elems = p.M * p.N * p.BT;

@@ -872,9 +872,9 @@ inline unsigned split_group(const SplitJob* const* jobs, int n, SplitGroup* g) {
   return (unsigned)(g->turns ? most * n : total);
 }
 void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
-void launch_split_f32(const SplitParams& p, const LaunchArgs& a);
+void launch_split_f32(const SplitParams& p, const LaunchArgs& a, bool thin);      // thin: tiles of 128 x 32 instead of 128 x 128
 void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
-void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, hipStream_t stream);
 
 // defined in gemm_f32.hip / gemm_f64.hip
 void launch_f32(const GemmParams& p, const LaunchArgs& a);

@@ -80,7 +80,8 @@ __device__ __forceinline__ int lds_at(int r, int h) { return r * 2 + (h ^ ((r >>
 // scalar one for the step, and whatever lies past the end (rows, k) reads as zero.
 template <int ROWS, bool KC>
 struct Side {
-  static constexpr int NS = ROWS * 2 / NT;
+  static constexpr bool ALL = ROWS * 2 >= NT;      // every lane owns a piece
+  static constexpr int NS = ALL ? ROWS * 2 / NT : 1;
   __amdgpu_buffer_rsrc_t rsrc;
   uint32_t off[NS];                         // bytes
   int at[NS];
@@ -97,6 +98,7 @@ struct Side {
       off[i] = (uint32_t)(r0 + r < rows ? r0 + r : rows - 1) * rs + 8 * h * ks;   // (rows past the end: never stored)
       at[i] = lds_at(r, h);
     }
+    if (!ALL && t >= ROWS * 2) off[0] = 0x80000000u;      // (past the end with whatever is added)
   }
   // A whole step that starts at k0.
   __device__ __forceinline__ void load(int k0, Slot* s) const {
@@ -126,6 +128,7 @@ struct Side {
   }
   // parts: [3][ROWS * 2] of 16 bytes
   __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, float& largest) const {
+    if (!ALL && threadIdx.x >= ROWS * 2) return;
     u4 h, m, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -156,9 +159,13 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
   }
 }
 
-template <bool AKC, bool BKC>
+// THIN: tiles of 128 x 32 for products with at most 32 columns (weight gradients of narrow layers), bound by the loads of A:
+// a step is 10 KB of loads and six instructions a wavefront, one step ahead, so four blocks (114 to 124 registers, 30 KB of
+// LDS) hide one another's trips to memory.  128 x 28 over 28 x 5000, 87 MB: 23.7 us = 3.7 TB/s, the 32 x 32 tiles of the fp32
+// instruction, which read A for every 32 rows of it and B four times, 33.0.
+template <bool AKC, bool BKC, bool THIN>
 __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int nr, int nsplits, int batch) {
-  constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 32 x 32 blocks of each
+  constexpr int WM = THIN ? 4 : 2, WN = THIN ? 1 : 2, TM = THIN ? 1 : 2, TN = THIN ? 1 : 2;          // wavefronts, and 32 x 32 blocks of each
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr int PA = 3 * BM * 2, PB = 3 * BN * 2;       // 16-byte elements of one buffer
   __shared__ u4 lds[2][PA + PB];
@@ -355,19 +362,19 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
     for (int j = 0; j < TN; ++j) put(i, j, acc[i][j] + low[i][j], kUnscale);
 }
 
-template <bool AKC, bool BKC>
-__global__ void __launch_bounds__(NT, 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
-  gemm_split_body<AKC, BKC>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
+template <bool AKC, bool BKC, bool THIN>
+__global__ void __launch_bounds__(NT, THIN ? 4 : 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
+  gemm_split_body<AKC, BKC, THIN>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
 }
 
-template <bool AKC, bool BKC>
-__global__ void __launch_bounds__(NT, 2) k_gemm_split_group(SplitGroup g) {
+template <bool AKC, bool BKC, bool THIN>
+__global__ void __launch_bounds__(NT, THIN ? 4 : 2) k_gemm_split_group(SplitGroup g) {
   int nr;
   const int k = split_job(g, blockIdx.x, &nr);
   if (k < 0) return;
   const SplitJob& j = g.job[k];
   const int per_batch = j.tiles * j.splits, batch = nr / per_batch;
-  gemm_split_body<AKC, BKC>(j.p, (const float*)j.A, (const float*)j.B, (float*)j.C, nr - batch * per_batch, j.splits, batch);
+  gemm_split_body<AKC, BKC, THIN>(j.p, (const float*)j.A, (const float*)j.B, (float*)j.C, nr - batch * per_batch, j.splits, batch);
 }
 
 template <typename F>
@@ -384,19 +391,31 @@ void launch_as(const LaunchArgs& a, F kernel, const SplitParams& p) {
 namespace hg {
 namespace gemm {
 
-void launch_split_f32(const SplitParams& p, const LaunchArgs& a) {
-  if (a.va && a.vb) launch_as(a, k_gemm_split<true, true>, p);
-  else if (a.va) launch_as(a, k_gemm_split<true, false>, p);
-  else if (a.vb) launch_as(a, k_gemm_split<false, true>, p);
-  else launch_as(a, k_gemm_split<false, false>, p);
+template <bool THIN>
+static void launch_split(const SplitParams& p, const LaunchArgs& a) {
+  if (a.va && a.vb) launch_as(a, k_gemm_split<true, true, THIN>, p);
+  else if (a.va) launch_as(a, k_gemm_split<true, false, THIN>, p);
+  else if (a.vb) launch_as(a, k_gemm_split<false, true, THIN>, p);
+  else launch_as(a, k_gemm_split<false, false, THIN>, p);
 }
 
-void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
+void launch_split_f32(const SplitParams& p, const LaunchArgs& a, bool thin) {
+  if (thin) launch_split<true>(p, a);
+  else launch_split<false>(p, a);
+}
+
+template <bool THIN>
+static void launch_split_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, g); };
-  if (akc && bkc) go(k_gemm_split_group<true, true>);
-  else if (akc) go(k_gemm_split_group<true, false>);
-  else if (bkc) go(k_gemm_split_group<false, true>);
-  else go(k_gemm_split_group<false, false>);
+  if (akc && bkc) go(k_gemm_split_group<true, true, THIN>);
+  else if (akc) go(k_gemm_split_group<true, false, THIN>);
+  else if (bkc) go(k_gemm_split_group<false, true, THIN>);
+  else go(k_gemm_split_group<false, false, THIN>);
+}
+
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, hipStream_t stream) {
+  if (thin) launch_split_group<true>(g, grid, akc, bkc, stream);
+  else launch_split_group<false>(g, grid, akc, bkc, stream);
 }
 
 }  // namespace gemm
