@@ -226,6 +226,12 @@ struct WideJob;
 // gemm.hip: launches up to kMaxWideJobs products of one kernel (the caller holds launch_mu)
 hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n);
 constexpr int kMaxWideJobs = 4;
+// gemm.hip: row sums that a held product hands out beside its result (see join_wide_rows)
+int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride);
+void wide_take_rows(WideJob& job, void* part, const void* factor);
+// smallk.hip: the sums over K of n terms of M rows of fp32 elements, each term times the one element `factor` (null: 1), as
+// *part (rows x *shares, doubles) by a held product that reads the same rows; false: there is none
+bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
 // smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it
 void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
 // contract.hip: a program over a few elements (its last instruction's result is `out`), to be launched with held sums; false: left to the caller

@@ -1301,6 +1301,34 @@ int contract_terms(hgpu_ctx* ctx, int n, const hgpu_array* const* as, const hgpu
   return rc;
 }
 
+// Row sums of what a held product multiplies (the bias gradient beside a weight gradient, in a recording): that product's blocks add
+// them up as they stage its operand (gemm_split.hip).  Rows of fp32 elements side by side, all terms alike, the other factor
+// (where there is one) one element, the same for all terms; its terms are all there are of this sum.
+static int rows_with_product(hgpu_ctx* ctx, int n, const hgpu_array* const* as, const hgpu_array* const* bs, int n_keep, const hgpu_array* out, bool* handled) {
+  const hgpu_array* a = as[0];
+  if (!ctx->cap || a->dtype != HGPU_F32 || n > kGemmMaxTerms || !out->buf || nelem(a) == 0 || nelem(out) >= 65536) return HGPU_OK;
+  const hgpu_array* b = bs ? bs[0] : nullptr;
+  for (int t = 0; b && t < n; ++t) {
+    if (data_ptr(bs[t]) != data_ptr(b)) return HGPU_OK;
+    for (int d = 0; d < b->rank; ++d)
+      if (b->shape[d] > 1 && bs[t]->strides[d] != 0) return HGPU_OK;
+  }
+  Dims keep, red;
+  const int64_t* ks[1] = {a->strides};
+  const int64_t* rs[1] = {a->strides + n_keep};
+  if (!collapse(n_keep, a->shape, 1, ks, &keep) || !collapse(a->rank - n_keep, a->shape + n_keep, 1, rs, &red)) return HGPU_OK;
+  if (keep.nd != 1 || red.nd != 1 || red.st[0][0] != 1 || keep.st[0][0] < 0) return HGPU_OK;
+  const void* ptrs[kGemmMaxTerms];
+  for (int t = 0; t < n; ++t) ptrs[t] = data_ptr(as[t]);
+  hgpu_buffer* part = nullptr;
+  int shares = 0;
+  if (!join_wide_rows(ctx, n, ptrs, keep.shape[0], red.shape[0], keep.st[0][0], b ? b->buf : nullptr, b ? data_ptr(b) : nullptr, &part, &shares)) return HGPU_OK;
+  const int rc = sum_partial_rows(ctx, a->dtype, keep.shape[0], shares, part, out);
+  buffer_release(part);
+  *handled = !rc;
+  return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1340,6 +1368,7 @@ int hgpu_contract_sum(hgpu_ctx* ctx, int n, const hgpu_array* const* as, const h
       rc = new_dense(ctx, a->dtype, n_keep, a->shape, &part);
       bool handled = false;
       if (!rc) rc = try_gemm(ctx, ga[0], gb[0], n_keep, part, &handled, (int)ga.size(), ga.data(), gb.data());
+      if (!rc && !handled) rc = rows_with_product(ctx, (int)ga.size(), ga.data(), gb.data(), n_keep, part, &handled);
       if (!rc && !handled && nelem(part) > 0) {   // not a matrix product: the grouped reduction
         rc = contract_terms(ctx, (int)ga.size(), ga.data(), gb.data(), n_keep, part);
         handled = !rc;
@@ -1412,7 +1441,8 @@ int hgpu_contract(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n
   if (rc) { hgpu_release(o); return rc; }
   if (handled) { *out = o; return HGPU_OK; }
 
-  rc = reduce_views(ctx, a, b, n_keep, data_ptr(o), nullptr, 0, o);
+  rc = rows_with_product(ctx, 1, &a, b ? &b : nullptr, n_keep, o, &handled);
+  if (!rc && !handled) rc = reduce_views(ctx, a, b, n_keep, data_ptr(o), nullptr, 0, o);
   if (rc) { hgpu_release(o); return rc; }
   *out = o;
   return HGPU_OK;

@@ -443,7 +443,9 @@ hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
   memset(&g, 0, sizeof g);
   const SplitJob* js[kMaxSplitGroup];
   for (int k = 0; k < n; ++k) js[k] = &jobs[k]->j;
-  if (n == 1) {
+  bool rows = false;
+  for (int k = 0; k < n; ++k) rows = rows || js[k]->p.rows;
+  if (n == 1 && !rows) {
     const SplitJob& j = *js[0];
     LaunchArgs la{ctx->stream, 0, 0, 0, jobs[0]->akc, jobs[0]->bkc, dim3((unsigned)j.tiles, (unsigned)j.splits, (unsigned)j.batches), j.A, j.B, j.C, nullptr, nullptr};
     if (jobs[0]->f64) launch_wide_f64(j.p, la);
@@ -452,8 +454,25 @@ hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
   }
   const unsigned grid = split_group(js, n, &g);
   if (jobs[0]->f64) launch_wide_f64_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
-  else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, jobs[0]->thin, ctx->stream);
+  else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, jobs[0]->thin, rows, ctx->stream);
   return hipGetLastError();
+}
+
+// The shares of K of a held product that can also hand out the sums of the rows at `as` (n terms of M x K elements, rows
+// `row_stride` apart); 0: it cannot.  The terms may come in another order: each is added up by itself and all meet in one sum.
+int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride) {
+  const SplitParams& p = job.j.p;
+  if (job.f64 || !job.akc || p.rows || job.j.batches != 1 || p.M != M || p.K != K || p.sam != (uint64_t)row_stride * 4 || std::max(p.n_terms, 1) != n) return 0;
+  std::vector<const void*> x(as, as + n), y(1, job.j.A);
+  if (p.n_terms > 0) y.assign(p.a_term, p.a_term + n);
+  std::sort(x.begin(), x.end());
+  std::sort(y.begin(), y.end());
+  return x == y ? job.j.splits : 0;
+}
+
+void wide_take_rows(WideJob& job, void* part, const void* factor) {
+  job.j.p.rows = (double*)part;
+  job.j.p.row_factor = (const float*)factor;
 }
 
 int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, hgpu_array* out, bool* handled,

@@ -790,6 +790,8 @@ struct SplitParams {
   int n_terms, term_split;
   const void* a_term[kMaxTerms];
   const void* b_term[kMaxTerms];
+  double* rows;                 // sums of A's rows over the block's share of K, times *row_factor (rows x shares of K; null: not asked for)
+  const float* row_factor;      // null: 1
 };
 // The share of such a product that a block computes: rows from m0, columns from n0, k in [kbeg, kend), operands of its term
 // and batch element; s numbers the (term, K chunk) pairs.
@@ -826,7 +828,7 @@ __device__ __forceinline__ SplitShare<T> split_share(const SplitParams& p, const
 // their shares of K run at one time, so their blocks take turns, eight at a time (one per XCD), where all have about as many.
 // us, one after another / so: three of 128 x 128 over 27 x 5000 fp32 141 / 133, over 27 x 150 fp64 23.4 / 15.7; 300 x 784 and
 // 100 x 300 over 5000 fp64 64.5 / 66.0, and the sums of both in one launch then; 2048 x 784 and 2048 x 2048 over 8192 fp32
-// 600 / 575.  (K is cut as for each alone: a replay gives the bits that the same work submitted one by one gives.)
+// 600 / 575.  (K is cut as for each alone: a replay gives the bits that the same products submitted one by one give.)
 constexpr int kMaxSplitGroup = 4;
 struct SplitJob {
   SplitParams p;
@@ -874,7 +876,8 @@ inline unsigned split_group(const SplitJob* const* jobs, int n, SplitGroup* g) {
 void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a, bool thin);      // thin: tiles of 128 x 32 instead of 128 x 128
 void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
-void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, hipStream_t stream);
+// (rows: products among them hand out the sums of A's rows, A is contiguous along K)
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, bool rows, hipStream_t stream);
 
 // defined in gemm_f32.hip / gemm_f64.hip
 void launch_f32(const GemmParams& p, const LaunchArgs& a);

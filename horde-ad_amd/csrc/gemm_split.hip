@@ -163,7 +163,12 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
 // a step is 10 KB of loads and six instructions a wavefront, one step ahead, so four blocks (114 to 124 registers, 30 KB of
 // LDS) hide one another's trips to memory.  128 x 28 over 28 x 5000, 87 MB: 23.7 us = 3.7 TB/s, the 32 x 32 tiles of the fp32
 // instruction, which read A for every 32 rows of it and B four times, 33.0.
-template <bool AKC, bool BKC, bool THIN>
+// ROWS: the lanes also add up, in fp64, the elements of A they stage: a bias gradient is the row sums of what the weight
+// gradient multiplies.  Blocks of the first column of tiles do, for products that ask (split_job).  Reading A once more for
+// them: 28 x 128 rows of 5000 17.5 us, 2048 rows of 8192 17.4; here
+// the recurrent network's three products of 128 x 128 take 139 us for 135 and the one of 128 x 28 32 for 29.  (The large tile keeps
+// 16 to 20 bytes of a lane in scratch memory then, outside of its loop's loads.)
+template <bool AKC, bool BKC, bool THIN, bool ROWS>
 __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = THIN ? 4 : 2, WN = THIN ? 1 : 2, TM = THIN ? 1 : 2, TN = THIN ? 1 : 2;          // wavefronts, and 32 x 32 blocks of each
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
@@ -192,6 +197,16 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
 
   const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
   Slot ra[NA], rb[NB];
+  static_assert(!ROWS || (AKC && NA == 1 && BM * 2 == NT), "lane t stages a half of row t / 2");
+  const bool sum_rows = ROWS && p.rows != nullptr && n0 == 0;
+  double row_sum = 0;
+  auto store_a = [&](int u, u4* to) {
+    sa.store(ra[u], u, to, top_a);
+    if (sum_rows) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) row_sum += (double)ra[u].v[j];
+    }
+  };
   auto fetch = [&](int i) {                 // (chosen outside the main loop: a load on one side of a branch would be waited for where the sides meet)
     sa.load(kbeg + i * SK, ra);
     sb.load(kbeg + i * SK, rb);
@@ -203,7 +218,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   if (whole > 0) fetch(0);
   else fetch_tail(0);
 #pragma unroll
-  for (int i = 0; i < NA; ++i) sa.store(ra[i], i, lds[0], top_a);
+  for (int i = 0; i < NA; ++i) store_a(i, lds[0]);
 #pragma unroll
   for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, top_b);
   __syncthreads();
@@ -252,7 +267,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
         constexpr int first = 1;
         if (j >= first) {
           const int u = j - first;
-          if (u < NA) sa.store(ra[u], u, ln, top_a);
+          if (u < NA) store_a(u, ln);
           else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, top_b);
         }
       }
@@ -261,7 +276,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
       constexpr int first = 1;
 #pragma unroll
       for (int u = TN - first; u < NA + NB; ++u) {
-        if (u < NA) sa.store(ra[u], u, ln, top_a);
+        if (u < NA) store_a(u, ln);
         else sb.store(rb[u - NA], u - NA, ln + PA, top_b);
       }
     }
@@ -276,6 +291,11 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   }
   step(i0, std::integral_constant<int, 0>{});
 
+  if (sum_rows) {
+    row_sum += __shfl_xor(row_sum, 1);
+    if (p.row_factor) row_sum *= (double)*p.row_factor;
+    if (!(t & 1) && m0 + t / 2 < p.M) p.rows[(int64_t)(m0 + t / 2) * nsplits + share.s] = row_sum;
+  }
   float* Cout = C + (int64_t)batch * p.bsc + (int64_t)share.s * p.c_split_stride;
   auto put = [&](int i, int j, const f16v& c, float scale) {
     const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
@@ -364,17 +384,17 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
 
 template <bool AKC, bool BKC, bool THIN>
 __global__ void __launch_bounds__(NT, THIN ? 4 : 2) k_gemm_split(SplitParams p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C) {
-  gemm_split_body<AKC, BKC, THIN>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
+  gemm_split_body<AKC, BKC, THIN, false>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
 }
 
-template <bool AKC, bool BKC, bool THIN>
+template <bool AKC, bool BKC, bool THIN, bool ROWS>
 __global__ void __launch_bounds__(NT, THIN ? 4 : 2) k_gemm_split_group(SplitGroup g) {
   int nr;
   const int k = split_job(g, blockIdx.x, &nr);
   if (k < 0) return;
   const SplitJob& j = g.job[k];
   const int per_batch = j.tiles * j.splits, batch = nr / per_batch;
-  gemm_split_body<AKC, BKC, THIN>(j.p, (const float*)j.A, (const float*)j.B, (float*)j.C, nr - batch * per_batch, j.splits, batch);
+  gemm_split_body<AKC, BKC, THIN, ROWS>(j.p, (const float*)j.A, (const float*)j.B, (float*)j.C, nr - batch * per_batch, j.splits, batch);
 }
 
 template <typename F>
@@ -405,17 +425,19 @@ void launch_split_f32(const SplitParams& p, const LaunchArgs& a, bool thin) {
 }
 
 template <bool THIN>
-static void launch_split_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
+static void launch_split_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool rows, hipStream_t stream) {
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, g); };
-  if (akc && bkc) go(k_gemm_split_group<true, true, THIN>);
-  else if (akc) go(k_gemm_split_group<true, false, THIN>);
-  else if (bkc) go(k_gemm_split_group<false, true, THIN>);
-  else go(k_gemm_split_group<false, false, THIN>);
+  if (rows && bkc) go(k_gemm_split_group<true, true, THIN, true>);
+  else if (rows) go(k_gemm_split_group<true, false, THIN, true>);
+  else if (akc && bkc) go(k_gemm_split_group<true, true, THIN, false>);
+  else if (akc) go(k_gemm_split_group<true, false, THIN, false>);
+  else if (bkc) go(k_gemm_split_group<false, true, THIN, false>);
+  else go(k_gemm_split_group<false, false, THIN, false>);
 }
 
-void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, hipStream_t stream) {
-  if (thin) launch_split_group<true>(g, grid, akc, bkc, stream);
-  else launch_split_group<false>(g, grid, akc, bkc, stream);
+void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, bool rows, hipStream_t stream) {
+  if (thin) launch_split_group<true>(g, grid, akc, bkc, rows, stream);
+  else launch_split_group<false>(g, grid, akc, bkc, rows, stream);
 }
 
 }  // namespace gemm

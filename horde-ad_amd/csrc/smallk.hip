@@ -1330,6 +1330,33 @@ void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const ch
   hold_item_locked(ctx, std::move(d));
 }
 
+bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares) {
+  // (memory is taken with the queue unlocked: the allocator may want it)
+  std::shared_ptr<WideJob> job;
+  {
+    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    if (!ctx->dq) return false;
+    if (factor && (!written_by(ctx->dq->items, {factor}).empty() || !written_by(ctx->dq->maps, {factor}).empty())) return false;
+    for (auto& d : ctx->dq->items)
+      if (d.wide && (*shares = wide_row_shares(*d.wide, n, as, M, K, row_stride)) > 0) { job = d.wide; break; }
+  }
+  if (!job || buffer_alloc(ctx, (size_t)M * (size_t)*shares * 8, part)) return false;
+  {
+    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    for (auto& d : ctx->dq->items) {
+      if (d.wide != job) continue;
+      wide_take_rows(*job, (*part)->ptr, factor);
+      d.writes.push_back(*part);
+      buffer_retain(*part);
+      if (factor_buf) { d.reads.push_back(factor_buf); buffer_retain(factor_buf); }
+      return true;
+    }
+  }
+  buffer_release(*part);      // (it has gone out meanwhile)
+  *part = nullptr;
+  return false;
+}
+
 // An elementwise pass joins the queue: it waits for passes that read none of the held results (an optimizer's
 // updates, one per parameter), and goes out when something that reads its result, or may do so, is enqueued.
 void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes) {

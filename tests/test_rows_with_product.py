@@ -1,0 +1,122 @@
+"""Sums of the rows that a waiting fp32 product multiplies come from that product's blocks (csrc/gemm_split.hip) in a recording."""
+import numpy as np
+import pytest
+
+import test_held_sums as held
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def host():
+    return held.pkg.hostapi.Host()
+
+
+def check(host, program, want, size, n):
+    """Every replay against what the program gives submitted one by one, where row sums are launches of their own: both are sums in
+    doubles, rounded once to fp32, and once more for each of at most two additions of results."""
+    eager = [v.numpy() for v in program()]
+    graph, res = host.capture(program)
+    bound = [4 * (2.0 ** -24 + n * 2.0 ** -53) * s for s in size]
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            for got, e in list(zip(res, eager))[len(want):]:      # the products themselves: bit for bit
+                assert np.array_equal(got.numpy(), e, equal_nan=True)
+            for got, e, w, b in zip(res, eager, want, bound):
+                got = got.numpy()
+                fine = np.isfinite(w)
+                assert np.array_equal(got[~fine], w[~fine].astype(np.float32), equal_nan=True)
+                assert np.all(np.abs(got[fine] - w[fine]) <= b[fine]) and np.all(np.abs(got[fine] - e[fine]) <= b[fine])
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
+
+
+def rows(a):
+    return a.stranspose([1, 0]).ssum()
+
+
+@pytest.mark.parametrize("lay", ["K", "R"])
+@pytest.mark.parametrize("m,n,k", [(128, 128, 30000), (129, 300, 20011), (300, 784, 5000), (2050, 130, 4099), (128, 28, 35000), (257, 9, 20003), (34, 32, 9001)])
+def test_row_sums(host, m, n, k, lay):
+    """Whole and ragged tiles of both widths, several columns of tiles, a tail of K; two sums of the same rows, of other rows and of
+    rows of which a part is multiplied; rows with infinities and NaNs."""
+    rng = np.random.default_rng(m)
+    x, z = (rng.uniform(-1, 1, (m, k)).astype(np.float32) for _ in range(2))
+    y = rng.uniform(0, 1, (k, n) if lay == "R" else (n, k)).astype(np.float32)
+    x[3, k - 1], x[7, 0], x[9, 5], x[9, 6] = np.inf, np.nan, np.inf, -np.inf
+    z[5, 11] = -np.inf
+    a, c, b = host.concrete(x), host.concrete(z), host.concrete(y)
+    if lay == "K":
+        b = b.stranspose([1, 0])
+
+    def program():
+        products = [a.smatmul2(b), c.smatmul2(b)]
+        return [rows(a), rows(c), rows(a) + rows(c), -rows(a)] + products
+
+    with np.errstate(invalid="ignore"):
+        sx, sz = x.astype(np.float64).sum(1), z.astype(np.float64).sum(1)
+        want = [sx, sz, sx + sz, -sx]
+        size = [np.abs(x).sum(1, dtype=np.float64), np.abs(z).sum(1, dtype=np.float64)]
+    size += [size[0] + size[1], size[0]]
+
+    check(host, program, want, size, k)
+
+
+def test_operand_written_between(host):
+    """Rows that are overwritten after the product was submitted: the sum is that of what they hold when it is asked for."""
+    rng = np.random.default_rng(1)
+    m, n, k = 128, 128, 20000
+    x, y, z = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n), (m, k)))
+    a, b, c = (host.concrete(v) for v in (x, y, z))
+
+    def program():
+        a.assign(c)
+        p = a.smatmul2(b)
+        s = rows(a)
+        return [p, s]
+
+    [v.numpy() for v in program()]
+    graph, (p, s) = host.capture(program)
+    try:
+        for _ in range(3):
+            a.overwrite(x)
+            graph.launch()
+            host.sync()
+            w = z.astype(np.float64)
+            assert np.all(np.abs(s.numpy() - w.sum(1)) <= 4 * (2.0 ** -24 + k * 2.0 ** -53) * np.abs(w).sum(1))
+            assert np.all(np.abs(p.numpy() - w @ y) <= (k / 16 + 17) * 2.0 ** -24 * (np.abs(w) @ np.abs(y.astype(np.float64))))
+    finally:
+        graph.free()
+
+
+def test_sums_of_terms(host):
+    """A recurrence's weight and bias gradients: several products into one, and the sum of all their rows."""
+    rng = np.random.default_rng(2)
+    m, n, k, t = 130, 96, 5000, 6
+    xs, ys = [rng.uniform(-1, 1, (m, k)).astype(np.float32) for _ in range(t)], [rng.uniform(-1, 1, (k, n)).astype(np.float32) for _ in range(t)]
+    a, b = [host.concrete(x) for x in xs], [host.concrete(y) for y in ys]
+
+    def program():
+        p = a[0].smatmul2(b[0])
+        for u, v in zip(a[1:], b[1:]):
+            p = p + u.smatmul2(v)
+        s = rows(a[-1])
+        for u in a[-2::-1]:      # (in the other order)
+            s = s + rows(u)
+        return [s, p.ssum()]
+
+    x64 = np.concatenate(xs, 1).astype(np.float64)
+    w, mag = x64.sum(1), np.abs(x64).sum(1)
+    eager = [v.numpy() for v in program()]
+    graph, (s, q) = host.capture(program)
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            assert np.all(np.abs(s.numpy() - w) <= 4 * ((t + 1) * 2.0 ** -24 + t * k * 2.0 ** -53) * mag)
+            assert np.array_equal(q.numpy(), eager[1])
+    finally:
+        graph.free()
