@@ -549,6 +549,19 @@ __global__ void __launch_bounds__(kBlock) k_argminmax(Dims keep, int64_t n_out, 
   }
 }
 
+// Where a row's elements are shared out between lanes: a NaN is neither greater nor smaller than anything, so it is no
+// candidate (bi stays INT64_MAX until a number comes), but in the first place of its row, where it stays.
+template <typename T>
+__device__ __forceinline__ bool takes(T x, T best, int64_t bi, int want_max) {
+  return bi == INT64_MAX ? x == x : (want_max ? (x > best) : (x < best));
+}
+template <typename T>
+__device__ __forceinline__ void put_extremum(T first, T best, int64_t bi, int64_t* out, T* val) {
+  const bool keep_first = !(first == first);
+  *out = keep_first ? 0 : bi;
+  if (val) *val = keep_first ? first : best;
+}
+
 // The same with one wavefront per row, for long rows: every lane scans a
 // strided subsequence keeping its first extremum, then lanes combine; on equal
 // values the smaller index wins, which keeps "first occurrence".
@@ -561,16 +574,13 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_wave(Dims keep, int64_t n_
     int64_t ko[1];
     decompose<1>(keep, o, ko);
     const T* p = a + ko[0];
-    bool have = lane < L;
-    T best = have ? p[(int64_t)lane * sl] : T(0);
-    int64_t bi = lane;
-    for (int64_t j = lane + 64; j < L; j += 64) {
+    T best = T(0);
+    int64_t bi = INT64_MAX;
+    for (int64_t j = lane; j < L; j += 64) {
       T x = p[j * sl];
-      bool better = want_max ? (x > best) : (x < best);
-      if (better) { best = x; bi = j; }
+      if (takes(x, best, bi, want_max)) { best = x; bi = j; }
     }
     for (int off = 32; off > 0; off >>= 1) {
-      int o_have = __shfl_down((int)have, off, 64);
       long long o_bi = __shfl_down((long long)bi, off, 64);
       T o_best;
       if constexpr (sizeof(T) == 8) {
@@ -587,15 +597,9 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_wave(Dims keep, int64_t n_
         int w = __shfl_down((int)best, off, 64);
         o_best = (T)w;
       }
-      if (o_have) {
-        bool better = !have || (want_max ? (o_best > best) : (o_best < best)) || (o_best == best && o_bi < bi);
-        if (better) { best = o_best; bi = o_bi; have = true; }
-      }
+      if (o_bi != INT64_MAX && (takes(o_best, best, bi, want_max) || (o_best == best && o_bi < bi))) { best = o_best; bi = o_bi; }
     }
-    if (lane == 0) {
-      out[o] = bi;
-      if (vals) vals[o] = best;
-    }
+    if (lane == 0) put_extremum(p[0], best, bi, out + o, vals ? vals + o : nullptr);
   }
 }
 
@@ -610,7 +614,6 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
   decompose<1>(keep, blockIdx.x, ko);
   const T* p = a + ko[0];
   const int t = threadIdx.x;
-  // a NaN is neither greater nor smaller than anything: it counts only in the first place, where it stays (below)
   T best = t < L ? p[(int64_t)t * sl] : T(0);
   int64_t bi = t < L && best == best ? t : INT64_MAX;
   // eight loads in flight; the comparisons keep the order of the positions
@@ -621,14 +624,12 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
     for (int u = 0; u < 8; ++u) x[u] = p[(j + u * 1024) * sl];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      bool better = bi == INT64_MAX ? x[u] == x[u] : (want_max ? (x[u] > best) : (x[u] < best));
-      if (better) { best = x[u]; bi = j + u * 1024; }
+      if (takes(x[u], best, bi, want_max)) { best = x[u]; bi = j + u * 1024; }
     }
   }
   for (; j < L; j += 1024) {
     T x = p[j * sl];
-    bool better = bi == INT64_MAX ? x == x : (want_max ? (x > best) : (x < best));
-    if (better) { best = x; bi = j; }
+    if (takes(x, best, bi, want_max)) { best = x; bi = j; }
   }
   sbest[t] = best;
   sidx[t] = bi;
@@ -645,12 +646,7 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
     }
     __syncthreads();
   }
-  if (t == 0) {
-    const T first = p[0];
-    const bool keep_first = !(first == first);
-    out[blockIdx.x] = keep_first ? 0 : sidx[0];
-    if (vals) vals[blockIdx.x] = keep_first ? first : sbest[0];
-  }
+  if (t == 0) put_extremum(p[0], sbest[0], sidx[0], out + blockIdx.x, vals ? vals + blockIdx.x : nullptr);
 }
 
 // A few very long rows whose data one CU cannot fetch fast enough (a block
@@ -661,7 +657,7 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
 // then the ticket is drawn.  One row of 50,000 fp64: 9.9 us in two launches, 7.3 in one, with 48 pieces for 24 6.6.
 // The extremum of a row among its G candidates, by one wavefront.
 template <typename T, typename V, typename I>
-__device__ __forceinline__ void pick_body(int G, int want_max, const V& value_of, const I& index_of, int64_t* __restrict__ out, T* __restrict__ vals) {
+__device__ __forceinline__ void pick_body(int G, int want_max, const V& value_of, const I& index_of, T first, int64_t* __restrict__ out, T* __restrict__ vals) {
   const int lane = threadIdx.x & 63;
   T best = T(0);
   int64_t bi = INT64_MAX;
@@ -680,10 +676,7 @@ __device__ __forceinline__ void pick_body(int G, int want_max, const V& value_of
       if (better) { best = ob; bi = oi; }
     }
   }
-  if (lane == 0) {
-    *out = bi;
-    if (vals) *vals = best;
-  }
+  if (lane == 0) put_extremum(first, best, bi, out, vals);
 }
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t L, int64_t sl, int want_max, int G, int64_t piece, const T* __restrict__ a,
@@ -706,14 +699,12 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t 
     for (int u = 0; u < 4; ++u) x[u] = p[(j + u * kBlock) * sl];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      bool better = bi == INT64_MAX || (want_max ? (x[u] > best) : (x[u] < best));
-      if (better) { best = x[u]; bi = j + u * kBlock; }
+      if (takes(x[u], best, bi, want_max)) { best = x[u]; bi = j + u * kBlock; }
     }
   }
   for (; j < j1; j += kBlock) {
     T x = p[j * sl];
-    bool better = bi == INT64_MAX || (want_max ? (x > best) : (x < best));
-    if (better) { best = x; bi = j; }
+    if (takes(x, best, bi, want_max)) { best = x; bi = j; }
   }
   sbest[t] = best;
   sidx[t] = bi;
@@ -750,13 +741,15 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t 
   asm volatile("" ::: "memory");
   auto load = [&](int at) { return __hip_atomic_load(handed + 2 * (int64_t)row * G + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   pick_body<T>(G, want_max, [&](int c) { const unsigned long long u = load(2 * c); T x; __builtin_memcpy(&x, &u, sizeof(T)); return x; },
-               [&](int c) { return (int64_t)load(2 * c + 1); }, out + row, vals ? vals + row : nullptr);
+               [&](int c) { return (int64_t)load(2 * c + 1); }, p[0], out + row, vals ? vals + row : nullptr);
 }
 template <typename T>
-__global__ void __launch_bounds__(64) k_argminmax_pick(int G, int want_max, const T* __restrict__ pbest, const int64_t* __restrict__ pidx, int64_t* __restrict__ out,
+__global__ void __launch_bounds__(64) k_argminmax_pick(Dims keep, int G, int want_max, const T* __restrict__ a, const T* __restrict__ pbest, const int64_t* __restrict__ pidx, int64_t* __restrict__ out,
                                                         T* __restrict__ vals) {
   const int row = blockIdx.x;
-  pick_body<T>(G, want_max, [&](int g) { return pbest[row * G + g]; }, [&](int g) { return pidx[row * G + g]; }, out + row, vals ? vals + row : nullptr);
+  int64_t ko[1];
+  decompose<1>(keep, row, ko);
+  pick_body<T>(G, want_max, [&](int g) { return pbest[row * G + g]; }, [&](int g) { return pidx[row * G + g]; }, a[ko[0]], out + row, vals ? vals + row : nullptr);
 }
 
 // A few very long rows, in pieces: see k_argminmax_pieces (the caller's guard is held).
@@ -774,7 +767,7 @@ int extremum_pieces(hgpu_ctx* ctx, const Dims& keep, int64_t n_out, int64_t L, i
   int64_t* pi = (int64_t*)scratch->ptr + (size_t)n_out * G;
   hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, sl, want_max, G, piece, (const T*)a, pv, pi,
   handed, tickets, (int64_t*)out, (T*)vp);
-  if (!tickets) hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, G, want_max, (const T*)pv, (const int64_t*)pi, (int64_t*)out, (T*)vp);
+  if (!tickets) hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, keep, G, want_max, (const T*)a, (const T*)pv, (const int64_t*)pi, (int64_t*)out, (T*)vp);
   buffer_release(scratch);
   return HGPU_OK;
 }

@@ -64,3 +64,39 @@ def test_rows_of_the_types_own_extremum(gpu, dt):
         vals, idx = gpu.upload(x).extremum_last(want_max)
         assert idx.numpy().tolist() == [0, 1499, 1030, 0]
         assert np.array_equal(vals.numpy(), np.array([end, 3, 3, end], dt))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("rows,n", [(1, 16383), (1, 16384), (3, 50001), (16, 131073), (3, 300), (70, 700)])
+def test_extrema_beside_nans_whoever_shares_a_row(gpu, dt, rows, n):
+    """One rule for a block, for pieces of a row and for a wavefront: a NaN that comes first in a row stays, any other is no candidate --
+    first of a piece, first of a lane, or of every lane; nothing but NaNs behind the first element."""
+    rng = np.random.default_rng(n)
+    base = rng.uniform(-1, 1, (rows, n)).astype(dt)
+    pieces = max(1, min(128, n // 1024))
+    step = (n + pieces - 1) // pieces
+    hidden = min(n - 1, 64 if n < 1024 else 256)      # of the lane that met the NaN first
+    cases = []
+    x = base.copy()
+    x[-1, 0] = np.nan
+    cases.append(x)
+    for end in (5, -5):
+        x = base.copy()
+        x[:, step::step] = np.nan
+        x[:, (step if n > step else 0) + hidden - (0 if n > step else 1)] = end
+        cases.append(x)
+        x = base.copy()
+        x[:, 1:hidden + 1] = np.nan
+        x[:, min(n - 1, 2 * hidden)] = end
+        cases.append(x)
+    x = base.copy()
+    x[0, 1:] = np.nan
+    cases.append(x)
+    cases.append(np.full((rows, n), np.nan, dt))
+    for x in cases:
+        seen = np.where(np.isnan(x[:, :1]), np.arange(n) == 0, ~np.isnan(x))
+        for want_max in (True, False):
+            vals, idx = gpu.upload(x).extremum_last(want_max)
+            want = np.where(seen, np.nan_to_num(x) if want_max else -np.nan_to_num(x), -np.inf).argmax(1)
+            assert np.array_equal(idx.numpy(), want)
+            assert np.array_equal(vals.numpy(), np.take_along_axis(x, want[:, None], 1)[:, 0], equal_nan=True)
