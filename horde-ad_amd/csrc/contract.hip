@@ -651,8 +651,8 @@ __global__ void __launch_bounds__(1024) k_argminmax_block(Dims keep, int64_t L, 
 
 // A few very long rows whose data one CU cannot fetch fast enough (a block
 // draws some tens of GB/s): G blocks per row scan consecutive pieces, then one
-// wavefront per row picks among the G candidates, the earlier piece winning ties: of the block that finishes last (`tickets`
-// not null: a counter per row, 128 bytes apart, zero between launches), or of a second launch.  The candidates travel as the
+// wavefront per row, of the block that finishes last (`tickets`: a counter per row, 128 bytes apart, zero between launches),
+// picks among the G candidates, the earlier piece winning ties.  The candidates travel as the
 // partial sums of the fused sums do: exchanged in by atomics of device scope, the returned value says that they have arrived,
 // then the ticket is drawn.  One row of 50,000 fp64: 9.9 us in two launches, 7.3 in one, with 48 pieces for 24 6.6.
 // The extremum of a row among its G candidates, by one wavefront.
@@ -680,7 +680,6 @@ __device__ __forceinline__ void pick_body(int G, int want_max, const V& value_of
 }
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t L, int64_t sl, int want_max, int G, int64_t piece, const T* __restrict__ a,
-                                                              T* __restrict__ pbest, int64_t* __restrict__ pidx,
                                                               unsigned long long* handed, unsigned* tickets, int64_t* __restrict__ out, T* __restrict__ vals) {
   __shared__ T sbest[kBlock];
   __shared__ int64_t sidx[kBlock];
@@ -721,10 +720,6 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t 
     }
     __syncthreads();
   }
-  if (!tickets) {
-    if (t == 0) { pbest[blockIdx.x] = sbest[0]; pidx[blockIdx.x] = sidx[0]; }
-    return;
-  }
   __shared__ bool last;
   if (t == 0) {
     unsigned long long bits = 0;
@@ -743,33 +738,17 @@ __global__ void __launch_bounds__(kBlock) k_argminmax_pieces(Dims keep, int64_t 
   pick_body<T>(G, want_max, [&](int c) { const unsigned long long u = load(2 * c); T x; __builtin_memcpy(&x, &u, sizeof(T)); return x; },
                [&](int c) { return (int64_t)load(2 * c + 1); }, p[0], out + row, vals ? vals + row : nullptr);
 }
-template <typename T>
-__global__ void __launch_bounds__(64) k_argminmax_pick(Dims keep, int G, int want_max, const T* __restrict__ a, const T* __restrict__ pbest, const int64_t* __restrict__ pidx, int64_t* __restrict__ out,
-                                                        T* __restrict__ vals) {
-  const int row = blockIdx.x;
-  int64_t ko[1];
-  decompose<1>(keep, row, ko);
-  pick_body<T>(G, want_max, [&](int g) { return pbest[row * G + g]; }, [&](int g) { return pidx[row * G + g]; }, a[ko[0]], out + row, vals ? vals + row : nullptr);
-}
 
-// A few very long rows, in pieces: see k_argminmax_pieces (the caller's guard is held).
+// A few very long rows, in pieces: see k_argminmax_pieces (the caller's guard is held; `scratch` holds 16 bytes per piece).
 // (One row of 10,000 fp64: ten pieces 6.6 us, one block of 1024 lanes 6.4.)
-constexpr int64_t kPiecesFrom = 16384, kPiece = 1024;
+constexpr int64_t kPiecesFrom = 16384, kPiece = 1024, kPiecesRows = 16;
+int pieces_of(int64_t L) { return (int)std::min<int64_t>(128, L / kPiece); }
 template <typename T>
-int extremum_pieces(hgpu_ctx* ctx, const Dims& keep, int64_t n_out, int64_t L, int64_t sl, int want_max, const void* a, unsigned* tickets, void* out, void* vp) {
-  const int G = (int)std::min<int64_t>(128, L / kPiece);
+void extremum_pieces(hgpu_ctx* ctx, const Dims& keep, int64_t n_out, int64_t L, int64_t sl, int want_max, const void* a, void* scratch, unsigned* tickets, void* out, void* vp) {
+  const int G = pieces_of(L);
   const int64_t piece = (L + G - 1) / G;
-  hgpu_buffer* scratch = nullptr;
-  const int rc = buffer_alloc(ctx, (size_t)n_out * G * 16, &scratch);
-  if (rc) return rc;
-  T* pv = (T*)scratch->ptr;
-  unsigned long long* handed = tickets ? (unsigned long long*)scratch->ptr : nullptr;
-  int64_t* pi = (int64_t*)scratch->ptr + (size_t)n_out * G;
-  hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, sl, want_max, G, piece, (const T*)a, pv, pi,
-  handed, tickets, (int64_t*)out, (T*)vp);
-  if (!tickets) hipLaunchKernelGGL(k_argminmax_pick<T>, dim3((unsigned)n_out), dim3(64), 0, ctx->stream, keep, G, want_max, (const T*)a, (const T*)pv, (const int64_t*)pi, (int64_t*)out, (T*)vp);
-  buffer_release(scratch);
-  return HGPU_OK;
+  hipLaunchKernelGGL(k_argminmax_pieces<T>, dim3((unsigned)(n_out * G)), dim3(kBlock), 0, ctx->stream, keep, L, sl, want_max, G, piece, (const T*)a,
+                     (unsigned long long*)scratch, tickets, (int64_t*)out, (T*)vp);
 }
 
 // The buffers of a reduction whose launch may be held back (see RedJob): what it reads and what it writes.
@@ -1483,18 +1462,19 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
     const int64_t* ks[1] = {a->strides};
     Dims keep;
     if (!collapse(a->rank - 1, a->shape, 1, ks, &keep)) { hgpu_release(o); if (v) hgpu_release(v); return fail(ctx, HGPU_ERR_UNSUPPORTED, "argminmax: too many dims"); }
-    const bool pieces = L >= kPiecesFrom && n_out <= 16;
+    const bool pieces = L >= kPiecesFrom && n_out <= kPiecesRows;
     void* tickets = nullptr;
-    if (pieces && (ctx->ticket_block || !ctx->cap)) rc = ticket_block(ctx, &tickets);
+    hgpu_buffer* scratch = nullptr;
+    if (pieces) rc = ticket_block(ctx, &tickets);
+    if (pieces && !rc) rc = buffer_alloc(ctx, (size_t)(n_out * pieces_of(L)) * 16, &scratch);
     if (rc) { hgpu_release(o); if (v) hgpu_release(v); return rc; }
     const std::vector<const void*> reads = reads_of(1, &a);
     LaunchGuard lg(ctx, "argminmax", (double)n_out * (L * dtype_size(a->dtype) + 8 + (v ? dtype_size(a->dtype) : 0)), (double)n_out * L, &reads);
     void* vp = v ? data_ptr(v) : nullptr;
     if (pieces) {
       // very few, very long rows: pieces of a row to many blocks, then one pick per row
-      // (a recording that meets the first such row of the process gets two launches: the counters cannot be cleared in it)
-      HG_DISPATCH_DTYPE(a->dtype, T, rc = extremum_pieces<T>(ctx, keep, n_out, L, a->strides[a->rank - 1], want_max, data_ptr(a), (unsigned*)tickets, data_ptr(o), vp));
-      if (rc) { hgpu_release(o); if (v) hgpu_release(v); return rc; }
+      HG_DISPATCH_DTYPE(a->dtype, T, extremum_pieces<T>(ctx, keep, n_out, L, a->strides[a->rank - 1], want_max, data_ptr(a), scratch->ptr, (unsigned*)tickets, data_ptr(o), vp));
+      buffer_release(scratch);
     } else if (L >= 512 && n_out <= 64) {
       // few long rows: a whole block per row (one row of 2500 fp32, a minibatch's logits: a wavefront, load after load, takes
       // 14.4 us, a block 5.8; one of 1500 fp64 9.9 and 5.0)

@@ -99,9 +99,6 @@ struct FDims {
 
 }  // namespace
 
-namespace hg {
-}
-
 // hgpu_fused_map, and with sum_slot >= 0 hgpu_fused_map_dimsum: the same pass
 // also adds up slot sum_slot over every dim but keep_dim.
 static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, int n_out, const int* out_slots,
