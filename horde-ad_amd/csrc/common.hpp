@@ -95,6 +95,10 @@ struct hgpu_ctx {
   std::set<std::string> label_pool;
   std::mutex label_mu;                    // guards label_pool: labels are made on any calling thread
   std::vector<ProfRec> prof;
+  // A launch that goes into a recording is counted by its label; nothing is timed there.
+  void count_recorded(const char* name, double bytes, double flops) {
+    if (profiling && cap && name) prof.push_back({name, nullptr, nullptr, bytes, flops});
+  }
   hgpu_buffer* zero_block = nullptr;     // 256 zero bytes, for kernels that want a dummy table
   hgpu_buffer* ticket_block = nullptr;   // counters (zero between launches) for kernels whose last block finishes a reduction
   hgpu_cap_pool* cap = nullptr;          // non-null while the stream is capturing into a graph
@@ -229,6 +233,7 @@ constexpr int kMaxWideJobs = 4;
 // gemm.hip: row sums that a held product hands out beside its result (see join_wide_rows)
 int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride);
 void wide_take_rows(WideJob& job, void* part, const void* factor);
+bool wide_takes_rows(const WideJob& job);
 // smallk.hip: the sums over K of n terms of M rows of fp32 elements, each term times the one element `factor` (null: 1), as
 // *part (rows x *shares, doubles) by a held product that reads the same rows; false: there is none
 bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
@@ -293,6 +298,7 @@ struct LaunchGuard {
     else if (c->dq_pending) flush_deferred_locked(c);   // stream order is program order
     static const bool trace = getenv("HORDEAD_GPU_TRACE_LAUNCHES") != nullptr;   // one line per launch, in program order
     if (trace && name) fprintf(stderr, "hordead_gpu: launch %s\n", name);
+    c->count_recorded(name, bytes, flops);
     if (c->profiling && name && !c->cap) {
       hgpu_ctx::ProfRec r{name, nullptr, nullptr, bytes, flops};
       if (hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess) {

@@ -470,6 +470,7 @@ int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M,
   return x == y ? job.j.splits : 0;
 }
 
+bool wide_takes_rows(const WideJob& job) { return job.j.p.rows != nullptr; }
 void wide_take_rows(WideJob& job, void* part, const void* factor) {
   job.j.p.rows = (double*)part;
   job.j.p.row_factor = (const float*)factor;

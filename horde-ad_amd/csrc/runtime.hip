@@ -517,8 +517,9 @@ int hgpu_profile_enable(hgpu_ctx* ctx, int on) {
   if (!ctx) return HGPU_ERR_INVALID;
   std::lock_guard<std::mutex> g(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
-  (void)hipStreamSynchronize(ctx->stream);
-  for (auto& r : ctx->prof) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
+  if (!ctx->cap) (void)hipStreamSynchronize(ctx->stream);
+  for (auto& r : ctx->prof)
+    if (r.a) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   ctx->prof.clear();
   ctx->profiling = on != 0;
   ctx->profile_shapes = on == 2;
@@ -529,12 +530,12 @@ int hgpu_profile_report(hgpu_ctx* ctx, char* buf, size_t n) {
   if (!ctx || !buf || n == 0) return HGPU_ERR_INVALID;
   std::lock_guard<std::mutex> g(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
-  (void)hipStreamSynchronize(ctx->stream);
+  if (!ctx->cap) (void)hipStreamSynchronize(ctx->stream);
   struct Agg { long count = 0; double ms = 0, bytes = 0, flops = 0; };
   std::map<std::string, Agg> agg;
   for (auto& r : ctx->prof) {
     float ms = 0;
-    if (hipEventElapsedTime(&ms, r.a, r.b) != hipSuccess) continue;
+    if (r.a && hipEventElapsedTime(&ms, r.a, r.b) != hipSuccess) continue;
     Agg& a = agg[r.name];
     a.count++;
     a.ms += ms;
@@ -542,10 +543,10 @@ int hgpu_profile_report(hgpu_ctx* ctx, char* buf, size_t n) {
     a.flops += r.flops;
   }
   std::string out;
-  char line[256];
+  char line[96];
   for (auto& kv : agg) {
-    snprintf(line, sizeof line, "%s %ld %.6f %.0f %.0f\n", kv.first.c_str(), kv.second.count, kv.second.ms, kv.second.bytes, kv.second.flops);
-    out += line;
+    snprintf(line, sizeof line, " %ld %.6f %.0f %.0f\n", kv.second.count, kv.second.ms, kv.second.bytes, kv.second.flops);
+    out += kv.first + line;
   }
   snprintf(buf, n, "%s", out.c_str());
   return HGPU_OK;

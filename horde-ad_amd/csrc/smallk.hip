@@ -933,6 +933,7 @@ static void launch_maps(hgpu_ctx* ctx, std::vector<Deferred>& items) {
       if (items[i].map.fn == m.fn) jobs.push_back(&items[i].map);
     hgpu_ctx::ProfRec r{jobs.size() > 1 ? "fused_map_group" : m.label, nullptr, nullptr, 0, 0};
     for (auto* j : jobs) { r.bytes += j->bytes; r.flops += j->flops; }
+    ctx->count_recorded(r.name, r.bytes, r.flops);
     const bool timed = ctx->profiling && !ctx->cap && hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess;
     std::vector<uint64_t> block;       // struct Group of the kernel's text: the jobs' arguments, then the first block of each
     std::vector<void*> args;
@@ -1002,6 +1003,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     return;
   }
   auto timed_launch = [&](hipFunction_t fn, unsigned grid, const std::vector<const void*>& ar, const char* label, double bytes, double flops, unsigned block = 256) {
+    ctx->count_recorded(label, bytes, flops);
     // (timed: the launch carries its record's two events, which then hold the kernel's own begin and end)
     hipEvent_t ea = nullptr, eb = nullptr;
     if (ctx->profiling && !ctx->cap && (uint64_t)grid * block <= 0xffffffffull) {
@@ -1103,7 +1105,17 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
       for (size_t g0 = 0, g1 = 0; g0 < wide.size(); g0 = g1) {
         const WideJob* jobs[kMaxWideJobs];
         int n = 0;
-        for (; g1 < wide.size() && n < kMaxWideJobs && wide[g1]->wide_kernel == wide[g0]->wide_kernel; ++g1) jobs[n++] = wide[g1]->wide.get();
+        double bytes = 0, flops = 0;
+        for (; g1 < wide.size() && n < kMaxWideJobs && wide[g1]->wide_kernel == wide[g0]->wide_kernel; ++g1) {
+          jobs[n++] = wide[g1]->wide.get();
+          bytes += wide[g1]->bytes;
+          flops += wide[g1]->flops;
+        }
+        if (ctx->profiling) {
+          std::string lab = n > 1 ? "gemm_wide_group[" : "";
+          for (size_t i = g0; i < g1; ++i) lab += (i > g0 ? "|" : "") + std::string(wide[i]->label) + (wide_takes_rows(*wide[i]->wide) ? "+rows" : "");
+          ctx->count_recorded(intern_label(ctx, lab + (n > 1 ? "]" : "")), bytes, flops);
+        }
         const hipError_t err = launch_wide_group(ctx, jobs, n);
         if (err != hipSuccess) {
           int rc = check_hip(ctx, err, "grouped product launch");
@@ -1136,6 +1148,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
             label = intern_label(ctx, lab + "]");
           }
         }
+        ctx->count_recorded(label, bytes, flops);
         bool timed = false;
         if (ctx->profiling && !ctx->cap) {
           hgpu_ctx::ProfRec r{label, nullptr, nullptr, bytes, flops};

@@ -124,7 +124,8 @@ int hgpu_inject_alloc_failure(hgpu_ctx* ctx, int64_t limit);
  * dispatch (a few microseconds more per launch).  The report has one
  * line per kernel family: "name launches total_ms algorithmic_bytes
  * algorithmic_flops".  Enabling (or disabling) clears the records.  on = 2
- * makes the matrix-product labels carry the problem shape. */
+ * makes the matrix-product labels carry the problem shape.  Launches that go
+ * into a recording are counted under their labels and take no time. */
 int hgpu_profile_enable(hgpu_ctx* ctx, int on);
 int hgpu_profile_report(hgpu_ctx* ctx, char* buf, size_t n);
 

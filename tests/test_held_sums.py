@@ -1,4 +1,6 @@
 """Sums of partial results wait for one another (csrc/smallk.hip, make_way_locked; csrc/contract.hip, k_contract_group)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -8,6 +10,22 @@ from test_gemm_split import product
 pytestmark = pytest.mark.gpu
 
 EPS = {np.float64: 2.0 ** -53, np.float32: 2.0 ** -24}
+
+
+def recorded(host, program):
+    """The recorded program, its results, and how often each kernel is launched by it."""
+    lib, ctx = pkg.capi.Lib(), host.dll.hh_array_ctx(host.h)
+    assert lib.profile_enable(ctx, 2) == 0
+    graph, res = host.capture(program)
+    report = C.create_string_buffer(1 << 16)
+    assert lib.profile_report(ctx, report, len(report)) == 0 and lib.profile_enable(ctx, 0) == 0
+    return graph, res, {line.rsplit(None, 4)[0]: int(line.rsplit(None, 4)[1]) for line in report.value.decode().splitlines()}
+
+
+def force(host, *values):
+    """Submitted now, in this order (products and sums of a program are submitted when they are asked for)."""
+    for v in values:
+        host.check(host.dll.hh_force(host.h, v.h))
 
 
 class Value:
@@ -178,7 +196,10 @@ def test_products_of_a_recording_go_out_together(host, dt, shapes, lay):
         return out + [a.stranspose([1, 0]).ssum() for a, _ in ops[:2]]
 
     eager = [v.numpy() for v in program()]
-    graph, res = host.capture(program)
+    graph, res, labels = recorded(host, program)
+    # (products of one layout, a launch takes four of them)
+    alike = len(pairs) if dt == np.float64 or min(min(m, n) for m, n, _ in shapes) > 32 else sum(min(m, n) <= 32 for m, n, _ in shapes)
+    assert alike < 2 or sum(k.count("|gemm_f") * v for k, v in labels.items() if k.startswith("gemm_wide_group[")) >= (alike + 1) // 2, labels
     try:
         for _ in range(3):
             graph.launch()

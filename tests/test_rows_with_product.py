@@ -12,11 +12,12 @@ def host():
     return held.pkg.hostapi.Host()
 
 
-def check(host, program, want, size, n):
-    """Every replay against what the program gives submitted one by one, where row sums are launches of their own: both are sums in
+def check(host, program, want, size, n, joined):
+    """`joined` of the recording's sums come from a product's blocks.  Every replay against what the program gives submitted one by one, where row sums are launches of their own: both are sums in
     doubles, rounded once to fp32, and once more for each of at most two additions of results."""
     eager = [v.numpy() for v in program()]
-    graph, res = host.capture(program)
+    graph, res, labels = held.recorded(host, program)
+    assert sum(k.count("+rows") * v for k, v in labels.items()) == joined, labels
     bound = [4 * (2.0 ** -24 + n * 2.0 ** -53) * s for s in size]
     try:
         for _ in range(3):
@@ -39,10 +40,11 @@ def rows(a):
 
 
 @pytest.mark.parametrize("lay", ["K", "R"])
+@pytest.mark.parametrize("first", ["products", "sums"])
 @pytest.mark.parametrize("m,n,k", [(128, 128, 30000), (129, 300, 20011), (300, 784, 5000), (2050, 130, 4099), (128, 28, 35000), (257, 9, 20003), (34, 32, 9001)])
-def test_row_sums(host, m, n, k, lay):
+def test_row_sums(host, m, n, k, first, lay):
     """Whole and ragged tiles of both widths, several columns of tiles, a tail of K; two sums of the same rows, of other rows and of
-    rows of which a part is multiplied; rows with infinities and NaNs."""
+    rows of which a part is multiplied; rows with infinities and NaNs.  A sum that is asked for before the products are is a launch of its own."""
     rng = np.random.default_rng(m)
     x, z = (rng.uniform(-1, 1, (m, k)).astype(np.float32) for _ in range(2))
     y = rng.uniform(0, 1, (k, n) if lay == "R" else (n, k)).astype(np.float32)
@@ -54,6 +56,8 @@ def test_row_sums(host, m, n, k, lay):
 
     def program():
         products = [a.smatmul2(b), c.smatmul2(b)]
+        if first == "products":
+            held.force(host, *products)
         return [rows(a), rows(c), rows(a) + rows(c), -rows(a)] + products
 
     with np.errstate(invalid="ignore"):
@@ -62,7 +66,7 @@ def test_row_sums(host, m, n, k, lay):
         size = [np.abs(x).sum(1, dtype=np.float64), np.abs(z).sum(1, dtype=np.float64)]
     size += [size[0] + size[1], size[0]]
 
-    check(host, program, want, size, k)
+    check(host, program, want, size, k, 2 if first == "products" else 0)
 
 
 def test_operand_written_between(host):
@@ -75,11 +79,13 @@ def test_operand_written_between(host):
     def program():
         a.assign(c)
         p = a.smatmul2(b)
+        held.force(host, p)
         s = rows(a)
         return [p, s]
 
     [v.numpy() for v in program()]
-    graph, (p, s) = host.capture(program)
+    graph, (p, s), labels = held.recorded(host, program)
+    assert any("+rows" in k for k in labels), labels
     try:
         for _ in range(3):
             a.overwrite(x)
@@ -97,21 +103,24 @@ def test_sums_of_terms(host):
     rng = np.random.default_rng(2)
     m, n, k, t = 130, 96, 5000, 6
     xs, ys = [rng.uniform(-1, 1, (m, k)).astype(np.float32) for _ in range(t)], [rng.uniform(-1, 1, (k, n)).astype(np.float32) for _ in range(t)]
-    a, b = [host.concrete(x) for x in xs], [host.concrete(y) for y in ys]
+    a, b, one = [host.concrete(x) for x in xs], [host.concrete(y) for y in ys], host.concrete(np.ones((), np.float32))
 
     def program():
         p = a[0].smatmul2(b[0])
         for u, v in zip(a[1:], b[1:]):
             p = p + u.smatmul2(v)
-        s = rows(a[-1])
+        held.force(host, p)
+        ones = one.sreplicate(k).sreplicate(m)
+        s = a[-1].sdot1In(ones)
         for u in a[-2::-1]:      # (in the other order)
-            s = s + rows(u)
+            s = s + u.sdot1In(ones)
         return [s, p.ssum()]
 
     x64 = np.concatenate(xs, 1).astype(np.float64)
     w, mag = x64.sum(1), np.abs(x64).sum(1)
     eager = [v.numpy() for v in program()]
-    graph, (s, q) = host.capture(program)
+    graph, (s, q), labels = held.recorded(host, program)
+    assert any("+rows" in k for k in labels), labels
     try:
         for _ in range(3):
             graph.launch()
