@@ -790,7 +790,7 @@ struct SplitParams {
   int n_terms, term_split;
   const void* a_term[kMaxTerms];
   const void* b_term[kMaxTerms];
-  double* rows;                 // sums of A's rows over the block's share of K, times *row_factor (rows x shares of K; null: not asked for)
+  double* rows;                 // sums of A's rows over the block's share of K, each element times *row_factor (rows x shares of K; null: not asked for)
   const float* row_factor;      // null: 1
 };
 // The share of such a product that a block computes: rows from m0, columns from n0, k in [kbeg, kend), operands of its term

@@ -167,7 +167,7 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
 // gradient multiplies.  Blocks of the first column of tiles do, for products that ask (split_job).  Reading A once more for
 // them: 28 x 128 rows of 5000 17.5 us, 2048 rows of 8192 17.4; here
 // the recurrent network's three products of 128 x 128 take 139 us for 135 and the one of 128 x 28 32 for 29.  (The large tile keeps
-// 16 to 20 bytes of a lane in scratch memory then, outside of its loop's loads.)
+// 12 to 20 bytes of a lane in scratch memory then, outside of its loop's loads.)
 template <bool AKC, bool BKC, bool THIN, bool ROWS>
 __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = THIN ? 4 : 2, WN = THIN ? 1 : 2, TM = THIN ? 1 : 2, TN = THIN ? 1 : 2;          // wavefronts, and 32 x 32 blocks of each
@@ -199,12 +199,14 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   Slot ra[NA], rb[NB];
   static_assert(!ROWS || (AKC && NA == 1 && BM * 2 == NT), "lane t stages a half of row t / 2");
   const bool sum_rows = ROWS && p.rows != nullptr && n0 == 0;
-  double row_sum = 0;
-  auto store_a = [&](int u, u4* to) {
+  double row_sum = 0, row_factor = 1;
+  if (sum_rows && p.row_factor) row_factor = (double)*p.row_factor;
+  auto store_a = [&](int u, u4* to, int left) {      // left: elements of k that the step has, 16 and more: all
     sa.store(ra[u], u, to, top_a);
     if (sum_rows) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) row_sum += (double)ra[u].v[j];
+      for (int j = 0; j < 8; ++j)
+        if (left >= SK || 8 * (t & 1) + j < left) row_sum = __builtin_fma((double)ra[u].v[j], row_factor, row_sum);      // (the product is exact)
     }
   };
   auto fetch = [&](int i) {                 // (chosen outside the main loop: a load on one side of a branch would be waited for where the sides meet)
@@ -218,7 +220,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   if (whole > 0) fetch(0);
   else fetch_tail(0);
 #pragma unroll
-  for (int i = 0; i < NA; ++i) store_a(i, lds[0]);
+  for (int i = 0; i < NA; ++i) store_a(i, lds[0], kend - kbeg);
 #pragma unroll
   for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, top_b);
   __syncthreads();
@@ -236,6 +238,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
     const u4* la = lds[cur] + fra;
     const u4* lb = lds[cur] + PA + frb;
     u4* ln = lds[cur ^ 1];
+    const int left = decltype(next)::value == 2 ? kend - kbeg - (i0 + 1) * SK : SK;
     bf8 fa[TM][3];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -267,7 +270,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
         constexpr int first = 1;
         if (j >= first) {
           const int u = j - first;
-          if (u < NA) store_a(u, ln);
+          if (u < NA) store_a(u, ln, left);
           else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, top_b);
         }
       }
@@ -276,7 +279,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
       constexpr int first = 1;
 #pragma unroll
       for (int u = TN - first; u < NA + NB; ++u) {
-        if (u < NA) store_a(u, ln);
+        if (u < NA) store_a(u, ln, left);
         else sb.store(rb[u - NA], u - NA, ln + PA, top_b);
       }
     }
@@ -293,7 +296,6 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
 
   if (sum_rows) {
     row_sum += __shfl_xor(row_sum, 1);
-    if (p.row_factor) row_sum *= (double)*p.row_factor;
     if (!(t & 1) && m0 + t / 2 < p.M) p.rows[(int64_t)(m0 + t / 2) * nsplits + share.s] = row_sum;
   }
   float* Cout = C + (int64_t)batch * p.bsc + (int64_t)share.s * p.c_split_stride;

@@ -129,3 +129,24 @@ def test_sums_of_terms(host):
             assert np.array_equal(q.numpy(), eager[1])
     finally:
         graph.free()
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 128, 30000), (129, 28, 20011)])
+@pytest.mark.parametrize("f", [np.inf, -0.75, 0.0, 3e38])
+def test_factor_of_a_row_sum(host, m, n, k, f):
+    """Every element is multiplied before it is added: an infinite factor over a row that has a zero, or both signs, gives no number."""
+    rng = np.random.default_rng(m)
+    x, y = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(0, 1, (k, n)).astype(np.float32)
+    x[1, 17], x[2, k - 1], x[5, :2], x[m - 1, 0] = 0.0, -1.0, (np.inf, -np.inf), np.nan
+    a, b, c = host.concrete(x), host.concrete(y), host.concrete(np.asarray(f, np.float32))
+
+    def program():
+        p = a.smatmul2(b)
+        held.force(host, p)
+        return [a.sdot1In(c.sreplicate(k).sreplicate(m)), p]
+
+    with np.errstate(invalid="ignore"):
+        terms = x.astype(np.float64) * np.float64(np.float32(f))
+        want, size = terms.sum(1), np.abs(terms).sum(1)
+        big = np.where(np.abs(want) >= 2.0 ** 128, np.sign(want) * np.inf, want)
+    check(host, program, [big], [size], k, 1)
