@@ -100,6 +100,9 @@ struct Chunk {
 
 struct Spec {
   bool f64;
+  // fp32 elements, sums in fp64: see try_smallk
+  bool wide = false;
+  bool sums64() const { return f64 || wide; }
   int64_t P, Q;
   int BP, BQ, WP, WQ;
   std::vector<Term> terms;
@@ -116,7 +119,7 @@ struct Spec {
   // (a bare product writes whole partial results instead, which wait for other sums to be added up with: sum_partials;
   // 784 x 128 over 1000 fp64, the launch that finished it was 4.7 us)
   int splits = 1, chunks_per_split = 0;
-  bool bare() const { return n_instr == 0 && n_in == 1 && out_slots.size() == 1; }
+  bool bare() const { return !wide && n_instr == 0 && n_in == 1 && out_slots.size() == 1; }
   bool finishes() const { return splits > 1 && !bare(); }
   // WK = 4: a 16 x 16 tile per block, each wavefront a quarter of every chunk's k (see choose_flat); 1: wavefronts share K
   int WK = 1;
@@ -237,12 +240,12 @@ std::string generate_body(const Spec& sp) {
   const int S = sp.splits;
   const int64_t nblk = nbp * nbq, per_xcd = (nblk * S + 7) / 8;
   const bool flat = sp.WK > 1;
-  const bool vec_epi = !flat && !sp.f64 && sp.P % 4 == 0;
+  const bool vec_epi = !flat && !sp.sums64() && sp.P % 4 == 0;
   s << "typedef " << (sp.f64 ? "double" : "float") << " T;\n";
   s << "typedef T V2 __attribute__((ext_vector_type(2), aligned(" << (sp.f64 ? 8 : 4) << ")));\n";
   s << "typedef T V4 __attribute__((ext_vector_type(4), aligned(" << (sp.f64 ? 8 : 4) << ")));\n";
   s << "typedef T A2 __attribute__((ext_vector_type(2)));\ntypedef T A4 __attribute__((ext_vector_type(4)));\n";
-  s << "typedef T Acc __attribute__((ext_vector_type(4)));\n";
+  s << "typedef " << (sp.sums64() ? "double" : "float") << " S;\ntypedef S Acc __attribute__((ext_vector_type(4)));\n";
   // vectors of four for every type the program reads or writes
   s << "template <typename E> struct Vec4 { typedef E type __attribute__((ext_vector_type(4), aligned(sizeof(E)))); };\n";
   s << "struct Args {\n";
@@ -250,7 +253,7 @@ std::string generate_body(const Spec& sp) {
   for (int i = 0; i < sp.n_in; ++i)
     if (i != sp.c_slot) s << "  const " << ctype(sp.dt[(size_t)i]) << "* i" << i << ";\n";
   for (size_t o = 0; o < sp.out_slots.size(); ++o) s << "  " << ctype(sp.dt[(size_t)sp.out_slots[o]]) << "* o" << o << ";\n";
-  if (sp.finishes()) s << "  T* part;\n";
+  if (sp.finishes()) s << "  S* part;\n";
   s << "};\n";
   for (size_t c = 0; c < sp.chunks.size(); ++c) {
     emit_stage_fn(s, ("x" + std::to_string(c)).c_str(), sp.chunks[c].x, sp.chunks[c], "", "");
@@ -276,7 +279,7 @@ std::string generate_body(const Spec& sp) {
   s << "#pragma unroll\n  for (int j0 = 0; j0 < NS; j0 += G) {\n    const int cur = (j0 / G) & 1;\n    if (j0 + G < NS) rd(cur ^ 1, j0 + G);\n    __builtin_amdgcn_sched_barrier(0);\n";
   s << "#pragma unroll\n    for (int u = 0; u < G; ++u) {\n      if (j0 + u >= NS) break;\n";
   s << "#pragma unroll\n      for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n        for (int b = 0; b < " << TQ << "; ++b)\n";
-  if (sp.f64) s << "          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(yf[cur][u][b], xf[cur][u][a], acc[a][b], 0, 0, 0);\n";
+  if (sp.sums64()) s << "          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64((S)yf[cur][u][b], (S)xf[cur][u][a], acc[a][b], 0, 0, 0);\n";
   else s << "          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[cur][u][a], yf[cur][u][b], acc[a][b], 0, 0, 0);\n";
   s << "    }\n    __builtin_amdgcn_sched_barrier(0);\n  }\n}\n";
   // The program over one accumulator block.  What it reads besides the
@@ -288,8 +291,8 @@ std::string generate_body(const Spec& sp) {
     if (i == sp.c_slot) continue;
     const char* ct = ctype(sp.dt[(size_t)i]);
     if (vec_epi && sp.in_sp[(size_t)i] == 1) s << "  Vec4<" << ct << ">::type w" << i << ";\n";
-    else if (sp.in_sp[(size_t)i] == 0 && !sp.f64) s << "  " << ct << " w" << i << ";\n";      // one q per lane
-    else if (sp.in_sp[(size_t)i] == 0) s << "  " << ct << " w" << i << "x[4];\n";                  // fp64: a lane's four values are four q
+    else if (sp.in_sp[(size_t)i] == 0 && !sp.sums64()) s << "  " << ct << " w" << i << ";\n";      // one q per lane
+    else if (sp.in_sp[(size_t)i] == 0) s << "  " << ct << " w" << i << "x[4];\n";                  // sums in fp64: a lane's four values are four q
     else s << "  " << ct << " w" << i << "[4];\n";
   }
   s << "  int unused;\n};\n";
@@ -311,12 +314,12 @@ std::string generate_body(const Spec& sp) {
     for (int i = 0; i < sp.n_in; ++i) any_q = any_q || (i != sp.c_slot);
     if (any_q) {
       s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n" << skip;
-      if (sp.f64) s << "    i64 p = pb + r, q = qb + 4 * e + g;\n";
+      if (sp.sums64()) s << "    i64 p = pb + r, q = qb + 4 * e + g;\n";
       else s << "    i64 p = pb + 4 * g + e, q = qb + r;\n";
       s << "    p = p > " << sp.P - 1 << "LL ? " << sp.P - 1 << "LL : p;\n    q = q > " << sp.Q - 1 << "LL ? " << sp.Q - 1 << "LL : q;\n";
       for (int i = 0; i < sp.n_in; ++i) {
         if (i == sp.c_slot) continue;
-        if (sp.in_sp[(size_t)i] == 0 && !sp.f64) s << (flat ? "    z.w" : "    if (e == 0) z.w") << i << " = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
+        if (sp.in_sp[(size_t)i] == 0 && !sp.sums64()) s << (flat ? "    z.w" : "    if (e == 0) z.w") << i << " = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
         else if (sp.in_sp[(size_t)i] == 0) s << "    z.w" << i << "x[e] = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL];\n";
         else s << "    z.w" << i << "[e] = ar.i" << i << "[q * " << sp.in_sq[(size_t)i] << "LL + p * " << sp.in_sp[(size_t)i] << "LL];\n";
       }
@@ -346,13 +349,13 @@ std::string generate_body(const Spec& sp) {
     }
   } else {
     s << "#pragma unroll\n  for (int e = 0; e < 4; ++e) {\n" << skip;
-    if (sp.f64) s << "    const i64 p = pb + r, q = qb + 4 * e + g;\n";
+    if (sp.sums64()) s << "    const i64 p = pb + r, q = qb + 4 * e + g;\n";
     else s << "    const i64 p = pb + 4 * g + e, q = qb + r;\n";
     s << "    if (p >= " << sp.P << "LL || q >= " << sp.Q << "LL) continue;\n";
     for (int i = 0; i < sp.n_in; ++i) {
       const char* ct = ctype(sp.dt[(size_t)i]);
-      if (i == sp.c_slot) s << "    const T v" << i << " = c[e];\n";
-      else if (sp.in_sp[(size_t)i] == 0 && !sp.f64) s << "    const " << ct << " v" << i << " = z.w" << i << ";\n";
+      if (i == sp.c_slot) s << "    const T v" << i << " = (T)c[e];\n";
+      else if (sp.in_sp[(size_t)i] == 0 && !sp.sums64()) s << "    const " << ct << " v" << i << " = z.w" << i << ";\n";
       else if (sp.in_sp[(size_t)i] == 0) s << "    const " << ct << " v" << i << " = z.w" << i << "x[e];\n";
       else s << "    const " << ct << " v" << i << " = z.w" << i << "[e];\n";
     }
@@ -425,8 +428,9 @@ std::string generate_body(const Spec& sp) {
         << kq * (ch.x.layout == 0 ? ch.x.pitch : 1) << ", ys + " << yat[c] << " + w * " << kq * (ch.y.layout == 0 ? ch.y.pitch : 1) << ", acc, r, g, wp, wq);\n";
     }
     // the quarters meet in LDS (free once every wavefront has read its fragments); wavefront w finishes register w of every lane
-    s << "  __syncthreads();\n#pragma unroll\n  for (int e = 0; e < 4; ++e) lds[(w * 4 + e) * 64 + lane] = acc[0][0][e];\n  __syncthreads();\n";
-    s << "  {\n    const T* q4 = lds + w * 64 + lane;\n    const T t = (q4[0] + q4[256]) + (q4[512] + q4[768]);\n    acc[0][0] = Acc{t, t, t, t};\n  }\n";
+    s << "  S* const sums = reinterpret_cast<S*>(lds);\n";
+    s << "  __syncthreads();\n#pragma unroll\n  for (int e = 0; e < 4; ++e) sums[(w * 4 + e) * 64 + lane] = acc[0][0][e];\n  __syncthreads();\n";
+    s << "  {\n    const S* q4 = sums + w * 64 + lane;\n    const S t = (q4[0] + q4[256]) + (q4[512] + q4[768]);\n    acc[0][0] = Acc{t, t, t, t};\n  }\n";
   } else if (S == 1) {
     run_chunks(0, nc);
   } else {
@@ -440,7 +444,7 @@ std::string generate_body(const Spec& sp) {
   if (sp.finishes()) {
     // hand the partial tile over: the registers of a lane side by side for the block's 256 lanes
     const int nreg = TP * TQ * 4;
-    s << "  {\n    T* mine = ar.part + ((blk * " << S << " + sidx) * " << nreg << "LL) * 256 + tid;\n";
+    s << "  {\n    S* mine = ar.part + ((blk * " << S << " + sidx) * " << nreg << "LL) * 256 + tid;\n";
     s << "#pragma unroll\n    for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n      for (int b = 0; b < " << TQ << "; ++b)\n#pragma unroll\n        for (int e = 0; e < 4; ++e) {\n";
     s << "          mine[((a * " << TQ << " + b) * 4 + e) * 256] = acc[a][b][e];\n        }\n  }\n";
     s << "}\n";
@@ -454,7 +458,7 @@ std::string generate_body(const Spec& sp) {
     s << "  Acc acc[" << TP << "][" << TQ << "];\n";
     if (n_read > 0) s << "  EpiIn ei[" << TP << "][" << TQ << "];\n";
     s << "#pragma unroll\n  for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n    for (int b = 0; b < " << TQ << "; ++b) acc[a][b] = Acc{0, 0, 0, 0};\n";
-    s << "  for (int sj = 0; sj < " << S << "; ++sj) {\n    const T* theirs = ar.part + ((blk * " << S << " + sj) * " << nreg << "LL) * 256 + tid;\n";
+    s << "  for (int sj = 0; sj < " << S << "; ++sj) {\n    const S* theirs = ar.part + ((blk * " << S << " + sj) * " << nreg << "LL) * 256 + tid;\n";
     s << "#pragma unroll\n    for (int a = 0; a < " << TP << "; ++a)\n#pragma unroll\n      for (int b = 0; b < " << TQ << "; ++b)\n#pragma unroll\n        for (int e = 0; e < 4; ++e)\n";
     s << "          acc[a][b][e] += theirs[((a * " << TQ << " + b) * 4 + e) * 256];\n  }\n";
   }
@@ -510,7 +514,7 @@ void choose_tile(hgpu_ctx* ctx, Spec& sp, int64_t ktot) {
   static const int cand[][4] = {{16, 64, 1, 4}, {64, 16, 4, 1}, {32, 32, 2, 2}, {32, 64, 2, 2}, {64, 32, 2, 2}, {16, 128, 1, 4},
                                 {64, 64, 2, 2}, {32, 128, 2, 2}, {128, 32, 2, 2}, {64, 128, 2, 2}, {128, 64, 2, 2}};
   const double es = sp.f64 ? 8 : 4;
-  const double cu_flops = (sp.f64 ? 78.6e12 : 157.3e12) / ctx->num_cu;
+  const double cu_flops = (sp.sums64() ? 78.6e12 : 157.3e12) / ctx->num_cu;
   const double cu_load = 150e9, latency = 1.0e-6;
   const int kc = (int)std::min<int64_t>(ktot, 64);
   double best = 1e300;
@@ -589,7 +593,7 @@ bool plan_chunks(Spec& sp) {
         k0 += c.kc;
       }
     }
-    sp.x_elems = (std::max(sp.x_elems, 1024) + 3) / 4 * 4;      // (the exchange of the quarters: 4 x 256 elements)
+    sp.x_elems = (std::max(sp.x_elems, sp.wide ? 2048 : 1024) + 3) / 4 * 4;      // (the exchange of the quarters: 4 x 256 sums)
     return true;
   }
   for (int t = 0; t < (int)sp.terms.size(); ++t) {
@@ -619,7 +623,7 @@ bool plan_chunks(Spec& sp) {
 static_assert(sizeof(Spec) == 232 && sizeof(Chunk) == 96 && sizeof(Term) == 56, "spec_key must cover every field of Spec, Chunk, Operand and Term");
 Key spec_key(const Spec& sp) {
   Key k;
-  k.put(sp.f64).put(sp.P).put(sp.Q).put(sp.BP).put(sp.BQ).put(sp.WP).put(sp.WQ).put(sp.terms.size());
+  k.put(sp.f64).put(sp.wide).put(sp.P).put(sp.Q).put(sp.BP).put(sp.BQ).put(sp.WP).put(sp.WQ).put(sp.terms.size());
   for (const Term& t : sp.terms) k.put(t.K).put(t.sxp).put(t.sxk).put(t.syq).put(t.syk);
   k.put(sp.chunks.size());
   for (const Chunk& c : sp.chunks) {
@@ -790,8 +794,8 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   // can be no chain (smallk_chain.hpp): here whatever the size, but for single products of fewer rows than
   // half a tile has, and of fewer than a tile's where K, too, is less than 32 (both paddings: three quarters of the tile's work).
   // Gradients in recorded graphs, us, with a million as the line for these too / without: dense 784-64-64-10 batch 32 fp32
-  // 83 / 56, batch 130 fp64 81 / 55; two recurrent layers of 12 steps, fp32, batch 64 width 32 571 / 104 and width 80
-  // 876 / 117, fp64 batch 300 width 50 393 / 139.
+  // 86 / 50, batch 130 fp64 81 / 55; two recurrent layers of 12 steps, fp32, batch 64 width 32 558 / 78 and width 80
+  // 867 / 103, fp64 batch 300 width 50 393 / 139.
   // (A readout of ten rows, K = 128, as a product and a pass 9 us, here 4.8.)
   const bool whatever_size = n_terms > 1 || (n_instr > 0 && (sp.Q >= 16 || (sp.Q >= 8 && ktot >= 32)));
   if (sp.P < 16 || sp.Q < 4 || (!whatever_size && (double)sp.P * sp.Q * ktot < 1.0e6)) return HGPU_OK;
@@ -799,6 +803,10 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     if (out_slots[o] < n_in && out_slots[o] != c_slot) return HGPU_OK;   // a copy of an input: not this kernel's business
     if (!outs[o]->buf) return HGPU_OK;
   }
+  // The kernels that small fp32 products come from (contract.hip) add in fp64, and so do these: fp32 sums of 28 to 128
+  // products are off by 0.4 units of 2^-24 of their magnitudes (root mean square), fp64 sums rounded once by 0.05 to 0.1.
+  // It costs little at this size (the gradients above with fp32 sums: 49, 77 and 91 us; 28 steps, batch 40, width 128 143, so 160).
+  sp.wide = !sp.f64 && (double)sp.P * sp.Q * ktot < 1.0e6;
   sp.n_in = n_in;
   sp.c_slot = c_slot;
   sp.n_instr = n_instr;
@@ -833,7 +841,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   }
 
   char kname[96];
-  snprintf(kname, sizeof kname, "smallk_%s_p%lld_q%lld_k%lld_t%d_in%d_instr%d_out%d", sp.f64 ? "f64" : "f32", (long long)sp.P, (long long)sp.Q, (long long)ktot, n_terms, n_in - 1,
+  snprintf(kname, sizeof kname, "smallk_%s_p%lld_q%lld_k%lld_t%d_in%d_instr%d_out%d", sp.f64 ? "f64" : sp.wide ? "f32s64" : "f32", (long long)sp.P, (long long)sp.Q, (long long)ktot, n_terms, n_in - 1,
            n_instr, n_out);
   Deferred d;
   hipFunction_t finish_fn = nullptr;
@@ -875,7 +883,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   const double es = sp.f64 ? 8 : 4;
   hgpu_buffer* part = nullptr;
   if (sp.splits > 1) {
-    int rc = buffer_alloc(ctx, sp.finishes() ? (size_t)nblk * (size_t)sp.BP * (size_t)sp.BQ * (size_t)es : (size_t)sp.splits * (size_t)sp.P * (size_t)sp.Q * (size_t)es, &part);
+    int rc = buffer_alloc(ctx, sp.finishes() ? (size_t)nblk * (size_t)sp.BP * (size_t)sp.BQ * (sp.sums64() ? 8 : 4) : (size_t)sp.splits * (size_t)sp.P * (size_t)sp.Q * (size_t)es, &part);
     if (rc) return rc;
   }
   for (int o = 0; o < n_out; ++o) d.args.push_back(part && !sp.finishes() ? part->ptr : data_ptr(outs[o]));
@@ -892,7 +900,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     for (auto& tm : sp.terms) ks += (ks.empty() ? "" : "+") + std::to_string(tm.K);
     char splits[24] = "";
     if (sp.splits > 1) snprintf(splits, sizeof splits, ",splits%d", sp.splits);
-    snprintf(buf, sizeof buf, "%s[M%lldxN%lldxK%sxB1,wholeK,t%dx%d,chunks%d%s,lds%dK,map(in%d,instr%d,out%d)]", d.label, (long long)sp.Q, (long long)sp.P, ks.c_str(), sp.BQ,
+    snprintf(buf, sizeof buf, "%s[M%lldxN%lldxK%sxB1,wholeK%s,t%dx%d,chunks%d%s,lds%dK,map(in%d,instr%d,out%d)]", d.label, (long long)sp.Q, (long long)sp.P, ks.c_str(), sp.wide ? ",sums64" : "", sp.BQ,
              sp.BP, (int)sp.chunks.size(), splits, (int)((sp.x_elems + sp.y_elems) * (int)es / 1024), n_in - 1, n_instr, n_out);
     d.label = intern_label(ctx, buf);
   }

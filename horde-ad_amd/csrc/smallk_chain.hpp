@@ -17,7 +17,8 @@
 //     from there to memory while the next level runs; operands from outside the chain are fetched a level ahead.
 //   * fp32: v_mfma_f32_4x4x1 with the columns as the A operand, one of four blocks of four lanes broadcast to its group
 //     (cbsz 2): 16 rows x 4 columns x 4 k an instruction, every group of 16 lanes a quarter of k; the quarters meet by
-//     two lane swaps.  fp64: v_mfma_f64_4x4x4 with the weights as the A operand.  Tiles of four columns cost the same
+//     two lane swaps.  fp64, and fp32 products whose sums are fp64 (smallk.hip): v_mfma_f64_4x4x4 with the weights as the A
+//     operand.  Tiles of four columns cost the same
 //     per product as the large ones (probe, 250 CUs, all operands resident: fp32 103 TFLOP/s with NC up to 3, 123 from
 //     4 on; fp64 59-64) and let 5000 columns be 250 blocks of 20.
 //
@@ -56,6 +57,7 @@ struct ChainItem {
   const Known* kn;
   int64_t Q;
   int rows, role = 0;
+  bool wide() const { return kn->spec.wide; }      // fp32 elements, sums in fp64
   std::vector<ChainX> x;
   std::vector<ChainIn> in;
   std::vector<ChainOut> out;
@@ -164,8 +166,8 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
         for (size_t i = 0; i < it.in.size(); ++i)
           if (it.in[i].kind == kind)
             for (int u = 0; u < mt.units; ++u) {
-              const std::string row = row_of(mt, u) + " + ql";
-              fn(it.in[i], row + " < " + str(it.Q) + " ? " + row + " : " + str(it.Q - 1), str((long long)j) + "_" + str((long long)i) + "_" + str(u));
+              const std::string row = row_of(mt, u) + (it.wide() ? " + qw" : " + ql");
+              fn(it, it.in[i], row + " < " + str(it.Q) + " ? " + row + " : " + str(it.Q - 1), str((long long)j) + "_" + str((long long)i) + "_" + str(u));
             }
       }
     };
@@ -188,14 +190,14 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       }
     };
     auto load_lanes = [&](const char* base, const char* pre) {
-      each_in(3, [&](const ChainIn& in, const std::string& row, const std::string& nm) {
+      each_in(3, [&](const ChainItem& it, const ChainIn& in, const std::string& row, const std::string& nm) {
         s << "    " << ctype(in.dtype) << " " << pre << nm << "[NC];\n    {\n      const " << ctype(in.dtype) << "* a = (const " << ctype(in.dtype) << "*)ar.p[" << base << " + " << in.ptr
           << "] + (i64)(" << row << ") * " << in.sq << "LL;\n";
-        s << "#pragma unroll\n      for (int cc = 0; cc < NC; ++cc) {\n        const i64 p = p0 + 4 * cc + pl;\n        " << pre << nm << "[cc] = a[(p < P ? p : P - 1) * " << in.sp << "LL];\n      }\n    }\n";
+        s << "#pragma unroll\n      for (int cc = 0; cc < NC; ++cc) {\n        const i64 p = p0 + 4 * cc + " << (it.wide() ? "pw" : "pl") << ";\n        " << pre << nm << "[cc] = a[(p < P ? p : P - 1) * " << in.sp << "LL];\n      }\n    }\n";
       });
     };
     auto landed_lanes = [&](const char* pre) {
-      each_in(3, [&](const ChainIn& in, const std::string&, const std::string& nm) {
+      each_in(3, [&](const ChainItem&, const ChainIn& in, const std::string&, const std::string& nm) {
         if (dtype_size(in.dtype) >= 4) s << "#pragma unroll\n    for (int cc = 0; cc < NC; ++cc) landed(" << pre << nm << "[cc]);\n";
       });
     };
@@ -212,7 +214,7 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
           s << "            *reinterpret_cast<V4*>(a + (i64)qq * P + p) = V4{v[0], v[1], v[2], v[3]};\n          }\n        }\n      }\n";
         }
     };
-    each_in(1, [&](const ChainIn& in, const std::string& row, const std::string& nm) {
+    each_in(1, [&](const ChainItem&, const ChainIn& in, const std::string& row, const std::string& nm) {
       s << "    const " << ctype(in.dtype) << " b" << nm << " = ((const " << ctype(in.dtype) << "*)ar.p[" << in.ptr << "])[(i64)(" << row << ") * " << in.sq << "LL];\n";
     });
     s << "    {\n";
@@ -241,15 +243,16 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       for (size_t j : js) {
         const ChainItem& it = sec.items[j];
         const std::string acc = "acc" + str((long long)j);
-        s << "        Acc " << acc << "[U][NC][NA];\n#pragma unroll\n        for (int u = 0; u < U; ++u)\n#pragma unroll\n          for (int cc = 0; cc < NC; ++cc)\n"
-             "#pragma unroll\n            for (int a = 0; a < NA; ++a) " << acc << "[u][cc][a] = " << (c.f64 ? "T(0)" : "Acc{0, 0, 0, 0}") << ";\n";
+        const bool d64 = c.f64 || it.wide();      // on the fp64 instruction
+        s << "        " << (it.wide() ? "double " : "Acc ") << acc << "[U][NC][NA];\n#pragma unroll\n        for (int u = 0; u < U; ++u)\n#pragma unroll\n          for (int cc = 0; cc < NC; ++cc)\n"
+             "#pragma unroll\n            for (int a = 0; a < NA; ++a) " << acc << "[u][cc][a] = " << (it.wide() ? "0.0" : c.f64 ? "T(0)" : "Acc{0, 0, 0, 0}") << ";\n";
         for (auto& x : it.x) {
           const ChainMat& mt = c.mats[(size_t)x.mat];
           if (x.kind == 2) s << "        {\n          const T xv = *(const T*)ar.p[at + " << x.ptr << "];\n";
-          else s << "        {\n          const T* xb = " << (x.kind == 1 ? "prv" : "cur") << " + " << x.off << (c.f64 ? " + g * 8 + (lane & 3)" : " + lane") << ";\n";
+          else s << "        {\n          const T* xb = " << (x.kind == 1 ? "prv" : "cur") << " + " << x.off << (it.wide() ? " + g * 16 + (lane & 3)" : c.f64 ? " + g * 8 + (lane & 3)" : " + lane") << ";\n";
           // fragment of the columns (tile t, for fp64 of its half e)
-          const std::string frag = x.kind != 2 ? "xb[cc * " + str(x.rows * 4 + 4) + (c.f64 ? " + 32 * t + 4 * e]" : " + 64 * t]")
-                                               : std::string(c.f64 ? "8 * t + 2 * g + e" : "16 * t + (lane >> 2)") + " < " + str(x.K) + " ? xv : T(0)";
+          const std::string frag = x.kind != 2 ? "xb[cc * " + str(x.rows * 4 + 4) + (it.wide() ? " + 64 * t + 4 * e]" : c.f64 ? " + 32 * t + 4 * e]" : " + 64 * t]")
+                                               : std::string(it.wide() ? "16 * t + 4 * g + e" : c.f64 ? "8 * t + 2 * g + e" : "16 * t + (lane >> 2)") + " < " + str(x.K) + " ? xv : T(0)";
           int in_regs[kChainMaxUnits];
           std::vector<int> cuts{0, mt.nf / VK};
           for (int u = 0; u < U; ++u) {
@@ -262,16 +265,16 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
           for (size_t q = 0; q + 1 < cuts.size(); ++q) {
             if (cuts[q] == cuts[q + 1]) continue;
             s << "#pragma unroll\n          for (int t = " << cuts[q] << "; t < " << cuts[q + 1] << "; ++t) {\n";
-            if (!c.f64) s << "            T a[NC];\n#pragma unroll\n            for (int cc = 0; cc < NC; ++cc) a[cc] = " << frag << ";\n";
-            else s << "            T a[VK][NC];\n#pragma unroll\n            for (int e = 0; e < VK; ++e)\n#pragma unroll\n              for (int cc = 0; cc < NC; ++cc) a[e][cc] = " << frag << ";\n";
+            if (!d64) s << "            T a[NC];\n#pragma unroll\n            for (int cc = 0; cc < NC; ++cc) a[cc] = " << frag << ";\n";
+            else s << "            " << (it.wide() ? "double" : "T") << " a[VK][NC];\n#pragma unroll\n            for (int e = 0; e < VK; ++e)\n#pragma unroll\n              for (int cc = 0; cc < NC; ++cc) a[e][cc] = " << frag << ";\n";
             for (int e = 0; e < VK; ++e)
               for (int u = 0; u < U; ++u) {
                 s << "            { const T wv = ";
                 if (cuts[q] < in_regs[u] / VK) s << (mt.kept() ? "w" + str(x.mat) + "_" + str(u) : "ws" + str(u)) << "[" << VK << " * t + " << e << "];\n";
                 else s << "lds[" << mt.lds[u] - 64 * mt.w0 << " + tid + (" << VK << " * t + " << e - in_regs[u] << ") * " << 64 * mt.waves(u) << "];\n";
                 s << "#pragma unroll\n              for (int cc = 0; cc < NC; ++cc) " << acc << "[" << u << "][cc][" << e % NA << "] = ";
-                if (!c.f64) s << "mm<" << e << ">(a[cc], wv, " << acc << "[" << u << "][cc][" << e % NA << "]); }\n";
-                else s << "__builtin_amdgcn_mfma_f64_4x4x4f64(wv, a[" << e << "][cc], " << acc << "[" << u << "][cc][" << e % NA << "], 0, 0, 0); }\n";
+                if (!d64) s << "mm<" << e << ">(a[cc], wv, " << acc << "[" << u << "][cc][" << e % NA << "]); }\n";
+                else s << "__builtin_amdgcn_mfma_f64_4x4x4f64((double)wv, a[" << e << "][cc], " << acc << "[" << u << "][cc][" << e % NA << "], 0, 0, 0); }\n";
               }
             s << "          }\n";
           }
@@ -285,14 +288,14 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
         const ChainMat& m0 = c.mats[(size_t)it.x[0].mat];
         for (int u = 0; u < U; ++u) {
           const std::string sfx = "_" + str((long long)j) + "_" + str(u), acc = "acc" + str((long long)j) + "[" + str(u) + "][cc]";
-          s << "          const int q" << sfx << " = " << row_of(m0, u) << " + ql;\n#pragma unroll\n          for (int a = 1; a < NA; ++a) " << acc << "[0] += " << acc << "[a];\n";
+          s << "          const int q" << sfx << " = " << row_of(m0, u) << (it.wide() ? " + qw" : " + ql") << ";\n#pragma unroll\n          for (int a = 1; a < NA; ++a) " << acc << "[0] += " << acc << "[a];\n";
           for (size_t i = 0; i < it.in.size(); ++i) {
             const ChainIn& in = it.in[i];
             s << "          const " << ctype(in.dtype) << " v" << i << sfx << " = ";
-            if (in.kind == 0) s << (c.f64 ? acc + "[0]" : "meet(" + acc + "[0])") << ";\n";
+            if (in.kind == 0) s << (it.wide() ? "(T)" + acc + "[0]" : c.f64 ? acc + "[0]" : "meet(" + acc + "[0])") << ";\n";
             else if (in.kind == 1) s << "b" << j << "_" << i << "_" << u << ";\n";
             else if (in.kind == 3) s << "e" << j << "_" << i << "_" << u << "[cc];\n";
-            else s << (in.kind == 2 ? "prv[" : "cur[") << in.off << " + cc * " << it.rows * 4 + 4 << " + q" << sfx << " * 4 + pl];\n";
+            else s << (in.kind == 2 ? "prv[" : "cur[") << in.off << " + cc * " << it.rows * 4 + 4 << " + q" << sfx << " * 4 + " << (it.wide() ? "pw" : "pl") << "];\n";
           }
           emit_program(s, sp.n_in, sp.n_instr, sp.prog, sp.dt, "          ", sfx);
         }
@@ -303,11 +306,11 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
           const std::string sfx = "_" + str((long long)j) + "_" + str(u);
           bool direct = false;
           for (auto& o : it.out) {
-            if (o.staged) s << "          cur[" << o.off << " + cc * " << it.rows * 4 + 4 << " + q" << sfx << " * 4 + pl] = q" << sfx << " < " << it.Q << " ? v" << o.slot << sfx << " : T(0);\n";
+            if (o.staged) s << "          cur[" << o.off << " + cc * " << it.rows * 4 + 4 << " + q" << sfx << " * 4 + " << (it.wide() ? "pw" : "pl") << "] = q" << sfx << " < " << it.Q << " ? v" << o.slot << sfx << " : T(0);\n";
             else direct = true;
           }
           if (!direct) continue;
-          s << "          {\n            const i64 p = p0 + 4 * cc + pl;\n            if (q" << sfx << " < " << it.Q << " && p < P) {\n";
+          s << "          {\n            const i64 p = p0 + 4 * cc + " << (it.wide() ? "pw" : "pl") << ";\n            if (q" << sfx << " < " << it.Q << " && p < P) {\n";
           for (auto& o : it.out)
             if (!o.staged) s << "              ((" << ctype(o.dtype) << "*)ar.p[at + " << o.ptr << "])[(i64)q" << sfx << " * P + p] = v" << o.slot << sfx << ";\n";
           s << "            }\n          }\n";
@@ -337,7 +340,7 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
     landed_lanes("f");
     s << "      if (more) {\n";
     put_staged("prv", "y");
-    each_in(3, [&](const ChainIn&, const std::string&, const std::string& nm) { s << "#pragma unroll\n        for (int cc = 0; cc < NC; ++cc) e" << nm << "[cc] = f" << nm << "[cc];\n"; });
+    each_in(3, [&](const ChainItem&, const ChainIn&, const std::string&, const std::string& nm) { s << "#pragma unroll\n        for (int cc = 0; cc < NC; ++cc) e" << nm << "[cc] = f" << nm << "[cc];\n"; });
     s << "      }\n      __syncthreads();\n      at += " << sec.n_ptr << ";\n      T* const z = cur;\n      cur = prv;\n      prv = z;\n    }\n";
     write_out("at - " + str(sec.n_ptr));
     s << "  }\n";
@@ -389,7 +392,7 @@ std::string chain_source(const ChainPlan& c, const std::string& kname) {
   s << "  __shared__ __attribute__((aligned(16))) T lds[" << c.lds_elems << "];\n";
   s << "  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, w = __builtin_amdgcn_readfirstlane(tid >> 6);\n";
   if (c.f64) s << "  const int ql = 4 * ((lane >> 2) & 3) + g, pl = lane & 3;      // row and column of this lane's result\n";
-  else s << "  const int ql = lane & 15, pl = g;\n";
+  else s << "  const int ql = lane & 15, pl = g, qw = 4 * ((lane >> 2) & 3) + g, pw = lane & 3;      // (w: where sums are fp64)\n";
   // consecutive blocks go round the eight XCDs: neighbouring columns, whose lines of memory overlap, belong to one XCD
   const int64_t nblk = chain_blocks(c), per_xcd = (nblk + 7) / 8;
   s << "  const int blk = (int)(blockIdx.x % 8) * " << per_xcd << " + (int)(blockIdx.x / 8);\n  if (blk >= " << nblk << ") return;\n";
@@ -556,7 +559,7 @@ bool place_weights(ChainPlan& c, int slack) {
     int most = 0;
     const int movers = role == c.roles - 1 ? 64 * (c.roles > 1 ? 8 - role_end(c, role - 1) : 8) : 0;
     for (auto& s : c.sections) {
-      int ahead = 0, mine = 0, consts = 0;
+      int ahead = 0, mine = 0, consts = 0, wide = 0;
       for (auto& it : s.items) {
         for (auto& x : it.x)
           if (x.kind == 0 && movers) ahead += (x.rows * c.NC + movers - 1) / movers * 4;
@@ -564,14 +567,15 @@ bool place_weights(ChainPlan& c, int slack) {
           if (in.kind == 4 && movers) ahead += (it.rows * c.NC + movers - 1) / movers * 4;
         if (it.role != role) continue;
         const int units = c.mats[(size_t)it.x[0].mat].units;
-        mine += units * c.NC * (c.f64 ? 1 : 4);
+        mine += units * c.NC * (c.f64 ? 1 : it.wide() ? 2 : 4);
+        if (it.wide()) wide = 44 + 8 * c.NC;      // (an fp64 program's overhead, columns as doubles)
         for (auto& in : it.in) {
           if (in.kind == 3) ahead += 2 * c.NC * units;
           if (in.kind == 1) consts += units;
         }
       }
       // (with many accumulators the compiler keeps about as many other values)
-      most = std::max(most, ahead + mine + consts + 2 * c.NC + (c.f64 ? 0 : 2 * std::max(0, mine - 40)));
+      most = std::max(most, ahead + mine + consts + wide + 2 * c.NC + (c.f64 ? 0 : 2 * std::max(0, mine - 40)));
     }
     int regs = std::max(0, (256 - regs_per * most - (c.f64 ? 84 : 40) - slack) / regs_per / vk * vk);
     for (int u = 0; u < kChainMaxUnits; ++u)
@@ -597,14 +601,17 @@ bool pays(const ChainPlan& c, int num_cu) {
   const double rounds = (double)((chain_blocks(c) + num_cu - 1) / num_cu);
   double chain = 0, levels = 0;
   for (auto& s : c.sections) {
-    double mul = 0, flops = 0;
-    for (auto& it : s.items)
+    double mul = 0, flops = 0, after = 0.9e-6;      // mul, flops: seconds
+    for (auto& it : s.items) {
+      const bool d64 = c.f64 || it.wide();
+      if (d64) after = 1.2e-6;
       for (auto& x : it.x) {
-        mul += (double)it.rows * x.rows * 4 * c.NC;
-        flops += 2.0 * (double)it.Q * (double)x.K * (double)c.P;
+        mul += (double)it.rows * x.rows * 4 * c.NC / (d64 ? 122e9 : 246e9);
+        flops += 2.0 * (double)it.Q * (double)x.K * (double)c.P / (d64 ? 33e12 : 49e12);
       }
-    chain += s.n_levels * rounds * (mul / (c.f64 ? 122e9 : 246e9) * 1.15 + (c.f64 ? 1.2e-6 : 0.9e-6));
-    levels += s.n_levels * std::max(4.7e-6, flops / (c.f64 ? 33e12 : 49e12));
+    }
+    chain += s.n_levels * rounds * (mul * 1.15 + after);
+    levels += s.n_levels * std::max(4.7e-6, flops);
   }
   return chain + 5e-6 * rounds < levels;
 }
