@@ -739,6 +739,8 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   }
   std::vector<int> dt;
   if (int rc = check_program(ctx, n_in, in, n_instr, prog, &dt)) return rc;
+  const int asked = slot;
+  if (slot >= 0) slot &= ~HGPU_SUM_PRODUCTS;
   if (slot < 0 || slot >= n_in + n_instr) return fail(ctx, HGPU_ERR_INVALID, "fused_sum: bad slot");
   const int odt = dt[(size_t)slot];
   if (odt == HGPU_BOOL) return fail(ctx, HGPU_ERR_INVALID, "fused_sum: Bool values have no sum");
@@ -816,7 +818,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
       s << ";\n";
     }
     emit_program(s, n_in, n_instr, prog, dt, "      ", suf);
-    s << "      acc += (ACC)v" << slot << suf << ";\n    }\n";
+    s << "      acc += (ACC)" << summand(n_in, prog, dt, asked, suf) << ";\n    }\n";
   }
   s << "  }\n";
   s << "  const i64 t = nv * " << vec << " + (i64)blockIdx.x * " << NT << " + threadIdx.x;\n";
@@ -827,7 +829,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
     s << ";\n";
   }
   emit_program(s, n_in, n_instr, prog, dt, "    ", "_t");
-  s << "    acc += (ACC)v" << slot << "_t;\n  }\n";
+  s << "    acc += (ACC)" << summand(n_in, prog, dt, asked, "_t") << ";\n  }\n";
   s << "  acc = wave_sum(acc);\n";
   s << "  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n";
   s << "  __syncthreads();\n";
@@ -902,6 +904,11 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
   if (int rc = check_program(ctx, n_in, in, n_instr, prog, &dt)) return rc;
   for (int o = 0; o < n_out; ++o)
     if (out_slots[o] < 0 || out_slots[o] >= n_in + n_instr) return fail(ctx, HGPU_ERR_INVALID, "fused_map_sums: bad output slot");
+  const int* const asked = sum_slots;
+  std::vector<int> plain(sum_slots, sum_slots + n_sum);
+  for (int& v : plain)
+    if (v >= 0) v &= ~HGPU_SUM_PRODUCTS;
+  sum_slots = plain.data();
   for (int j = 0; j < n_sum; ++j) {
     if (sum_slots[j] < 0 || sum_slots[j] >= n_in + n_instr) return fail(ctx, HGPU_ERR_INVALID, "fused_map_sums: bad sum slot");
     if (dt[(size_t)sum_slots[j]] == HGPU_BOOL) return fail(ctx, HGPU_ERR_INVALID, "fused_map_sums: Bool values have no sum");
@@ -953,7 +960,7 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
   Key key;
   key.put(std::string("fused_map_sums")).put(n_out).put(n_sum);
   for (int o = 0; o < n_out; ++o) key.put(out_slots[o]);
-  for (int j = 0; j < n_sum; ++j) key.put(sum_slots[j]);
+  for (int j = 0; j < n_sum; ++j) key.put(asked[j]);
   put_inputs(key, n_in, in, n_instr, prog);
   const Known* hit = find_known(ctx, key);
   Src s(!hit || check_keys());
@@ -994,7 +1001,7 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     }
     emit_program(s, n_in, n_instr, prog, dt, "      ", suf);
     for (int o = 0; o < n_out; ++o) s << "      r" << o << ".v[" << e << "] = v" << out_slots[o] << suf << ";\n";
-    for (int j = 0; j < n_sum; ++j) s << "      acc" << j << " += (" << acc_t(j) << ")v" << sum_slots[j] << suf << ";\n";
+    for (int j = 0; j < n_sum; ++j) s << "      acc" << j << " += (" << acc_t(j) << ")" << summand(n_in, prog, dt, asked[j], suf) << ";\n";
     s << "    }\n";
   }
   for (int o = 0; o < n_out; ++o) s << "    reinterpret_cast<Vec<" << ctype(res[(size_t)o]->dtype) << ", " << vec << ">*>(o" << o << ")[i] = r" << o << ";\n";
@@ -1008,7 +1015,7 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
   }
   emit_program(s, n_in, n_instr, prog, dt, "    ", "_t");
   for (int o = 0; o < n_out; ++o) s << "    o" << o << "[t] = v" << out_slots[o] << "_t;\n";
-  for (int j = 0; j < n_sum; ++j) s << "    acc" << j << " += (" << acc_t(j) << ")v" << sum_slots[j] << "_t;\n";
+  for (int j = 0; j < n_sum; ++j) s << "    acc" << j << " += (" << acc_t(j) << ")" << summand(n_in, prog, dt, asked[j], "_t") << ";\n";
   s << "  }\n";
   for (int j = 0; j < n_sum; ++j) {
     s << "  acc" << j << " = wave_sum(acc" << j << ");\n";

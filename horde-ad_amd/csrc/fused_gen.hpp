@@ -220,6 +220,15 @@ inline void emit_program(Src& s, int n_in, int n_instr, const hgpu_fused_instr* 
   }
 }
 
+// What a sum adds for one element of a slot (see HGPU_SUM_PRODUCTS): its value, or the product of its two factors before
+// it is rounded.
+inline std::string summand(int n_in, const hgpu_fused_instr* prog, const std::vector<int>& dt, int slot, const std::string& lane_suffix) {
+  auto v = [&](int s) { return "v" + std::to_string(s) + lane_suffix; };
+  const bool products = slot & HGPU_SUM_PRODUCTS;
+  slot &= ~HGPU_SUM_PRODUCTS;
+  if (!products || slot < n_in || dt[(size_t)slot] != HGPU_F32 || prog[slot - n_in].kind != HGPU_FUSED_OP2 || prog[slot - n_in].op != HGPU_MUL) return v(slot);
+  return "((double)" + v(prog[slot - n_in].a) + " * (double)" + v(prog[slot - n_in].b) + ")";
+}
 
 }  // namespace fusedgen
 }  // namespace hg

@@ -243,6 +243,7 @@ struct ArrHolder {
   // expressions of the same shape out (an objective's value in the pass of its
   // gradient), or by a pass of its own when somebody needs it first.
   std::shared_ptr<ArrHolder> ssrc;
+  bool sdot = false;   // ... of the product of its two factors, added before it is rounded (a dot product)
   // A stand-in without data that view operations are tried on to learn the
   // strides they produce (vmeta holds its shape and strides).
   bool probe = false;

@@ -750,6 +750,8 @@ static void run_program(Backend* be, const std::vector<ArrHolder*>& all_roots) {
       std::vector<int> slots;
       number_program(all, &ins, &prog, &slots);
       std::vector<int> sum_slots(slots.begin() + (long)roots.size(), slots.end());
+      for (size_t j = 0; j < sums.size(); ++j)
+        if (sums[j]->sdot) sum_slots[j] |= HGPU_SUM_PRODUCTS;
       std::vector<hgpu_array*> souts(sums.size(), nullptr);
       int rc = api->fused_map_sums(be->ctx, (int)ins.size(), ins.data(), (int)prog.size(), prog.data(), (int)roots.size(), slots.data(), outs.data(),
                                    (int)sums.size(), sum_slots.data(), souts.data());
@@ -936,10 +938,14 @@ void ArrHolder::force() {
       number_program({e.holder().get()}, &ins, &prog, &slots);
       if ((int)ins.size() <= 12 && (int)prog.size() <= 96) {
         hgpu_array* o = nullptr;
-        int rc = api->fused_sum(be->ctx, (int)ins.size(), ins.data(), (int)prog.size(), prog.data(), slots[0], &o);
+        int rc = api->fused_sum(be->ctx, (int)ins.size(), ins.data(), (int)prog.size(), prog.data(), slots[0] | (sdot ? HGPU_SUM_PRODUCTS : 0), &o);
         if (rc == HGPU_OK) r = T(be, o);
         else if (rc != HGPU_ERR_UNSUPPORTED) be->check(rc);
       }
+    }
+    if (!r.valid() && sdot && e.pending_expr()) {
+      const T a(e.holder()->fa), b(e.holder()->fb);
+      r = contract_now(a, &b, 0);
     }
     if (!r.valid()) r = contract_now(e, nullptr, 0);
     be->check(be->api->retain(r.h()));
@@ -1526,6 +1532,7 @@ T contract(const T& a, const T* b, int n_keep) {
       Backend* be = a.be();
       auto p = new_holder(be, nullptr);
       p->ssrc = make_expr(HGPU_FUSED_OP2, HGPU_MUL, a.dtype(), a, b, nullptr).holder();
+      p->sdot = true;
       auto& ps = be->pending_sums;
       ps.erase(std::remove_if(ps.begin(), ps.end(), [](const std::weak_ptr<ArrHolder>& w) { auto q = w.lock(); return !q || q->h || !q->ssrc; }), ps.end());
       ps.push_back(p);

@@ -267,7 +267,12 @@ int hgpu_fused_map_dimsum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
 /* tssum0 of such a program's result (OpsConcrete.hs:229-230), evaluated on the
  * fly: the result itself is never written.  Inputs must be dense or one
  * broadcast element (else HGPU_ERR_UNSUPPORTED: write the result out and sum
- * that).  Accumulates in double / int64 in an order fixed by the size. */
+ * that).  Accumulates in double / int64 in an order fixed by the size.
+ * A sum slot of this call or of hgpu_fused_map_sums that is an fp32 product may
+ * carry HGPU_SUM_PRODUCTS (slot | HGPU_SUM_PRODUCTS): the products are then added
+ * before they are rounded, as hgpu_contract of the two factors adds them
+ * (tsdot0, OpsConcrete.hs:231).  On any other slot it says nothing. */
+enum { HGPU_SUM_PRODUCTS = 1 << 16 };
 int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, int slot, hgpu_array** out);
 /* The first extremum of such a program's result along its trailing n_reduce
  * dims (taken together, row-major), evaluated on the fly: the result itself is

@@ -796,6 +796,18 @@ int horc_fused_extremum(hgpu_ctx* c, int n_in, const hgpu_array* const* in, int 
 }
 
 int horc_fused_sum(hgpu_ctx* c, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, int slot, hgpu_array** out) {
+  const bool products = slot >= 0 && (slot & HGPU_SUM_PRODUCTS);
+  if (products) slot &= ~HGPU_SUM_PRODUCTS;
+  if (products && slot >= n_in && slot < n_in + n_instr && prog[slot - n_in].kind == HGPU_FUSED_OP2 && prog[slot - n_in].op == HGPU_MUL) {   // the contraction of the two factors
+    const int factors[2] = {prog[slot - n_in].a, prog[slot - n_in].b};
+    hgpu_array* f[2] = {nullptr, nullptr};
+    int rc = horc_fused_map(c, n_in, in, n_instr, prog, 2, factors, f);
+    if (rc) return rc;
+    rc = horc_contract(c, f[0], f[1], 0, out);
+    horc_release(f[0]);
+    horc_release(f[1]);
+    return rc;
+  }
   hgpu_array* r = nullptr;
   int rc = horc_fused_map(c, n_in, in, n_instr, prog, 1, &slot, &r);
   if (rc) return rc;

@@ -289,3 +289,22 @@ def test_programs_over_a_few_elements(host, dt):
             [v.numpy() for v in program()]
     finally:
         graph.free()
+
+
+@pytest.mark.parametrize("n", [64, 65, 1000, 2500, 4095, 4096, 100003])
+@pytest.mark.parametrize("with_pass", [False, True])
+def test_dot_products_of_expressions_round_once(host, n, with_pass):
+    """fp32: neighbouring products cancel but for what rounding them to fp32 would leave; summed alone, and in the pass that writes
+    another expression of this shape."""
+    rng = np.random.default_rng(n)
+    x, y = (rng.uniform(0.5, 1, n).astype(np.float32) for _ in range(2))
+    y[1::2] = -(x[0:n - 1:2] * y[0:n - 1:2] / x[1::2])
+    y[n // 2 * 2:] = 0
+    a, b = host.concrete(x), host.concrete(y)
+
+    e = -a
+    s = e.sdot0(b)
+    if with_pass:
+        assert np.array_equal((e * b).numpy(), -x * y)
+    p = x.astype(np.float64) * y
+    assert abs(float(s.numpy()) + p.sum()) <= 2.0 ** -24 * abs(p.sum()) + n * 2.0 ** -52 * np.abs(p).sum()

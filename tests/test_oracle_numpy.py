@@ -341,6 +341,13 @@ def test_fused_table_definitions(oracle):
     o = C.c_void_p()
     assert fs(oracle.h, 1, ins, 1, flat, 1, C.byref(o)) == 0
     assert abs(capi.Array(oracle, o).numpy() - (-x).sum()) <= 1e-12
+    # ... and of a product's factors, before it is rounded
+    p, q = np.array([3.0, -1.0, 2.0], np.float32) / np.float32(7), np.array([1 / 3, 1.0, 5.0], np.float32)
+    up, uq = oracle.upload(p), oracle.upload(q)
+    pq = (C.c_void_p * 2)(up.h, uq.h)
+    mul = (C.c_int32 * 6)(1, O2["mul"], 0, 0, 1, 0)
+    assert fs(oracle.h, 2, pq, 1, mul, 2 | 1 << 16, C.byref(o)) == 0
+    assert float(capi.Array(oracle, o).numpy()) == np.float32((p.astype(np.float64) * q).sum())
     # fused_map_dimsum: the program's results, and one slot summed over every dim but one
     fd = dll.horc_fused_map_dimsum
     fd.restype, fd.argtypes = I, [P, I, PP, I, P, I, C.POINTER(C.c_int), PP, I, I, PP]
