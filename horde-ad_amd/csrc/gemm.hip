@@ -536,8 +536,9 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
   }
   // Weight gradients of narrow layers, fp32: 8 to 32 rows or columns under a long K, bound by the loads of the long side, which
   // a tile of 128 x 32 reads once.  us with the sums, tiles of the fp32 instruction / so: 128 x 28 over 28 x 5000 34.9 / 25.7,
-  // 50 x 28 over 20 x 1000 9.4 / 8.4, 2048 x 10 over 8192 26.1 / 21.4, 784 x 32 over 8192 24.5 / 16.6; error against fp64 0.4 to 0.6 of
-  // what it was.  Fewer columns leave the tile empty (784 x 4 over 8 x 10000 61 / 83); with rows further apart than 65536
+  // 50 x 28 over 20 x 1000 9.4 / 8.4, 2048 x 10 over 8192 26.1 / 21.4, 784 x 32 over 8192 24.5 / 16.6 (with six part products a tile;
+  // with all eight, as now, 2 to 3 % more); error against fp64 0.4 to 0.6 of what it was, a sum of one product that product rounded,
+  // as there.  Fewer columns leave the tile empty (784 x 4 over 8 x 10000 61 / 83); with rows further apart than 65536
   // elements the wider tiles read longer pieces (1000 x 20 over 50000 57.6 / 54.0, over 100,000 101 / 104).
   const int64_t k_all = p.K * (n_terms > 0 ? n_terms : 1);
   const bool thin = a->dtype == HGPU_F32 && std::min(p.M, p.N) >= 8 && std::min(p.M, p.N) <= 32 && std::max(p.M, p.N) > 32 && p.K >= 64 && p.K <= 65536 && k_all >= 4096;

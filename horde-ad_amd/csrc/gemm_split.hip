@@ -17,8 +17,8 @@
 //     uniform in 0 .. 1         0.67  (3.8)    0.84  (4.7)    0.66  (3.5)
 //     e^-uniform(0, 100)        0.24  (2.2)    0.27  (2.1)    0.29  (2.1)
 //     one product, no others    0.366 (1.7)    0.361 (1.0)    0.457 (2.4)
-// With all eight terms the last row is 0.361 (1.0) too, and every product takes a fifth longer (464 -> 557 us below):
-// left at six.
+// With m l' and l m' as well the last row is 0.361 (1.0) too, and a product on tiles of 128 x 128 takes a fifth longer
+// (464 -> 557 us below): left at six there.  The thin tiles form all eight.
 //
 // Range.  Operands are multiplied by 2^23 on their way into the split (the first remainder is one fma, so it costs one
 // multiplication an element), the sums by 2^-46 on their way out: the smallest fp32 number, 2^-149, is then 2^-126, and no
@@ -160,8 +160,9 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
 }
 
 // THIN: tiles of 128 x 32 for products with at most 32 columns (weight gradients of narrow layers), bound by the loads of A:
-// a step is 10 KB of loads and six instructions a wavefront, one step ahead, so four blocks (114 to 124 registers, 30 KB of
-// LDS) hide one another's trips to memory.  128 x 28 over 28 x 5000, 87 MB: 23.7 us = 3.7 TB/s, the 32 x 32 tiles of the fp32
+// a step is 10 KB of loads and eight instructions a wavefront, one step ahead, so four blocks (114 to 128 registers, 30 KB of
+// LDS) hide one another's trips to memory (with six instructions the same products take 2 to 3 % less: 128 x 28 over 28 x 5000
+// with its sums 26.0 for 26.6 us, 784 x 32 over 8192 13.4 for 13.8).  128 x 28 over 28 x 5000, 87 MB: 23.7 us = 3.7 TB/s, the 32 x 32 tiles of the fp32
 // instruction, which read A for every 32 rows of it and B four times, 33.0.
 // ROWS: the lanes also add up, in fp64, the elements of A they stage: a bias gradient is the row sums of what the weight
 // gradient multiplies.  Blocks of the first column of tiles do, for products that ask (split_job).  Reading A once more for
@@ -258,6 +259,10 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
         for (int r = 0; r < 16; ++r) zero[r] = 0;
         auto add = [&](int qa, int qb, const f16v& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[qb], c, 0, 0, 0); };
         const f16v c = add(0, 0, zero);
+        if constexpr (THIN) {
+          low[i][j] = add(2, 1, low[i][j]);
+          low[i][j] = add(1, 2, low[i][j]);
+        }
         low[i][j] = add(2, 0, low[i][j]);
         low[i][j] = add(0, 2, low[i][j]);
         low[i][j] = add(1, 1, low[i][j]);

@@ -78,3 +78,17 @@ def test_infinities_nans_and_large_elements(gpu):
 @pytest.mark.parametrize("lay", ["KK", "RK"])
 def test_products_of_a_recording(lay):
     held.test_products_of_a_recording_go_out_together(held.pkg.hostapi.Host(), np.float32, [(130, 28, 5000), (130, 32, 5000), (128, 128, 30000), (500, 17, 9001)], lay)
+
+
+@pytest.mark.parametrize("lay", ["KK", "RR"])
+@pytest.mark.parametrize("m,n,k", [(300, 28, 4100), (9, 700, 4100)])
+def test_one_dominating_product(gpu, m, n, k, lay):
+    """A sum that is one product is that product rounded: the parts of both factors are multiplied with one another but for the last with
+    the last (2^-34 of the product), and the small ones, 2^-7 of it, lose less than 2^-23 of themselves in each of seven additions."""
+    rng = np.random.default_rng(m)
+    x, y = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    x[:, 7], y[:, 7] = rng.uniform(1, 2, m), rng.uniform(1, 2, n)
+    out, taken, labels = sum_of(gpu, [x], [y], lay)
+    assert taken, labels
+    want = x.astype(np.float64) @ y.astype(np.float64).T
+    assert np.max(np.abs(out - want) / want) <= (1 + 7 * 2.0 ** -6 + 2.0 ** -9) * 2.0 ** -24
