@@ -308,3 +308,22 @@ def test_dot_products_of_expressions_round_once(host, n, with_pass):
         assert np.array_equal((e * b).numpy(), -x * y)
     p = x.astype(np.float64) * y
     assert abs(float(s.numpy()) + p.sum()) <= 2.0 ** -24 * abs(p.sum()) + n * 2.0 ** -52 * np.abs(p).sum()
+
+
+@pytest.mark.parametrize("terms", [9, 15, 23, 31])
+def test_partial_results_are_added_in_short_chains(gpu, terms):
+    """One partial result of 1 and others of a quarter of its last place: of eight chains the one that has the 1 loses the others of its
+    own, and the chains meet in three roundings."""
+    m, k = 300, 64
+    pairs = []
+    for t in range(terms):
+        x, y = np.zeros((m, k), np.float32), np.zeros((m, k), np.float32)
+        x[:, t], y[:, t] = 1 if t == 0 else 2.0 ** -25, 1
+        pairs.append((gpu.upload(x).replicate([m]).transpose([1, 0, 2]), gpu.upload(y).replicate([m])))
+    gpu.profile(2)
+    got = gpu.contract_sum(pairs, 2).numpy().astype(np.float64)
+    labels = list(gpu.profile_report())
+    gpu.profile(0)
+    assert any("s%d," % terms in s for s in labels) and "gemm_sum_partials" in labels, labels
+    want = 1 + (terms - 1) * 2.0 ** -25
+    assert np.all(np.abs(got - want) <= (terms - 1) // 8 * 2.0 ** -25 + 3 * 2.0 ** -24), np.unique((got - want) * 2 ** 24)
