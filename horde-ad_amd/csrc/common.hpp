@@ -15,6 +15,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "hordead_gpu.h"
@@ -45,6 +46,7 @@ struct hgpu_buffer {
   enum { kUnknown = 0, kIotaI64 = 1, kZeroScalar = 2 };
   int known = kUnknown;
   bool known_relied_on = false;
+  int held = 0;      // how often launches that are held back read or write it (guarded by the context's launch_mu)
 };
 
 struct hgpu_array {
@@ -73,6 +75,17 @@ void drop_deferred(hgpu_ctx* ctx);            // flush, then free the queue
 void forget_remembered_sums(hgpu_ctx* ctx);   // results kept for a later call, and the arrays held for them (footprint.hip)
 }  // namespace hg
 
+// A mutex that knows whether the calling thread has it: what is held back may have to go out for an allocation, which some
+// callers make under it and most do not.
+class LaunchMutex {
+  std::mutex m_;
+  std::atomic<std::thread::id> owner_{std::thread::id()};
+ public:
+  void lock() { m_.lock(); owner_.store(std::this_thread::get_id(), std::memory_order_relaxed); }
+  void unlock() { owner_.store(std::thread::id(), std::memory_order_relaxed); m_.unlock(); }
+  bool mine() const { return owner_.load(std::memory_order_relaxed) == std::this_thread::get_id(); }
+};
+
 struct hgpu_ctx {
   int device;
   hipStream_t stream;
@@ -83,7 +96,7 @@ struct hgpu_ctx {
   std::string err;
   void* staging = nullptr;       // pinned host staging block
   size_t staging_bytes = 0;
-  std::mutex launch_mu;          // serialises enqueue order across host threads
+  LaunchMutex launch_mu;         // serialises enqueue order across host threads
   uint64_t write_epoch = 0;      // counts the writes into existing arrays (hgpu_overwrite, hgpu_assign): results remembered for given inputs end with it
   int num_cu = 256;
   // JIT cache of fused elementwise kernels, keyed by generated source.
@@ -133,7 +146,7 @@ inline bool dtype_is_int(int dt) { return dt >= HGPU_I64 && dt <= HGPU_I8; }
 int fail(hgpu_ctx* ctx, int code, const char* fmt, ...);
 int check_hip(hgpu_ctx* ctx, hipError_t e, const char* what);
 
-// Allocator (runtime.hip).
+// Allocator (runtime.hip).  A request that the device cannot serve sends out what is held back, whose memory then comes back.
 int buffer_alloc(hgpu_ctx* ctx, size_t bytes, hgpu_buffer** out);
 int zero_block(hgpu_ctx* ctx, const void** out);   // a context-lifetime block of 256 zero bytes
 // Context-lifetime counters (1024 of 32 bits, zero between launches) for kernels whose blocks draw tickets: the

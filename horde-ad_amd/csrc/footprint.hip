@@ -2045,7 +2045,7 @@ void remember_sum(hgpu_ctx* ctx, const VirtualOp& v, const std::vector<int>& kep
   MemoSum m{expression_key(v, kept), sum, {}, 0};
   for (int i = 0; i < v.n_in; ++i)
     if (v.in[i]->buf) { buffer_retain(v.in[i]->buf); m.held.push_back(v.in[i]->buf); }
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   m.epoch = ctx->write_epoch;
   MemoSums& ms = memo_of(ctx);
   for (size_t i = 0; i < ms.items.size();)
@@ -2057,7 +2057,7 @@ void remember_sum(hgpu_ctx* ctx, const VirtualOp& v, const std::vector<int>& kep
 // The remembered sum (a new reference), or nullptr.
 hgpu_array* recall_sum(hgpu_ctx* ctx, const VirtualOp& v, const std::vector<int>& kept) {
   const std::string key = expression_key(v, kept);
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   MemoSums& ms = memo_of(ctx);
   for (auto& m : ms.items)
     if (m.epoch == ctx->write_epoch && m.key == key) { hgpu_retain(m.sum); return m.sum; }
@@ -2667,7 +2667,7 @@ bool classify_contraction(int rank, const int64_t* shape, const int64_t* st_a, c
 void forget_remembered_sums(hgpu_ctx* ctx) {
   std::vector<MemoSum> gone;
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     gone.swap(memo_of(ctx).items);
   }
   for (auto& m : gone) forget(m);

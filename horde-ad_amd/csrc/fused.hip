@@ -59,7 +59,7 @@ int compile(hgpu_ctx* ctx, const std::string& src, Compiled* out, const char* kn
 // Kernels found again by what their text depends on (the inputs' layouts and the program).
 struct Known { Compiled c; std::string text; };
 const Known* find_known(hgpu_ctx* ctx, const Key& key) {
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   auto kit = ctx->jit_cache.find("__fused_known__");
   if (kit == ctx->jit_cache.end()) return nullptr;
   auto& known = *static_cast<std::unordered_map<std::string, Known>*>(kit->second);
@@ -470,7 +470,7 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     for (int i = 0; i < n_in; ++i) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(in[i])); if (in[i]->buf) reads.push_back(in[i]->buf); }
     for (int o = 0; o < n_out; ++o) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(res[(size_t)o])); writes.push_back(res[(size_t)o]->buf); }
     {
-      std::lock_guard<std::mutex> lk(ctx->launch_mu);
+      std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
       (void)hipSetDevice(ctx->device);
       Compiled kernel;
       if (int rc = kernel_for(ctx, key, hit, src, kernel_name, &kernel)) { release_all(); return rc; }

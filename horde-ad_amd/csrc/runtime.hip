@@ -59,41 +59,62 @@ static void drop_cache_locked(hgpu_ctx* ctx) {
 // last element of an array without leaving the block.
 constexpr size_t kSlack = 16;
 
+// A block of *blk bytes from the cache or the device (the allocator's mutex is held).  At the last try what the cache holds
+// is given up for it: freed, or, where a recording's launches may use those blocks again, handed out larger than asked (*blk).
+static int take_block(hgpu_ctx* ctx, size_t* blk, bool last_try, void** out) {
+  std::multimap<size_t, void*>& cache = ctx->cap ? ctx->cap->cache : ctx->cache;
+  auto from_cache = [&](std::multimap<size_t, void*>::iterator it) {
+    *blk = it->first;
+    *out = it->second;
+    cache.erase(it);
+    ctx->in_use += *blk;
+    return HGPU_OK;
+  };
+  auto it = cache.find(*blk);
+  if (it != cache.end()) return from_cache(it);
+  const bool injected = ctx->fail_after >= 0 && (int64_t)ctx->n_device_allocs >= ctx->fail_after;
+  (void)hipSetDevice(ctx->device);
+  hipError_t e = injected ? hipErrorOutOfMemory : hipMalloc(out, *blk);
+  if (e != hipSuccess && last_try) {
+    if (!injected) (void)hipGetLastError();
+    if (ctx->cap) {
+      it = cache.lower_bound(*blk);
+      if (it != cache.end()) return from_cache(it);
+    } else if (!injected) {
+      // Cached blocks may still be read by enqueued kernels: drain first.
+      (void)hipStreamSynchronize(ctx->stream);
+      drop_cache_locked(ctx);
+      e = hipMalloc(out, *blk);
+    }
+  }
+  if (e != hipSuccess) {
+    if (!injected) (void)hipGetLastError();
+    char msg[160];
+    snprintf(msg, sizeof msg, "device allocation of %zu bytes failed%s%s", *blk, injected ? " (injected)" : ": ", injected ? "" : hipGetErrorString(e));
+    ctx->err = msg;
+    return HGPU_ERR_OOM;
+  }
+  ctx->reserved += *blk;
+  ctx->n_device_allocs++;
+  ctx->in_use += *blk;
+  return HGPU_OK;
+}
+
 int buffer_alloc(hgpu_ctx* ctx, size_t bytes, hgpu_buffer** out) {
   size_t blk = round_block(bytes + kSlack);
   void* p = nullptr;
+  int rc;
   {
     std::lock_guard<std::mutex> g(ctx->mu);
-    std::multimap<size_t, void*>& cache = ctx->cap ? ctx->cap->cache : ctx->cache;
-    auto it = cache.find(blk);
-    if (it != cache.end()) {
-      p = it->second;
-      cache.erase(it);
-    } else {
-      if (ctx->fail_after >= 0 && (int64_t)ctx->n_device_allocs >= ctx->fail_after) {
-        ctx->err = "device allocation failed (injected)";
-        return HGPU_ERR_OOM;
-      }
-      (void)hipSetDevice(ctx->device);
-      hipError_t e = hipMalloc(&p, blk);
-      if (e != hipSuccess && !ctx->cap) {
-        (void)hipGetLastError();
-        // Cached blocks may still be read by enqueued kernels: drain first.
-        (void)hipStreamSynchronize(ctx->stream);
-        drop_cache_locked(ctx);
-        e = hipMalloc(&p, blk);
-      }
-      if (e != hipSuccess) {
-        (void)hipGetLastError();
-        char msg[160];
-        snprintf(msg, sizeof msg, "device allocation of %zu bytes failed: %s", blk, hipGetErrorString(e));
-        ctx->err = msg;
-        return HGPU_ERR_OOM;
-      }
-      ctx->reserved += blk;
-      ctx->n_device_allocs++;
-    }
-    ctx->in_use += blk;
+    rc = take_block(ctx, &blk, false, &p);
+  }
+  if (rc) {
+    // Launches that are held back keep their blocks: out they go.  (Not under the allocator's mutex, which they give them back by.)
+    if (ctx->launch_mu.mine()) flush_deferred_locked(ctx);
+    else flush_deferred(ctx);
+    std::lock_guard<std::mutex> g(ctx->mu);
+    rc = take_block(ctx, &blk, true, &p);
+    if (rc) return rc;
   }
   hgpu_buffer* b = new hgpu_buffer;
   b->ctx = ctx;
@@ -394,7 +415,7 @@ int hgpu_capture_end(hgpu_ctx* ctx, hgpu_graph** out) {
   flush_deferred(ctx);          // launches still held back belong to the graph
   int held_rc;
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     held_rc = take_deferred_rc(ctx);
   }
   hgpu_cap_pool* pool;
@@ -423,7 +444,7 @@ int hgpu_graph_launch(hgpu_graph* gr) {
   if (!gr) return HGPU_ERR_INVALID;
   hgpu_ctx* ctx = gr->ctx;
   if (ctx->cap) return fail(ctx, HGPU_ERR_INVALID, "graph_launch: not inside a capture");
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   (void)hipSetDevice(ctx->device);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
   if (int rc = take_deferred_rc(ctx)) return rc;
@@ -469,7 +490,7 @@ int hgpu_sync(hgpu_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   flush_deferred(ctx);
   int rc = check_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   if (int held_rc = take_deferred_rc(ctx)) rc = held_rc;      // a launch that was held back failed after its call had returned
   return rc;
 }
@@ -515,7 +536,7 @@ int hgpu_inject_alloc_failure(hgpu_ctx* ctx, int64_t limit) {
 
 int hgpu_profile_enable(hgpu_ctx* ctx, int on) {
   if (!ctx) return HGPU_ERR_INVALID;
-  std::lock_guard<std::mutex> g(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> g(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
   if (!ctx->cap) (void)hipStreamSynchronize(ctx->stream);
   for (auto& r : ctx->prof)
@@ -528,7 +549,7 @@ int hgpu_profile_enable(hgpu_ctx* ctx, int on) {
 
 int hgpu_profile_report(hgpu_ctx* ctx, char* buf, size_t n) {
   if (!ctx || !buf || n == 0) return HGPU_ERR_INVALID;
-  std::lock_guard<std::mutex> g(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> g(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
   if (!ctx->cap) (void)hipStreamSynchronize(ctx->stream);
   struct Agg { long count = 0; double ms = 0, bytes = 0, flops = 0; };
@@ -610,7 +631,7 @@ int hgpu_assign(hgpu_ctx* ctx, hgpu_array* dst, const hgpu_array* src) {
   if (dst->buf->known_relied_on) return fail(ctx, HGPU_ERR_INVALID, "assign: a kernel has been chosen for the destination's contents (an index vector or a zero constant)");
   dst->buf->known = hgpu_buffer::kUnknown;
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     ctx->write_epoch++;
   }
   // Dense copies wait for the ones that follow (a step hands back all its parameters and moments, one call

@@ -710,6 +710,11 @@ hipFunction_t compiled_kernel(hgpu_ctx* ctx, const std::vector<const std::string
 }
 
 constexpr size_t kMaxHeld = 256;          // launches held back at most
+// ... and the memory they keep from being used again, blocks of all they read and write: where nobody asks for them, the
+// weight gradients of a recording would keep every layer's cotangent, and sums submitted one by one whole blocks of which
+// they read a part.  (Gradients: two recurrent layers over 28 steps at batch 5000 hold
+// 0.45 GB, the wide dense network 0.4, the others under 0.1.)
+constexpr size_t kMaxHeldBytes = (size_t)4 << 30;
 constexpr size_t kMaxGroup = 4;           // problems in one kernel at most
 constexpr int64_t kGroupBlocksPerCu = 4;  // a problem with more blocks than this per CU fills the device alone
 
@@ -751,6 +756,15 @@ struct DeferredQueue {
   std::vector<Deferred> maps;
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
+  size_t held_bytes = 0;             // of the blocks that items and maps keep
+  void keep(hgpu_buffer* b) {
+    buffer_retain(b);
+    if (b->held++ == 0) held_bytes += b->bytes;
+  }
+  void let_go(hgpu_buffer* b) {
+    if (--b->held == 0) held_bytes -= b->bytes;
+    buffer_release(b);
+  }
 };
 }  // namespace hg
 
@@ -852,7 +866,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   d.grid = (unsigned)grid;
   d.lds_bytes = (sp.x_elems + sp.y_elems) * (sp.f64 ? 8 : 4);
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);   // the kernel caches are shared with the thread that launches what is held back
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);   // the kernel caches are shared with the thread that launches what is held back
     auto& known = known_of(ctx).problems;
     const Key key = spec_key(sp);
     auto it = known.find(key.bytes);
@@ -911,7 +925,7 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
     for (int i = 0; i < n_in; ++i)
       if (i != c_slot) d.reads.push_back(in[i]->buf);
     for (int o = 0; o < n_out; ++o) d.writes.push_back(outs[o]->buf);
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     hold_item_locked(ctx, std::move(d));
     *handled = true;
     return HGPU_OK;
@@ -974,10 +988,10 @@ static void launch_maps(hgpu_ctx* ctx, std::vector<Deferred>& items) {
   }
 }
 
-static void release_held(std::vector<Deferred>& items) {
+static void release_held(DeferredQueue& q, std::vector<Deferred>& items) {
   for (auto& d : items) {
-    for (auto* b : d.reads) buffer_release(b);
-    for (auto* b : d.writes) buffer_release(b);
+    for (auto* b : d.reads) q.let_go(b);
+    for (auto* b : d.writes) q.let_go(b);
   }
 }
 
@@ -990,7 +1004,7 @@ static void release_held(std::vector<Deferred>& items) {
 static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, DeferredQueue::Kind kind) {
   if (items.empty()) return;
   (void)hipSetDevice(ctx->device);
-  auto release_items = [&] { release_held(items); };
+  auto release_items = [&] { release_held(*ctx->dq, items); };
   if (kind == DeferredQueue::kCopies) {
     std::vector<const CopyJob*> jobs;
     double bytes = 0;
@@ -1246,7 +1260,7 @@ static void flush_maps_locked(hgpu_ctx* ctx) {
   if (maps.empty()) return;
   (void)hipSetDevice(ctx->device);
   launch_maps(ctx, maps);
-  release_held(maps);
+  release_held(*ctx->dq, maps);
 }
 
 static void flush_items_locked(hgpu_ctx* ctx) {
@@ -1277,10 +1291,10 @@ static std::set<const hgpu_buffer*> written_by(const std::vector<Deferred>& item
 
 // A product or reduction joins the queue (which retains its buffers).
 static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
-  for (auto* b : d.reads) buffer_retain(b);
-  for (auto* b : d.writes) buffer_retain(b);
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
+  for (auto* b : d.reads) q.keep(b);
+  for (auto* b : d.writes) q.keep(b);
   if (q.items.size() >= kMaxHeld || q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
   if (!q.maps.empty()) {
     std::vector<const void*> reads;
@@ -1289,6 +1303,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
   }
   q.items.push_back(std::move(d));
   ctx->dq_pending = true;
+  if (q.held_bytes > kMaxHeldBytes) flush_deferred_locked(ctx);
 }
 
 // Only large products, reductions and sums of partial results wait beyond the launch that asks: they are the ends of a reverse pass's
@@ -1333,7 +1348,7 @@ bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads,
     if (reads[i]) d.reads.push_back(reads[i]);
   d.writes.push_back(write);
   if (write2) d.writes.push_back(write2);
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   hold_item_locked(ctx, std::move(d));
   return true;
 }
@@ -1347,15 +1362,15 @@ void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const ch
   d.flops = flops;
   d.reads = reads;
   d.writes.push_back(write);
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   hold_item_locked(ctx, std::move(d));
 }
 
 bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares) {
-  // (memory is taken with the queue unlocked: the allocator may want it)
+  // (memory is taken with the queue unlocked: for want of it the allocator sends the queue out)
   std::shared_ptr<WideJob> job;
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     if (!ctx->dq) return false;
     if (factor && (!written_by(ctx->dq->items, {factor}).empty() || !written_by(ctx->dq->maps, {factor}).empty())) return false;
     for (auto& d : ctx->dq->items)
@@ -1363,13 +1378,13 @@ bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int6
   }
   if (!job || buffer_alloc(ctx, (size_t)M * (size_t)*shares * 8, part)) return false;
   {
-    std::lock_guard<std::mutex> lk(ctx->launch_mu);
+    std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     for (auto& d : ctx->dq->items) {
       if (d.wide != job) continue;
       wide_take_rows(*job, (*part)->ptr, factor);
       d.writes.push_back(*part);
-      buffer_retain(*part);
-      if (factor_buf) { d.reads.push_back(factor_buf); buffer_retain(factor_buf); }
+      ctx->dq->keep(*part);
+      if (factor_buf) { d.reads.push_back(factor_buf); ctx->dq->keep(factor_buf); }
       return true;
     }
   }
@@ -1393,9 +1408,10 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
   d.map = std::move(job);
   d.reads = reads;
   d.writes = writes;
-  for (auto* b : d.reads) buffer_retain(b);
-  for (auto* b : d.writes) buffer_retain(b);
+  for (auto* b : d.reads) q.keep(b);
+  for (auto* b : d.writes) q.keep(b);
   ctx->dq_pending = true;
+  if (q.held_bytes > kMaxHeldBytes) flush_deferred_locked(ctx);
 }
 
 // A copy into an existing array joins the queue.  It waits only for copies: anything else that is enqueued goes
@@ -1407,11 +1423,11 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   d.bytes = 2.0 * (double)job.bytes;
   d.reads.push_back(src);
   d.writes.push_back(dst);
-  buffer_retain(src);
-  buffer_retain(dst);
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
+  q.keep(src);
+  q.keep(dst);
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
   bool fits = q.maps.empty() && (q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs));
   for (size_t i = 0; fits && i < q.items.size(); ++i) {
@@ -1426,13 +1442,13 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
 }
 
 void flush_deferred(hgpu_ctx* ctx) {
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
 }
 
 // Launches what is held back and gives the queue's own memory back (hgpu_shutdown).
 void drop_deferred(hgpu_ctx* ctx) {
-  std::lock_guard<std::mutex> lk(ctx->launch_mu);
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
   delete ctx->dq;
   ctx->dq = nullptr;

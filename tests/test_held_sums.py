@@ -327,3 +327,64 @@ def test_partial_results_are_added_in_short_chains(gpu, terms):
     assert any("s%d," % terms in s for s in labels) and "gemm_sum_partials" in labels, labels
     want = 1 + (terms - 1) * 2.0 ** -25
     assert np.all(np.abs(got - want) <= (terms - 1) // 8 * 2.0 ** -25 + 3 * 2.0 ** -24), np.unique((got - want) * 2 ** 24)
+
+
+def test_memory_of_held_work_comes_back_for_an_allocation(gpu):
+    """Sums that wait keep the arrays they read, which nobody else has any more: a request that the device cannot serve sends them out."""
+    x = gpu.upload(np.ones((200, 100003), np.float32))
+    big = x.ewise1("neg")                                  # (blocks of this size exist, and none is left)
+    try:
+        gpu.check(gpu.lib.inject_alloc_failure(gpu.h, 1))      # for the sums
+        s = big.slice(0, 0, 100).slice(1, 0, 4096).contract(None, 1)
+        del big                                            # only the held sum has it now
+        y = x.ewise1("neg")
+    finally:
+        gpu.check(gpu.lib.inject_alloc_failure(gpu.h, -1))
+    assert np.array_equal(s.numpy(), np.full(100, -4096, np.float32)) and y.numpy()[0, 0] == -1
+
+
+def test_held_work_keeps_a_bounded_amount_of_memory(gpu):
+    """Sums of small parts of large arrays that are released at once."""
+    fresh = pkg.capi.Lib().context(0)
+    n = 1 << 27                                            # 512 MB
+    x = fresh.upload(np.zeros(1, np.float32)).replicate([n]).reshape([n])
+    before = fresh.mem_stats()[1]
+    sums = []
+    for _ in range(24):
+        big = x.ewise1("cos")
+        sums.append(big.slice(0, 0, 100 * 4096).reshape([100, 4096]).contract(None, 1))
+        del big
+    assert fresh.mem_stats()[1] - before <= 6 << 30
+    for s in sums:
+        assert np.array_equal(s.numpy(), np.full(100, 4096, np.float32))
+    del x, sums, s
+    fresh.shutdown()
+
+
+def test_a_recording_takes_the_memory_it_has(gpu):
+    """Inside a recording blocks cannot be freed: held work goes out, and a larger block serves where none of the size is left."""
+    ctx = pkg.capi.Lib().context(0)
+    dll = ctx.lib.dll
+    x = np.random.default_rng(1).uniform(-1, 1, (300, 20000)).astype(np.float32)
+    ctx.check(ctx.lib.inject_alloc_failure(ctx.h, 4))      # for the two arrays here, and the first two below
+    a, large = ctx.upload(x), ctx.upload(np.zeros(200 << 20, np.int8))
+    ctx.sync()
+    del large
+    ctx.check(dll.hgpu_capture_begin(ctx.h))
+    try:
+        neg = a.ewise1("neg")
+        s = neg.slice(1, 0, 4096).contract(None, 1)        # waits
+        del neg
+        y = a.ewise1("abs")                                # the block of neg, which the sum had
+        z = a.ewise1("neg")                                # the large one
+    finally:
+        g = C.c_void_p()
+        ctx.check(dll.hgpu_capture_end(ctx.h, C.byref(g)))
+    ctx.check(ctx.lib.inject_alloc_failure(ctx.h, -1))
+    for _ in range(2):
+        ctx.check(dll.hgpu_graph_launch(g))
+        ctx.sync()
+        want = -x[:, :4096].astype(np.float64).sum(1)
+        assert np.array_equal(y.numpy(), np.abs(x)) and np.array_equal(z.numpy(), -x)
+        assert np.all(np.abs(s.numpy() - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -40)
+    ctx.check(dll.hgpu_graph_destroy(g))
