@@ -1380,7 +1380,7 @@ bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int6
   {
     std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
     for (auto& d : ctx->dq->items) {
-      if (d.wide != job) continue;
+      if (d.wide != job || wide_takes_rows(*job)) continue;      // (another thread's sum was faster)
       wide_take_rows(*job, (*part)->ptr, factor);
       d.writes.push_back(*part);
       ctx->dq->keep(*part);

@@ -1,4 +1,7 @@
 """Sums of the rows that a waiting fp32 product multiplies come from that product's blocks (csrc/gemm_split.hip) in a recording."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -150,3 +153,35 @@ def test_factor_of_a_row_sum(host, m, n, k, f):
         want, size = terms.sum(1), np.abs(terms).sum(1)
         big = np.where(np.abs(want) >= 2.0 ** 128, np.sign(want) * np.inf, want)
     check(host, program, [big], [size], k, 1)
+
+
+def test_two_threads_ask_for_the_same_rows():
+    """One of the sums joins the product, the other is a launch of its own."""
+    ctx = held.pkg.capi.Lib().context(0)
+    m, n, k = 256, 64, 20000
+    rng = np.random.default_rng(5)
+    x, y = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(0, 1, (n, k)).astype(np.float32)
+    a, b = ctx.upload(x), ctx.upload(y)
+    w, size = x.astype(np.float64).sum(1), np.abs(x).sum(1, dtype=np.float64)
+    for _ in range(12):
+        sums, start = [None] * 2, threading.Barrier(2)
+
+        def ask(i):
+            start.wait()
+            sums[i] = a.contract(None, 1)
+
+        g = C.c_void_p()
+        ctx.check(ctx.lib.dll.hgpu_capture_begin(ctx.h))
+        try:
+            p = a.replicate([n]).transpose([1, 0, 2]).contract(b.replicate([m]), 2)
+            threads = [threading.Thread(target=ask, args=(i,)) for i in range(2)]
+            [t.start() for t in threads]
+            [t.join() for t in threads]
+        finally:
+            ctx.check(ctx.lib.dll.hgpu_capture_end(ctx.h, C.byref(g)))
+        ctx.check(ctx.lib.dll.hgpu_graph_launch(g))
+        ctx.sync()
+        for s in sums:
+            assert np.all(np.abs(s.numpy() - w) <= (2.0 ** -24 + k * 2.0 ** -53) * size)
+        del p, sums, s
+        ctx.check(ctx.lib.dll.hgpu_graph_destroy(g))
