@@ -252,8 +252,8 @@ bool wide_takes_rows(const WideJob& job);
 bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
 // smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it
 void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
-// contract.hip: a program over a few elements (its last instruction's result is `out`), to be launched with held sums; false: left to the caller
-bool hold_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out);
+// contract.hip: a program over a few elements (its last instruction's result is `out`), in a recording launched with held sums; false: left to the caller
+bool try_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out);
 // contract.hip: *acc += x, taking over x (the first term becomes the accumulator); the addition is held back where it can share a launch
 int add_into(hgpu_ctx* ctx, hgpu_array** acc, hgpu_array* x);
 // smallk.hip: holds the launch back (retaining the buffers it reads and writes); false: the caller launches it now

@@ -443,7 +443,7 @@ __device__ __forceinline__ void pair_body(const SumArgs& g, unsigned bid, unsign
   for (int64_t i = nv * V + at; i < g.n; i += step) o[i] = a[i] + b[i];
 }
 
-// See hold_tiny_map.
+// See try_tiny_map.
 template <typename T>
 __device__ __forceinline__ void tiny_body(const SumArgs& g) {
 #pragma clang fp contract(off)
@@ -1137,8 +1137,9 @@ int scratch_of(hgpu_ctx* ctx, void** out) {
 namespace hg {
 // A program over a few elements that an objective ends with (`negate sum * c`) joins the launch of a gradient's last sums: a
 // pass of its own is 4 us in a graph.  One or two operands, up to four negations, additions, subtractions and
-// multiplications: 12 bits each, in the order of the program, and above them which operands move.
-bool hold_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out) {
+// multiplications: 12 bits each, in the order of the program, and above them which operands move.  Submitted one by one it
+// goes out at once, by the same kernel: the host is about to ask for an objective's value, and what waits starts when it does.
+bool try_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_instr, const hgpu_fused_instr* prog, const hgpu_array* out) {
   const int64_t n = nelem(out);
   if (n_in < 1 || n_in > 2 || n_instr < 1 || n_instr > 4 || !dtype_is_float(out->dtype) || n < 1 || n > 64 || !out->buf) return false;
   uint64_t code = 0;
@@ -1176,7 +1177,12 @@ bool hold_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_i
   j.a = data_ptr(in[0]);
   j.b = n_in > 1 ? data_ptr(in[1]) : j.a;
   j.out = data_ptr(out);
-  return hold_reduction(ctx, j, reads, n_in, out->buf);
+  if (ctx->cap) return hold_reduction(ctx, j, reads, n_in, out->buf);
+  const std::vector<const void*> from{j.a, j.b};
+  LaunchGuard lg(ctx, j.label, j.bytes, j.flops, &from);
+  if (j.dtype == HGPU_F64) launch_sum<double>(ctx, j);
+  else launch_sum<float>(ctx, j);
+  return hipGetLastError() == hipSuccess;
 }
 
 // *acc += x, taking over x (the first term becomes the accumulator).

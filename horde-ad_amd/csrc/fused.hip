@@ -128,6 +128,12 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     return HGPU_OK;
   }
 
+  // (asked before any text is written: a kernel that is never compiled is never found again)
+  if (sum_slot < 0 && n_out == 1 && out_slots[0] == n_in + n_instr - 1 && n <= 64 && try_tiny_map(ctx, n_in, in, n_instr, prog, res[0])) {
+    outs[0] = res[0];
+    return HGPU_OK;
+  }
+
   // the sum over all dims but keep_dim: blocks take (element of keep_dim, chunk of the rest)
   int64_t dsO = 1, dsC = 1, dsI = 1;
   if (sum_slot >= 0) {
@@ -460,10 +466,6 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
   // 182 -> 167 us).  From a million elements on a pass is worth a launch of its own.  Submitted one by one the host is
   // what takes the time, and holding a pass costs it more than a launch's gap gives back (24 x 24 CNN: 642 -> 651 us).
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
-  if (sum_slot < 0 && n_out == 1 && out_slots[0] == n_in + n_instr - 1 && n <= 64 && hold_tiny_map(ctx, n_in, in, n_instr, prog, res[0])) {
-    outs[0] = res[0];
-    return HGPU_OK;
-  }
   if (hold && ctx->cap && all_simple && n <= (1 << 20)) {
     std::vector<hgpu_buffer*> reads, writes;
     MapJob j{nullptr, nullptr, grid_for((n + vec - 1) / vec, 256, ctx->num_cu * 16), {(uint64_t)n}, label, bytes, (double)n * n_instr};

@@ -388,3 +388,36 @@ def test_a_recording_takes_the_memory_it_has(gpu):
         assert np.array_equal(y.numpy(), np.abs(x)) and np.array_equal(z.numpy(), -x)
         assert np.all(np.abs(s.numpy() - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -40)
     ctx.check(dll.hgpu_graph_destroy(g))
+
+
+def test_the_end_of_an_objective_waits_in_recordings_only(host, gpu):
+    """`negate sum * c` joins the last sums of a recording; submitted one by one it is a launch of its own, which goes out at once."""
+    prog = [(0, pkg.capi.OP1["neg"], 0, 0, 0, 0), (1, pkg.capi.OP2["mul"], 0, 2, 1, 0)]
+    ins = [gpu.upload(np.asarray(v, np.float32)) for v in (3.0, 0.5)]
+    x = gpu.upload(np.ones((100, 5000), np.float32))
+    gpu.profile(2)
+    s = x.contract(None, 1)                                # waits
+    got = [gpu.fused_map(ins, prog, [3])[0] for _ in range(2)]
+    labels = gpu.profile_report()
+    gpu.profile(0)
+    assert labels["tiny_map"][0] == 2 and not any("|" in k for k in labels), labels
+    assert [float(v.numpy()) for v in got] == [-1.5, -1.5] and np.array_equal(s.numpy(), np.full(100, 5000, np.float32))
+    x = host.concrete(np.random.default_rng(1).uniform(-1, 1, (100, 5000)).astype(np.float32))
+    c = host.concrete(np.asarray(0.25, np.float32))
+
+    def program():
+        s = x.ssum0()
+        force(host, s)
+        return [-s * c, x.stranspose([1, 0]).ssum()]
+
+    eager = [v.numpy() for v in program()]
+    graph, res, labels = recorded(host, program)
+    try:
+        assert any("tiny_map" in k for k in labels), labels
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            assert all(np.array_equal(r.numpy(), e) for r, e in zip(res, eager))
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
