@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -66,11 +67,32 @@ struct hgpu_array {
 };
 
 namespace hg {
+// The addresses of what a launch reads: a few of them, in place (every launch has such a list).
+class Reads {
+  const void* few_[20];
+  std::vector<const void*> many_;
+  size_t n_ = 0;
+ public:
+  Reads() {}
+  Reads(std::initializer_list<const void*> l) { add(l.begin(), l.end()); }
+  explicit Reads(const std::vector<const void*>& v) { add(v.begin(), v.end()); }
+  void push_back(const void* p) {
+    if (n_ < sizeof few_ / sizeof few_[0]) few_[n_] = p;
+    else {
+      if (many_.empty()) many_.assign(few_, few_ + n_);
+      many_.push_back(p);
+    }
+    ++n_;
+  }
+  template <typename I> void add(I from, I to) { for (; from != to; ++from) push_back(*from); }
+  const void* const* begin() const { return many_.empty() ? few_ : many_.data(); }
+  const void* const* end() const { return begin() + n_; }
+};
 struct DeferredQueue;                         // launches held back to be grouped (smallk.hip)
 void flush_deferred_locked(hgpu_ctx* ctx);    // the caller holds launch_mu
 void flush_deferred(hgpu_ctx* ctx);
 // Before a launch that reads the blocks of `reads` and writes new arrays only: launches what it needs of the held-back work (the caller holds launch_mu).
-void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads);
+void make_way_locked(hgpu_ctx* ctx, const Reads& reads);
 void drop_deferred(hgpu_ctx* ctx);            // flush, then free the queue
 void forget_remembered_sums(hgpu_ctx* ctx);   // results kept for a later call, and the arrays held for them (footprint.hip)
 }  // namespace hg
@@ -304,7 +326,7 @@ int copy_view(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const vo
 struct LaunchGuard {
   hgpu_ctx* ctx;
   bool timed = false;
-  explicit LaunchGuard(hgpu_ctx* c, const char* name = nullptr, double bytes = 0, double flops = 0, const std::vector<const void*>* reads = nullptr) : ctx(c) {
+  explicit LaunchGuard(hgpu_ctx* c, const char* name = nullptr, double bytes = 0, double flops = 0, const Reads* reads = nullptr) : ctx(c) {
     c->launch_mu.lock();
     (void)hipSetDevice(c->device);
     if (c->dq_pending && reads) make_way_locked(c, *reads);
@@ -339,8 +361,8 @@ struct LaunchGuard {
 };
 
 // What launches over these arrays read (see LaunchGuard).
-inline std::vector<const void*> reads_of(int n, const hgpu_array* const* in) {
-  std::vector<const void*> r;
+inline Reads reads_of(int n, const hgpu_array* const* in) {
+  Reads r;
   for (int i = 0; i < n; ++i) r.push_back(data_ptr(in[i]));
   return r;
 }

@@ -833,10 +833,10 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     hgpu_buffer* reads[2] = {hold->a, hold->b};
     if (hold_reduction(ctx, j, reads, hold->b ? 2 : 1, hold->out)) return HGPU_OK;
   }
-  std::vector<const void*> reads{a, b};
+  Reads reads{a, b};
   if (tp.n) {
-    reads.insert(reads.end(), tp.a, tp.a + tp.n);
-    reads.insert(reads.end(), tp.b, tp.b + tp.n);
+    reads.add(tp.a, tp.a + tp.n);
+    reads.add(tp.b, tp.b + tp.n);
   }
   LaunchGuard lg(ctx, label, bytes, flops, fresh ? &reads : nullptr);
   if (use_wave && S == 0) {       // one block per output, no partials
@@ -922,7 +922,7 @@ static int queue_sum(hgpu_ctx* ctx, RedJob& j, hgpu_buffer* part, const hgpu_arr
   // (Submitted one by one, an objective's value goes out at once: the device would come to it only when the host asks.)
   if (out1->buf && (!out2 || out2->buf) && (double)part->bytes <= kMaxHeldPartials && (ctx->cap || j.n_out >= 16) &&
       hold_reduction(ctx, j, &part, 1, out1->buf, out2 ? out2->buf : nullptr)) return HGPU_OK;
-  const std::vector<const void*> reads{j.a};
+  const Reads reads{j.a};
   LaunchGuard ls(ctx, j.label, j.bytes, j.flops, &reads);
   if (j.dtype == HGPU_F64) launch_sum<double>(ctx, j);
   else launch_sum<float>(ctx, j);
@@ -1178,7 +1178,7 @@ bool try_tiny_map(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, int n_in
   j.b = n_in > 1 ? data_ptr(in[1]) : j.a;
   j.out = data_ptr(out);
   if (ctx->cap) return hold_reduction(ctx, j, reads, n_in, out->buf);
-  const std::vector<const void*> from{j.a, j.b};
+  const Reads from{j.a, j.b};
   LaunchGuard lg(ctx, j.label, j.bytes, j.flops, &from);
   if (j.dtype == HGPU_F64) launch_sum<double>(ctx, j);
   else launch_sum<float>(ctx, j);
@@ -1482,7 +1482,7 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
     if (pieces) rc = ticket_block(ctx, &tickets);
     if (pieces && !rc) rc = buffer_alloc(ctx, (size_t)(n_out * pieces_of(L)) * 16, &scratch);
     if (rc) { hgpu_release(o); if (v) hgpu_release(v); return rc; }
-    const std::vector<const void*> reads = reads_of(1, &a);
+    const Reads reads = reads_of(1, &a);
     LaunchGuard lg(ctx, "argminmax", (double)n_out * (L * dtype_size(a->dtype) + 8 + (v ? dtype_size(a->dtype) : 0)), (double)n_out * L, &reads);
     void* vp = v ? data_ptr(v) : nullptr;
     if (pieces) {

@@ -452,7 +452,7 @@ int hgpu_pad(hgpu_ctx* ctx, const hgpu_array* a, const int64_t* lo, const int64_
       snprintf(buf + w, sizeof buf - w, "]");
       label = intern_label(ctx, buf);
     }
-    const std::vector<const void*> reads = reads_of(1, &a);
+    const Reads reads = reads_of(1, &a);
     LaunchGuard lg(ctx, label, (double)(n + nelem(a)) * dtype_size(a->dtype), 0, &reads);
     const void* src = data_ptr(a);
     void* dst = data_ptr(o);
@@ -562,7 +562,7 @@ int hgpu_ewise1(hgpu_ctx* ctx, int op, const hgpu_array* a, hgpu_array** out) {
   if (rc) return rc;
   int64_t n = nelem(o);
   if (n > 0) {
-    const std::vector<const void*> reads = reads_of(1, &a);
+    const Reads reads = reads_of(1, &a);
     LaunchGuard lg(ctx, "ewise1", 2.0 * n * dtype_size(a->dtype), (double)n, &reads);
     if (layout_class(a) == 1 && aligned16(data_ptr(a))) {
       unsigned g = grid_for(n, kBlock * 4, max_blocks(ctx));
@@ -602,7 +602,7 @@ int hgpu_ewise2(hgpu_ctx* ctx, int op, const hgpu_array* a, const hgpu_array* b,
   if (rc) return rc;
   int64_t n = nelem(o);
   if (n > 0) {
-    const std::vector<const void*> reads{data_ptr(a), data_ptr(b)};
+    const Reads reads{data_ptr(a), data_ptr(b)};
     LaunchGuard lg(ctx, "ewise2", 3.0 * n * dtype_size(a->dtype), (double)n, &reads);
     int la = layout_class(a), lb = layout_class(b);
     bool fast = la != 0 && lb != 0 && !(la == 2 && lb == 2) && (la == 2 || aligned16(data_ptr(a))) && (lb == 2 || aligned16(data_ptr(b)));

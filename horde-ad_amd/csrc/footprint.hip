@@ -1327,9 +1327,9 @@ int try_footprint_virtual(hgpu_ctx* ctx, const GemmParams& p, int dtype, const v
       label = intern_label(ctx, buf);
     }
     {
-      std::vector<const void*> reads{pa, pb};
-      reads.insert(reads.end(), vxa.begin(), vxa.end());
-      reads.insert(reads.end(), vya.begin(), vya.end());
+      Reads reads{pa, pb};
+      reads.add(vxa.begin(), vxa.end());
+      reads.add(vya.begin(), vya.end());
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       hipError_t e = launch_module(lg, kernel.fn, (unsigned)grid, 256u * (unsigned)pl.ks, args.data());
       if (e != hipSuccess) { if (part) buffer_release(part); if (colsum) hgpu_release(colsum); return check_hip(ctx, e, "footprint gemm launch"); }
@@ -1803,8 +1803,8 @@ int try_contract_map(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, in
                has_ext ? (L == 4 ? ",ext4" : (L == 2 ? ",ext2" : ",ext1")) : "");
       label = intern_label(ctx, buf);
     }
-    std::vector<const void*> reads{pa, pb};
-    reads.insert(reads.end(), ea.begin(), ea.end());
+    Reads reads{pa, pb};
+    reads.add(ea.begin(), ea.end());
     LaunchGuard lg(ctx, label, bytes, flops, &reads);
     hipError_t err = launch_module(lg, kernel.fn, (unsigned)grid, 256u * (unsigned)pl.ks, args);
     if (err != hipSuccess) { release_all(); return check_hip(ctx, err, "contract_map launch"); }
@@ -2193,7 +2193,8 @@ int try_mapped_sum(hgpu_ctx* ctx, const VirtualOp& v, const hgpu_operand* o, int
       snprintf(buf, sizeof buf, "mapped_sum[out%lld,R%lld,S%lld,in%d,instr%d,vec%d%s]", (long long)n_out, (long long)R, (long long)S, v.n_in, v.n_instr, W, v.padded ? ",padded" : "");
       label = intern_label(ctx, buf);
     }
-    LaunchGuard lg(ctx, label, bytes, (double)n_out * R * (v.n_instr + 1), &vxa);
+    const Reads reads(vxa);
+    LaunchGuard lg(ctx, label, bytes, (double)n_out * R * (v.n_instr + 1), &reads);
     hipError_t e = launch_module(lg, it->second.fn, (unsigned)(n_out * S), 256, args);
     if (e != hipSuccess) { if (part) buffer_release(part); return check_hip(ctx, e, "mapped_sum launch"); }
   }
@@ -2645,7 +2646,7 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
       snprintf(buf, sizeof buf, "onehot_contract[rows%d,cols%d,chunks%lld,positions%lld,onehot%lld,in%d,instr%d,es%d]", MR, NC, (long long)nch, (long long)G, (long long)EH, v.n_in, v.n_instr, es);
       label = intern_label(ctx, buf);
     }
-    std::vector<const void*> reads = ia;
+    Reads reads(ia);
     reads.push_back(data_ptr(x));
     LaunchGuard lg(ctx, label, bytes, 2.0 * MR * NC * (double)G * (double)nch, &reads);
     hipError_t e = launch_module(lg, kn.c.fn, (unsigned)grid, 256, args);

@@ -483,7 +483,7 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     for (int o = 0; o < n_out; ++o) outs[o] = res[(size_t)o];
     return HGPU_OK;
   }
-  const std::vector<const void*> reads = reads_of(n_in, in);
+  const Reads reads = reads_of(n_in, in);
   std::unique_ptr<LaunchGuard> guard(new LaunchGuard(ctx, label, bytes, (double)n * n_instr, &reads));   // ends before the partial sums' own launch
   LaunchGuard& lg = *guard;
   Compiled kernel;
@@ -660,7 +660,7 @@ extern "C" int hgpu_fused_extremum(hgpu_ctx* ctx, int n_in, const hgpu_array* co
       if (in[i]->strides[d] != 0) distinct *= in[i]->shape[d];
     bytes += (double)distinct * dtype_size(in[i]->dtype);
   }
-  const std::vector<const void*> reads = reads_of(n_in, in);
+  const Reads reads = reads_of(n_in, in);
   LaunchGuard lg(ctx, label, bytes, (double)n_out * L * (n_instr + 1), &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_extremum", &kernel);
@@ -867,7 +867,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
       if (data_ptr(in[j]) == data_ptr(in[i]) && layout[(size_t)j] != 's') dup = true;
     if (!dup) bytes += (double)n * dtype_size(in[i]->dtype);
   }
-  const std::vector<const void*> reads = reads_of(n_in, in);
+  const Reads reads = reads_of(n_in, in);
   LaunchGuard lg(ctx, label, bytes, (double)n * (n_instr + 1), &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_sum", &kernel);
@@ -1064,7 +1064,7 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     if (!dup) bytes += (double)n * dtype_size(in[i]->dtype);
   }
   for (int o = 0; o < n_out; ++o) bytes += (double)n * dtype_size(res[(size_t)o]->dtype);
-  const std::vector<const void*> reads = reads_of(n_in, in);
+  const Reads reads = reads_of(n_in, in);
   LaunchGuard lg(ctx, label, bytes, (double)n * n_instr, &reads);
   Compiled kernel;
   rc = kernel_for(ctx, key, hit, src, "fused_map_sums", &kernel);

@@ -103,10 +103,10 @@ int64_t total(const Group& g) {
 }
 
 // What a product's launch reads: see LaunchGuard.
-std::vector<const void*> product_reads(const void* pa, const void* pb, int n_terms, const void* const* as, const void* const* bs) {
-  std::vector<const void*> r{pa, pb};
-  r.insert(r.end(), as, as + n_terms);
-  r.insert(r.end(), bs, bs + n_terms);
+Reads product_reads(const void* pa, const void* pb, int n_terms, const void* const* as, const void* const* bs) {
+  Reads r{pa, pb};
+  r.add(as, as + n_terms);
+  r.add(bs, bs + n_terms);
   return r;
 }
 
@@ -182,7 +182,7 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
     }
     // the helper launches are timed under their own names, the label times the MFMA kernel alone
     if (p.k.nd > 1) {
-      const std::vector<const void*> none;
+      const Reads none;
       LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0, &none);
       hipLaunchKernelGGL(k_koff, dim3((unsigned)((Kp + 255) / 256)), dim3(256), 0, ctx->stream, p.k, p.K, Kp, ka, kb);
       p.kmask = -1;
@@ -209,7 +209,7 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
     const bool va = k_vector(pa, p.a_term, p.k.sa, p.m.sa, p.m, p.bt.sa), vb = k_vector(pb, p.b_term, p.k.sb, p.n.sb, p.n, p.bt.sb);
     LaunchArgs la{ctx->stream, -1, tm, tn, va, vb, grid, pa, pb, cdst, ka, kb};
     {
-      const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
+      const Reads reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
@@ -348,7 +348,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
       job->j = SplitJob{q, la.A, la.B, cdst, (int)tiles, split, (int)p.BT};
       hold_wide(ctx, std::move(job), (thin ? 8 : f64 ? 4 : 0) + (sak == 1 ? 2 : 0) + (sbk == 1 ? 1 : 0), label, bytes, flops, operands, split > 1 ? part : out->buf);
     } else {
-      const std::vector<const void*> reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
+      const Reads reads = product_reads(pa, pb, n_terms, p.a_term, p.b_term);
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();
@@ -706,7 +706,7 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     }
     // the helper launches are timed under their own names, the label times the MFMA kernel alone
     if (p.k.nd > 1) {
-      const std::vector<const void*> none;
+      const Reads none;
       LaunchGuard lk(ctx, "gemm_k_offsets", (double)Kp * 16, 0, &none);
       hipLaunchKernelGGL(k_koff, dim3((unsigned)((Kp + 255) / 256)), dim3(256), 0, ctx->stream, p.k, p.K, Kp, ka, kb);
       p.kmask = -1;
@@ -720,7 +720,7 @@ int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep
     void* cdst = split > 1 ? part->ptr : data_ptr(out);
     LaunchArgs la{ctx->stream, cfg, 0, 0, va, vb, grid, data_ptr(a), data_ptr(b), cdst, ka, kb};
     {
-      const std::vector<const void*> reads = product_reads(data_ptr(a), data_ptr(b), n_terms, p.a_term, p.b_term);
+      const Reads reads = product_reads(data_ptr(a), data_ptr(b), n_terms, p.a_term, p.b_term);
       LaunchGuard lg(ctx, label, bytes, flops, &reads);
       la.ev_start = lg.start_event();
       la.ev_stop = lg.stop_event();

@@ -932,7 +932,8 @@ int try_smallk(hgpu_ctx* ctx, int n_terms, const hgpu_array* const* as, const hg
   }
   hipError_t err = hipSuccess;
   {
-    LaunchGuard lg(ctx, d.label, d.bytes, d.flops, &d.args);
+    const Reads reads(d.args);
+    LaunchGuard lg(ctx, d.label, d.bytes, d.flops, &reads);
     void* args[] = {(void*)d.args.data()};
     err = launch_module(lg, d.fn, d.grid, 256, args, true, finish_fn == nullptr);
     if (err == hipSuccess && finish_fn) err = launch_module(lg, finish_fn, (unsigned)((ntiles + 7) / 8 * 8), 256, args, false, true);
@@ -1090,6 +1091,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     d.level = -1;
     if (gone[i]) continue;
     d.level = 0;
+    if (items.size() == 1) continue;
     for (auto* b : d.reads) {
       auto it = written_at.find(b);
       if (it != written_at.end()) d.level = std::max(d.level, it->second + 1);
@@ -1098,7 +1100,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
     top = std::max(top, d.level);
   }
   // A reduction that no held product reads goes out as late as it can, where the sums that need other levels go too.
-  {
+  if (top > 0) {
     std::map<const hgpu_buffer*, int> read_at;
     for (size_t i = items.size(); i-- > 0;) {
       Deferred& d = items[i];
@@ -1280,7 +1282,7 @@ void flush_deferred_locked(hgpu_ctx* ctx) {
 }
 
 // The blocks of `reads` that a held item writes.
-static std::set<const hgpu_buffer*> written_by(const std::vector<Deferred>& items, const std::vector<const void*>& reads) {
+static std::set<const hgpu_buffer*> written_by(const std::vector<Deferred>& items, const Reads& reads) {
   std::set<const hgpu_buffer*> s;
   for (auto& d : items)
     for (auto* w : d.writes)
@@ -1297,7 +1299,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
   for (auto* b : d.writes) q.keep(b);
   if (q.items.size() >= kMaxHeld || q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
   if (!q.maps.empty()) {
-    std::vector<const void*> reads;
+    Reads reads;
     for (auto* b : d.reads) reads.push_back(b->ptr);
     if (!written_by(q.maps, reads).empty()) flush_maps_locked(ctx);
   }
@@ -1309,7 +1311,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
 // Only large products, reductions and sums of partial results wait beyond the launch that asks: they are the ends of a reverse pass's
 // branches, and the later they go out the more of them share a launch.  Held products go with the first that is needed,
 // as before: their groups and chains are found among all of them.
-void make_way_locked(hgpu_ctx* ctx, const std::vector<const void*>& reads) {
+void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
   DeferredQueue& q = *ctx->dq;
   if (q.kind != DeferredQueue::kProducts) {
     flush_deferred_locked(ctx);
@@ -1398,7 +1400,7 @@ bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int6
 void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes) {
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
-  std::vector<const void*> from;
+  Reads from;
   for (auto* b : reads) from.push_back(b->ptr);
   // (one reduction asked for sends them all: the next passes, an optimizer's, will ask for the others)
   if (q.kind != DeferredQueue::kProducts || !written_by(q.items, from).empty()) flush_items_locked(ctx);

@@ -424,6 +424,9 @@ size_t arg_of_out(const Spec& sp, int o) { return 2 * sp.terms.size() + (size_t)
 // by column (a whole result as the columns factor of a term, or as an input of the program), and nothing else that is
 // held back.  Returns the number of levels, 0 when there is none.
 int find_chain(const std::vector<Deferred>& items, std::vector<ChainCand>& cand) {
+  int n_small = 0;
+  for (auto& d : items) n_small += d.kn != nullptr;
+  if (n_small < kChainMinLevels) return 0;
   std::map<std::pair<int64_t, bool>, int> count;
   std::map<const hgpu_buffer*, int> writer;
   for (size_t i = 0; i < items.size(); ++i) {
