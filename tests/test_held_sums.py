@@ -421,3 +421,19 @@ def test_the_end_of_an_objective_waits_in_recordings_only(host, gpu):
             [v.numpy() for v in program()]
     finally:
         graph.free()
+
+
+def test_sums_that_nobody_reads_do_not_gather(gpu):
+    """Submitted one by one, pass after pass: what is held goes out after a few launches that did not need it."""
+    fresh = pkg.capi.Lib().context(0)
+    x = fresh.upload(np.ones((100, 100003), np.float32))   # 40 MB
+    sums, size = [], fresh.mem_stats()[1]
+    for _ in range(48):
+        big = x.ewise1("neg")
+        sums.append(big.slice(1, 0, 4096).contract(None, 1))
+        del big
+    assert fresh.mem_stats()[1] - size <= 12 * (41 << 20)
+    for s in sums:
+        assert np.array_equal(s.numpy(), np.full(100, -4096, np.float32))
+    del x, sums, s
+    fresh.shutdown()
