@@ -31,7 +31,10 @@
 
 constexpr int kChainMaxPtrs = 448;      // pointers in the kernel's arguments (3.5 KB)
 constexpr int kChainMaxSections = 12;
-constexpr int kChainMinLevels = 8;      // a chain pays for reading the weights once (5-10 us); a level's launch costs 4.5 us, of which it saves about 3
+// Levels from which a chain is looked for at all.  (What it costs, reading the weights once, is 5 to 10 us, and a level saves about
+// 3 of the 4.5 us of its launch, so that fewer would do where pays() says so: not measured, recurrences of up to seven steps
+// keep a launch a level.)
+constexpr int kChainMinLevels = 8;
 constexpr int kChainMaxWidth = 4;       // products of one level
 constexpr int kChainLds = 160 * 1024;
 
@@ -350,7 +353,6 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
 std::string chain_source(const ChainPlan& c, const std::string& kname) {
   Src s;
   const int NC = c.NC, VK = chain_vk(c.f64);
-  const int half = c.out_elems + c.ext_elems;
   const bool whole4 = c.P % 4 == 0;      // a group of four columns is inside the array or outside
   s << kPrelude;
   s << "typedef " << (c.f64 ? "double" : "float") << " T;\n";
@@ -422,7 +424,8 @@ size_t arg_of_out(const Spec& sp, int o) { return 2 * sp.terms.size() + (size_t)
 
 // The held-back products that form a chain: those with P columns of one type that read one another's results column
 // by column (a whole result as the columns factor of a term, or as an input of the program), and nothing else that is
-// held back.  Returns the number of levels, 0 when there is none.
+// held back.  Returns the number of levels, 0 when there is none, or when one of them reads a result from further back than the
+// level before, or a level has more than kChainMaxWidth of them.
 int find_chain(const std::vector<Deferred>& items, std::vector<ChainCand>& cand) {
   int n_small = 0;
   for (auto& d : items) n_small += d.kn != nullptr;

@@ -182,3 +182,30 @@ def test_values_that_are_no_numbers_stay_in_their_column(gpu):
     bad = np.zeros(b, bool)
     bad[[7, 100, 202]] = True
     assert np.all(np.isfinite(got[:, ~bad])) and np.all(np.isnan(got[:, bad]))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_a_chain_longer_than_a_kernels_arguments(gpu, dt):
+    """h_t = tanh (W x_t + V h_(t-1) + e_t) over 150 steps, three arrays a step: a second kernel goes on where the first one's pointers end,
+    with the last result of the first read as an array."""
+    rng = np.random.default_rng(11)
+    width, batch, steps = 64, 96, 150
+    w, v = (rng.uniform(-0.3, 0.3, (width, width)).astype(dt) for _ in range(2))
+    xs, es = ([rng.uniform(-1, 1, (width, batch)).astype(dt) for _ in range(steps)] for _ in range(2))
+    prog = [(1, O2["add"], 0, 0, 1, 0), (0, O1["tanh"], 0, 2, 0, 0)]
+
+    def work():
+        up = gpu.upload
+        wa, va, h, xa, ea, res = up(w), up(v), up(np.zeros((), dt)).replicate([batch]).replicate([width]), [up(x) for x in xs], [up(e) for e in es], []
+        for t in range(steps):
+            h = gpu.contract_sum_map([matmul_views(wa, xa[t]), matmul_views(va, h)], 2, [None, ea[t]], prog, [3])[0]
+            res.append(h)
+        return [a.numpy().astype(np.float64) for a in res]
+
+    got, n, labels = chains(gpu, work)
+    assert n == 2, labels
+    prev = np.zeros((width, batch))
+    for t in range(steps):
+        want = np.tanh(w.astype(np.float64) @ xs[t] + v.astype(np.float64) @ prev + es[t])
+        assert np.max(np.abs(got[t] - want)) <= step_bound(dt, [width, width]), t
+        prev = got[t]
