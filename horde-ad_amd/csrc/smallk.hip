@@ -1326,15 +1326,14 @@ void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
   }
   if (!q.maps.empty() && !written_by(q.maps, reads).empty()) flush_maps_locked(ctx);
   std::set<const hgpu_buffer*> needed = written_by(q.items, reads);
-  if (needed.empty()) {
-    if (!ctx->cap && ++q.passed >= kMaxPassed) flush_deferred_locked(ctx);
-    return;
-  }
+  const bool late = needed.empty();
+  if (late && (ctx->cap || ++q.passed < kMaxPassed)) return;
+  q.passed = 0;
   // an item reads results of earlier ones only: from the last to the first, what goes out adds what it reads
   std::vector<char> go(q.items.size(), 0);
   for (size_t i = q.items.size(); i-- > 0;) {
     Deferred& d = q.items[i];
-    go[i] = !d.may_wait();
+    go[i] = d.may_wait() == late;      // (late: what has waited long enough, and of the products those that it reads)
     for (auto* w : d.writes) go[i] = go[i] || needed.count(w);
     if (go[i]) needed.insert(d.reads.begin(), d.reads.end());
   }
