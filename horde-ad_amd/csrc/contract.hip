@@ -371,40 +371,45 @@ __device__ __forceinline__ void partials_body(const SumArgs& a, unsigned bid, un
 // their lane groups without one, and for many outputs, where they would go around several times and wait for their loads
 // each time (300 x 784 outputs of 15 fp64 partials with five other problems of a group: 23.7 us in such blocks, 18.2 so; 2048 x 784 of 9
 // fp32 ones, 4.5 to launch among them, 22 and 16).  Up to eight are added one after another (0 + p0 + p1 + ...),
-// more of them in eight interleaved chains, eight loads in flight.  (Chains as short as those of the blocks above, which meet
+// more of them in eight interleaved chains, eight to fifteen loads in flight.  (Chains as short as those of the blocks above, which meet
 // in pairs: the error is 0.8 to 0.9 of theirs; four chains and the rest of S one after another had 1.1 to 1.5 of it.)
 template <typename T>
 __device__ __forceinline__ void partials_lane_body(const SumArgs& g, unsigned bid, unsigned nb) {
   const int64_t step = (int64_t)nb * 256;
-  for (int64_t i = (int64_t)bid * 256 + threadIdx.x; i < g.n; i += step) {
+  auto put = [&](int64_t i, T v) {
+    if (i < g.n1) ((T*)g.out)[i] = v;
+    else ((T*)g.out2)[i - g.n1] = v;
+  };
+  const int64_t first = (int64_t)bid * 256 + threadIdx.x;
+  // (Two loops, the end of S asked for first: in one loop, and with the end behind the eights, an output's loads waited for the
+  // store of the one before.  2048 x 784 of 9 and 2048 x 2048 of 2 fp32 partials in one launch, us: 39.4, so 32.3.)
+  if (g.S <= 8) {
+    for (int64_t i = first; i < g.n; i += step) {
+      const T* p = (const T*)g.part + i;
+      T x[8], acc = T(0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = u == 0 || u < g.S ? p[(int64_t)u * g.stride] : T(0);      // (a sum that begins with +0 is never -0)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += x[u];
+      put(i, acc);
+    }
+    return;
+  }
+  const int whole = g.S / 8 * 8;
+  for (int64_t i = first; i < g.n; i += step) {
     const T* p = (const T*)g.part + i;
-    T c[8] = {};
-    int s = 0;
-    if (g.S > 8) {
-      for (; s + 7 < g.S; s += 8) {
-        T x[8];
+    T x[8], rest[8], c[8] = {};
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = p[(int64_t)(s + u) * g.stride];
+    for (int u = 0; u < 8; ++u) rest[u] = whole + u < g.S ? p[(int64_t)(whole + u) * g.stride] : T(0);
+    for (int s = 0; s < whole; s += 8) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) c[u] += x[u];
-      }
+      for (int u = 0; u < 8; ++u) x[u] = p[(int64_t)(s + u) * g.stride];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c[u] += x[u];
     }
-    T x[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = s + u < g.S ? p[(int64_t)(s + u) * g.stride] : T(0);
-    T acc = T(0);
-    if (g.S > 8) {
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s + u < g.S) c[u] += x[u];
-      acc = ((c[0] + c[4]) + (c[2] + c[6])) + ((c[1] + c[5]) + (c[3] + c[7]));
-    } else {
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s + u < g.S) acc += x[u];
-    }
-    if (i < g.n1) ((T*)g.out)[i] = acc;
-    else ((T*)g.out2)[i - g.n1] = acc;
+    for (int u = 0; u < 8; ++u) c[u] += rest[u];
+    put(i, ((c[0] + c[4]) + (c[2] + c[6])) + ((c[1] + c[5]) + (c[3] + c[7])));
   }
 }
 

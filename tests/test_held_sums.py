@@ -310,7 +310,7 @@ def test_dot_products_of_expressions_round_once(host, n, with_pass):
     assert abs(float(s.numpy()) + p.sum()) <= 2.0 ** -24 * abs(p.sum()) + n * 2.0 ** -52 * np.abs(p).sum()
 
 
-@pytest.mark.parametrize("terms", [9, 15, 23, 31])
+@pytest.mark.parametrize("terms", [9, 15, 16, 23, 24, 31, 32])
 def test_partial_results_are_added_in_short_chains(gpu, terms):
     """One partial result of 1 and others of a quarter of its last place: of eight chains the one that has the 1 loses the others of its
     own, and the chains meet in three roundings."""
