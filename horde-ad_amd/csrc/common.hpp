@@ -48,6 +48,7 @@ struct hgpu_buffer {
   int known = kUnknown;
   bool known_relied_on = false;
   int held = 0;      // how often launches that are held back read or write it (guarded by the context's launch_mu)
+  int level = 0;     // among the levels of what goes out at one time (launch_held_locked in smallk.hip; guarded likewise)
 };
 
 struct hgpu_array {

@@ -1090,39 +1090,36 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
         for (int i : levels[(size_t)l]) gone[(size_t)i] = 1;
     }
   }
-  std::map<const hgpu_buffer*, int> written_at;
+  auto each_block = [&](auto&& f) {
+    for (size_t i = 0; i < items.size(); ++i) {
+      if (gone[i]) continue;
+      for (auto* b : items[i].reads) f(b);
+      for (auto* b : items[i].writes) f(b);
+    }
+  };
+  each_block([](hgpu_buffer* b) { b->level = -1; });      // the level that writes it
   int top = 0;
   for (size_t i = 0; i < items.size(); ++i) {
     Deferred& d = items[i];
     d.level = -1;
     if (gone[i]) continue;
     d.level = 0;
-    if (items.size() == 1) continue;
-    for (auto* b : d.reads) {
-      auto it = written_at.find(b);
-      if (it != written_at.end()) d.level = std::max(d.level, it->second + 1);
-    }
-    for (auto* b : d.writes) written_at[b] = d.level;
+    for (auto* b : d.reads) d.level = std::max(d.level, b->level + 1);
+    for (auto* b : d.writes) b->level = d.level;
     top = std::max(top, d.level);
   }
   // A reduction that no held product reads goes out as late as it can, where the sums that need other levels go too.
   if (top > 0) {
-    std::map<const hgpu_buffer*, int> read_at;
+    each_block([](hgpu_buffer* b) { b->level = INT32_MAX; });      // the first level that reads it
     for (size_t i = items.size(); i-- > 0;) {
       Deferred& d = items[i];
       if (gone[i]) continue;
       if (d.is_reduction) {
         int last = top;
-        for (auto* b : d.writes) {
-          auto it = read_at.find(b);
-          if (it != read_at.end()) last = std::min(last, it->second - 1);
-        }
+        for (auto* b : d.writes) last = std::min(last, b->level == INT32_MAX ? top : b->level - 1);
         d.level = std::max(d.level, last);
       }
-      for (auto* b : d.reads) {
-        auto it = read_at.emplace(b, d.level).first;
-        it->second = std::min(it->second, d.level);
-      }
+      for (auto* b : d.reads) b->level = std::min(b->level, d.level);
     }
   }
   for (int lv = 0; lv <= top; ++lv) {
@@ -1279,6 +1276,8 @@ static void flush_items_locked(hgpu_ctx* ctx) {
   const DeferredQueue::Kind kind = ctx->dq->kind;
   ctx->dq->kind = DeferredQueue::kProducts;
   launch_held_locked(ctx, items, kind);
+  items.clear();
+  if (ctx->dq->items.empty()) ctx->dq->items.swap(items);      // (its memory is kept: an item is a kilobyte to move)
 }
 
 void flush_deferred_locked(hgpu_ctx* ctx) {
@@ -1337,9 +1336,14 @@ void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
     for (auto* w : d.writes) go[i] = go[i] || needed.count(w);
     if (go[i]) needed.insert(d.reads.begin(), d.reads.end());
   }
-  std::vector<Deferred> out, stay;
-  for (size_t i = 0; i < q.items.size(); ++i) (go[i] ? out : stay).push_back(std::move(q.items[i]));
-  q.items.swap(stay);
+  std::vector<Deferred> out;
+  out.reserve(q.items.size());
+  size_t stay = 0;
+  for (size_t i = 0; i < q.items.size(); ++i) {
+    if (go[i]) out.push_back(std::move(q.items[i]));
+    else if (stay++ != i) q.items[stay - 1] = std::move(q.items[i]);
+  }
+  q.items.resize(stay);
   ctx->dq_pending = !q.items.empty() || !q.maps.empty();
   launch_held_locked(ctx, out, DeferredQueue::kProducts);
 }
