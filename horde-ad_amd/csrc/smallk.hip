@@ -36,7 +36,7 @@
 //
 // A problem of this size cannot fill the device and pays a launch and a round
 // of memory latency for a few microseconds of arithmetic, so launches are held
-// back (DeferredQueue) until something else needs the stream, and held-back
+// back (DeferredQueue) until something reads them (make_way_locked), and held-back
 // problems that do not read one another's results run as one kernel: each
 // problem's code in a namespace of its own, the first blocks of the grid for
 // problem 0, the next for problem 1, ...  Eight levels and more of problems
@@ -1348,7 +1348,7 @@ void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
   launch_held_locked(ctx, out, DeferredQueue::kProducts);
 }
 
-// A single-launch reduction joins the queue: held back until something else needs the stream, levelled with
+// A single-launch reduction joins the queue: held back until something reads it (make_way_locked), levelled with
 // the held products by who reads whose results, and launched together with the other reductions of its level.
 bool hold_reduction(hgpu_ctx* ctx, const RedJob& job, hgpu_buffer* const* reads, int n_reads, hgpu_buffer* write, hgpu_buffer* write2) {
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
