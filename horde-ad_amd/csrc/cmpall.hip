@@ -70,8 +70,7 @@ extern "C" int hgpu_compare_all(hgpu_ctx* ctx, int cmp, const hgpu_array* a, con
       hipLaunchKernelGGL(k_decide<T>, dim3(1), dim3(1), 0, ctx->stream, d, n, cmp, (const T*)data_ptr(a), (const T*)data_ptr(b), first, flag);
     });
     e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&host, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = read_back_locked(ctx, flag, sizeof(int), &host);
   }
   buffer_release(scratch);
   if (held_rc) return held_rc;

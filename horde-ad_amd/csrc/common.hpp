@@ -117,8 +117,8 @@ struct hgpu_ctx {
   uint64_t in_use = 0, reserved = 0, n_device_allocs = 0;
   int64_t fail_after = -1;
   std::string err;
-  void* staging = nullptr;       // pinned host staging block
-  size_t staging_bytes = 0;
+  void* staging = nullptr;       // pinned host memory: kReadBytes read back, then the number of the last read-back (read_back_locked)
+  uint64_t reads_back = 0;       // guarded by launch_mu, like the staging block
   LaunchMutex launch_mu;         // serialises enqueue order across host threads
   uint64_t write_epoch = 0;      // counts the writes into existing arrays (hgpu_overwrite, hgpu_assign): results remembered for given inputs end with it
   int num_cu = 256;
@@ -176,6 +176,10 @@ int zero_block(hgpu_ctx* ctx, const void** out);   // a context-lifetime block o
 // last one finishes the reduction and sets its counter back to zero.  Launches on the context's stream follow one
 // another, so the same counters serve them all.
 int ticket_block(hgpu_ctx* ctx, void** out);
+// At most this many bytes go to the host, or to the device, by a kernel instead of a copy of the runtime's (runtime.hip).
+constexpr size_t kReadBytes = 4096, kStoreBytes = 256;
+// The `bytes` bytes at the device address p, once everything enqueued before has written them (runtime.hip; the caller holds launch_mu).
+hipError_t read_back_locked(hgpu_ctx* ctx, const void* p, size_t bytes, void* host);
 // Fails (HGPU_ERR_UNSUPPORTED) when the stream is capturing: for entry points that must talk to the host.
 int no_capture(hgpu_ctx* ctx, const char* what);
 void buffer_retain(hgpu_buffer* b);
