@@ -138,6 +138,7 @@ struct hgpu_ctx {
   hgpu_buffer* zero_block = nullptr;     // 256 zero bytes, for kernels that want a dummy table
   hgpu_buffer* ticket_block = nullptr;   // counters (zero between launches) for kernels whose last block finishes a reduction
   hgpu_cap_pool* cap = nullptr;          // non-null while the stream is capturing into a graph
+  std::vector<const void*> recorded_functions;   // the run-time compiled kernels of the open recording (guarded by launch_mu)
   // Small products whose launch is held back until something else needs the
   // stream: those that do not depend on one another then go out as one kernel.
   hg::DeferredQueue* dq = nullptr;
@@ -150,6 +151,8 @@ struct hgpu_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hgpu_cap_pool* pool = nullptr;
+  struct Kernel { hipKernelNodeParams params; bool module; };   // the arguments are the graph's; module: compiled at run time
+  std::vector<Kernel> direct;                                   // a short recording's kernels (direct_kernels in runtime.hip)
 };
 
 namespace hg {
@@ -372,9 +375,15 @@ inline Reads reads_of(int n, const hgpu_array* const* in) {
   return r;
 }
 
+// A recording's launches of run-time compiled kernels, which its graph names by their handles (the caller holds launch_mu).
+inline void note_recorded(hgpu_ctx* c, hipFunction_t fn) {
+  if (c->cap) c->recorded_functions.push_back((const void*)fn);
+}
+
 // Launch of a run-time compiled kernel under a guard: `first` / `last` say whether this is the first / last
 // launch the guard's record is to cover.
 inline hipError_t launch_module(LaunchGuard& lg, hipFunction_t fn, unsigned grid, unsigned block, void** args, bool first = true, bool last = true) {
+  note_recorded(lg.ctx, fn);
   if (!lg.timed || (uint64_t)grid * block > 0xffffffffull) return hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, 0, lg.ctx->stream, args, nullptr);
   return hipExtModuleLaunchKernel(fn, grid * block, 1, 1, block, 1, 1, 0, lg.ctx->stream, args, nullptr, first ? lg.start_event() : nullptr,
                                   last ? lg.stop_event() : nullptr, 0);

@@ -10,6 +10,7 @@
 #include <sys/types.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <cerrno>
 #include <chrono>
 #include <cstdlib>
@@ -452,6 +453,7 @@ int hgpu_capture_begin(hgpu_ctx* ctx) {
   hipError_t e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) return check_hip(ctx, e, "capture_begin");
   hgpu_cap_pool* pool = new hgpu_cap_pool;
+  ctx->recorded_functions.clear();
   {
     // The warm blocks of the context move into the capture's pool: a capture
     // after a warm-up run allocates nothing.
@@ -476,6 +478,34 @@ static void retire_pool(hgpu_ctx* ctx, hgpu_cap_pool* pool) {
   for (auto& kv : pool->cache) ctx->cache.emplace(kv.first, kv.second);
   pool->cache.clear();
   if (--pool->refs == 0) delete pool;
+}
+
+// The kernels of a short recording in their order, to be launched one by one; empty where the recording holds anything
+// else, or more of them.  A graph's launch costs the device about 4.7 us before its first kernel and the host 15 to 16,
+// a kernel's launch the host 2.4 and the device nothing beside the kernel before it.  One kernel of 31 us over and over:
+// 36.8 us a pass as a graph, 32.0 so; two 68.6 / 63.9; four 132.0 / 127.8; eight 258.6 / 255.2; seventeen 543.7 / 542.1.
+// Where the kernels are short, though, eight are as fast either way (21.5 / 20.4) and slower so for who waits for each pass
+// (34.5 / 47.3; four of them 33.1 / 19.9): the line is drawn at four.
+constexpr size_t kDirectKernels = 4;
+static std::vector<hgpu_graph::Kernel> direct_kernels(hgpu_ctx* ctx, hipGraph_t graph) {
+  std::vector<hgpu_graph::Kernel> r;
+  hipGraphNode_t nodes[kDirectKernels], from[kDirectKernels], to[kDirectKernels];
+  size_t n = 0, edges = 0;
+  if (hipGraphGetNodes(graph, nullptr, &n) != hipSuccess || n == 0 || n > kDirectKernels) return r;
+  if (hipGraphGetEdges(graph, nullptr, nullptr, &edges) != hipSuccess || edges != n - 1) return r;
+  if (hipGraphGetNodes(graph, nodes, &n) != hipSuccess || (edges && hipGraphGetEdges(graph, from, to, &edges) != hipSuccess)) return r;
+  for (size_t k = 0; k < n; ++k) {
+    // one stream's recording is a chain in the order of its launches; anything else is the graph's business
+    bool follows = k == 0;
+    for (size_t e = 0; e < edges; ++e) follows = follows || (from[e] == nodes[k - 1] && to[e] == nodes[k]);
+    hipGraphNodeType type;
+    hipKernelNodeParams kp;
+    memset(&kp, 0, sizeof kp);
+    if (!follows || hipGraphNodeGetType(nodes[k], &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
+        hipGraphKernelNodeGetParams(nodes[k], &kp) != hipSuccess || !kp.func || !kp.kernelParams) return {};
+    r.push_back({kp, std::find(ctx->recorded_functions.begin(), ctx->recorded_functions.end(), kp.func) != ctx->recorded_functions.end()});
+  }
+  return r;
 }
 
 int hgpu_capture_end(hgpu_ctx* ctx, hgpu_graph** out) {
@@ -506,6 +536,8 @@ int hgpu_capture_end(hgpu_ctx* ctx, hgpu_graph** out) {
     delete gr;
     return held_rc ? held_rc : check_hip(ctx, e, "capture_end");   // a recording that lacks a launch is no recording
   }
+  gr->direct = direct_kernels(ctx, gr->graph);
+  (void)hipGetLastError();
   *out = gr;
   return HGPU_OK;
 }
@@ -518,7 +550,15 @@ int hgpu_graph_launch(hgpu_graph* gr) {
   (void)hipSetDevice(ctx->device);
   if (ctx->dq_pending) flush_deferred_locked(ctx);
   if (int rc = take_deferred_rc(ctx)) return rc;
-  return check_hip(ctx, hipGraphLaunch(gr->exec, ctx->stream), "hipGraphLaunch");
+  if (gr->direct.empty() || stream_recorded(ctx)) return check_hip(ctx, hipGraphLaunch(gr->exec, ctx->stream), "hipGraphLaunch");
+  for (const auto& k : gr->direct) {
+    const hipKernelNodeParams& p = k.params;
+    const hipError_t e = k.module ? hipModuleLaunchKernel((hipFunction_t)p.func, p.gridDim.x, p.gridDim.y, p.gridDim.z, p.blockDim.x, p.blockDim.y, p.blockDim.z,
+                                                          p.sharedMemBytes, ctx->stream, p.kernelParams, nullptr)
+                                  : hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes, ctx->stream);
+    if (e != hipSuccess) return check_hip(ctx, e, "graph_launch");
+  }
+  return HGPU_OK;
 }
 
 int hgpu_graph_destroy(hgpu_graph* gr) {

@@ -984,6 +984,7 @@ static void launch_maps(hgpu_ctx* ctx, std::vector<Deferred>& items) {
     } else {
       for (auto& w : m.args) args.push_back(&w);
     }
+    note_recorded(ctx, fn);
     const hipError_t err = timed ? hipExtModuleLaunchKernel(fn, grid * 256, 1, 1, 256, 1, 1, 0, ctx->stream, args.data(), nullptr, r.a, r.b, 0)
                                  : hipModuleLaunchKernel(fn, grid, 1, 1, 256, 1, 1, 0, ctx->stream, args.data(), nullptr);
     if (timed) ctx->prof.push_back(r);
@@ -1044,6 +1045,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
       }
     }
     void* args[] = {(void*)ar.data()};
+    note_recorded(ctx, fn);
     hipError_t err = ea ? hipExtModuleLaunchKernel(fn, grid * block, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr, ea, eb, 0)
                         : hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr);
     if (err != hipSuccess) {

@@ -47,3 +47,38 @@ def test_overwrite_is_in_order_and_takes_a_copy():
             assert np.array_equal(o, w * w + w)
     finally:
         graph.free()
+
+
+@pytest.mark.parametrize("kernels", [1, 2, 4, 5])
+def test_short_recordings_replay(kernels):
+    """Recordings of up to four kernels are launched one by one, longer ones as a graph: each replay reads its inputs
+    anew and gives the bits of the eager run, with eager work between the replays.  Column sums of ever narrower
+    arrays: run-time compiled and precompiled kernels in one chain."""
+    host = H.Host()
+    rng = np.random.default_rng(kernels)
+    x = rng.uniform(-1, 1, (3,) * kernels + (2000,))
+    v = host.concrete(x)
+
+    def program():
+        y = v
+        for k in range(kernels):
+            y = y.op1("sin") if k % 2 == 0 else y.ssum()
+            y = y.dense()
+        return y
+    want = program().numpy()
+    graph, out = host.capture(program)
+    try:
+        for replay in range(4):
+            graph.launch()
+            assert np.array_equal(out.numpy(), want), replay
+            _ = (host.concrete(rng.uniform(-1, 1, 333 + replay)) * 2.0).numpy()
+            graph.launch()
+            graph.launch()
+            host.sync()
+            assert np.array_equal(out.numpy(), want), replay
+        v.overwrite(x * 0.5)
+        graph.launch()
+        half = out.numpy()
+        assert np.array_equal(half, program().numpy()) and not np.array_equal(half, want)
+    finally:
+        graph.free()
