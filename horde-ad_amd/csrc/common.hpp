@@ -280,6 +280,17 @@ bool wide_takes_rows(const WideJob& job);
 // smallk.hip: the sums over K of n terms of M rows of fp32 elements, each term times the one element `factor` (null: 1), as
 // *part (rows x *shares, doubles) by a held product that reads the same rows; false: there is none
 bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
+// One gather of whole slices that may be held back (index.hip): its arguments and its result's block.
+struct GatherJob;
+hipError_t launch_gather(hgpu_ctx* ctx, const GatherJob& job);       // the caller holds launch_mu
+const char* gather_label(const GatherJob& job, double* bytes);
+// smallk.hip: holds the gather back (retaining the buffers) until something reads its result or writes to an array that exists;
+// it never runs if nobody has the result any more by then.  false: the caller launches it now (it reads held results)
+bool hold_gather(hgpu_ctx* ctx, const std::shared_ptr<GatherJob>& job, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
+// smallk.hip: the held gather that will write this block, if there is one (the caller holds launch_mu)
+std::shared_ptr<GatherJob> gather_into_locked(hgpu_ctx* ctx, const hgpu_buffer* b);
+// index.hip: *o (one element) = sum of a * b, where a held gather is to write a or b and need not for this; *handled: taken
+int try_gather_dot(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, const hgpu_array* o, bool* handled);
 // smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it
 void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const char* label, double bytes, double flops, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
 // contract.hip: a program over a few elements (its last instruction's result is `out`), in a recording launched with held sums; false: left to the caller
@@ -318,8 +329,8 @@ inline unsigned grid_for(int64_t n, int block, int max_blocks) {
 // (or an unwritable directory) means no files.  `what` names the caller in errors.
 int rtc_compile(hgpu_ctx* ctx, const std::string& src, const char* what, std::vector<char>* code);
 
-// Zeroes `bytes` bytes (rounded up to 16) with a fill kernel (ewise.hip).
-int zero_fill(hgpu_ctx* ctx, void* p, size_t bytes);
+// Zeroes `bytes` bytes (rounded up to 16) with a fill kernel (ewise.hip); fresh: of a block that nothing has been enqueued for.
+int zero_fill(hgpu_ctx* ctx, void* p, size_t bytes, bool fresh = false);
 // Strided copy between two views of equal shape (ewise.hip).
 int copy_view(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const void* src,
               const int64_t* sst, void* dst, const int64_t* dst_st);

@@ -1425,6 +1425,12 @@ int hgpu_contract(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n
     return HGPU_OK;
   }
   rc = new_dense(ctx, a->dtype, n_keep, a->shape, &o);
+  if (!rc && b && n_keep == 0) {
+    bool handled = false;
+    rc = try_gather_dot(ctx, a, b, o, &handled);
+    if (rc) { hgpu_release(o); return rc; }
+    if (handled) { *out = o; return HGPU_OK; }
+  }
   if (rc) return rc;
 
   bool handled = false;

@@ -313,12 +313,13 @@ inline int max_blocks(hgpu_ctx* ctx) { return ctx->num_cu * 8; }
 
 namespace hg {
 
-int zero_fill(hgpu_ctx* ctx, void* p, size_t bytes) {
+int zero_fill(hgpu_ctx* ctx, void* p, size_t bytes, bool fresh) {
   // Blocks come from the allocator in multiples of 256 bytes, so rounding the
   // length up to 16 stays inside the block.
   int64_t n16 = (int64_t)((bytes + 15) / 16);
   if (n16 == 0) return HGPU_OK;
-  LaunchGuard lg(ctx, "zero_fill", (double)bytes, 0);
+  const Reads none;
+  LaunchGuard lg(ctx, "zero_fill", (double)bytes, 0, fresh ? &none : nullptr);
   hipLaunchKernelGGL(k_zero16, dim3(grid_for(n16, kBlock, max_blocks(ctx))), dim3(kBlock), 0, ctx->stream, n16, (uint4*)p);
   HG_CHECK_LAUNCH(ctx, "zero_fill");
   return HGPU_OK;

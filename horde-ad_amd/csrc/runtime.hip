@@ -234,7 +234,7 @@ int new_zeros(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, hgpu_arr
   int64_t n = nelem(*out);
   if (n > 0) {
     // A fill kernel, not hipMemsetAsync: callers may capture the stream.
-    rc = zero_fill(ctx, data_ptr(*out), (size_t)n * dtype_size(dtype));
+    rc = zero_fill(ctx, data_ptr(*out), (size_t)n * dtype_size(dtype), true);
     if (rc) {
       hgpu_release(*out);
       *out = nullptr;
@@ -696,7 +696,8 @@ int hgpu_upload(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const 
       hgpu_release(a);
       return fail(ctx, HGPU_ERR_INVALID, "null host pointer");
     }
-    LaunchGuard lg(ctx);
+    const Reads none;      // (a new array: what is held back stays so)
+    LaunchGuard lg(ctx, nullptr, 0, 0, &none);
     hipError_t e = store_locked(ctx, data_ptr(a), bytes, host);
     if (e != hipSuccess) {
       hgpu_release(a);

@@ -759,6 +759,9 @@ struct DeferredQueue {
   std::vector<Deferred> items;
   enum Kind { kProducts, kCopies } kind = kProducts;     // what `items` holds
   std::vector<Deferred> maps;
+  struct Gather { std::shared_ptr<GatherJob> job; std::vector<hgpu_buffer*> reads; hgpu_buffer* write; };
+  std::vector<Gather> gathers;       // they read no held result, and nothing held reads theirs
+  bool any() const { return !items.empty() || !maps.empty() || !gathers.empty(); }
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
   size_t held_bytes = 0;             // of the blocks that items and maps keep
@@ -1263,7 +1266,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
 static void flush_maps_locked(hgpu_ctx* ctx) {
   std::vector<Deferred> maps;
   maps.swap(ctx->dq->maps);
-  ctx->dq_pending = !ctx->dq->items.empty();
+  ctx->dq_pending = ctx->dq->any();
   if (maps.empty()) return;
   (void)hipSetDevice(ctx->device);
   launch_maps(ctx, maps);
@@ -1274,7 +1277,7 @@ static void flush_items_locked(hgpu_ctx* ctx) {
   std::vector<Deferred> items;
   items.swap(ctx->dq->items);
   ctx->dq->passed = 0;
-  ctx->dq_pending = !ctx->dq->maps.empty();
+  ctx->dq_pending = ctx->dq->any();
   const DeferredQueue::Kind kind = ctx->dq->kind;
   ctx->dq->kind = DeferredQueue::kProducts;
   launch_held_locked(ctx, items, kind);
@@ -1282,9 +1285,49 @@ static void flush_items_locked(hgpu_ctx* ctx) {
   if (ctx->dq->items.empty()) ctx->dq->items.swap(items);      // (its memory is kept: an item is a kilobyte to move)
 }
 
+// The held gathers that `take` names go out; one whose result only the queue has left is forgotten.
+template <typename F>
+static void flush_gathers_locked(hgpu_ctx* ctx, const F& take) {
+  DeferredQueue& q = *ctx->dq;
+  std::vector<DeferredQueue::Gather> out;
+  for (size_t i = 0; i < q.gathers.size();) {
+    if (!take(q.gathers[i])) { ++i; continue; }
+    out.push_back(std::move(q.gathers[i]));
+    q.gathers.erase(q.gathers.begin() + (long)i);
+  }
+  ctx->dq_pending = q.any();
+  if (!out.empty()) (void)hipSetDevice(ctx->device);
+  for (auto& g : out) {
+    if (g.write->refs.load() > 1) {
+      hgpu_ctx::ProfRec r{nullptr, nullptr, nullptr, 0, 0};
+      r.name = gather_label(*g.job, &r.bytes);
+      ctx->count_recorded(r.name, r.bytes, 0);
+      const bool timed = ctx->profiling && !ctx->cap && hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess;
+      if (timed) (void)hipEventRecord(r.a, ctx->stream);
+      const hipError_t e = launch_gather(ctx, *g.job);
+      if (timed) {
+        (void)hipEventRecord(r.b, ctx->stream);
+        ctx->prof.push_back(r);
+      }
+      if (e != hipSuccess) {
+        int rc = check_hip(ctx, e, "gather launch");
+        if (!ctx->deferred_rc) ctx->deferred_rc = rc;
+      }
+    }
+    for (auto* b : g.reads) q.let_go(b);
+    q.let_go(g.write);
+  }
+}
+static void flush_gathers_locked(hgpu_ctx* ctx) { flush_gathers_locked(ctx, [](const DeferredQueue::Gather&) { return true; }); }
+// ... those whose results a launch that reads `blocks` needs.
+static void gathers_for_locked(hgpu_ctx* ctx, const std::vector<hgpu_buffer*>& blocks) {
+  if (!ctx->dq->gathers.empty()) flush_gathers_locked(ctx, [&](const DeferredQueue::Gather& g) { return std::find(blocks.begin(), blocks.end(), g.write) != blocks.end(); });
+}
+
 void flush_deferred_locked(hgpu_ctx* ctx) {
   ctx->dq_pending = false;
   if (!ctx->dq) return;
+  flush_gathers_locked(ctx);
   flush_items_locked(ctx);
   flush_maps_locked(ctx);
 }
@@ -1305,6 +1348,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
   DeferredQueue& q = *ctx->dq;
   for (auto* b : d.reads) q.keep(b);
   for (auto* b : d.writes) q.keep(b);
+  gathers_for_locked(ctx, d.reads);
   if (q.items.size() >= kMaxHeld || q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
   if (!q.maps.empty()) {
     Reads reads;
@@ -1321,6 +1365,12 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
 // as before: their groups and chains are found among all of them.
 void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
   DeferredQueue& q = *ctx->dq;
+  if (!q.gathers.empty())
+    flush_gathers_locked(ctx, [&](const DeferredQueue::Gather& g) {
+      for (const void* r : reads)
+        if (r >= g.write->ptr && r < (const char*)g.write->ptr + g.write->bytes) return true;
+      return false;
+    });
   if (q.kind != DeferredQueue::kProducts) {
     flush_deferred_locked(ctx);
     return;
@@ -1346,7 +1396,7 @@ void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
     else if (stay++ != i) q.items[stay - 1] = std::move(q.items[i]);
   }
   q.items.resize(stay);
-  ctx->dq_pending = !q.items.empty() || !q.maps.empty();
+  ctx->dq_pending = q.any();
   launch_held_locked(ctx, out, DeferredQueue::kProducts);
 }
 
@@ -1417,6 +1467,7 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
   DeferredQueue& q = *ctx->dq;
   Reads from;
   for (auto* b : reads) from.push_back(b->ptr);
+  gathers_for_locked(ctx, reads);
   // (one reduction asked for sends them all: the next passes, an optimizer's, will ask for the others)
   if (q.kind != DeferredQueue::kProducts || !written_by(q.items, from).empty()) flush_items_locked(ctx);
   if (q.maps.size() >= kMaxHeld || !written_by(q.maps, from).empty()) flush_maps_locked(ctx);
@@ -1445,6 +1496,7 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   DeferredQueue& q = *ctx->dq;
   q.keep(src);
   q.keep(dst);
+  flush_gathers_locked(ctx);      // (they may read what the copy writes)
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
   bool fits = q.maps.empty() && (q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs));
   for (size_t i = 0; fits && i < q.items.size(); ++i) {
@@ -1456,6 +1508,36 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   q.kind = DeferredQueue::kCopies;
   ctx->dq_pending = true;
   if (!hold) flush_deferred_locked(ctx);
+}
+
+// The held gathers at most: results that nobody has read yet, each with its block.
+constexpr size_t kMaxHeldGathers = 4;
+
+bool hold_gather(hgpu_ctx* ctx, const std::shared_ptr<GatherJob>& job, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write) {
+  static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
+  if (!hold || !write) return false;
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
+  if (!ctx->dq) ctx->dq = new DeferredQueue;
+  DeferredQueue& q = *ctx->dq;
+  if (q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);      // copies into arrays that exist
+  gathers_for_locked(ctx, reads);
+  Reads from;
+  for (auto* b : reads) from.push_back(b->ptr);
+  if (!written_by(q.items, from).empty() || !written_by(q.maps, from).empty()) return false;
+  if (q.gathers.size() >= kMaxHeldGathers) flush_gathers_locked(ctx);
+  for (auto* b : reads) q.keep(b);
+  q.keep(write);
+  q.gathers.push_back({job, reads, write});
+  ctx->dq_pending = true;
+  if (q.held_bytes > kMaxHeldBytes) flush_deferred_locked(ctx);
+  return true;
+}
+
+std::shared_ptr<GatherJob> gather_into_locked(hgpu_ctx* ctx, const hgpu_buffer* b) {
+  if (ctx->dq)
+    for (auto& g : ctx->dq->gathers)
+      if (g.write == b) return g.job;
+  return nullptr;
 }
 
 void flush_deferred(hgpu_ctx* ctx) {
