@@ -274,12 +274,12 @@ struct WideJob;
 hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n);
 constexpr int kMaxWideJobs = 4;
 // gemm.hip: row sums that a held product hands out beside its result (see join_wide_rows)
-int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride);
+int wide_row_shares(const WideJob& job, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride);
 void wide_take_rows(WideJob& job, void* part, const void* factor);
 bool wide_takes_rows(const WideJob& job);
-// smallk.hip: the sums over K of n terms of M rows of fp32 elements, each term times the one element `factor` (null: 1), as
+// smallk.hip: the sums over K of n terms of M rows of floats of `dtype`, each term times the one element `factor` (null: 1), as
 // *part (rows x *shares, doubles) by a held product that reads the same rows; false: there is none
-bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
+bool join_wide_rows(hgpu_ctx* ctx, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
 // One gather of whole slices that may be held back (index.hip): its arguments and its result's block.
 struct GatherJob;
 hipError_t launch_gather(hgpu_ctx* ctx, const GatherJob& job);       // the caller holds launch_mu

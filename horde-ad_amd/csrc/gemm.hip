@@ -453,16 +453,19 @@ hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
     return hipGetLastError();
   }
   const unsigned grid = split_group(js, n, &g);
-  if (jobs[0]->f64) launch_wide_f64_group(g, grid, jobs[0]->akc, jobs[0]->bkc, ctx->stream);
+  if (jobs[0]->f64) launch_wide_f64_group(g, grid, jobs[0]->akc, jobs[0]->bkc, rows, ctx->stream);
   else launch_split_f32_group(g, grid, jobs[0]->akc, jobs[0]->bkc, jobs[0]->thin, rows, ctx->stream);
   return hipGetLastError();
 }
 
 // The shares of K of a held product that can also hand out the sums of the rows at `as` (n terms of M x K elements, rows
 // `row_stride` apart); 0: it cannot.  The terms may come in another order: each is added up by itself and all meet in one sum.
-int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride) {
+// (fp64: only of several terms, which would be a launch of their own, 4.7 us for the rows of 28 x 128 x 150 where the products
+// take 1.1 more for them.  A single term's sum waits with the other reductions of its kind, and fp64 additions hold the matrix cores
+// up: rows of 300 x 5000 and 100 x 5000 cost their products 4.4 us, that launch 1.6.)
+int wide_row_shares(const WideJob& job, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride) {
   const SplitParams& p = job.j.p;
-  if (job.f64 || !job.akc || p.rows || job.j.batches != 1 || p.M != M || p.K != K || p.sam != (uint64_t)row_stride * 4 || std::max(p.n_terms, 1) != n) return 0;
+  if (job.f64 != (dtype == HGPU_F64) || (job.f64 && n < 2) || !job.akc || p.rows || job.j.batches != 1 || p.M != M || p.K != K || p.sam != (uint64_t)row_stride * dtype_size(dtype) || std::max(p.n_terms, 1) != n) return 0;
   std::vector<const void*> x(as, as + n), y(1, job.j.A);
   if (p.n_terms > 0) y.assign(p.a_term, p.a_term + n);
   std::sort(x.begin(), x.end());
@@ -473,7 +476,7 @@ int wide_row_shares(const WideJob& job, int n, const void* const* as, int64_t M,
 bool wide_takes_rows(const WideJob& job) { return job.j.p.rows != nullptr; }
 void wide_take_rows(WideJob& job, void* part, const void* factor) {
   job.j.p.rows = (double*)part;
-  job.j.p.row_factor = (const float*)factor;
+  job.j.p.row_factor = factor;
 }
 
 int try_gemm(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, hgpu_array* out, bool* handled,

@@ -791,7 +791,7 @@ struct SplitParams {
   const void* a_term[kMaxTerms];
   const void* b_term[kMaxTerms];
   double* rows;                 // sums of A's rows over the block's share of K, each element times *row_factor (rows x shares of K; null: not asked for)
-  const float* row_factor;      // null: 1
+  const void* row_factor;       // one element; null: 1
 };
 // The share of such a product that a block computes: rows from m0, columns from n0, k in [kbeg, kend), operands of its term
 // and batch element; s numbers the (term, K chunk) pairs.
@@ -875,8 +875,8 @@ inline unsigned split_group(const SplitJob* const* jobs, int n, SplitGroup* g) {
 }
 void launch_wide_f64(const SplitParams& p, const LaunchArgs& a);
 void launch_split_f32(const SplitParams& p, const LaunchArgs& a, bool thin);      // thin: tiles of 128 x 32 instead of 128 x 128
-void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream);
 // (rows: products among them hand out the sums of A's rows, A is contiguous along K)
+void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool rows, hipStream_t stream);
 void launch_split_f32_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool thin, bool rows, hipStream_t stream);
 
 // defined in gemm_f32.hip / gemm_f64.hip

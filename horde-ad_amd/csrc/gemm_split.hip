@@ -201,7 +201,7 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   static_assert(!ROWS || (AKC && NA == 1 && BM * 2 == NT), "lane t stages a half of row t / 2");
   const bool sum_rows = ROWS && p.rows != nullptr && n0 == 0;
   double row_sum = 0, row_factor = 1;
-  if (sum_rows && p.row_factor) row_factor = (double)*p.row_factor;
+  if (sum_rows && p.row_factor) row_factor = (double)*(const float*)p.row_factor;
   auto store_a = [&](int u, u4* to, int left) {      // left: elements of k that the step has, 16 and more: all
     sa.store(ra[u], u, to, top_a);
     if (sum_rows) {

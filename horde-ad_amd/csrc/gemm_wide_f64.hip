@@ -79,7 +79,9 @@ struct Side {
 };
 
 // AKC, BKC: the operand is contiguous along k (lanes stage 16 bytes of a row; otherwise a row each, 8 bytes of two k).
-template <bool AKC, bool BKC>
+// ROWS: the lanes also add up the elements of A they stage, eight lanes to a row (see gemm_split.hip); blocks of the first
+// column of tiles do, for products that ask.
+template <bool AKC, bool BKC, bool ROWS>
 __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = 2, WN = 2, TM = 2, TN = 2;          // wavefronts, and 16 x 16 blocks of each
   constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
@@ -104,6 +106,24 @@ __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const d
 
   const int steps = (kend - kbeg + SK - 1) / SK, whole = (kend - kbeg) / SK;
   u4 ra[NA], rb[NB];
+  static_assert(!ROWS || AKC, "the lanes of a row stage pieces of it");
+  const bool sum_rows = ROWS && p.rows != nullptr && n0 == 0;
+  double row_sum[NA], row_factor = 1;
+#pragma unroll
+  for (int i = 0; i < NA; ++i) row_sum[i] = 0;
+  if (sum_rows && p.row_factor) row_factor = *(const double*)p.row_factor;
+  auto store_a = [&](u4* to, int left) {      // left: elements of k that the step has, SK and more: all
+    sa.store(ra, to);
+    if (sum_rows) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const d2 x = __builtin_bit_cast(d2, ra[i]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (left >= SK || 2 * (t % 8) + j < left) row_sum[i] = __builtin_fma(x[j], row_factor, row_sum[i]);
+      }
+    }
+  };
   auto fetch = [&](int i) {
     sa.load(kbeg + i * SK, ra);
     sb.load(kbeg + i * SK, rb);
@@ -114,7 +134,7 @@ __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const d
   };
   if (whole > 0) fetch(0);
   else fetch_tail(0);
-  sa.store(ra, lds[0]);
+  store_a(lds[0], kend - kbeg);
   sb.store(rb, lds[0] + BM * 8);
   __syncthreads();
 
@@ -150,7 +170,7 @@ __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const d
           for (int j = 0; j < TN; ++j) acc[i][j] = MfmaF64::run(a[h][i][u], b[h][j][u], acc[i][j]);
     if constexpr (decltype(next)::value != 0) {
       __builtin_amdgcn_sched_barrier(0);
-      sa.store(ra, lds[cur ^ 1]);
+      store_a(lds[cur ^ 1], decltype(next)::value == 1 ? SK : kend - kbeg - (i0 + 1) * SK);
       sb.store(rb, lds[cur ^ 1] + BM * 8);
     }
     __syncthreads();
@@ -180,6 +200,15 @@ __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const d
     step(i0, b0, b0);
   }
 
+  if (sum_rows) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      double v = row_sum[i];
+      for (int o = 1; o < 8; o <<= 1) v += __shfl_xor(v, o);
+      const int m = m0 + (t + i * NT) / 8;
+      if (t % 8 == 0 && m < p.M) p.rows[(int64_t)m * nsplits + share.s] = v;
+    }
+  }
   double* Cout = C + (int64_t)batch * p.bsc + (int64_t)share.s * p.c_split_stride;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
@@ -198,17 +227,17 @@ __device__ __forceinline__ void gemm_wide_f64_body(const SplitParams& p, const d
 
 template <bool AKC, bool BKC>
 __global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64(SplitParams p, const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C) {
-  gemm_wide_f64_body<AKC, BKC>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
+  gemm_wide_f64_body<AKC, BKC, false>(p, A, B, C, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y, blockIdx.z);
 }
 
-template <bool AKC, bool BKC>
+template <bool AKC, bool BKC, bool ROWS>
 __global__ void __launch_bounds__(NT, 4) k_gemm_wide_f64_group(SplitGroup g) {
   int nr;
   const int k = split_job(g, blockIdx.x, &nr);
   if (k < 0) return;
   const SplitJob& j = g.job[k];
   const int per_batch = j.tiles * j.splits, batch = nr / per_batch;
-  gemm_wide_f64_body<AKC, BKC>(j.p, (const double*)j.A, (const double*)j.B, (double*)j.C, nr - batch * per_batch, j.splits, batch);
+  gemm_wide_f64_body<AKC, BKC, ROWS>(j.p, (const double*)j.A, (const double*)j.B, (double*)j.C, nr - batch * per_batch, j.splits, batch);
 }
 
 }  // namespace
@@ -225,12 +254,14 @@ void launch_wide_f64(const SplitParams& p, const LaunchArgs& a) {
   else launch_kernel(a, k_gemm_wide_f64<false, false>, p, A, B, C);
 }
 
-void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, hipStream_t stream) {
+void launch_wide_f64_group(const SplitGroup& g, unsigned grid, bool akc, bool bkc, bool rows, hipStream_t stream) {
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, g); };
-  if (akc && bkc) go(k_gemm_wide_f64_group<true, true>);
-  else if (akc) go(k_gemm_wide_f64_group<true, false>);
-  else if (bkc) go(k_gemm_wide_f64_group<false, true>);
-  else go(k_gemm_wide_f64_group<false, false>);
+  if (rows && bkc) go(k_gemm_wide_f64_group<true, true, true>);
+  else if (rows) go(k_gemm_wide_f64_group<true, false, true>);
+  else if (akc && bkc) go(k_gemm_wide_f64_group<true, true, false>);
+  else if (akc) go(k_gemm_wide_f64_group<true, false, false>);
+  else if (bkc) go(k_gemm_wide_f64_group<false, true, false>);
+  else go(k_gemm_wide_f64_group<false, false, false>);
 }
 
 }  // namespace gemm

@@ -1433,7 +1433,7 @@ void hold_wide(hgpu_ctx* ctx, std::shared_ptr<WideJob> job, int kernel, const ch
   hold_item_locked(ctx, std::move(d));
 }
 
-bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares) {
+bool join_wide_rows(hgpu_ctx* ctx, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares) {
   // (memory is taken with the queue unlocked: for want of it the allocator sends the queue out)
   std::shared_ptr<WideJob> job;
   {
@@ -1441,7 +1441,7 @@ bool join_wide_rows(hgpu_ctx* ctx, int n, const void* const* as, int64_t M, int6
     if (!ctx->dq) return false;
     if (factor && (!written_by(ctx->dq->items, {factor}).empty() || !written_by(ctx->dq->maps, {factor}).empty())) return false;
     for (auto& d : ctx->dq->items)
-      if (d.wide && (*shares = wide_row_shares(*d.wide, n, as, M, K, row_stride)) > 0) { job = d.wide; break; }
+      if (d.wide && (*shares = wide_row_shares(*d.wide, dtype, n, as, M, K, row_stride)) > 0) { job = d.wide; break; }
   }
   if (!job || buffer_alloc(ctx, (size_t)M * (size_t)*shares * 8, part)) return false;
   {
