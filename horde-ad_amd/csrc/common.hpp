@@ -280,15 +280,26 @@ bool wide_takes_rows(const WideJob& job);
 // smallk.hip: the sums over K of n terms of M rows of floats of `dtype`, each term times the one element `factor` (null: 1), as
 // *part (rows x *shares, doubles) by a held product that reads the same rows; false: there is none
 bool join_wide_rows(hgpu_ctx* ctx, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride, hgpu_buffer* factor_buf, const void* factor, hgpu_buffer** part, int* shares);
-// One gather of whole slices that may be held back (index.hip): its arguments and its result's block.
-struct GatherJob;
-hipError_t launch_gather(hgpu_ctx* ctx, const GatherJob& job);       // the caller holds launch_mu
-const char* gather_label(const GatherJob& job, double* bytes);
-// smallk.hip: holds the gather back (retaining the buffers) until something reads its result or writes to an array that exists;
-// it never runs if nobody has the result any more by then.  false: the caller launches it now (it reads held results)
-bool hold_gather(hgpu_ctx* ctx, const std::shared_ptr<GatherJob>& job, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write);
-// smallk.hip: the held gather that will write this block, if there is one (the caller holds launch_mu)
-std::shared_ptr<GatherJob> gather_into_locked(hgpu_ctx* ctx, const hgpu_buffer* b);
+// One launch that is held back by itself (a gather of whole slices, index.hip; a small objective's reductions, fused.hip).
+struct HeldJob {
+  const char* label = nullptr;
+  double bytes = 0, flops = 0;
+  virtual ~HeldJob() {}
+  virtual hipError_t launch(hgpu_ctx* ctx, hipEvent_t start, hipEvent_t stop) = 0;       // the caller holds launch_mu; events: null, or carried by the launch
+};
+// smallk.hip: holds the launch back (retaining the buffers) until something reads its results or writes to an array that exists;
+// it never runs if nobody has any of the results any more by then.  What it reads of held results goes out first, or, with
+// ready_only, it is not held (false: the caller launches it now).
+bool hold_job(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes, bool ready_only);
+// smallk.hip, the caller holds launch_mu: the held launch that will write this block, if there is one; a held launch reads and writes more
+std::shared_ptr<HeldJob> held_writer_locked(hgpu_ctx* ctx, const hgpu_buffer* b);
+bool extend_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);
+// ... goes out now; forgotten: it does not (another launch has done its work)
+void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, bool forgotten);
+// fused.hip: holds the extremum of one dense row back, to be one launch with the sums over the same elements that follow; false: left to the caller
+bool try_hold_extremum(hgpu_ctx* ctx, const hgpu_array* a, int want_max, const hgpu_array* index, const hgpu_array* value);
+// contract.hip: the extremum of one row by a block (the caller holds launch_mu)
+hipError_t launch_extremum_row(hgpu_ctx* ctx, int dtype, int64_t n, int want_max, const void* a, void* index, void* value);
 // index.hip: *o (one element) = sum of a * b, where a held gather is to write a or b and need not for this; *handled: taken
 int try_gather_dot(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, const hgpu_array* o, bool* handled);
 // smallk.hip: holds the product back (retaining the buffers) to be launched with those of the same kernel that do not depend on it

@@ -886,6 +886,16 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
 }  // namespace
 
 namespace hg {
+hipError_t launch_extremum_row(hgpu_ctx* ctx, int dtype, int64_t n, int want_max, const void* a, void* index, void* value) {
+  Dims keep;
+  memset(&keep, 0, sizeof keep);
+  keep.nd = 1;
+  for (auto& e : keep.shape) e = 1;
+  if (dtype == HGPU_F64) hipLaunchKernelGGL(k_argminmax_block<double>, dim3(1), dim3(1024), 0, ctx->stream, keep, n, (int64_t)1, want_max, (const double*)a, (int64_t*)index, (double*)value);
+  else hipLaunchKernelGGL(k_argminmax_block<float>, dim3(1), dim3(1024), 0, ctx->stream, keep, n, (int64_t)1, want_max, (const float*)a, (int64_t*)index, (float*)value);
+  return hipGetLastError();
+}
+
 static SumArgs sum_args(const RedJob& j) {
   SumArgs s;
   memset(&s, 0, sizeof s);
@@ -1575,6 +1585,11 @@ int hgpu_extremum_last(hgpu_ctx* ctx, const hgpu_array* a, int want_max, hgpu_ar
     const int64_t* ks[1] = {a->strides};
     Dims keep;
     if (!collapse(a->rank - 1, a->shape, 1, ks, &keep)) { hgpu_release(o); if (v) hgpu_release(v); return fail(ctx, HGPU_ERR_UNSUPPORTED, "argminmax: too many dims"); }
+    if (v && n_out == 1 && try_hold_extremum(ctx, a, want_max, o, v)) {
+      *out = o;
+      *values = v;
+      return HGPU_OK;
+    }
     const bool pieces = L >= kPiecesFrom && n_out <= kPiecesRows;
     void* tickets = nullptr;
     hgpu_buffer* scratch = nullptr;

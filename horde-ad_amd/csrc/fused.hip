@@ -58,13 +58,16 @@ int compile(hgpu_ctx* ctx, const std::string& src, Compiled* out, const char* kn
 
 // Kernels found again by what their text depends on (the inputs' layouts and the program).
 struct Known { Compiled c; std::string text; };
-const Known* find_known(hgpu_ctx* ctx, const Key& key) {
-  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
+const Known* find_known_locked(hgpu_ctx* ctx, const Key& key) {
   auto kit = ctx->jit_cache.find("__fused_known__");
   if (kit == ctx->jit_cache.end()) return nullptr;
   auto& known = *static_cast<std::unordered_map<std::string, Known>*>(kit->second);
   auto it = known.find(key.bytes);
   return it == known.end() ? nullptr : &it->second;
+}
+const Known* find_known(hgpu_ctx* ctx, const Key& key) {
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
+  return find_known_locked(ctx, key);
 }
 // The kernel of a call: the known one (`hit`; with HORDEAD_GPU_CHECK_KEYS its text is compared with the one just written),
 // else the one with the text `src`, compiled if need be and remembered under the key.  Call with launch_mu held.
@@ -725,6 +728,293 @@ template <typename A> __device__ __forceinline__ A sum_of_blocks(unsigned long l
 }
 )HG";
 
+// ---- the reductions of a small objective as one launch ------------------------------------------------------------
+//
+// A soft-max cross entropy asks, one after another, for the minimum of its logits, for the sum of their exponentials over it, and
+// for a pass that writes the cotangent and sums the objective's value.  Each is one block where the logits are few, with
+// two trips to memory and a launch for a microsecond of arithmetic.  The extremum waits (HeadJob); a sum that reads its value
+// from it, and a map with sums that reads those, join it; the last one launches them all as one block whose phases hand their
+// scalars on through registers.  Batches of 10 logits, us of the launches under the profiler: 150 fp64 5.4 + 4.7 + 5.3, so 8.6;
+// 250 fp32 5.4 + 4.6 + 4.6, so 7.3 (a training step 123.0 -> 119.7); 1000 fp64 6.5 + 4.8 + 4.8, so 19.6: a trip of 2048 elements is
+// 2.4 us of exponentials and logarithms on the one CU, hence the limit (loading every phase's first vectors before the first
+// changes nothing at these sizes, the arithmetic and its code do).
+constexpr int64_t kHeadMost = 32768;      // bytes
+constexpr size_t kHeadStages = 3;
+
+namespace {
+
+struct HeadStage {
+  int64_t n;
+  int vec;
+  std::vector<int> in_dt, from;          // from: an array (-1), one element in memory (-2), or the number of a scalar of an earlier phase
+  std::vector<const void*> in;
+  std::vector<hgpu_fused_instr> prog;
+  std::vector<int> dt, out_slots, asked;
+  std::vector<void*> outs, sums;
+  int sum_dt(size_t j) const { return dt[(size_t)(asked[j] & ~HGPU_SUM_PRODUCTS)]; }
+};
+
+struct HeadJob : HeldJob {
+  int dtype, want_max;
+  int64_t n;
+  const void* a;
+  void *index, *value;
+  std::vector<HeadStage> stages;
+  std::vector<const void*> scalars;      // where the scalars of the phases so far go
+  std::vector<int> scalar_dt;
+
+  // The arrays' first vectors of a lane, each loaded once, before the first phase: load k serves the inputs numbered k.
+  struct Load { const void* p; int dt, vec; int64_t n; std::string name, count; };
+  std::vector<Load> loads() const {
+    std::vector<Load> r{{a, dtype, 16 / (int)dtype_size(dtype), n, "a", "n"}};
+    for (size_t k = 0; k < stages.size(); ++k)
+      for (size_t i = 0; i < stages[k].in.size(); ++i)
+        if (stages[k].from[i] == -1 && load_of(r, k, i) == (int)r.size())
+          r.push_back({stages[k].in[i], stages[k].in_dt[i], stages[k].vec, stages[k].n, "i" + std::to_string(k) + "_" + std::to_string(i), "n" + std::to_string(k)});
+    return r;
+  }
+  int load_of(const std::vector<Load>& r, size_t k, size_t i) const {
+    const HeadStage& st = stages[k];
+    size_t q = 0;
+    while (q < r.size() && !(r[q].p == st.in[i] && r[q].dt == st.in_dt[i] && r[q].vec == st.vec && r[q].n == st.n)) ++q;
+    return (int)q;
+  }
+
+  Key key() const {
+    Key k;
+    const std::vector<Load> ld = loads();
+    k.put(std::string("fused_head")).put(dtype).put(want_max).put(stages.size());
+    for (size_t j = 0; j < stages.size(); ++j) {
+      const HeadStage& st = stages[j];
+      k.put(st.vec).put(st.in_dt).put(st.from).put((int)st.prog.size(), st.prog.data()).put(st.out_slots).put(st.asked);
+      for (size_t i = 0; i < st.in.size(); ++i) k.put(st.from[i] == -1 ? load_of(ld, j, i) : -1);
+    }
+    return k;
+  }
+
+  void write(Src& s) const {
+    const char* T = ctype(dtype);
+    s << kPrelude;
+    s << "template <typename T, int N> struct alignas(sizeof(T) * N) Vec { T v[N]; };\n"
+         "template <typename A> __device__ __forceinline__ A from_lane(A v, int off) {\n"
+         "  unsigned long long u = 0;\n"
+         "  __builtin_memcpy(&u, &v, sizeof(A));\n"
+         "  const unsigned lo = __shfl_down((unsigned)(u & 0xffffffffu), off, 64), hi = __shfl_down((unsigned)(u >> 32), off, 64);\n"
+         "  u = ((unsigned long long)hi << 32) | lo;\n"
+         "  __builtin_memcpy(&v, &u, sizeof(A));\n"
+         "  return v;\n}\n"
+         "template <typename A> __device__ __forceinline__ A block_sum(A v, unsigned long long* red) {\n"
+         "  for (int off = 32; off > 0; off >>= 1) v += from_lane(v, off);\n"
+         "  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = *reinterpret_cast<unsigned long long*>(&v);\n"
+         "  __syncthreads();\n"
+         "  A tot = 0;\n"
+         "  for (int k = 0; k < 16; ++k) tot += *reinterpret_cast<A*>(&red[k]);\n"
+         "  __syncthreads();\n"
+         "  return tot;\n}\n";
+    // (the rules of k_argminmax_block: a NaN is no candidate, but in the first place; the smaller index wins)
+    s << "#define NONE 0x7fffffffffffffffll\n"
+         "template <typename T> __device__ __forceinline__ bool takes(T x, T best, i64 bi) { return bi == NONE ? x == x : x " << (want_max ? ">" : "<") << " best; }\n";
+    s << "extern \"C\" __global__ void __launch_bounds__(1024) fused_head(i64 n, const " << T << "* __restrict__ a, i64* __restrict__ index, " << T << "* __restrict__ value";
+    for (size_t k = 0; k < stages.size(); ++k) {
+      const HeadStage& st = stages[k];
+      s << ", i64 n" << k;
+      for (size_t i = 0; i < st.in.size(); ++i)
+        if (st.from[i] < 0) s << ", const " << ctype(st.in_dt[i]) << "* __restrict__ i" << k << "_" << i;
+      for (size_t o = 0; o < st.outs.size(); ++o) s << ", " << ctype(st.dt[(size_t)st.out_slots[o]]) << "* __restrict__ o" << k << "_" << o;
+      for (size_t j = 0; j < st.sums.size(); ++j) s << ", " << ctype(st.sum_dt(j)) << "* __restrict__ sum" << k << "_" << j;
+    }
+    s << ") {\n  __shared__ unsigned long long red[16];\n  __shared__ i64 at[16];\n  const int t = threadIdx.x, w = t >> 6;\n";
+    const int vec = 16 / (int)dtype_size(dtype);
+    const std::vector<Load> ld = loads();
+    for (size_t q = 0; q < ld.size(); ++q)
+      s << "  typedef Vec<" << ctype(ld[q].dt) << ", " << ld[q].vec << "> F" << q << ";\n  F" << q << " f" << q << ";\n  if (t < " << ld[q].count << " / " << ld[q].vec << ") f" << q
+        << " = reinterpret_cast<const F" << q << "*>(" << ld[q].name << ")[t];\n";
+    for (size_t k = 0; k < stages.size(); ++k)
+      for (size_t i = 0; i < stages[k].in.size(); ++i)
+        if (stages[k].from[i] == -2) s << "  const " << ctype(stages[k].in_dt[i]) << " s" << k << "_" << i << " = i" << k << "_" << i << "[0];\n";
+    s << "  " << T << " h0;\n  {\n    typedef Vec<" << T << ", " << vec << "> V;\n    " << T << " best = 0;\n    i64 bi = NONE;\n    const i64 nv = n / " << vec << ";\n"
+         "    const " << T << " first = a[0];\n    i64 i = t;\n    V l = f0;\n"
+         "    for (; i < nv; i += 1024) {\n      const V c = l;\n      if (i + 1024 < nv) l = reinterpret_cast<const V*>(a)[i + 1024];\n"
+         "      for (int e = 0; e < " << vec << "; ++e)\n        if (takes(c.v[e], best, bi)) { best = c.v[e]; bi = i * " << vec << " + e; }\n    }\n"
+         "    i = nv * " << vec << " + t;\n    if (i < n && takes(a[i], best, bi)) { best = a[i]; bi = i; }\n"
+         "    for (int off = 32; off > 0; off >>= 1) {\n      const " << T << " ob = from_lane(best, off);\n      const i64 oi = from_lane(bi, off);\n"
+         "      if (oi != NONE && (takes(ob, best, bi) || (ob == best && oi < bi))) { best = ob; bi = oi; }\n    }\n"
+         "    if ((t & 63) == 0) { unsigned long long u = 0; __builtin_memcpy(&u, &best, sizeof best); red[w] = u; at[w] = bi; }\n    __syncthreads();\n"
+         "    __builtin_memcpy(&best, &red[0], sizeof best);\n    bi = at[0];\n"
+         "    for (int k = 1; k < 16; ++k) {\n      " << T << " ob;\n      __builtin_memcpy(&ob, &red[k], sizeof ob);\n      const i64 oi = at[k];\n"
+         "      if (oi != NONE && (takes(ob, best, bi) || (ob == best && oi < bi))) { best = ob; bi = oi; }\n    }\n    __syncthreads();\n"
+         "    const bool keep_first = !(first == first);\n    h0 = keep_first ? first : best;\n    if (t == 0) { value[0] = h0; index[0] = keep_first ? 0 : bi; }\n  }\n";
+    int next = 1;
+    for (size_t k = 0; k < stages.size(); ++k) {
+      const HeadStage& st = stages[k];
+      const int n_in = (int)st.in.size(), n_instr = (int)st.prog.size();
+      auto acc_t = [&](size_t j) { return dtype_is_float(st.sum_dt(j)) ? "double" : "i64"; };
+      for (size_t j = 0; j < st.sums.size(); ++j) s << "  " << ctype(st.sum_dt(j)) << " h" << next + (int)j << ";\n";
+      s << "  {\n    const i64 nv = n" << k << " / " << st.vec << ";\n    i64 i = t;\n";
+      for (int i = 0; i < n_in; ++i) {
+        if (st.from[(size_t)i] == -1) s << "    typedef Vec<" << ctype(st.in_dt[(size_t)i]) << ", " << st.vec << "> V" << i << ";\n    V" << i << " l" << i << " = f" << load_of(ld, k, (size_t)i) << ";\n";
+        else if (st.from[(size_t)i] == -2) s << "    const " << ctype(st.in_dt[(size_t)i]) << " s" << i << " = s" << k << "_" << i << ";\n";
+        else s << "    const " << ctype(st.in_dt[(size_t)i]) << " s" << i << " = h" << st.from[(size_t)i] << ";\n";
+      }
+      for (size_t j = 0; j < st.sums.size(); ++j) s << "    " << acc_t(j) << " acc" << j << " = 0;\n";
+      auto fetch = [&](const char* ind, const char* where) {
+        for (int i = 0; i < n_in; ++i)
+          if (st.from[(size_t)i] == -1) s << ind << "l" << i << " = reinterpret_cast<const V" << i << "*>(i" << k << "_" << i << ")[" << where << "];\n";
+      };
+      s << "    for (; i < nv; i += 1024) {\n";
+      for (int i = 0; i < n_in; ++i)
+        if (st.from[(size_t)i] == -1) s << "      const V" << i << " c" << i << " = l" << i << ";\n";
+      s << "      if (i + 1024 < nv) {\n";
+      fetch("        ", "i + 1024");
+      s << "      }\n";
+      for (size_t o = 0; o < st.outs.size(); ++o) s << "      Vec<" << ctype(st.dt[(size_t)st.out_slots[o]]) << ", " << st.vec << "> r" << o << ";\n";
+      auto element = [&](const char* ind, const std::string& suf, int e) {      // e < 0: one of the few behind the last whole vector
+        for (int i = 0; i < n_in; ++i) {
+          s << ind << "const " << ctype(st.in_dt[(size_t)i]) << " v" << i << suf << " = ";
+          if (st.from[(size_t)i] != -1) s << "s" << i;
+          else if (e >= 0) s << "c" << i << ".v[" << e << "]";
+          else s << "i" << k << "_" << i << "[i]";
+          s << ";\n";
+        }
+        emit_program(s, n_in, n_instr, st.prog.data(), st.dt, ind, suf);
+        for (size_t o = 0; o < st.outs.size(); ++o) {
+          if (e >= 0) s << ind << "r" << o << ".v[" << e << "]";
+          else s << ind << "o" << k << "_" << o << "[i]";
+          s << " = v" << st.out_slots[o] << suf << ";\n";
+        }
+        for (size_t j = 0; j < st.sums.size(); ++j) s << ind << "acc" << j << " += (" << acc_t(j) << ")" << summand(n_in, st.prog.data(), st.dt, st.asked[j], suf) << ";\n";
+      };
+      for (int e = 0; e < st.vec; ++e) {
+        s << "      {\n";
+        element("        ", "_" + std::to_string(e), e);
+        s << "      }\n";
+      }
+      for (size_t o = 0; o < st.outs.size(); ++o)
+        s << "      reinterpret_cast<Vec<" << ctype(st.dt[(size_t)st.out_slots[o]]) << ", " << st.vec << ">*>(o" << k << "_" << o << ")[i] = r" << o << ";\n";
+      s << "    }\n    i = nv * " << st.vec << " + t;\n    if (i < n" << k << ") {\n";
+      element("      ", "_t", -1);
+      s << "    }\n";
+      for (size_t j = 0; j < st.sums.size(); ++j)
+        s << "    h" << next + (int)j << " = (" << ctype(st.sum_dt(j)) << ")block_sum(acc" << j << ", red);\n    if (t == 0) sum" << k << "_" << j << "[0] = h" << next + (int)j << ";\n";
+      s << "  }\n";
+      next += (int)st.sums.size();
+    }
+    s << "}\n";
+  }
+
+  hipError_t launch(hgpu_ctx* ctx, hipEvent_t start, hipEvent_t stop) override {
+    if (stages.empty()) {
+      if (start) (void)hipEventRecord(start, ctx->stream);
+      const hipError_t e = launch_extremum_row(ctx, dtype, n, want_max, a, index, value);
+      if (stop) (void)hipEventRecord(stop, ctx->stream);
+      return e;
+    }
+    const Key kk = key();
+    const Known* hit = find_known_locked(ctx, kk);
+    Src s(!hit || check_keys());
+    if (s.on) write(s);
+    Compiled kernel;
+    if (kernel_for(ctx, kk, hit, s.str(), "fused_head", &kernel)) return hipErrorInvalidImage;
+    std::vector<void*> args{&n, &a, &index, &value};
+    for (auto& st : stages) {
+      args.push_back(&st.n);
+      for (size_t i = 0; i < st.in.size(); ++i)
+        if (st.from[i] < 0) args.push_back(&st.in[i]);
+      for (auto& o : st.outs) args.push_back(&o);
+      for (auto& o : st.sums) args.push_back(&o);
+    }
+    note_recorded(ctx, kernel.fn);
+    return start || stop ? hipExtModuleLaunchKernel(kernel.fn, 1024, 1, 1, 1024, 1, 1, 0, ctx->stream, args.data(), nullptr, start, stop, 0)
+                         : hipModuleLaunchKernel(kernel.fn, 1, 1, 1, 1024, 1, 1, 0, ctx->stream, args.data(), nullptr);
+  }
+};
+
+// A pass over arrays of n elements (layout: 'd' dense and aligned, 's' one element) joins the held launch that one of its single
+// elements comes from, with its results in outs and sums; last: the launch goes out with it.
+bool join_head(hgpu_ctx* ctx, int64_t n, int n_in, const hgpu_array* const* in, const std::string& layout, int n_instr, const hgpu_fused_instr* prog, const std::vector<int>& dt,
+               int n_out, const int* out_slots, hgpu_array* const* outs, int n_sum, const int* asked, hgpu_array* const* sums, int vec, bool last) {
+  if (n < 1) return false;
+  std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
+  if (!ctx->dq_pending) return false;
+  std::shared_ptr<HeadJob> job;
+  for (int i = 0; i < n_in && !job; ++i)
+    if (layout[(size_t)i] == 's') job = std::dynamic_pointer_cast<HeadJob>(held_writer_locked(ctx, in[i]->buf));
+  if (!job || n > job->n || job->stages.size() >= kHeadStages - 1) return false;
+  HeadStage st;
+  st.n = n;
+  st.vec = vec;
+  Reads reads;
+  std::vector<hgpu_buffer*> read, write;
+  for (int i = 0; i < n_in; ++i) {
+    int from = layout[(size_t)i] == 's' ? -2 : -1;
+    if (held_writer_locked(ctx, in[i]->buf) == job) {
+      const auto at = std::find(job->scalars.begin(), job->scalars.end(), data_ptr(in[i]));
+      if (from != -2 || at == job->scalars.end()) return false;      // (the place of the extremum)
+      from = (int)(at - job->scalars.begin());
+      if (job->scalar_dt[(size_t)from] != in[i]->dtype) return false;
+    } else {
+      reads.push_back(data_ptr(in[i]));
+      read.push_back(in[i]->buf);
+    }
+    st.from.push_back(from);
+    st.in.push_back(data_ptr(in[i]));
+    st.in_dt.push_back(in[i]->dtype);
+  }
+  make_way_locked(ctx, reads);
+  st.prog.assign(prog, prog + n_instr);
+  st.dt = dt;
+  for (int o = 0; o < n_out; ++o) {
+    st.out_slots.push_back(out_slots[o]);
+    st.outs.push_back(data_ptr(outs[o]));
+    write.push_back(outs[o]->buf);
+  }
+  for (int j = 0; j < n_sum; ++j) {
+    st.asked.push_back(asked[j]);
+    st.sums.push_back(data_ptr(sums[j]));
+    write.push_back(sums[j]->buf);
+  }
+  if (!extend_job_locked(ctx, job, read, write)) return false;       // (it has gone out with what was in the way)
+  for (int j = 0; j < n_sum; ++j) {
+    job->scalars.push_back(st.sums[(size_t)j]);
+    job->scalar_dt.push_back(st.sum_dt((size_t)j));
+  }
+  job->stages.push_back(std::move(st));
+  job->label = "fused_head";
+  for (int i = 0; i < n_in; ++i)
+    if (layout[(size_t)i] == 'd') job->bytes += (double)n * (double)dtype_size(in[i]->dtype);
+  for (int o = 0; o < n_out; ++o) job->bytes += (double)n * (double)dtype_size(outs[o]->dtype);
+  job->flops += (double)n * (n_instr + n_sum);
+  if (ctx->profiling && ctx->profile_shapes) {
+    char buf[96];
+    snprintf(buf, sizeof buf, "fused_head[%lld,phases%d]", (long long)n, (int)job->stages.size() + 1);
+    job->label = intern_label(ctx, buf);
+  }
+  if (last) end_job_locked(ctx, job, false);
+  return true;
+}
+
+}  // namespace
+
+namespace hg {
+bool try_hold_extremum(hgpu_ctx* ctx, const hgpu_array* a, int want_max, const hgpu_array* index, const hgpu_array* value) {
+  const int64_t n = nelem(a);
+  if (!dtype_is_float(a->dtype) || n < 64 || n * (int64_t)dtype_size(a->dtype) > kHeadMost || !is_dense(a) || ((uintptr_t)data_ptr(a) & 15) != 0) return false;
+  auto job = std::make_shared<HeadJob>();
+  job->label = "argminmax";
+  job->bytes = (double)n * (double)dtype_size(a->dtype);
+  job->flops = (double)n;
+  job->dtype = a->dtype;
+  job->want_max = want_max;
+  job->n = n;
+  job->a = data_ptr(a);
+  job->index = data_ptr(index);
+  job->value = data_ptr(value);
+  job->scalars = {job->value};
+  job->scalar_dt = {a->dtype};
+  return hold_job(ctx, job, {a->buf}, {index->buf, value->buf}, false);
+}
+}  // namespace hg
+
 // The sum of all elements of an elementwise program's result, evaluated on the
 // fly (the result is never written): per-block partial sums in double / int64,
 // added up in a fixed order by the block that finishes last.  Inputs must be dense
@@ -763,6 +1053,7 @@ extern "C" int hgpu_fused_sum(hgpu_ctx* ctx, int n_in, const hgpu_array* const* 
   int rc = n == 0 ? new_zeros(ctx, odt, 0, nullptr, &o) : new_dense(ctx, odt, 0, nullptr, &o);   // the last launch writes it
   if (rc) return rc;
   if (n == 0) { *out = o; return HGPU_OK; }
+  if (join_head(ctx, n, n_in, in, layout, n_instr, prog, dt, 0, nullptr, nullptr, 1, &asked, &o, vec, false)) { *out = o; return HGPU_OK; }
   const bool fp = dtype_is_float(odt);
   const char* acc = fp ? "double" : "i64";
   // Very few elements: one block of 1024 threads sums them and writes the result.
@@ -941,6 +1232,11 @@ extern "C" int hgpu_fused_map_sums(hgpu_ctx* ctx, int n_in, const hgpu_array* co
     widest = std::max(widest, dtype_size(dt[(size_t)sum_slots[j]]));
   }
   const int vec = (int)(16 / widest);
+  if (join_head(ctx, n, n_in, in, layout, n_instr, prog, dt, n_out, out_slots, res.data(), n_sum, asked, sres.data(), vec, true)) {
+    for (int o = 0; o < n_out; ++o) outs[o] = res[(size_t)o];
+    for (int j = 0; j < n_sum; ++j) sums[j] = sres[(size_t)j];
+    return HGPU_OK;
+  }
   // Very few elements: one block of 1024 threads writes the outputs and the finished sums.
   const bool single = (n + vec - 1) / vec <= 1024;
   const int NT = single ? 1024 : 256;

@@ -1013,29 +1013,27 @@ int build_space(hgpu_ctx* ctx, const char* who, int n_ix, const hgpu_array* cons
 
 namespace hg {
 
-struct GatherJob {
+struct GatherJob : HeldJob {
   IxSpace sp;
   int64_t M, N, units, epu;     // positions, elements of a slice; of `unit` bytes each: units of a slice, elements of a unit
   int unit;                     // 0: element by element
   int dtype;
   const void* src;
   void* out;
-  const char* label;
-  double bytes;
+  hipError_t launch(hgpu_ctx* ctx, hipEvent_t start, hipEvent_t stop) override {
+    const dim3 g(grid_for(M * units, kBlock, ctx->num_cu * 16));
+    auto go = [&](auto* u) {
+      using U = std::remove_pointer_t<decltype(u)>;
+      if (start || stop) hipExtLaunchKernelGGL(k_gather_units<U>, g, dim3(kBlock), 0, ctx->stream, start, stop, 0, sp, M, units, epu, (const U*)src, (U*)out);
+      else hipLaunchKernelGGL(k_gather_units<U>, g, dim3(kBlock), 0, ctx->stream, sp, M, units, epu, (const U*)src, (U*)out);
+    };
+    if (unit == 16) go((uint4*)nullptr);
+    else if (unit == 8) go((uint64_t*)nullptr);
+    else go((uint32_t*)nullptr);
+    return hipGetLastError();
+  }
 };
-
-hipError_t launch_gather(hgpu_ctx* ctx, const GatherJob& j) {
-  const unsigned g = grid_for(j.M * j.units, kBlock, ctx->num_cu * 16);
-  if (j.unit == 16) hipLaunchKernelGGL(k_gather_units<uint4>, dim3(g), dim3(kBlock), 0, ctx->stream, j.sp, j.M, j.units, j.epu, (const uint4*)j.src, (uint4*)j.out);
-  else if (j.unit == 8) hipLaunchKernelGGL(k_gather_units<uint64_t>, dim3(g), dim3(kBlock), 0, ctx->stream, j.sp, j.M, j.units, j.epu, (const uint64_t*)j.src, (uint64_t*)j.out);
-  else hipLaunchKernelGGL(k_gather_units<uint32_t>, dim3(g), dim3(kBlock), 0, ctx->stream, j.sp, j.M, j.units, j.epu, (const uint32_t*)j.src, (uint32_t*)j.out);
-  return hipGetLastError();
-}
-
-const char* gather_label(const GatherJob& j, double* bytes) {
-  *bytes = j.bytes;
-  return j.label;
-}
+std::shared_ptr<GatherJob> gather_into_locked(hgpu_ctx* ctx, const hgpu_buffer* b) { return std::dynamic_pointer_cast<GatherJob>(held_writer_locked(ctx, b)); }
 
 // The held gather's result must be all of a or b, side by side, and the other operand dense too: then both run along the same
 // linear index.  The gather stays held; it is dropped if nobody else has its result.
@@ -1145,12 +1143,23 @@ int hgpu_gather(hgpu_ctx* ctx, const hgpu_array* src, int n_ix, const hgpu_array
       }
     }
     if (unit) {
-      auto job = std::make_shared<GatherJob>(GatherJob{sp, M, N, N * es / unit, unit / es, unit, src->dtype, data_ptr(src), data_ptr(o), label, bytes});
+      auto job = std::make_shared<GatherJob>();
+      job->label = label;
+      job->bytes = bytes;
+      job->sp = sp;
+      job->M = M;
+      job->N = N;
+      job->units = N * es / unit;
+      job->epu = unit / es;
+      job->unit = unit;
+      job->dtype = src->dtype;
+      job->src = data_ptr(src);
+      job->out = data_ptr(o);
       std::vector<hgpu_buffer*> read{src->buf};
       for (int k = 0; k < n_ix; ++k) read.push_back(ix[k]->buf);
-      if (floats && hold_gather(ctx, job, read, o->buf)) { *out = o; return HGPU_OK; }
+      if (floats && hold_job(ctx, job, read, {o->buf}, true)) { *out = o; return HGPU_OK; }
       LaunchGuard lg(ctx, label, bytes, 0);      // (integers, or a gather that reads held results)
-      const hipError_t e = launch_gather(ctx, *job);
+      const hipError_t e = job->launch(ctx, lg.start_event(), lg.stop_event());
       if (e != hipSuccess) { hgpu_release(o); return check_hip(ctx, e, "gather"); }
       *out = o;
       return HGPU_OK;

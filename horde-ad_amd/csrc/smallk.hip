@@ -759,9 +759,9 @@ struct DeferredQueue {
   std::vector<Deferred> items;
   enum Kind { kProducts, kCopies } kind = kProducts;     // what `items` holds
   std::vector<Deferred> maps;
-  struct Gather { std::shared_ptr<GatherJob> job; std::vector<hgpu_buffer*> reads; hgpu_buffer* write; };
-  std::vector<Gather> gathers;       // they read no held result, and nothing held reads theirs
-  bool any() const { return !items.empty() || !maps.empty() || !gathers.empty(); }
+  struct Single { std::shared_ptr<HeldJob> job; std::vector<hgpu_buffer*> reads, writes; };
+  std::vector<Single> singles;       // they read no held result, and nothing held reads theirs
+  bool any() const { return !items.empty() || !maps.empty() || !singles.empty(); }
   std::map<size_t, int> seen;        // how often a set of problems came up together, by the hash of their ids, grids and LDS bytes
   long n_launches = 0, n_grouped = 0;
   size_t held_bytes = 0;             // of the blocks that items and maps keep
@@ -1285,49 +1285,52 @@ static void flush_items_locked(hgpu_ctx* ctx) {
   if (ctx->dq->items.empty()) ctx->dq->items.swap(items);      // (its memory is kept: an item is a kilobyte to move)
 }
 
-// The held gathers that `take` names go out; one whose result only the queue has left is forgotten.
+// The launches held by themselves that `take` names go out; one whose results only the queue has left is forgotten.
 template <typename F>
-static void flush_gathers_locked(hgpu_ctx* ctx, const F& take) {
+static void flush_singles_locked(hgpu_ctx* ctx, const F& take) {
   DeferredQueue& q = *ctx->dq;
-  std::vector<DeferredQueue::Gather> out;
-  for (size_t i = 0; i < q.gathers.size();) {
-    if (!take(q.gathers[i])) { ++i; continue; }
-    out.push_back(std::move(q.gathers[i]));
-    q.gathers.erase(q.gathers.begin() + (long)i);
+  std::vector<DeferredQueue::Single> out;
+  for (size_t i = 0; i < q.singles.size();) {
+    if (!take(q.singles[i])) { ++i; continue; }
+    out.push_back(std::move(q.singles[i]));
+    q.singles.erase(q.singles.begin() + (long)i);
   }
   ctx->dq_pending = q.any();
   if (!out.empty()) (void)hipSetDevice(ctx->device);
   for (auto& g : out) {
-    if (g.write->refs.load() > 1) {
-      hgpu_ctx::ProfRec r{nullptr, nullptr, nullptr, 0, 0};
-      r.name = gather_label(*g.job, &r.bytes);
-      ctx->count_recorded(r.name, r.bytes, 0);
+    bool wanted = false;
+    for (auto* b : g.writes) wanted = wanted || b->refs.load() > 1;
+    if (wanted) {
+      HeldJob& j = *g.job;
+      hgpu_ctx::ProfRec r{j.label, nullptr, nullptr, j.bytes, j.flops};
+      ctx->count_recorded(j.label, j.bytes, j.flops);
       const bool timed = ctx->profiling && !ctx->cap && hipEventCreate(&r.a) == hipSuccess && hipEventCreate(&r.b) == hipSuccess;
-      if (timed) (void)hipEventRecord(r.a, ctx->stream);
-      const hipError_t e = launch_gather(ctx, *g.job);
-      if (timed) {
-        (void)hipEventRecord(r.b, ctx->stream);
-        ctx->prof.push_back(r);
-      }
+      const hipError_t e = j.launch(ctx, timed ? r.a : nullptr, timed ? r.b : nullptr);
+      if (timed) ctx->prof.push_back(r);
       if (e != hipSuccess) {
-        int rc = check_hip(ctx, e, "gather launch");
+        int rc = check_hip(ctx, e, j.label);
         if (!ctx->deferred_rc) ctx->deferred_rc = rc;
       }
     }
     for (auto* b : g.reads) q.let_go(b);
-    q.let_go(g.write);
+    for (auto* b : g.writes) q.let_go(b);
   }
 }
-static void flush_gathers_locked(hgpu_ctx* ctx) { flush_gathers_locked(ctx, [](const DeferredQueue::Gather&) { return true; }); }
+static void flush_singles_locked(hgpu_ctx* ctx) { flush_singles_locked(ctx, [](const DeferredQueue::Single&) { return true; }); }
 // ... those whose results a launch that reads `blocks` needs.
-static void gathers_for_locked(hgpu_ctx* ctx, const std::vector<hgpu_buffer*>& blocks) {
-  if (!ctx->dq->gathers.empty()) flush_gathers_locked(ctx, [&](const DeferredQueue::Gather& g) { return std::find(blocks.begin(), blocks.end(), g.write) != blocks.end(); });
+static void singles_for_locked(hgpu_ctx* ctx, const std::vector<hgpu_buffer*>& blocks) {
+  if (ctx->dq->singles.empty()) return;
+  flush_singles_locked(ctx, [&](const DeferredQueue::Single& g) {
+    for (auto* w : g.writes)
+      if (std::find(blocks.begin(), blocks.end(), w) != blocks.end()) return true;
+    return false;
+  });
 }
 
 void flush_deferred_locked(hgpu_ctx* ctx) {
   ctx->dq_pending = false;
   if (!ctx->dq) return;
-  flush_gathers_locked(ctx);
+  flush_singles_locked(ctx);
   flush_items_locked(ctx);
   flush_maps_locked(ctx);
 }
@@ -1348,7 +1351,7 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
   DeferredQueue& q = *ctx->dq;
   for (auto* b : d.reads) q.keep(b);
   for (auto* b : d.writes) q.keep(b);
-  gathers_for_locked(ctx, d.reads);
+  singles_for_locked(ctx, d.reads);
   if (q.items.size() >= kMaxHeld || q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);
   if (!q.maps.empty()) {
     Reads reads;
@@ -1365,10 +1368,11 @@ static void hold_item_locked(hgpu_ctx* ctx, Deferred&& d) {
 // as before: their groups and chains are found among all of them.
 void make_way_locked(hgpu_ctx* ctx, const Reads& reads) {
   DeferredQueue& q = *ctx->dq;
-  if (!q.gathers.empty())
-    flush_gathers_locked(ctx, [&](const DeferredQueue::Gather& g) {
-      for (const void* r : reads)
-        if (r >= g.write->ptr && r < (const char*)g.write->ptr + g.write->bytes) return true;
+  if (!q.singles.empty())
+    flush_singles_locked(ctx, [&](const DeferredQueue::Single& g) {
+      for (auto* w : g.writes)
+        for (const void* r : reads)
+          if (r >= w->ptr && r < (const char*)w->ptr + w->bytes) return true;
       return false;
     });
   if (q.kind != DeferredQueue::kProducts) {
@@ -1467,7 +1471,7 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
   DeferredQueue& q = *ctx->dq;
   Reads from;
   for (auto* b : reads) from.push_back(b->ptr);
-  gathers_for_locked(ctx, reads);
+  singles_for_locked(ctx, reads);
   // (one reduction asked for sends them all: the next passes, an optimizer's, will ask for the others)
   if (q.kind != DeferredQueue::kProducts || !written_by(q.items, from).empty()) flush_items_locked(ctx);
   if (q.maps.size() >= kMaxHeld || !written_by(q.maps, from).empty()) flush_maps_locked(ctx);
@@ -1496,7 +1500,7 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   DeferredQueue& q = *ctx->dq;
   q.keep(src);
   q.keep(dst);
-  flush_gathers_locked(ctx);      // (they may read what the copy writes)
+  flush_singles_locked(ctx);      // (they may read what the copy writes)
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
   bool fits = q.maps.empty() && (q.items.empty() || (q.kind == DeferredQueue::kCopies && q.items.size() < (size_t)kMaxCopyJobs));
   for (size_t i = 0; fits && i < q.items.size(); ++i) {
@@ -1510,34 +1514,69 @@ void hold_copy(hgpu_ctx* ctx, const CopyJob& job, hgpu_buffer* src, hgpu_buffer*
   if (!hold) flush_deferred_locked(ctx);
 }
 
-// The held gathers at most: results that nobody has read yet, each with its block.
-constexpr size_t kMaxHeldGathers = 4;
+// Launches held by themselves, at most: results that nobody has read yet, each with its block.
+constexpr size_t kMaxSingles = 4;
 
-bool hold_gather(hgpu_ctx* ctx, const std::shared_ptr<GatherJob>& job, const std::vector<hgpu_buffer*>& reads, hgpu_buffer* write) {
+bool hold_job(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes, bool ready_only) {
   static const bool hold = getenv("HORDEAD_NO_GROUPED_LAUNCH") == nullptr;
-  if (!hold || !write) return false;
+  if (!hold) return false;
+  for (auto* b : writes)
+    if (!b) return false;
   std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
   if (!ctx->dq) ctx->dq = new DeferredQueue;
   DeferredQueue& q = *ctx->dq;
   if (q.kind != DeferredQueue::kProducts) flush_deferred_locked(ctx);      // copies into arrays that exist
-  gathers_for_locked(ctx, reads);
   Reads from;
   for (auto* b : reads) from.push_back(b->ptr);
-  if (!written_by(q.items, from).empty() || !written_by(q.maps, from).empty()) return false;
-  if (q.gathers.size() >= kMaxHeldGathers) flush_gathers_locked(ctx);
+  if (ready_only) {
+    singles_for_locked(ctx, reads);
+    if (!written_by(q.items, from).empty() || !written_by(q.maps, from).empty()) return false;
+  } else if (q.any()) {
+    make_way_locked(ctx, from);
+  }
+  if (q.singles.size() >= kMaxSingles) flush_singles_locked(ctx);
   for (auto* b : reads) q.keep(b);
-  q.keep(write);
-  q.gathers.push_back({job, reads, write});
+  for (auto* b : writes) q.keep(b);
+  q.singles.push_back({job, reads, writes});
   ctx->dq_pending = true;
   if (q.held_bytes > kMaxHeldBytes) flush_deferred_locked(ctx);
   return true;
 }
 
-std::shared_ptr<GatherJob> gather_into_locked(hgpu_ctx* ctx, const hgpu_buffer* b) {
+std::shared_ptr<HeldJob> held_writer_locked(hgpu_ctx* ctx, const hgpu_buffer* b) {
   if (ctx->dq)
-    for (auto& g : ctx->dq->gathers)
-      if (g.write == b) return g.job;
+    for (auto& g : ctx->dq->singles)
+      if (std::find(g.writes.begin(), g.writes.end(), b) != g.writes.end()) return g.job;
   return nullptr;
+}
+
+bool extend_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes) {
+  if (ctx->dq)
+    for (auto& g : ctx->dq->singles) {
+      if (g.job != job) continue;
+      for (auto* b : reads) { ctx->dq->keep(b); g.reads.push_back(b); }
+      for (auto* b : writes) { ctx->dq->keep(b); g.writes.push_back(b); }
+      return true;
+    }
+  return false;
+}
+
+void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, bool forgotten) {
+  if (!ctx->dq) return;
+  DeferredQueue& q = *ctx->dq;
+  if (!forgotten) {
+    flush_singles_locked(ctx, [&](const DeferredQueue::Single& g) { return g.job == job; });
+    return;
+  }
+  for (size_t i = 0; i < q.singles.size(); ++i) {
+    if (q.singles[i].job != job) continue;
+    DeferredQueue::Single g = std::move(q.singles[i]);
+    q.singles.erase(q.singles.begin() + (long)i);
+    for (auto* b : g.reads) q.let_go(b);
+    for (auto* b : g.writes) q.let_go(b);
+    break;
+  }
+  ctx->dq_pending = q.any();
 }
 
 void flush_deferred(hgpu_ctx* ctx) {
