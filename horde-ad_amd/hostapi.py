@@ -1,4 +1,5 @@
-"""ctypes binding of include/hordead_host.h (libhordead_host.so).
+"""Binding of include/hordead_host.h (libhordead_host.so): values and their operations through the CPython extension
+`lib/_pyvalues.so` (host/pyvalues.cpp), everything else through ctypes.
 
 `Host` is a context of the host layer on some provider of the array ABI, `V` a
 tensor value whose methods carry the names of horde-ad's tensor operations
@@ -8,6 +9,9 @@ operators, so that an index function is written as a lambda exactly like the
 reference's `\\[i, k] -> [i + k]` and is called once, symbolically.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
+import os
 
 import numpy as np
 
@@ -47,19 +51,51 @@ SIG = {
     "adam_apply": (I, [P, P, D, D, D, P, P, P, P, PP, PP, PP]),
 }
 
+def _extension():
+    path = os.path.join(capi.HERE, "lib", "_pyvalues.so")
+    loader = importlib.machinery.ExtensionFileLoader("_pyvalues", path)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_pyvalues", path, loader=loader))
+    loader.exec_module(mod)
+    return mod
+
+
+_py = _extension()
 _dll = None
+# entry points called through the extension: name -> (arguments, result); pyvalues.cpp says what the letters are
+NATIVE = {
+    "tape_reset": ("", "N"), "constant": ("idS", "V"), "ewise1": ("iv", "V"), "ewise2": ("ivv", "V"), "compare": ("ivv", "V"),
+    "select": ("vvv", "V"), "convert": ("vii", "V"), "tssumN": ("vi", "V"), "tssum0": ("v", "V"), "tsdot0": ("vv", "V"),
+    "tsdot1In": ("vv", "V"), "tsdotNIn": ("vvi", "V"), "tD": ("vv", "V"), "tprimalPart": ("v", "V"), "as_input": ("v", "V"),
+    "tsmatvecmul": ("vv", "V"), "tsmatmul2": ("vv", "V"), "tsreplicateN": ("vS", "V"), "tsappend": ("vv", "V"), "tsslice": ("vii", "V"),
+    "tsreverse": ("v", "V"), "tstranspose": ("vQ", "V"), "tsreshape": ("vS", "V"), "tsindex": ("vS", "V"), "tsargminmax": ("vi", "V"),
+    "tsiota": ("ii", "V"), "dense": ("v", "V"), "tsgather": ("vSK", "V"), "tconvert": ("ivS", "V"),
+    "ix_var": ("Si", "X"), "ix_const": ("Sid", "X"), "ix_lift": ("Sv", "X"), "ix_op1": ("ix", "X"), "ix_op2": ("ixx", "X"),
+    "ix_compare": ("ixx", "X"), "ix_select": ("xxx", "X"), "ix_convert": ("xii", "X"), "ix_index0": ("vK", "X"),
+    "ix_argminmax": ("vKi", "X"), "ix_from_val": ("v", "X"), "ix_to_val": ("x", "V"),
+    "force": ("v", "N"), "download": ("vp", "N"), "overwrite": ("vp", "N"), "assign": ("vv", "N"), "graph_launch": ("p", "N"),
+}
+
+
+class _Native:
+    """The entry points of NATIVE as functions of a host and their arguments, once the library is loaded."""
+
+
+_c = _Native()
 
 
 def _lib():
     global _dll
     if _dll is None:
-        import os
         if not os.path.exists(capi.HOST_LIB):
             raise FileNotFoundError(f"{capi.HOST_LIB} is not built; run __graft_entry__.build()")
         dll = C.CDLL(capi.HOST_LIB)
         for name, (res, args) in SIG.items():
             fn = getattr(dll, "hh_" + name)
             fn.restype, fn.argtypes = res, args
+        address = lambda name: C.cast(getattr(dll, "hh_" + name), C.c_void_p).value  # noqa: E731
+        _py.setup(V, IxV, HgpuError, *[address(f) for f in ("free", "ix_free", "val_rank", "val_dtype", "val_shape", "ix_dtype", "last_error", "backward")])
+        for name, (args, out) in NATIVE.items():
+            setattr(_c, name, _py.Fn(address(name), args, out))
         _dll = dll
     return _dll
 
@@ -77,7 +113,7 @@ class Graph:
         self.host, self.h = host, h
 
     def launch(self):
-        self.host.check(self.host.dll.hh_graph_launch(self.host.h, self.h))
+        _c.graph_launch(self.host, self.h)
 
     def free(self):
         if self.h:
@@ -86,7 +122,7 @@ class Graph:
             self.keeps = None
 
 
-class Host:
+class Host(_py.HostBase):
     """A host-layer context: on the gfx950 library by default, or on the provider
     whose ABI table `api_lib.get_api()` returns."""
 
@@ -101,6 +137,7 @@ class Host:
         if rc:
             raise HgpuError(rc, "cannot create a host-layer context (no usable device?)")
         self.h = h
+        self._bind(h)
 
     def check(self, rc):
         if rc:
@@ -122,7 +159,7 @@ class Host:
         return int(self.dll.hh_counter(self.h, name.encode()))
 
     def tape_reset(self):
-        self.check(self.dll.hh_tape_reset(self.h))
+        _c.tape_reset(self)
 
     def destroy(self):
         self.dll.hh_destroy(self.h)
@@ -136,7 +173,7 @@ class Host:
         try:
             result = program()
             for v in _values(result):
-                self.check(self.dll.hh_force(self.h, v.h))
+                _c.force(self, v)
         except BaseException:
             g = C.c_void_p()
             self.dll.hh_capture_end(self.h, C.byref(g))
@@ -177,17 +214,14 @@ class Host:
 
     def srepl(self, shape, value, dtype=capi.F64):
         """sconcrete (sreplicate shape value)"""
-        return self._out(self.dll.hh_constant, dtype, float(value), len(shape), _larr(shape))
+        return _c.constant(self, dtype, float(value), shape)
 
     def siota(self, n, dtype=capi.I64):
-        return self._out(self.dll.hh_tsiota, n, dtype)
+        return _c.tsiota(self, n, dtype)
 
     def grad(self, out, inputs, dt=None):
         """Cotangents of `inputs` for d(out) = dt (default: ones, as `grad` uses)."""
-        arr = (C.c_void_p * len(inputs))(*[v.h for v in inputs])
-        outs = (C.c_void_p * len(inputs))()
-        self.check(self.dll.hh_backward(self.h, out.h, dt.h if dt is not None else None, len(inputs), arr, outs))
-        return [V(self, C.c_void_p(o)) for o in outs]
+        return _py.backward(self, out, dt, inputs)
 
     # -- host loops of the tensor class (the reference's `Concrete` instance runs
     #    these closures once per index on the host as well)
@@ -242,12 +276,7 @@ class Host:
 
     # -- index functions
     def ix_space(self, shm):
-        return [IxV(self, self._ixo(self.dll.hh_ix_var, len(shm), _larr(shm), d), tuple(shm)) for d in range(len(shm))]
-
-    def _ixo(self, fn, *args):
-        o = C.c_void_p()
-        self.check(fn(self.h, *args, C.byref(o)))
-        return o
+        return [_c.ix_var(self, shm, d) for d in range(len(shm))]
 
     def _apply_index_fn(self, shm, f):
         shm = tuple(int(s) for s in shm)
@@ -257,47 +286,29 @@ class Host:
         return shm, res
 
 
-def _ixarr(ixs):
-    return (C.c_void_p * max(len(ixs), 1))(*[x.h for x in ixs])
-
-
-class IxV:
-    """A scalar inside an index function, for all positions at once."""
-
-    def __init__(self, host, h, shm):
-        self.host, self.h, self.shm = host, h, shm
-
-    def __del__(self):
-        try:
-            self.host.dll.hh_ix_free(self.h)
-        except Exception:
-            pass
+class IxV(_py.Lane):
+    """A scalar inside an index function, for all positions at once (`host`, `h`, `shm`: its index space, `dtype`)."""
 
     @staticmethod
     def const(host, shm, value, dtype=capi.I64):
-        return IxV(host, host._ixo(host.dll.hh_ix_const, len(shm), _larr(shm), dtype, float(value)), shm)
+        return _c.ix_const(host, shm, dtype, float(value))
 
     @staticmethod
     def from_val(v):
         """The elements of an array as a lane value over the array's own index space
         (what the scalar closure of tsmap0N / tszipWith0N is applied to)."""
-        return IxV(v.host, v.host._ixo(v.host.dll.hh_ix_from_val, v.h), tuple(v.shape))
+        return _c.ix_from_val(v.host, v)
 
     def to_val(self):
         """This lane value as an array of shape shm."""
-        return self.host._out(self.host.dll.hh_ix_to_val, self.h)
-
-    @property
-    def dtype(self):
-        return int(self.host.dll.hh_ix_dtype(self.h))
+        return _c.ix_to_val(self.host, self)
 
     def _coerce(self, o, dtype=None):
         """A Python number beside a lane value is a literal of the lane value's element type."""
-        return o if isinstance(o, IxV) else IxV.const(self.host, self.shm, o, self.dtype if dtype is None else dtype)
+        return o if isinstance(o, IxV) else _c.ix_const(self.host, self.shm, self.dtype if dtype is None else dtype, float(o))
 
     def _op2(self, op, o, dtype=None):
-        o = self._coerce(o, dtype)
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_op2, OP2[op], self.h, o.h), self.shm)
+        return _c.ix_op2(self.host, OP2[op], self, o if isinstance(o, IxV) else self._coerce(o, dtype))
 
     def _rop2(self, op, o, dtype=None):
         return self._coerce(o, dtype)._op2(op, self)
@@ -316,16 +327,15 @@ class IxV:
     def __rtruediv__(self, o): return self._rop2("div", o)
     def __pow__(self, o): return self._op2("pow", o)
     def atan2H(self, o): return self._op2("atan2", o)
-    def __neg__(self): return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_op1, OP1["neg"], self.h), self.shm)
+    def __neg__(self): return _c.ix_op1(self.host, OP1["neg"], self)
     def quotH(self, o): return self._op2("quot", o)
     def remH(self, o): return self._op2("rem_scalar", o)      # scalar rule: remH a 0 = a (Types.hs:402-419)
     def minH(self, o): return self._op2("min", o)
     def maxH(self, o): return self._op2("max", o)
-    def op1(self, name): return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_op1, OP1[name], self.h), self.shm)
+    def op1(self, name): return _c.ix_op1(self.host, OP1[name], self)
 
     def _cmp(self, c, o, dtype):
-        o = self._coerce(o, dtype)
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_compare, CMP[c], self.h, o.h), self.shm)
+        return _c.ix_compare(self.host, CMP[c], self, self._coerce(o, dtype))
 
     def leq(self, o, dtype=None): return self._cmp("leq", o, dtype)     # <=.
     def lt(self, o, dtype=None): return self._cmp("lt", o, dtype)       # <.
@@ -334,7 +344,7 @@ class IxV:
     def andB(self, o): return self._op2("and", o)                        # &&*
 
     def convert(self, dtype, mode=0):
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_convert, self.h, dtype, mode), self.shm)
+        return _c.ix_convert(self.host, self, dtype, mode)
 
 
 def ifH(cond, a, b, dtype=None):
@@ -344,37 +354,15 @@ def ifH(cond, a, b, dtype=None):
         dtype = a.dtype if isinstance(a, IxV) else b.dtype if isinstance(b, IxV) else capi.I64
     a = a if isinstance(a, IxV) else IxV.const(cond.host, cond.shm, a, dtype)
     b = b if isinstance(b, IxV) else IxV.const(cond.host, cond.shm, b, dtype)
-    return IxV(cond.host, cond.host._ixo(cond.host.dll.hh_ix_select, cond.h, a.h, b.h), cond.shm)
+    return _c.ix_select(cond.host, cond, a, b)
 
 
-class V:
-    """A tensor value of the `Gpu` carrier (possibly carrying a tape node)."""
-
-    def __init__(self, host, h):
-        self.host, self.h = host, h
-
-    def __del__(self):
-        try:
-            if self.h:
-                self.host.dll.hh_free(self.h)
-                self.h = None
-        except Exception:
-            pass
-
-    @property
-    def shape(self):
-        r = self.host.dll.hh_val_rank(self.h)
-        buf = (C.c_int64 * max(r, 1))()
-        self.host.dll.hh_val_shape(self.h, buf)
-        return tuple(buf[i] for i in range(r))
-
-    @property
-    def dtype(self):
-        return self.host.dll.hh_val_dtype(self.h)
+class V(_py.Val):
+    """A tensor value of the `Gpu` carrier, possibly carrying a tape node (`host`, `h`, `shape`, `dtype`)."""
 
     def numpy(self):
         out = np.empty(self.shape, dtype=_DT2NP[self.dtype])
-        self.host.check(self.host.dll.hh_download(self.host.h, self.h, out.ctypes.data_as(C.c_void_p)))
+        _c.download(self.host, self, out.__array_interface__["data"][0])
         return out
 
     def overwrite(self, x):
@@ -383,15 +371,12 @@ class V:
         if not x.flags.c_contiguous:
             x = x.copy(order="C")
         assert tuple(x.shape) == tuple(self.shape)
-        self.host.check(self.host.dll.hh_overwrite(self.host.h, self.h, x.ctypes.data_as(C.c_void_p)))
+        _c.overwrite(self.host, self, x.__array_interface__["data"][0])
 
     def assign(self, src):
         """This array's memory takes src's elements (how a recorded training step
         hands updated parameters to its next launch)."""
-        self.host.check(self.host.dll.hh_assign(self.host.h, self.h, src.h))
-
-    def _o(self, fn, *args):
-        return self.host._out(fn, *args)
+        _c.assign(self.host, self, src)
 
     def _lift(self, o):
         if isinstance(o, V):
@@ -399,14 +384,9 @@ class V:
         return self.host.srepl(self.shape, o, self.dtype)
 
     # -- Num / Fractional / Floating
-    def op1(self, name): return self._o(self.host.dll.hh_ewise1, OP1[name], self.h)
-    def op2(self, name, o):
-        o = self._lift(o)   # keeps the lifted constant alive across the call
-        return self._o(self.host.dll.hh_ewise2, OP2[name], self.h, o.h)
-
-    def _cmp(self, c, o):
-        o = self._lift(o)
-        return self._o(self.host.dll.hh_compare, CMP[c], self.h, o.h)
+    def op1(self, name): return _c.ewise1(self.host, OP1[name], self)
+    def op2(self, name, o): return _c.ewise2(self.host, OP2[name], self, o if isinstance(o, V) else self._lift(o))
+    def _cmp(self, c, o): return _c.compare(self.host, CMP[c], self, o if isinstance(o, V) else self._lift(o))
     def __add__(self, o): return self.op2("add", o)
     def __radd__(self, o): return self._lift(o).op2("add", self)
     def __sub__(self, o): return self.op2("sub", o)
@@ -433,11 +413,11 @@ class V:
 
     def select(self, a, b):
         """Elementwise ifH on a Bool tensor."""
-        return self._o(self.host.dll.hh_select, self.h, a.h, b.h)
+        return _c.select(self.host, self, a, b)
 
-    def scast(self, dtype): return self._o(self.host.dll.hh_convert, self.h, dtype, 0)
-    def sfromIntegral(self, dtype): return self._o(self.host.dll.hh_convert, self.h, dtype, 0)
-    def sfloor(self, dtype=capi.I64): return self._o(self.host.dll.hh_convert, self.h, dtype, 1)
+    def scast(self, dtype): return _c.convert(self.host, self, dtype, 0)
+    def sfromIntegral(self, dtype): return _c.convert(self.host, self, dtype, 0)
+    def sfloor(self, dtype=capi.I64): return _c.convert(self.host, self, dtype, 1)
 
     # -- maps of scalar closures (Ops.hs:929-941): the closure runs once, on lane values
     def smap0N(self, f):
@@ -451,75 +431,75 @@ class V:
         return f(IxV.from_val(self), IxV.from_val(o)).to_val()
 
     # -- reductions and contractions
-    def ssum(self): return self._o(self.host.dll.hh_tssumN, self.h, 1)
-    def ssumN(self, k): return self._o(self.host.dll.hh_tssumN, self.h, k)
-    def ssum0(self): return self._o(self.host.dll.hh_tssum0, self.h)
-    def sdot0(self, o): return self._o(self.host.dll.hh_tsdot0, self.h, o.h)
-    def sdot1In(self, o): return self._o(self.host.dll.hh_tsdot1In, self.h, o.h)
-    def sdotNIn(self, o, n): return self._o(self.host.dll.hh_tsdotNIn, self.h, o.h, n)
-    def as_input(self): return self._o(self.host.dll.hh_as_input, self.h)
-    def sprimalPart(self): return self._o(self.host.dll.hh_tprimalPart, self.h)
-    def tD(self, dual): return self._o(self.host.dll.hh_tD, self.h, dual.h)
+    def ssum(self): return _c.tssumN(self.host, self, 1)
+    def ssumN(self, k): return _c.tssumN(self.host, self, k)
+    def ssum0(self): return _c.tssum0(self.host, self)
+    def sdot0(self, o): return _c.tsdot0(self.host, self, o)
+    def sdot1In(self, o): return _c.tsdot1In(self.host, self, o)
+    def sdotNIn(self, o, n): return _c.tsdotNIn(self.host, self, o, n)
+    def as_input(self): return _c.as_input(self.host, self)
+    def sprimalPart(self): return _c.tprimalPart(self.host, self)
+    def tD(self, dual): return _c.tD(self.host, self, dual)
     def tconvert(self, conv, shape=None):
         """ConvertTensor: "kfromS", "sfromK", "sfromR", "rfromS", "sfromX", "xfromS", "nest", "unnest";
         shape = the shape the shaped type names (sfromR / sfromX) or the outer dims (nest / unnest)."""
         kinds = ["kfromS", "sfromK", "sfromR", "rfromS", "sfromX", "xfromS", "nest", "unnest"]
         sh = list(shape) if shape is not None else []
-        return self._o(self.host.dll.hh_tconvert, kinds.index(conv), self.h, len(sh), _larr(sh))
+        return _c.tconvert(self.host, kinds.index(conv), self, sh)
 
-    def smatvecmul(self, v): return self._o(self.host.dll.hh_tsmatvecmul, self.h, v.h)
-    def smatmul2(self, o): return self._o(self.host.dll.hh_tsmatmul2, self.h, o.h)
-    def sargMax(self): return self._o(self.host.dll.hh_tsargminmax, self.h, 1)
-    def sargMin(self): return self._o(self.host.dll.hh_tsargminmax, self.h, 0)
+    def smatvecmul(self, v): return _c.tsmatvecmul(self.host, self, v)
+    def smatmul2(self, o): return _c.tsmatmul2(self.host, self, o)
+    def sargMax(self): return _c.tsargminmax(self.host, self, 1)
+    def sargMin(self): return _c.tsargminmax(self.host, self, 0)
 
     # -- structure
-    def sreplicate(self, k): return self._o(self.host.dll.hh_tsreplicateN, self.h, 1, _larr([k]))
-    def sreplicateN(self, shm): return self._o(self.host.dll.hh_tsreplicateN, self.h, len(shm), _larr(shm))
+    def sreplicate(self, k): return _c.tsreplicateN(self.host, self, (k,))
+    def sreplicateN(self, shm): return _c.tsreplicateN(self.host, self, shm)
     sreplicate0N = sreplicateN
-    def sappend(self, o): return self._o(self.host.dll.hh_tsappend, self.h, o.h)
-    def sslice(self, i, n): return self._o(self.host.dll.hh_tsslice, self.h, i, n)
-    def sreverse(self): return self._o(self.host.dll.hh_tsreverse, self.h)
-    def stranspose(self, perm): return self._o(self.host.dll.hh_tstranspose, self.h, len(perm), (C.c_int * max(len(perm), 1))(*perm))
+    def sappend(self, o): return _c.tsappend(self.host, self, o)
+    def sslice(self, i, n): return _c.tsslice(self.host, self, i, n)
+    def sreverse(self): return _c.tsreverse(self.host, self)
+    def stranspose(self, perm): return _c.tstranspose(self.host, self, perm)
     def str_(self): return self.stranspose([1, 0])
-    def sreshape(self, shape): return self._o(self.host.dll.hh_tsreshape, self.h, len(shape), _larr(shape))
-    def sindex(self, ix): return self._o(self.host.dll.hh_tsindex, self.h, len(ix), _larr(ix))   # `!$` with concrete indices
+    def sreshape(self, shape): return _c.tsreshape(self.host, self, shape)
+    def sindex(self, ix): return _c.tsindex(self.host, self, ix)   # `!$` with concrete indices
 
     # -- indexing with index functions
     def dense(self):
         """The primal part as a dense row-major array (a copy when the value is a strided view)."""
-        return self._o(self.host.dll.hh_dense, self.h)
+        return _c.dense(self.host, self)
 
     def sgather(self, shm, f):
         """sgather @shm self (\\[i...] -> [ix...])"""
         shm, ix = self.host._apply_index_fn(shm, f)
-        return self._o(self.host.dll.hh_tsgather, self.h, len(shm), _larr(shm), len(ix), _ixarr(ix))
+        return _c.tsgather(self.host, self, shm, ix)
 
     def sscatter(self, rank_m, shp, f):
         """sscatter @shm self (\\[i...] -> [ix...]) with shm = the first rank_m dims; result shp ++ rest"""
         shm, ix = self.host._apply_index_fn(self.shape[:rank_m], f)
         if len(ix) != len(shp):
             raise HgpuError(1, "sscatter: the index function must return one index per dim of shp")
-        return self._o(self.host.dll.hh_tsscatter, self.h, rank_m, len(ix), _larr(shp), _ixarr(ix))
+        return self.host._out(self.host.dll.hh_tsscatter, self.h, rank_m, len(ix), _larr(shp), (C.c_void_p * max(len(ix), 1))(*[x.h for x in ix]))
 
     # inside index functions
     def sindex0(self, ix):
         """self `sindex0` [ix...] with lane-batched indices"""
         first = next(x for x in ix if isinstance(x, IxV))
         ix = [x if isinstance(x, IxV) else IxV.const(self.host, first.shm, x) for x in ix]
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_index0, self.h, len(ix), _ixarr(ix)), first.shm)
+        return _c.ix_index0(self.host, self, ix)
 
     def kargMax(self, ix, want_max=True):
         """kargMax (self !$ [ix...])"""
         first = next(x for x in ix if isinstance(x, IxV))
         ix = [x if isinstance(x, IxV) else IxV.const(self.host, first.shm, x) for x in ix]
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_argminmax, self.h, len(ix), _ixarr(ix), int(want_max)), first.shm)
+        return _c.ix_argminmax(self.host, self, ix, int(want_max))
 
     def kargMin(self, ix):
         return self.kargMax(ix, want_max=False)
 
     def lift(self, shm):
         """A rank-0 tensor as a scalar of the position space shm."""
-        return IxV(self.host, self.host._ixo(self.host.dll.hh_ix_lift, len(shm), _larr(shm), self.h), tuple(shm))
+        return _c.ix_lift(self.host, shm, self)
 
 
 # Ranked (`tr*`, user-facing `r*`) and mixed (`tx*` / `x*`) methods of the tensor

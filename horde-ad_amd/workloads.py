@@ -17,6 +17,8 @@ way horde-ad's interpreter drives a `BaseTensor` instance:
 Inputs are synthetic, drawn from numpy's counter-based Philox generator with
 fixed seeds, so that every provider of the array ABI sees the same numbers.
 """
+import math
+
 import numpy as np
 
 from . import capi
@@ -66,7 +68,7 @@ def reluS_select(v):
 
 def sminimum(u):
     """sindex0 tf [kargMin tf] on the flattened tensor."""
-    n = int(np.prod(u.shape))
+    n = math.prod(u.shape)
     tf = u.sreshape([n])
     arg = tf.sargMin()
     return tf.sgather((), lambda: [arg.lift(())])
@@ -156,7 +158,7 @@ def convMnistTwoS(inp, params, layer=None):
     b = inp.shape[0]
     t1 = layer(k1, inp, b1)
     t2 = layer(k2, t1, b2)
-    m1 = t2.sreshape([b, int(np.prod(t2.shape[1:]))])
+    m1 = t2.sreshape([b, math.prod(t2.shape[1:])])
     dense = wd.smatmul2(m1.str_()) + bd.sreplicate(b).str_()
     return wr.smatmul2(reluS(dense)) + br.sreplicate(b).str_()
 
