@@ -30,13 +30,17 @@
 // probability under e^-69 the second way, 3.9 ms instead of 0.41 for 2048 x 8192 over 2048, and let products just
 // below 2^128 overflow.)
 //
-// What bounds it: the vector instructions beside the products (an element's split, 7 of them, and the rounded
-// additions) and the power the matrix cores draw; orders of the loop's instructions that differ by a fifth in stalls
-// measure the same.  Six bf16 instructions of 32 x 32 x 16 do the work of eight fp32 ones of 32 x 32 x 2.  2048 x 8192
-// over 2048, normally distributed / behind a relu: fp32 instruction 649 / 615 us, here 464 / 428 one after another
-// (380 to 410 in the wide dense network's gradient, among shorter kernels, on two cards).  (256 x 256 tiles split an
-// element half as often, but two sets of accumulators do not fit: all six terms in one chain 407 / 378, the second
-// set added up by vector instructions 480 / 445.  256 x 128 tiles: 489 / 456.)
+// What bounds it: the mix of instructions beside the products and the power all of them draw.  Six bf16 instructions of
+// 32 x 32 x 16 do the work of eight fp32 ones of 32 x 32 x 2.  Loops of nothing but the step's instructions, TFLOP/s of bf16 on
+// normal numbers: products alone 1787, with the reads of LDS 1647, with the rounded additions too 1499, with the split's vector
+// instructions (7 an element) 1324, with the writes to LDS 1230, with the barriers 1207, with loads that a step waits for 1027.
+// The loads are a step ahead of their use: they go out when the registers of the step before are split (the compiler, left to itself,
+// waited for loads of the same step behind a sixth of its products), 1033 -> 1064 here.  2048 x 8192 over 2048, normally
+// distributed / behind a relu, one after another: 398 / 385 us with loads of the same step, 388 / 374 now (fp32 instruction 649 / 615
+// on another card); three of 128 x 128 over 27 x 5000 in one launch 126 / 117, bound by their loads (377 MB).
+// (256 x 256 tiles split an element half as often, but two sets of accumulators do not fit: all six terms in one
+// chain, or the second set added up by vector instructions, were no faster; nor were 256 x 128 tiles.  Remainders formed
+// by v_dot2_f32_bf16, two instructions less a remainder: wrong results.)
 #include "gemm_kernel.hpp"
 
 using namespace hg;
@@ -126,23 +130,20 @@ struct Side {
         s[i].v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, h + j < left ? off[i] + (k0 + j) * ks : 0xfffffff0u, 0, 0));
     }
   }
-  // parts: [3][ROWS * 2] of 16 bytes
-  __device__ __forceinline__ void store(const Slot& s, int i, u4* parts, float& largest) const {
+  // Elements 2 j and 2 j + 1 of a piece become theirs of its three parts.
+  static __device__ __forceinline__ void split(const Slot& s, int j, u4* parts, float& largest) {
+    uint32_t h, m, l;
+    split2(s.v[2 * j], s.v[2 * j + 1], h, m, l);
+    parts[0][j] = h;
+    parts[1][j] = m;
+    parts[2][j] = l;
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(s.v[2 * j]), "v"(s.v[2 * j + 1]));      // (passes NaNs over: their parts are NaNs)
+  }
+  // to: [3][ROWS * 2] of 16 bytes
+  __device__ __forceinline__ void put(const u4* parts, int i, u4* to) const {
     if (!ALL && threadIdx.x >= ROWS * 2) return;
-    u4 h, m, l;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float a = s.v[2 * j], b = s.v[2 * j + 1];
-      uint32_t ph, pm, pl;
-      split2(a, b, ph, pm, pl);
-      h[j] = ph;
-      m[j] = pm;
-      l[j] = pl;
-      asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(a), "v"(b));      // (passes NaNs over: their parts are NaNs)
-    }
-    parts[at[i]] = h;
-    parts[ROWS * 2 + at[i]] = m;
-    parts[ROWS * 4 + at[i]] = l;
+    for (int q = 0; q < 3; ++q) to[q * ROWS * 2 + at[i]] = parts[q];
   }
 };
 
@@ -160,15 +161,14 @@ __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t rsrc, uint32_t row, 
 }
 
 // THIN: tiles of 128 x 32 for products with at most 32 columns (weight gradients of narrow layers), bound by the loads of A:
-// a step is 10 KB of loads and eight instructions a wavefront, one step ahead, so four blocks (114 to 128 registers, 30 KB of
-// LDS) hide one another's trips to memory (with six instructions the same products take 2 to 3 % less: 128 x 28 over 28 x 5000
-// with its sums 26.0 for 26.6 us, 784 x 32 over 8192 13.4 for 13.8).  128 x 28 over 28 x 5000, 87 MB: 23.7 us = 3.7 TB/s, the 32 x 32 tiles of the fp32
-// instruction, which read A for every 32 rows of it and B four times, 33.0.
+// a step is 10 KB of loads and eight instructions a wavefront, one step ahead, so four blocks (124 to 128 registers, 30 KB of
+// LDS) hide one another's trips to memory (with six instructions the same products take 2 to 3 % less).  128 x 28 over 28 x 5000
+// with its row sums, 87 MB, in the recurrent network's gradient: 30.1 us with loads of the same step, 26.5 now; the 32 x 32 tiles of the fp32
+// instruction, which read A for every 32 rows of it and B four times, 33.0 without sums.
 // ROWS: the lanes also add up, in fp64, the elements of A they stage: a bias gradient is the row sums of what the weight
 // gradient multiplies.  Blocks of the first column of tiles do, for products that ask (split_job).  Reading A once more for
 // them: 28 x 128 rows of 5000 17.5 us, 2048 rows of 8192 17.4; here
-// the recurrent network's three products of 128 x 128 take 139 us for 135 and the one of 128 x 28 32 for 29.  (The large tile keeps
-// 12 to 20 bytes of a lane in scratch memory then, outside of its loop's loads.)
+// they cost the recurrent network's products 3 to 4 us.
 template <bool AKC, bool BKC, bool THIN, bool ROWS>
 __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int nr, int nsplits, int batch) {
   constexpr int WM = THIN ? 4 : 2, WN = THIN ? 1 : 2, TM = THIN ? 1 : 2, TN = THIN ? 1 : 2;          // wavefronts, and 32 x 32 blocks of each
@@ -202,12 +202,23 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   const bool sum_rows = ROWS && p.rows != nullptr && n0 == 0;
   double row_sum = 0, row_factor = 1;
   if (sum_rows && p.row_factor) row_factor = (double)*(const float*)p.row_factor;
-  auto store_a = [&](int u, u4* to, int left) {      // left: elements of k that the step has, 16 and more: all
-    sa.store(ra[u], u, to, top_a);
-    if (sum_rows) {
+  // Pair number w of what the block stages of a step: split; with the last one of a piece its parts go to LDS.
+  // left: elements of k that the step has, 16 and more: all
+  constexpr int PAIRS = 4 * (NA + NB);
+  u4 parts[3];
+  auto stage = [&](int w, u4* to, int left) {
+    const int u = w / 4, j = w % 4;
+    if (u < NA) {
+      sa.split(ra[u], j, parts, top_a);
+      if (sum_rows) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (left >= SK || 8 * (t & 1) + j < left) row_sum = __builtin_fma((double)ra[u].v[j], row_factor, row_sum);      // (the product is exact)
+        for (int e = 2 * j; e < 2 * j + 2; ++e)
+          if (left >= SK || 8 * (t & 1) + e < left) row_sum = __builtin_fma((double)ra[u].v[e], row_factor, row_sum);      // (the product is exact)
+      }
+      if (j == 3) sa.put(parts, u, to);
+    } else {
+      sb.split(rb[u - NA], j, parts, top_b);
+      if (j == 3) sb.put(parts, u - NA, to + PA);
     }
   };
   auto fetch = [&](int i) {                 // (chosen outside the main loop: a load on one side of a branch would be waited for where the sides meet)
@@ -221,83 +232,101 @@ __device__ __forceinline__ void gemm_split_body(const SplitParams& p, const floa
   if (whole > 0) fetch(0);
   else fetch_tail(0);
 #pragma unroll
-  for (int i = 0; i < NA; ++i) store_a(i, lds[0], kend - kbeg);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) sb.store(rb[i], i, lds[0] + PA, top_b);
+  for (int w = 0; w < PAIRS; ++w) stage(w, lds[0], kend - kbeg);
+  if (whole > 1) fetch(1);
+  else if (steps > 1) fetch_tail(1);
   __syncthreads();
 
   const int fra = lds_at(wm * TM * 32 + (lane & 31), lane >> 5), frb = lds_at(wn * TN * 32 + (lane & 31), lane >> 5);
-  // One step: the loads of the next step go out, the products of this one are formed, and the
-  // next step's elements are split and stored to the other buffer behind the products.
-  // next: 0 = there is none, 1 = a whole step, 2 = the rest of K.
-  auto step = [&](int i0, auto next) {
+  // One step: its products are formed; behind them the next step's elements, which have been on their way for a
+  // step, are split and stored to the other buffer, and as soon as a piece's registers are free the loads of the step after that go out.
+  // next: the next step exists. load: 0 = the one after it does not, 1 = it is a whole one, 2 = the rest of K.
+  auto step = [&](int i0, auto next, auto load) {
     constexpr bool more = decltype(next)::value != 0;
+    constexpr int ld = decltype(load)::value;
     const int cur = i0 & 1;
-    if constexpr (decltype(next)::value == 1) fetch(i0 + 1);
-    if constexpr (decltype(next)::value == 2) fetch_tail(i0 + 1);
-    __builtin_amdgcn_sched_barrier(0);      // (left to itself the compiler moves the loads down to their use)
     const u4* la = lds[cur] + fra;
     const u4* lb = lds[cur] + PA + frb;
     u4* ln = lds[cur ^ 1];
-    const int left = decltype(next)::value == 2 ? kend - kbeg - (i0 + 1) * SK : SK;
-    bf8 fa[TM][3];
+    const int left = ld ? SK : kend - kbeg - (i0 + 1) * SK;
+    bf8 fa[TM][3], fb[TN][3];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int q = 0; q < 3; ++q) {
 #pragma unroll
-      for (int q = 0; q < 3; ++q) fa[i][q] = __builtin_bit_cast(bf8, la[q * BM * 2 + i * 64]);
+      for (int i = 0; i < TM; ++i) fa[i][q] = __builtin_bit_cast(bf8, la[q * BM * 2 + i * 64]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      bf8 fb[3];
+      for (int j = 0; j < TN; ++j) fb[j][q] = __builtin_bit_cast(bf8, lb[q * BN * 2 + j * 64]);
+    }
+    constexpr int TERMS = THIN ? 8 : 6, PRODUCTS = TM * TN * TERMS;
+    constexpr int FIRST = 3;               // (the loads have had a step to arrive; a little more does no harm)
+    auto until = [&](int product) {          // pairs staged before the product after this one
+      const int n = product < FIRST ? 0 : (product - FIRST + 1) * PAIRS / (PRODUCTS - FIRST - 1);
+      return n < PAIRS ? n : PAIRS;
+    };
+    auto behind = [&](int product) {        // what is staged behind a product
+      if constexpr (more) {
 #pragma unroll
-      for (int q = 0; q < 3; ++q) fb[q] = __builtin_bit_cast(bf8, lb[q * BN * 2 + j * 64]);
+        for (int w = 0; w < PAIRS; ++w) {
+          if (w < until(product - 1) || w >= until(product)) continue;
+          stage(w, ln, left);
+          if (w == 4 * NA - 1) {
+            if constexpr (ld == 1) sa.load(kbeg + (i0 + 2) * SK, ra);
+            if constexpr (ld == 2) sa.load_tail(t, kbeg + (i0 + 2) * SK, kend - kbeg - (i0 + 2) * SK, ra);
+          }
+          if (w == PAIRS - 1) {
+            if constexpr (ld == 1) sb.load(kbeg + (i0 + 2) * SK, rb);
+            if constexpr (ld == 2) sb.load_tail(t, kbeg + (i0 + 2) * SK, kend - kbeg - (i0 + 2) * SK, rb);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int b = 0; b < TM * TN; ++b) {
       // h h' of 16 k is summed from zero and added with one rounded addition; the five smaller terms are summed on the
       // matrix cores, the smallest first.
+      const int i = b % TM, j = b / TM;
+      int n = b * TERMS;
+      f16v zero;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        f16v zero;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) zero[r] = 0;
-        auto add = [&](int qa, int qb, const f16v& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[qb], c, 0, 0, 0); };
-        const f16v c = add(0, 0, zero);
-        if constexpr (THIN) {
-          low[i][j] = add(2, 1, low[i][j]);
-          low[i][j] = add(1, 2, low[i][j]);
-        }
-        low[i][j] = add(2, 0, low[i][j]);
-        low[i][j] = add(0, 2, low[i][j]);
-        low[i][j] = add(1, 1, low[i][j]);
-        low[i][j] = add(1, 0, low[i][j]);
-        low[i][j] = add(0, 1, low[i][j]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] += c[r];
+      for (int r = 0; r < 16; ++r) zero[r] = 0;
+      auto add = [&](int qa, int qb, const f16v& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[j][qb], c, 0, 0, 0); };
+      const f16v c = add(0, 0, zero);
+      behind(n++);
+      if constexpr (THIN) {
+        low[i][j] = add(2, 1, low[i][j]);
+        behind(n++);
+        low[i][j] = add(1, 2, low[i][j]);
+        behind(n++);
       }
-      if constexpr (more) {       // the loads have had the first columns' products to arrive
-        constexpr int first = 1;
-        if (j >= first) {
-          const int u = j - first;
-          if (u < NA) store_a(u, ln, left);
-          else if (u - NA < NB) sb.store(rb[u - NA], u - NA, ln + PA, top_b);
-        }
-      }
-    }
-    if constexpr (more) {
-      constexpr int first = 1;
+      low[i][j] = add(2, 0, low[i][j]);
+      behind(n++);
+      low[i][j] = add(0, 2, low[i][j]);
 #pragma unroll
-      for (int u = TN - first; u < NA + NB; ++u) {
-        if (u < NA) store_a(u, ln, left);
-        else sb.store(rb[u - NA], u - NA, ln + PA, top_b);
-      }
+      for (int r = 0; r < 5; ++r) acc[i][j][r] += c[r];
+      behind(n++);
+      low[i][j] = add(1, 1, low[i][j]);
+#pragma unroll
+      for (int r = 5; r < 10; ++r) acc[i][j][r] += c[r];
+      behind(n++);
+      low[i][j] = add(1, 0, low[i][j]);
+#pragma unroll
+      for (int r = 10; r < 16; ++r) acc[i][j][r] += c[r];
+      behind(n++);
+      low[i][j] = add(0, 1, low[i][j]);
+      behind(n++);
     }
     __syncthreads();
   };
+  constexpr std::integral_constant<int, 0> none{};
+  constexpr std::integral_constant<int, 1> full{};
+  constexpr std::integral_constant<int, 2> rest{};
   int i0 = 0;
 #pragma unroll 1
-  for (; i0 + 1 < whole; ++i0) step(i0, std::integral_constant<int, 1>{});
-  if (i0 + 1 < steps) {
-    step(i0, std::integral_constant<int, 2>{});
-    ++i0;
-  }
-  step(i0, std::integral_constant<int, 0>{});
+  for (; i0 + 2 < whole; ++i0) step(i0, full, full);
+  if (i0 + 2 < steps) step(i0++, full, rest);
+  if (i0 + 1 < steps) step(i0++, full, none);
+  step(i0, none, none);
 
   if (sum_rows) {
     row_sum += __shfl_xor(row_sum, 1);

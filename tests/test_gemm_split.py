@@ -47,6 +47,28 @@ def test_ragged_shapes(gpu, m, n, k, lay):
     assert_close(out, x, y, k)
 
 
+@pytest.mark.parametrize("lay", ["KK", "KR", "RR"])
+@pytest.mark.parametrize("k", [64, 65, 79, 80, 81, 95])
+def test_few_steps(gpu, k, lay):
+    """Loads run a step and splits half a step ahead: sums of a few steps, with and without a rest."""
+    rng = np.random.default_rng(k)
+    x, y = rng.standard_normal((130, k)).astype(np.float32), rng.standard_normal((100, k)).astype(np.float32)
+    assert_close(repeated(gpu, x, y, lay), x, y, k)
+
+
+@pytest.mark.parametrize("k", [20000, 20001, 20016, 20033, 20044])
+def test_last_share_of_k(gpu, k):
+    """K shared out: the last share is shorter than the others, down to less than a step."""
+    rng = np.random.default_rng(k)
+    x, y = rng.standard_normal((200, k)).astype(np.float32), rng.standard_normal((130, k)).astype(np.float32)
+    gpu.profile(2)
+    out = product(gpu, x, y, "KK").numpy()
+    labels = list(gpu.profile_report())
+    gpu.profile(0)
+    assert any("split3" in s and ",s1," not in s for s in labels), labels
+    assert_close(out, x, y, k)
+
+
 @pytest.mark.parametrize("rest", [0.0, 2.0 ** -40])
 @pytest.mark.parametrize("lay", ["KK", "RR"])
 @pytest.mark.parametrize("diagonal", [False, True])
