@@ -1071,11 +1071,12 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
       hipFunction_t fn = nullptr;
       // Fewer weights in registers where the compiler found too few for the rest, in small steps: LDS may have no room for many
       // more (two layers of width 128 transposed, fp64: 68 bytes of scratch, 52 with eight registers less, no plan with 24 less).
-      for (int slack = 0; !fn && slack <= 24; slack += 8) {
-        plan = ChainPlan();
-        if (!plan_chain(cand, levels, ctx->num_cu, slack, l0, &l1, &plan)) break;
-        fn = chain_kernel(ctx, plan);
-      }
+      for (bool lone : {true, false})
+        for (int slack = 0; !fn && slack <= 24; slack += 8) {
+          plan = ChainPlan();
+          if (!plan_chain(cand, levels, ctx->num_cu, slack, lone, l0, &l1, &plan)) break;
+          fn = chain_kernel(ctx, plan);
+        }
       if (!fn) break;
       std::vector<const void*> ar = plan.ptrs;
       ar.resize(kChainMaxPtrs, nullptr);
@@ -1086,7 +1087,7 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
       const char* label = items[(size_t)levels[(size_t)l0][0]].label;
       if (ctx->profiling && ctx->profile_shapes) {
         char buf[160];
-        snprintf(buf, sizeof buf, "gemm_%s[chain:P%lld,levels%d,products%d,t%d]", plan.f64 ? "f64" : "f32", (long long)plan.P, plan.n_levels, plan.n_items, 4 * plan.NC);
+        snprintf(buf, sizeof buf, "gemm_%s[chain:P%lld,levels%d,products%d,t%d]", plan.f64 ? "f64" : "f32", (long long)plan.P, plan.n_levels, plan.n_items, chain_columns(plan));
         label = intern_label(ctx, buf);
       }
       timed_launch(fn, (unsigned)((chain_blocks(plan) + 7) / 8 * 8), ar, label, plan.bytes, plan.flops, 512);

@@ -21,11 +21,16 @@
 //     operand.  Tiles of four columns cost the same
 //     per product as the large ones (probe, 250 CUs, all operands resident: fp32 103 TFLOP/s with NC up to 3, 123 from
 //     4 on; fp64 59-64) and let 5000 columns be 250 blocks of 20.
+//   * fp64 with up to two columns for every CU: lone columns on vector instructions, whose rate is that of the matrix ones and which
+//     need no four columns to be filled (lone_products): 150 columns are 150 blocks instead of 38, and a level multiplies for 0.4
+//     instead of 1.4 us.  A lane's program serves one row, not one of four columns, so a wavefront's two row groups share a pass of it.
 //
 // What bounds it: in fp32 with 20 columns a block the matrix cores, 4.3 of the 5.6 us a level (two layers 128 wide; a level
 // by itself 10.6), the rest LDS latency after the barrier and the program; with 4 columns the chain LDS read, multiply,
-// program, LDS write, barrier: 1.3-1.6 us in fp32, in fp64 2.5 without and 3.3 with a tanh (a level by itself 4.7).
-// Gradients of two layers 128 wide over 28 steps, before / so: fp32 batch 5000 844 / 629 us, fp64 batch 150 278 / 252 for the second of its two chains.
+// program, LDS write, barrier: 1.3-1.6 us in fp32, in fp64 2.5 without and 3.3 with a tanh (a level by itself 4.7); in fp64 with one column
+// 2.0, of which the barrier with the loads and stores around it about 1.  29 levels of two layers 128 wide, 150 columns of fp64: 99.7 us in groups of four
+// (44 of them the multiplications, 22 the tanh), 58.7 alone.
+// Gradients of two layers 128 wide over 28 steps, before / so: fp32 batch 5000 844 / 629 us.
 // Taken back: nontemporal stores of the results (no gain beside the movers' priority), all wavefronts on all layers (fp32
 // the same, fp64 forward 111 us for 100; still the form where one layer's weights do not fit its wavefronts).
 
@@ -39,6 +44,7 @@ constexpr int kChainMaxWidth = 4;       // products of one level
 constexpr int kChainLds = 160 * 1024;
 
 constexpr int kChainMaxUnits = 8;
+constexpr int kChainMaxLone = 2;        // lone columns of a block
 
 struct ChainMat {                // a weights factor, W[q][k]
   const void* ptr;
@@ -73,6 +79,7 @@ struct ChainSection {            // levels that do the same with other arrays
 };
 struct ChainPlan {
   bool f64 = false;
+  bool lone = false;             // columns one by one on vector instructions (NC of them a block) instead of groups of four
   int64_t P = 0;
   int NC = 1, roles = 1;
   std::vector<ChainMat> mats;
@@ -87,7 +94,7 @@ struct ChainPlan {
 // Everything chain_source reads.
 Key chain_key(const ChainPlan& c) {
   Key k;
-  k.put(c.f64).put(c.P).put(c.NC).put(c.roles).put(c.out_elems).put(c.ext_elems).put(c.lds_elems).put(c.n_const).put(c.mats.size());
+  k.put(c.f64).put(c.lone).put(c.P).put(c.NC).put(c.roles).put(c.out_elems).put(c.ext_elems).put(c.lds_elems).put(c.n_const).put(c.mats.size());
   for (auto& m : c.mats) {
     k.put(m.Q).put(m.K).put(m.sq).put(m.sk).put(m.kept()).put(m.role).put(m.w0).put(m.nw).put(m.units);
     for (int u = 0; u < m.units; ++u) k.put(m.reg[u]).put(m.lds[u]);
@@ -108,9 +115,11 @@ Key chain_key(const ChainPlan& c) {
 int chain_vk(bool f64) { return f64 ? 2 : 4; }
 int chain_kp(bool f64, int64_t K) { const int kt = 4 * chain_vk(f64); return (int)((K + kt - 1) / kt * kt); }
 // LDS elements of `rows` x 4 NC columns; a group of four columns is followed by four elements that keep the groups in different banks
-int chain_region(const ChainPlan& c, int rows) { return c.NC * (rows * 4 + 4); }
+int chain_pitch(const ChainPlan& c, int rows) { return c.lone ? rows : rows * 4 + 4; }
+int chain_region(const ChainPlan& c, int rows) { return c.NC * chain_pitch(c, rows); }
 
-int64_t chain_blocks(const ChainPlan& c) { return (c.P + 4 * c.NC - 1) / (4 * c.NC); }
+int chain_columns(const ChainPlan& c) { return c.lone ? c.NC : 4 * c.NC; }      // of a block
+int64_t chain_blocks(const ChainPlan& c) { return (c.P + chain_columns(c) - 1) / chain_columns(c); }
 // The wavefronts of a role end where the next one's begin.
 int role_end(const ChainPlan& c, int role) {
   for (auto& m : c.mats)
@@ -130,6 +139,10 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
   const std::string mtid = "(tid - " + str(64 * mw) + ")";
   auto targs = [&](const ChainMat& m) { return str(m.Q) + "LL, " + str(m.K) + "LL, " + str(m.sq) + "LL, " + str(m.sk) + "LL, "; };
   auto row_of = [&](const ChainMat& m, int u) { return "(w + " + str(m.nw * u - m.w0) + ") * 16"; };      // first row of the wavefront's u-th group
+  // lone columns: this lane's row of groups 2 v and 2 v + 1, which the halves of the wavefront hold (all of it the first where there is no other)
+  auto pair_row = [&](const ChainMat& m, int v, int units) {
+    return "(w + " + str(2 * m.nw * v - m.w0) + (2 * v + 1 < units ? " + (lane >> 5) * " + str(m.nw) : std::string()) + ") * 16 + (lane & 15)";
+  };
   // the weights that several levels multiply by
   for (size_t m = 0; m < c.mats.size(); ++m) {
     const ChainMat& mt = c.mats[m];
@@ -168,8 +181,8 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
         const ChainMat& mt = c.mats[(size_t)it.x[0].mat];
         for (size_t i = 0; i < it.in.size(); ++i)
           if (it.in[i].kind == kind)
-            for (int u = 0; u < mt.units; ++u) {
-              const std::string row = row_of(mt, u) + (it.wide() ? " + qw" : " + ql");
+            for (int u = 0; u < (c.lone ? (mt.units + 1) / 2 : mt.units); ++u) {
+              const std::string row = c.lone ? pair_row(mt, u, mt.units) : row_of(mt, u) + (it.wide() ? " + qw" : " + ql");
               fn(it, it.in[i], row + " < " + str(it.Q) + " ? " + row + " : " + str(it.Q - 1), str((long long)j) + "_" + str((long long)i) + "_" + str(u));
             }
       }
@@ -178,9 +191,10 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       if (!mover) return;
       for (auto& x : staged) {
         const int ns = (x.rows * NC + movers - 1) / movers;
-        s << "      A4 " << pre << x.nm << "[" << ns << "];\n      {\n        const T* a = (const T*)ar.p[" << base << " + " << x.ptr << "];\n#pragma unroll\n";
+        s << "      " << (c.lone ? "T " : "A4 ") << pre << x.nm << "[" << ns << "];\n      {\n        const T* a = (const T*)ar.p[" << base << " + " << x.ptr << "];\n#pragma unroll\n";
         s << "        for (int i = 0; i < " << ns << "; ++i) {\n          const int sl = " << mtid << " + " << movers << " * i, kk = sl / NC, cc = sl % NC;\n";
-        s << "          " << pre << x.nm << "[i] = cols<" << x.sp << "LL>(a + (i64)(kk < " << x.K << " ? kk : " << x.K - 1 << ") * " << x.sk << "LL, p0 + 4 * cc);\n        }\n      }\n";
+        if (c.lone) s << "          const i64 p = p0 + cc;\n          " << pre << x.nm << "[i] = a[(i64)(kk < " << x.K << " ? kk : " << x.K - 1 << ") * " << x.sk << "LL + (p < P ? p : P - 1) * " << x.sp << "LL];\n        }\n      }\n";
+        else s << "          " << pre << x.nm << "[i] = cols<" << x.sp << "LL>(a + (i64)(kk < " << x.K << " ? kk : " << x.K - 1 << ") * " << x.sk << "LL, p0 + 4 * cc);\n        }\n      }\n";
       }
     };
     auto put_staged = [&](const char* buf, const char* pre) {
@@ -188,7 +202,8 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       for (auto& x : staged) {
         const int ns = (x.rows * NC + movers - 1) / movers;
         s << "#pragma unroll\n      for (int i = 0; i < " << ns << "; ++i) {\n        const int sl = " << mtid << " + " << movers << " * i, kk = sl / NC, cc = sl % NC;\n";
-        s << "        if (sl < " << x.rows * NC << ") *reinterpret_cast<A4*>(" << buf << " + " << x.off << " + cc * " << x.rows * 4 + 4 << " + kk * 4) = kk < " << x.K << " ? " << pre << x.nm
+        if (c.lone) s << "        if (sl < " << x.rows * NC << ") " << buf << "[" << x.off << " + cc * " << x.rows << " + kk] = kk < " << x.K << " ? " << pre << x.nm << "[i] : T(0);\n      }\n";
+        else s << "        if (sl < " << x.rows * NC << ") *reinterpret_cast<A4*>(" << buf << " + " << x.off << " + cc * " << x.rows * 4 + 4 << " + kk * 4) = kk < " << x.K << " ? " << pre << x.nm
           << "[i] : A4{0, 0, 0, 0};\n      }\n";
       }
     };
@@ -196,7 +211,7 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       each_in(3, [&](const ChainItem& it, const ChainIn& in, const std::string& row, const std::string& nm) {
         s << "    " << ctype(in.dtype) << " " << pre << nm << "[NC];\n    {\n      const " << ctype(in.dtype) << "* a = (const " << ctype(in.dtype) << "*)ar.p[" << base << " + " << in.ptr
           << "] + (i64)(" << row << ") * " << in.sq << "LL;\n";
-        s << "#pragma unroll\n      for (int cc = 0; cc < NC; ++cc) {\n        const i64 p = p0 + 4 * cc + " << (it.wide() ? "pw" : "pl") << ";\n        " << pre << nm << "[cc] = a[(p < P ? p : P - 1) * " << in.sp << "LL];\n      }\n    }\n";
+        s << "#pragma unroll\n      for (int cc = 0; cc < NC; ++cc) {\n        const i64 p = p0 + " << (c.lone ? "cc" : it.wide() ? "4 * cc + pw" : "4 * cc + pl") << ";\n        " << pre << nm << "[cc] = a[(p < P ? p : P - 1) * " << in.sp << "LL];\n      }\n    }\n";
       });
     };
     auto landed_lanes = [&](const char* pre) {
@@ -211,7 +226,11 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
           if (!o.staged) continue;
           const int64_t n = it.Q * NC;
           s << "      {\n        T* a = (T*)ar.p[" << base << " + " << o.ptr << "];\n#pragma unroll\n";
-          s << "        for (int i = 0; i < " << (n + movers - 1) / movers << "; ++i) {\n          const int sl = " << mtid << " + " << movers << " * i, qq = sl / NC, cc = sl % NC;\n          const i64 p = p0 + 4 * cc;\n";
+          s << "        for (int i = 0; i < " << (n + movers - 1) / movers << "; ++i) {\n          const int sl = " << mtid << " + " << movers << " * i, qq = sl / NC, cc = sl % NC;\n          const i64 p = p0 + " << (c.lone ? "" : "4 * ") << "cc;\n";
+          if (c.lone) {
+            s << "          if (sl < " << n << " && p < P) a[(i64)qq * P + p] = prv[" << o.off << " + cc * " << it.rows << " + qq];\n        }\n      }\n";
+            continue;
+          }
           s << "          if (sl < " << n << " && p < P) {\n            const A4 v = *reinterpret_cast<const A4*>(prv + " << o.off << " + cc * " << it.rows * 4 + 4 << " + qq * 4);\n";
           if (!whole4) s << "            if (p + 3 >= P) {\n#pragma unroll\n              for (int e = 0; e < 3; ++e)\n                if (p + e < P) a[(i64)qq * P + p + e] = v[e];\n            } else\n";
           s << "            *reinterpret_cast<V4*>(a + (i64)qq * P + p) = V4{v[0], v[1], v[2], v[3]};\n          }\n        }\n      }\n";
@@ -321,6 +340,85 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       }
       s << "        }\n";
     };
+    // Lone columns: a group of sixteen lanes has a quarter of k, an element a lane, and every lane its row's weights of that
+    // quarter; an element reaches its group as the broadcast operand of the multiplication (row_newbcast).  Two row groups side by side; their
+    // quarters meet by lane swaps, which leave the first group's sums in the lower half of the wavefront and the second's in the upper.
+    auto lone_products = [&](const std::vector<size_t>& js, int U) {
+      for (size_t j : js) {
+        const ChainItem& it = sec.items[j];
+        const std::string acc = "acc" + str((long long)j);
+        s << "        T " << acc << "[NC][" << 2 * ((U + 1) / 2) << "] = {};\n";
+        for (auto& x : it.x) {
+          const ChainMat& mt = c.mats[(size_t)x.mat];
+          const int nx = (mt.nf + 15) / 16;
+          s << "        {\n          T xr[NC][" << nx << "];\n";
+          if (x.kind == 2) s << "          const T xv = *(const T*)ar.p[at + " << x.ptr << "];\n";
+          else s << "          const T* xb = " << (x.kind == 1 ? "prv" : "cur") << " + " << x.off << " + kl;\n";
+          s << "#pragma unroll\n          for (int cc = 0; cc < NC; ++cc)\n#pragma unroll\n            for (int i = 0; i < " << nx << "; ++i) xr[cc][i] = ";
+          if (x.kind == 2) s << "64 * i + kl < " << x.K << " ? xv : T(0);\n";
+          else s << "xb[cc * " << x.rows << " + 64 * i];\n";
+          if (!mt.kept())
+            for (int u = 0; u < U; ++u)
+              s << "          T ws" << u << "[" << mt.nf << "];\n          frags<" << targs(mt) << mt.nf << ", false>((const T*)ar.p[" << x.mat << "], ws" << u << ", 0, 0, " << row_of(mt, u) << " + (lane & 15), g);\n";
+          auto weight = [&](int u, int f) {
+            if (!mt.kept()) return "ws" + str(u) + "[" + str(f) + "]";
+            if (f < mt.reg[u]) return "w" + str(x.mat) + "_" + str(u) + "[" + str(f) + "]";
+            return "lds[" + str(mt.lds[u] - 64 * mt.w0 + (f - mt.reg[u]) * 64 * mt.waves(u)) + " + tid]";
+          };
+          for (int f = 0; f < mt.nf; f += 8) {
+            const int n = std::min(8, mt.nf - f);
+            for (int u = 0; u < U; u += 2) {
+              const bool two = u + 1 < U;      // (a lone row group: two sums in turn, one after the other they would wait for each other)
+              for (int cc = 0; cc < NC; ++cc) {
+                s << "          asm(\"s_nop 1\\n\"\n";       // (two states between another write of the broadcast operand and its use, which the compiler does not see)
+                for (int e = 0; e < n; ++e)
+                  for (int a = 0; a < (two ? 2 : 1); ++a)
+                    s << "              \"v_fmac_f64_dpp %" << (two ? a : e & 1) << ", %2, %" << 3 + a * n + e << " row_newbcast:" << (f + e) % 16 << " row_mask:0xf bank_mask:0xf\\n\"\n";
+                s << "              \"s_nop 1\" : \"+v\"(" << acc << "[" << cc << "][" << u << "]), \"+v\"(" << acc << "[" << cc << "][" << u + 1 << "]) : \"v\"(xr[" << cc << "][" << f / 16 << "])";
+                for (int a = 0; a < (two ? 2 : 1); ++a)
+                  for (int e = 0; e < n; ++e) s << ", \"v\"(" << weight(u + a, f + e) << ")";
+                s << ");\n";
+              }
+            }
+          }
+          s << "        }\n";
+        }
+      }
+      s << "#pragma unroll\n        for (int cc = 0; cc < NC; ++cc) {\n          const i64 p = p0 + cc;\n";
+      for (size_t j : js) {
+        const ChainItem& it = sec.items[j];
+        const Spec& sp = it.kn->spec;
+        const ChainMat& m0 = c.mats[(size_t)it.x[0].mat];
+        for (int v = 0; 2 * v < U; ++v) {
+          const bool two = 2 * v + 1 < U;
+          const std::string sfx = "_" + str((long long)j) + "_" + str(v), acc = "acc" + str((long long)j) + "[cc][";
+          s << "          const int q" << sfx << " = " << pair_row(m0, v, U) << ";\n";
+          for (size_t i = 0; i < it.in.size(); ++i) {
+            const ChainIn& in = it.in[i];
+            s << "          const " << ctype(in.dtype) << " v" << i << sfx << " = ";
+            if (in.kind == 0) {
+              if (two) s << "meet(" << acc << 2 * v << "], " << acc << 2 * v + 1 << "]);\n";
+              else s << "meet(" << acc << 2 * v << "] + " << acc << 2 * v + 1 << "], " << acc << 2 * v << "] + " << acc << 2 * v + 1 << "]);\n";
+            } else if (in.kind == 1) s << "b" << j << "_" << i << "_" << v << ";\n";
+            else if (in.kind == 3) s << "e" << j << "_" << i << "_" << v << "[cc];\n";
+            else s << (in.kind == 2 ? "prv[" : "cur[") << in.off << " + cc * " << it.rows << " + q" << sfx << "];\n";
+          }
+          emit_program(s, sp.n_in, sp.n_instr, sp.prog, sp.dt, "          ", sfx);
+          // (a wavefront without the second group computes the first one's rows in both halves, the upper with that group's operands)
+          const std::string mine = two ? "" : "lane < 32 && ";
+          for (auto& o : it.out) {
+            if (o.staged) {
+              if (!two) s << "          if (lane < 32) ";
+              else s << "          ";
+              s << "cur[" << o.off << " + cc * " << it.rows << " + q" << sfx << "] = q" << sfx << " < " << it.Q << " ? v" << o.slot << sfx << " : T(0);\n";
+            } else {
+              s << "          if (" << mine << "q" << sfx << " < " << it.Q << " && p < P) ((" << ctype(o.dtype) << "*)ar.p[at + " << o.ptr << "])[(i64)q" << sfx << " * P + p] = v" << o.slot << sfx << ";\n";
+            }
+          }
+        }
+      }
+      s << "        }\n";
+    };
     std::vector<char> taken(sec.items.size(), 0);
     for (size_t j = 0; j < sec.items.size(); ++j) {
       if (sec.items[j].role != role || taken[j]) continue;
@@ -332,11 +430,11 @@ void chain_role(Src& s, const ChainPlan& c, int role) {
       s << "      ";
       if (rem < m0.nw) s << "if (w < " << m0.w0 + rem << ") ";
       s << "{\n";
-      products(js, m0.units);
+      c.lone ? lone_products(js, m0.units) : products(js, m0.units);
       s << "      }\n";
       if (rem < m0.nw && m0.units > 1) {
         s << "      else {\n";
-        products(js, m0.units - 1);
+        c.lone ? lone_products(js, m0.units - 1) : products(js, m0.units - 1);
         s << "      }\n";
       }
     }
@@ -386,6 +484,15 @@ std::string chain_source(const ChainPlan& c, const std::string& kname) {
   } else {
     s << "typedef T Acc;\n";
   }
+  if (c.lone) {
+    // The quarters of k, by groups of sixteen lanes: afterwards the lower half of the lanes holds the sums of a, the upper those of b.
+    s << "__device__ __forceinline__ T halves(T a, T b, bool far) {\n"
+         "  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);\n"
+         "  auto lo = far ? __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false) : __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);\n"
+         "  auto hi = far ? __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false) : __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);\n"
+         "  return __longlong_as_double((unsigned long long)hi[0] << 32 | lo[0]) + __longlong_as_double((unsigned long long)hi[1] << 32 | lo[1]);\n}\n"
+         "__device__ __forceinline__ T meet(T a, T b) {\n  const T s = halves(a, b, true);\n  return halves(s, s, false);\n}\n";
+  }
   // Four neighbouring columns from p on of a row that starts at a; past the end the last column (never stored)
   s << "template <i64 SP> __device__ __forceinline__ A4 cols(const T* __restrict__ a, i64 p) {\n  A4 v;\n";
   if (whole4) s << "  if constexpr (SP == 1) {\n    const V4 z = *reinterpret_cast<const V4*>(a + (p < P ? p : P - 4));\n    v = A4{z[0], z[1], z[2], z[3]};\n    return v;\n  }\n";
@@ -393,12 +500,13 @@ std::string chain_source(const ChainPlan& c, const std::string& kname) {
   s << "extern \"C\" __global__ void __launch_bounds__(512) " << kname << "(Args ar) {\n";
   s << "  __shared__ __attribute__((aligned(16))) T lds[" << c.lds_elems << "];\n";
   s << "  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, w = __builtin_amdgcn_readfirstlane(tid >> 6);\n";
-  if (c.f64) s << "  const int ql = 4 * ((lane >> 2) & 3) + g, pl = lane & 3;      // row and column of this lane's result\n";
+  if (c.lone) s << "  const int kl = 8 * ((lane & 15) >> 1) + 2 * g + (lane & 1);      // which of 64 k this lane holds for its group\n";
+  else if (c.f64) s << "  const int ql = 4 * ((lane >> 2) & 3) + g, pl = lane & 3;      // row and column of this lane's result\n";
   else s << "  const int ql = lane & 15, pl = g, qw = 4 * ((lane >> 2) & 3) + g, pw = lane & 3;      // (w: where sums are fp64)\n";
   // consecutive blocks go round the eight XCDs: neighbouring columns, whose lines of memory overlap, belong to one XCD
   const int64_t nblk = chain_blocks(c), per_xcd = (nblk + 7) / 8;
   s << "  const int blk = (int)(blockIdx.x % 8) * " << per_xcd << " + (int)(blockIdx.x / 8);\n  if (blk >= " << nblk << ") return;\n";
-  s << "  const i64 p0 = (i64)blk * (4 * NC);\n";
+  s << "  const i64 p0 = (i64)blk * (" << (c.lone ? "" : "4 * ") << "NC);\n";
   for (int role = 0; role < c.roles; ++role) {
     s << "  // ---- role " << role << "\n  ";
     if (role + 1 < c.roles) s << "if (w < " << role_end(c, role) << ") ";
@@ -568,9 +676,9 @@ bool place_weights(ChainPlan& c, int slack) {
       int ahead = 0, mine = 0, consts = 0, wide = 0;
       for (auto& it : s.items) {
         for (auto& x : it.x)
-          if (x.kind == 0 && movers) ahead += (x.rows * c.NC + movers - 1) / movers * 4;
+          if (x.kind == 0 && movers) ahead += (x.rows * c.NC + movers - 1) / movers * (c.lone ? 1 : 4);
         for (auto& in : it.in)
-          if (in.kind == 4 && movers) ahead += (it.rows * c.NC + movers - 1) / movers * 4;
+          if (in.kind == 4 && movers) ahead += (it.rows * c.NC + movers - 1) / movers * (c.lone ? 1 : 4);
         if (it.role != role) continue;
         const int units = c.mats[(size_t)it.x[0].mat].units;
         mine += units * c.NC * (c.f64 ? 1 : it.wide() ? 2 : 4);
@@ -594,7 +702,7 @@ bool place_weights(ChainPlan& c, int slack) {
         if (at > room) return false;
       }
   }
-  c.lds_elems = at + 16;
+  c.lds_elems = at + (c.lone ? 64 : 16);      // (lone columns are read 64 k at a time)
   return true;
 }
 
@@ -612,7 +720,7 @@ bool pays(const ChainPlan& c, int num_cu) {
       const bool d64 = c.f64 || it.wide();
       if (d64) after = 1.2e-6;
       for (auto& x : it.x) {
-        mul += (double)it.rows * x.rows * 4 * c.NC / (d64 ? 122e9 : 246e9);
+        mul += (double)it.rows * x.rows * chain_columns(c) / (c.lone ? 102e9 : d64 ? 122e9 : 246e9);
         flops += 2.0 * (double)it.Q * (double)x.K * (double)c.P / (d64 ? 33e12 : 49e12);
       }
     }
@@ -623,7 +731,7 @@ bool pays(const ChainPlan& c, int num_cu) {
 }
 
 // The plan of levels [l0, ...) as far as the kernel's arguments hold their pointers; *l1 is the first level left out.
-bool plan_chain(const std::vector<ChainCand>& cand, const std::vector<std::vector<int>>& levels, int num_cu, int slack, int l0, int* l1, ChainPlan* plan) {
+bool plan_chain(const std::vector<ChainCand>& cand, const std::vector<std::vector<int>>& levels, int num_cu, int slack, bool lone, int l0, int* l1, ChainPlan* plan) {
   ChainPlan& c = *plan;
   const Spec& first = cand[(size_t)levels[(size_t)l0][0]].d->kn->spec;
   c.f64 = first.f64;
@@ -790,15 +898,29 @@ bool plan_chain(const std::vector<ChainCand>& cand, const std::vector<std::vecto
         if (load[r].second == root((int)m)) c.mats[m].role = (int)r;
     c.roles = (int)load.size();
   }
-  // Columns per block: the fewest that let all blocks run at once, fewer when LDS or registers do not hold that many.
+  // Columns per block: the fewest that let all blocks run at once, fewer when LDS or registers do not hold that many.  fp64 by lone
+  // columns where one or two to a block are enough, two only where a wavefront has two row groups (with one, each column's program
+  // leaves half of the lanes idle).  Gradients of two layers over 28 steps, groups of four / lone, us: 128 wide, batch 40 250 / 166, 150 244 / 156, 256
+  // 255 / 164, 300 257 / 204, 500 275 / 225; 64 wide, batch 150 134 / 112, 512 149 / 158; 160 wide, 12 steps, batch 150 288 / 280.
   const int64_t groups = (c.P + 3) / 4;
   const int64_t rounds = (groups + 8 * (int64_t)num_cu - 1) / (8 * (int64_t)num_cu);
   // With a wavefront's registers and LDS too few for the weights of its own layer, every wavefront takes all layers.
-  for (int nc = (int)((groups + num_cu * rounds - 1) / (num_cu * rounds)), apart = 1; nc >= 1; apart ? apart = 0 : (--nc, apart = 1)) {
+  struct Form { bool lone; int nc, apart; };
+  std::vector<Form> forms;
+  if (c.f64 && lone)
+    for (int nc = (int)((c.P + num_cu - 1) / num_cu); nc <= kChainMaxLone; ++nc)
+      for (int apart = 1; apart >= 0; --apart) forms.push_back({true, nc, apart});
+  for (int nc = (int)((groups + num_cu * rounds - 1) / (num_cu * rounds)); nc >= 1; --nc)
+    for (int apart = 1; apart >= 0; --apart) forms.push_back({false, nc, apart});
+  for (const Form& f : forms) {
+    const bool apart = f.apart != 0;
     if (apart && c.roles == 1) continue;
     ChainPlan t = c;
-    t.NC = nc;
-    if (!share_wavefronts(t, apart != 0) || !place_weights(t, slack) || !pays(t, num_cu)) continue;
+    t.lone = f.lone;
+    t.NC = f.nc;
+    if (!share_wavefronts(t, apart)) continue;
+    if (t.lone && t.NC > 1 && std::any_of(t.mats.begin(), t.mats.end(), [](const ChainMat& m) { return m.kept() && m.units < 2; })) continue;
+    if (!place_weights(t, slack) || !pays(t, num_cu)) continue;
     // operands from inside the chain: where the level before put that result
     for (size_t k = 0; k < t.sections.size(); ++k) {
       // (the level before the section's first one, and within the section the section itself, which has the same layout)
@@ -824,7 +946,7 @@ hipFunction_t chain_kernel(hgpu_ctx* ctx, const ChainPlan& plan) {
   auto& chains = known_of(ctx).chains;
   const Key key = chain_key(plan);
   char kname[80];
-  snprintf(kname, sizeof kname, "smallk_chain_%s_p%lld_t%d_s%d", plan.f64 ? "f64" : "f32", (long long)plan.P, 4 * plan.NC, (int)plan.sections.size());
+  snprintf(kname, sizeof kname, "smallk_chain_%s_p%lld_t%d_s%d", plan.f64 ? "f64" : "f32", (long long)plan.P, chain_columns(plan), (int)plan.sections.size());
   auto it = chains.find(key.bytes);
   if (it != chains.end()) {
     if (check_keys() && it->second.src != chain_source(plan, kname)) {

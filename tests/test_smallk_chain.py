@@ -37,6 +37,14 @@ def step_bound(dt, ks):
     (16, 5000, 28, 10, 1),      # one row group, 20 columns a block
     (40, 700, 48, 9, 3),        # three layers: four, two and two wavefronts
     (100, 515, 33, 8, 2),
+    # fp64 by lone columns, one and two to a block
+    (128, 256, 28, 8, 2),       # a block for every CU
+    (128, 511, 28, 8, 2),       # two columns, the last block has one
+    (100, 257, 33, 8, 2),       # a wavefront with one row group beside those with two
+    (130, 200, 5, 8, 1),        # one layer
+    (17, 131, 30, 9, 2),        # the second row group one row high
+    (40, 61, 70, 9, 3),         # k of no whole 64, three layers
+    (64, 512, 17, 8, 2),        # two columns with one row group a wavefront: in groups of four
 ])
 def test_recurrence_forward(gpu, dt, width, batch, k_in, steps, layers):
     rng = np.random.default_rng(width + batch)
@@ -66,6 +74,9 @@ def test_recurrence_forward(gpu, dt, width, batch, k_in, steps, layers):
 
     (hs, out), n, labels = chains(gpu, work)
     assert n == 1, labels
+    if dt == np.float64 and layers > 1:      # lone columns where one or two to each of 256 CUs are enough
+        lone = 1 if batch <= 256 else 2 if batch <= 512 and width > 64 else None
+        assert any(",t%d]" % lone in k for k in labels) if lone else not any(",t1]" in k or ",t2]" in k for k in labels), labels
     for l in range(layers):
         for t in range(steps):
             x = (xs[t] if l == 0 else hs[l - 1][t]).astype(np.float64)
@@ -81,7 +92,7 @@ def test_recurrence_forward(gpu, dt, width, batch, k_in, steps, layers):
 
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
-@pytest.mark.parametrize("width,batch,steps", [(128, 150, 9), (48, 1030, 10), (40, 701, 10), (100, 250, 9)])
+@pytest.mark.parametrize("width,batch,steps", [(128, 150, 9), (48, 1030, 10), (40, 701, 10), (100, 250, 9), (72, 203, 10), (128, 301, 9)])
 def test_recurrence_backward(gpu, dt, width, batch, steps):
     """d2_t = (V2^T d2_(t+1)) * (1 - h2_t^2) + d2_(t+1), d1_t = (W2^T d2_t + V1^T d1_(t+1)) * (1 - h1_t^2): weights transposed,
     whole arrays as inputs of the program, among them a result of the chain."""
@@ -163,12 +174,13 @@ def test_what_breaks_a_chain(gpu, dt):
             prev = g.astype(np.float64)
 
 
-def test_values_that_are_no_numbers_stay_in_their_column(gpu):
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_values_that_are_no_numbers_stay_in_their_column(gpu, dt):
     """Infinities and NaN in some columns of the input reach the results of those columns only."""
     rng = np.random.default_rng(6)
     n, b, steps = 80, 203, 9
-    w = rng.uniform(-0.3, 0.3, (n, n)).astype(np.float32)
-    x = rng.uniform(-1, 1, (n, b)).astype(np.float32)
+    w = rng.uniform(-0.3, 0.3, (n, n)).astype(dt)
+    x = rng.uniform(-1, 1, (n, b)).astype(dt)
     x[3, 7], x[79, 100], x[0, 202] = np.inf, np.nan, -np.inf
     wa, h = gpu.upload(w), gpu.upload(x)
 
