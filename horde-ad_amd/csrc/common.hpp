@@ -272,6 +272,11 @@ hipError_t launch_reduction_group(hgpu_ctx* ctx, const RedJob* const* jobs, int 
 struct WideJob;
 // gemm.hip: launches up to kMaxWideJobs products of one kernel (the caller holds launch_mu)
 hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n);
+bool longer_wide_shares(hgpu_ctx* ctx, const WideJob* const* jobs, int n, int* shares);
+void set_wide_shares(WideJob& job, int shares);      // of a term's K
+int wide_shares(const WideJob& job);                 // of all terms: as many partial results
+const void* wide_partials(const WideJob& job);
+const void* wide_row_partials(const WideJob& job);   // null: none
 constexpr int kMaxWideJobs = 4;
 // gemm.hip: row sums that a held product hands out beside its result (see join_wide_rows)
 int wide_row_shares(const WideJob& job, int dtype, int n, const void* const* as, int64_t M, int64_t K, int64_t row_stride);

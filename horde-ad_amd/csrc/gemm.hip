@@ -227,6 +227,8 @@ int gemm_direct(hgpu_ctx* ctx, GemmParams p, int dtype, const void* pa, const vo
   return HGPU_OK;
 }
 
+int wide_chunk(int K, int shares) { return ((K + shares - 1) / shares + 15) / 16 * 16; }
+
 // Products whose row, column, contracted and batch indices are single dims with strides that a 32-bit byte offset
 // reaches: fp32 on the bf16 matrix cores (gemm_split.hip), fp64 in tiles without address arithmetic (gemm_wide_f64.hip).
 int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* pa, const void* pb, hgpu_array* out, bool* handled, int n_terms, hgpu_array** partials_out,
@@ -311,7 +313,7 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
   }
   const int64_t BM = f64 ? 64 : 128, BN = thin ? 32 : BM;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  q.kchunk = (int)(((p.K + split - 1) / split + 15) / 16 * 16);
+  q.kchunk = wide_chunk(q.K, split);
   q.term_split = (int)((p.K + q.kchunk - 1) / q.kchunk);
   split = (int)(q.term_split * nt);
   if (split > 65535 || tiles * split > 0x3fffffff || (split > 1 && (double)out_n * split > 5e8)) return HGPU_OK;
@@ -437,6 +439,58 @@ bool classify_contraction(int rank, const int64_t* shape, const int64_t* st_a, c
   p->BT = total(p->bt);
   return true;
 }
+
+// Sums of as many products are a recurrence's; those of fewer keep, in a recording too, the shares of K and so the bits that
+// they have submitted one by one.
+constexpr int kRecurrenceTerms = 8;
+
+// Shares of K for fp32 products on tiles of 128 x 128 that go out together: each was cut to fill the device alone, and together they
+// take several rounds of short blocks, which fetch their first operands and leave partial results each.  Longer shares where
+// the model of the single product, with two blocks to a CU, says so; never more of them, so that the partial results have their memory.  False:
+// as they are.  The three products of 128 x 128 over 27 x 5000 of a recurrence, 18 / 9 / 6 / 5 / 4 / 3 shares a term (504 to 84 blocks each), us of its whole
+// gradient: 569 / 543 / 530 / 530 / 532 / 554.   (Products whose blocks differ in
+// length fill one another's gaps: 2048 x 784 and 2048 x 2048 over 8192, 57 and 256 steps, lost 12 us of their gradient by this model.  fp64 and thin products come
+// with more blocks to a CU, whose sums are short: not looked at.)
+// The gradients' error against fp64 does not grow (weights of 128 x 128 at batch 3000 to 5000, 28 steps: 8.8e-8 to 9.6e-8 of the
+// result before, 7.9e-8 to 9.5e-8 with fewer fp32 results to add up).
+bool longer_wide_shares(hgpu_ctx* ctx, const WideJob* const* jobs, int n, int* shares) {
+  const int slots = 2 * ctx->num_cu;
+  double first = 0, best = 1e300;
+  for (int d = 1; d <= 8; ++d) {
+    int64_t blocks = 0, steps = 0, least = INT64_MAX;
+    double sums = 0;
+    int cut[kMaxWideJobs];
+    for (int k = 0; k < n; ++k) {
+      const SplitJob& j = jobs[k]->j;
+      if (jobs[k]->f64 || jobs[k]->thin || j.p.n_terms < kRecurrenceTerms) return false;
+      cut[k] = (j.p.term_split + d - 1) / d;
+      const int64_t chunk = wide_chunk(j.p.K, cut[k]);
+      cut[k] = (int)((j.p.K + chunk - 1) / chunk);
+      const int64_t all = (int64_t)cut[k] * std::max(j.p.n_terms, 1);
+      blocks += j.tiles * all * j.batches;
+      steps = std::max(steps, chunk / 16);
+      least = std::min(least, chunk / 16);
+      sums += (double)j.p.c_split_stride * (double)all * 4 / 3.2e6;
+    }
+    const double us = (double)((blocks + slots - 1) / slots) * (double)steps * 1.84 + sums;
+    if (d == 1) {
+      if (4 * steps > 5 * least) return false;      // (blocks of different length fill one another's gaps)
+      first = us;
+    }
+    if (us >= best) continue;
+    best = us;
+    std::copy(cut, cut + n, shares);
+  }
+  return best < 0.97 * first;
+}
+void set_wide_shares(WideJob& job, int shares) {
+  job.j.p.kchunk = wide_chunk(job.j.p.K, shares);
+  job.j.p.term_split = shares;
+  job.j.splits = shares * std::max(job.j.p.n_terms, 1);
+}
+int wide_shares(const WideJob& job) { return job.j.splits; }
+const void* wide_partials(const WideJob& job) { return job.j.C; }
+const void* wide_row_partials(const WideJob& job) { return job.j.p.rows; }
 
 hipError_t launch_wide_group(hgpu_ctx* ctx, const WideJob* const* jobs, int n) {
   SplitGroup g;

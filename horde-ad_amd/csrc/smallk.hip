@@ -1144,6 +1144,28 @@ static void launch_held_locked(hgpu_ctx* ctx, std::vector<Deferred>& items, Defe
           bytes += wide[g1]->bytes;
           flops += wide[g1]->flops;
         }
+        // Longer shares of K for all of them, where whoever adds up their partial results waits here too and hears of it
+        int shares[kMaxWideJobs];
+        if (n > 1 && longer_wide_shares(ctx, jobs, n, shares)) {
+          std::vector<std::pair<Deferred*, int>> sums;
+          bool all = true;
+          for (int k = 0; all && k < n; ++k) {
+            Deferred& w = *wide[g1 - (size_t)n + (size_t)k];
+            size_t found = 0;
+            for (auto& d : items)
+              for (auto* b : w.writes) {
+                if (std::find(d.reads.begin(), d.reads.end(), b) == d.reads.end()) continue;
+                const bool own = d.is_reduction && d.red.is_sum() && d.red.R == wide_shares(*w.wide) && (d.red.a == wide_partials(*w.wide) || d.red.a == wide_row_partials(*w.wide));
+                all = all && own;
+                if (own) sums.push_back({&d, k}), ++found;
+              }
+            all = all && found == w.writes.size();      // (a product that is in one piece has no sum)
+          }
+          if (all) {
+            for (int k = 0; k < n; ++k) set_wide_shares(*wide[g1 - (size_t)n + (size_t)k]->wide, shares[k]);
+            for (auto& s : sums) s.first->red.R = wide_shares(*jobs[s.second]);
+          }
+        }
         if (ctx->profiling) {
           std::string lab = n > 1 ? "gemm_wide_group[" : "";
           for (size_t i = g0; i < g1; ++i) lab += (i > g0 ? "|" : "") + std::string(wide[i]->label) + (wide_takes_rows(*wide[i]->wide) ? "+rows" : "");

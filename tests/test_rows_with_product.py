@@ -185,3 +185,47 @@ def test_two_threads_ask_for_the_same_rows():
             assert np.all(np.abs(s.numpy() - w) <= (2.0 ** -24 + k * 2.0 ** -53) * size)
         del p, sums, s
         ctx.check(ctx.lib.dll.hgpu_graph_destroy(g))
+
+
+@pytest.mark.parametrize("t,sizes", [(8, [(128, 128)] * 3), (9, [(128, 100), (128, 128)]), (8, [(130, 96)] * 4), (7, [(128, 128)] * 3)])
+def test_products_of_a_recurrence_together(host, t, sizes):
+    """Weight gradients of eight and more terms that go out together take longer shares of K than each by itself, and the sums of
+    their partial results, with the row sums beside them, go by the new shares."""
+    rng = np.random.default_rng(t + len(sizes))
+    k = 5003
+    xs, ys = [], []
+    for m, n in sizes:
+        xs.append([rng.uniform(-1, 1, (m, k)).astype(np.float32) for _ in range(t)])
+        ys.append([rng.uniform(-1, 1, (k, n)).astype(np.float32) for _ in range(t)])
+    a, b = [[host.concrete(x) for x in x1] for x1 in xs], [[host.concrete(y) for y in y1] for y1 in ys]
+
+    def program():
+        products = []
+        for a1, b1 in zip(a, b):
+            s = a1[0].smatmul2(b1[0])
+            for u, v in zip(a1[1:], b1[1:]):
+                s = s + u.smatmul2(v)
+            products.append(s)
+        held.force(host, *products)
+        total = rows(a[0][0])
+        for u in a[0][1:]:
+            total = total + rows(u)
+        return products + [total]
+
+    eager = [v.numpy() for v in program()]
+    graph, res, labels = held.recorded(host, program)
+    together = [s for s in labels if s.startswith("gemm_wide_group[")]
+    assert len(together) == 1 and together[0].count("|") == len(sizes) - 1, labels
+    want = [sum(x.astype(np.float64) @ y for x, y in zip(x1, y1)) for x1, y1 in zip(xs, ys)] + [sum(x.sum(1, dtype=np.float64) for x in xs[0])]
+    size = [sum(np.abs(x).astype(np.float64) @ np.abs(y) for x, y in zip(x1, y1)) for x1, y1 in zip(xs, ys)] + [sum(np.abs(x).sum(1, dtype=np.float64) for x in xs[0])]
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            for got, e, w, s in zip(res, eager, want, size):
+                # sixteen products to a rounded addition, and the sum of the partial results
+                assert np.all(np.abs(got.numpy() - w) <= (t * k / 16 + 17) * 2.0 ** -24 * s)
+                assert t >= 8 or e.ndim < 2 or np.array_equal(got.numpy(), e)      # fewer terms: the bits of the products one by one
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
