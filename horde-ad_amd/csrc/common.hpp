@@ -301,6 +301,17 @@ std::shared_ptr<HeldJob> held_writer_locked(hgpu_ctx* ctx, const hgpu_buffer* b)
 bool extend_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);
 // ... goes out now; forgotten: it does not (another launch has done its work)
 void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, bool forgotten);
+// A zero-extension (ewise.hip) that waits until something reads its result: a kernel that copies its operand to LDS reads the
+// array that is extended instead (footprint.hip).  Dims as they lie in the dense result, from dst on.
+struct PadJob : HeldJob {
+  int dtype, nd;
+  int64_t shape[HG_KDIMS], lo[HG_KDIMS], ext[HG_KDIMS], sst[HG_KDIMS];      // of the result; zeros in front; of the source, and its strides
+  int64_t n;                   // elements of the result
+  hgpu_buffer* src_buf;        // (kept by the queue as long as the job waits)
+  const void* src;
+  void* dst;
+  hipError_t launch(hgpu_ctx* ctx, hipEvent_t start, hipEvent_t stop) override;
+};
 // fused.hip: holds the extremum of one dense row back, to be one launch with the sums over the same elements that follow; false: left to the caller
 bool try_hold_extremum(hgpu_ctx* ctx, const hgpu_array* a, int want_max, const hgpu_array* index, const hgpu_array* value);
 // contract.hip: the extremum of one row by a block (the caller holds launch_mu)

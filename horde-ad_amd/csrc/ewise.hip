@@ -309,6 +309,31 @@ inline int layout_class(const hgpu_array* a) {
 
 inline int max_blocks(hgpu_ctx* ctx) { return ctx->num_cu * 8; }
 
+// rows whose extents, paddings and addresses are all multiples of 16 bytes move as 16-byte elements
+hipError_t launch_pad(hgpu_ctx* ctx, PadDims d, int64_t n, size_t es, const void* src, void* dst) {
+  const int64_t f = 16 / (int64_t)es;
+  const int in = d.nd - 1;
+  bool wide = es < 16 && d.sst[in] == 1 && d.shape[in] % f == 0 && d.lo[in] % f == 0 && d.ext[in] % f == 0 && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
+  for (int i = 0; i < in && wide; ++i) wide = d.sst[i] % f == 0;
+  if (wide) {
+    d.shape[in] /= f;
+    d.lo[in] /= f;
+    d.ext[in] /= f;
+    for (int i = 0; i < in; ++i) d.sst[i] /= f;
+    n /= f;
+    es = 16;
+  }
+  unsigned g = grid_for(n, kBlock, max_blocks(ctx));
+  switch (es) {
+    case 16: hipLaunchKernelGGL(k_pad<Bytes16>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const Bytes16*)src, (Bytes16*)dst); break;
+    case 8: hipLaunchKernelGGL(k_pad<uint64_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint64_t*)src, (uint64_t*)dst); break;
+    case 4: hipLaunchKernelGGL(k_pad<uint32_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint32_t*)src, (uint32_t*)dst); break;
+    case 2: hipLaunchKernelGGL(k_pad<uint16_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint16_t*)src, (uint16_t*)dst); break;
+    default: hipLaunchKernelGGL(k_pad<uint8_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint8_t*)src, (uint8_t*)dst); break;
+  }
+  return hipGetLastError();
+}
+
 }  // namespace
 
 namespace hg {
@@ -377,6 +402,16 @@ int copy_view(hgpu_ctx* ctx, int dtype, int rank, const int64_t* shape, const vo
   return HGPU_OK;
 }
 
+hipError_t PadJob::launch(hgpu_ctx* ctx, hipEvent_t start, hipEvent_t stop) {
+  PadDims d;
+  d.nd = nd;
+  for (int i = 0; i < nd; ++i) { d.shape[i] = shape[i]; d.lo[i] = lo[i]; d.ext[i] = ext[i]; d.sst[i] = sst[i]; }
+  if (start) (void)hipEventRecord(start, ctx->stream);
+  const hipError_t e = launch_pad(ctx, d, n, dtype_size(dtype), src, dst);
+  if (stop) (void)hipEventRecord(stop, ctx->stream);
+  return e;
+}
+
 }  // namespace hg
 
 extern "C" {
@@ -391,6 +426,10 @@ int hgpu_materialize(hgpu_ctx* ctx, const hgpu_array* a, hgpu_array** out) {
   *out = o;
   return HGPU_OK;
 }
+
+// Zero-extensions of floats from here on wait (elements of the result): a product that reads less is too small for the kernel that
+// does without them.
+constexpr int64_t kPadsWait = 16384;
 
 int hgpu_pad(hgpu_ctx* ctx, const hgpu_array* a, const int64_t* lo, const int64_t* hi, hgpu_array** out) {
   if (!ctx || !a || !out) return HGPU_ERR_INVALID;
@@ -453,33 +492,23 @@ int hgpu_pad(hgpu_ctx* ctx, const hgpu_array* a, const int64_t* lo, const int64_
       snprintf(buf + w, sizeof buf - w, "]");
       label = intern_label(ctx, buf);
     }
+    const double bytes = (double)(n + nelem(a)) * dtype_size(a->dtype);
+    if (dtype_is_float(a->dtype) && n >= kPadsWait && nelem(a) > 0) {
+      auto job = std::make_shared<PadJob>();
+      job->label = label;
+      job->bytes = bytes;
+      job->dtype = a->dtype;
+      job->nd = d.nd;
+      for (int i = 0; i < d.nd; ++i) { job->shape[i] = d.shape[i]; job->lo[i] = d.lo[i]; job->ext[i] = d.ext[i]; job->sst[i] = d.sst[i]; }
+      job->n = n;
+      job->src_buf = a->buf;
+      job->src = data_ptr(a);
+      job->dst = data_ptr(o);
+      if (hold_job(ctx, job, {a->buf}, {o->buf}, true)) { *out = o; return HGPU_OK; }
+    }
     const Reads reads = reads_of(1, &a);
-    LaunchGuard lg(ctx, label, (double)(n + nelem(a)) * dtype_size(a->dtype), 0, &reads);
-    const void* src = data_ptr(a);
-    void* dst = data_ptr(o);
-    // rows whose extents, paddings and addresses are all multiples of 16 bytes move as 16-byte elements
-    size_t es = dtype_size(a->dtype);
-    const int64_t f = 16 / (int64_t)es;
-    const int in = d.nd - 1;
-    bool wide = es < 16 && d.sst[in] == 1 && d.shape[in] % f == 0 && d.lo[in] % f == 0 && d.ext[in] % f == 0 && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
-    for (int i = 0; i < in && wide; ++i) wide = d.sst[i] % f == 0;
-    if (wide) {
-      d.shape[in] /= f;
-      d.lo[in] /= f;
-      d.ext[in] /= f;
-      for (int i = 0; i < in; ++i) d.sst[i] /= f;
-      n /= f;
-      es = 16;
-    }
-    unsigned g = grid_for(n, kBlock, max_blocks(ctx));
-    switch (es) {
-      case 16: hipLaunchKernelGGL(k_pad<Bytes16>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const Bytes16*)src, (Bytes16*)dst); break;
-      case 8: hipLaunchKernelGGL(k_pad<uint64_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint64_t*)src, (uint64_t*)dst); break;
-      case 4: hipLaunchKernelGGL(k_pad<uint32_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint32_t*)src, (uint32_t*)dst); break;
-      case 2: hipLaunchKernelGGL(k_pad<uint16_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint16_t*)src, (uint16_t*)dst); break;
-      default: hipLaunchKernelGGL(k_pad<uint8_t>, dim3(g), dim3(kBlock), 0, ctx->stream, d, n, (const uint8_t*)src, (uint8_t*)dst); break;
-    }
-    hipError_t e = hipGetLastError();
+    LaunchGuard lg(ctx, label, bytes, 0, &reads);
+    const hipError_t e = launch_pad(ctx, d, n, dtype_size(a->dtype), data_ptr(a), data_ptr(o));
     if (e != hipSuccess) { hgpu_release(o); return check_hip(ctx, e, "pad"); }
   }
   *out = o;

@@ -80,10 +80,13 @@ std::vector<T> Tape::backward(const D& out, const T& dt_or_none, const std::vect
     ~Scope() { unit_factors = before; }
   };
   T dt = dt_or_none;
+  if (out.node >= (int)recs.size()) throw HostError(HGPU_ERR_INVALID, "backward: the value's tape has been reset");
   std::vector<T> slots(recs.size());
   std::vector<bool> keep(recs.size(), false);
-  for (auto& i : inputs)
+  for (auto& i : inputs) {
+    if (i.node >= (int)recs.size()) throw HostError(HGPU_ERR_INVALID, "backward: an input's tape has been reset");
     if (i.node >= 0) keep[(size_t)i.node] = true;
+  }
   if (out.node >= 0) {
     if (!dt.valid()) dt = broadcast_scalar(seed_one(be, out.primal.dtype()), out.primal.shape());
     if (dt.shape() != out.primal.shape()) throw HostError(HGPU_ERR_INVALID, "backward: cotangent shape differs from the result's");

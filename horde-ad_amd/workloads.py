@@ -183,7 +183,9 @@ class Workload:
         host.tape_reset()
         ps = [p.as_input() for p in ps]    # parameters are fresh tape inputs for every gradient
         loss = self.objective(ps, ds)
-        return loss, host.grad(loss, ps)
+        grads = host.grad(loss, ps)
+        host.tape_reset()                  # what only the tape held is not waited for
+        return loss, grads
 
 
 def c0_elementwise(n=4096, m=4096, dtype=F64):
