@@ -887,7 +887,8 @@ struct VirtualOp {
 // The kernel then copies that array's elements to LDS and zeros around them; the extension is never written where nobody else
 // reads it.  The place of a staged vector in the array that is extended is worked out once a lane, zeros are a select, and a
 // footprint is fetched without its zeros: the second layer's forward product of the 28 x 28 network (1000 images of 16 x 14 x 14 fp64,
-// extended to 18 x 18) takes 55.7 us for 54.8 before, its kernel gradient 53.9 for 56.6, and the extension of 12.6 us does not happen.
+// extended to 18 x 18) takes 55.7 us for 54.8 before, its kernel gradient 53.9 for 56.6, and the extension of 12.6 us does not happen; of the
+// first layer onehot_contract 31.2 for 31.9, the extension 5.6.
 struct Extended {
   VirtualOp v;
   hgpu_array* in = nullptr;
@@ -2342,7 +2343,8 @@ struct OnehotKnown {
 };
 
 // The plan and the kernel's text for x (an array) times the expression v seen through yo; kn->taken stays false when the kernel does not fit.
-void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo, int n_keep, int64_t out_n, int which_in, int where_in, OnehotKnown* kn, std::string* text) {
+// (ext: x as a zero-extension that waits, or null)
+void plan_onehot(const hgpu_array* x, const Extended* ext, const VirtualOp& v, const hgpu_operand* yo, int n_keep, int64_t out_n, int which_in, int where_in, OnehotKnown* kn, std::string* text) {
   const int rank = yo->rank;
   const size_t re = v.E.size(), rm = v.M.size();
   // ---- the one-hot dims of the inputs' shape: where `which` moves; `where` must stand still there
@@ -2471,6 +2473,7 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
   const int64_t span = hi - lo + 1;
   const int es = v.dtype == HGPU_F64 ? 8 : 4;
   if (span * es > 64 * 1024 || span < 1) return;
+  if (ext && span > 16 * 256) return;                  // (a thread keeps the places of the elements it stages)
   for (int64_t a : gy) if (a < 0 || a > INT32_MAX) return;
   const VD& chd = vd[(size_t)chunk];
   const int64_t nch = chd.e, chx = chd.sx, chy = chd.sy;
@@ -2517,10 +2520,13 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
   if (!fits32) return;
   Src s;
   char kname[160];
-  snprintf(kname, sizeof kname, "onehot_contract_%s_m%d_n%d_k%lldx%lld_onehot%lld", es == 8 ? "f64" : "f32", MR, NC, (long long)nch, (long long)G, (long long)EH);
+  snprintf(kname, sizeof kname, "onehot_contract_%s_m%d_n%d_k%lldx%lld_onehot%lld%s", es == 8 ? "f64" : "f32", MR, NC, (long long)nch, (long long)G, (long long)EH, ext ? "_xmap" : "");
   s << "typedef long long i64;\n";
   s << "typedef " << (es == 8 ? "double" : "float") << " T;\n";
   s << hg::fusedgen::kPrelude;
+  const int64_t xbase = ext ? ext->offset + lo : 0;
+  if (ext) s << "template <int> using Vec = T;\n" << vops_source(ext->v, "x", 1, chx, xbase + (nch - 1) * chx + span);
+  const int n_stage = (int)((span + 255) / 256);
   auto itab = [&](const std::string& name, const std::vector<int64_t>& t, int64_t shift) {
     std::vector<int> t2;
     for (int64_t a : t) t2.push_back((int)(a - shift));
@@ -2546,7 +2552,7 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
   static const int knob_batch = getenv("HORDEAD_ONEHOT_BATCH") ? atoi(getenv("HORDEAD_ONEHOT_BATCH")) : 16;
   const int RB = 4;       // rows of the result added up per round at the end
   const int MA = MR + 1;  // the rows, and the plain sum of the expression's values per column
-  s << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "(const T* __restrict__ X, Ins ins, T* __restrict__ part) {\n";
+  s << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "(const T* __restrict__ X, Ins ins, T* __restrict__ part" << (ext ? ", VArgs_x vax" : "") << ") {\n";
   s << "  __shared__ T xs[" << span << "];\n  __shared__ T red[" << RB * 256 << "];\n";
   s << "  const int tid = threadIdx.x, col = tid / " << TPC << ", li = tid % " << TPC << ";\n  const int cq = col < " << NC << " ? col : 0;\n";
   for (int i = 0; i < v.n_in; ++i) {
@@ -2554,6 +2560,9 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
     else if (rep[(size_t)i] == i) s << "  const int c" << i << " = kCol" << i << "[cq];\n";
   }
   s << "  T acc[" << MA << "];\n#pragma unroll\n  for (int m = 0; m < " << MA << "; ++m) acc[m] = T(0);\n";
+  if (ext)
+    s << "  const VHoist_x hsx = vhoist_x(vax);\n  VPre_x vpx[" << n_stage << "];\n#pragma unroll\n  for (int j = 0; j < " << n_stage << "; ++j) vpx[j] = vpre_x(" << xbase
+      << "ll + (tid + 256 * j < " << span << " ? tid + 256 * j : " << span - 1 << "));\n";
   // A thread's positions of a chunk are taken a batch at a time: all the loads of `where`, then all the loads
   // of the expression's inputs at the places they name, then the multiplications -- each step's trips to memory overlap.
   // When one batch holds all of a thread's positions, its loads of `where` are issued before the chunk's footprint
@@ -2571,7 +2580,11 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
   s << "  for (i64 ch = blockIdx.x; ch < " << nch << "ll; ch += gridDim.x) {\n";
   if (early_where) where_loads("li");
   s << "    __syncthreads();\n";
-  s << "    for (int u = tid; u < " << span << "; u += 256) xs[u] = X[ch * " << chx << "ll + u];\n";
+  if (ext)
+    s << "    {\n      VRaw_x raw[" << n_stage << "];\n#pragma unroll\n      for (int j = 0; j < " << n_stage << "; ++j) raw[j] = vfetch_x(vax, vpx[j], ch);\n#pragma unroll\n      for (int j = 0; j < "
+      << n_stage << "; ++j)\n        if (tid + 256 * j < " << span << ") xs[tid + 256 * j] = vfinish_x(hsx, vpx[j], raw[j]);\n    }\n";
+  else
+    s << "    for (int u = tid; u < " << span << "; u += 256) xs[u] = X[ch * " << chx << "ll + u];\n";
   s << "    __syncthreads();\n";
   s << "    if (col < " << NC << ") {\n";
   if (early_where) {
@@ -2632,7 +2645,7 @@ void plan_onehot(const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo
 }
 
 // x: the operand that is an array; y: the expression operand.  Both seen through views of `rank` dims of one shape.
-int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, const hgpu_operand* yo, int n_keep, hgpu_array* out, bool* handled) {
+int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const Extended* ext, const VirtualOp& v, const hgpu_operand* yo, int n_keep, hgpu_array* out, bool* handled) {
   *handled = false;
   static const bool disabled = getenv("HORDEAD_NO_ONEHOT") != nullptr;
   if (disabled) return HGPU_OK;
@@ -2642,7 +2655,8 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
   if (!onehot_gate(v, v.slot, &which_in, &where_in)) return HGPU_OK;
   const int64_t out_n = nelem(out);
   Key key;
-  key.put(which_in).put(where_in).put(x->dtype).put(x->rank, x->shape).put(x->rank, x->strides).put((int)((uintptr_t)data_ptr(x) & 63));
+  key.put(which_in).put(where_in).put(x->dtype).put(x->rank, x->shape).put(x->rank, x->strides).put((int)((uintptr_t)data_ptr(x) & 63)).put(ext != nullptr);
+  if (ext) { put_virtual(key, ext->v, 1, 0, 0); key.put(ext->offset); }
   put_virtual(key, v, 0, 0, 0);
   for (int i = 0; i < v.n_in; ++i) key.put(v.in[i]->offset);
   key.put(yo->rank, yo->shape).put(yo->rank, yo->strides).put(yo->offset).put(n_keep).put(out_n);
@@ -2653,7 +2667,7 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
   if (found == known.end() || check_keys()) {
     OnehotKnown fresh;
     std::string text;
-    plan_onehot(x, v, yo, n_keep, out_n, which_in, where_in, &fresh, &text);
+    plan_onehot(x, ext, v, yo, n_keep, out_n, which_in, where_in, &fresh, &text);
     if (found != known.end()) {
       if (fresh.taken != found->second.taken || (fresh.taken && text != found->second.text)) return fail(ctx, HGPU_ERR_DEVICE, "onehot_contract: two different kernels under one key");
     } else {
@@ -2694,7 +2708,9 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
   void* pdst = part->ptr;
   std::vector<const void*> ia;
   for (int i = 0; i < v.n_in; ++i) ia.push_back(data_ptr(v.in[i]));
-  void* args[] = {(void*)&xp, (void*)ia.data(), (void*)&pdst};
+  const void* xa = ext ? data_ptr(ext->in) : nullptr;
+  void* args[] = {(void*)&xp, (void*)ia.data(), (void*)&pdst, (void*)&xa};
+  if (ext) xp = nullptr;
   {
     double bytes = (double)nch * span * es;
     for (int i = 0; i < v.n_in; ++i) {
@@ -2711,8 +2727,13 @@ int try_onehot_contract(hgpu_ctx* ctx, const hgpu_array* x, const VirtualOp& v, 
       label = intern_label(ctx, buf);
     }
     Reads reads(ia);
-    reads.push_back(data_ptr(x));
+    reads.push_back(ext ? xa : data_ptr(x));
     LaunchGuard lg(ctx, label, bytes, 2.0 * MR * NC * (double)G * (double)nch, &reads);
+    if (ext && !ext->v.still_waits_locked(ctx)) {      // (another thread has sent the extension out)
+      buffer_release(part);
+      hgpu_release(colsum);
+      return HGPU_OK;
+    }
     hipError_t e = launch_module(lg, kn.c.fn, (unsigned)grid, 256, args);
     if (e != hipSuccess) { buffer_release(part); hgpu_release(colsum); return check_hip(ctx, e, "onehot_contract launch"); }
   }
@@ -2780,9 +2801,15 @@ extern "C" int hgpu_contract_operands(hgpu_ctx* ctx, const hgpu_operand* a, cons
       }
       rc = try_mapped_sum(ctx, va, a, n_keep, o, &handled);
     } else if ((a->array || va.total < (1LL << 31)) && (b->array || vb.total < (1LL << 31))) {
+      Extended ext;
+      ext.find(ctx, a->array ? a->array : b->array ? b->array : nullptr);
       // one operand an array, the other an expression that is one-hot along contracted dims
-      if (a->array && !b->array) rc = try_onehot_contract(ctx, a->array, vb, b, n_keep, o, &handled);
-      else if (b->array && !a->array) rc = try_onehot_contract(ctx, b->array, va, a, n_keep, o, &handled);
+      auto onehot = [&](const Extended* e) {
+        if (a->array && !b->array) rc = try_onehot_contract(ctx, a->array, e, vb, b, n_keep, o, &handled);
+        else if (b->array && !a->array) rc = try_onehot_contract(ctx, b->array, e, va, a, n_keep, o, &handled);
+      };
+      if (ext) onehot(&ext);
+      if (!rc && !handled) onehot(nullptr);
       if (rc || handled) {
         if (rc) hgpu_release(o); else *out = o;
         return rc;
@@ -2794,8 +2821,6 @@ extern "C" int hgpu_contract_operands(hgpu_ctx* ctx, const hgpu_operand* a, cons
         const size_t es = dtype_size(dtype);
         const void* pa = a->array ? data_ptr(a->array) : (const void*)(uintptr_t)(a->offset * (int64_t)es);
         const void* pb = b->array ? data_ptr(b->array) : (const void*)(uintptr_t)(b->offset * (int64_t)es);
-        Extended ext;
-        ext.find(ctx, a->array ? a->array : b->array ? b->array : nullptr);
         const void* pe = (const void*)(uintptr_t)(ext.offset * (int64_t)es);
         if (ext) rc = hg::try_footprint_virtual(ctx, p, dtype, a->array ? pe : pa, a->array ? pb : pe, o, &handled, a->array ? &ext.v : &va, a->array ? &vb : &ext.v);
         if (!rc && !handled) rc = hg::try_footprint_virtual(ctx, p, dtype, pa, pb, o, &handled, a->array ? nullptr : &va, b->array ? nullptr : &vb);

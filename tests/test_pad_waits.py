@@ -160,3 +160,38 @@ def test_extensions_of_a_recording():
             [q.numpy() for q in program()]
     finally:
         graph.free()
+
+
+@pytest.mark.parametrize("batch,h,w,k,c,dt,written", [
+    (130, 28, 28, 5, 16, np.float64, 0),
+    (130, 28, 28, 5, 16, np.float32, 0),
+    (260, 20, 24, 3, 12, np.float64, None),
+    (260, 16, 32, 5, 8, np.float32, None),
+    (300, 32, 32, 5, 4, np.float64, None),
+])
+def test_gradients_of_convolutions(batch, h, w, k, c, dt, written):
+    """The network's gradient against numpy's, recorded and not; `written`: extensions that the recording writes."""
+    import ref_numpy
+    import test_held_sums as held
+    wl = pkg.workloads.c3_cnn(batch, pkg.capi.F64 if dt == np.float64 else pkg.capi.F32, h, w, k, c, 32)
+    host = pkg.hostapi.Host()
+    ps, ds = wl.upload(host)
+    program = lambda: (lambda loss, grads: [loss] + grads)(*wl.gradient(host, ps, ds))
+    eager = [v.numpy() for v in program()]
+    loss, grads = ref_numpy.cnn([p.astype(np.float64) for p in wl.params], *[d.astype(np.float64) for d in wl.data])
+    tol = 1e-11 if dt == np.float64 else 1e-4      # (single precision: an arg-maximum or a relu near its edge goes the other way)
+    for got, want in zip(eager, [np.asarray(loss)] + list(grads)):
+        assert np.max(np.abs(got - want)) <= tol * np.max(np.abs(want))
+    graph, res, labels = held.recorded(host, program)
+    pads = [n for n in labels if n.startswith("pad[")]
+    if written is not None:
+        assert len(pads) == written and any(n.startswith("onehot") for n in labels), labels
+    try:
+        for _ in range(3):
+            graph.launch()
+            host.sync()
+            for got, want in zip(res, eager):
+                assert np.max(np.abs(got.numpy() - want)) <= (1e-12 if dt == np.float64 else 1e-5) * np.max(np.abs(want))
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
