@@ -277,12 +277,16 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     // Microseconds, as measured: a step of 16 k of a 64 x 64 tile takes 0.62 alone on its CU, 0.56 with another one
     // there, 0.5 with more; 5 for the launch; partial results as below.  (300 x 784 over 5000, main kernel / with the
     // sums: 4 chunks = 260 blocks 82 / 89, 7 = 455 56 / 63, 10 = 650 54 / 63, 32 = 2080 52 / 65.)
+    // Partial results at 4 TB/s, between other kernels that want the caches too (6 TB/s when nothing else runs, and for the two
+    // or three that a program reads itself): gradients of dense 784-300-100-10, batch 5000, 6 / 4 TB/s 197.4 / 190.8 us (15 / 11 shares
+    // of the first weights' gradient), 784-2000-300-10, batch 1500, 385 / 380, 784-128-900-10, batch 3000, 192 / 187; at 2.5 TB/s
+    // 784-650-333-10, batch 4000, goes from 374 to 408.
     double best = 1e300;
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64) * p.BT * nt;
     for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
       const int64_t per_cu = (tiles * sp + ctx->num_cu - 1) / ctx->num_cu, steps = ((p.K + sp - 1) / sp + 15) / 16;
       const double step = per_cu == 1 ? 0.62 : per_cu == 2 ? 1.12 : 0.5 * per_cu;
-      const double us = 5 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 8 / 6e6 : 0);
+      const double us = 5 + steps * step + (sp * nt > 1 ? 6 + (double)out_n * (sp * nt + 1) * 8 / (partials_out && sp * nt <= 3 ? 6e6 : 4e6) : 0);
       if (us < best) { best = us; split = (int)sp; }
     }
   } else if (thin) {
