@@ -261,6 +261,14 @@ struct MapJob {
   std::vector<uint64_t> args;
   const char* label;
   double bytes, flops;
+  int n_in = 0;
+  std::vector<char> dense;           // per input: an array, not one element
+  std::vector<uint64_t> depends;     // per output: inputs that must have been loaded for it to be stored, a bit for each
+  std::vector<int> out_size;         // bytes of an output's element
+  // Copies of whole results into existing arrays that came while the pass waited (hold_copy): where nobody else has the result by the time
+  // the pass goes out, it is written to the copy's destination instead.
+  struct Copy { int out; CopyJob job; hgpu_buffer *src, *dst; };
+  std::vector<Copy> copies;
 };
 // smallk.hip: holds an elementwise pass back (retaining the buffers) to be launched with those of the same kernel that follow it; the caller holds launch_mu
 void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);

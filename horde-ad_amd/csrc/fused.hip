@@ -474,6 +474,24 @@ static int fused_map_impl(hgpu_ctx* ctx, int n_in, const hgpu_array* const* in, 
     MapJob j{nullptr, nullptr, grid_for((n + vec - 1) / vec, 256, ctx->num_cu * 16), {(uint64_t)n}, label, bytes, (double)n * n_instr};
     for (int i = 0; i < n_in; ++i) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(in[i])); if (in[i]->buf) reads.push_back(in[i]->buf); }
     for (int o = 0; o < n_out; ++o) { j.args.push_back((uint64_t)(uintptr_t)data_ptr(res[(size_t)o])); writes.push_back(res[(size_t)o]->buf); }
+    j.n_in = n_in;
+    for (char c : layout) j.dense.push_back(c == 'd');
+    // (Per slot.  Only floating-point arithmetic counts, whose result no compiler can give without the operand.)
+    std::vector<uint64_t> needs;
+    for (int i = 0; i < n_in; ++i) needs.push_back(i < 64 ? (uint64_t)1 << i : 0);
+    for (int k = 0; k < n_instr; ++k) {
+      const hgpu_fused_instr& q = prog[k];
+      const bool one = (q.kind == HGPU_FUSED_OP1 && q.op != HGPU_SIGNUM) || q.kind == HGPU_FUSED_CONVERT;
+      const bool two = q.kind == HGPU_FUSED_OP2 && (q.op == HGPU_ADD || q.op == HGPU_SUB || q.op == HGPU_MUL || q.op == HGPU_DIV);
+      auto is_float = [&](int slot) { return dt[(size_t)slot] == HGPU_F64 || dt[(size_t)slot] == HGPU_F32; };
+      uint64_t m = 0;
+      if ((one || two) && is_float(q.a) && is_float(n_in + k)) m = needs[(size_t)q.a] | (two ? needs[(size_t)q.b] : 0);
+      needs.push_back(m);
+    }
+    for (int o = 0; o < n_out; ++o) {
+      j.depends.push_back(needs[(size_t)out_slots[o]]);
+      j.out_size.push_back((int)dtype_size(res[(size_t)o]->dtype));
+    }
     {
       std::lock_guard<LaunchMutex> lk(ctx->launch_mu);
       (void)hipSetDevice(ctx->device);

@@ -161,6 +161,11 @@ class Host(_py.HostBase):
     def tape_reset(self):
         _c.tape_reset(self)
 
+    def submit(self, *values):
+        """Sends out now what gives these values, not when they are read."""
+        for v in values:
+            _c.force(self, v)
+
     def destroy(self):
         self.dll.hh_destroy(self.h)
 

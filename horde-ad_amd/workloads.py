@@ -185,6 +185,7 @@ class Workload:
         loss = self.objective(ps, ds)
         grads = host.grad(loss, ps)
         host.tape_reset()                  # what only the tape held is not waited for
+        host.submit(loss)                  # (beside the gradients' own last sums, not in a launch of its own when it is read)
         return loss, grads
 
 
