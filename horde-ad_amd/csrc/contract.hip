@@ -63,17 +63,25 @@ __device__ __forceinline__ A wave_sum(A v) {
 
 // Work item = (output o, chunk s); s-th chunk covers reduced linear indices
 // [s*chunk, min(R, (s+1)*chunk)).  out is dense [n_out, S].
+// A block takes 256 outputs of one chunk, so that all its lanes walk through the same reduced indices: their offsets are found
+// once per 256 of them, each by one lane, and read from LDS, and eight loads per operand are in flight.  With an odometer of its own
+// in every lane one load waited for the other.  us, before / so: 4096 columns of 4096 elements fp64 68.1 / 27.9, fp32 67.8 / 18.6, 20,000
+// columns of 300 products fp32 26.7 / 9.6; a gradient of the convolution network at batch 7 (27 kernels, seven of them such
+// reductions) with flat_sum below 314 / 272.
 // (`bid` of `nb` blocks: the kernels below pass their own block index; the grouped kernel at the end of this
 // file passes a block's place among the blocks of its problem.  tp == nullptr: one product.)
 template <typename TI, typename TO, bool HASB, typename D>
 __device__ __forceinline__ void lane_body(const D& keep, const D& red, int64_t n_out, int64_t R, int S, int64_t chunk,
                                           const TI* __restrict__ a0, const TI* __restrict__ b0, TO* __restrict__ out, const TermPtrs* tp, unsigned bid, unsigned nb) {
   using A = typename acc_of<TI>::type;
-  int64_t items = n_out * S;
-  int64_t step = (int64_t)nb * kBlock;
-  for (int64_t item = (int64_t)bid * kBlock + threadIdx.x; item < items; item += step) {
-    int64_t o = item % n_out, s = item / n_out;
-    const int64_t s_all = s;
+  constexpr int U = 8;
+  __shared__ int64_t offs[HASB ? 2 : 1][kBlock];
+  const int64_t per_chunk = (n_out + kBlock - 1) / kBlock, tiles = per_chunk * S;
+  int64_t filled = -1;                 // the first of the indices whose offsets are there
+  for (int64_t tile = bid; tile < tiles; tile += nb) {
+    const int64_t s_all = tile / per_chunk, mine = (tile - s_all * per_chunk) * kBlock + threadIdx.x;
+    const int64_t o = mine < n_out ? mine : n_out - 1;
+    int64_t s = s_all;
     const TI* a = a0;
     const TI* b = b0;
     if (tp && tp->n) {
@@ -84,44 +92,44 @@ __device__ __forceinline__ void lane_body(const D& keep, const D& red, int64_t n
     }
     int64_t ko[2];
     decompose<2>(keep, o, ko);
-    int64_t r0 = s * chunk, r1 = r0 + chunk;
-    if (r1 > R) r1 = R;
-    // odometer over the reduced dims, started at r0
-    int64_t idx[HG_KDIMS];
-    int64_t oa = ko[0], ob = ko[1];
-    {
-      int64_t r = r0;
-      for (int i = red.nd - 1; i >= 0; --i) {
-        int64_t q = i > 0 ? r / red.shape[i] : 0;
-        int64_t c = i > 0 ? r - q * red.shape[i] : r;
-        idx[i] = c;
-        oa += c * red.st[0][i];
-        ob += c * red.st[1][i];
-        r = q;
-      }
-    }
+    a += ko[0];
+    if (HASB) b += ko[1];
+    const int64_t r0 = s * chunk, r1 = r0 + chunk < R ? r0 + chunk : R;
     A acc = 0;
-    const int last = red.nd - 1;
-    for (int64_t r = r0; r < r1; ++r) {
-      A x = (A)a[oa];
-      if (HASB) x *= (A)b[ob];
-      acc += x;
-      // advance
-      int i = last;
-      idx[i]++;
-      oa += red.st[0][i];
-      ob += red.st[1][i];
-      while (i > 0 && idx[i] == red.shape[i]) {
-        oa -= idx[i] * red.st[0][i];
-        ob -= idx[i] * red.st[1][i];
-        idx[i] = 0;
-        --i;
-        idx[i]++;
-        oa += red.st[0][i];
-        ob += red.st[1][i];
+    for (int64_t r = r0; r < r1; r += kBlock) {
+      const int m = r1 - r < kBlock ? (int)(r1 - r) : kBlock;
+      if (r != filled) {               // (the same for all lanes)
+        __syncthreads();
+        if ((int)threadIdx.x < m) {
+          int64_t ro[2];
+          decompose<2>(red, r + threadIdx.x, ro);
+          offs[0][threadIdx.x] = ro[0];
+          if (HASB) offs[HASB ? 1 : 0][threadIdx.x] = ro[1];
+        }
+        __syncthreads();
+        filled = r;
+      }
+      int k = 0;
+      for (; k + U <= m; k += U) {
+        A x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          x[u] = (A)a[offs[0][k + u]];
+          if (HASB) y[u] = (A)b[offs[HASB ? 1 : 0][k + u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (HASB) x[u] *= y[u];
+          acc += x[u];
+        }
+      }
+      for (; k < m; ++k) {
+        A x = (A)a[offs[0][k]];
+        if (HASB) x *= (A)b[offs[HASB ? 1 : 0][k]];
+        acc += x;
       }
     }
-    out[o * S + s_all] = (TO)acc;
+    if (mine < n_out) out[o * S + s_all] = (TO)acc;
   }
 }
 template <typename TI, typename TO, bool HASB>
@@ -195,16 +203,104 @@ __device__ __forceinline__ A wide_sum(const TI* __restrict__ pa, const TI* __res
   for (; j < j1; ++j) acc[1] += HASB ? (A)pa[j] * (vb ? (A)pb[j] : one_b) : (A)pa[j];      // (less than a vector, one lane's)
   return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
-// Rows that the WIDE kernels take.  Not fp64 beside a b that runs along too, where the additional registers cost more than the wide loads
+// Rows that the WIDE kernels take (not those that rows_sum takes four at a time).  Not fp64 beside a b that runs along too, where the additional registers cost more than the wide loads
 // give: us, wide / not, 10,000 rows of 1000 29.5 / 27.7, 5000 of 3000 37.0 / 36.1, 1100 of 14712 38.9 / 40.1; fp32 18.7 / 18.4, 23.1 / 23.2,
 // 24.6 / 25.5, 300 rows of 65000 28.4 / 30.8.
-bool wide_rows(size_t es, int64_t sa, const void* b, int64_t sb) { return sa == 1 && (!b || sb == 0 || (sb == 1 && es == 4)); }
+bool wide_rows(size_t es, int64_t Q, int64_t Lin, int64_t sa, const void* b, int64_t sb) {
+  return (Q == 1 || Lin > 1024) && sa == 1 && (!b || sb == 0 || (sb == 1 && es == 4));
+}
 template <typename TI, typename A, bool HASB, bool WIDE>
 __device__ __forceinline__ A row_sum(const TI* __restrict__ pa, const TI* __restrict__ pb, int64_t sa, int64_t sb, int64_t j0, int64_t j1, int lane) {
   if constexpr (WIDE && std::is_floating_point<TI>::value) {
     if (j1 - j0 >= 4096 / (int64_t)sizeof(TI)) return wide_sum<TI, A, HASB>(pa, pb, sb, j0, j1, lane);
   }
   return lane_strided_sum<TI, A, HASB>(pa, pb, sa, sb, j0 + lane, j1);
+}
+
+// (32-bit indices)
+template <typename D>
+__device__ __forceinline__ void decompose_small(const D& d, uint32_t r, int64_t& oa, int64_t& ob) {
+  oa = ob = 0;
+  for (int i = d.nd - 1; i > 0; --i) {
+    const uint32_t s = (uint32_t)d.shape[i], q = r / s, c = r - q * s;
+    r = q;
+    oa += (int64_t)c * d.st[0][i];
+    ob += (int64_t)c * d.st[1][i];
+  }
+  oa += (int64_t)r * d.st[0][0];
+  ob += (int64_t)r * d.st[1][0];
+}
+
+// Sum over the elements f = first, first + step, ... < f1 of rows that lie in one (row f / Lin, element f % Lin): rows shorter than a
+// wavefront, which would leave lanes idle, four elements a lane in flight.  us, before / so: 300 sums of 10,000 rows of 6 fp64
+// 1121 / 74, of 2000 rows of 32 231 / 45, 36 of 168 rows of 24 (four to a launch) 5.6 / 3.2, 500 of 500 rows of 30 33.4 / 14.5.
+// (Rows of 64 and more fill the wavefront, and an index less to find for each element counts once the memory is what bounds it.)
+template <typename TI, typename A, bool HASB, typename D>
+__device__ __forceinline__ A flat_sum(const D& red, uint32_t Lin, const TI* __restrict__ a, const TI* __restrict__ b, int64_t sa_in, int64_t sb_in, uint32_t first, uint32_t step, uint32_t f1) {
+  constexpr uint32_t U = 4;
+  A c[U] = {0, 0, 0, 0};
+  for (uint32_t f = first; f < f1; f += U * step) {
+    A x[U], y[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const bool in = f + u * step < f1;
+      const uint32_t g = in ? f + u * step : f, q = g / Lin, j = g - q * Lin;
+      int64_t oa, ob;
+      decompose_small(red, q, oa, ob);
+      x[u] = (A)a[oa + j * sa_in];
+      if (!in) x[u] = 0;
+      if (HASB) y[u] = in ? (A)b[ob + j * sb_in] : (A)0;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      if (HASB) x[u] *= y[u];
+      c[u] += x[u];
+    }
+  }
+  return (c[0] + c[1]) + (c[2] + c[3]);
+}
+// (indices up to f1 + 4 * step are formed)
+__device__ __forceinline__ bool flat_rows(int64_t Q, int64_t Lin) { return Q > 1 && Lin < 64 && Q * Lin < ((int64_t)1 << 30); }
+
+// Sum over the rows q = first, first + step, ... < q1, four at a time where they are short, so that a lane has four loads per operand
+// in flight although a row gives it only a few elements.
+template <typename TI, typename A, bool HASB, bool WIDE, typename D>
+__device__ __forceinline__ A rows_sum(const D& red, int64_t first, int64_t step, int64_t q1, const TI* __restrict__ a, const TI* __restrict__ b, int64_t sa_in, int64_t sb_in,
+                                      int64_t j0, int64_t j1, bool in_fours, int lane) {
+  A acc = 0;
+  int64_t q = first;
+  if (!WIDE && in_fours) {
+    for (; q + 3 * step < q1; q += 4 * step) {
+      const TI* pa[4];
+      const TI* pb[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        int64_t oa, ob;
+        decompose_small(red, (uint32_t)(q + u * step), oa, ob);
+        pa[u] = a + oa;
+        pb[u] = HASB ? b + ob : nullptr;
+      }
+      A c[4] = {0, 0, 0, 0};
+      for (int64_t j = j0 + lane; j < j1; j += 64) {
+        A x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = (A)pa[u][j * sa_in];
+        if (HASB) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u] *= (A)pb[u][j * sb_in];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c[u] += x[u];
+      }
+      acc += (c[0] + c[1]) + (c[2] + c[3]);
+    }
+  }
+  for (; q < q1; q += step) {
+    int64_t ro[2];
+    decompose<2>(red, q, ro);
+    acc += row_sum<TI, A, HASB, WIDE>(a + ro[0], HASB ? b + ro[1] : nullptr, sa_in, sb_in, j0, j1, lane);
+  }
+  return acc;
 }
 
 // One wavefront per work item.  `red` has its innermost dim split off:
@@ -234,43 +330,10 @@ __device__ __forceinline__ void wave_body(const D& keep, const D& red, int64_t n
     int64_t q0 = 0, q1 = Q, j0 = 0, j1 = Lin;
     if (Q > 1) { q0 = s * chunk; q1 = q0 + chunk; if (q1 > Q) q1 = Q; }
     else { j0 = s * chunk; j1 = j0 + chunk; if (j1 > Lin) j1 = Lin; }
-    A acc = 0;
-    int64_t q = q0;
-    if (Lin <= 1024) {
-      // short inner rows: four outer indices at a time, so that a lane has four
-      // loads per operand in flight although a row gives it only a few elements
-      for (; q + 3 < q1; q += 4) {
-        const TI* pa[4];
-        const TI* pb[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          int64_t ro[2];
-          decompose<2>(red, q + u, ro);
-          pa[u] = a + ko[0] + ro[0];
-          pb[u] = HASB ? b + ko[1] + ro[1] : nullptr;
-        }
-        A c[4] = {0, 0, 0, 0};
-        for (int64_t j = j0 + lane; j < j1; j += 64) {
-          A x[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) x[u] = (A)pa[u][j * sa_in];
-          if (HASB) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] *= (A)pb[u][j * sb_in];
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) c[u] += x[u];
-        }
-        acc += (c[0] + c[1]) + (c[2] + c[3]);
-      }
-    }
-    for (; q < q1; ++q) {
-      int64_t ro[2];
-      decompose<2>(red, q, ro);
-      const TI* pa = a + ko[0] + ro[0];
-      const TI* pb = HASB ? b + ko[1] + ro[1] : nullptr;
-      acc += row_sum<TI, A, HASB, WIDE>(pa, pb, sa_in, sb_in, j0, j1, lane);
-    }
+    const TI *pa = a + ko[0], *pb = HASB ? b + ko[1] : nullptr;
+    A acc;
+    if (!WIDE && flat_rows(Q, Lin)) acc = flat_sum<TI, A, HASB>(red, (uint32_t)Lin, pa, pb, sa_in, sb_in, (uint32_t)(q0 * Lin) + lane, 64, q1 > q0 ? (uint32_t)(q1 * Lin) : 0);
+    else acc = rows_sum<TI, A, HASB, WIDE>(red, q0, 1, q1, pa, pb, sa_in, sb_in, j0, j1, Lin <= 1024 && Q <= INT32_MAX, lane);
     acc = wave_sum<A>(acc);
     if (lane == 0) out[item] = (TO)acc;
   }
@@ -285,7 +348,8 @@ __global__ void __launch_bounds__(kBlock) k_contract_wave(Dims keep, Dims red, i
 // thousand reduced elements each, where one wavefront per output leaves most of
 // the device idle and splitting into chunks would cost a second launch.  The
 // wavefronts take every fourth outer reduced index (or a quarter of the inner
-// dim when there is no outer one) and combine through LDS in a fixed order.
+// dim when there is no outer one; the lanes every 256th element of short rows)
+// and combine through LDS in a fixed order.
 template <typename TI, typename TO, bool HASB, bool WIDE, typename D>
 __device__ __forceinline__ void block_body(const D& keep, const D& red, int64_t n_out, int64_t Q, int64_t Lin, int64_t sa_in, int64_t sb_in,
                                            const TI* __restrict__ a, const TI* __restrict__ b, TO* __restrict__ out, unsigned bid, unsigned nb) {
@@ -296,17 +360,16 @@ __device__ __forceinline__ void block_body(const D& keep, const D& red, int64_t 
   for (int64_t o = bid; o < n_out; o += nb) {
     int64_t ko[2];
     decompose<2>(keep, o, ko);
+    const TI *pa = a + ko[0], *pb = HASB ? b + ko[1] : nullptr;
     A acc = 0;
-    if (Q > 1) {
-      for (int64_t q = w; q < Q; q += NW) {
-        int64_t ro[2];
-        decompose<2>(red, q, ro);
-        acc += row_sum<TI, A, HASB, WIDE>(a + ko[0] + ro[0], HASB ? b + ko[1] + ro[1] : nullptr, sa_in, sb_in, 0, Lin, lane);
-      }
+    if (!WIDE && flat_rows(Q, Lin)) {
+      acc = flat_sum<TI, A, HASB>(red, (uint32_t)Lin, pa, pb, sa_in, sb_in, threadIdx.x, kBlock, (uint32_t)(Q * Lin));
+    } else if (Q > 1) {
+      acc = rows_sum<TI, A, HASB, WIDE>(red, w, NW, Q, pa, pb, sa_in, sb_in, 0, Lin, Lin <= 1024 && Q <= INT32_MAX, lane);
     } else {
       const int64_t quarter = (Lin + NW - 1) / NW;
       const int64_t j0 = w * quarter, j1 = j0 + quarter < Lin ? j0 + quarter : Lin;
-      acc = row_sum<TI, A, HASB, WIDE>(a + ko[0], HASB ? b + ko[1] : nullptr, sa_in, sb_in, j0, j1, lane);
+      acc = row_sum<TI, A, HASB, WIDE>(pa, pb, sa_in, sb_in, j0, j1, lane);
     }
     acc = wave_sum<A>(acc);
     if (lane == 0) part[w] = acc;
@@ -516,7 +579,10 @@ struct RedGroup {
 static_assert(sizeof(RedGroup) <= 4000, "the grouped reduction's arguments must fit the kernel argument block");
 
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_contract_group(RedGroup g) {
+__global__ void __launch_bounds__(kBlock) k_contract_group(RedGroup args) {
+  // read where the launch has put it: with this many uses of a by-value argument the compiler copies all of it to every lane's memory
+  // (3248 bytes of scratch; 1500 sums of 30 rows of 28, four to a launch: 5.9 -> 63.7 us)
+  const RedGroup& g = *(const RedGroup*)__builtin_amdgcn_kernarg_segment_ptr();
   unsigned bid = blockIdx.x;
   int k = 0;
   while (k < g.n && bid >= g.j[k].grid) { bid -= g.j[k].grid; ++k; }
@@ -852,7 +918,7 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     if (red.nd > 1) { red.nd -= 1; } else { red.shape[0] = 1; red.st[0][0] = red.st[1][0] = 0; }
     unsigned g = (unsigned)(n_out < (int64_t)maxb ? n_out : maxb);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, (const TI*)a, (const TI*)b, (TO*)out); };
-    const bool wide = wide_rows(sizeof(TI), sa, b, sb);
+    const bool wide = wide_rows(sizeof(TI), Q, Lin, sa, b, sb);
     if (b && wide) go(k_contract_block<TI, TO, true, true>);
     else if (b) go(k_contract_block<TI, TO, true, false>);
     else if (wide) go(k_contract_block<TI, TO, false, true>);
@@ -868,14 +934,14 @@ int launch_stage(hgpu_ctx* ctx, bool use_wave, const Dims& keep, const Dims& red
     int64_t items = n_out * S;
     unsigned g = grid_for(items * 64, kBlock, maxb);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g), dim3(kBlock), 0, ctx->stream, keep, red, n_out, Q, Lin, sa, sb, S, chunk, (const TI*)a, (const TI*)b, (TO*)out, tp); };
-    const bool wide = wide_rows(sizeof(TI), sa, b, sb);
+    const bool wide = wide_rows(sizeof(TI), Q, Lin, sa, b, sb);
     if (b && wide) go(k_contract_wave<TI, TO, true, true>);
     else if (b) go(k_contract_wave<TI, TO, true, false>);
     else if (wide) go(k_contract_wave<TI, TO, false, true>);
     else go(k_contract_wave<TI, TO, false, false>);
   } else {
     int64_t chunk = (R + S_per - 1) / S_per;
-    unsigned g = grid_for(n_out * S, kBlock, maxb);
+    unsigned g = grid_for((n_out + kBlock - 1) / kBlock * kBlock * S, kBlock, maxb);
     if (b) hipLaunchKernelGGL((k_contract_lane<TI, TO, true>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red_full, n_out, R, S, chunk, (const TI*)a, (const TI*)b, (TO*)out, tp);
     else hipLaunchKernelGGL((k_contract_lane<TI, TO, false>), dim3(g), dim3(kBlock), 0, ctx->stream, keep, red_full, n_out, R, S, chunk, (const TI*)a, (const TI*)nullptr, (TO*)out, tp);
   }
