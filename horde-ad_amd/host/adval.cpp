@@ -19,14 +19,21 @@ D Tape::input(const T& t) {
   return d;
 }
 
-int Tape::push(std::function<void(const T&, std::vector<T>&)> f) {
+int64_t Tape::push(std::function<void(const T&, std::vector<T>&)> f) {
   recs.push_back(Rec{std::move(f)});
-  return (int)recs.size() - 1;
+  return first + (int64_t)recs.size() - 1;
 }
 
-static void accum(std::vector<T>& slots, int node, const T& cot) {
-  if (node < 0) return;
-  T& s = slots[(size_t)node];
+void Tape::reset() {
+  first += (int64_t)recs.size();
+  recs.clear();
+}
+
+// The number of the record that the first slot of the reverse pass under way belongs to.
+static thread_local int64_t first_slot = 0;
+static void accum(std::vector<T>& slots, int64_t node, const T& cot) {
+  if (node < first_slot) return;       // (a constant, or recorded before the tape was reset)
+  T& s = slots[(size_t)(node - first_slot)];
   s = s.valid() ? add_cotangents(s, cot) : cot;
 }
 
@@ -76,23 +83,26 @@ std::vector<T> Tape::backward(const D& out, const T& dt_or_none, const std::vect
   std::vector<std::shared_ptr<ArrHolder>> units;
   struct Scope {
     std::vector<std::shared_ptr<ArrHolder>>* before;
-    explicit Scope(std::vector<std::shared_ptr<ArrHolder>>* u) : before(unit_factors) { unit_factors = u; }
-    ~Scope() { unit_factors = before; }
+    int64_t slot_before;
+    Scope(std::vector<std::shared_ptr<ArrHolder>>* u, int64_t first) : before(unit_factors), slot_before(first_slot) { unit_factors = u; first_slot = first; }
+    ~Scope() { unit_factors = before; first_slot = slot_before; }
   };
   T dt = dt_or_none;
-  if (out.node >= (int)recs.size()) throw HostError(HGPU_ERR_INVALID, "backward: the value's tape has been reset");
-  std::vector<T> slots(recs.size());
-  std::vector<bool> keep(recs.size(), false);
-  for (auto& i : inputs) {
-    if (i.node >= (int)recs.size()) throw HostError(HGPU_ERR_INVALID, "backward: an input's tape has been reset");
-    if (i.node >= 0) keep[(size_t)i.node] = true;
-  }
-  if (out.node >= 0) {
+  // A value recorded before the tape was reset is a constant to everything since; its derivative by something of its own time is lost.
+  const bool live = out.node >= first;
+  for (auto& i : inputs)
+    if (out.node >= 0 && i.node >= 0 && i.node < first) throw HostError(HGPU_ERR_INVALID, "backward: the tape has been reset since an input was made");
+  std::vector<T> slots(live ? recs.size() : 0);
+  auto slot = [&](const D& d) -> T& { return slots[(size_t)(d.node - first)]; };
+  std::vector<bool> keep(slots.size(), false);
+  for (auto& i : inputs)
+    if (live && i.node >= 0) keep[(size_t)(i.node - first)] = true;
+  if (live) {
     if (!dt.valid()) dt = broadcast_scalar(seed_one(be, out.primal.dtype()), out.primal.shape());
     if (dt.shape() != out.primal.shape()) throw HostError(HGPU_ERR_INVALID, "backward: cotangent shape differs from the result's");
-    Scope scope(&units);
-    slots[(size_t)out.node] = dt;
-    for (int n = out.node; n >= 0; --n) {
+    Scope scope(&units, first);
+    slot(out) = dt;
+    for (int64_t n = out.node - first; n >= 0; --n) {
       if (!slots[(size_t)n].valid()) continue;
       recs[(size_t)n].back(slots[(size_t)n], slots);
       if (!keep[(size_t)n]) slots[(size_t)n] = T();
@@ -100,8 +110,8 @@ std::vector<T> Tape::backward(const D& out, const T& dt_or_none, const std::vect
   }
   std::vector<T> res;
   for (auto& i : inputs) {
-    if (i.node >= 0 && slots[(size_t)i.node].valid()) {
-      res.push_back(slots[(size_t)i.node]);
+    if (live && i.node >= 0 && slot(i).valid()) {
+      res.push_back(slot(i));
       continue;
     }
     T z = zeros(be, i.primal.dtype(), i.primal.shape());   // tdefTarget
@@ -149,7 +159,7 @@ D d_ewise1(Tape& tp, int op, const D& a) {
   r.primal = ewise1(op, a.primal);
   if (a.node < 0 || !differentiable(r.primal) || op == HGPU_SIGNUM) return r;
   T u = a.primal, y = r.primal;
-  int an = a.node;
+  int64_t an = a.node;
   T scale;  // dScale scale u'
   switch (op) {
     case HGPU_NEG: scale = T(); break;
@@ -183,7 +193,7 @@ D d_ewise2(Tape& tp, int op, const D& a, const D& b) {
   r.primal = ewise2(op, a.primal, b.primal);
   if ((a.node < 0 && b.node < 0) || !differentiable(r.primal)) return r;
   T u = a.primal, v = b.primal, y = r.primal;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   switch (op) {
     case HGPU_ADD:
       r.node = tp.push([an, bn](const T& c, std::vector<T>& s) { accum(s, an, c); accum(s, bn, c); });
@@ -245,7 +255,7 @@ D d_select(Tape& tp, const T& cond, const D& a, const D& b) {
   D r;
   r.primal = select(cond, a.primal, b.primal);
   if ((a.node < 0 && b.node < 0) || !differentiable(r.primal)) return r;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   r.node = tp.push([an, bn, cond](const T& c, std::vector<T>& s) {
     T z = zeros(c.be(), c.dtype(), c.shape());
     if (an >= 0) accum(s, an, select(cond, c, z));
@@ -259,7 +269,7 @@ D d_convert(Tape& tp, const D& a, int dtype, int mode) {
   D r;
   r.primal = convert(a.primal, dtype, mode);
   if (a.node < 0 || !differentiable(r.primal) || mode != HGPU_CONV_CAST) return r;
-  int an = a.node, src = a.primal.dtype();
+  int64_t an = a.node, src = a.primal.dtype();
   r.node = tp.push([an, src](const T& c, std::vector<T>& s) { accum(s, an, convert(c, src, HGPU_CONV_CAST)); });
   return r;
 }
@@ -271,7 +281,7 @@ D d_tssumN(Tape& tp, const D& t, int k) {
   if (t.node < 0 || k == 0) { if (k == 0) r.node = t.node; return r; }
   Shape sh = t.primal.shape();
   Shape shm(sh.begin(), sh.begin() + k);
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn, shm](const T& c, std::vector<T>& s) { accum(s, tn, tsreplicateN(c, shm)); });
   return r;
 }
@@ -282,7 +292,7 @@ D d_tssum0(Tape& tp, const D& t) {
   r.primal = tssum0(t.primal);
   if (t.node < 0) return r;
   Shape sh = t.primal.shape();
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn, sh](const T& c, std::vector<T>& s) { accum(s, tn, tsreplicate0N(c, sh)); });
   return r;
 }
@@ -293,7 +303,7 @@ D d_tsdot0(Tape& tp, const D& a, const D& b) {
   r.primal = tsdot0(a.primal, b.primal);
   if (a.node < 0 && b.node < 0) return r;
   T u = a.primal, v = b.primal;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   r.node = tp.push([an, bn, u, v](const T& c, std::vector<T>& s) {
     T cc = tsreplicate0N(c, u.shape());
     if (an >= 0) accum(s, an, mul(v, cc));
@@ -318,7 +328,7 @@ D d_tsdot1In(Tape& tp, const D& a, const D& b) {
   r.primal = tsdot1In(a.primal, b.primal);
   if (a.node < 0 && b.node < 0) return r;
   T u = a.primal, v = b.primal;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   int64_t n = u.shape().back();
   r.node = tp.push([an, bn, u, v, n](const T& c, std::vector<T>& s) {
     T cc = expand_inner(c, n);
@@ -342,7 +352,7 @@ D d_tsdotNIn(Tape& tp, const D& a, const D& b, int n) {
   r.primal = tsdotNIn(a.primal, b.primal, n);
   if (a.node < 0 && b.node < 0) return r;
   T u = a.primal, v = b.primal;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   Shape sh = u.shape();
   Shape inner(sh.end() - n, sh.end());
   r.node = tp.push([an, bn, u, v, inner](const T& c, std::vector<T>& s) {
@@ -370,7 +380,7 @@ D d_tsmatmul2(Tape& tp, const D& a, const D& b) {
   r.primal = tsmatmul2(a.primal, b.primal);
   if (a.node < 0 && b.node < 0) return r;
   T u = a.primal, v = b.primal;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   r.node = tp.push([an, bn, u, v](const T& c, std::vector<T>& s) {
     if (an >= 0) accum(s, an, tsmatmul2(c, transpose(v, {1, 0})));
     if (bn >= 0) accum(s, bn, tsmatmul2(transpose(u, {1, 0}), c));
@@ -384,7 +394,7 @@ D d_tsreplicateN(Tape& tp, const D& t, const Shape& shm) {
   r.primal = tsreplicateN(t.primal, shm);
   if (t.node < 0) return r;
   if (shm.empty()) { r.node = t.node; return r; }
-  int tn = t.node, k = (int)shm.size();
+  int64_t tn = t.node, k = (int)shm.size();
   r.node = tp.push([tn, k](const T& c, std::vector<T>& s) { accum(s, tn, tssumN(c, k)); });
   return r;
 }
@@ -394,7 +404,7 @@ D d_tsappend(Tape& tp, const D& a, const D& b) {
   D r;
   r.primal = tsappend(a.primal, b.primal);
   if (a.node < 0 && b.node < 0) return r;
-  int an = a.node, bn = b.node;
+  int64_t an = a.node, bn = b.node;
   int64_t m = a.primal.shape().at(0), n = b.primal.shape().at(0);
   r.node = tp.push([an, bn, m, n](const T& c, std::vector<T>& s) {
     if (an >= 0) accum(s, an, tsslice(c, 0, m));
@@ -408,7 +418,7 @@ D d_tsslice(Tape& tp, const D& t, int64_t i, int64_t n) {
   D r;
   r.primal = tsslice(t.primal, i, n);
   if (t.node < 0) return r;
-  int tn = t.node, rank = t.primal.rank();
+  int64_t tn = t.node, rank = t.primal.rank();
   int64_t k = t.primal.shape().at(0) - i - n;
   r.node = tp.push([tn, rank, i, k](const T& c, std::vector<T>& s) {
     Shape lo((size_t)rank, 0), hi((size_t)rank, 0);
@@ -424,7 +434,7 @@ D d_tsreverse(Tape& tp, const D& t) {
   D r;
   r.primal = tsreverse(t.primal);
   if (t.node < 0) return r;
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn](const T& c, std::vector<T>& s) { accum(s, tn, tsreverse(c)); });
   return r;
 }
@@ -436,7 +446,7 @@ D d_tstranspose(Tape& tp, const D& t, const std::vector<int>& perm) {
   if (t.node < 0) return r;
   std::vector<int> inv(perm.size());
   for (size_t i = 0; i < perm.size(); ++i) inv[(size_t)perm[i]] = (int)i;
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn, inv](const T& c, std::vector<T>& s) { accum(s, tn, tstranspose(c, inv)); });
   return r;
 }
@@ -447,7 +457,7 @@ D d_tsreshape(Tape& tp, const D& t, const Shape& sh) {
   r.primal = tsreshape(t.primal, sh);
   if (t.node < 0) return r;
   Shape back = t.primal.shape();
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn, back](const T& c, std::vector<T>& s) { accum(s, tn, tsreshape(c, back)); });
   return r;
 }
@@ -459,7 +469,7 @@ D d_tsindex(Tape& tp, const D& t, const Shape& ix) {
   if (t.node < 0) return r;
   Shape sh = t.primal.shape();
   Shape shp(sh.begin(), sh.begin() + (long)ix.size());
-  int tn = t.node;
+  int64_t tn = t.node;
   r.node = tp.push([tn, ix, shp](const T& c, std::vector<T>& s) { accum(s, tn, tsoneHot(c, ix, shp)); });
   return r;
 }
@@ -471,7 +481,7 @@ D d_tsgather(Tape& tp, const D& src, const Shape& shm, const std::vector<Ix>& ix
   if (src.node < 0) return r;
   Shape ssh = src.primal.shape();
   Shape shp(ssh.begin(), ssh.begin() + (long)ix.size());
-  int sn = src.node, rank_m = (int)shm.size();
+  int64_t sn = src.node, rank_m = (int)shm.size();
   r.node = tp.push([sn, rank_m, shp, ix](const T& c, std::vector<T>& s) { accum(s, sn, tsscatter(c, rank_m, shp, ix)); });
   return r;
 }
@@ -483,7 +493,7 @@ D d_tsscatter(Tape& tp, const D& src, int rank_m, const Shape& shp, const std::v
   if (src.node < 0) return r;
   Shape ssh = src.primal.shape();
   Shape shm(ssh.begin(), ssh.begin() + rank_m);
-  int sn = src.node;
+  int64_t sn = src.node;
   r.node = tp.push([sn, shm, ix](const T& c, std::vector<T>& s) { accum(s, sn, tsgather(c, shm, ix)); });
   return r;
 }

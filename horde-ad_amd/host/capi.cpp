@@ -78,7 +78,7 @@ int hh_create_gpu(int device, hh_ctx** out) { return hh_create(hgpu_get_api(), d
 
 int hh_destroy(hh_ctx* c) {
   if (!c) return HGPU_OK;
-  c->tape.recs.clear();
+  c->tape.reset();
   c->be.iota_cache.clear();
   c->be.const_cache.clear();
   for (auto& s : c->be.seed_one) s.reset();
@@ -91,7 +91,7 @@ const char* hh_last_error(hh_ctx* c) { return c ? c->err.c_str() : "no context";
 int hh_sync(hh_ctx* c) { return guarded(c, [&] { c->be.check(c->be.api->sync(c->be.ctx)); }); }
 hgpu_ctx* hh_array_ctx(hh_ctx* c) { return c ? c->be.ctx : nullptr; }
 int hh_set_fusion(hh_ctx* c, int on) { c->be.fuse = on != 0; return HGPU_OK; }
-int hh_tape_reset(hh_ctx* c) { c->tape.recs.clear(); return HGPU_OK; }
+int hh_tape_reset(hh_ctx* c) { c->tape.reset(); return HGPU_OK; }
 
 int hh_upload(hh_ctx* c, int dtype, int rank, const int64_t* shape, const void* host, int rg, hh_val** out) {
   return guarded(c, [&] {

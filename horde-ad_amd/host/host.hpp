@@ -485,7 +485,7 @@ T tsscatter(const T& src, int rank_m, const Shape& shp, const std::vector<Ix>& i
 struct Tape;
 struct D {
   T primal;
-  int node = -1;               // index into the tape; -1 = no derivative flows
+  int64_t node = -1;           // number of its record; -1 = no derivative flows
 };
 
 struct Tape {
@@ -494,9 +494,11 @@ struct Tape {
   };
   Backend* be;
   std::vector<Rec> recs;
+  int64_t first = 0;                                       // number of recs[0]: a reset does not number anew
+  void reset();
   explicit Tape(Backend* b) : be(b) {}
   D input(const T& t);                                     // differentiable leaf
-  int push(std::function<void(const T&, std::vector<T>&)> f);
+  int64_t push(std::function<void(const T&, std::vector<T>&)> f);
   // Cotangents of `inputs` given d(out) = dt (an empty T: one at every position).  Each has memory of its own.
   std::vector<T> backward(const D& out, const T& dt, const std::vector<D>& inputs);
 };
