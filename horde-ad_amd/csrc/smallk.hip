@@ -1497,7 +1497,11 @@ bool join_wide_rows(hgpu_ctx* ctx, int dtype, int n, const void* const* as, int6
       wide_take_rows(*job, (*part)->ptr, factor);
       d.writes.push_back(*part);
       ctx->dq->keep(*part);
-      if (factor_buf) { d.reads.push_back(factor_buf); ctx->dq->keep(factor_buf); }
+      if (factor_buf) {
+        d.reads.push_back(factor_buf);
+        ctx->dq->keep(factor_buf);
+        singles_for_locked(ctx, {factor_buf});      // (a gathered element, an extremum: whatever sends the product out need not read it)
+      }
       return true;
     }
   }

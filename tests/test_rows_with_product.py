@@ -155,6 +155,52 @@ def test_factor_of_a_row_sum(host, m, n, k, f):
     check(host, program, [big], [size], k, 1)
 
 
+@pytest.mark.parametrize("dt,terms,m,n,k", [(np.float32, 1, 128, 128, 30000), (np.float32, 6, 130, 96, 5000), (np.float64, 3, 65, 130, 3001)])
+@pytest.mark.parametrize("by", ["gather", "extremum"])
+def test_factor_that_waits(host, dt, terms, m, n, k, by):
+    """The factor is the result of a launch that is held back by itself: it goes out before the product that reads it, also where
+    something sends that product out which does not read the factor."""
+    rng = np.random.default_rng(m)
+    xs, ys = [rng.uniform(0.5, 1, (m, k)).astype(dt) for _ in range(terms)], [rng.uniform(0, 1, (k, n)).astype(dt) for _ in range(terms)]
+    a, b = [host.concrete(x) for x in xs], [host.concrete(y) for y in ys]
+    values = rng.uniform(1, 2, 100).astype(dt)
+    table, at = host.concrete(values), host.concrete(np.asarray(3, np.int64))
+
+    def program():
+        p = a[0].smatmul2(b[0])
+        for u, v in zip(a[1:], b[1:]):
+            p = p + u.smatmul2(v)
+        held.force(host, p)
+        f = table.sgather((), lambda: [at.lift(())]) if by == "gather" else held.pkg.workloads.sminimum(table)
+        held.force(host, f)
+        by_f = f.sreplicate(k).sreplicate(m)
+        s = a[0].sdot1In(by_f)
+        for u in a[1:]:
+            s = s + u.sdot1In(by_f)
+        held.force(host, s)
+        q = p * 2.0
+        held.force(host, q)
+        return [s, q]
+
+    total, size = sum(x.sum(1, dtype=np.longdouble) for x in xs).astype(np.float64), 2.0 * sum(np.abs(x).sum(1, dtype=np.float64) for x in xs)
+    [v.numpy() for v in program()]
+    graph, (s, q), labels = held.recorded(host, program)
+    assert any("+rows" in v for v in labels), labels
+    try:
+        for i in (5, 70, 11, 70):
+            at.overwrite(np.asarray(i, np.int64))
+            now = values.copy()
+            now[20] = i / 128
+            table.overwrite(now)
+            f = float(now[i] if by == "gather" else now.min())
+            graph.launch()
+            host.sync()
+            assert np.all(np.abs(s.numpy() - f * total) <= 2 * (2.0 ** (-24 if dt == np.float32 else -53) + terms * k * 2.0 ** -53) * size), i
+            [v.numpy() for v in program()]
+    finally:
+        graph.free()
+
+
 def test_two_threads_ask_for_the_same_rows():
     """One of the sums joins the product, the other is a launch of its own."""
     ctx = held.pkg.capi.Lib().context(0)
