@@ -750,8 +750,9 @@ struct Deferred {
   int level = 0;
 };
 
-// Products, reductions and elementwise passes write new arrays only; copies write
-// existing ones.  The queue holds either products and reductions, and beside them
+// Products, reductions and single launches write new arrays only; copies write existing
+// ones, and so does an elementwise pass with which copies of its results wait
+// (copy_with_map_locked).  The queue holds either products and reductions, and beside them
 // elementwise passes that read no result of one another, or copies that touch no memory
 // of one another: whatever does not fit flushes it first.  No held pass reads the
 // result of a held product or reduction, and none of those the result of a held pass.
@@ -1536,7 +1537,8 @@ void hold_map_locked(hgpu_ctx* ctx, MapJob&& job, const std::vector<hgpu_buffer*
 // a launch of 4.9 us and their bytes twice; a training step of the f32 convolution network, batch 250: 106.8 -> 103.3 us), if the result can be written to its destination by that pass:
 //   * no other held pass reads or writes the destination's block, nor does another copy;
 //   * of the pass's own inputs those that lie in it are the destination itself, element by element, and each of the result's elements
-//     cannot be computed without that input's: it has been loaded when the result is stored, whatever order the compiler gives the rest.
+//     comes from that input's, as an update's does.  The pass's text loads all inputs of an element before it stores any result, and
+//     promises nothing about which arrays are apart (fused_map_impl), so its other results may come from that input too.
 // (The caller holds launch_mu and has retained both buffers.)
 static bool copy_with_map_locked(DeferredQueue& q, const CopyJob& job, hgpu_buffer* src, hgpu_buffer* dst) {
   if (q.maps.empty() || q.kind != DeferredQueue::kProducts || ((uintptr_t)job.dst & 15) != 0) return false;

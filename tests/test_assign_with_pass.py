@@ -154,3 +154,39 @@ def test_destinations_amid_an_array(gpu):
             whole.assign(gpu.upload(np.zeros(1000)))
     finally:
         gpu.check(dll.hgpu_graph_destroy(g))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_two_results_of_an_input_that_one_is_written_to(dt, tmp_path, monkeypatch):
+    """The other result reads the overwritten input too: the kernel promises the compiler nothing about which arrays are apart, and
+    every replay gives the bits of the pass into new arrays."""
+    monkeypatch.setenv("HORDEAD_GPU_KEEP_SOURCES", str(tmp_path))
+    ctx = pkg.capi.Lib().context(0)                  # (none of its kernels is known yet)
+    dll, O2 = ctx.lib.dll, pkg.capi.OP2
+    prog = [(1, O2["mul"], 0, 0, 1, 0), (1, O2["add"], 0, 2, 0, 0), (1, O2["sub"], 0, 0, 3, 0)]
+    rng = np.random.default_rng(7)
+    x, y = rng.uniform(-1, 1, (2, 70003)).astype(dt)
+    a, b, c = ctx.upload(x), ctx.upload(y), ctx.upload(np.zeros_like(x))
+    want = []
+    now = ctx.upload(x)
+    for _ in range(3):
+        now, other = ctx.fused_map([now, b], prog, [3, 4])
+        want.append((now.numpy(), other.numpy()))
+    ctx.profile(2)
+    g = C.c_void_p()
+    ctx.check(dll.hgpu_capture_begin(ctx.h))
+    r = ctx.fused_map([a, b], prog, [3, 4])
+    a.assign(r[0])
+    c.assign(r[1])
+    del r
+    ctx.check(dll.hgpu_capture_end(ctx.h, C.byref(g)))
+    assert not any("copy" in n for n in ctx.profile_report())
+    ctx.profile(0)
+    try:
+        for wa, wc in want:
+            ctx.check(dll.hgpu_graph_launch(g))
+            assert np.array_equal(a.numpy(), wa) and np.array_equal(c.numpy(), wc)
+    finally:
+        ctx.check(dll.hgpu_graph_destroy(g))
+    texts = [t for t in (f.read_text() for f in tmp_path.iterdir()) if "fused_map_group(" in t]
+    assert len(texts) == 1 and "__restrict__" not in texts[0]
