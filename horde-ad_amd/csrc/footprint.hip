@@ -1604,10 +1604,13 @@ bool refine_view(int n_keep, const int64_t* kshape, int view_rank, const int64_t
   return true;
 }
 
+// *through: whether the rows operand may be read through a waiting zero-extension; afterwards, whether it was to be.
 int try_contract_map(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, int n_keep, int n_in, const hgpu_array* const* in, int c_slot, int n_instr,
                      const hgpu_fused_instr* prog, const std::vector<int>& dt, int n_out, const int* out_slots, hgpu_array** outs, int ext_slot, int view_rank,
-                     const int64_t* view_shape, const int64_t* view_strides, int n_reduce, int want_max, hgpu_array** values, hgpu_array** indices, bool* handled) {
+                     const int64_t* view_shape, const int64_t* view_strides, int n_reduce, int want_max, hgpu_array** values, hgpu_array** indices, bool* through, bool* handled) {
   *handled = false;
+  const bool look = *through;
+  *through = false;
   if (a->dtype != HGPU_F64 && a->dtype != HGPU_F32) return HGPU_OK;
   const bool f64 = a->dtype == HGPU_F64;
   const int es = f64 ? 8 : 4;
@@ -1687,7 +1690,8 @@ int try_contract_map(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_array* b, in
   const char* pa = (const char*)data_ptr(a);
   const char* pb = (const char*)data_ptr(b);
   Extended ext;                // the rows operand, where a waiting zero-extension is to write it
-  ext.find(ctx, swapped ? b : a);
+  if (look) ext.find(ctx, swapped ? b : a);
+  *through = (bool)ext;
   if (ext) (swapped ? pb : pa) = (const char*)(uintptr_t)(ext.offset * es);
   const VirtualOp* vx = ext ? &ext.v : nullptr;
   Plan pl;
@@ -1925,9 +1929,18 @@ extern "C" int hgpu_contract_map(hgpu_ctx* ctx, const hgpu_array* a, const hgpu_
     if (hi >= n_kept) return fail(ctx, HGPU_ERR_INVALID, "contract_map: the view leaves the result");
   }
   if (n_kept > 0) {
-    bool handled = false;
-    int rc = try_contract_map(ctx, a, b, n_keep, n_in, in, c_slot, n_instr, prog, dt, n_out, out_slots, outs, ext_slot, view_rank, view_shape, view_strides, n_reduce,
-                              want_max, values, indices, &handled);
+    // An extension that does not fit the plan is written: with an odd number of zeros in front it is staged element by element, four times the
+    // loads of the written array in fp32.  Kernels of 3 x 3 over 16 channels of 26 x 26, 300 images fp32: product, pass and extremum over the
+    // written extension 75.1 us with it, one kernel over it 63.3; 32 channels of 22 x 22 87.5 / 71.2, 1000 images with 32 channels of 20 x 24 189 / 143,
+    // 20 of 26 x 34 242 / 234.  (Written or not, 1000 images with 16 channels of 28 x 36 are faster in three launches, 251 / 281, and 250 are not far from it,
+    // 82 / 85: a matter of the one kernel, not of who extends.)
+    bool handled = false, through = true;
+    int rc = HGPU_OK;
+    for (int turn = 0; turn < 2 && !rc && !handled && through; ++turn) {
+      through = turn == 0;
+      rc = try_contract_map(ctx, a, b, n_keep, n_in, in, c_slot, n_instr, prog, dt, n_out, out_slots, outs, ext_slot, view_rank, view_shape, view_strides, n_reduce,
+                            want_max, values, indices, &through, &handled);
+    }
     if (rc || handled) return rc;
   }
   // one entry point after another

@@ -102,6 +102,32 @@ def test_products_read_what_is_extended(gpu, B, Ci, Co, H, W, k, dt, lo, how):
         assert any("footprint" in n for n in labels) and not any(n.startswith("pad[") for n in labels), labels
 
 
+@pytest.mark.parametrize("Ci,H,dt,written", [
+    (16, 24, np.float32, False),      # 10,816 elements of an image, element by element: fits
+    (16, 26, np.float32, True),       # 12,544: two loads a lane too many
+    (32, 22, np.float32, True),       # ... by far
+    (16, 22, np.float64, False),
+])
+def test_layers_whose_extension_does_not_fit(gpu, Ci, H, dt, written):
+    """One zero in front, so the extension is staged element by element: where that is too much, the layer is still one kernel, over
+    the written extension."""
+    rng = np.random.default_rng(H)
+    x = rng.uniform(-1, 1, (150, Ci, H, H)).astype(dt)
+    ker, bias = rng.uniform(-0.4, 0.4, (16, Ci, 3, 3)).astype(dt), rng.uniform(-0.4, 0.4, (16,)).astype(dt)
+    s = gpu.upload(x)
+    p = s.pad([0, 0, 1, 1], [0, 0, 1, 1])
+    gpu.sync()                            # written
+    want = [o.numpy() for o in forward(gpu, p, ker, bias, H, H)]
+    gpu.profile(2)
+    got = [o.numpy() for o in forward(gpu, s.pad([0, 0, 1, 1], [0, 0, 1, 1]), ker, bias, H, H)]
+    labels = list(gpu.profile_report())
+    gpu.profile(0)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+    assert any("footprint" in n and ",map(" in n for n in labels) and not any(n == "argminmax" for n in labels), labels
+    assert any(n.startswith("pad[") for n in labels) == written, labels
+
+
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_others_find_the_extension_written(gpu, dt):
     rng = np.random.default_rng(2)
