@@ -5,8 +5,8 @@
 // finalizer that is again such a call.  Here a value is a C object (its handle goes back in its deallocator), and a `Fn`
 // is an entry point with a signature that says how its arguments are laid out:
 //
-//   v  a value          x  a lane value        i  an integer         d  a double         p  an address (an int)
-//   S  integers, as their number and an int64_t array         Q  the same with an int array
+//   v  a value          x  a lane value        i  an int             n  an int64_t       d  a double         p  an address (an int)
+//   S  sizes, as their number and an int64_t array (whatever int() takes)         Q  ints, as their number and an int array
 //   K  lane values, as their number and an array of handles
 //
 // after the host, whose context handle is the first argument of every call.  What comes back: "V" a value, "X" a lane value
@@ -17,6 +17,7 @@
 #include <Python.h>
 #include <structmember.h>
 
+#include <climits>
 #include <cstdint>
 #include <cstring>
 
@@ -197,16 +198,26 @@ struct Fn {
   char out;
 };
 
-bool integer(PyObject* o, int64_t* out) {
-  if (PyLong_Check(o)) {
-    *out = PyLong_AsLongLong(o);
-  } else {      // (int(): numpy's integers, floats with whole values)
-    PyObject* l = PyNumber_Long(o);
-    if (!l) return false;
-    *out = PyLong_AsLongLong(l);
-    Py_DECREF(l);
-  }
-  return !(*out == -1 && PyErr_Occurred());
+// What stands for an integer (numpy's integers too, no fractions and no texts), from lo to hi
+bool integer(PyObject* o, int64_t* out, int64_t lo, int64_t hi) {
+  PyObject* l = PyNumber_Index(o);
+  if (!l) return false;
+  *out = PyLong_AsLongLong(l);
+  Py_DECREF(l);
+  if (*out == -1 && PyErr_Occurred()) return false;
+  if (*out >= lo && *out <= hi) return true;
+  PyErr_SetString(PyExc_OverflowError, "an integer is too large for its parameter");
+  return false;
+}
+bool integer(PyObject* o, int64_t* out) { return integer(o, out, INT64_MIN, INT64_MAX); }
+bool small_integer(PyObject* o, int64_t* out) { return integer(o, out, INT_MIN, INT_MAX); }
+// One of a list of sizes: int() of it
+bool size(PyObject* o, int64_t* out) {
+  if (PyLong_Check(o)) return integer(o, out);
+  PyObject* l = PyNumber_Long(o);
+  const bool ok = l && integer(l, out);
+  Py_XDECREF(l);
+  return ok;
 }
 
 PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw) {
@@ -239,6 +250,8 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
       if (!space) space = ((Lane*)o)->shm;
       a[na++] = (int64_t)((Lane*)o)->h;
     } else if (c == 'i') {
+      if (!small_integer(o, &a[na++])) return stop();
+    } else if (c == 'n') {
       if (!integer(o, &a[na++])) return stop();
     } else if (c == 'p') {
       if (!address(o, (void**)&a[na++])) return stop();
@@ -259,7 +272,7 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
           l[i] = (int64_t)((Lane*)e)->h;
         } else {
           int64_t v;
-          if (!integer(e, &v)) return stop();
+          if (!(c == 'Q' ? small_integer(e, &v) : size(e, &v))) return stop();
           if (c == 'Q') ((int*)l)[i] = (int)v;
           else l[i] = v;
         }
@@ -308,7 +321,7 @@ PyObject* fn_new(PyTypeObject* type, PyObject* args, PyObject*) {
   if (!PyArg_ParseTuple(args, "Oss", &at, &sig, &out)) return nullptr;
   int words = 1 + (out[0] != 'N'), lists = 0, doubles = 0;
   for (const char* c = sig; *c; ++c) {
-    if (!strchr("vxidpSQK", *c)) { PyErr_SetString(PyExc_ValueError, "unknown letter in a signature"); return nullptr; }
+    if (!strchr("vxindpSQK", *c)) { PyErr_SetString(PyExc_ValueError, "unknown letter in a signature"); return nullptr; }
     const bool list = *c == 'S' || *c == 'Q' || *c == 'K';
     words += list ? 2 : *c != 'd';
     lists += list;

@@ -66,9 +66,9 @@ NATIVE = {
     "tape_reset": ("", "N"), "constant": ("idS", "V"), "ewise1": ("iv", "V"), "ewise2": ("ivv", "V"), "compare": ("ivv", "V"),
     "select": ("vvv", "V"), "convert": ("vii", "V"), "tssumN": ("vi", "V"), "tssum0": ("v", "V"), "tsdot0": ("vv", "V"),
     "tsdot1In": ("vv", "V"), "tsdotNIn": ("vvi", "V"), "tD": ("vv", "V"), "tprimalPart": ("v", "V"), "as_input": ("v", "V"),
-    "tsmatvecmul": ("vv", "V"), "tsmatmul2": ("vv", "V"), "tsreplicateN": ("vS", "V"), "tsappend": ("vv", "V"), "tsslice": ("vii", "V"),
+    "tsmatvecmul": ("vv", "V"), "tsmatmul2": ("vv", "V"), "tsreplicateN": ("vS", "V"), "tsappend": ("vv", "V"), "tsslice": ("vnn", "V"),
     "tsreverse": ("v", "V"), "tstranspose": ("vQ", "V"), "tsreshape": ("vS", "V"), "tsindex": ("vS", "V"), "tsargminmax": ("vi", "V"),
-    "tsiota": ("ii", "V"), "dense": ("v", "V"), "tsgather": ("vSK", "V"), "tconvert": ("ivS", "V"),
+    "tsiota": ("ni", "V"), "dense": ("v", "V"), "tsgather": ("vSK", "V"), "tconvert": ("ivS", "V"),
     "ix_var": ("Si", "X"), "ix_const": ("Sid", "X"), "ix_lift": ("Sv", "X"), "ix_op1": ("ix", "X"), "ix_op2": ("ixx", "X"),
     "ix_compare": ("ixx", "X"), "ix_select": ("xxx", "X"), "ix_convert": ("xii", "X"), "ix_index0": ("vK", "X"),
     "ix_argminmax": ("vKi", "X"), "ix_from_val": ("v", "X"), "ix_to_val": ("x", "V"),

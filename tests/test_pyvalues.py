@@ -31,6 +31,24 @@ def test_integers_as_python_has_them(host):
     assert host.siota(n=3).numpy().tolist() == [0, 1, 2] and v.sslice(i=0, n=2).shape == (2, 3, 4) and v.sdotNIn(v, n=2).shape == (2,)
 
 
+@pytest.mark.parametrize("wrong", [
+    lambda h, v: v.sslice(1.7, 2.2), lambda h, v: v.sslice("1", "2"), lambda h, v: v.sslice(0, np.float64(2)), lambda h, v: v.ssumN(1.9), lambda h, v: h.siota(3.9),
+    lambda h, v: h.siota("3"), lambda h, v: v.stranspose([1.0, 0.9, 2]), lambda h, v: v.stranspose("102"), lambda h, v: v.stranspose([2 ** 32 + 1, 0, 2]),
+    lambda h, v: v.ssumN(2 ** 32 + 1), lambda h, v: v.ssumN(1 - 2 ** 32), lambda h, v: v.sslice(2 ** 64, 2), lambda h, v: v.sdotNIn(v, 1.5), lambda h, v: v.scast(2 ** 33)])
+def test_no_integers(host, wrong):
+    """Fractions, texts and what the parameter cannot hold are refused, not cut to an integer."""
+    with pytest.raises((TypeError, OverflowError)):
+        wrong(host, host.concrete(np.arange(24.0).reshape(2, 3, 4)))
+
+
+def test_sizes_are_what_int_gives(host):
+    v = host.concrete(np.arange(24.0))
+    assert v.sreshape([6.0, 4]).shape == v.sreshape(["6", np.float32(4)]).shape == (6, 4) and v.sreplicate(2.5).shape == (2, 24)
+    assert v.sslice(np.int64(5), np.int8(2)).numpy().tolist() == [5, 6] and host.siota(2 ** 33 % 7).shape == (2 ** 33 % 7,)
+    with pytest.raises(OverflowError):
+        v.sreshape([2 ** 64, 1])
+
+
 def test_lane_values(host):
     v = host.concrete(np.arange(12.0).reshape(3, 4))
     seen = []
