@@ -231,12 +231,18 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
   double d = 0;
   int64_t lists[2][kMaxRank];
   int n_lists = 0;
-  PyObject *space = nullptr, *seq = nullptr, *made = nullptr;      // the index space of a lane value (borrowed), a sequence at hand, a tuple made here
+  PyObject *space = nullptr, *seq = nullptr, *lanes = nullptr;      // the index space of a lane value, a sequence at hand, the lane values of a K argument
   const Val* first = nullptr;
   auto stop = [&]() -> PyObject* {
     Py_XDECREF(seq);
-    Py_XDECREF(made);
+    Py_XDECREF(lanes);
+    Py_XDECREF(space);
     return nullptr;
+  };
+  auto over = [&](const PyObject* lane) {
+    if (space) return;
+    space = ((const Lane*)lane)->shm;
+    Py_XINCREF(space);
   };
   for (int k = 0; f->sig[k]; ++k) {
     PyObject* o = args[k + 1];
@@ -247,7 +253,7 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
       a[na++] = (int64_t)((Val*)o)->h;
     } else if (c == 'x') {
       if (!PyObject_TypeCheck(o, &LaneType)) { PyErr_Format(PyExc_TypeError, "argument %d is not a lane value", k + 1); return stop(); }
-      if (!space) space = ((Lane*)o)->shm;
+      over(o);
       a[na++] = (int64_t)((Lane*)o)->h;
     } else if (c == 'i') {
       if (!small_integer(o, &a[na++])) return stop();
@@ -259,7 +265,8 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
       d = PyFloat_AsDouble(o);
       if (d == -1 && PyErr_Occurred()) return stop();
     } else {      // S, Q, K
-      seq = PySequence_Fast(o, "a sequence is expected");
+      // (lane values are kept by a tuple until the call is over: an iterator's are nobody else's, and a list may change while other threads run)
+      seq = c == 'K' ? PySequence_Tuple(o) : PySequence_Fast(o, "a sequence is expected");
       if (!seq) return stop();
       const Py_ssize_t len = PySequence_Fast_GET_SIZE(seq);
       if (len > kMaxRank) { PyErr_SetString(PyExc_ValueError, "too many dims"); return stop(); }
@@ -268,7 +275,7 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
         PyObject* e = PySequence_Fast_GET_ITEM(seq, i);
         if (c == 'K') {
           if (!PyObject_TypeCheck(e, &LaneType)) { PyErr_Format(PyExc_TypeError, "index %d is not a lane value", (int)i); return stop(); }
-          if (!space) space = ((Lane*)e)->shm;
+          over(e);
           l[i] = (int64_t)((Lane*)e)->h;
         } else {
           int64_t v;
@@ -280,16 +287,16 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
       a[na++] = (int64_t)len;
       a[na++] = (int64_t)l;
       if (c == 'S' && f->out == 'X') {
-        made = PyTuple_New(len);
-        for (Py_ssize_t i = 0; made && i < len; ++i) {
+        Py_XSETREF(space, PyTuple_New(len));
+        for (Py_ssize_t i = 0; space && i < len; ++i) {
           PyObject* e = PyLong_FromLongLong(l[i]);
           if (!e) return stop();
-          PyTuple_SET_ITEM(made, i, e);
+          PyTuple_SET_ITEM(space, i, e);
         }
-        if (!made) return stop();
-        space = made;
+        if (!space) return stop();
       }
-      Py_CLEAR(seq);
+      if (c == 'K') lanes = seq, seq = nullptr;
+      else Py_CLEAR(seq);
     }
   }
   void* out = nullptr;
@@ -302,16 +309,20 @@ PyObject* fn_call(PyObject* self, PyObject* const* args, size_t nf, PyObject* kw
     stop();
     return raise_status(ctx, rc);
   }
-  if (f->out == 'V') return make_value(args[0], out);
-  if (f->out == 'N') Py_RETURN_NONE;
-  if (!space && first) space = made = shape_tuple(first->h);
-  if (!space) {
+  if (f->out == 'X' && !space && first) space = shape_tuple(first->h);
+  PyObject* r = nullptr;
+  if (f->out == 'V') {
+    r = make_value(args[0], out);
+  } else if (f->out == 'N') {
+    r = Py_None;
+    Py_INCREF(r);
+  } else if (space) {
+    r = make_lane(args[0], out, space);
+  } else {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "no index space");
     p_ix_free(out);
-    return stop();
   }
-  PyObject* r = make_lane(args[0], out, space);
-  Py_XDECREF(made);
+  stop();
   return r;
 }
 
@@ -319,15 +330,16 @@ PyObject* fn_new(PyTypeObject* type, PyObject* args, PyObject*) {
   PyObject* at;
   const char *sig, *out;
   if (!PyArg_ParseTuple(args, "Oss", &at, &sig, &out)) return nullptr;
-  int words = 1 + (out[0] != 'N'), lists = 0, doubles = 0;
+  int words = 1 + (out[0] != 'N'), lists = 0, doubles = 0, kept = 0;
   for (const char* c = sig; *c; ++c) {
     if (!strchr("vxindpSQK", *c)) { PyErr_SetString(PyExc_ValueError, "unknown letter in a signature"); return nullptr; }
     const bool list = *c == 'S' || *c == 'Q' || *c == 'K';
     words += list ? 2 : *c != 'd';
     lists += list;
     doubles += *c == 'd';
+    kept += *c == 'K';
   }
-  if (strlen(sig) >= sizeof(Fn::sig) || words > 8 || lists > 2 || doubles > 1 || !strchr("VXN", out[0])) { PyErr_SetString(PyExc_ValueError, "signature"); return nullptr; }
+  if (strlen(sig) >= sizeof(Fn::sig) || words > 8 || lists > 2 || doubles > 1 || kept > 1 || !strchr("VXN", out[0])) { PyErr_SetString(PyExc_ValueError, "signature"); return nullptr; }
   void* p;
   if (!address(at, &p)) return nullptr;
   Fn* f = (Fn*)type->tp_alloc(type, 0);
@@ -344,13 +356,13 @@ PyObject* backward(PyObject*, PyObject* args) {      // host, out, dt or None, i
   PyObject *host, *out, *dt, *inputs;
   if (!PyArg_ParseTuple(args, "O!O!OO", &HostBaseType, &host, &ValType, &out, &dt, &inputs)) return nullptr;
   if (dt != Py_None && !PyObject_TypeCheck(dt, &ValType)) { PyErr_SetString(PyExc_TypeError, "the cotangent is not a value"); return nullptr; }
-  PyObject* seq = PySequence_Fast(inputs, "the inputs are a sequence of values");
+  PyObject* seq = PySequence_Tuple(inputs);      // (keeps the values until the call is over)
   if (!seq) return nullptr;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  const Py_ssize_t n = PyTuple_GET_SIZE(seq);
   void** h = (void**)PyMem_Calloc((size_t)(n ? 2 * n : 1), sizeof(void*));
   if (!h) { Py_DECREF(seq); return PyErr_NoMemory(); }
   for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject* e = PySequence_Fast_GET_ITEM(seq, i);
+    PyObject* e = PyTuple_GET_ITEM(seq, i);
     if (!PyObject_TypeCheck(e, &ValType)) {
       PyErr_Format(PyExc_TypeError, "input %d is not a value", (int)i);
       PyMem_Free(h);

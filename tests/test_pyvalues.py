@@ -1,5 +1,8 @@
 """Values and calls of the CPython extension (host/pyvalues.cpp), on the CPU checker."""
 import gc
+import os
+import subprocess
+import sys
 import threading
 import weakref
 
@@ -94,6 +97,32 @@ def test_values_go_when_nobody_has_them(host):
     kept = [again * k for k in range(200)]
     del kept
     assert np.array_equal(again.numpy(), np.arange(3.0))
+
+
+ITERATORS = """
+import numpy as np
+from conftest import capi, entry, pkg
+H = pkg.hostapi
+host = H.Host(api_lib=capi.Lib(entry.ORACLE_LIB, "horc_"))
+x = np.arange(12.0).reshape(3, 4)
+v = host.concrete(x)
+for _ in range(300):
+    got = H._c.tsgather(host, v, (3, 4), ((i + 0 for i in host.ix_space((3, 4)))))
+    assert np.array_equal(got.numpy(), x)
+    lane = H._c.ix_index0(host, v, (i + 0 for i in host.ix_space((3, 4))))
+    assert lane.shm == (3, 4) and np.array_equal(lane.to_val().numpy(), x)
+    p = v.as_input()
+    host.tape_reset()
+    loss = (p * p).ssum0()
+    assert [g.shape for g in host.grad(loss, (v * k for k in (1.0, 2.0)))] == [(3, 4)] * 2
+print("all of them")
+"""
+
+
+def test_arguments_that_nobody_else_has():
+    """Lane values and inputs that an iterator makes live until the call is over (in a process of its own: what reads freed memory may end it)."""
+    r = subprocess.run([sys.executable, "-c", ITERATORS], cwd=os.path.dirname(os.path.abspath(__file__)), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert r.returncode == 0 and "all of them" in r.stdout, r.stdout[-2000:]
 
 
 def test_threads_with_contexts_of_their_own():
