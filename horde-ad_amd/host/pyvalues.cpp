@@ -463,6 +463,7 @@ PyMODINIT_FUNC PyInit__pyvalues() {
   FnType.tp_vectorcall_offset = offsetof(Fn, call);
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
+  if (PyModule_AddStringConstant(m, "SOURCE", PYVALUES_SOURCE) < 0) { Py_DECREF(m); return nullptr; }
   struct { const char* name; PyTypeObject* t; } types[] = {{"HostBase", &HostBaseType}, {"Val", &ValType}, {"Lane", &LaneType}, {"Fn", &FnType}};
   for (auto& t : types) {
     if (PyType_Ready(t.t) < 0) { Py_DECREF(m); return nullptr; }

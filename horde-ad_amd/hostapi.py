@@ -1,5 +1,5 @@
 """Binding of include/hordead_host.h (libhordead_host.so): values and their operations through the CPython extension
-`lib/_pyvalues.so` (host/pyvalues.cpp), everything else through ctypes.
+`lib/_pyvalues.*.so` (host/pyvalues.cpp), everything else through ctypes.
 
 `Host` is a context of the host layer on some provider of the array ABI, `V` a
 tensor value whose methods carry the names of horde-ad's tensor operations
@@ -9,9 +9,11 @@ operators, so that an index function is written as a lambda exactly like the
 reference's `\\[i, k] -> [i + k]` and is called once, symbolically.
 """
 import ctypes as C
+import hashlib
 import importlib.machinery
 import importlib.util
 import os
+import sysconfig
 
 import numpy as np
 
@@ -51,12 +53,23 @@ SIG = {
     "adam_apply": (I, [P, P, D, D, D, P, P, P, P, PP, PP, PP]),
 }
 
+EXTENSION = os.path.join(capi.HERE, "lib", "_pyvalues" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
 def _extension():
-    path = os.path.join(capi.HERE, "lib", "_pyvalues.so")
-    loader = importlib.machinery.ExtensionFileLoader("_pyvalues", path)
-    mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_pyvalues", path, loader=loader))
+    loader = importlib.machinery.ExtensionFileLoader("_pyvalues", EXTENSION)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_pyvalues", EXTENSION, loader=loader))
     loader.exec_module(mod)
+    _check_source(mod.SOURCE, os.path.join(capi.HERE, "host", "pyvalues.cpp"))
     return mod
+
+
+def _check_source(built_from, path):
+    """The extension takes signatures and addresses on trust: one that another source was built to is not used."""
+    if os.path.exists(path):
+        with open(path, "rb") as f:
+            if hashlib.sha256(f.read()).hexdigest()[:16] != built_from:
+                raise ImportError(f"{EXTENSION} is not built from {path} as it is now; run __graft_entry__.build()")
 
 
 _py = _extension()

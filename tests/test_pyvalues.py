@@ -3,6 +3,7 @@ import gc
 import os
 import subprocess
 import sys
+import sysconfig
 import threading
 import weakref
 
@@ -97,6 +98,18 @@ def test_values_go_when_nobody_has_them(host):
     kept = [again * k for k in range(200)]
     del kept
     assert np.array_equal(again.numpy(), np.arange(3.0))
+
+
+def test_built_from_the_source_that_is_there(tmp_path):
+    source = os.path.join(capi.HERE, "host", "pyvalues.cpp")
+    H._check_source(H._py.SOURCE, source)
+    H._check_source(H._py.SOURCE, str(tmp_path / "none"))
+    changed = tmp_path / "pyvalues.cpp"
+    with open(source) as f:
+        changed.write_text(f.read() + "// another line\n")
+    with pytest.raises(ImportError, match="build"):
+        H._check_source(H._py.SOURCE, str(changed))
+    assert H.EXTENSION.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and os.path.samefile(H._py.__file__, H.EXTENSION)
 
 
 ITERATORS = """
