@@ -307,8 +307,8 @@ bool hold_job(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vec
 // smallk.hip, the caller holds launch_mu: the held launch that will write this block, if there is one; a held launch reads and writes more
 std::shared_ptr<HeldJob> held_writer_locked(hgpu_ctx* ctx, const hgpu_buffer* b);
 bool extend_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const std::vector<hgpu_buffer*>& reads, const std::vector<hgpu_buffer*>& writes);
-// ... goes out now; forgotten: it does not (another launch has done its work)
-void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, bool forgotten);
+// ... goes out now
+void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job);
 // A zero-extension (ewise.hip) that waits until something reads its result: a kernel that copies its operand to LDS reads the
 // array that is extended instead (footprint.hip).  Dims as they lie in the dense result, from dst on.
 struct PadJob : HeldJob {

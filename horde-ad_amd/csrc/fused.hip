@@ -1011,7 +1011,7 @@ bool join_head(hgpu_ctx* ctx, int64_t n, int n_in, const hgpu_array* const* in, 
     snprintf(buf, sizeof buf, "fused_head[%lld,phases%d]", (long long)n, (int)job->stages.size() + 1);
     job->label = intern_label(ctx, buf);
   }
-  if (last) end_job_locked(ctx, job, false);
+  if (last) end_job_locked(ctx, job);
   return true;
 }
 

@@ -1651,22 +1651,8 @@ bool extend_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, const
   return false;
 }
 
-void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job, bool forgotten) {
-  if (!ctx->dq) return;
-  DeferredQueue& q = *ctx->dq;
-  if (!forgotten) {
-    flush_singles_locked(ctx, [&](const DeferredQueue::Single& g) { return g.job == job; });
-    return;
-  }
-  for (size_t i = 0; i < q.singles.size(); ++i) {
-    if (q.singles[i].job != job) continue;
-    DeferredQueue::Single g = std::move(q.singles[i]);
-    q.singles.erase(q.singles.begin() + (long)i);
-    for (auto* b : g.reads) q.let_go(b);
-    for (auto* b : g.writes) q.let_go(b);
-    break;
-  }
-  ctx->dq_pending = q.any();
+void end_job_locked(hgpu_ctx* ctx, const std::shared_ptr<HeldJob>& job) {
+  if (ctx->dq) flush_singles_locked(ctx, [&](const DeferredQueue::Single& g) { return g.job == job; });
 }
 
 void flush_deferred(hgpu_ctx* ctx) {
