@@ -277,10 +277,11 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     // Microseconds, as measured: a step of 16 k of a 64 x 64 tile takes 0.62 alone on its CU, 0.56 with another one
     // there, 0.5 with more; 5 for the launch; partial results as below.  (300 x 784 over 5000, main kernel / with the
     // sums: 4 chunks = 260 blocks 82 / 89, 7 = 455 56 / 63, 10 = 650 54 / 63, 32 = 2080 52 / 65.)
-    // Partial results at 4 TB/s, between other kernels that want the caches too (6 TB/s when nothing else runs, and for the two
-    // or three that a program reads itself): gradients of dense 784-300-100-10, batch 5000, 6 / 4 TB/s 197.4 / 190.8 us (15 / 11 shares
+    // Partial results at 4 TB/s, between other kernels that want the caches too (6 TB/s when nothing else runs): gradients of dense 784-300-100-10, batch 5000, 6 / 4 TB/s 197.4 / 190.8 us (15 / 11 shares
     // of the first weights' gradient), 784-2000-300-10, batch 1500, 385 / 380, 784-128-900-10, batch 3000, 192 / 187; at 2.5 TB/s
-    // 784-650-333-10, batch 4000, goes from 374 to 408.
+    // 784-650-333-10, batch 4000, goes from 374 to 408.  Two or three of them that the pass behind the product reads itself (a layer's forward
+    // product) at 6 TB/s: no launch adds them up.  One layer in fifty takes other shares for it; gradients of dense 784-523-64-10, batch 1815, with 4 / 6 TB/s
+    // 156.2 / 147.5 us, 784-325-64-10, 2905, 154.3 / 145.5, 784-1202-915-10, 2452, 596 / 583, 784-1814-895-10, 658, 316 / 298, 784-470-1995-10, 584, 225 / 226.
     double best = 1e300;
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64) * p.BT * nt;
     for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
@@ -297,9 +298,11 @@ int gemm_single_dims(hgpu_ctx* ctx, const GemmParams& p, int dtype, const void* 
     auto chunks = [&](int64_t per_cu) { return std::max<int64_t>(1, std::min<int64_t>(per_cu * ctx->num_cu / tiles, p.K / 64)); };
     split = (int)(p.K >= 512 * chunks(2) ? chunks(4) : chunks(2));
   } else {
-    // Microseconds, as measured: a step of 16 k of a 128 x 128 tile 1.4 alone on its CU and 0.92 for each of several;
-    // 8 for the launch with its first loads and last stores; for partial results a second launch and their bytes once
-    // out and once in.  (One after another, without the sums: 2048 x 8192 over 2048 464, 2048 x 784 over 8192 217, 300 x 5000 over 784 29.)
+    // Microseconds, as they were while the loop waited for its loads: a step of 16 k of a 128 x 128 tile 1.4 alone on its CU and 0.92 for each of
+    // several; 8 for the launch with its first loads and last stores; for partial results a second launch and their bytes once
+    // out and once in.  (With loads a step ahead it is 0.89 alone and 0.78 for each of two, 2048 x 2048 and 2048 x 4096 over 2048 to 8192; 2048 x 784 over
+    // 8192 198 us without the sums, then 217, 300 x 5000 over 784 30 for 29.  Shares and the line below are still by the old steps, whose
+    // choices are the ones measured; products just short of the line may be faster here by now.)
     double best = 1e300;
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128) * p.BT * nt;
     for (int64_t sp = 1; sp <= 64 && sp <= p.K / 64; ++sp) {
@@ -450,7 +453,7 @@ constexpr int kRecurrenceTerms = 8;
 
 // Shares of K for fp32 products on tiles of 128 x 128 that go out together: each was cut to fill the device alone, and together they
 // take several rounds of short blocks, which fetch their first operands and leave partial results each.  Longer shares where
-// the model of the single product, with two blocks to a CU, says so; never more of them, so that the partial results have their memory.  False:
+// the model of the single product (gemm_single_dims: 0.92 us a step for each of two blocks on a CU) says so; never more of them, so that the partial results have their memory.  False:
 // as they are.  The three products of 128 x 128 over 27 x 5000 of a recurrence, 18 / 9 / 6 / 5 / 4 / 3 shares a term (504 to 84 blocks each), us of its whole
 // gradient: 569 / 543 / 530 / 530 / 532 / 554.   (Products whose blocks differ in
 // length fill one another's gaps: 2048 x 784 and 2048 x 2048 over 8192, 57 and 256 steps, lost 12 us of their gradient by this model.  fp64 and thin products come

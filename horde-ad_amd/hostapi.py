@@ -238,7 +238,13 @@ class Host(_py.HostBase):
         return _c.tsiota(self, n, dtype)
 
     def grad(self, out, inputs, dt=None):
-        """Cotangents of `inputs` for d(out) = dt (default: ones, as `grad` uses)."""
+        """Cotangents of `inputs` for d(out) = dt (default: ones, as `grad` uses).
+
+        The tape keeps what the reverse pass may read until `tape_reset`, and what it keeps counts as wanted: a
+        zero-extension that a convolution's kernels read through, or a gather that is multiplied and summed at once, is
+        written after all while the tape has it.  Reset the tape when the gradients have been asked for, as
+        `Workload.gradient` does; values made before stay usable as constants, but an input made before a reset
+        has no derivative after it."""
         return _py.backward(self, out, dt, inputs)
 
     # -- host loops of the tensor class (the reference's `Concrete` instance runs

@@ -41,7 +41,8 @@ hgpu_ctx* hh_array_ctx(hh_ctx* ctx);
 /* Elementwise operations are deferred and handed to the provider as fused
  * programs (default, when the provider has fused_map); 0 runs them one by one. */
 int hh_set_fusion(hh_ctx* ctx, int on);
-/* Forgets the recorded operations; values made before stay usable as constants. */
+/* Forgets the recorded operations, and with them what only they kept; values made before stay usable as constants
+ * (hh_backward by an input made before is HGPU_ERR_INVALID). */
 int hh_tape_reset(hh_ctx* ctx);
 
 /* tsconcrete (OpsConcrete.hs:120-124): a value from host data; `requires_grad`
