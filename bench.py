@@ -50,6 +50,15 @@ def array_ctx(capi, host):
     return ctx
 
 
+def short(o, key=None):
+    """What the line holds beside its results with five digits: a line that runs to 20,000 characters is cut where logs are kept."""
+    if isinstance(o, float):
+        return o if key in ("value", "loss", "ms_per_step", "samples_per_s") else float("%.5g" % o)
+    if isinstance(o, dict):
+        return {k: short(v, k) for k, v in o.items()}
+    return [short(v) for v in o] if isinstance(o, list) else o
+
+
 def time_steps(host, wl, ps, ds, steps, warmup):
     for _ in range(warmup):
         wl.gradient(host, ps, ds)
@@ -287,6 +296,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--workload", default="c3", help="headline config: c0..c4")
     ap.add_argument("--only", action="store_true", help="measure the headline config only")
+    ap.add_argument("--all-kernels", action="store_true", help="every kernel of every config, not the three dearest of those beside the headline")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--eager", action="store_true", help="time op-by-op submission instead of the recorded graph")
     ap.add_argument("--train", action="store_true",
@@ -425,7 +435,10 @@ def main():
         line["riders"] = riders
     if train:
         line["training_step"] = train
-    print(json.dumps(line))
+    if not args.all_kernels:
+        for c in line["configs"].values():
+            c["kernels"] = c["kernels"][:3]
+    print(json.dumps(short(line)))
 
 
 if __name__ == "__main__":
